@@ -76,6 +76,16 @@ int vui_codec_reset(vui_codec* c, vui_stream_t stream);
  * frames between two resets; further frames raise the status flag and reuse the last position. */
 int vui_codec_decode_frame(vui_codec* c, const int64_t* codes, int32_t n_q, float* audio_out, vui_stream_t stream);
 
+/* Most frames of one vui_codec_decode_block call (32, or max_seq where that is less). */
+int32_t vui_codec_block_frames(const vui_codec* c);
+
+/* n_frames consecutive frames in one pass: codes (n_frames, n_q) int64 -> audio_out (n_frames * hop), the samples that
+ * as many vui_codec_decode_frame calls give (sums in another order), and the same state behind them, so that blocks and
+ * single frames may follow each other.  Every weight is read once per block.  The block must fit in front of max_seq:
+ * one that does not raises the status flag and its samples are not the frames' own.  No counterpart in the reference,
+ * whose offline forward (qwen_codec.py:1191-1224) takes all frames at once. */
+int vui_codec_decode_block(vui_codec* c, const int64_t* codes, int32_t n_frames, int32_t n_q, float* audio_out, vui_stream_t stream);
+
 /* The one-column steps of a frame (codebook rows ... first upsampling conv) run as one persistent kernel when
  * the device can keep 256 workgroups resident and the dimensions fit, otherwise as separate launches (same
  * sums in another order).  enable = 1/0 switches the persistent form on/off, -1 only queries; returns 1 when

@@ -214,3 +214,51 @@ def test_full_dims_codec_ctx_session(full):
     assert ctx.n_frames == 130
     ctx.reset()
     assert not dec.is_streaming
+
+
+@pytest.mark.parametrize("T", [2, 3, 31, 32, 33, 40])
+def test_blocks_of_frames_equal_single_frames(small, T):
+    """Offline calls take up to 32 frames per pass: against the oracle, and against the same frames one at a time (fp32
+    sums in another order through ~60 layers: 2e-5, measured 2e-6), whatever is in the rings from before."""
+    d, ora, dec = small
+    codes = torch.randint(0, d.codebook_size, (1, d.n_codebooks, T), generator=torch.Generator().manual_seed(T))
+    ref = ora.forward(codes)
+    got = dec(codes.cuda())
+    with dec.streaming(1):
+        one = torch.cat([dec(codes[:, :, t:t + 1].cuda()).clone() for t in range(T)], dim=-1)
+    assert err(got, ref) < TOL and err(got, one.cpu()) < 2e-5
+
+
+def test_blocks_and_single_frames_in_one_stream(small):
+    """A stream may change between blocks and single frames anywhere; past max_seq frames only the flag is raised."""
+    d, ora, dec = small
+    codes = torch.randint(0, d.codebook_size, (1, d.n_codebooks, d.max_seq + 2), generator=torch.Generator().manual_seed(6)).cuda()
+    with dec.streaming(1):
+        one = torch.cat([dec(codes[:, :, t:t + 1]).clone() for t in range(d.max_seq)], dim=-1)
+        assert dec.frames_since_reset() == d.max_seq
+    with dec.streaming(1):
+        parts, t = [], 0
+        for n in (1, 2, 5, 1, 1, 16, 3, 9, 2):
+            parts.append(dec(codes[:, :, t:t + n]).clone())
+            t += n
+        assert t == d.max_seq and dec.frames_since_reset() == t
+    assert err(torch.cat(parts, dim=-1), one.cpu()) < 2e-5
+    with dec.streaming(1):
+        got = dec(codes)  # two frames more than fit
+        assert err(got[..., :one.shape[-1]], one.cpu()) < 2e-5
+        with pytest.raises(RuntimeError, match="max_seq"):
+            dec.frames_since_reset()
+
+
+def test_full_dims_blocks_equal_single_frames(full):
+    d, sd, dec, fx = full
+    codes = torch.randint(0, d.codebook_size, (1, d.n_codebooks, 45), generator=torch.Generator().manual_seed(7)).cuda()
+    got = dec(codes)
+    for n in (True, False):
+        try:
+            dec.persistent(int(n))
+            with dec.streaming(1):
+                one = torch.cat([dec(codes[:, :, t:t + 1]).clone() for t in range(codes.shape[2])], dim=-1)
+        finally:
+            dec.persistent(1)
+        assert err(got, one.cpu()) < 5e-5  # measured 1e-5

@@ -207,6 +207,8 @@ class QwenCodecDecoder:
         self.handle = h
         self.hop = self.cfg.hop
         self._streaming = False
+        self._frames = 0  # frames since the last reset (of the calls made here)
+        self._block = int(lib.vui_codec_block_frames(h))
         self._cap_stream = torch.cuda.Stream(device=self.device)
         self._graphs: dict[int, object] = {}
         self._stream_codes_in = torch.zeros(self.cfg.n_codebooks, dtype=torch.long, device=self.device)
@@ -273,6 +275,7 @@ class QwenCodecDecoder:
         return _Stream(self)
 
     def reset_streaming(self) -> None:
+        self._frames = 0
         _lib.check(self.lib.vui_codec_reset(self.handle, torch.cuda.current_stream().cuda_stream), "vui_codec_reset")
 
     def frames_since_reset(self) -> int:
@@ -312,6 +315,7 @@ class QwenCodecDecoder:
     # ---- forward ----
     def _frame(self, codes_q: Tensor, out: Tensor) -> None:
         n_q = codes_q.shape[0]
+        self._frames += 1
         g = self._graphs.get(n_q)
         if g is not None:
             self._stream_codes_in[:n_q].copy_(codes_q)
@@ -341,8 +345,18 @@ class QwenCodecDecoder:
             return self._stream_out
         audio = torch.empty(1, 1, T * self.hop, dtype=torch.float32, device=self.device)
         flat = audio.view(-1)
-        for t in range(T):
-            self._frame(ct[t], flat[t * self.hop:(t + 1) * self.hop])
+        st = torch.cuda.current_stream().cuda_stream
+        t = 0
+        while t < T:  # blocks of frames; single frames past the decoder's window, where only the status flag is left to raise
+            n = min(T - t, self._block)
+            if n > 1 and self._frames + n <= self.cfg.max_seq:
+                _lib.check(self.lib.vui_codec_decode_block(self.handle, ct[t].data_ptr(), n, n_q, flat[t * self.hop:].data_ptr(), st),
+                           "vui_codec_decode_block")
+                self._frames += n
+            else:
+                n = 1
+                self._frame(ct[t], flat[t * self.hop:(t + 1) * self.hop])
+            t += n
         if offline:
             self.reset_streaming()
         return audio

@@ -32,10 +32,11 @@ typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 
 struct Ring {
   float* p;
-  int rs;     // columns per channel (power of two)
-  int mask;   // rs - 1
+  int rs;     // columns per channel (power of two; a buffer of several frames: any)
+  int mask;   // rs - 1 (a buffer of several frames: all ones)
   int pad;    // history columns in front of a frame
   int tstep;  // columns a frame adds (0: plain buffer, always at column 0)
+  int id;     // host side: its place in vui_codec::twins
 };
 
 __device__ __forceinline__ int ring_base(const Ring& r, int f) { return (f * r.tstep) & r.mask; }
@@ -64,11 +65,13 @@ struct CvGemm {
   Ring out_act;   // p may be null: snake with (ea, ib) of the consumer
   const float* ea;
   const float* ib;
-  const int* ctr;  // frames started; this frame is *ctr - 1
+  const int* ctr;  // frames started; this pass is frames *ctr - nf ... *ctr - 1
+  int nf;
   int splits;      // workgroups that share one tile's (tap, channel) units; > 1: parts meet in `part`
   float* part;     // (tiles, splits, TT*64*4) partial sums
   int* cnt;        // (tiles) arrival counters, zero between launches
-  int tt;          // 16-column blocks per tile (host side: picks the instantiation)
+  int tt;          // 16-column blocks per tile (host side: picks the instantiation); 0: cv_wide_kernel with tile kWide[wide]
+  int wide;
 };
 
 // A vocoder that shares the GPU with other kernels (vui_codec_workgroups) reads its weights - 423 MB per frame, each
@@ -93,6 +96,7 @@ template <bool NT> __device__ __forceinline__ float4 cv_ld_w(const float* p) {
 template <int TT, bool DB> struct Nu { static constexpr int N = TT == 1 ? 8 : (TT == 2 ? (DB ? 5 : 6) : 3); };
 
 #define CV_NW 4  // waves per workgroup
+#define CV_WIDE_T 64  // columns from which cv_wide_kernel takes a product of several frames
 
 // One 16-row x 16*TT-column output tile.  `red` is CV_NW * TT * 64 * 4 floats of LDS.
 template <int TT, bool DB, bool NT>
@@ -167,7 +171,7 @@ __device__ __forceinline__ void cv_gemm_tile(const CvGemm& p, const int m0, cons
 
   constexpr int STEP = NU;
   load_a(ub, a0);
-  const int f = *p.ctr - 1;
+  const int f = *p.ctr - p.nf;
   ib_ = ring_base(p.in, f);
   load_b(ub, b0);
   // what the epilogue adds is requested now as well
@@ -191,7 +195,26 @@ __device__ __forceinline__ void cv_gemm_tile(const CvGemm& p, const int m0, cons
   }
   // 1/rms of the input column while the first operands are in flight; applied to the sums at the end
   float rstd = 1.f;
-  if (p.in_mode == IN_RMS) {
+  if (p.in_mode == IN_RMS && p.T > 1) {  // a column per frame: 16 threads share one
+    __shared__ float sq[TT * 256];
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt) {
+      const int t = min(t0 + tt * 16 + (tid & 15), p.T - 1);
+      float ss = 0.f;
+      for (int c = tid >> 4; c < Cin; c += 16) {
+        const float v = *ring_ptr(p.in, ib_, c, p.in.pad + t);
+        ss = fmaf(v, v, ss);
+      }
+      sq[tt * 256 + (tid & 15) * 16 + (tid >> 4)] = ss;
+    }
+    __syncthreads();
+    if (tid < TT * 64) {
+      float ss = 0.f;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) ss += sq[(tid >> 6) * 256 + (tid & 15) * 16 + i];
+      rstd = 1.0f / sqrtf(ss / (float)Cin + p.eps);
+    }
+  } else if (p.in_mode == IN_RMS) {
     float ss = 0.f;
     for (int c = lane; c < Cin; c += WAVE) {
       const float v = *ring_ptr(p.in, ib_, c, p.in.pad);
@@ -264,7 +287,7 @@ __device__ __forceinline__ void cv_gemm_tile(const CvGemm& p, const int m0, cons
     const int tt = tid >> 6, l = tid & 63;
     const int t = t0 + tt * 16 + (l & 15);
     if (t >= p.T) return;
-    if (p.epi == EPI_SILU_PAIR) {  // one column per frame
+    if (p.epi == EPI_SILU_PAIR) {
 #pragma unroll
       for (int r = 0; r < 4; r += 2) {
         const float ga = v[r] * rstd, up = v[r + 1] * rstd;
@@ -301,25 +324,230 @@ __global__ __launch_bounds__(CV_NW * 64, 2) void cv_gemm1_kernel(const CvGemm p)
   cv_gemm_tile<TT, false, NT>(p, blockIdx.x * 16, blockIdx.y * (16 * TT), red, blockIdx.y * gridDim.x + blockIdx.x, blockIdx.z);
 }
 
-// ---- codebook rows of one frame: [sum of the semantic rows | sum of the acoustic rows]; starts the frame ----
+// ---- the same product for many columns (several frames at once) ----
+// Bound by the fp32 matrix instructions (157 TFLOP/s): 256 flops per CU and cycle against 8 bytes of operands, so
+// tiles of BM x BN = 128 x 128 (or what divides M) through LDS: a K step is one (tap, 32-channel) unit, fetched into
+// registers while the one before it is multiplied, two LDS buffers, one barrier per step.  v_mfma_f32_32x32x2_f32; the
+// lane halves take k = 8j + s and 8j + 4 + s, so that a lane's weights of four steps are one 16-byte LDS read.
+// Where the tiles are fewer than the CUs their units are split over workgroups, and cv_finish_kernel adds the parts.
+typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
+
+#define CVW_RUN 4
+#define CVW_AS 36  // floats between weight rows in LDS: 16-byte reads of 8 rows fall on different banks
+
+// bias, activation or residual, and the outputs of one column of eight rows m, m + step, ... (uniform over a wave)
+struct CvBases { int res, raw, act; };
+__device__ __forceinline__ void cv_finish_rows(const CvGemm& p, const CvBases& b, int m, int step, int t, float (&y)[8]) {
+  // one condition around eight rows each: with the conditions inside the rows every load was waited for by itself
+  int ch[8], col[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) { ch[e] = m + e * step; col[e] = t; }
+  if (p.bias) {
+    float v[8];
+    if (p.bias_div == 1) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = p.bias[ch[e]];
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = p.bias[ch[e] / p.bias_div];
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) y[e] += v[e];
+  }
+  if (p.tc_stride > 0) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int c = ch[e] / p.tc_stride;
+      col[e] = t * p.tc_stride + (ch[e] - c * p.tc_stride);
+      ch[e] = c;
+    }
+  }
+  if (p.epi == EPI_GELU) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) y[e] = 0.5f * y[e] * (1.0f + erff(y[e] * 0.70710678118654752f));
+  } else if (p.epi == EPI_RES || p.epi == EPI_SCALE_RES) {
+    float v[8], sc[8] = {1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = *ring_ptr(p.res, b.res, ch[e], p.res.pad + col[e]);
+    if (p.epi == EPI_SCALE_RES) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) sc[e] = p.scale[ch[e]];
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) y[e] = v[e] + sc[e] * y[e];
+  }
+  if (p.out_raw.p) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) *ring_ptr(p.out_raw, b.raw, ch[e], p.out_raw.pad + col[e]) = y[e];
+  }
+  if (p.out_act.p) {
+    float ea[8], ib[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) { ea[e] = p.ea[ch[e]]; ib[e] = p.ib[ch[e]]; }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float s = sinf(y[e] * ea[e]);
+      *ring_ptr(p.out_act, b.act, ch[e], p.out_act.pad + col[e]) = y[e] + ib[e] * s * s;
+    }
+  }
+}
+
+template <int MI, int NI, int WM, int WN>
+__global__ __launch_bounds__(512, MI * WM == 4 ? 4 : 2) void cv_wide_kernel(const CvGemm p) {
+  constexpr int NT = 512, BM = 32 * MI * WM, BN = 32 * NI * WN, BS = BN + 8;  // BS: rows 4 apart start 32 banks apart
+  constexpr int NA = (BM * 8 + NT - 1) / NT, NB = 32 * BN / NT, KR = NT / BN;  // 16-byte / 4-byte loads per thread and step
+  static_assert(WM * WN == 8 && NT % BN == 0, "eight waves, whole rows per pass");
+  constexpr int OPS = 2 * (BM * CVW_AS + 32 * BS);
+  __shared__ __align__(16) float lds[OPS > BM * BS ? OPS : BM * BS];  // the operands, then the sums
+  auto la = [&](int b, int i) -> float& { return lds[b * BM * CVW_AS + i]; };
+  auto lb = [&](int b, int i) -> float& { return lds[2 * BM * CVW_AS + b * 32 * BS + i]; };
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int l32 = lane & 31, h = lane >> 5, wm = wave % WM, wn = wave / WM;
+  const int m0 = blockIdx.x * BM, t0 = blockIdx.y * BN, z = blockIdx.z;
+  const int G = p.Cin >> 5, Uall = p.taps * G;
+  const int ub = (int)((int64_t)Uall * z / p.splits), ue = (int)((int64_t)Uall * (z + 1) / p.splits);
+  const int f = *p.ctr - p.nf, ib_ = ring_base(p.in, f);
+
+  // acc: the products of CVW_RUN units; sum: those before.  One chain over all units (168 of them in block 1) would
+  // round each step against the full sum: 1.4 times the error against 64 bits of the audio.
+  floatx16 acc[MI][NI], sum[MI][NI];
+  const floatx16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int n = 0; n < NI; ++n) acc[i][n] = sum[i][n] = zero;
+
+  const int bc = tid % BN, bk = tid / BN;  // this thread's column and first channel of a step
+  floatx4 ra[NA];  // native vectors: an array of HIP's float4 structs stayed in scratch memory
+  float rb[NB];
+  int tap = ub / G, grp = ub - tap * G;
+  auto fetch = [&]() {
+    const float* wp = p.W + ((size_t)tap * p.M + m0 + (tid >> 3)) * p.Cin + grp * 32 + (tid & 7) * 4;
+#pragma unroll
+    for (int i = 0; i < NA; ++i)
+      if ((i + 1) * (NT / 8) <= BM || (tid >> 3) + i * (NT / 8) < BM) ra[i] = *reinterpret_cast<const floatx4*>(wp + (size_t)i * (NT / 8) * p.Cin);
+    // columns behind T are whatever the ring holds there: they reach no output
+    const float* xp = ring_ptr(p.in, ib_, grp * 32 + bk, t0 + bc + tap * p.dil);
+#pragma unroll
+    for (int i = 0; i < NB; ++i) rb[i] = xp[(size_t)i * KR * p.in.rs];
+    if (++grp == G) { grp = 0; ++tap; }
+  };
+  auto stage = [&](int b) {
+#pragma unroll
+    for (int i = 0; i < NA; ++i)
+      if ((i + 1) * (NT / 8) <= BM || (tid >> 3) + i * (NT / 8) < BM)
+        *reinterpret_cast<floatx4*>(&la(b, ((tid >> 3) + (NT / 8) * i) * CVW_AS + (tid & 7) * 4)) = ra[i];
+#pragma unroll
+    for (int i = 0; i < NB; ++i) lb(b, (bk + KR * i) * BS + bc) = rb[i];
+  };
+  if (ub < ue) {
+    fetch();
+    stage(0);
+  }
+  __syncthreads();
+  for (int u = ub; u < ue; ++u) {
+    const int b = (u - ub) & 1;
+    if (u + 1 < ue) fetch();
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      floatx4 a[MI];
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+        a[i] = *reinterpret_cast<const floatx4*>(&la(b, ((wm * MI + i) * 32 + l32) * CVW_AS + 8 * j + 4 * h));
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        float x[NI];
+#pragma unroll
+        for (int n = 0; n < NI; ++n) x[n] = lb(b, (8 * j + 4 * h + s) * BS + (wn * NI + n) * 32 + l32);
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+#pragma unroll
+          for (int n = 0; n < NI; ++n) acc[i][n] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][s], x[n], acc[i][n], 0, 0, 0);
+        }
+      }
+    }
+    if ((u - ub) % CVW_RUN == CVW_RUN - 1 || u + 1 == ue) {
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int n = 0; n < NI; ++n) { sum[i][n] += acc[i][n]; acc[i][n] = zero; }
+    }
+    if (u + 1 < ue) stage(b ^ 1);
+    __syncthreads();
+  }
+
+  if (p.splits > 1) {  // cv_finish_kernel adds the parts
+    float* part = p.part + ((size_t)z * p.M + m0) * (gridDim.y * BN) + t0 + wn * NI * 32 + l32;
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+#pragma unroll
+        for (int n = 0; n < NI; ++n)
+          part[(size_t)((wm * MI + i) * 32 + 8 * (r >> 2) + 4 * h + (r & 3)) * (gridDim.y * BN) + n * 32] = sum[i][n][r];
+    return;
+  }
+  // The sums go through LDS so that a wave finishes whole rows: what depends on the row is scalar, and 64 columns are
+  // written in a run.
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int n = 0; n < NI; ++n)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        lds[((wm * MI + i) * 32 + 8 * (r >> 2) + 4 * h + (r & 3)) * BS + (wn * NI + n) * 32 + l32] = sum[i][n][r];
+  __syncthreads();
+  constexpr int RW = NT / BN;  // rows that the workgroup finishes side by side
+  const int t = t0 + tid % BN, row0 = wave / (BN / 64);
+  if (t >= p.T) return;
+  const CvBases b{ring_base(p.res, f), ring_base(p.out_raw, f), ring_base(p.out_act, f)};
+  static_assert(BM % (8 * RW) == 0, "whole batches of rows");
+  for (int row = row0; row < BM; row += 8 * RW) {
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = lds[(row + e * RW) * BS + tid % BN];
+    cv_finish_rows(p, b, m0 + row, RW, t, v);
+  }
+}
+
+// Parts of the tiles of cv_wide_kernel, (splits, M, cols), added in order: a wave per 64 columns x 8 rows.  A launch of
+// its own: with the last of a tile's workgroups adding and finishing 128 x 128 results by itself, the 1x1 convolutions of
+// block 1 took 85 us per 32 frames, 7 us of it products.
+__global__ __launch_bounds__(256) void cv_finish_kernel(const CvGemm p, int cols) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t = blockIdx.x * 64 + (threadIdx.x & 63);
+  const int m = blockIdx.y * 32 + wave * 8;
+  if (t >= p.T) return;
+  float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  for (int z = 0; z < p.splits; ++z) {
+    const float* src = p.part + ((size_t)z * p.M + m) * cols + t;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] += src[(size_t)e * cols];
+  }
+  const int f = *p.ctr - p.nf;
+  cv_finish_rows(p, CvBases{ring_base(p.res, f), ring_base(p.out_raw, f), ring_base(p.out_act, f)}, m, 1, t, v);
+}
+
+// ---- codebook rows of one frame per workgroup: [sum of the semantic rows | sum of the acoustic rows]; starts the pass ----
 struct CvVq {
-  const int64_t* codes;
+  const int64_t* codes;  // (nf, n_q)
   int n_q, n_sem, CS, cd;
   const float* embed;  // (n_codebooks, CS, cd)
-  float* x;            // (2*cd) as a one-column plain buffer with rs = 1
+  float* x;            // (2*cd, rs): a column per frame
+  int rs, nf;
   int* ctr;
   int* err;
   int max_seq;
 };
 
 __global__ __launch_bounds__(256) void cv_vq_kernel(const CvVq p) {
+  const int64_t* codes = p.codes + (size_t)blockIdx.x * p.n_q;
   for (int c = threadIdx.x; c < p.cd; c += blockDim.x) {
     float s0 = 0.f, s1 = 0.f;
     for (int i0 = 0; i0 < p.n_q; i0 += 16) {  // 16 codes, then their 16 rows, are requested together
       long code[16];
       float e[16];
 #pragma unroll
-      for (int k = 0; k < 16; ++k) code[k] = i0 + k < p.n_q ? p.codes[i0 + k] : 0;
+      for (int k = 0; k < 16; ++k) code[k] = i0 + k < p.n_q ? codes[i0 + k] : 0;
 #pragma unroll
       for (int k = 0; k < 16; ++k) {
         if (code[k] < 0 || code[k] >= p.CS) { code[k] = code[k] < 0 ? 0 : p.CS - 1; if (c == 0) *p.err = 1; }
@@ -330,26 +558,39 @@ __global__ __launch_bounds__(256) void cv_vq_kernel(const CvVq p) {
         if (i0 + k < p.n_sem) s0 += e[k]; else s1 += e[k];
       }
     }
-    p.x[c] = s0;
-    p.x[p.cd + c] = s1;
+    p.x[(size_t)c * p.rs + blockIdx.x] = s0;
+    p.x[(size_t)(p.cd + c) * p.rs + blockIdx.x] = s1;
   }
-  if (threadIdx.x == 0) {
+  if (threadIdx.x == 0 && blockIdx.x == 0) {
     int f = *p.ctr;
-    if (f >= p.max_seq) { *p.err = 2; f = p.max_seq - 1; }  // stay on the last position: nothing runs out of bounds
-    *p.ctr = f + 1;
+    if (f + p.nf > p.max_seq) { *p.err = 2; f = p.max_seq - p.nf; }  // stay on the last positions: nothing runs out of bounds
+    *p.ctr = f + p.nf;
   }
 }
 
-// ---- pre-transformer attention of one new position: rotate-half RoPE, cache append, softmax, P.V ----
+// ---- pre-transformer attention of nf new positions: rotate-half RoPE, cache append, softmax, P.V ----
 struct CvAttn {
-  const float* qkv;  // (3*A): q | k | v
+  const float* qkv;  // (3*A, rs): q | k | v, a column per position
   float* kc;         // (H, max_seq, hd)
   float* vc;
-  float* out;        // (A)
+  float* out;        // (A, rs_out)
   const float* inv_freq;  // (hd/2)
-  int H, hd, max_seq;
+  int rs, rs_out, H, hd, max_seq, nf;
   const int* ctr;
 };
+
+// keys and values of several positions, ahead of the launch that attends: workgroup (head, position)
+__global__ __launch_bounds__(64) void cv_append_kernel(const CvAttn p) {
+  const int h = blockIdx.x, i = blockIdx.y, d = threadIdx.x, hd = p.hd, half = hd >> 1, A = p.H * hd;
+  const int pos = *p.ctr - p.nf + i;
+  if (d >= hd) return;
+  const float ang = (float)pos * p.inv_freq[d % half];
+  const float* kk = p.qkv + (size_t)(A + h * hd) * p.rs + i;
+  const float kr = d < half ? -kk[(size_t)(d + half) * p.rs] : kk[(size_t)(d - half) * p.rs];
+  const size_t at = ((size_t)h * p.max_seq + pos) * hd + d;
+  p.kc[at] = kk[(size_t)d * p.rs] * cosf(ang) + kr * sinf(ang);
+  p.vc[at] = p.qkv[(size_t)(2 * A + h * hd + d) * p.rs + i];
+}
 
 __global__ __launch_bounds__(256) void cv_attn_kernel(const CvAttn p) {
   extern __shared__ float sm[];  // q[hd] | sc[max_seq] | part[4][hd] | red[8]
@@ -359,19 +600,22 @@ __global__ __launch_bounds__(256) void cv_attn_kernel(const CvAttn p) {
   float* red = part + 4 * p.hd;
   const int h = blockIdx.x, tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int hd = p.hd, half = hd >> 1, A = p.H * hd;
-  const int pos = *p.ctr - 1;
+  const int pos = *p.ctr - p.nf + (int)blockIdx.y;
   float* kh = p.kc + (size_t)h * p.max_seq * hd;
   float* vh = p.vc + (size_t)h * p.max_seq * hd;
   if (tid < hd) {
     const float ang = (float)pos * p.inv_freq[tid % half];
     const float cs = cosf(ang), sn = sinf(ang);
-    const float* qq = p.qkv + h * hd;
-    const float* kk = p.qkv + A + h * hd;
-    const float qr = tid < half ? -qq[tid + half] : qq[tid - half];
-    const float kr = tid < half ? -kk[tid + half] : kk[tid - half];
-    q[tid] = qq[tid] * cs + qr * sn;
-    kh[(size_t)pos * hd + tid] = kk[tid] * cs + kr * sn;
-    vh[(size_t)pos * hd + tid] = p.qkv[2 * A + h * hd + tid];
+    const size_t rs = p.rs;
+    const float* qq = p.qkv + h * hd * rs + blockIdx.y;
+    const float qr = tid < half ? -qq[(tid + half) * rs] : qq[(tid - half) * rs];
+    q[tid] = qq[tid * rs] * cs + qr * sn;
+    if (p.nf == 1) {
+      const float* kk = qq + A * rs;
+      const float kr = tid < half ? -kk[(tid + half) * rs] : kk[(tid - half) * rs];
+      kh[(size_t)pos * hd + tid] = kk[tid * rs] * cs + kr * sn;
+      vh[(size_t)pos * hd + tid] = kk[(A + tid) * rs];
+    }
   }
   __syncthreads();  // this workgroup's own cache row is visible to all its threads after the barrier
   // scores: a group of 16 lanes per key (features l16, l16 + 16, ...), four keys of a group in flight
@@ -424,7 +668,7 @@ __global__ __launch_bounds__(256) void cv_attn_kernel(const CvAttn p) {
     part[wave * hd + lane] = o;
   }
   __syncthreads();
-  if (tid < hd) p.out[h * hd + tid] = ((part[tid] + part[hd + tid]) + (part[2 * hd + tid] + part[3 * hd + tid])) / sum;
+  if (tid < hd) p.out[(size_t)(h * hd + tid) * p.rs_out + blockIdx.y] = ((part[tid] + part[hd + tid]) + (part[2 * hd + tid] + part[3 * hd + tid])) / sum;
 }
 
 // =============================================================================================
@@ -851,28 +1095,39 @@ struct CvDwLn {
   const float* lnw;
   const float* lnb;
   float* out;        // (C, rs_out) plain
-  int rs_out, C, k;
+  int rs_out, C, nf;
   float eps;
   const int* ctr;
 };
 
 #define DW_MAXC 8  // channels per thread
+#define DW_K 7     // taps
 
 __global__ __launch_bounds__(256) void cv_dwln_kernel(const CvDwLn p) {
   __shared__ float red[8];
   const int t = blockIdx.x, tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int f = *p.ctr - 1, base = ring_base(p.in, f);
+  const int f = *p.ctr - p.nf, base = ring_base(p.in, f);
   float v[DW_MAXC];
   float s = 0.f;
+  // every load of four channels is requested before the first is needed (a loop over a tap count known only at run time
+  // took a round trip per tap: 9.7 us per launch of one frame)
 #pragma unroll
-  for (int i = 0; i < DW_MAXC; ++i) {
-    const int c = tid + 256 * i;
-    v[i] = 0.f;
-    if (c < p.C) {
-      float a = p.b[c];
-      for (int k = 0; k < p.k; ++k) a = fmaf(p.w[c * p.k + k], *ring_ptr(p.in, base, c, t + k), a);
-      v[i] = a;
-      s += a;
+  for (int i0 = 0; i0 < DW_MAXC; i0 += 4) {
+    if (256 * i0 >= p.C) break;
+    float x[4][DW_K], w[4][DW_K], a[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int c = min(tid + 256 * (i0 + i), p.C - 1);
+      a[i] = p.b[c];
+#pragma unroll
+      for (int k = 0; k < DW_K; ++k) { x[i][k] = *ring_ptr(p.in, base, c, t + k); w[i][k] = p.w[c * DW_K + k]; }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+#pragma unroll
+      for (int k = 0; k < DW_K; ++k) a[i] = fmaf(w[i][k], x[i][k], a[i]);
+      v[i0 + i] = a[i];
+      if (tid + 256 * (i0 + i) < p.C) s += a[i];
     }
   }
   s = wave_sum(s);
@@ -902,7 +1157,7 @@ struct CvFinal {
   const float* w;  // (C, k)
   const float* b;  // (1)
   float* audio;
-  int C, k, T;
+  int C, k, T, nf;
   const int* ctr;
 };
 
@@ -916,7 +1171,7 @@ __global__ __launch_bounds__(256) void cv_final_kernel(const CvFinal p) {
   float* part = xs + n;
   float* ws = part + 256;
   for (int i = tid; i < p.C * p.k; i += 256) ws[i] = p.w[i];
-  const int f = *p.ctr - 1, base = ring_base(p.in, f);
+  const int f = *p.ctr - p.nf, base = ring_base(p.in, f);
   for (int i0 = tid; i0 < n; i0 += 256 * 12) {
     float v[12];
 #pragma unroll
@@ -984,11 +1239,25 @@ __global__ void cv_snake_tab_kernel(const float* alpha, const float* beta, float
 __global__ void cv_fill_kernel(float* p, size_t n, float v) {
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) p[i] = v;
 }
+// The history columns of every ring into the buffer that stands for it during a block (out = 0), and those behind the
+// block's last frame back into the ring.
+struct CvHist { Ring ring, buf; int C; };
+__global__ void cv_history_kernel(const CvHist* h, const int* ctr, int nf, int out) {
+  const CvHist r = h[blockIdx.y];
+  const int base = ring_base(r.ring, *ctr - (out ? 0 : nf)), at = out ? nf * r.ring.tstep : 0;
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < r.C * r.ring.pad; i += gridDim.x * blockDim.x) {
+    const int c = i / r.ring.pad, t = i - c * r.ring.pad;
+    float* ring = ring_ptr(r.ring, base, c, t);
+    float* buf = r.buf.p + (size_t)c * r.buf.rs + at + t;
+    if (out) *ring = *buf; else *buf = *ring;
+  }
+}
 __global__ void cv_set_int_kernel(int* p, int v0, int v1) { p[0] = v0; p[1] = v1; }
 
 // =================================== host side ===================================
 struct Step {
   int kind;  // 0 gemm, 1 attn, 2 dwln
+  int ln;    // dwln: the twin of its output
   CvGemm g;
   CvAttn a;
   CvDwLn d;
@@ -1001,10 +1270,14 @@ struct vui_codec {
   int64_t ws_bytes;
   float* state0;  // start of the zeroed-on-reset region (rings)
   size_t state_floats;
+  std::vector<Ring> twins;  // what stands for each ring and buffer while several frames are decoded at once
+  CvHist* hist;             // device: the rings and their twins
+  int n_hist = 0;
   int* ctr;  // [0] frames started since reset, [1] error flag
   int* cnt;  // arrival counters of split tiles
   size_t part_floats = 0, cnt_ints = 0;
   CvVq vq;
+  int vqx, qkv, att;  // twins of buffers that are not part of a product
   std::vector<Step> steps;
   CvFinal fin;
   // the persistent form of the one-column steps (0: the kernel sequence runs them)
@@ -1084,18 +1357,103 @@ struct Arena {
   }
 };
 
-static Ring mk_ring(Arena& ar, int C, int pad, int T, bool stream) {
-  Ring r;
-  r.rs = ipow2(pad + T);
-  r.mask = r.rs - 1;
-  r.pad = pad;
-  r.tstep = stream ? T : 0;
-  r.p = ar.take((size_t)C * r.rs);
-  return r;
-}
-static Ring no_ring() { Ring r; r.p = nullptr; r.rs = 1; r.mask = 0; r.pad = 0; r.tstep = 0; return r; }
+// Frames that one pass takes at most (vui_codec_decode_block).  At 32 the weights pass once per 32 frames (3 us of a
+// frame's 84) and a product's launch costs 0.15 us per frame; the buffers take 0.25 GB.
+#define CV_BLOCK 32
+static int block_frames(const vui_codec_config& k) { return k.max_seq < CV_BLOCK ? k.max_seq : CV_BLOCK; }
+
+// Rings and buffers of one frame, and of each its twin: a plain buffer of a whole block of frames with the history
+// columns in front.  A ring of 32 frames for both would need no copies of histories (two launches per block), but its
+// lines are never in the caches again when a single frame comes to them: 1 % of the streamed vocoder.
+struct RingMaker {
+  Arena& ar;
+  int frames;
+  std::vector<Ring> twins;
+  std::vector<size_t> floats;
+  std::vector<int> share;     // twins of one group >= 0 take turns in the same memory
+  std::vector<CvHist> hist;
+  Ring make(int C, int pad, int T, bool stream, int group = -1) {
+    Ring r;
+    r.rs = ipow2(pad + T);
+    r.mask = r.rs - 1;
+    r.pad = pad;
+    r.tstep = stream ? T : 0;
+    r.id = (int)twins.size();
+    r.p = ar.take((size_t)C * r.rs);
+    Ring t = r;
+    t.rs = (pad + T * frames + 3) & ~3;
+    t.mask = 0x7fffffff;
+    t.tstep = 0;
+    twins.push_back(t);
+    floats.push_back((size_t)C * t.rs + 256);  // a tile reads up to 256 columns behind the last channel's
+    share.push_back(group);
+    if (stream && pad) hist.push_back(CvHist{r, t, C});
+    return r;
+  }
+  void place() {  // once every ring is known
+    std::vector<size_t> most;
+    for (size_t i = 0; i < twins.size(); ++i)
+      if (share[i] >= 0) {
+        if ((int)most.size() <= share[i]) most.resize(share[i] + 1, 0);
+        if (floats[i] > most[share[i]]) most[share[i]] = floats[i];
+      }
+    std::vector<float*> common;
+    for (size_t n : most) common.push_back(ar.take(n));
+    for (size_t i = 0; i < twins.size(); ++i) twins[i].p = share[i] >= 0 ? common[share[i]] : ar.take(floats[i]);
+    for (CvHist& h : hist) h.buf = twins[h.ring.id];
+  }
+};
+static Ring no_ring() { Ring r; r.p = nullptr; r.rs = 1; r.mask = 0; r.pad = 0; r.tstep = 0; r.id = -1; return r; }
 
 static void grid_for(size_t n, dim3& g) { size_t b = (n + 255) / 256; g = dim3((unsigned)(b > 4096 ? 4096 : (b ? b : 1))); }
+
+// ---- launch shapes ----
+struct CvScratch { size_t part, cnt; };  // floats of partial sums, arrival counters
+// tiles of cv_wide_kernel, and what one unit of a tile costs against 128 x 128 (measured: 2.2 us)
+struct WideTile { int bm, bn; float unit; };
+static const WideTile kWide[] = {{128, 128, 1.0f}, {96, 256, 1.5f}, {64, 256, 1.0f}, {128, 64, 0.74f}, {32, 256, 0.74f}};
+
+// Chooses tile width, splits and kernel for g.T columns.
+static CvScratch cv_plan(CvGemm& g) {
+  const int U = g.taps * (g.Cin / 32), M = g.M, T = g.T;
+  if (g.nf > 1 && T >= CV_WIDE_T && M % 32 == 0 && g.in_mode == IN_PLAIN && g.epi != EPI_SILU_PAIR) {
+    // Tile and splits: the number of rounds over 256 CUs times a workgroup's work in units (about 4 more for what a
+    // tile costs besides its products), and for split tiles the second launch and its traffic.
+    size_t part = 0;
+    double cost = 0;
+    for (int i = 0; i < 5; ++i) {
+      const WideTile& w = kWide[i];
+      if (M % w.bm) continue;
+      const int cols = (T + w.bn - 1) / w.bn * w.bn, tiles = (M / w.bm) * (cols / w.bn);
+      for (int sp = 1; sp <= 16 && (sp == 1 || U / sp >= 4); ++sp) {
+        const double c = (double)((tiles * sp + 255) / 256) * ((U + sp - 1) / sp + 4) * w.unit + (sp > 1 ? 3 + 9e-7 * sp * M * T : 0);
+        if (cost && c >= cost) continue;
+        cost = c;
+        g.tt = 0; g.wide = i; g.splits = sp;
+        part = sp > 1 ? (size_t)sp * M * cols : 0;
+      }
+    }
+    return CvScratch{part, 0};
+  }
+  // Tile width: the one that pads the columns least, the wider one on a tie (a wave reuses its weight
+  // registers for every 16-column block).  Then workgroups share a tile's units until about 512 (one
+  // column block: the layer streams weights) or 200 (wider: the layer computes) are in flight, each wave
+  // keeping at least four units.  Measured per layer shape on MI355X.
+  auto tiles = [&](int tt) { return (M / 16) * ((T + 16 * tt - 1) / (16 * tt)); };
+  g.tt = 1;
+  for (int tt : {2, 4})
+    if (T > 8 * tt && tiles(tt) * tt <= tiles(g.tt) * g.tt) g.tt = tt;
+  int sp = 1;
+  if (U >= 64) {
+    const int target = g.tt == 1 ? 512 : 200;
+    sp = (2 * target + tiles(g.tt)) / (2 * tiles(g.tt));  // rounded
+    if (sp > U / 16) sp = U / 16;
+    if (sp > 8) sp = 8;
+    if (sp < 1) sp = 1;
+  }
+  g.splits = sp;
+  return CvScratch{(size_t)tiles(g.tt) * sp * g.tt * 256, (size_t)tiles(g.tt)};
+}
 
 // Lays out the workspace and (when tensors != nullptr) packs weights and records the launch plan.
 static int cv_build(vui_codec* cc, const vui_codec_config* c, const void* const* tensors, char* ws, hipStream_t st, int64_t* need,
@@ -1133,8 +1491,6 @@ static int cv_build(vui_codec* cc, const vui_codec_config* c, const void* const*
     return s;
   };
   int* ctr = (int*)ar.take(64);
-  // launch-shape targets: workgroups in flight for weight-streaming (one column block) and for wider tiles
-  const int wg_target = 512, wg_target2 = 200;
   // meeting place of split tiles: sized by a first pass (the sizes do not depend on the pointers)
   size_t part_floats = 0, cnt_ints = 0;
   float* part = ar.take(part_cap);
@@ -1144,27 +1500,15 @@ static int cv_build(vui_codec* cc, const vui_codec_config* c, const void* const*
     memset(&g, 0, sizeof(g));
     g.W = W; g.bias = bias; g.M = M; g.Cin = Cin; g.taps = taps; g.dil = dil; g.T = T; g.bias_div = 1;
     g.in = in; g.in_mode = IN_PLAIN; g.eps = 1e-6f; g.epi = EPI_NONE;
-    g.res = no_ring(); g.out_raw = no_ring(); g.out_act = no_ring(); g.ctr = ctr;
-    // Tile width: the one that pads the columns least, the wider one on a tie (a wave reuses its weight
-    // registers for every 16-column block).  Then workgroups share a tile's units until about 512 (one
-    // column block: the layer streams weights) or 200 (wider: the layer computes) are in flight, each wave
-    // keeping at least four units.  Measured per layer shape on MI355X.
-    const int U = taps * (Cin / 32);
-    auto tiles = [&](int tt) { return (M / 16) * ((T + 16 * tt - 1) / (16 * tt)); };
-    g.tt = 1;
-    for (int tt : {2, 4})
-      if (T > 8 * tt && tiles(tt) * tt <= tiles(g.tt) * g.tt) g.tt = tt;
-    int sp = 1;
-    if (U >= 64) {
-      const int target = g.tt == 1 ? wg_target : wg_target2;
-      sp = (2 * target + tiles(g.tt)) / (2 * tiles(g.tt));  // rounded
-      if (sp > U / 16) sp = U / 16;
-      if (sp > 8) sp = 8;
-      if (sp < 1) sp = 1;
+    g.res = no_ring(); g.out_raw = no_ring(); g.out_act = no_ring(); g.ctr = ctr; g.nf = 1;
+    g.part = part; g.cnt = cnt;
+    for (int n = block_frames(*c); n >= 1; --n) {  // the frame's own plan is made last and stays
+      g.T = n * T;
+      g.nf = n;
+      const CvScratch need = cv_plan(g);
+      if (need.part > part_floats) part_floats = need.part;
+      if (need.cnt > cnt_ints) cnt_ints = need.cnt;
     }
-    g.splits = sp; g.part = part; g.cnt = cnt;
-    if ((size_t)tiles(g.tt) * sp * g.tt * 256 > part_floats) part_floats = (size_t)tiles(g.tt) * sp * g.tt * 256;
-    if ((size_t)tiles(g.tt) > cnt_ints) cnt_ints = tiles(g.tt);
     return g;
   };
   auto push_gemm = [&](const CvGemm& g) { if (real) { Step s; memset((void*)&s, 0, sizeof(s)); s.kind = 0; s.g = g; cc->steps.push_back(s); } };
@@ -1184,33 +1528,34 @@ static int cv_build(vui_codec* cc, const vui_codec_config* c, const void* const*
     }
   }
   // ---- state region (zeroed by reset) starts here: all rings ----
+  RingMaker rings{ar, block_frames(*c)};
   const size_t state_begin = ar.off;
-  Ring pre_in = mk_ring(ar, c->vq_dim, 2, 1, true);
+  Ring pre_in = rings.make(c->vq_dim, 2, 1, true);
   std::vector<Ring> dw_in, tc_in, ru_in;
   int T = 1;
-  for (int i = 0; i < c->n_up; ++i) { T *= c->up_ratios[i]; dw_in.push_back(mk_ring(ar, L, 6, T, true)); }
+  for (int i = 0; i < c->n_up; ++i) { T *= c->up_ratios[i]; dw_in.push_back(rings.make(L, 6, T, true)); }
   const int T_lat = T;
-  Ring dec0_in = mk_ring(ar, L, 6, T_lat, true);
+  Ring dec0_in = rings.make(L, 6, T_lat, true);
   {
     int dim = c->decoder_dim, t = T_lat;
     for (int i = 0; i < c->n_rates; ++i) {
-      tc_in.push_back(mk_ring(ar, dim, 1, t, true));
+      tc_in.push_back(rings.make(dim, 1, t, true));
       t *= c->rates[i];
       dim /= 2;
-      for (int j = 0; j < 3; ++j) { const int dil = j == 0 ? 1 : (j == 1 ? 3 : 9); ru_in.push_back(mk_ring(ar, dim, 6 * dil, t, true)); }
+      for (int j = 0; j < 3; ++j) { const int dil = j == 0 ? 1 : (j == 1 ? 3 : 9); ru_in.push_back(rings.make(dim, 6 * dil, t, true)); }
     }
   }
   int fin_dim = c->decoder_dim >> c->n_rates;
   const int hop = vui_codec_hop(c);
-  Ring fin_in = mk_ring(ar, fin_dim, 6, hop, true);
+  Ring fin_in = rings.make(fin_dim, 6, hop, true);
   const size_t state_end = ar.off;
   // ---- plain activation buffers ----
-  Ring vqx = mk_ring(ar, 2 * cd, 0, 1, false);
-  Ring pre_out = mk_ring(ar, L, 0, 1, false);
-  Ring xres = mk_ring(ar, D, 0, 1, false);
-  Ring qkv = mk_ring(ar, 3 * A, 0, 1, false);
-  Ring att = mk_ring(ar, A, 0, 1, false);
-  Ring gu = mk_ring(ar, c->mlp_dim, 0, 1, false);
+  Ring vqx = rings.make(2 * cd, 0, 1, false);
+  Ring pre_out = rings.make(L, 0, 1, false);
+  Ring xres = rings.make(D, 0, 1, false);
+  Ring qkv = rings.make(3 * A, 0, 1, false);
+  Ring att = rings.make(A, 0, 1, false);
+  Ring gu = rings.make(c->mlp_dim, 0, 1, false);
   float* kc = ar.take((size_t)c->n_layers * A * c->max_seq);
   float* vc = ar.take((size_t)c->n_layers * A * c->max_seq);
   float* inv_freq = ar.take(c->head_dim / 2);
@@ -1270,6 +1615,7 @@ static int cv_build(vui_codec* cc, const vui_codec_config* c, const void* const*
       Step s; memset((void*)&s, 0, sizeof(s)); s.kind = 1;
       s.a.qkv = qkv.p; s.a.kc = kc + (size_t)l * A * c->max_seq; s.a.vc = vc + (size_t)l * A * c->max_seq;
       s.a.out = att.p; s.a.inv_freq = inv_freq; s.a.H = c->n_heads; s.a.hd = c->head_dim; s.a.max_seq = c->max_seq; s.a.ctr = ctr;
+      s.a.rs = qkv.rs; s.a.rs_out = att.rs; s.a.nf = 1;
       cc->steps.push_back(s);
     }
     g = gemm(Wo, nullptr, D, A, 1, 1, 1, att);
@@ -1285,7 +1631,7 @@ static int cv_build(vui_codec* cc, const vui_codec_config* c, const void* const*
     push_gemm(g);
     tl[l].msc = g.scale;
   }
-  Ring cur = mk_ring(ar, L, 0, 1, false);  // output of the transformer = input of the first upsample stage
+  Ring cur = rings.make(L, 0, 1, false);  // output of the transformer = input of the first upsample stage
   {
     const float* nw = next(); const float* w = next(); const float* b = next();
     float* Wout = ar.take((size_t)L * D);
@@ -1309,17 +1655,17 @@ static int cv_build(vui_codec* cc, const vui_codec_config* c, const void* const*
     push_gemm(g);
     if (i == 0) { tk.Wt0 = g.W; tk.bt0 = g.bias; tk.r0 = r; tk.out = dw_in[0]; if (real) trunk_steps = (int)cc->steps.size(); }
     const float* dww = next(); const float* dwb = next(); const float* lnw = next(); const float* lnb = next();
-    Ring ln = mk_ring(ar, L, 0, T, false);
+    Ring ln = rings.make(L, 0, T, false);
     float* dwwp = vec(dww, L * 7); float* dwbp = vec(dwb, L); float* lnwp = vec(lnw, L); float* lnbp = vec(lnb, L);
     if (real) {
       Step s; memset((void*)&s, 0, sizeof(s)); s.kind = 2;
       s.d.in = dw_in[i]; s.d.w = dwwp; s.d.b = dwbp; s.d.lnw = lnwp; s.d.lnb = lnbp;
-      s.d.out = ln.p; s.d.rs_out = ln.rs; s.d.C = L; s.d.k = 7; s.d.eps = 1e-6f; s.d.ctr = ctr;
+      s.ln = ln.id; s.d.out = ln.p; s.d.rs_out = ln.rs; s.d.C = L; s.d.eps = 1e-6f; s.d.ctr = ctr; s.d.nf = 1;
       s.g.T = T;  // grid
       cc->steps.push_back(s);
     }
     const float* w1 = next(); const float* b1 = next(); const float* w2 = next(); const float* b2 = next(); const float* gam = next();
-    Ring pw = mk_ring(ar, 4 * L, 0, T, false);
+    Ring pw = rings.make(4 * L, 0, T, false);
     float* W1 = ar.take((size_t)4 * L * L);
     pack_copy(w1, W1, 4 * L, L, L, 0);
     g = gemm(W1, vec(b1, 4 * L), 4 * L, L, 1, 1, T, ln);
@@ -1329,7 +1675,7 @@ static int cv_build(vui_codec* cc, const vui_codec_config* c, const void* const*
     pack_copy(w2, W2, L, 4 * L, 4 * L, 0);
     g = gemm(W2, vec(b2, L), L, 4 * L, 1, 1, T, pw);
     g.epi = EPI_SCALE_RES; g.scale = vec(gam, L); g.res = dw_in[i];
-    if (i + 1 < c->n_up) { cur = mk_ring(ar, L, 0, T, false); g.out_raw = cur; } else g.out_raw = dec0_in;
+    if (i + 1 < c->n_up) { cur = rings.make(L, 0, T, false); g.out_raw = cur; } else g.out_raw = dec0_in;
     push_gemm(g);
   }
   // ---- BigVGAN-style decoder ----
@@ -1348,8 +1694,8 @@ static int cv_build(vui_codec* cc, const vui_codec_config* c, const void* const*
       const float* tw = next(); const float* tb = next();
       CvGemm tg = gemm(pack_tconv(tw, dim, out, rate, 2), vec(tb, out), out * rate, dim, 2, 1, tin, tc_in[i]);
       tg.bias_div = rate; tg.tc_stride = rate;
-      Ring R = mk_ring(ar, out, 0, t, false);
-      Ring hbuf = mk_ring(ar, out, 0, t, false);
+      Ring R = rings.make(out, 0, t, false, 0);  // a stage's own: the next stage's take their place
+      Ring hbuf = rings.make(out, 0, t, false, 1);
       tg.out_raw = R;
       pending = tg;
       for (int j = 0; j < 3; ++j) {
@@ -1379,9 +1725,11 @@ static int cv_build(vui_codec* cc, const vui_codec_config* c, const void* const*
     const float* fw = next(); const float* fb = next();
     float* fwp = vec(fw, dim * 7); float* fbp = vec(fb, 1);
     if (real) {
-      cc->fin.in = fin_in; cc->fin.w = fwp; cc->fin.b = fbp; cc->fin.audio = nullptr; cc->fin.C = dim; cc->fin.k = 7; cc->fin.T = hop; cc->fin.ctr = ctr;
+      cc->fin.in = fin_in; cc->fin.w = fwp; cc->fin.b = fbp; cc->fin.audio = nullptr; cc->fin.C = dim; cc->fin.k = 7; cc->fin.T = hop; cc->fin.ctr = ctr; cc->fin.nf = 1;
     }
   }
+  rings.place();
+  CvHist* hist_dev = (CvHist*)ar.take((sizeof(CvHist) * rings.hist.size() + 3) / 4);
   if (need) *need = (int64_t)ar.off;
   if (part_need) *part_need = part_floats;
   if (cnt_need) *cnt_need = cnt_ints;
@@ -1397,15 +1745,20 @@ static int cv_build(vui_codec* cc, const vui_codec_config* c, const void* const*
       hipLaunchKernelGGL(cv_fill_kernel, g, dim3(256), 0, st, (float*)ll, ll_words * 2, 0.0f);
       hipLaunchKernelGGL(cv_fill_kernel, dim3(1), dim3(64), 0, st, (float*)tctl, (size_t)16, 0.0f);
     }
-    HIP_TRY(hipStreamSynchronize(st));  // tl goes out of scope
+    HIP_TRY(hipMemcpyAsync(hist_dev, rings.hist.data(), sizeof(CvHist) * rings.hist.size(), hipMemcpyHostToDevice, st));
+    HIP_TRY(hipStreamSynchronize(st));  // tl and rings go out of scope
     cc->trunk = tk;
     cc->trunk_steps = trunk_steps;
     if (part_floats > part_cap || cnt_ints > cnt_cap) { vui_set_error("codec: internal scratch sizing"); return VUI_EINVAL; }
     cc->ctr = ctr; cc->cnt = cnt; cc->cnt_ints = cnt_cap;
     cc->state0 = (float*)(ws + state_begin);
     cc->state_floats = (state_end - state_begin) / 4;
+    cc->hist = hist_dev;
+    cc->n_hist = (int)rings.hist.size();
+    cc->twins = rings.twins;
+    cc->vqx = vqx.id; cc->qkv = qkv.id; cc->att = att.id;
     cc->vq.codes = nullptr; cc->vq.n_q = 0; cc->vq.n_sem = c->n_semantic; cc->vq.CS = CS; cc->vq.cd = cd;
-    cc->vq.embed = embed; cc->vq.x = vqx.p; cc->vq.ctr = ctr; cc->vq.err = ctr + 1; cc->vq.max_seq = c->max_seq;
+    cc->vq.embed = embed; cc->vq.x = vqx.p; cc->vq.rs = vqx.rs; cc->vq.nf = 1; cc->vq.ctr = ctr; cc->vq.err = ctr + 1; cc->vq.max_seq = c->max_seq;
     if (ti != vui_codec_n_tensors(c)) { vui_set_error("codec: internal tensor count %d != %d", ti, vui_codec_n_tensors(c)); return VUI_EINVAL; }
     HIP_TRY(hipGetLastError());
   }
@@ -1498,6 +1851,19 @@ int vui_codec_persistent(vui_codec* c, int enable) {
 
 static int launch_cv_gemm(const CvGemm& g, bool w_nt, hipStream_t st) {
   if (g.M % 16 || g.Cin % 32 || g.T < 1) { vui_set_error("codec gemm: bad shape M=%d Cin=%d T=%d", g.M, g.Cin, g.T); return VUI_EINVAL; }
+  if (g.tt == 0) {
+    const WideTile& w = kWide[g.wide];
+    const dim3 grid(g.M / w.bm, (g.T + w.bn - 1) / w.bn, g.splits);
+#define CV_WIDE(...) hipLaunchKernelGGL((cv_wide_kernel<__VA_ARGS__>), grid, dim3(512), 0, st, g)
+    if (g.wide == 0) CV_WIDE(2, 1, 2, 4);
+    else if (g.wide == 1) CV_WIDE(3, 1, 1, 8);
+    else if (g.wide == 2) CV_WIDE(2, 1, 1, 8);
+    else if (g.wide == 3) CV_WIDE(1, 1, 4, 2);
+    else CV_WIDE(1, 1, 1, 8);
+#undef CV_WIDE
+    if (g.splits > 1) hipLaunchKernelGGL(cv_finish_kernel, dim3((g.T + 63) / 64, g.M / 32), dim3(256), 0, st, g, (int)grid.y * w.bn);
+    return VUI_OK;
+  }
   const dim3 grid(g.M / 16, (g.T + 16 * g.tt - 1) / (16 * g.tt), g.splits);
   const dim3 block(64 * CV_NW);
   // units a wave of one part works through; one single-buffered round holds 8 / 6 / 3 of them
@@ -1552,6 +1918,51 @@ int vui_codec_decode_frame(vui_codec* c, const int64_t* codes, int32_t n_q, floa
   }
   CvFinal fin = c->fin;
   fin.audio = audio_out;
+  hipLaunchKernelGGL(cv_final_kernel, dim3((fin.T + FIN_TW - 1) / FIN_TW), dim3(256), (size_t)(fin.C * (FIN_TW + fin.k - 1) + 256 + fin.C * fin.k) * 4, st, fin);
+  HIP_TRY(hipGetLastError());
+  return VUI_OK;
+}
+
+int32_t vui_codec_block_frames(const vui_codec* c) {
+  if (!c) { vui_set_error("NULL codec"); return VUI_EINVAL; }
+  return block_frames(c->cfg);
+}
+
+int vui_codec_decode_block(vui_codec* c, const int64_t* codes, int32_t n_frames, int32_t n_q, float* audio_out, vui_stream_t stream) {
+  if (!c) { vui_set_error("NULL codec"); return VUI_EINVAL; }
+  if (!codes || !audio_out) { vui_set_error("NULL argument"); return VUI_EINVAL; }
+  if (n_q < 1 || n_q > c->cfg.n_codebooks) { vui_set_error("n_q=%d outside [1,%d]", n_q, c->cfg.n_codebooks); return VUI_EINVAL; }
+  if (n_frames < 1 || n_frames > block_frames(c->cfg)) { vui_set_error("codec: %d frames outside [1, %d]", n_frames, block_frames(c->cfg)); return VUI_EINVAL; }
+  if (n_frames == 1) return vui_codec_decode_frame(c, codes, n_q, audio_out, stream);
+  hipStream_t st = (hipStream_t)stream;
+  auto twin = [&](const Ring& r) { return r.id < 0 ? r : c->twins[r.id]; };
+  CvVq vq = c->vq;
+  vq.codes = codes; vq.n_q = n_q; vq.nf = n_frames; vq.x = c->twins[c->vqx].p; vq.rs = c->twins[c->vqx].rs;
+  hipLaunchKernelGGL(cv_vq_kernel, dim3(n_frames), dim3(256), 0, st, vq);
+  hipLaunchKernelGGL(cv_history_kernel, dim3(16, c->n_hist), dim3(256), 0, st, c->hist, c->ctr, n_frames, 0);
+  for (const Step& s0 : c->steps) {
+    Step s = s0;
+    if (s.kind == 0) {
+      s.g.T *= n_frames; s.g.nf = n_frames;
+      s.g.in = twin(s.g.in); s.g.res = twin(s.g.res); s.g.out_raw = twin(s.g.out_raw); s.g.out_act = twin(s.g.out_act);
+      cv_plan(s.g);
+      int rc = launch_cv_gemm(s.g, c->w_nt != 0, st);
+      if (rc) return rc;
+    } else if (s.kind == 1) {
+      s.a.nf = n_frames;
+      s.a.qkv = c->twins[c->qkv].p; s.a.rs = c->twins[c->qkv].rs; s.a.out = c->twins[c->att].p; s.a.rs_out = c->twins[c->att].rs;
+      const size_t lds = (size_t)(s.a.hd + s.a.max_seq + 4 * s.a.hd + 8) * 4;
+      hipLaunchKernelGGL(cv_append_kernel, dim3(s.a.H, n_frames), dim3(64), 0, st, s.a);
+      hipLaunchKernelGGL(cv_attn_kernel, dim3(s.a.H, n_frames), dim3(256), lds, st, s.a);
+    } else {
+      const Ring ln = c->twins[s.ln];
+      s.d.nf = n_frames; s.d.in = twin(s.d.in); s.d.out = ln.p; s.d.rs_out = ln.rs;
+      hipLaunchKernelGGL(cv_dwln_kernel, dim3(s.g.T * n_frames), dim3(256), 0, st, s.d);
+    }
+  }
+  hipLaunchKernelGGL(cv_history_kernel, dim3(16, c->n_hist), dim3(256), 0, st, c->hist, c->ctr, n_frames, 1);
+  CvFinal fin = c->fin;
+  fin.audio = audio_out; fin.nf = n_frames; fin.T *= n_frames; fin.in = twin(fin.in);
   hipLaunchKernelGGL(cv_final_kernel, dim3((fin.T + FIN_TW - 1) / FIN_TW), dim3(256), (size_t)(fin.C * (FIN_TW + fin.k - 1) + 256 + fin.C * fin.k) * 4, st, fin);
   HIP_TRY(hipGetLastError());
   return VUI_OK;
