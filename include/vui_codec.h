@@ -1,6 +1,6 @@
 /*
- * vui_codec.h - C ABI of the MI355X-native streaming vocoder frame step (codes of one codec frame ->
- * 1920 audio samples), the decoder half of the reference's codec.
+ * vui_codec.h - C ABI of the MI355X-native streaming vocoder (codes of one codec frame, or of a block of
+ * frames, -> 1920 audio samples each), the decoder half of the reference's codec.
  *
  * Same conventions as vui_amd.h: 0 on success, a negative VUI_E* code on failure with the message
  * in vui_last_error(); every pointer is a device pointer unless stated; all work is asynchronous
@@ -53,8 +53,8 @@ int32_t vui_codec_hop(const vui_codec_config* cfg);
  * decoder.*; qwen_codec.py:1087-1125). */
 int32_t vui_codec_n_tensors(const vui_codec_config* cfg);
 
-/* Bytes of workspace: repacked weights (one copy, tap-major), activation rings, the
- * pre-transformer cache, tables and counters. */
+/* Bytes of workspace: repacked weights (one copy, tap-major), activation rings, the buffers of a block of
+ * frames, the pre-transformer cache, tables and counters. */
 int64_t vui_codec_workspace_bytes(const vui_codec_config* cfg);
 
 /* Builds a decoder: repacks the fp32 tensors (reference layouts: Conv1d (out, in, k),

@@ -18,6 +18,10 @@
 // scattered to column t*stride + r.  A workgroup owns 16 output rows x 16*TT columns; its waves split
 // the (tap, 32-channel) units, multiply on v_mfma_f32_16x16x4_f32 with both operands read straight from
 // global memory / L2 one step ahead, and add their parts through LDS in a fixed order.
+//
+// Several frames at once (vui_codec_decode_block: offline calls, the seeding of a stream): the same steps over
+// frames x columns, on buffers that hold a whole block with the histories in front; wide products run in
+// cv_wide_kernel.  93 frames: 56.6 ms one after the other, 7.9 ms in blocks of 32 (MI355X).
 #include "common.h"
 #include "internal.h"
 #include "../../include/vui_codec.h"
