@@ -465,3 +465,19 @@ def test_generation_with_a_large_vocabulary():
     eng = U.engine(cfg, sd, max_rows=2, max_seq=40)
     reqs = [TokenRequest(U.tokens(n, 9001, n), max_new=5) for n in (3, 20, 9)]
     assert eng.generate(reqs) == [O.greedy(cfg, sd, r.tokens, 5) for r in reqs]
+
+
+@pytest.mark.parametrize("T", [129, 255, 640, 1024, 1100])
+def test_large_products_of_a_prompt(T):
+    """Products whose rows and features fill large tiles (64 x 64 ... 128 x 192, by T), sizes that end inside them, against
+    the same tokens in portions of 100, which take the small tiles.  Both are bf16 evaluations (0.5 % each): 4 % per position."""
+    from vui_amd.synthetic import token_lm_config, token_lm_state_dict
+
+    cfg = token_lm_config(1000, 7, 5000, 120, 60, 72, 500, 3, vocab=301)
+    eng = U.engine(cfg, token_lm_state_dict(cfg, 3, "cuda"), BF16, max_seq=1152)
+    toks = torch.tensor(U.tokens(T, 301, T))
+    with eng.new_row() as row:
+        whole = row.extend(toks, range(T)).clone()
+        row.reset()
+        parts = torch.cat([row.extend(toks[i:i + 100], range(len(toks[i:i + 100]))).clone() for i in range(0, T, 100)])
+    assert U.err(whole, parts) < 0.04

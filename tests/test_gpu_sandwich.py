@@ -545,3 +545,20 @@ def test_lengths_of_several_thousand():
         with eng.new_row() as row:
             outs = [row.extend(toks[:2100], [2099]).clone()] + [row.extend([t], [0]).clone() for t in toks[2100:]]
             assert U.err(torch.cat(outs), ref) < 2 * TOL[dt]
+
+
+@pytest.mark.parametrize("T", [129, 255, 640, 1024, 1100])
+def test_large_products_of_a_prompt(T):
+    """As in test_gpu_lm: dense layers, whose projections, activations and outputs fill large tiles, against portions of 100."""
+    from vui_amd.synthetic import sandwich_lm_config, token_lm_state_dict
+
+    cfg = sandwich_lm_config(1000, 8, 2, 120, 6000, 8, 2, 2, vocab=301)
+    for layer in cfg["layers"]:
+        layer["mlp"] = {"kind": "dense", "ff": 6000}
+    eng = U.engine(cfg, token_lm_state_dict(cfg, 3, "cuda"), torch.bfloat16, max_seq=1152)
+    toks = torch.tensor(U.tokens(T, 301, T))
+    with eng.new_row() as row:
+        whole = row.extend(toks, range(T)).clone()
+        row.reset()
+        parts = torch.cat([row.extend(toks[i:i + 100], range(len(toks[i:i + 100]))).clone() for i in range(0, T, 100)])
+    assert U.err(whole, parts) < TOL[torch.bfloat16]

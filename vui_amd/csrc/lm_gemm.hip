@@ -9,13 +9,27 @@
 #include "lm.h"
 #include "tile.h"
 
-__device__ __forceinline__ float lm_sigmoid(float v) { return 1.0f / (1.0f + expf(-v)); }
+// fp32 contexts: the library's exponential and division.  bf16 contexts: a prompt's epilogues evaluate ten million of
+// these per layer and were bound by their instructions, so the exponential is v_exp_f32 with the rounding of its argument
+// made good, the division v_rcp_f32 with a Newton step: half the instructions, relative error against 64 bits 4.1e-8
+// root mean square where the library's form has 3.9e-8 (|v| <= 20), and the result is rounded to 16 bits.
+template <typename T> __device__ __forceinline__ float lm_sigmoid(float v) {
+  if constexpr (sizeof(T) == 4) {
+    return 1.0f / (1.0f + expf(-v));
+  } else {
+    const float x = fminf(-v, 87.f), h = x * 1.4426950408889634f;
+    const float lo = fmaf(x, 1.4426950408889634f, -h) + x * 1.925963033500011e-8f;
+    const float ex = __builtin_amdgcn_exp2f(h), d = 1.0f + fmaf(ex, lo * 0.6931471805599453f, ex);
+    const float r = __builtin_amdgcn_rcpf(d);
+    return v < -3e38f ? 0.f : v != v ? v : v > 3e38f ? 1.f : fmaf(fmaf(-d, r, 1.0f), r, r);
+  }
+}
 
 // gated feed-forward with clamped branches, two features from interleaved (gate, up) pairs
-__device__ __forceinline__ float lm_ff(float g, float u, float limit) {
+template <typename T> __device__ __forceinline__ float lm_ff(float g, float u, float limit) {
   g = fminf(g, limit);
   u = fminf(fmaxf(u, -limit), limit);
-  return g * lm_sigmoid(1.702f * g) * (u + 1.0f);
+  return g * lm_sigmoid<T>(1.702f * g) * (u + 1.0f);
 }
 
 // rotates two pairs held as (u0, v0, u1, v1); pair indices i, i + 1; pairs at or beyond n pass
@@ -36,6 +50,139 @@ __device__ __forceinline__ float lm_act(float z, int kind, float pos, float neg)
   if (kind == VUI_LM_ACT_RELU2) { z = fmaxf(z, 0.f); return z * z; }
   const float m = fminf(z, 0.f);
   return (z > 0.f ? pos * z * z : neg * (expm1f(m) - m)) + 0.5f * z;
+}
+
+// What a unit's epilogue reads besides the sums, requested ahead of the operands (few rows).
+struct LmPre {
+  int slot, pos;
+  float4 a, b, c;
+};
+
+// One unit of 16 rows x 16 features: a lane holds features n ... n + 3 of row m (LM_EXPAND_V: rows m ... m + 3 of feature
+// n).  mix: the unit is the update gate of a recurrence, xv and gv the candidate and the output gate beside it.
+template <typename T, int EPI, bool PRE>
+__device__ __forceinline__ void lm_unit(const LmGemm& p, const int m, const int nb, const int n, const int l16, const int kg,
+                                        const bool live, const bool mix, float (&v)[4], const float (&xv)[4], const float (&gv)[4],
+                                        const LmPre& e) {
+  constexpr bool GRU = EPI == LM_IN_GRU_STEP || EPI == LM_IN_GRU_SEQ;
+  constexpr bool LOGITS = EPI == LM_LOGITS || EPI == LM_HEAD;
+  if (GRU && mix) {
+    const int ch = (nb / 3) * 16 + 4 * kg;  // blocks come in threes: update gate, candidate, output gate
+    if (!live) return;
+    const float4 b0 = PRE ? e.b : *reinterpret_cast<const float4*>(p.bz + ch), b1 = PRE ? e.c : *reinterpret_cast<const float4*>(p.bx + ch);
+    const float zb[4] = {b0.x, b0.y, b0.z, b0.w}, xb[4] = {b1.x, b1.y, b1.z, b1.w};
+    float keep[4], in[4], sg[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float zz = v[r] + zb[r], uu = xv[r] + xb[r];
+      const float z = lm_sigmoid<T>(zz);
+      keep[r] = lm_sigmoid<T>(-zz);
+      in[r] = z * (uu >= 0.f ? uu + 0.5f : lm_sigmoid<T>(uu));
+      sg[r] = gv[r] * lm_sigmoid<T>(gv[r]);
+    }
+    if (EPI == LM_IN_GRU_STEP) {
+      float4* sp = reinterpret_cast<float4*>(p.state + (size_t)e.slot * p.d.gru16 + ch);
+      const float4 old = e.pos > 0 ? e.a : make_float4(0.f, 0.f, 0.f, 0.f);
+      const float4 nw = make_float4(fmaf(keep[0], old.x, in[0]), fmaf(keep[1], old.y, in[1]), fmaf(keep[2], old.z, in[2]),
+                                    fmaf(keep[3], old.w, in[3]));
+      *sp = nw;
+      const float o[4] = {nw.x * sg[0], nw.y * sg[1], nw.z * sg[2], nw.w * sg[3]};
+      Tl<T>::st4((T*)p.act + tl_off<T>(m, ch, p.d.out_k), o);
+    } else {
+      float4* up = reinterpret_cast<float4*>(p.upd + (size_t)m * p.d.gru16 + ch);
+      up[0] = make_float4(keep[0], in[0], keep[1], in[1]);
+      up[1] = make_float4(keep[2], in[2], keep[3], in[3]);
+      Tl<T>::st4((T*)p.sg + (size_t)m * p.d.gru16 + ch, sg);
+    }
+    return;
+  }
+  if (EPI == LM_IN_ATTN || GRU) {
+    if (!live) return;
+    if (nb >= p.mix_blocks) {  // (gate, up) pairs
+      const int f = (n - p.mix_blocks * 16) >> 1;
+      Tl<T>::st2((T*)p.act + tl_off<T>(m, p.d.ff_off + f, p.d.out_k), lm_ff<T>(v[0], v[1], p.limit), lm_ff<T>(v[2], v[3], p.limit));
+      return;
+    }
+    if (EPI == LM_IN_ATTN) {
+      if (nb < p.b_qr) {
+        const int dq = p.d.dim16 >> 4, h = nb / dq, o = (nb - h * dq) * 16 + 4 * kg;
+        Tl<T>::st4((T*)p.qu + h * p.qu_z + tl_off<T>(m, o, p.d.dim64), v);
+      } else if (nb < p.b_c) {
+        const int dr = p.d.rot16 >> 4, b = nb - p.b_qr, h = b / dr, o = (b - h * dr) * 16 + 4 * kg;
+        const int slot = PRE ? e.slot : lm_slot(p.rows, m), pos = min(max(PRE ? e.pos : lm_pos(p.rows, m, slot), 0), p.rows.S - 1);
+        lm_rotate2(v, p.rope, pos, p.rot_pairs, o >> 1);
+        Tl<T>::st4((T*)p.qr + h * p.qr_z + tl_off<T, 32>(m, o, p.d.rot32), v);
+      } else if (nb < p.b_kr) {
+        const int o = (nb - p.b_c) * 16 + 4 * kg;
+        *reinterpret_cast<float4*>(p.craw + (size_t)m * p.d.rank16 + o) = make_float4(v[0], v[1], v[2], v[3]);
+      } else if (nb < p.b_g) {
+        const int o = (nb - p.b_kr) * 16 + 4 * kg;
+        const int slot = PRE ? e.slot : lm_slot(p.rows, m), pos = PRE ? e.pos : lm_pos(p.rows, m, slot);
+        if (pos >= 0 && pos < p.rows.S) {
+          lm_rotate2(v, p.rope, pos, p.rot_pairs, o >> 1);
+          Tl<T>::st4((T*)p.kr_cache + (size_t)slot * p.d.s64 * p.d.rot32 + tl_off<T, 32>(pos, o, p.d.rot32), v);
+        }
+      } else {
+        const int o = (nb - p.b_g) * 16 + 4 * kg;
+        if (o < p.d.heads16)  // the blocks behind the gates only fill the last tile of the mixer part
+          *reinterpret_cast<float4*>(p.gate + (size_t)m * p.d.heads16 + o) =
+              make_float4(lm_sigmoid<T>(v[0]), lm_sigmoid<T>(v[1]), lm_sigmoid<T>(v[2]), lm_sigmoid<T>(v[3]));
+      }
+    }
+    return;
+  }
+  if (EPI == LM_OUT) {
+    float sq = 0.f;
+    if (live) {
+      float4* xp = reinterpret_cast<float4*>(p.x + (size_t)m * p.d.w64 + n);
+      const float4 old = PRE ? e.a : *xp;
+      v[0] += old.x; v[1] += old.y; v[2] += old.z; v[3] += old.w;
+      *xp = make_float4(v[0], v[1], v[2], v[3]);
+      Tl<T>::st4((T*)p.xt + tl_off<T>(m, n, p.d.w64), v);
+      sq = (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
+      if (p.layer_out)
+        for (int r = 0; r < 4; ++r) if (n + r < p.width) p.layer_out[(size_t)m * p.width + n + r] = v[r];
+    }
+    sq = rows_sum(sq);  // the 16 columns of this row's block
+    if (live && kg == 0 && nb < p.np) p.ssq_out[(size_t)m * p.np + nb] = sq;
+    return;
+  }
+  if (LOGITS) {
+    if (live)
+      for (int r = 0; r < 4; ++r) if (n + r < p.vocab) p.logits[(size_t)m * p.vocab + n + r] = v[r];
+    return;
+  }
+  if (EPI == LM_PROJ || EPI == LM_PLAIN || EPI == LM_MOE_DOWN) {
+    const int r = EPI == LM_MOE_DOWN ? p.ent[m] : m;
+    if (!live || r < 0) return;
+    if (EPI != LM_MOE_DOWN && p.bias) {
+      const float4 b = *reinterpret_cast<const float4*>(p.bias + n);
+      v[0] += b.x; v[1] += b.y; v[2] += b.z; v[3] += b.w;
+    }
+    if (EPI == LM_PROJ) Tl<T>::st4((T*)p.out + (size_t)r * p.ldo + n, v);
+    else Tl<float>::st4((float*)p.out + (size_t)r * p.ldo + n, v);
+    return;
+  }
+  if (EPI == LM_ACT || EPI == LM_MOE_UP) {
+    if (!live) return;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = lm_act(v[r], p.act_kind, p.act_pos, p.act_neg);
+    Tl<T>::st4((T*)p.act + tl_off<T>(m, n, p.act_k), v);
+    return;
+  }
+  if (EPI == LM_EXPAND_K) {
+    if (live) Tl<T>::st4((T*)p.kv_out + blockIdx.z * p.kv_z + tl_off<T>(m, n, p.d.dim64), v);
+    return;
+  }
+  if (EPI == LM_EXPAND_V) {
+    // blocks of 16 value dims x 32 keys; a lane of the attention kernel reads the keys 4 kg .. + 3 of both halves
+    if (live) {
+      T* dst = (T*)p.kv_out + blockIdx.z * p.kv_z + ((size_t)nb * (p.d.s64 >> 5) + (m >> 5)) * 512 +
+               (l16 + 16 * ((m & 15) >> 2)) * 8 + 4 * ((m & 31) >> 4);
+      Tl<T>::st4(dst, v);
+    }
+    return;
+  }
 }
 
 template <typename T, int MB, int NB, int WAVES, int EPI>
@@ -100,18 +247,19 @@ __global__ __launch_bounds__(64 * WAVES) void lm_gemm_kernel(const LmGemm p) {
   }
   constexpr bool PRE = MB == 1 && (EPI == LM_IN_ATTN || EPI == LM_IN_GRU_STEP || EPI == LM_OUT);
   const int pm = min(m0 + l16, p.M - 1), pb = min(nb0 + min(wave, NB - 1), NBL - 1);  // row and block of unit `wave`
-  int e_slot = 0, e_pos = 0;
-  float4 e_a = make_float4(0.f, 0.f, 0.f, 0.f), e_b = e_a, e_c = e_a;
+  LmPre e;
+  e.slot = e.pos = 0;
+  e.a = e.b = e.c = make_float4(0.f, 0.f, 0.f, 0.f);
   if (PRE && EPI != LM_OUT) {
-    e_slot = lm_slot(p.rows, pm);
-    e_pos = lm_pos(p.rows, pm, e_slot);
+    e.slot = lm_slot(p.rows, pm);
+    e.pos = lm_pos(p.rows, pm, e.slot);
   }
-  if (PRE && EPI == LM_OUT) e_a = *reinterpret_cast<const float4*>(p.x + (size_t)pm * p.d.w64 + pb * 16 + 4 * kg);
+  if (PRE && EPI == LM_OUT) e.a = *reinterpret_cast<const float4*>(p.x + (size_t)pm * p.d.w64 + pb * 16 + 4 * kg);
   if (PRE && EPI == LM_IN_GRU_STEP && nb0 < p.mix_blocks) {
     const int ch = (nb0 / 3) * 16 + 4 * kg;
-    e_a = *reinterpret_cast<const float4*>(p.state + (size_t)e_slot * p.d.gru16 + ch);
-    e_b = *reinterpret_cast<const float4*>(p.bz + ch);
-    e_c = *reinterpret_cast<const float4*>(p.bx + ch);
+    e.a = *reinterpret_cast<const float4*>(p.state + (size_t)e.slot * p.d.gru16 + ch);
+    e.b = *reinterpret_cast<const float4*>(p.bz + ch);
+    e.c = *reinterpret_cast<const float4*>(p.bx + ch);
   }
 
   tl_f32x4 acc[NB][MB];
@@ -183,126 +331,12 @@ __global__ __launch_bounds__(64 * WAVES) void lm_gemm_kernel(const LmGemm p) {
     };
     gather(i0, v);
 
+    float xv[4] = {0.f, 0.f, 0.f, 0.f}, gv[4] = {0.f, 0.f, 0.f, 0.f};
     if (GRU && mix) {
-      float xv[4], gv[4];
       gather(NB > 1 ? 1 : 0, xv);
       gather(NB > 2 ? 2 : 0, gv);
-      const int ch = (nb / 3) * 16 + 4 * kg;  // blocks come in threes: update gate, candidate, output gate
-      if (!live) continue;
-      const float4 b0 = PRE ? e_b : *reinterpret_cast<const float4*>(p.bz + ch), b1 = PRE ? e_c : *reinterpret_cast<const float4*>(p.bx + ch);
-      const float zb[4] = {b0.x, b0.y, b0.z, b0.w}, xb[4] = {b1.x, b1.y, b1.z, b1.w};
-      float keep[4], in[4], sg[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float zz = v[r] + zb[r], uu = xv[r] + xb[r];
-        const float z = lm_sigmoid(zz);
-        keep[r] = lm_sigmoid(-zz);
-        in[r] = z * (uu >= 0.f ? uu + 0.5f : lm_sigmoid(uu));
-        sg[r] = gv[r] * lm_sigmoid(gv[r]);
-      }
-      if (EPI == LM_IN_GRU_STEP) {
-        float4* sp = reinterpret_cast<float4*>(p.state + (size_t)e_slot * p.d.gru16 + ch);
-        const float4 old = e_pos > 0 ? e_a : make_float4(0.f, 0.f, 0.f, 0.f);
-        const float4 nw = make_float4(fmaf(keep[0], old.x, in[0]), fmaf(keep[1], old.y, in[1]), fmaf(keep[2], old.z, in[2]),
-                                      fmaf(keep[3], old.w, in[3]));
-        *sp = nw;
-        const float o[4] = {nw.x * sg[0], nw.y * sg[1], nw.z * sg[2], nw.w * sg[3]};
-        Tl<T>::st4((T*)p.act + tl_off<T>(m, ch, p.d.out_k), o);
-      } else {
-        float4* up = reinterpret_cast<float4*>(p.upd + (size_t)m * p.d.gru16 + ch);
-        up[0] = make_float4(keep[0], in[0], keep[1], in[1]);
-        up[1] = make_float4(keep[2], in[2], keep[3], in[3]);
-        Tl<T>::st4((T*)p.sg + (size_t)m * p.d.gru16 + ch, sg);
-      }
-      continue;
     }
-    if (EPI == LM_IN_ATTN || GRU) {
-      if (!live) continue;
-      if (nb >= p.mix_blocks) {  // (gate, up) pairs
-        const int f = (n - p.mix_blocks * 16) >> 1;
-        Tl<T>::st2((T*)p.act + tl_off<T>(m, p.d.ff_off + f, p.d.out_k), lm_ff(v[0], v[1], p.limit), lm_ff(v[2], v[3], p.limit));
-        continue;
-      }
-      if (EPI == LM_IN_ATTN) {
-        if (nb < p.b_qr) {
-          const int dq = p.d.dim16 >> 4, h = nb / dq, o = (nb - h * dq) * 16 + 4 * kg;
-          Tl<T>::st4((T*)p.qu + h * p.qu_z + tl_off<T>(m, o, p.d.dim64), v);
-        } else if (nb < p.b_c) {
-          const int dr = p.d.rot16 >> 4, b = nb - p.b_qr, h = b / dr, o = (b - h * dr) * 16 + 4 * kg;
-          const int slot = PRE ? e_slot : lm_slot(p.rows, m), pos = min(max(PRE ? e_pos : lm_pos(p.rows, m, slot), 0), p.rows.S - 1);
-          lm_rotate2(v, p.rope, pos, p.rot_pairs, o >> 1);
-          Tl<T>::st4((T*)p.qr + h * p.qr_z + tl_off<T, 32>(m, o, p.d.rot32), v);
-        } else if (nb < p.b_kr) {
-          const int o = (nb - p.b_c) * 16 + 4 * kg;
-          *reinterpret_cast<float4*>(p.craw + (size_t)m * p.d.rank16 + o) = make_float4(v[0], v[1], v[2], v[3]);
-        } else if (nb < p.b_g) {
-          const int o = (nb - p.b_kr) * 16 + 4 * kg;
-          const int slot = PRE ? e_slot : lm_slot(p.rows, m), pos = PRE ? e_pos : lm_pos(p.rows, m, slot);
-          if (pos >= 0 && pos < p.rows.S) {
-            lm_rotate2(v, p.rope, pos, p.rot_pairs, o >> 1);
-            Tl<T>::st4((T*)p.kr_cache + (size_t)slot * p.d.s64 * p.d.rot32 + tl_off<T, 32>(pos, o, p.d.rot32), v);
-          }
-        } else {
-          const int o = (nb - p.b_g) * 16 + 4 * kg;
-          if (o < p.d.heads16)  // the blocks behind the gates only fill the last tile of the mixer part
-            *reinterpret_cast<float4*>(p.gate + (size_t)m * p.d.heads16 + o) =
-                make_float4(lm_sigmoid(v[0]), lm_sigmoid(v[1]), lm_sigmoid(v[2]), lm_sigmoid(v[3]));
-        }
-      }
-      continue;
-    }
-    if (EPI == LM_OUT) {
-      float sq = 0.f;
-      if (live) {
-        float4* xp = reinterpret_cast<float4*>(p.x + (size_t)m * p.d.w64 + n);
-        const float4 old = PRE ? e_a : *xp;
-        v[0] += old.x; v[1] += old.y; v[2] += old.z; v[3] += old.w;
-        *xp = make_float4(v[0], v[1], v[2], v[3]);
-        Tl<T>::st4((T*)p.xt + tl_off<T>(m, n, p.d.w64), v);
-        sq = (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
-        if (p.layer_out)
-          for (int r = 0; r < 4; ++r) if (n + r < p.width) p.layer_out[(size_t)m * p.width + n + r] = v[r];
-      }
-      sq = rows_sum(sq);  // the 16 columns of this row's block
-      if (live && kg == 0 && nb < p.np) p.ssq_out[(size_t)m * p.np + nb] = sq;
-      continue;
-    }
-    if (LOGITS) {
-      if (live)
-        for (int r = 0; r < 4; ++r) if (n + r < p.vocab) p.logits[(size_t)m * p.vocab + n + r] = v[r];
-      continue;
-    }
-    if (EPI == LM_PROJ || EPI == LM_PLAIN || EPI == LM_MOE_DOWN) {
-      const int r = EPI == LM_MOE_DOWN ? p.ent[m] : m;
-      if (!live || r < 0) continue;
-      if (EPI != LM_MOE_DOWN && p.bias) {
-        const float4 b = *reinterpret_cast<const float4*>(p.bias + n);
-        v[0] += b.x; v[1] += b.y; v[2] += b.z; v[3] += b.w;
-      }
-      if (EPI == LM_PROJ) Tl<T>::st4((T*)p.out + (size_t)r * p.ldo + n, v);
-      else Tl<float>::st4((float*)p.out + (size_t)r * p.ldo + n, v);
-      continue;
-    }
-    if (EPI == LM_ACT || EPI == LM_MOE_UP) {
-      if (!live) continue;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) v[r] = lm_act(v[r], p.act_kind, p.act_pos, p.act_neg);
-      Tl<T>::st4((T*)p.act + tl_off<T>(m, n, p.act_k), v);
-      continue;
-    }
-    if (EPI == LM_EXPAND_K) {
-      if (live) Tl<T>::st4((T*)p.kv_out + blockIdx.z * p.kv_z + tl_off<T>(m, n, p.d.dim64), v);
-      continue;
-    }
-    if (EPI == LM_EXPAND_V) {
-      // blocks of 16 value dims x 32 keys; a lane of the attention kernel reads the keys 4 kg .. + 3 of both halves
-      if (live) {
-        T* dst = (T*)p.kv_out + blockIdx.z * p.kv_z + ((size_t)nb * (p.d.s64 >> 5) + (m >> 5)) * 512 +
-                 (l16 + 16 * ((m & 15) >> 2)) * 8 + 4 * ((m & 31) >> 4);
-        Tl<T>::st4(dst, v);
-      }
-      continue;
-    }
+    lm_unit<T, EPI, PRE>(p, m, nb, n, l16, kg, live, mix, v, xv, gv, e);
   }
   if (LOGITS && p.upd_lens && blockIdx.x == 0) {
     if (p.upd_inc) {
@@ -311,6 +345,191 @@ __global__ __launch_bounds__(64 * WAVES) void lm_gemm_kernel(const LmGemm p) {
       for (int b = tid; b < p.upd_rows; b += 64 * WAVES) atomicAdd(&p.upd_lens[lm_slot(p.rows, b)], 1);
     }
   }
+}
+
+// ---- many rows, bf16: the operands go through LDS, whole tiles per wave ----
+// A prompt's products are bound by the matrix instructions only if a tile is large enough for what feeds it: lm_gemm_kernel
+// splits K over its waves, so every wave fetches all operands of its 32 x 32 or 64 x 64 tile from L2 (16 flops per byte).
+// Here a workgroup's four waves share (16 MBW WM) x (16 NBW WN) tiles; S stages of one 32-column step each are in flight,
+// written to LDS by the loads themselves (a piece of the operand layout is 1 KiB in lane order on both sides), and a wave
+// waits only for the oldest.  Large products: tiles of one feature range follow each other on one XCD, whose L2 then
+// holds its weights.
+// 16 bytes per lane from g to LDS at byte `at` + 16 lane (wave-uniform).  There is no register for the compiler to wait
+// for: the kernel counts these loads itself (vmcnt).  Through the builtin the compiler waited for all of them in front of
+// every LDS read.
+__device__ __forceinline__ void lm_to_lds(const char* g, uint32_t at) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(at), "v"(g) : "memory");
+}
+
+template <int EPI, int MBW, int NBW, int WM, int WN, int S, int KS>
+__global__ __launch_bounds__(256, 2) void lm_wide_kernel(const LmGemm p) {
+  constexpr bool SCALED = EPI == LM_IN_ATTN || EPI == LM_IN_GRU_SEQ;
+  constexpr bool GRU = EPI == LM_IN_GRU_SEQ, MOE = EPI == LM_MOE_UP || EPI == LM_MOE_DOWN;
+  constexpr int MB = MBW * WM, NB = NBW * WN, PIECES = (MB + NB) * KS, L = PIECES / 4;
+  static_assert(WM * WN == 4 && PIECES % 4 == 0, "four waves, the same number of pieces each");
+  static_assert(!GRU || NBW % 3 == 0, "a recurrence's blocks come in threes");
+  __shared__ __align__(16) char lds[S * PIECES * 1024];
+  __shared__ float srow[MB * 16];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int l16 = lane & 15, kg = lane >> 4, wm = wave % WM, wn = wave / WM;
+  const int MBL = (p.M + 15) >> 4, NBL = p.N >> 4, MT = MOE ? p.max_tiles : (MBL + MB - 1) / MB, NT = (NBL + NB - 1) / NB;
+  int t, nt;
+  if (MOE) {
+    nt = (int)blockIdx.x % NT; t = (int)blockIdx.x / NT;
+    if (t >= p.n_tiles[0]) return;  // uniform
+  } else if (p.by_xcd) {  // workgroup i is on XCD i % 8
+    const int slice = (int)blockIdx.x >> 3;
+    t = slice % MT; nt = slice / MT * 8 + ((int)blockIdx.x & 7);
+    if (nt >= NT) return;
+  } else {
+    t = (int)blockIdx.x % MT; nt = (int)blockIdx.x / MT;
+  }
+  const int mb0 = t * MB, nb0 = nt * NB, m0 = mb0 * 16;
+  const int Q = p.K / (32 * KS);  // steps
+  const size_t wz = MOE ? (size_t)p.tile_e[t] * p.wz : blockIdx.z * p.wz;
+
+  // pieces wave, wave + 4, ... of a stage are this wave's: row blocks first, then feature blocks
+  const char* src[L];
+#pragma unroll
+  for (int i = 0; i < L; ++i) {
+    const int q = (wave + 4 * i) / KS;
+    src[i] = q < MB ? (const char*)p.X + (size_t)(MOE ? mb0 + q : min(mb0 + q, MBL - 1)) * Q * (KS * 1024)
+                    : (const char*)p.W + wz * 2 + (size_t)min(nb0 + q - MB, NBL - 1) * Q * (KS * 1024);
+    src[i] += (wave + 4 * i) % KS * 1024 + lane * 16;
+  }
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
+  auto issue = [&](int q, int slot) {
+#pragma unroll
+    for (int i = 0; i < L; ++i)
+      lm_to_lds(src[i] + (size_t)q * (KS * 1024), lds0 + (uint32_t)(slot * PIECES + wave + 4 * i) * 1024u);
+  };
+#pragma unroll
+  for (int q = 0; q < S - 1; ++q)
+    if (q < Q) issue(q, q);
+
+  if (SCALED) {
+    // 16 lanes add up one row's sums of squares, in a fixed order, the loads of all the wave's rows side by side (one
+    // after the other they took longer than the products: 98 against 61 us at 1024 x 11776 x 2048)
+    constexpr int G = MB;  // rows per 16 lanes: 16 MB rows over 16 groups
+    const int grp = wave * 4 + kg;
+    float a[G];
+#pragma unroll
+    for (int i = 0; i < G; ++i) a[i] = 0.f;
+    if ((p.np & 3) == 0) {
+      for (int c = 4 * l16; c < p.np; c += 64) {
+        float4 v[G];
+#pragma unroll
+        for (int i = 0; i < G; ++i) v[i] = *reinterpret_cast<const float4*>(p.ssq + (size_t)min(m0 + grp * G + i, p.M - 1) * p.np + c);
+#pragma unroll
+        for (int i = 0; i < G; ++i) a[i] += (v[i].x + v[i].y) + (v[i].z + v[i].w);
+      }
+    } else {
+      for (int c = l16; c < p.np; c += 16) {
+        float v[G];
+#pragma unroll
+        for (int i = 0; i < G; ++i) v[i] = p.ssq[(size_t)min(m0 + grp * G + i, p.M - 1) * p.np + c];
+#pragma unroll
+        for (int i = 0; i < G; ++i) a[i] += v[i];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < G; ++i) {
+      const float t = group16_sum(a[i]);
+      if (l16 == 0) srow[grp * G + i] = p.norm[0] / sqrtf(t / (float)p.width + p.eps);
+    }
+  }
+
+  tl_f32x4 acc[NBW][MBW];
+#pragma unroll
+  for (int i = 0; i < NBW; ++i)
+#pragma unroll
+    for (int j = 0; j < MBW; ++j) acc[i][j] = tl_f32x4{0.f, 0.f, 0.f, 0.f};
+  int slot = 0;
+  for (int q = 0; q < Q; ++q) {
+    // the oldest stage has landed once no more than the stages behind it are outstanding, for every wave behind the
+    // barrier; the fragments read from the slot that is filled next have arrived as well
+    if (q + S - 1 <= Q) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((S - 2) * L) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (q + S - 1 < Q) issue(q + S - 1, slot == 0 ? S - 1 : slot - 1);
+    const char* st = lds + slot * PIECES * 1024 + lane * 16;
+    uint4 xa[KS][MBW], wa[KS][NBW];
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+#pragma unroll
+      for (int j = 0; j < MBW; ++j) xa[k][j] = *reinterpret_cast<const uint4*>(st + ((wm * MBW + j) * KS + k) * 1024);
+#pragma unroll
+      for (int i = 0; i < NBW; ++i) wa[k][i] = *reinterpret_cast<const uint4*>(st + ((MB + wn * NBW + i) * KS + k) * 1024);
+    }
+#pragma unroll
+    for (int k = 0; k < KS; ++k)
+#pragma unroll
+      for (int i = 0; i < NBW; ++i)
+#pragma unroll
+        for (int j = 0; j < MBW; ++j) acc[i][j] = Tl<bf16_t>::mma(wa[k][i], xa[k][j], acc[i][j]);
+    slot = slot == S - 1 ? 0 : slot + 1;
+  }
+  // The sums pass through this wave's share of LDS, so that the epilogue is a loop: unrolled over the units it is 100 KB of
+  // instructions, and fetching those took longer than the products (98 against 61 us at 1024 x 11776 x 2048).
+  constexpr int ROOM = S * PIECES / 4, CH0 = ROOM / MBW < NBW ? ROOM / MBW : NBW, CH = GRU ? CH0 / 3 * 3 : CH0;  // blocks at a time
+  static_assert(CH > 0, "a block of sums fits the wave's share");
+  __syncthreads();
+  char* own = lds + wave * ROOM * 1024 + lane * 16;
+#pragma unroll
+  for (int c = 0; c < NBW; c += CH) {
+#pragma unroll
+    for (int i = c; i < c + CH && i < NBW; ++i)
+#pragma unroll
+      for (int j = 0; j < MBW; ++j) *reinterpret_cast<tl_f32x4*>(own + ((i - c) * MBW + j) * 1024) = acc[i][j];
+    const int n_blocks = min(CH, NBW - c);
+#pragma unroll 1
+    for (int i = 0; i < n_blocks; ++i) {  // the MBW units of a block side by side: their loads and exponentials overlap
+      const int nb = nb0 + wn * NBW + c + i, n = nb * 16 + 4 * kg;
+      const bool mix = GRU && nb - i % 3 < p.mix_blocks;  // uniform
+      if (nb >= NBL || (mix && i % 3)) continue;
+      auto sums = [&](int blk, int j, float* o) {
+        const tl_f32x4 a = *reinterpret_cast<const tl_f32x4*>(own + (blk * MBW + j) * 1024);
+        const float sc = SCALED ? srow[(wm * MBW + j) * 16 + l16] : 1.f;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[r] = a[r] * sc;
+      };
+      const int mw = m0 + wm * MBW * 16 + l16;
+      if ((EPI == LM_IN_ATTN || GRU) && nb >= p.mix_blocks) {  // (gate, up) pairs
+        const int f = p.d.ff_off + ((n - p.mix_blocks * 16) >> 1);
+#pragma unroll
+        for (int j = 0; j < MBW; ++j) {
+          float v[4];
+          sums(i, j, v);
+          if (mw + 16 * j < p.M)
+            Tl<bf16_t>::st2((bf16_t*)p.act + tl_off<bf16_t>(mw + 16 * j, f, p.d.out_k), lm_ff<bf16_t>(v[0], v[1], p.limit), lm_ff<bf16_t>(v[2], v[3], p.limit));
+        }
+        continue;
+      }
+      LmPre e[MBW];
+#pragma unroll
+      for (int j = 0; j < MBW; ++j)
+        if (EPI == LM_OUT) e[j].a = *reinterpret_cast<const float4*>(p.x + (size_t)min(mw + 16 * j, p.M - 1) * p.d.w64 + n);
+#pragma unroll
+      for (int j = 0; j < MBW; ++j) {
+        float v[4], xv[4] = {0.f, 0.f, 0.f, 0.f}, gv[4] = {0.f, 0.f, 0.f, 0.f};
+        sums(i, j, v);
+        if (GRU && mix) { sums(i + 1, j, xv); sums(i + 2, j, gv); }
+        lm_unit<bf16_t, EPI, EPI == LM_OUT>(p, mw + 16 * j, nb, n, l16, kg, MOE || mw + 16 * j < p.M, mix, v, xv, gv, e[j]);
+      }
+    }
+  }
+}
+
+template <int EPI, int MBW, int NBW, int WM, int WN, int S, int KS>
+static int go_wide(LmGemm g, int nz, hipStream_t st) {
+  const int MT = (g.M + 16 * MBW * WM - 1) / (16 * MBW * WM), NT = (g.N / 16 + NBW * WN - 1) / (NBW * WN);
+  const bool moe = EPI == LM_MOE_UP || EPI == LM_MOE_DOWN;
+  g.by_xcd = !moe && NT >= 24;  // with fewer, whole XCDs would have nothing or twice as much to do
+  const int tiles = moe ? g.max_tiles * NT : g.by_xcd ? MT * ((NT + 7) & ~7) : MT * NT;
+  hipLaunchKernelGGL((lm_wide_kernel<EPI, MBW, NBW, WM, WN, S, KS>), dim3((unsigned)tiles, 1, nz), dim3(256), 0, st, g);
+  HIP_TRY(hipGetLastError());
+  return VUI_OK;
 }
 
 template <typename T, int MB, int NB, int WAVES, int EPI>
@@ -323,21 +542,53 @@ static int go(const LmGemm& g, int nz, hipStream_t st) {
   return VUI_OK;
 }
 
+// Which kernel takes an M x N x K product of a prompt, and with which tile: estimated microseconds besides the launch and
+// the epilogue (MI355X).  A step of 32 columns takes a tile of lm_wide_kernel `wait` us when its CU has nothing else to do
+// and `work` us per tile when it has; lm_gemm_kernel's waves split K, which is quicker for the smaller products, at 0.38 us per
+// thousand 32 x 32 tiles and 64 columns, and keeps what is close.  Measured (us, lm_gemm_kernel / lm_wide_kernel): 1024 x 11776 x 2048 147 / 61,
+// 1024 x 2048 x 6144 82 / 39, 1024 x 5120 x 768 26 / 17, 1024 x 768 x 2816 16 / 17, 300 x 768 x 2816 9 / 17.
+enum { LM_SPLIT_K = -1, LM_T128 = 0, LM_T64x128 = 1, LM_T64 = 2 };
+static int lm_tile(int epi, int M, int N, int K) {
+  static const struct { int bm, bn; double wait, work; } tile[] = {{128, 128, 0.335, 0.144}, {64, 128, 0.21, 0.08}, {64, 64, 0.17, 0.059}};
+  if (M < 128) return LM_SPLIT_K;
+  int best = LM_SPLIT_K;
+  double cost = 0.85 * 0.38e-3 * ((M + 31) / 32) * ((N + 31) / 32) * (K / 64);
+  if (epi == LM_IN_GRU_SEQ) {  // 128 x 192, and 20 us more in the epilogue (160 / 98 at 1024 x 14336 x 2048, 30 / 35 at 1024 x 6400 x 768)
+    const double work = (double)(((M + 127) / 128 * ((N + 191) / 192) + 255) / 256) * 0.2;
+    return 20 + (K / 32) * (work > 0.4 ? work : 0.4) < cost ? LM_T128 : LM_SPLIT_K;
+  }
+  for (int i = 0; i < 3; ++i) {
+    const long tiles = (long)((M + tile[i].bm - 1) / tile[i].bm) * ((N + tile[i].bn - 1) / tile[i].bn);
+    const double work = (double)((tiles + 255) / 256) * tile[i].work, c = (K / 32) * (work > tile[i].wait ? work : tile[i].wait);
+    if (c < cost) { best = i; cost = c; }
+  }
+  return best;
+}
+template <int EPI>
+static int pick_wide(int tile, const LmGemm& g, hipStream_t st) {
+  switch (tile) {
+    case LM_T128: return go_wide<EPI, 4, 4, 2, 2, 4, 1>(g, 1, st);
+    case LM_T64x128: return go_wide<EPI, 4, 2, 1, 4, 3, 2>(g, 1, st);
+    default: return go_wide<EPI, 2, 2, 2, 2, 4, 2>(g, 1, st);
+  }
+}
+
 // up to 16 rows: one row block, more waves per tile (the weights are streamed once, latency counts)
 template <typename T>
 static int pick(int epi, const LmGemm& g, int nz, hipStream_t st) {
   const bool few = g.M <= 16;
-  // many rows: tiles of 64 x 64, or 64 x 32 where the former would leave half of the chip idle
-  const long tiles = (long)((g.M + 63) / 64) * ((g.N + 63) / 64);
-  if (sizeof(T) == 2 && g.M >= 256 && tiles >= 64) {
-    const bool wide = tiles >= 160;
-    if (epi == LM_PROJ) return wide ? go<T, 4, 4, 4, LM_PROJ>(g, nz, st) : go<T, 4, 2, 4, LM_PROJ>(g, nz, st);
-    if (epi == LM_PLAIN) return wide ? go<T, 4, 4, 4, LM_PLAIN>(g, nz, st) : go<T, 4, 2, 4, LM_PLAIN>(g, nz, st);
-    if (epi == LM_ACT) return wide ? go<T, 4, 4, 4, LM_ACT>(g, nz, st) : go<T, 4, 2, 4, LM_ACT>(g, nz, st);
+  const int tile = sizeof(T) == 2 && nz == 1 ? lm_tile(epi, g.M, g.N, g.K) : LM_SPLIT_K;
+  if (tile != LM_SPLIT_K) {
+    if (epi == LM_IN_ATTN) return pick_wide<LM_IN_ATTN>(tile, g, st);
+    if (epi == LM_IN_GRU_SEQ) return go_wide<LM_IN_GRU_SEQ, 4, 6, 2, 2, 3, 1>(g, 1, st);
+    if (epi == LM_OUT) return pick_wide<LM_OUT>(tile, g, st);
+    if (epi == LM_PROJ) return pick_wide<LM_PROJ>(tile, g, st);
+    if (epi == LM_PLAIN) return pick_wide<LM_PLAIN>(tile, g, st);
+    if (epi == LM_ACT) return pick_wide<LM_ACT>(tile, g, st);
   }
   if (sizeof(T) == 2 && g.tile_rows == 64) {
-    if (epi == LM_MOE_UP) return go<T, 4, 4, 4, LM_MOE_UP>(g, nz, st);
-    if (epi == LM_MOE_DOWN) return go<T, 4, 4, 4, LM_MOE_DOWN>(g, nz, st);
+    if (epi == LM_MOE_UP) return go_wide<LM_MOE_UP, 4, 2, 1, 4, 3, 2>(g, nz, st);
+    if (epi == LM_MOE_DOWN) return go_wide<LM_MOE_DOWN, 4, 2, 1, 4, 3, 2>(g, nz, st);
   }
   // few rows and few features: one block of features per workgroup, so that more of the chip takes part
   if (few && (long)g.N * (g.max_tiles > 0 ? g.max_tiles : 1) <= 4096) {

@@ -117,7 +117,7 @@ class _NativeLM:
 class TokenLM:
     """Decoder-only token model: weights in the kernels' layout, prefill and decode over a slot cache."""
 
-    PREFILL_CHUNK = 1024  # most positions of one native prefill call
+    PREFILL_CHUNK = 2048  # most positions of one native prefill call
 
     def __init__(self, config: LMConfig, state_dict: "dict[str, Tensor]", device="cuda", dtype=torch.bfloat16,
                  max_seqlen: int = 4096):
