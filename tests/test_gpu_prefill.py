@@ -154,3 +154,29 @@ def test_prefill_other_head_dims(heads, kv, rope_dim):
         assert rel_err(got, want) <= BF16_TOL, rel_err(got, want)
     for mine, theirs in ((m.decoder._k, m2.decoder._k), (m.decoder._v, m2.decoder._v)):
         assert rel_err(mine[:, 0, :pos], theirs[:, 0, :pos]) <= BF16_TOL
+
+
+@pytest.mark.parametrize("int8", [False, True])
+def test_prefill_tiles_of_every_size(int8):
+    """Block lengths that choose every form of the products (16- and 32-row tiles of 8 to 16 waves, 32 x 32 tiles, large
+    tiles) and end inside one, at Vui Nano dims on two layers: against the position-by-position path, or in portions of
+    290 positions for the longest.  Two bf16 evaluations: the tolerance of the test above."""
+    d = O.Dims(n_layers=2)
+    sd = O.synthetic_state_dict(d, seed=1)
+    m = make_model(d, sd, BF, int8=int8, max_seqlen=1216)
+    m.decoder.allocate_flash_kv_cache(1, m.device, BF, max_seqlen=1216)
+    seq = m.decoder.flash_kv_caches[0].seq_lens
+    emb = (torch.randn(1, 1187, d.d_model, generator=torch.Generator().manual_seed(4)) * 0.08).to(BF).cuda()
+
+    def run(x, portion, minimum=4):
+        seq.zero_()
+        m.decoder.PREFILL_MIN = minimum
+        h = torch.cat([m.decoder.forward_flash(x[:, i:i + portion].contiguous(), None) for i in range(0, x.shape[1], portion)], dim=1)
+        return h, m.decoder._k[:, 0, :x.shape[1]].clone(), m.decoder._v[:, 0, :x.shape[1]].clone()
+
+    for T in (5, 16, 17, 45, 130, 251, 777, 1187):
+        x = emb[:, :T].contiguous()
+        got = run(x, T)
+        want = run(x, T, 10 ** 9) if T < 300 else run(x, 290)
+        for a, b in zip(got, want):
+            assert rel_err(a, b) <= BF16_TOL, (T, rel_err(a, b))

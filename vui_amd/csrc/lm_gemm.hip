@@ -7,7 +7,7 @@
 // row, in pieces of 16 columns (LM_OUT, the embedding), so no launch is spent on norms.
 #include "common.h"
 #include "lm.h"
-#include "tile.h"
+#include "wide.h"
 
 // fp32 contexts: the library's exponential and division.  bf16 contexts: a prompt's epilogues evaluate ten million of
 // these per layer and were bound by their instructions, so the exponential is v_exp_f32 with the rounding of its argument
@@ -347,28 +347,16 @@ __global__ __launch_bounds__(64 * WAVES) void lm_gemm_kernel(const LmGemm p) {
   }
 }
 
-// ---- many rows, bf16: the operands go through LDS, whole tiles per wave ----
-// A prompt's products are bound by the matrix instructions only if a tile is large enough for what feeds it: lm_gemm_kernel
-// splits K over its waves, so every wave fetches all operands of its 32 x 32 or 64 x 64 tile from L2 (16 flops per byte).
-// Here a workgroup's four waves share (16 MBW WM) x (16 NBW WN) tiles; S stages of one 32-column step each are in flight,
-// written to LDS by the loads themselves (a piece of the operand layout is 1 KiB in lane order on both sides), and a wave
-// waits only for the oldest.  Large products: tiles of one feature range follow each other on one XCD, whose L2 then
-// holds its weights.
-// 16 bytes per lane from g to LDS at byte `at` + 16 lane (wave-uniform).  There is no register for the compiler to wait
-// for: the kernel counts these loads itself (vmcnt).  Through the builtin the compiler waited for all of them in front of
-// every LDS read.
-__device__ __forceinline__ void lm_to_lds(const char* g, uint32_t at) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(at), "v"(g) : "memory");
-}
-
+// ---- many rows, bf16: large tiles through LDS (wide.h) ----
+// Tiles of one feature range follow each other on one XCD where there are enough of them, whose L2 then holds those weights.
 template <int EPI, int MBW, int NBW, int WM, int WN, int S, int KS>
 __global__ __launch_bounds__(256, 2) void lm_wide_kernel(const LmGemm p) {
   constexpr bool SCALED = EPI == LM_IN_ATTN || EPI == LM_IN_GRU_SEQ;
   constexpr bool GRU = EPI == LM_IN_GRU_SEQ, MOE = EPI == LM_MOE_UP || EPI == LM_MOE_DOWN;
-  constexpr int MB = MBW * WM, NB = NBW * WN, PIECES = (MB + NB) * KS, L = PIECES / 4;
-  static_assert(WM * WN == 4 && PIECES % 4 == 0, "four waves, the same number of pieces each");
+  typedef WideTile<MBW, NBW, WM, WN, S, KS> Tile;
+  constexpr int MB = Tile::MB, NB = Tile::NB;
   static_assert(!GRU || NBW % 3 == 0, "a recurrence's blocks come in threes");
-  __shared__ __align__(16) char lds[S * PIECES * 1024];
+  __shared__ __align__(16) char lds[Tile::LDS];
   __shared__ float srow[MB * 16];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int l16 = lane & 15, kg = lane >> 4, wm = wave % WM, wn = wave / WM;
@@ -388,24 +376,11 @@ __global__ __launch_bounds__(256, 2) void lm_wide_kernel(const LmGemm p) {
   const int Q = p.K / (32 * KS);  // steps
   const size_t wz = MOE ? (size_t)p.tile_e[t] * p.wz : blockIdx.z * p.wz;
 
-  // pieces wave, wave + 4, ... of a stage are this wave's: row blocks first, then feature blocks
-  const char* src[L];
-#pragma unroll
-  for (int i = 0; i < L; ++i) {
-    const int q = (wave + 4 * i) / KS;
-    src[i] = q < MB ? (const char*)p.X + (size_t)(MOE ? mb0 + q : min(mb0 + q, MBL - 1)) * Q * (KS * 1024)
-                    : (const char*)p.W + wz * 2 + (size_t)min(nb0 + q - MB, NBL - 1) * Q * (KS * 1024);
-    src[i] += (wave + 4 * i) % KS * 1024 + lane * 16;
-  }
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
-  auto issue = [&](int q, int slot) {
-#pragma unroll
-    for (int i = 0; i < L; ++i)
-      lm_to_lds(src[i] + (size_t)q * (KS * 1024), lds0 + (uint32_t)(slot * PIECES + wave + 4 * i) * 1024u);
-  };
-#pragma unroll
-  for (int q = 0; q < S - 1; ++q)
-    if (q < Q) issue(q, q);
+  Tile tile;
+  tile.begin(lds, wave, lane,
+             [&](int i) { return (const char*)p.X + (size_t)(MOE ? mb0 + i : min(mb0 + i, MBL - 1)) * Q * (KS * 1024); },
+             [&](int i) { return (const char*)p.W + wz * 2 + (size_t)min(nb0 + i, NBL - 1) * Q * (KS * 1024); });
+  tile.prologue(Q);
 
   if (SCALED) {
     // 16 lanes add up one row's sums of squares, in a fixed order, the loads of all the wave's rows side by side (one
@@ -440,39 +415,10 @@ __global__ __launch_bounds__(256, 2) void lm_wide_kernel(const LmGemm p) {
   }
 
   tl_f32x4 acc[NBW][MBW];
-#pragma unroll
-  for (int i = 0; i < NBW; ++i)
-#pragma unroll
-    for (int j = 0; j < MBW; ++j) acc[i][j] = tl_f32x4{0.f, 0.f, 0.f, 0.f};
-  int slot = 0;
-  for (int q = 0; q < Q; ++q) {
-    // the oldest stage has landed once no more than the stages behind it are outstanding, for every wave behind the
-    // barrier; the fragments read from the slot that is filled next have arrived as well
-    if (q + S - 1 <= Q) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((S - 2) * L) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    if (q + S - 1 < Q) issue(q + S - 1, slot == 0 ? S - 1 : slot - 1);
-    const char* st = lds + slot * PIECES * 1024 + lane * 16;
-    uint4 xa[KS][MBW], wa[KS][NBW];
-#pragma unroll
-    for (int k = 0; k < KS; ++k) {
-#pragma unroll
-      for (int j = 0; j < MBW; ++j) xa[k][j] = *reinterpret_cast<const uint4*>(st + ((wm * MBW + j) * KS + k) * 1024);
-#pragma unroll
-      for (int i = 0; i < NBW; ++i) wa[k][i] = *reinterpret_cast<const uint4*>(st + ((MB + wn * NBW + i) * KS + k) * 1024);
-    }
-#pragma unroll
-    for (int k = 0; k < KS; ++k)
-#pragma unroll
-      for (int i = 0; i < NBW; ++i)
-#pragma unroll
-        for (int j = 0; j < MBW; ++j) acc[i][j] = Tl<bf16_t>::mma(wa[k][i], xa[k][j], acc[i][j]);
-    slot = slot == S - 1 ? 0 : slot + 1;
-  }
+  tile.run(Q, acc);
   // The sums pass through this wave's share of LDS, so that the epilogue is a loop: unrolled over the units it is 100 KB of
   // instructions, and fetching those took longer than the products (98 against 61 us at 1024 x 11776 x 2048).
-  constexpr int ROOM = S * PIECES / 4, CH0 = ROOM / MBW < NBW ? ROOM / MBW : NBW, CH = GRU ? CH0 / 3 * 3 : CH0;  // blocks at a time
+  constexpr int ROOM = S * Tile::PIECES / 4, CH0 = ROOM / MBW < NBW ? ROOM / MBW : NBW, CH = GRU ? CH0 / 3 * 3 : CH0;  // blocks at a time
   static_assert(CH > 0, "a block of sums fits the wave's share");
   __syncthreads();
   char* own = lds + wave * ROOM * 1024 + lane * 16;
@@ -542,33 +488,20 @@ static int go(const LmGemm& g, int nz, hipStream_t st) {
   return VUI_OK;
 }
 
-// Which kernel takes an M x N x K product of a prompt, and with which tile: estimated microseconds besides the launch and
-// the epilogue (MI355X).  A step of 32 columns takes a tile of lm_wide_kernel `wait` us when its CU has nothing else to do
-// and `work` us per tile when it has; lm_gemm_kernel's waves split K, which is quicker for the smaller products, at 0.38 us per
-// thousand 32 x 32 tiles and 64 columns, and keeps what is close.  Measured (us, lm_gemm_kernel / lm_wide_kernel): 1024 x 11776 x 2048 147 / 61,
-// 1024 x 2048 x 6144 82 / 39, 1024 x 5120 x 768 26 / 17, 1024 x 768 x 2816 16 / 17, 300 x 768 x 2816 9 / 17.
-enum { LM_SPLIT_K = -1, LM_T128 = 0, LM_T64x128 = 1, LM_T64 = 2 };
+// Tile of a prompt's product (wide_pick); a minGRU projection takes 128 x 192, with 20 us more in the epilogue
+// (us, K-splitting / large tile: 160 / 98 at 1024 x 14336 x 2048, 30 / 35 at 1024 x 6400 x 768).
 static int lm_tile(int epi, int M, int N, int K) {
-  static const struct { int bm, bn; double wait, work; } tile[] = {{128, 128, 0.335, 0.144}, {64, 128, 0.21, 0.08}, {64, 64, 0.17, 0.059}};
-  if (M < 128) return LM_SPLIT_K;
-  int best = LM_SPLIT_K;
-  double cost = 0.85 * 0.38e-3 * ((M + 31) / 32) * ((N + 31) / 32) * (K / 64);
-  if (epi == LM_IN_GRU_SEQ) {  // 128 x 192, and 20 us more in the epilogue (160 / 98 at 1024 x 14336 x 2048, 30 / 35 at 1024 x 6400 x 768)
-    const double work = (double)(((M + 127) / 128 * ((N + 191) / 192) + 255) / 256) * 0.2;
-    return 20 + (K / 32) * (work > 0.4 ? work : 0.4) < cost ? LM_T128 : LM_SPLIT_K;
-  }
-  for (int i = 0; i < 3; ++i) {
-    const long tiles = (long)((M + tile[i].bm - 1) / tile[i].bm) * ((N + tile[i].bn - 1) / tile[i].bn);
-    const double work = (double)((tiles + 255) / 256) * tile[i].work, c = (K / 32) * (work > tile[i].wait ? work : tile[i].wait);
-    if (c < cost) { best = i; cost = c; }
-  }
-  return best;
+  double us;
+  const int t = wide_pick(M, N, K, 0.85, &us);
+  if (epi != LM_IN_GRU_SEQ) return t;
+  const double work = (double)(((M + 127) / 128 * ((N + 191) / 192) + 255) / 256) * 0.2;
+  return M >= 128 && 20 + (K / 32) * (work > 0.4 ? work : 0.4) < us ? WIDE_128 : WIDE_NONE;
 }
 template <int EPI>
 static int pick_wide(int tile, const LmGemm& g, hipStream_t st) {
   switch (tile) {
-    case LM_T128: return go_wide<EPI, 4, 4, 2, 2, 4, 1>(g, 1, st);
-    case LM_T64x128: return go_wide<EPI, 4, 2, 1, 4, 3, 2>(g, 1, st);
+    case WIDE_128: return go_wide<EPI, 4, 4, 2, 2, 4, 1>(g, 1, st);
+    case WIDE_64x128: return go_wide<EPI, 4, 2, 1, 4, 3, 2>(g, 1, st);
     default: return go_wide<EPI, 2, 2, 2, 2, 4, 2>(g, 1, st);
   }
 }
@@ -577,8 +510,8 @@ static int pick_wide(int tile, const LmGemm& g, hipStream_t st) {
 template <typename T>
 static int pick(int epi, const LmGemm& g, int nz, hipStream_t st) {
   const bool few = g.M <= 16;
-  const int tile = sizeof(T) == 2 && nz == 1 ? lm_tile(epi, g.M, g.N, g.K) : LM_SPLIT_K;
-  if (tile != LM_SPLIT_K) {
+  const int tile = sizeof(T) == 2 && nz == 1 ? lm_tile(epi, g.M, g.N, g.K) : WIDE_NONE;
+  if (tile != WIDE_NONE) {
     if (epi == LM_IN_ATTN) return pick_wide<LM_IN_ATTN>(tile, g, st);
     if (epi == LM_IN_GRU_SEQ) return go_wide<LM_IN_GRU_SEQ, 4, 6, 2, 2, 3, 1>(g, 1, st);
     if (epi == LM_OUT) return pick_wide<LM_OUT>(tile, g, st);

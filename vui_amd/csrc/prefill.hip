@@ -14,7 +14,7 @@
 // the norm, products of the rotation rounded before their sum, residual sums rounded).
 #include "common.h"
 #include "internal.h"
-#include "tile.h"
+#include "wide.h"
 #include <stdio.h>
 
 typedef tl_bf16x8 pf_bf16x8;
@@ -47,83 +47,74 @@ __global__ __launch_bounds__(256) void pf_tile_kernel(const bf16_t* __restrict__
 }
 
 // C = X W^T for the projections (K = d_model ... ffn; 64 x 64 tiles would give only 9 x 12 ... 9 x 64
-// workgroups at 576 positions, each a long serial walk over K): a workgroup owns 32 rows x 32 features and its four waves split
-// the K steps between them, so a wave's chain of dependent trips to memory is a quarter as long and four times as
-// many workgroups are in flight.  The four partial tiles meet in LDS and are added in wave order (a fixed order:
+// workgroups at 576 positions, each a long serial walk over K): a workgroup owns 16 MB rows x 16 NB features and its waves
+// split the K steps between them, so a wave's chain of dependent trips to memory is a fraction as long and more
+// workgroups are in flight.  The partial tiles meet in LDS and are added in wave order (a fixed order:
 // results do not depend on timing).
 // DUAL: two weight matrices against the same activations, h = rnd(rnd(silu(rnd(a))) * rnd(c)) written once
 // (SwiGLU, src/vui/model.py:282) instead of two products and a pass over both.
-// eight int8 -> four packed bf16 pairs, exact
-__device__ __forceinline__ uint4 pf_widen8(uint32_t lo, uint32_t hi) {
-  uint4 r;
-  r.x = f2bf2((float)(int8_t)(lo & 0xff), (float)(int8_t)((lo >> 8) & 0xff));
-  r.y = f2bf2((float)(int8_t)((lo >> 16) & 0xff), (float)(int8_t)(lo >> 24));
-  r.z = f2bf2((float)(int8_t)(hi & 0xff), (float)(int8_t)((hi >> 8) & 0xff));
-  r.w = f2bf2((float)(int8_t)((hi >> 16) & 0xff), (float)(int8_t)(hi >> 24));
-  return r;
-}
-
-template <int EPI, bool DUAL, bool I8>
-__global__ __launch_bounds__(256) void pf_gemm4_kernel(const PfGemm p, const void* __restrict__ W2, int c_tiled) {
-  constexpr int TILE = 1024;  // floats of one partial tile
+template <int EPI, bool DUAL, bool I8, int WAVES, int MB, int NB>
+__global__ __launch_bounds__(64 * WAVES) void pf_gemm_kernel(const PfGemm p, const void* __restrict__ W2, int c_tiled) {
+  constexpr int TILE = MB * NB * 256;  // floats of one partial tile
   constexpr int PW = (DUAL ? 2 : 1) * TILE;
-  __shared__ float part[4 * PW];
+  __shared__ __align__(16) float part[WAVES * PW];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int l16 = lane & 15, kg = lane >> 4;
-  const int MT = (p.M + 31) >> 5;
+  const int MT = (p.M + 16 * MB - 1) / (16 * MB);
   const int id = blockIdx.x;
-  const int m0 = (id % MT) * 32, n0 = (id / MT) * 32;
+  const int m0 = (id % MT) * 16 * MB, n0 = (id / MT) * 16 * NB;
   // A step covers 64 values of k, one block of the tiled operands per 16 rows: the lane's 16-byte piece of half h
   // (k = 64 s + 16 kg + 8 h ...; any assignment of k to lanes is valid as long as both operands share it) is at
   // block + 512 h + 8 lane.
   const int nsteps = p.K >> 6;
-  const int s0 = nsteps * wave / 4, s1 = nsteps * (wave + 1) / 4;
-  const int MB = (p.M + 15) >> 4, NB = (p.N + 15) >> 4;  // 16-row blocks; a tile past the end reads the last block again
-  const bf16_t* xr[2];
-  const char* wr[2];  // byte addresses: a block is 2048 bytes of bf16 (two 16-byte pieces per lane) or 1024 of int8 (one)
-  const char* vr[2];
+  const int s0 = nsteps * wave / WAVES, s1 = nsteps * (wave + 1) / WAVES;
+  const int MBL = (p.M + 15) >> 4, NBL = (p.N + 15) >> 4;  // 16-row blocks; a tile past the end reads the last block again
+  const bf16_t* xr[MB];
+  const char* wr[NB];  // byte addresses: a block is 2048 bytes of bf16 (two 16-byte pieces per lane) or 1024 of int8 (one)
+  const char* vr[NB];
   constexpr int WB = I8 ? 1024 : 2048, WL = 16;
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    xr[j] = p.X + (size_t)min((m0 >> 4) + j, MB - 1) * nsteps * 1024 + lane * 8;
-    const size_t wo = (size_t)min((n0 >> 4) + j, NB - 1) * nsteps * WB + lane * WL;
+  for (int j = 0; j < MB; ++j) xr[j] = p.X + (size_t)min((m0 >> 4) + j, MBL - 1) * nsteps * 1024 + lane * 8;
+#pragma unroll
+  for (int j = 0; j < NB; ++j) {
+    const size_t wo = (size_t)min((n0 >> 4) + j, NBL - 1) * nsteps * WB + lane * WL;
     wr[j] = (const char*)p.W + wo;
     vr[j] = DUAL ? (const char*)W2 + wo : (const char*)p.W + wo;
   }
-  pf_floatx4 acc[2][2], acc2[2][2];
+  pf_floatx4 acc[NB][MB], acc2[NB][MB];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < NB; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) { acc[i][j] = pf_floatx4{0.f, 0.f, 0.f, 0.f}; acc2[i][j] = acc[i][j]; }
+    for (int j = 0; j < MB; ++j) { acc[i][j] = pf_floatx4{0.f, 0.f, 0.f, 0.f}; acc2[i][j] = acc[i][j]; }
   // the residual values this thread will add to (its four outputs, see the epilogue) are requested with the first
   // operands instead of after the last product; clamped to the matrix, unused where the thread has no output
   uint2 old = make_uint2(0, 0);
   if (EPI == PF_RESID) {
-    const int em = min(m0 + 16 * (wave & 1) + l16, p.M - 1), en = min(n0 + 16 * (wave >> 1) + 4 * kg, p.N - 4);
+    const int em = min(m0 + 16 * (wave % MB) + l16, p.M - 1), en = min(n0 + 16 * (wave / MB % NB) + 4 * kg, p.N - 4);
     old = *reinterpret_cast<const uint2*>((const bf16_t*)p.C + (c_tiled ? pf_toff(em, en, p.N) : (size_t)em * p.ldc + en));
   }
   for (int s = s0; s < s1; ++s) {
     const int k = s << 10;
-    uint4 xa[2][2], wa[2][2], va[2][2];
+    uint4 xa[MB][2], wa[NB][2], va[NB][2];
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) xa[j][h] = *reinterpret_cast<const uint4*>(xr[j] + k + 512 * h);
+      for (int j = 0; j < MB; ++j) xa[j][h] = *reinterpret_cast<const uint4*>(xr[j] + k + 512 * h);
     if (I8) {
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
+      for (int j = 0; j < NB; ++j) {
         const uint4 w8 = *reinterpret_cast<const uint4*>(wr[j] + (size_t)s * WB);
-        wa[j][0] = pf_widen8(w8.x, w8.y); wa[j][1] = pf_widen8(w8.z, w8.w);
+        wa[j][0] = widen8_i8(w8.x, w8.y); wa[j][1] = widen8_i8(w8.z, w8.w);
         if (DUAL) {
           const uint4 v8 = *reinterpret_cast<const uint4*>(vr[j] + (size_t)s * WB);
-          va[j][0] = pf_widen8(v8.x, v8.y); va[j][1] = pf_widen8(v8.z, v8.w);
+          va[j][0] = widen8_i8(v8.x, v8.y); va[j][1] = widen8_i8(v8.z, v8.w);
         }
       }
     } else {
 #pragma unroll
       for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
+        for (int j = 0; j < NB; ++j) {
           wa[j][h] = *reinterpret_cast<const uint4*>(wr[j] + (size_t)s * WB + 1024 * h);
           if (DUAL) va[j][h] = *reinterpret_cast<const uint4*>(vr[j] + (size_t)s * WB + 1024 * h);
         }
@@ -131,31 +122,37 @@ __global__ __launch_bounds__(256) void pf_gemm4_kernel(const PfGemm p, const voi
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < NB; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
+        for (int j = 0; j < MB; ++j) {
           acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf_frag(wa[i][h]), pf_frag(xa[j][h]), acc[i][j], 0, 0, 0);
           if (DUAL) acc2[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf_frag(va[i][h]), pf_frag(xa[j][h]), acc2[i][j], 0, 0, 0);
         }
   }
   // partial tiles to LDS: [wave][(i, j)][lane] as float4
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < NB; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      *reinterpret_cast<pf_floatx4*>(&part[wave * PW + ((i * 2 + j) * 64 + lane) * 4]) = acc[i][j];
-      if (DUAL) *reinterpret_cast<pf_floatx4*>(&part[wave * PW + TILE + ((i * 2 + j) * 64 + lane) * 4]) = acc2[i][j];
+    for (int j = 0; j < MB; ++j) {
+      *reinterpret_cast<pf_floatx4*>(&part[wave * PW + ((i * MB + j) * 64 + lane) * 4]) = acc[i][j];
+      if (DUAL) *reinterpret_cast<pf_floatx4*>(&part[wave * PW + TILE + ((i * MB + j) * 64 + lane) * 4]) = acc2[i][j];
     }
   __syncthreads();
-  // thread: sub-tile (i, j) = its wave's two bits, features n0 + 16 i + 4 kg + r (r = 0..3) of row m0 + 16 j + l16
-  const int i = wave >> 1, j = wave & 1;
+  if (wave >= MB * NB) return;
+  // thread: sub-tile (i, j) of its wave, features n0 + 16 i + 4 kg + r (r = 0..3) of row m0 + 16 j + l16
+  const int i = wave / MB, j = wave % MB;
   const int m = m0 + 16 * j + l16, n = n0 + 16 * i + 4 * kg;
   float v[4], u[4];
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int e = tid * 4 + r;
-    v[r] = ((part[e] + part[PW + e]) + part[2 * PW + e]) + part[3 * PW + e];
-    if (DUAL) u[r] = ((part[TILE + e] + part[PW + TILE + e]) + part[2 * PW + TILE + e]) + part[3 * PW + TILE + e];
+    v[r] = part[e];
+    if (DUAL) u[r] = part[TILE + e];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) {
+      v[r] += part[w * PW + e];
+      if (DUAL) u[r] += part[w * PW + TILE + e];
+    }
   }
   if (m >= p.M || n >= p.N) return;
   if (I8) {  // y[n] = scale[n] * sum_k q[n, k] x[k]
@@ -180,6 +177,87 @@ __global__ __launch_bounds__(256) void pf_gemm4_kernel(const PfGemm p, const voi
   }
   if (n + 3 < p.N) *reinterpret_cast<uint2*>(c) = make_uint2(f2bf2(v[0], v[1]), f2bf2(v[2], v[3]));
   else for (int r = 0; r < 4; ++r) if (n + r < p.N) c[r] = f2bf(v[r]);
+}
+
+// The same product for prompts of a few hundred positions and more: large tiles through LDS (wide.h).  DUAL: a wave's first
+// NBW / 2 blocks are features of the first matrix, the others the same features of the second.  The sums pass through
+// the wave's share of LDS, so that the epilogue is a loop over blocks.
+template <int EPI, bool DUAL, bool I8, int MBW, int NBW, int WM, int WN, int S, int KS>
+__global__ __launch_bounds__(256, 2) void pf_wide_kernel(const PfGemm p, const void* __restrict__ W2, int c_tiled) {
+  typedef WideTile<MBW, NBW, WM, WN, S, KS, I8> Tile;
+  constexpr int NF = DUAL ? NBW / 2 : NBW, MB = Tile::MB, NB = NF * WN;  // feature blocks of a wave and of the tile
+  __shared__ __align__(16) char lds[Tile::LDS];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int l16 = lane & 15, kg = lane >> 4, wm = wave % WM, wn = wave / WM;
+  const int MBL = (p.M + 15) >> 4, NBL = p.N >> 4, MT = (MBL + MB - 1) / MB;
+  const int mb0 = (int)blockIdx.x % MT * MB, nb0 = (int)blockIdx.x / MT * NB;
+  const size_t xb = (size_t)p.K * 32, wb = (size_t)p.K * (I8 ? 16 : 32);  // bytes of a 16-row block
+  Tile tile;
+  tile.begin(lds, wave, lane, [&](int i) { return (const char*)p.X + min(mb0 + i, MBL - 1) * xb; },
+             [&](int i) {
+               const int w = i / NBW, b = i % NBW;  // wave and block of the tile's i-th
+               return (const char*)(DUAL && b >= NF ? W2 : p.W) + min(nb0 + w * NF + b % NF, NBL - 1) * wb;
+             });
+  const int Q = p.K / (32 * KS);
+  tile.prologue(Q);
+  tl_f32x4 acc[NBW][MBW];
+  tile.run(Q, acc);
+  __syncthreads();
+  constexpr int ROOM = S * Tile::PIECES / 4;
+  static_assert(ROOM >= NBW * MBW, "a wave's sums fit its share");
+  char* own = lds + wave * ROOM * 1024 + lane * 16;
+#pragma unroll
+  for (int i = 0; i < NBW; ++i)
+#pragma unroll
+    for (int j = 0; j < MBW; ++j) *reinterpret_cast<tl_f32x4*>(own + (i * MBW + j) * 1024) = acc[i][j];
+#pragma unroll 1
+  for (int i = 0; i < NF; ++i) {
+    const int nb = nb0 + wn * NF + i, n = nb * 16 + 4 * kg, mw = (mb0 + wm * MBW) * 16 + l16;
+    if (nb >= NBL) break;
+    float s1[4], s2[4];
+    if (I8) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) { s1[r] = bf2f(p.sc[n + r]); if (DUAL) s2[r] = bf2f(p.sc2[n + r]); }
+    }
+    uint2 old[MBW];
+#pragma unroll
+    for (int j = 0; j < MBW; ++j) {
+      const int m = min(mw + 16 * j, p.M - 1);
+      if (EPI == PF_RESID) old[j] = *reinterpret_cast<const uint2*>((const bf16_t*)p.C + (c_tiled ? pf_toff(m, n, p.N) : (size_t)m * p.ldc + n));
+    }
+#pragma unroll
+    for (int j = 0; j < MBW; ++j) {
+      const int m = mw + 16 * j;
+      const tl_f32x4 a = *reinterpret_cast<const tl_f32x4*>(own + (i * MBW + j) * 1024);
+      float v[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = I8 ? a[r] * s1[r] : a[r];
+      if (DUAL) {  // rnd(rnd(silu(rnd(a))) * rnd(c)), src/vui/model.py:282
+        const tl_f32x4 c = *reinterpret_cast<const tl_f32x4*>(own + ((NF + i) * MBW + j) * 1024);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float g = bf2f(f2bf(v[r])), u = bf2f(f2bf(I8 ? c[r] * s2[r] : c[r]));
+          v[r] = bf2f(f2bf(g / (1.0f + expf(-g)))) * u;
+        }
+      }
+      if (EPI == PF_RESID) {  // x = rnd(x + rnd(y)), src/vui/model.py:367, 374
+        v[0] = bf_lo(old[j].x) + bf2f(f2bf(v[0])); v[1] = bf_hi(old[j].x) + bf2f(f2bf(v[1]));
+        v[2] = bf_lo(old[j].y) + bf2f(f2bf(v[2])); v[3] = bf_hi(old[j].y) + bf2f(f2bf(v[3]));
+      }
+      if (m < p.M) *reinterpret_cast<uint2*>((bf16_t*)p.C + (c_tiled ? pf_toff(m, n, p.N) : (size_t)m * p.ldc + n)) = make_uint2(f2bf2(v[0], v[1]), f2bf2(v[2], v[3]));
+    }
+  }
+}
+
+template <int EPI, bool DUAL, bool I8>
+static int pf_wide(int tile, const PfGemm& g, const void* W2, int c_tiled, hipStream_t st) {
+  const int bm = tile == WIDE_128 ? 128 : 64, bn = (tile == WIDE_64 ? 64 : 128) / (DUAL ? 2 : 1);
+  const dim3 grid((unsigned)((long)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn)));
+  if (tile == WIDE_128) hipLaunchKernelGGL((pf_wide_kernel<EPI, DUAL, I8, 4, 4, 2, 2, I8 ? 3 : 4, I8 ? 2 : 1>), grid, dim3(256), 0, st, g, W2, c_tiled);
+  else if (tile == WIDE_64x128) hipLaunchKernelGGL((pf_wide_kernel<EPI, DUAL, I8, 4, 2, 1, 4, I8 ? 4 : 3, 2>), grid, dim3(256), 0, st, g, W2, c_tiled);
+  else hipLaunchKernelGGL((pf_wide_kernel<EPI, DUAL, I8, 2, 2, 2, 2, 4, 2>), grid, dim3(256), 0, st, g, W2, c_tiled);
+  HIP_TRY(hipGetLastError());
+  return VUI_OK;
 }
 
 // two-rounding RMSNorm of rows (src/vui/model.py:286-297); one wave per row
@@ -406,16 +484,37 @@ __global__ void pf_set_len_kernel(int32_t* seq_lens, int slot, int v) { seq_lens
 // bf16 out, K split over the waves of a workgroup; W2 != nullptr: the SwiGLU pair; i8: int8 matrices with g.sc / g.sc2
 static int pf_gemm4(int epi, const PfGemm& g, const void* W2, int c_tiled, bool i8, hipStream_t st) {
   if (g.K % 64 || g.N % 16 || g.M < 1 || g.N < 1 || (c_tiled && g.N % 64)) { vui_set_error("prefill GEMM: bad shape N=%d K=%d", g.N, g.K); return VUI_EINVAL; }
-  const dim3 grid((unsigned)(((g.M + 31) / 32) * ((g.N + 31) / 32)));
-  if (i8) {
-    if (W2) hipLaunchKernelGGL((pf_gemm4_kernel<PF_BF16, true, true>), grid, dim3(256), 0, st, g, W2, c_tiled);
-    else if (epi == PF_RESID) hipLaunchKernelGGL((pf_gemm4_kernel<PF_RESID, false, true>), grid, dim3(256), 0, st, g, W2, c_tiled);
-    else hipLaunchKernelGGL((pf_gemm4_kernel<PF_BF16, false, true>), grid, dim3(256), 0, st, g, W2, c_tiled);
-  } else {
-    if (W2) hipLaunchKernelGGL((pf_gemm4_kernel<PF_BF16, true, false>), grid, dim3(256), 0, st, g, W2, c_tiled);
-    else if (epi == PF_RESID) hipLaunchKernelGGL((pf_gemm4_kernel<PF_RESID, false, false>), grid, dim3(256), 0, st, g, W2, c_tiled);
-    else hipLaunchKernelGGL((pf_gemm4_kernel<PF_BF16, false, false>), grid, dim3(256), 0, st, g, W2, c_tiled);
+  // The pair's epilogue weighs more in large tiles, and below 768 rows the K-splitting form is quicker than estimated (us at
+  // 576 positions, K-splitting / large tile: W1 and W3 13.4 / 14.9, QKV of int8 10.2 / 10.8).
+  const int tile = g.K >= 256 ? wide_pick(g.M, W2 ? 2 * g.N : g.N, g.K, W2 ? 0.4 : g.M < 768 ? 0.6 : 0.85) : WIDE_NONE;
+  if (tile != WIDE_NONE) {
+    if (W2) return i8 ? pf_wide<PF_BF16, true, true>(tile, g, W2, c_tiled, st) : pf_wide<PF_BF16, true, false>(tile, g, W2, c_tiled, st);
+    if (epi == PF_RESID) return i8 ? pf_wide<PF_RESID, false, true>(tile, g, W2, c_tiled, st) : pf_wide<PF_RESID, false, false>(tile, g, W2, c_tiled, st);
+    return i8 ? pf_wide<PF_BF16, false, true>(tile, g, W2, c_tiled, st) : pf_wide<PF_BF16, false, false>(tile, g, W2, c_tiled, st);
   }
+  // Few tiles (short blocks): more waves, so that a wave's chain of dependent trips is one to three steps long, and 16
+  // features per workgroup, so that more of the chip pulls weights.  us per launch, 32 x 32 and 4 waves / as chosen here:
+  // 16 positions out_proj and W2 8.0 / 4.4, QKV 5.6 / 3.8, W1 and W3 5.9 / 5.0; whole pass of 16 positions 883 / 776
+  // (int8 902 / 745), of 230 positions 1069 / 1060 (1013 / 931).
+  const long t32 = (long)((g.M + 31) / 32) * ((g.N + 31) / 32);
+  const bool some = t32 <= 256 && g.K >= 512, few = some && t32 <= 128;
+  const int mb = few && g.M <= 16 ? 1 : 2, nb = few ? 1 : 2;
+  const unsigned tiles = (unsigned)(((g.M + 16 * mb - 1) / (16 * mb)) * ((g.N + 16 * nb - 1) / (16 * nb)));
+#define PF_GO(E, D, Q, W, MB, NB) hipLaunchKernelGGL((pf_gemm_kernel<E, D, Q, W, MB, NB>), dim3(tiles), dim3(64 * (W)), 0, st, g, W2, c_tiled)
+#define PF_SIZE(E, D, Q, W) \
+  do { \
+    if (!some) PF_GO(E, D, Q, 4, 2, 2); \
+    else if (!few) PF_GO(E, D, Q, (D ? 8 : 12), 2, 2); \
+    else if (mb == 1) PF_GO(E, D, Q, W, 1, 1); \
+    else PF_GO(E, D, Q, W, 2, 1); \
+  } while (0)
+#define PF_PICK(E, D, W) do { if (i8) PF_SIZE(E, D, true, W); else PF_SIZE(E, D, false, W); } while (0)
+  if (W2) PF_PICK(PF_BF16, true, 12);
+  else if (epi == PF_RESID) PF_PICK(PF_RESID, false, 16);
+  else PF_PICK(PF_BF16, false, 12);
+#undef PF_PICK
+#undef PF_SIZE
+#undef PF_GO
   HIP_TRY(hipGetLastError());
   return VUI_OK;
 }
