@@ -268,3 +268,28 @@ def test_trace_replay_bookkeeping(tmp_path):
 
     assert read(0) == [[1, 7, 3], [1, 5, 3]] and not (tmp_path / "1.f32").exists()
     assert read(2) == [[2, 9, 1], [3, 2, 2]] and read(3) == [[4, 4, 1]]  # 'a' ended: the name starts anew
+
+
+def test_slots_are_written_once_for_the_same_rows():
+    """decode_step tells the device its rows' slots only when they change, and again after a narrower replay padded them."""
+    from vui_amd.slots import SlotEngine
+
+    class Fake(SlotEngine):
+        def __init__(self):
+            self.max_rows, self.device = 4, torch.device("cpu")
+            self.seq_lens = torch.zeros(5, dtype=torch.int32)
+            self._setup_slots(8)
+
+        class _G:
+            def replay(self):
+                pass
+
+    e = Fake()
+    e._bucketed_graphs = {b: Fake._G() for b in e._buckets}
+    e._set_active_slots([2, 0, 3])
+    e._replay_bucket(3, None)
+    assert e._held == [2, 0, 3] and e._g_slot_idx.tolist() == [2, 0, 3, 4] and e._g_seq_inc.tolist() == [1, 0, 1, 1, 0]
+    e._replay_bucket(2, None)  # writes nothing over the first two: the bucket of two is full
+    assert e._held is None
+    e._set_active_slots([1])
+    assert e._held == [1] and e._g_seq_inc.tolist() == [0, 1, 0, 0, 0]

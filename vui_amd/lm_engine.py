@@ -129,7 +129,9 @@ class TokenEngine(SlotEngine):
     def decode_step(self, rows: "list[TokenRow]", tokens: Tensor) -> Tensor:
         """One token for each row (B) through the bucketed captured step; a view of the static logits (B, vocab)."""
         self._room(rows, 1)
-        self._set_active_slots([r.idx for r in rows])
+        slots = [r.idx for r in rows]
+        if slots != self._held:  # the same rows as in the step before: nothing to tell the device (60 us of a 240 us step)
+            self._set_active_slots(slots)
         self._g_tokens[:len(rows)] = tokens
         self._replay_bucket(len(rows), self._decode_body)
         for r in rows:

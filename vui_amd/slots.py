@@ -43,6 +43,7 @@ class SlotEngine:
         self._buckets = _make_buckets(self.max_rows)
         self._g_slot_idx = torch.full((self._buckets[-1],), self._pad_slot, device=dev, dtype=torch.int32)
         self._g_seq_inc = torch.zeros(self.max_rows + 1, device=dev, dtype=torch.int32)
+        self._held: "list[int] | None" = None  # the slots that _set_active_slots left in the two tensors above
         self._bucketed_graphs: dict[int, Graph] = {}
         self._free: set[int] = set(range(self.max_rows))
         self._rows: dict = {}
@@ -95,7 +96,10 @@ class SlotEngine:
         replay that bucket's graph (captured on first use with every row on the padding slot).  body(B, stream)
         enqueues the step of B rows.  run=False: only the capture, where it is missing.  Returns the bucket."""
         B_bucket = self._bucket(B_active)
-        self._g_slot_idx[B_active:B_bucket].fill_(self._pad_slot)
+        if B_active < B_bucket:
+            self._g_slot_idx[B_active:B_bucket].fill_(self._pad_slot)
+        if self._held is not None and B_active < len(self._held):
+            self._held = None
         g = self._bucketed_graphs.get(B_bucket)
         if g is None:
             saved_idx, saved_inc = self._g_slot_idx.clone(), self._g_seq_inc.clone()
@@ -115,6 +119,7 @@ class SlotEngine:
         self._g_slot_idx[:len(slots)] = t
         self._g_seq_inc.zero_()
         self._g_seq_inc[t.long()] = 1
+        self._held = list(slots)
         return t
 
     # ------------------------------------------------------------------ repetition penalty
