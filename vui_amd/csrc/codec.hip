@@ -99,11 +99,10 @@ template <bool NT> __device__ __forceinline__ float4 cv_ld_w(const float* p) {
 // round use the single-buffered form, which leaves room for two or three waves per SIMD.
 template <int TT, bool DB> struct Nu { static constexpr int N = TT == 1 ? 8 : (TT == 2 ? (DB ? 5 : 6) : 3); };
 
-#define CV_NW 4  // waves per workgroup
 #define CV_WIDE_T 64  // columns from which cv_wide_kernel takes a product of several frames
 
-// One 16-row x 16*TT-column output tile.  `red` is CV_NW * TT * 64 * 4 floats of LDS.
-template <int TT, bool DB, bool NT>
+// One 16-row x 16*TT-column output tile of NW waves.  `red` is NW * TT * 64 * 4 floats of LDS.
+template <int TT, bool DB, bool NT, int NW>
 __device__ __forceinline__ void cv_gemm_tile(const CvGemm& p, const int m0, const int t0, float* red,
                                              const int tile, const int part_idx) {
   constexpr int NU = Nu<TT, DB>::N;
@@ -115,7 +114,7 @@ __device__ __forceinline__ void cv_gemm_tile(const CvGemm& p, const int m0, cons
   // its 16 weight rows, 128 bytes of each per unit
   const int per = (Uall + p.splits - 1) / p.splits;
   const int wb = part_idx * per, we = min(Uall, wb + per);
-  const int per_wave = (we - wb + CV_NW - 1) / CV_NW;
+  const int per_wave = (we - wb + NW - 1) / NW;
   const int ub = min(we, wb + wave * per_wave), U = min(we, ub + per_wave);
 
   float4 a0[NU][2], a1[DB ? NU : 1][2];
@@ -252,7 +251,7 @@ __device__ __forceinline__ void cv_gemm_tile(const CvGemm& p, const int m0, cons
   float v[4] = {0.f, 0.f, 0.f, 0.f};
   if (tid < TT * 64) {
 #pragma unroll
-    for (int w = 0; w < CV_NW; ++w) {
+    for (int w = 0; w < NW; ++w) {
       const float4 q = *reinterpret_cast<const float4*>(red + ((size_t)w * TT * 64 + tid) * 4);
       v[0] += q.x; v[1] += q.y; v[2] += q.z; v[3] += q.w;
     }
@@ -318,14 +317,14 @@ __device__ __forceinline__ void cv_gemm_tile(const CvGemm& p, const int m0, cons
 }
 
 template <int TT, bool NT>
-__global__ __launch_bounds__(CV_NW * 64) void cv_gemm_kernel(const CvGemm p) {
-  __shared__ __align__(16) float red[CV_NW * TT * 64 * 4];
-  cv_gemm_tile<TT, true, NT>(p, blockIdx.x * 16, blockIdx.y * (16 * TT), red, blockIdx.y * gridDim.x + blockIdx.x, blockIdx.z);
+__global__ __launch_bounds__(256) void cv_gemm_kernel(const CvGemm p) {
+  __shared__ __align__(16) float red[4 * TT * 64 * 4];
+  cv_gemm_tile<TT, true, NT, 4>(p, blockIdx.x * 16, blockIdx.y * (16 * TT), red, blockIdx.y * gridDim.x + blockIdx.x, blockIdx.z);
 }
-template <int TT, bool NT>
-__global__ __launch_bounds__(CV_NW * 64, 2) void cv_gemm1_kernel(const CvGemm p) {
-  __shared__ __align__(16) float red[CV_NW * TT * 64 * 4];
-  cv_gemm_tile<TT, false, NT>(p, blockIdx.x * 16, blockIdx.y * (16 * TT), red, blockIdx.y * gridDim.x + blockIdx.x, blockIdx.z);
+template <int TT, bool NT, int NW>
+__global__ __launch_bounds__(NW * 64, 2) void cv_gemm1_kernel(const CvGemm p) {
+  __shared__ __align__(16) float red[NW * TT * 64 * 4];
+  cv_gemm_tile<TT, false, NT, NW>(p, blockIdx.x * 16, blockIdx.y * (16 * TT), red, blockIdx.y * gridDim.x + blockIdx.x, blockIdx.z);
 }
 
 // ---- the same product for many columns (several frames at once) ----
@@ -1447,10 +1446,14 @@ static CvScratch cv_plan(CvGemm& g) {
   g.tt = 1;
   for (int tt : {2, 4})
     if (T > 8 * tt && tiles(tt) * tt <= tiles(g.tt) * g.tt) g.tt = tt;
+  // a tile of 64 columns holds 3 units per wave and round, one of 32 columns 6: the narrower one where that saves the second
+  // round (192 channels x 640 columns: 18.8 / 11.5 us)
+  if (g.tt == 4 && U > 24 && U <= 48 && tiles(2) <= 256) g.tt = 2;
   int sp = 1;
   if (U >= 64) {
     const int target = g.tt == 1 ? 512 : 200;
     sp = (2 * target + tiles(g.tt)) / (2 * tiles(g.tt));  // rounded
+    if (g.tt == 1 && sp < (U + 63) / 64) sp = (U + 63) / 64;  // eight waves of one round each
     if (sp > U / 16) sp = U / 16;
     if (sp > 8) sp = 8;
     if (sp < 1) sp = 1;
@@ -1869,25 +1872,26 @@ static int launch_cv_gemm(const CvGemm& g, bool w_nt, hipStream_t st) {
     return VUI_OK;
   }
   const dim3 grid(g.M / 16, (g.T + 16 * g.tt - 1) / (16 * g.tt), g.splits);
-  const dim3 block(64 * CV_NW);
-  // units a wave of one part works through; one single-buffered round holds 8 / 6 / 3 of them
-  const int U = g.taps * (g.Cin / 32), per_wave = ((U + g.splits - 1) / g.splits + CV_NW - 1) / CV_NW;
-  const bool one_round = per_wave <= (g.tt == 1 ? 8 : (g.tt == 2 ? 6 : 3));
-#define CV_LAUNCH(K, TT_)                                                                         \
-  do {                                                                                            \
-    if (w_nt) hipLaunchKernelGGL((K<TT_, true>), grid, block, 0, st, g);                          \
-    else hipLaunchKernelGGL((K<TT_, false>), grid, block, 0, st, g);                              \
+  // units a wave of one part works through; one single-buffered round holds 8 / 6 / 3 of them.  Eight waves where four need
+  // more than a round: a second round is a second trip to memory (dilated convs of one frame: 16-18 us with four waves).
+  const int U = g.taps * (g.Cin / 32), part = (U + g.splits - 1) / g.splits, round = g.tt == 1 ? 8 : (g.tt == 2 ? 6 : 3);
+#define CV_TT(TT_)                                                                                                   \
+  do {                                                                                                               \
+    if ((part + 3) / 4 <= round) {                                                                                   \
+      if (w_nt) hipLaunchKernelGGL((cv_gemm1_kernel<TT_, true, 4>), grid, dim3(256), 0, st, g);                      \
+      else hipLaunchKernelGGL((cv_gemm1_kernel<TT_, false, 4>), grid, dim3(256), 0, st, g);                          \
+    } else if ((part + 7) / 8 <= round) {                                                                            \
+      if (w_nt) hipLaunchKernelGGL((cv_gemm1_kernel<TT_, true, 8>), grid, dim3(512), 0, st, g);                      \
+      else hipLaunchKernelGGL((cv_gemm1_kernel<TT_, false, 8>), grid, dim3(512), 0, st, g);                          \
+    } else {                                                                                                         \
+      if (w_nt) hipLaunchKernelGGL((cv_gemm_kernel<TT_, true>), grid, dim3(256), 0, st, g);                          \
+      else hipLaunchKernelGGL((cv_gemm_kernel<TT_, false>), grid, dim3(256), 0, st, g);                              \
+    }                                                                                                                \
   } while (0)
-  if (one_round) {
-    if (g.tt == 1) CV_LAUNCH(cv_gemm1_kernel, 1);
-    else if (g.tt == 2) CV_LAUNCH(cv_gemm1_kernel, 2);
-    else CV_LAUNCH(cv_gemm1_kernel, 4);
-  } else {
-    if (g.tt == 1) CV_LAUNCH(cv_gemm_kernel, 1);
-    else if (g.tt == 2) CV_LAUNCH(cv_gemm_kernel, 2);
-    else CV_LAUNCH(cv_gemm_kernel, 4);
-  }
-#undef CV_LAUNCH
+  if (g.tt == 1) CV_TT(1);
+  else if (g.tt == 2) CV_TT(2);
+  else CV_TT(4);
+#undef CV_TT
   return VUI_OK;
 }
 
