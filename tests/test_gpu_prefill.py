@@ -94,6 +94,27 @@ def test_prefill_window_and_errors():
         m.decoder.forward_flash(torch.zeros(1, 300, d.d_model, dtype=BF, device="cuda"), None)
 
 
+@pytest.mark.parametrize("window,kv", [(0, 2), (33, 4), (70, 2), (130, 1)])
+def test_prefill_attention_masks(window, kv):
+    """Steps of 32 keys that no query, some queries and all queries of a tile see, from both ends of a sliding window and
+    from a second portion that starts inside a step; grouped KV heads.  Against the position-by-position path."""
+    from tests.util import dims_to_config
+    from vui_amd.model import Vui
+
+    d = _dims(kv)
+    cfg = dims_to_config(d, 256)
+    cfg.model.window_size = window or None
+    m = Vui(cfg, O.synthetic_state_dict(d, **TINY_SD), device="cuda", dtype=BF)
+    m.decoder.allocate_flash_kv_cache(1, m.device, BF)
+    emb = (torch.randn(1, 234, d.d_model, generator=torch.Generator().manual_seed(6)) * 0.5).to(BF).cuda()
+    outs = []
+    for minimum in (4, 10 ** 9):
+        m.decoder.PREFILL_MIN = minimum
+        m.decoder.flash_kv_caches[0].seq_lens.zero_()
+        outs.append(torch.cat([m.decoder.forward_flash(emb[:, a:b].contiguous(), None) for a, b in ((0, 173), (173, 234))], dim=1))
+    assert rel_err(outs[0], outs[1]) <= BF16_TOL, rel_err(outs[0], outs[1])
+
+
 @pytest.mark.parametrize("int8", [False, True])
 def test_prefill_nano_576_positions(int8):
     """The benchmark's prompt (512 audio frames + 64 text tokens) at Vui Nano dims, with bf16 and with weight-only

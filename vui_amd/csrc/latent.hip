@@ -346,18 +346,23 @@ __global__ __launch_bounds__(512) void latent_value_kernel(const LatentArgs p, i
 // Waves take 32 keys at a time in turn.  Scores^T (keys x queries) = K q^T leave a lane with eight keys of one query,
 // which is operand layout for out^T = V^T p^T; the fp32 weights go in as a bf16 pair (value and remainder), so the
 // average keeps about 16 bits of them.  DB = dim64 / 64, RB = rot32 / 32, VT >= vdim16 / 16.
+// Bound by the keys and values that every tile of queries fetches from L2 (16 heads of 128 + 64 and 128, 1999 positions:
+// 1.7 GB in 56 us).  Neighbouring workgroups take different heads, so that an XCD's L2 holds few of them (68 -> 56 us);
+// masks and the rescaling of the sums only in the steps that need them (73 -> 68 us).  Two tiles of queries per wave: 47 us
+// there, but 11.4 instead of 8.2 us at 600 positions of eight heads, and nothing of it in the whole prompt's time.
 #define LPF_WAVES (VT <= 4 ? 8 : 4)
 template <int DB, int RB, int VT>
-__global__ __launch_bounds__(64 * LPF_WAVES) void latent_prefill_kernel(const LatentArgs p) {
+__global__ __launch_bounds__(64 * LPF_WAVES, 2) void latent_prefill_kernel(const LatentArgs p) {
   __shared__ __align__(16) float s_acc[LPF_WAVES][VT * 256];
   __shared__ float s_m[LPF_WAVES][16], s_l[LPF_WAVES][16];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int l16 = lane & 15, kg = lane >> 4;
-  const int qt = gridDim.x - 1 - blockIdx.x, h = blockIdx.y;  // the tiles with the most keys start first
+  const int qt = gridDim.y - 1 - blockIdx.y, h = blockIdx.x;  // the tiles with the most keys start first
   const int q0 = qt * 16, T = p.M, pos0 = p.rows.pos0;
   const int nvb = p.d.vdim16 >> 4;
   const int qlast = pos0 + min(q0 + l16, T - 1);  // last visible key of this lane's query
   const int kend = pos0 + min(q0 + 15, T - 1) + 1;
+  const float ls = p.scale * 1.44269504088896f;  // weights are powers of two, one v_exp_f32 each
   const bf16_t* qu = (const bf16_t*)p.qu + h * p.qu_z + (size_t)qt * DB * 1024 + lane * 8;
   const bf16_t* qr = (const bf16_t*)p.qr + h * p.qr_z + (size_t)qt * RB * 512 + lane * 8;
   uint4 qf[2 * DB + RB];
@@ -392,35 +397,41 @@ __global__ __launch_bounds__(64 * LPF_WAVES) void latent_prefill_kernel(const La
       sc[t] = tl_f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int i = 0; i < 2 * DB + RB; ++i) sc[t] = Tl<bf16_t>::mma(kf[t][i], qf[i], sc[t]);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sc[t][r] *= ls;
     }
-    float sv[8], mx = -INFINITY;
+    if (k0 + 31 > pos0 + q0) {  // a key that some query of the tile does not see
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+      for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int j = k0 + 16 * t + 4 * kg + r;
-        const float v = j <= qlast ? sc[t][r] * p.scale : -INFINITY;
-        sv[4 * t + r] = v;
-        mx = fmaxf(mx, v);
-      }
+        for (int r = 0; r < 4; ++r)
+          if (k0 + 16 * t + 4 * kg + r > qlast) sc[t][r] = -INFINITY;
+    }
+    float mx = fmaxf(sc[0][0], sc[1][0]);
+#pragma unroll
+    for (int r = 1; r < 4; ++r) mx = fmaxf(mx, fmaxf(sc[0][r], sc[1][r]));
     mx = rows_max(mx);
     const float m_new = fmaxf(m_run, mx);
     const float m_use = m_new == -INFINITY ? 0.f : m_new;
-    const float alpha = expf(m_run - m_use);
+    const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
     float pv[8], lo[8], ps = 0.f;
     uint4 hi4, lo4;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) { pv[e] = expf(sv[e] - m_use); ps += pv[e]; }
+    for (int e = 0; e < 8; ++e) { pv[e] = __builtin_amdgcn_exp2f(sc[e >> 2][e & 3] - m_use); ps += pv[e]; }
     l_run = l_run * alpha + ps;
     m_run = m_new;
     hi4.x = f2bf2(pv[0], pv[1]); hi4.y = f2bf2(pv[2], pv[3]); hi4.z = f2bf2(pv[4], pv[5]); hi4.w = f2bf2(pv[6], pv[7]);
     lo[0] = pv[0] - bf_lo(hi4.x); lo[1] = pv[1] - bf_hi(hi4.x); lo[2] = pv[2] - bf_lo(hi4.y); lo[3] = pv[3] - bf_hi(hi4.y);
     lo[4] = pv[4] - bf_lo(hi4.z); lo[5] = pv[5] - bf_hi(hi4.z); lo[6] = pv[6] - bf_lo(hi4.w); lo[7] = pv[7] - bf_hi(hi4.w);
     lo4.x = f2bf2(lo[0], lo[1]); lo4.y = f2bf2(lo[2], lo[3]); lo4.z = f2bf2(lo[4], lo[5]); lo4.w = f2bf2(lo[6], lo[7]);
+    if (__builtin_amdgcn_ballot_w64(alpha != 1.0f)) {  // few steps raise a maximum
+#pragma unroll
+      for (int d = 0; d < VT; ++d)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[d][r] *= alpha;
+    }
 #pragma unroll
     for (int d = 0; d < VT; ++d) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) acc[d][r] *= alpha;
       acc[d] = Tl<bf16_t>::mma(vf[d], hi4, acc[d]);
       acc[d] = Tl<bf16_t>::mma(vf[d], lo4, acc[d]);
     }
@@ -440,7 +451,7 @@ __global__ __launch_bounds__(64 * LPF_WAVES) void latent_prefill_kernel(const La
     float den = 0.f, o[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 0; w < LPF_WAVES; ++w) {
-      const float f = s_m[w][q] == -INFINITY ? 0.f : expf(s_m[w][q] - M);
+      const float f = s_m[w][q] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(s_m[w][q] - M);
       den = fmaf(f, s_l[w][q], den);
 #pragma unroll
       for (int r = 0; r < 4; ++r) o[r] = fmaf(f, s_acc[w][sl * 4 + r], o[r]);
@@ -530,7 +541,7 @@ bool latent_expand_ok(const vui_lm_dims& d) { return d.dim64 <= 128 && d.rot32 <
 
 template <int DB, int RB>
 static void lpf_go(const LatentArgs& a, hipStream_t st) {
-  const dim3 grid((a.M + 15) / 16, a.heads);
+  const dim3 grid(a.heads, (a.M + 15) / 16);
   if (a.d.vdim16 <= 32) hipLaunchKernelGGL((latent_prefill_kernel<DB, RB, 2>), grid, dim3(512), 0, st, a);
   else if (a.d.vdim16 <= 64) hipLaunchKernelGGL((latent_prefill_kernel<DB, RB, 4>), grid, dim3(512), 0, st, a);
   else hipLaunchKernelGGL((latent_prefill_kernel<DB, RB, 8>), grid, dim3(256), 0, st, a);

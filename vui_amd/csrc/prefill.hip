@@ -310,9 +310,14 @@ __device__ __forceinline__ uint4 pf_rope8(uint4 v, const float* __restrict__ rop
 // rows; the probabilities, rounded to bf16, are then already in operand layout for out^T (dims x queries) =
 // V^T p^T, with V^T read from the transposed copy in the same key order (any assignment of k to lanes is valid
 // when both operands share it).  HD32 = head_dim / 32.
+// Bound by the keys and values that every tile of queries fetches from L2 and by the instructions around the weights.
+// Neighbouring workgroups take different heads, so that an XCD's L2 holds the keys and values of few (eight heads of 96,
+// 1733 positions: 22 -> 16.3 us, all heads together are 5.3 MB); weights are one fma and one v_exp_f32, masks and the
+// rescaling of the sums only in the steps that need them (25.2 -> 22 us; at 576 positions 9.4 -> 6.3 us with both).
+// Two tiles of queries per wave or per workgroup, which halves the fetches, measured the same at 1733 and slower below.
 #define PF_ATT_WAVES (HD32 <= 3 ? 8 : 4)  // the partial outputs of the waves must fit 64 KiB of LDS
 template <int HD32>
-__global__ __launch_bounds__(64 * PF_ATT_WAVES) void pf_attn_kernel(const bf16_t* __restrict__ qkv, const bf16_t* __restrict__ kt,
+__global__ __launch_bounds__(64 * PF_ATT_WAVES, 2) void pf_attn_kernel(const bf16_t* __restrict__ qkv, const bf16_t* __restrict__ kt,
                                                       const bf16_t* __restrict__ vt, bf16_t* __restrict__ att, int T, int L,
                                                       int Lpad, int nq, int nkv, int gsz, int pos0, int window, float scale) {
   constexpr int HD = 32 * HD32, DT = 2 * HD32;
@@ -320,7 +325,9 @@ __global__ __launch_bounds__(64 * PF_ATT_WAVES) void pf_attn_kernel(const bf16_t
   __shared__ float s_m[PF_ATT_WAVES][16], s_l[PF_ATT_WAVES][16];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int l16 = lane & 15, kg = lane >> 4;
-  const int q0 = blockIdx.x * 16, h = blockIdx.y, kvh = h / gsz;
+  // neighbouring workgroups take different KV heads (one XCD meets few of them); the tiles with the most keys start first
+  const int nkvh = gridDim.x / gsz, kvh = blockIdx.x % nkvh, h = kvh * gsz + blockIdx.x / nkvh;
+  const int q0 = (gridDim.y - 1 - blockIdx.y) * 16;
   const int ldq = nq + 2 * nkv;
   // this lane's query (column of every product below)
   const int tq = min(q0 + l16, T - 1);
@@ -334,6 +341,9 @@ __global__ __launch_bounds__(64 * PF_ATT_WAVES) void pf_attn_kernel(const bf16_t
   const int t_hi = min(q0 + 15, T - 1);
   const int kend = pos0 + t_hi + 1;
   const int kbeg = (window > 0 ? max(0, pos0 + q0 - window) : 0) & ~31;
+  // steps that start in [kall, kmid) are visible to every query of the tile
+  const int kall = window > 0 ? max(0, pos0 + t_hi - window) : 0, kmid = pos0 + q0 - 30;
+  const float ls = scale * 1.44269504088896f;  // weights are 2^(ls * score - m): one fma and one v_exp_f32 each
   // staged keys / values of this KV head (pf_stage_kv_kernel): a fragment is 16 bytes per lane, 1 KiB contiguous per wave
   const bf16_t* kb = kt + (size_t)kvh * (Lpad >> 4) * HD32 * 512 + lane * 8;
   const bf16_t* vb = vt + (size_t)kvh * DT * (Lpad >> 5) * 512 + lane * 8;
@@ -365,33 +375,37 @@ __global__ __launch_bounds__(64 * PF_ATT_WAVES) void pf_attn_kernel(const bf16_t
         sc[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf_frag(kf[kt][c]), pf_frag(qf[c]), sc[kt], 0, 0, 0);
     }
     // the lane holds keys k0 + 16 kt + 4 kg + r of its query
-    float sv[8], mx = -INFINITY;
+    if (k0 < kall || k0 >= kmid) {
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
+      for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int j = k0 + 16 * kt + 4 * kg + r;
-        const float v = (j >= qfirst && j <= qlast) ? sc[kt][r] * scale : -INFINITY;
-        sv[4 * kt + r] = v;
-        mx = fmaxf(mx, v);
-      }
+        for (int r = 0; r < 4; ++r) {
+          const int j = k0 + 16 * kt + 4 * kg + r;
+          if (j < qfirst || j > qlast) sc[kt][r] = -INFINITY;
+        }
+    }
+    float mx = fmaxf(sc[0][0], sc[1][0]);
+#pragma unroll
+    for (int r = 1; r < 4; ++r) mx = fmaxf(mx, fmaxf(sc[0][r], sc[1][r]));
     mx = rows_max(mx);  // over the four lane rows: every key of the step for this query
-    const float m_new = fmaxf(m_run, mx);
+    const float m_new = fmaxf(m_run, mx * ls);
     const float m_use = (m_new == -INFINITY) ? 0.f : m_new;  // nothing visible yet: every weight below is zero
-    const float alpha = expf(m_run - m_use);                  // 0 on the first visible step (m_run = -inf)
+    const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);  // 0 on the first visible step (m_run = -inf)
     float pv[8], ps = 0.f;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) { pv[e] = expf(sv[e] - m_use); ps += pv[e]; }
+    for (int e = 0; e < 8; ++e) { pv[e] = __builtin_amdgcn_exp2f(fmaf(sc[e >> 2][e & 3], ls, -m_use)); ps += pv[e]; }
     l_run = l_run * alpha + ps;
     m_run = m_new;
     uint4 pf;
     pf.x = f2bf2(pv[0], pv[1]); pf.y = f2bf2(pv[2], pv[3]); pf.z = f2bf2(pv[4], pv[5]); pf.w = f2bf2(pv[6], pv[7]);
+    if (__builtin_amdgcn_ballot_w64(alpha != 1.0f)) {  // few steps raise a maximum
 #pragma unroll
-    for (int d = 0; d < DT; ++d) {
+      for (int d = 0; d < DT; ++d)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) acc[d][r] *= alpha;
-      acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf_frag(vf[d]), pf_frag(pf), acc[d], 0, 0, 0);
+        for (int r = 0; r < 4; ++r) acc[d][r] *= alpha;
     }
+#pragma unroll
+    for (int d = 0; d < DT; ++d) acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf_frag(vf[d]), pf_frag(pf), acc[d], 0, 0, 0);
   }
   // the waves' parts meet: lane holds dims 16 d + 4 kg + r of query l16
   l_run = rows_sum(l_run);
@@ -409,7 +423,7 @@ __global__ __launch_bounds__(64 * PF_ATT_WAVES) void pf_attn_kernel(const bf16_t
     float den = 0.f, o[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 0; w < PF_ATT_WAVES; ++w) {
-      const float f = (s_m[w][q] == -INFINITY) ? 0.f : expf(s_m[w][q] - M);
+      const float f = (s_m[w][q] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(s_m[w][q] - M);
       den = fmaf(f, s_l[w][q], den);
 #pragma unroll
       for (int r = 0; r < 4; ++r) o[r] = fmaf(f, s_acc[w][sl * 4 + r], o[r]);
@@ -627,7 +641,7 @@ int launch_prefill(const vui_config& c, const vui_weights& w, const void* tiled_
     hipLaunchKernelGGL(pf_stage_kv_kernel, dim3(Lpad / 32, (nkv + nq) / 32), dim3(256), 0, st, qkv, krow, vrow, kt, vt, rope_l, L, Lpad, nq, nkv,
                        hd, rope_dim_l, pos0);
     {
-      const dim3 grid((T + 15) / 16, H);
+      const dim3 grid(H, (T + 15) / 16);
       switch (hd / 32) {
         case 1: hipLaunchKernelGGL(pf_attn_kernel<1>, grid, dim3(512), 0, st, qkv, kt, vt, att, T, L, Lpad, nq, nkv, H / KV, pos0, window_l, scale); break;
         case 2: hipLaunchKernelGGL(pf_attn_kernel<2>, grid, dim3(512), 0, st, qkv, kt, vt, att, T, L, Lpad, nq, nkv, H / KV, pos0, window_l, scale); break;
