@@ -495,11 +495,14 @@ static int go(const LmGemm& g, int nz, hipStream_t st) {
   return VUI_OK;
 }
 
-// Tile of a prompt's product (wide_pick); a minGRU projection takes 128 x 192, with 20 us more in the epilogue
+// Tile of a prompt's product (wide_pick).  The K-splitting kernel is counted 1.5 times: 28.4 against 23 us at 650 x 1024 x 4608
+// with 18.4 estimated.  Whole prompts with 0.85 / 1.2 / 1.5 / 2 of the estimate, us: latent models of 2048 x 400 positions
+// 1033 / 869 / 865 / 870 and of 1024 x 900 760 / 701 / 691 / 697, x 500 487 / 487 / 497 / 553; experts of 2048 x 300
+// 1463 / 1404 / 1311 / 1320.  A minGRU projection takes 128 x 192, with 20 us more in the epilogue
 // (us, K-splitting / large tile: 160 / 98 at 1024 x 14336 x 2048, 30 / 35 at 1024 x 6400 x 768).
 static int lm_tile(int epi, int M, int N, int K) {
   double us;
-  const int t = wide_pick(M, N, K, 0.85, &us);
+  const int t = wide_pick(M, N, K, 1.5, &us);
   if (epi != LM_IN_GRU_SEQ) return t;
   const double work = (double)(((M + 127) / 128 * ((N + 191) / 192) + 255) / 256) * 0.2;
   return M >= 128 && 20 + (K / 32) * (work > 0.4 ? work : 0.4) < us ? WIDE_128 : WIDE_NONE;
