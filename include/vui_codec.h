@@ -53,8 +53,8 @@ int32_t vui_codec_hop(const vui_codec_config* cfg);
  * decoder.*; qwen_codec.py:1087-1125). */
 int32_t vui_codec_n_tensors(const vui_codec_config* cfg);
 
-/* Bytes of workspace: repacked weights (one copy, tap-major), activation rings, the buffers of a block of
- * frames, the pre-transformer cache, tables and counters. */
+/* Bytes of workspace: repacked weights (one copy, tap-major), activation rings, the pre-transformer cache,
+ * tables and counters. */
 int64_t vui_codec_workspace_bytes(const vui_codec_config* cfg);
 
 /* Builds a decoder: repacks the fp32 tensors (reference layouts: Conv1d (out, in, k),
@@ -82,9 +82,13 @@ int32_t vui_codec_block_frames(const vui_codec* c);
 /* n_frames consecutive frames in one pass: codes (n_frames, n_q) int64 -> audio_out (n_frames * hop), the samples that
  * as many vui_codec_decode_frame calls give (sums in another order), and the same state behind them, so that blocks and
  * single frames may follow each other.  Every weight is read once per block.  The block must fit in front of max_seq:
- * one that does not raises the status flag and its samples are not the frames' own.  No counterpart in the reference,
+ * one that does not raises the status flag and its samples are not the frames' own.  scratch: device memory of
+ * vui_codec_block_scratch_bytes(cfg) bytes (the block's activations, 257 MB at the reference's dims), 256-byte aligned,
+ * used only by this call (it holds nothing between calls; not needed for one frame).  No counterpart in the reference,
  * whose offline forward (qwen_codec.py:1191-1224) takes all frames at once. */
-int vui_codec_decode_block(vui_codec* c, const int64_t* codes, int32_t n_frames, int32_t n_q, float* audio_out, vui_stream_t stream);
+int64_t vui_codec_block_scratch_bytes(const vui_codec_config* cfg);
+int vui_codec_decode_block(vui_codec* c, const int64_t* codes, int32_t n_frames, int32_t n_q, float* audio_out, void* scratch,
+                           int64_t scratch_bytes, vui_stream_t stream);
 
 /* The one-column steps of a frame (codebook rows ... first upsampling conv) run as one persistent kernel when
  * the device can keep 256 workgroups resident and the dimensions fit, otherwise as separate launches (same

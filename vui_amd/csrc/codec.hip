@@ -1244,14 +1244,14 @@ __global__ void cv_fill_kernel(float* p, size_t n, float v) {
 }
 // The history columns of every ring into the buffer that stands for it during a block (out = 0), and those behind the
 // block's last frame back into the ring.
-struct CvHist { Ring ring, buf; int C; };
-__global__ void cv_history_kernel(const CvHist* h, const int* ctr, int nf, int out) {
+struct CvHist { Ring ring; size_t at; int rs, C; };  // at, rs: the buffer in the scratch memory of the block (floats), its row stride
+__global__ void cv_history_kernel(const CvHist* h, float* scratch, const int* ctr, int nf, int out) {
   const CvHist r = h[blockIdx.y];
   const int base = ring_base(r.ring, *ctr - (out ? 0 : nf)), at = out ? nf * r.ring.tstep : 0;
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < r.C * r.ring.pad; i += gridDim.x * blockDim.x) {
     const int c = i / r.ring.pad, t = i - c * r.ring.pad;
     float* ring = ring_ptr(r.ring, base, c, t);
-    float* buf = r.buf.p + (size_t)c * r.buf.rs + at + t;
+    float* buf = scratch + r.at + (size_t)c * r.rs + at + t;
     if (out) *ring = *buf; else *buf = *ring;
   }
 }
@@ -1273,8 +1273,11 @@ struct vui_codec {
   int64_t ws_bytes;
   float* state0;  // start of the zeroed-on-reset region (rings)
   size_t state_floats;
-  std::vector<Ring> twins;  // what stands for each ring and buffer while several frames are decoded at once
-  CvHist* hist;             // device: the rings and their twins
+  // what stands for each ring and buffer while several frames are decoded at once, in the caller's scratch memory
+  std::vector<Ring> twins;
+  std::vector<size_t> twin_at;  // floats from its start
+  int64_t block_bytes = 0;
+  CvHist* hist;                 // device: the rings and their twins
   int n_hist = 0;
   int* ctr;  // [0] frames started since reset, [1] error flag
   int* cnt;  // arrival counters of split tiles
@@ -1361,7 +1364,7 @@ struct Arena {
 };
 
 // Frames that one pass takes at most (vui_codec_decode_block).  At 32 the weights pass once per 32 frames (3 us of a
-// frame's 84) and a product's launch costs 0.15 us per frame; the buffers take 0.25 GB.
+// frame's 84) and a product's launch costs 0.15 us per frame; the buffers, scratch memory of the caller's, take 0.26 GB.
 #define CV_BLOCK 32
 static int block_frames(const vui_codec_config& k) { return k.max_seq < CV_BLOCK ? k.max_seq : CV_BLOCK; }
 
@@ -1372,7 +1375,7 @@ struct RingMaker {
   Arena& ar;
   int frames;
   std::vector<Ring> twins;
-  std::vector<size_t> floats;
+  std::vector<size_t> floats, at;
   std::vector<int> share;     // twins of one group >= 0 take turns in the same memory
   std::vector<CvHist> hist;
   Ring make(int C, int pad, int T, bool stream, int group = -1) {
@@ -1390,20 +1393,23 @@ struct RingMaker {
     twins.push_back(t);
     floats.push_back((size_t)C * t.rs + 256);  // a tile reads up to 256 columns behind the last channel's
     share.push_back(group);
-    if (stream && pad) hist.push_back(CvHist{r, t, C});
+    if (stream && pad) hist.push_back(CvHist{r, 0, t.rs, C});
     return r;
   }
-  void place() {  // once every ring is known
+  size_t place() {  // once every ring is known: the twins' places in the scratch memory, and its floats
+    size_t end = 0;
+    auto take = [&](size_t n) { const size_t o = end; end += (n + 63) & ~(size_t)63; return o; };
     std::vector<size_t> most;
     for (size_t i = 0; i < twins.size(); ++i)
       if (share[i] >= 0) {
         if ((int)most.size() <= share[i]) most.resize(share[i] + 1, 0);
         if (floats[i] > most[share[i]]) most[share[i]] = floats[i];
       }
-    std::vector<float*> common;
-    for (size_t n : most) common.push_back(ar.take(n));
-    for (size_t i = 0; i < twins.size(); ++i) twins[i].p = share[i] >= 0 ? common[share[i]] : ar.take(floats[i]);
-    for (CvHist& h : hist) h.buf = twins[h.ring.id];
+    std::vector<size_t> common;
+    for (size_t n : most) common.push_back(take(n));
+    for (size_t i = 0; i < twins.size(); ++i) at.push_back(share[i] >= 0 ? common[share[i]] : take(floats[i]));
+    for (CvHist& h : hist) h.at = at[h.ring.id];
+    return end;
   }
 };
 static Ring no_ring() { Ring r; r.p = nullptr; r.rs = 1; r.mask = 0; r.pad = 0; r.tstep = 0; r.id = -1; return r; }
@@ -1464,7 +1470,7 @@ static CvScratch cv_plan(CvGemm& g) {
 
 // Lays out the workspace and (when tensors != nullptr) packs weights and records the launch plan.
 static int cv_build(vui_codec* cc, const vui_codec_config* c, const void* const* tensors, char* ws, hipStream_t st, int64_t* need,
-                    size_t part_cap, size_t cnt_cap, size_t* part_need, size_t* cnt_need) {
+                    size_t part_cap, size_t cnt_cap, size_t* part_need, size_t* cnt_need, int64_t* block_need = nullptr) {
   Arena ar{ws};
   const bool real = ws != nullptr && tensors != nullptr;
   int ti = 0;
@@ -1735,7 +1741,8 @@ static int cv_build(vui_codec* cc, const vui_codec_config* c, const void* const*
       cc->fin.in = fin_in; cc->fin.w = fwp; cc->fin.b = fbp; cc->fin.audio = nullptr; cc->fin.C = dim; cc->fin.k = 7; cc->fin.T = hop; cc->fin.ctr = ctr; cc->fin.nf = 1;
     }
   }
-  rings.place();
+  const size_t twin_floats = rings.place();
+  if (block_need) *block_need = (int64_t)twin_floats * 4;
   CvHist* hist_dev = (CvHist*)ar.take((sizeof(CvHist) * rings.hist.size() + 3) / 4);
   if (need) *need = (int64_t)ar.off;
   if (part_need) *part_need = part_floats;
@@ -1763,6 +1770,8 @@ static int cv_build(vui_codec* cc, const vui_codec_config* c, const void* const*
     cc->hist = hist_dev;
     cc->n_hist = (int)rings.hist.size();
     cc->twins = rings.twins;
+    cc->twin_at = rings.at;
+    cc->block_bytes = (int64_t)twin_floats * 4;
     cc->vqx = vqx.id; cc->qkv = qkv.id; cc->att = att.id;
     cc->vq.codes = nullptr; cc->vq.n_q = 0; cc->vq.n_sem = c->n_semantic; cc->vq.CS = CS; cc->vq.cd = cd;
     cc->vq.embed = embed; cc->vq.x = vqx.p; cc->vq.rs = vqx.rs; cc->vq.nf = 1; cc->vq.ctr = ctr; cc->vq.err = ctr + 1; cc->vq.max_seq = c->max_seq;
@@ -1936,18 +1945,29 @@ int32_t vui_codec_block_frames(const vui_codec* c) {
   return block_frames(c->cfg);
 }
 
-int vui_codec_decode_block(vui_codec* c, const int64_t* codes, int32_t n_frames, int32_t n_q, float* audio_out, vui_stream_t stream) {
+int64_t vui_codec_block_scratch_bytes(const vui_codec_config* c) {
+  if (cv_check(c)) return VUI_EINVAL;
+  int64_t need = 0;
+  if (cv_build(nullptr, c, nullptr, nullptr, nullptr, nullptr, 0, 0, nullptr, nullptr, &need)) return VUI_EINVAL;
+  return need;
+}
+
+int vui_codec_decode_block(vui_codec* c, const int64_t* codes, int32_t n_frames, int32_t n_q, float* audio_out, void* scratch,
+                           int64_t scratch_bytes, vui_stream_t stream) {
   if (!c) { vui_set_error("NULL codec"); return VUI_EINVAL; }
   if (!codes || !audio_out) { vui_set_error("NULL argument"); return VUI_EINVAL; }
   if (n_q < 1 || n_q > c->cfg.n_codebooks) { vui_set_error("n_q=%d outside [1,%d]", n_q, c->cfg.n_codebooks); return VUI_EINVAL; }
   if (n_frames < 1 || n_frames > block_frames(c->cfg)) { vui_set_error("codec: %d frames outside [1, %d]", n_frames, block_frames(c->cfg)); return VUI_EINVAL; }
   if (n_frames == 1) return vui_codec_decode_frame(c, codes, n_q, audio_out, stream);
+  if (!scratch || ((uintptr_t)scratch) & 255) { vui_set_error("codec: the scratch memory must be given and 256-byte aligned"); return VUI_EINVAL; }
+  if (scratch_bytes < c->block_bytes) { vui_set_error("codec: scratch too small: %lld < %lld", (long long)scratch_bytes, (long long)c->block_bytes); return VUI_ENOMEM; }
   hipStream_t st = (hipStream_t)stream;
-  auto twin = [&](const Ring& r) { return r.id < 0 ? r : c->twins[r.id]; };
+  auto buf = [&](int id) { Ring t = c->twins[id]; t.p = (float*)scratch + c->twin_at[id]; return t; };
+  auto twin = [&](const Ring& r) { return r.id < 0 ? r : buf(r.id); };
   CvVq vq = c->vq;
-  vq.codes = codes; vq.n_q = n_q; vq.nf = n_frames; vq.x = c->twins[c->vqx].p; vq.rs = c->twins[c->vqx].rs;
+  vq.codes = codes; vq.n_q = n_q; vq.nf = n_frames; vq.x = buf(c->vqx).p; vq.rs = buf(c->vqx).rs;
   hipLaunchKernelGGL(cv_vq_kernel, dim3(n_frames), dim3(256), 0, st, vq);
-  hipLaunchKernelGGL(cv_history_kernel, dim3(16, c->n_hist), dim3(256), 0, st, c->hist, c->ctr, n_frames, 0);
+  hipLaunchKernelGGL(cv_history_kernel, dim3(16, c->n_hist), dim3(256), 0, st, c->hist, (float*)scratch, c->ctr, n_frames, 0);
   for (const Step& s0 : c->steps) {
     Step s = s0;
     if (s.kind == 0) {
@@ -1958,17 +1978,17 @@ int vui_codec_decode_block(vui_codec* c, const int64_t* codes, int32_t n_frames,
       if (rc) return rc;
     } else if (s.kind == 1) {
       s.a.nf = n_frames;
-      s.a.qkv = c->twins[c->qkv].p; s.a.rs = c->twins[c->qkv].rs; s.a.out = c->twins[c->att].p; s.a.rs_out = c->twins[c->att].rs;
+      s.a.qkv = buf(c->qkv).p; s.a.rs = buf(c->qkv).rs; s.a.out = buf(c->att).p; s.a.rs_out = buf(c->att).rs;
       const size_t lds = (size_t)(s.a.hd + s.a.max_seq + 4 * s.a.hd + 8) * 4;
       hipLaunchKernelGGL(cv_append_kernel, dim3(s.a.H, n_frames), dim3(64), 0, st, s.a);
       hipLaunchKernelGGL(cv_attn_kernel, dim3(s.a.H, n_frames), dim3(256), lds, st, s.a);
     } else {
-      const Ring ln = c->twins[s.ln];
+      const Ring ln = buf(s.ln);
       s.d.nf = n_frames; s.d.in = twin(s.d.in); s.d.out = ln.p; s.d.rs_out = ln.rs;
       hipLaunchKernelGGL(cv_dwln_kernel, dim3(s.g.T * n_frames), dim3(256), 0, st, s.d);
     }
   }
-  hipLaunchKernelGGL(cv_history_kernel, dim3(16, c->n_hist), dim3(256), 0, st, c->hist, c->ctr, n_frames, 1);
+  hipLaunchKernelGGL(cv_history_kernel, dim3(16, c->n_hist), dim3(256), 0, st, c->hist, (float*)scratch, c->ctr, n_frames, 1);
   CvFinal fin = c->fin;
   fin.audio = audio_out; fin.nf = n_frames; fin.T *= n_frames; fin.in = twin(fin.in);
   hipLaunchKernelGGL(cv_final_kernel, dim3((fin.T + FIN_TW - 1) / FIN_TW), dim3(256), (size_t)(fin.C * (FIN_TW + fin.k - 1) + 256 + fin.C * fin.k) * 4, st, fin);
