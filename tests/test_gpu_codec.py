@@ -262,3 +262,18 @@ def test_full_dims_blocks_equal_single_frames(full):
         finally:
             dec.persistent(1)
         assert err(got, one.cpu()) < 5e-5  # measured 1e-5
+
+
+@pytest.mark.parametrize("d_model", [1024, 1312, 2048])
+def test_blocks_of_wide_pre_transformers(d_model):
+    """Widths whose normed products take eight waves (25-48 units of 32 channels from 17 frames on, 33-64 below) or split
+    units: every block length around the 16-column tiles against the oracle and against single frames (2e-5 as above)."""
+    d = dataclasses.replace(small_dims(), d_model=d_model)
+    sd = O.synthetic_codec_state_dict(d, seed=5)
+    ora, dec = O.CodecDecoderOracle(d, sd), native(d, sd)
+    for T in (2, 16, 17, 32):
+        codes = torch.randint(0, d.codebook_size, (1, d.n_codebooks, T), generator=torch.Generator().manual_seed(T))
+        got = dec(codes.cuda())
+        with dec.streaming(1):
+            one = torch.cat([dec(codes[:, :, t:t + 1].cuda()).clone() for t in range(T)], dim=-1)
+        assert err(got, ora.forward(codes)) < TOL and err(got, one.cpu()) < 2e-5, T

@@ -198,23 +198,24 @@ __device__ __forceinline__ void cv_gemm_tile(const CvGemm& p, const int m0, cons
   }
   // 1/rms of the input column while the first operands are in flight; applied to the sums at the end
   float rstd = 1.f;
-  if (p.in_mode == IN_RMS && p.T > 1) {  // a column per frame: 16 threads share one
-    __shared__ float sq[TT * 256];
+  if (p.in_mode == IN_RMS && p.T > 1) {  // a column per frame: 4 threads of every wave share one
+    constexpr int SH = 4 * NW;
+    __shared__ float sq[TT * 16 * SH];
 #pragma unroll
     for (int tt = 0; tt < TT; ++tt) {
       const int t = min(t0 + tt * 16 + (tid & 15), p.T - 1);
       float ss = 0.f;
-      for (int c = tid >> 4; c < Cin; c += 16) {
+      for (int c = tid >> 4; c < Cin; c += SH) {
         const float v = *ring_ptr(p.in, ib_, c, p.in.pad + t);
         ss = fmaf(v, v, ss);
       }
-      sq[tt * 256 + (tid & 15) * 16 + (tid >> 4)] = ss;
+      sq[(tt * 16 + (tid & 15)) * SH + (tid >> 4)] = ss;
     }
     __syncthreads();
     if (tid < TT * 64) {
       float ss = 0.f;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) ss += sq[(tid >> 6) * 256 + (tid & 15) * 16 + i];
+      for (int i = 0; i < SH; ++i) ss += sq[((tid >> 6) * 16 + (tid & 15)) * SH + i];
       rstd = 1.0f / sqrtf(ss / (float)Cin + p.eps);
     }
   } else if (p.in_mode == IN_RMS) {
