@@ -293,3 +293,54 @@ def test_slots_are_written_once_for_the_same_rows():
     assert e._held is None
     e._set_active_slots([1])
     assert e._held == [1] and e._g_seq_inc.tolist() == [0, 1, 0, 0, 0]
+
+
+def test_a_failed_capture_leaves_the_rows_slots():
+    """decode_step after one whose capture raised, for the same rows, a subset and again the first: every replay meets the
+    slots of its own rows, and only a change of rows writes them."""
+    from vui_amd.lm_engine import TokenEngine
+
+    class Row:
+        def __init__(self, idx):
+            self.idx, self._length = idx, 0
+
+    class Fake(TokenEngine):
+        def __init__(self):
+            self.max_rows, self.device, self.max_seq = 4, torch.device("cpu"), 16
+            self.seq_lens = torch.zeros(5, dtype=torch.int32)
+            self._setup_slots(8)
+            self._g_tokens, self._g_logits = torch.zeros(4, dtype=torch.long), torch.zeros(4, 8)
+            self.fail, self.seen, self.writes = True, [], 0
+
+        def _capture(self, body):
+            if self.fail:
+                raise RuntimeError("out of memory")
+            eng = self
+
+            class G:
+                def replay(self):
+                    eng.seen.append((eng._g_slot_idx.tolist(), eng._g_seq_inc.tolist()))
+
+            return G()
+
+        def _set_active_slots(self, slots):
+            self.writes += 1
+            return super()._set_active_slots(slots)
+
+    e = Fake()
+    rows, toks = [Row(2), Row(0), Row(3)], torch.tensor([1, 2, 3])
+    with pytest.raises(RuntimeError, match="out of memory"):
+        e.decode_step(rows, toks)
+    assert [r._length for r in rows] == [0, 0, 0]
+    e.fail = False
+    full = ([2, 0, 3, 4], [1, 0, 1, 1, 0])
+    e.decode_step(rows, toks)  # captures, on the padding slot
+    assert e.seen.pop() == full
+    writes = e.writes
+    e.decode_step(rows, toks)
+    assert e.seen.pop() == full and e.writes == writes
+    e.decode_step(rows[:2], toks[:2])  # captures the narrower step
+    assert e.seen.pop() == ([2, 0, 3, 4], [1, 0, 1, 0, 0]) and e.writes == writes + 1
+    e.decode_step(rows, toks)
+    assert e.seen.pop() == full and e.writes == writes + 2
+    assert [r._length for r in rows] == [4, 4, 3]

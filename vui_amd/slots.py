@@ -102,12 +102,16 @@ class SlotEngine:
             self._held = None
         g = self._bucketed_graphs.get(B_bucket)
         if g is None:
+            held, self._held = self._held, None  # the tensors hold no rows' slots until they are restored
             saved_idx, saved_inc = self._g_slot_idx.clone(), self._g_seq_inc.clone()
-            self._g_slot_idx[:B_bucket].fill_(self._pad_slot)
-            self._g_seq_inc.zero_()
-            g = self._capture(lambda st: body(B_bucket, st))
-            self._g_slot_idx.copy_(saved_idx)
-            self._g_seq_inc.copy_(saved_inc)
+            try:
+                self._g_slot_idx[:B_bucket].fill_(self._pad_slot)
+                self._g_seq_inc.zero_()
+                g = self._capture(lambda st: body(B_bucket, st))
+            finally:
+                self._g_slot_idx.copy_(saved_idx)
+                self._g_seq_inc.copy_(saved_inc)
+            self._held = held
             self._bucketed_graphs[B_bucket] = g
         if run:
             g.replay()
@@ -115,6 +119,7 @@ class SlotEngine:
 
     def _set_active_slots(self, slots: "list[int]") -> Tensor:
         """The rows of the next bucketed steps: their slots, and which lengths advance.  Returns the slots (int32)."""
+        self._held = None  # until both tensors are written
         t = torch.tensor(slots, dtype=torch.int32, device=self.device)
         self._g_slot_idx[:len(slots)] = t
         self._g_seq_inc.zero_()
