@@ -10,11 +10,11 @@
 #pragma once
 #include "tile.h"
 
-// 16 bytes per lane from g to LDS at byte `at` + 16 lane (wave-uniform).  There is no register for the compiler to wait
-// for: the loop counts these loads itself (vmcnt).  Through the builtin the compiler waited for all of them in front of
-// every LDS read.
+// 16 bytes per lane from g to LDS at byte `at` + 16 lane (wave-uniform; taken from m0, which the compiler loads and so
+// knows to be overwritten).  There is no register for the compiler to wait for: the loop counts these loads itself (vmcnt).
+// Through the builtin the compiler waited for all of them in front of every LDS read.
 __device__ __forceinline__ void wide_to_lds(const char* g, uint32_t at) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(at), "v"(g) : "memory");
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"{m0}"(at), "v"(g) : "memory");
 }
 
 // eight int8 -> four packed bf16 pairs, exact
