@@ -347,9 +347,10 @@ __global__ __launch_bounds__(512) void latent_value_kernel(const LatentArgs p, i
 // which is operand layout for out^T = V^T p^T; the fp32 weights go in as a bf16 pair (value and remainder), so the
 // average keeps about 16 bits of them.  DB = dim64 / 64, RB = rot32 / 32, VT >= vdim16 / 16.
 // Bound by the keys and values that every tile of queries fetches from L2 (16 heads of 128 + 64 and 128, 1999 positions:
-// 1.7 GB in 56 us).  Neighbouring workgroups take different heads, so that an XCD's L2 holds few of them (68 -> 56 us);
-// masks and the rescaling of the sums only in the steps that need them (73 -> 68 us).  Two tiles of queries per wave: 47 us
-// there, but 11.4 instead of 8.2 us at 600 positions of eight heads, and nothing of it in the whole prompt's time.
+// 1.7 GB in 60 us).  Neighbouring workgroups take different heads, so that an XCD's L2 holds few of them, masks and the
+// rescaling of the sums only in the steps that need them: 73 -> 60 us there (56 us with weights by v_exp_f32 alone, which are
+// less exact than expf's).  Two tiles of queries per wave were quicker there and slower at 600 positions of eight heads,
+// and gave nothing of it in the whole prompt's time.
 #define LPF_WAVES (VT <= 4 ? 8 : 4)
 template <int DB, int RB, int VT>
 __global__ __launch_bounds__(64 * LPF_WAVES, 2) void latent_prefill_kernel(const LatentArgs p) {
@@ -362,7 +363,6 @@ __global__ __launch_bounds__(64 * LPF_WAVES, 2) void latent_prefill_kernel(const
   const int nvb = p.d.vdim16 >> 4;
   const int qlast = pos0 + min(q0 + l16, T - 1);  // last visible key of this lane's query
   const int kend = pos0 + min(q0 + 15, T - 1) + 1;
-  const float ls = p.scale * 1.44269504088896f;  // weights are powers of two, one v_exp_f32 each
   const bf16_t* qu = (const bf16_t*)p.qu + h * p.qu_z + (size_t)qt * DB * 1024 + lane * 8;
   const bf16_t* qr = (const bf16_t*)p.qr + h * p.qr_z + (size_t)qt * RB * 512 + lane * 8;
   uint4 qf[2 * DB + RB];
@@ -398,7 +398,7 @@ __global__ __launch_bounds__(64 * LPF_WAVES, 2) void latent_prefill_kernel(const
 #pragma unroll
       for (int i = 0; i < 2 * DB + RB; ++i) sc[t] = Tl<bf16_t>::mma(kf[t][i], qf[i], sc[t]);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) sc[t][r] *= ls;
+      for (int r = 0; r < 4; ++r) sc[t][r] *= p.scale;
     }
     if (k0 + 31 > pos0 + q0) {  // a key that some query of the tile does not see
 #pragma unroll
@@ -413,11 +413,11 @@ __global__ __launch_bounds__(64 * LPF_WAVES, 2) void latent_prefill_kernel(const
     mx = rows_max(mx);
     const float m_new = fmaxf(m_run, mx);
     const float m_use = m_new == -INFINITY ? 0.f : m_new;
-    const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
+    const float alpha = expf(m_run - m_use);
     float pv[8], lo[8], ps = 0.f;
     uint4 hi4, lo4;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) { pv[e] = __builtin_amdgcn_exp2f(sc[e >> 2][e & 3] - m_use); ps += pv[e]; }
+    for (int e = 0; e < 8; ++e) { pv[e] = expf(sc[e >> 2][e & 3] - m_use); ps += pv[e]; }
     l_run = l_run * alpha + ps;
     m_run = m_new;
     hi4.x = f2bf2(pv[0], pv[1]); hi4.y = f2bf2(pv[2], pv[3]); hi4.z = f2bf2(pv[4], pv[5]); hi4.w = f2bf2(pv[6], pv[7]);
@@ -451,7 +451,7 @@ __global__ __launch_bounds__(64 * LPF_WAVES, 2) void latent_prefill_kernel(const
     float den = 0.f, o[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 0; w < LPF_WAVES; ++w) {
-      const float f = s_m[w][q] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(s_m[w][q] - M);
+      const float f = s_m[w][q] == -INFINITY ? 0.f : expf(s_m[w][q] - M);
       den = fmaf(f, s_l[w][q], den);
 #pragma unroll
       for (int r = 0; r < 4; ++r) o[r] = fmaf(f, s_acc[w][sl * 4 + r], o[r]);

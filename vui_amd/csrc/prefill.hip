@@ -311,9 +311,10 @@ __device__ __forceinline__ uint4 pf_rope8(uint4 v, const float* __restrict__ rop
 // V^T p^T, with V^T read from the transposed copy in the same key order (any assignment of k to lanes is valid
 // when both operands share it).  HD32 = head_dim / 32.
 // Bound by the keys and values that every tile of queries fetches from L2 and by the instructions around the weights.
-// Neighbouring workgroups take different heads, so that an XCD's L2 holds the keys and values of few (eight heads of 96,
-// 1733 positions: 22 -> 16.3 us, all heads together are 5.3 MB); weights are one fma and one v_exp_f32, masks and the
-// rescaling of the sums only in the steps that need them (25.2 -> 22 us; at 576 positions 9.4 -> 6.3 us with both).
+// Neighbouring workgroups take different heads, so that an XCD's L2 holds the keys and values of few (all heads together
+// are 5.3 MB at eight heads of 96, 1733 positions); masks and the rescaling of the sums only in the steps that need them:
+// 25.2 -> 19.0 us there, 9.4 -> 7.0 us at 576 positions.  Weights as powers of two, one fma and one v_exp_f32 each, took
+// 16.3 / 6.3 us, but up to 2.7 times the error of expf against 64 bits (heads of 64, scores of deviation 12: 3.9e-7 against 1.4e-7).
 // Two tiles of queries per wave or per workgroup, which halves the fetches, measured the same at 1733 and slower below.
 #define PF_ATT_WAVES (HD32 <= 3 ? 8 : 4)  // the partial outputs of the waves must fit 64 KiB of LDS
 template <int HD32>
@@ -343,7 +344,6 @@ __global__ __launch_bounds__(64 * PF_ATT_WAVES, 2) void pf_attn_kernel(const bf1
   const int kbeg = (window > 0 ? max(0, pos0 + q0 - window) : 0) & ~31;
   // steps that start in [kall, kmid) are visible to every query of the tile
   const int kall = window > 0 ? max(0, pos0 + t_hi - window) : 0, kmid = pos0 + q0 - 30;
-  const float ls = scale * 1.44269504088896f;  // weights are 2^(ls * score - m): one fma and one v_exp_f32 each
   // staged keys / values of this KV head (pf_stage_kv_kernel): a fragment is 16 bytes per lane, 1 KiB contiguous per wave
   const bf16_t* kb = kt + (size_t)kvh * (Lpad >> 4) * HD32 * 512 + lane * 8;
   const bf16_t* vb = vt + (size_t)kvh * DT * (Lpad >> 5) * 512 + lane * 8;
@@ -375,6 +375,10 @@ __global__ __launch_bounds__(64 * PF_ATT_WAVES, 2) void pf_attn_kernel(const bf1
         sc[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf_frag(kf[kt][c]), pf_frag(qf[c]), sc[kt], 0, 0, 0);
     }
     // the lane holds keys k0 + 16 kt + 4 kg + r of its query
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sc[kt][r] *= scale;
     if (k0 < kall || k0 >= kmid) {
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt)
@@ -388,12 +392,12 @@ __global__ __launch_bounds__(64 * PF_ATT_WAVES, 2) void pf_attn_kernel(const bf1
 #pragma unroll
     for (int r = 1; r < 4; ++r) mx = fmaxf(mx, fmaxf(sc[0][r], sc[1][r]));
     mx = rows_max(mx);  // over the four lane rows: every key of the step for this query
-    const float m_new = fmaxf(m_run, mx * ls);
+    const float m_new = fmaxf(m_run, mx);
     const float m_use = (m_new == -INFINITY) ? 0.f : m_new;  // nothing visible yet: every weight below is zero
-    const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);  // 0 on the first visible step (m_run = -inf)
+    const float alpha = expf(m_run - m_use);                  // 0 on the first visible step (m_run = -inf)
     float pv[8], ps = 0.f;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) { pv[e] = __builtin_amdgcn_exp2f(fmaf(sc[e >> 2][e & 3], ls, -m_use)); ps += pv[e]; }
+    for (int e = 0; e < 8; ++e) { pv[e] = expf(sc[e >> 2][e & 3] - m_use); ps += pv[e]; }
     l_run = l_run * alpha + ps;
     m_run = m_new;
     uint4 pf;
@@ -423,7 +427,7 @@ __global__ __launch_bounds__(64 * PF_ATT_WAVES, 2) void pf_attn_kernel(const bf1
     float den = 0.f, o[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 0; w < PF_ATT_WAVES; ++w) {
-      const float f = (s_m[w][q] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(s_m[w][q] - M);
+      const float f = (s_m[w][q] == -INFINITY) ? 0.f : expf(s_m[w][q] - M);
       den = fmaf(f, s_l[w][q], den);
 #pragma unroll
       for (int r = 0; r < 4; ++r) o[r] = fmaf(f, s_acc[w][sl * 4 + r], o[r]);
