@@ -481,3 +481,17 @@ def test_large_products_of_a_prompt(T):
         row.reset()
         parts = torch.cat([row.extend(toks[i:i + 100], range(len(toks[i:i + 100]))).clone() for i in range(0, T, 100)])
     assert U.err(whole, parts) < 0.04
+
+
+@BOTH
+@pytest.mark.parametrize("T", [5, 150])
+def test_gates_far_below_zero(T, dt):
+    """Gates of magnitudes up to 1e38: closed ones (sigmoid 0) add nothing, open ones sit at the limit; few and many rows."""
+    cfg = U.config([U.gru(16)], width=144, ff=700, limit=0.25)
+    sd = U.weights(cfg, 31)
+    sd["l0.mix.o"].zero_()
+    sd["l0.mlp.gate"] = (sd["l0.mlp.gate"].double() * 1e37).to(torch.bfloat16)
+    eng = U.engine(cfg, sd, dt, max_seq=160)
+    toks = U.tokens(T, cfg["vocab"], 17)
+    with eng.new_row() as row:
+        assert U.err(run_all(row, toks), O.forward(cfg, sd, toks)) < U.TOL[dt]

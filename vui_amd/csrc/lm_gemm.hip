@@ -9,27 +9,13 @@
 #include "lm.h"
 #include "wide.h"
 
-// fp32 contexts: the library's exponential and division.  bf16 contexts: a prompt's epilogues evaluate ten million of
-// these per layer and were bound by their instructions, so the exponential is v_exp_f32 with the rounding of its argument
-// made good, the division v_rcp_f32 with a Newton step: half the instructions, relative error against 64 bits 4.1e-8
-// root mean square where the library's form has 3.9e-8 (|v| <= 20), and the result is rounded to 16 bits.
-template <typename T> __device__ __forceinline__ float lm_sigmoid(float v) {
-  if constexpr (sizeof(T) == 4) {
-    return 1.0f / (1.0f + expf(-v));
-  } else {
-    const float x = fminf(-v, 87.f), h = x * 1.4426950408889634f;
-    const float lo = fmaf(x, 1.4426950408889634f, -h) + x * 1.925963033500011e-8f;
-    const float ex = __builtin_amdgcn_exp2f(h), d = 1.0f + fmaf(ex, lo * 0.6931471805599453f, ex);
-    const float r = __builtin_amdgcn_rcpf(d);
-    return v < -3e38f ? 0.f : v != v ? v : v > 3e38f ? 1.f : fmaf(fmaf(-d, r, 1.0f), r, r);
-  }
-}
+__device__ __forceinline__ float lm_sigmoid(float v) { return 1.0f / (1.0f + expf(-v)); }
 
 // gated feed-forward with clamped branches, two features from interleaved (gate, up) pairs
-template <typename T> __device__ __forceinline__ float lm_ff(float g, float u, float limit) {
+__device__ __forceinline__ float lm_ff(float g, float u, float limit) {
   g = fminf(g, limit);
   u = fminf(fmaxf(u, -limit), limit);
-  return g * lm_sigmoid<T>(1.702f * g) * (u + 1.0f);
+  return g * lm_sigmoid(1.702f * g) * (u + 1.0f);
 }
 
 // rotates two pairs held as (u0, v0, u1, v1); pair indices i, i + 1; pairs at or beyond n pass
@@ -75,10 +61,10 @@ __device__ __forceinline__ void lm_unit(const LmGemm& p, const int m, const int 
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const float zz = v[r] + zb[r], uu = xv[r] + xb[r];
-      const float z = lm_sigmoid<T>(zz);
-      keep[r] = lm_sigmoid<T>(-zz);
-      in[r] = z * (uu >= 0.f ? uu + 0.5f : lm_sigmoid<T>(uu));
-      sg[r] = gv[r] * lm_sigmoid<T>(gv[r]);
+      const float z = lm_sigmoid(zz);
+      keep[r] = lm_sigmoid(-zz);
+      in[r] = z * (uu >= 0.f ? uu + 0.5f : lm_sigmoid(uu));
+      sg[r] = gv[r] * lm_sigmoid(gv[r]);
     }
     if (EPI == LM_IN_GRU_STEP) {
       float4* sp = reinterpret_cast<float4*>(p.state + (size_t)e.slot * p.d.gru16 + ch);
@@ -100,7 +86,7 @@ __device__ __forceinline__ void lm_unit(const LmGemm& p, const int m, const int 
     if (!live) return;
     if (nb >= p.mix_blocks) {  // (gate, up) pairs
       const int f = (n - p.mix_blocks * 16) >> 1;
-      Tl<T>::st2((T*)p.act + tl_off<T>(m, p.d.ff_off + f, p.d.out_k), lm_ff<T>(v[0], v[1], p.limit), lm_ff<T>(v[2], v[3], p.limit));
+      Tl<T>::st2((T*)p.act + tl_off<T>(m, p.d.ff_off + f, p.d.out_k), lm_ff(v[0], v[1], p.limit), lm_ff(v[2], v[3], p.limit));
       return;
     }
     if (EPI == LM_IN_ATTN) {
@@ -126,7 +112,7 @@ __device__ __forceinline__ void lm_unit(const LmGemm& p, const int m, const int 
         const int o = (nb - p.b_g) * 16 + 4 * kg;
         if (o < p.d.heads16)  // the blocks behind the gates only fill the last tile of the mixer part
           *reinterpret_cast<float4*>(p.gate + (size_t)m * p.d.heads16 + o) =
-              make_float4(lm_sigmoid<T>(v[0]), lm_sigmoid<T>(v[1]), lm_sigmoid<T>(v[2]), lm_sigmoid<T>(v[3]));
+              make_float4(lm_sigmoid(v[0]), lm_sigmoid(v[1]), lm_sigmoid(v[2]), lm_sigmoid(v[3]));
       }
     }
     return;
@@ -455,7 +441,7 @@ __global__ __launch_bounds__(256, 2) void lm_wide_kernel(const LmGemm p) {
           float v[4];
           sums(i, j, v);
           if (mw + 16 * j < p.M)
-            Tl<bf16_t>::st2((bf16_t*)p.act + tl_off<bf16_t>(mw + 16 * j, f, p.d.out_k), lm_ff<bf16_t>(v[0], v[1], p.limit), lm_ff<bf16_t>(v[2], v[3], p.limit));
+            Tl<bf16_t>::st2((bf16_t*)p.act + tl_off<bf16_t>(mw + 16 * j, f, p.d.out_k), lm_ff(v[0], v[1], p.limit), lm_ff(v[2], v[3], p.limit));
         }
         continue;
       }
