@@ -68,13 +68,18 @@ struct WideTile {
     for (int q = 0; q < S - 1; ++q)
       if (q < Q) issue(q);
   }
-  __device__ __forceinline__ void run(int Q, tl_f32x4 (&acc)[NBW][MBW]) {
+  // The sums of a quarter of K each (in whole 64 columns) are added in order, as the waves of a K-splitting workgroup leave
+  // them, so that a chain of fp32 sums is no longer than there and both forms give the same bits.
+  __device__ __forceinline__ void run(int Q, tl_f32x4 (&sum)[NBW][MBW]) {
     const int wm = wave % WM, wn = wave / WM;
+    const tl_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    tl_f32x4 acc[NBW][MBW];
 #pragma unroll
     for (int i = 0; i < NBW; ++i)
 #pragma unroll
-      for (int j = 0; j < MBW; ++j) acc[i][j] = tl_f32x4{0.f, 0.f, 0.f, 0.f};
-    int slot = 0;
+      for (int j = 0; j < MBW; ++j) acc[i][j] = sum[i][j] = zero;
+    const int n64 = Q * KS / 2;
+    int slot = 0, part = 1, end = (n64 >> 2) * 2 / KS;  // the first step behind this quarter
     for (int q = 0; q < Q; ++q) {
       // the oldest stage has landed once no more than the stages behind it are outstanding, for every wave behind the
       // barrier; the fragments read from the slot that is filled next have arrived as well
@@ -102,6 +107,14 @@ struct WideTile {
 #pragma unroll
           for (int i = 0; i < NBW; ++i) wa[k][i] = *reinterpret_cast<const uint4*>(st + (MB * KS + (wn * NBW + i) * KS + k) * 1024);
       }
+      if (q == end) {  // while the fragments arrive
+#pragma unroll
+        for (int i = 0; i < NBW; ++i)
+#pragma unroll
+          for (int j = 0; j < MBW; ++j) { sum[i][j] += acc[i][j]; acc[i][j] = zero; }
+        do end = (n64 * ++part >> 2) * 2 / KS;
+        while (end == q);
+      }
 #pragma unroll
       for (int k = 0; k < KS; ++k)
 #pragma unroll
@@ -110,6 +123,10 @@ struct WideTile {
           for (int j = 0; j < MBW; ++j) acc[i][j] = Tl<bf16_t>::mma(wa[k][i], xa[k][j], acc[i][j]);
       slot = slot == S - 1 ? 0 : slot + 1;
     }
+#pragma unroll
+    for (int i = 0; i < NBW; ++i)
+#pragma unroll
+      for (int j = 0; j < MBW; ++j) sum[i][j] += acc[i][j];
   }
 };
 
