@@ -499,12 +499,39 @@ __global__ __launch_bounds__(256) void pf_stage_kv_kernel(bf16_t* __restrict__ q
 
 __global__ void pf_set_len_kernel(int32_t* seq_lens, int slot, int v) { seq_lens[slot] = v; }
 
+// The form of a product of M rows (pair: two matrices of N features): estimated microseconds of the large tiles - a launch,
+// and per step of 32 columns `wait` or `work` for each round of 256 tiles - and of the K-splitting form, whose time follows its
+// trips to memory and its tiles; with an odd number of row tiles every XCD meets all rows, which costs where they exceed
+// its L2.  Up to 256 tiles of 32 x 32 the K-splitting form runs with more waves and is quicker.
+// Fitted to 384 products (130 ... 2048 rows, widths 512, 768, 1024, bf16 and int8, weights of 22 layers in turn): on average 2 %
+// above the best form of each and 6 % below K-splitting alone; 6 products are more than 5 % above that, 19 % at most.
+// us, K-splitting / 128 x 128 / 64 x 128 / 64 x 64, bf16 at width 768: W1 and W3 at 577 rows 13.3 / 13.5 / 14.5 / 14.0, at 1000
+// 16.9 / 14.0 / 13.7 / 16.4, at 1733 25.3 / 19.3 / 22.7 / 25.6; W2 at 577 10.6 / 26.2 / 17.3 / 12.0, at 1733 29.4 / 26.3 / 17.6 / 17.8.
+static int pf_pick(int M, int N, int K, bool pair, bool i8) {
+  static const struct { int bm, bn; double base[2], wait[2], work[2]; } tile[] = {  // of bf16 and int8 weights
+      {128, 128, {7.0, 7.3}, {0.275, 0.325}, {0.244, 0.274}},
+      {64, 128, {5.1, 5.3}, {0.198, 0.204}, {0.198, 0.181}},
+      {64, 64, {3.9, 4.8}, {0.143, 0.141}, {0.143, 0.112}}};
+  static const struct { double base, k256, tile, over; } split[2] = {{2.8, 0.66, 0.27e-3, 2.6e-6}, {4.3, 0.146, 0.262e-3, 0.44e-6}};
+  const long rows = (M + 31) / 32;
+  if (M < 128 || K < 256 || rows * ((N + 31) / 32) <= 256) return WIDE_NONE;
+  if (pair) N *= 2;
+  int best = WIDE_NONE;
+  double us = split[i8].base + split[i8].k256 * (K / 256.0) + split[i8].tile * rows * ((N + 31) / 32) * (K / 64);
+  const double over = 2.0 * M * K - 3e6;
+  if ((rows & 1) && over > 0) us += split[i8].over * over;
+  for (int i = 0; i < 3; ++i) {
+    const long rounds = ((long)((M + tile[i].bm - 1) / tile[i].bm) * ((N + tile[i].bn - 1) / tile[i].bn) + 255) / 256;
+    const double work = rounds * tile[i].work[i8], c = tile[i].base[i8] + (K / 32) * (work > tile[i].wait[i8] ? work : tile[i].wait[i8]);
+    if (c < us) { best = i; us = c; }
+  }
+  return best;
+}
+
 // bf16 out, K split over the waves of a workgroup; W2 != nullptr: the SwiGLU pair; i8: int8 matrices with g.sc / g.sc2
 static int pf_gemm4(int epi, const PfGemm& g, const void* W2, int c_tiled, bool i8, hipStream_t st) {
   if (g.K % 64 || g.N % 16 || g.M < 1 || g.N < 1 || (c_tiled && g.N % 64)) { vui_set_error("prefill GEMM: bad shape N=%d K=%d", g.N, g.K); return VUI_EINVAL; }
-  // The pair's epilogue weighs more in large tiles, and below 768 rows the K-splitting form is quicker than estimated (us at
-  // 576 positions, K-splitting / large tile: W1 and W3 13.4 / 14.9, QKV of int8 10.2 / 10.8).
-  const int tile = g.K >= 256 ? wide_pick(g.M, W2 ? 2 * g.N : g.N, g.K, W2 ? 0.4 : g.M < 768 ? 0.6 : 0.85) : WIDE_NONE;
+  const int tile = pf_pick(g.M, g.N, g.K, W2 != nullptr, i8);
   if (tile != WIDE_NONE) {
     if (W2) return i8 ? pf_wide<PF_BF16, true, true>(tile, g, W2, c_tiled, st) : pf_wide<PF_BF16, true, false>(tile, g, W2, c_tiled, st);
     if (epi == PF_RESID) return i8 ? pf_wide<PF_RESID, false, true>(tile, g, W2, c_tiled, st) : pf_wide<PF_RESID, false, false>(tile, g, W2, c_tiled, st);
