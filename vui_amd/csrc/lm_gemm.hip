@@ -460,11 +460,12 @@ __global__ __launch_bounds__(256, 2) void lm_wide_kernel(const LmGemm p) {
   }
 }
 
+#define WIDE_BY_XCD 24  // feature tiles from which an XCD's share is taken (with fewer, whole XCDs would have nothing or twice as much to do)
 template <int EPI, int MBW, int NBW, int WM, int WN, int S, int KS>
 static int go_wide(LmGemm g, int nz, hipStream_t st) {
   const int MT = (g.M + 16 * MBW * WM - 1) / (16 * MBW * WM), NT = (g.N / 16 + NBW * WN - 1) / (NBW * WN);
   const bool moe = EPI == LM_MOE_UP || EPI == LM_MOE_DOWN;
-  g.by_xcd = !moe && NT >= 24;  // with fewer, whole XCDs would have nothing or twice as much to do
+  g.by_xcd = !moe && NT >= WIDE_BY_XCD;
   const int tiles = moe ? g.max_tiles * ((NT + 7) & ~7) : g.by_xcd ? MT * ((NT + 7) & ~7) : MT * NT;
   hipLaunchKernelGGL((lm_wide_kernel<EPI, MBW, NBW, WM, WN, S, KS>), dim3((unsigned)tiles, 1, nz), dim3(256), 0, st, g);
   HIP_TRY(hipGetLastError());
@@ -484,14 +485,18 @@ static int go(const LmGemm& g, int nz, hipStream_t st) {
 // Tile of a prompt's product (wide_pick).  The K-splitting kernel is counted 1.5 times: 28.4 against 23 us at 650 x 1024 x 4608
 // with 18.4 estimated.  Whole prompts with 0.85 / 1.2 / 1.5 / 2 of the estimate, us: latent models of 2048 x 400 positions
 // 1033 / 869 / 865 / 870 and of 1024 x 900 760 / 701 / 691 / 697, x 500 487 / 487 / 497 / 553; experts of 2048 x 300
-// 1463 / 1404 / 1311 / 1320.  A minGRU projection takes 128 x 192, with 20 us more in the epilogue
-// (us, K-splitting / large tile: 160 / 98 at 1024 x 14336 x 2048, 30 / 35 at 1024 x 6400 x 768).
+// 1463 / 1404 / 1311 / 1320.
 static int lm_tile(int epi, int M, int N, int K) {
-  double us;
-  const int t = wide_pick(M, N, K, 1.5, &us);
-  if (epi != LM_IN_GRU_SEQ) return t;
-  const double work = (double)(((M + 127) / 128 * ((N + 191) / 192) + 255) / 256) * 0.2;
-  return M >= 128 && 20 + (K / 32) * (work > 0.4 ? work : 0.4) < us ? WIDE_128 : WIDE_NONE;
+  if (epi != LM_IN_GRU_SEQ) return wide_pick(M, N, K, 1.5);
+  // A minGRU projection takes 128 x 192, whose tiles fill an XCD 64 at a time, or the K-splitting form, which is bound by the
+  // weights' way to the chip and by its tiles.  us, K-splitting / large tile (50 products of 130 ... 2048
+  // rows, the quicker form is taken in 49): 900 x 6400 x 768 27.6 / 30.0, 1200 32.1 / 31.1, 1600 39.7 / 46.5; 640 x 8704 x 1024 33.1 / 31.9; 300 x 11776 x 1024
+  // 33.7 / 31.4, 1200 79 / 64; 130 x 14336 x 2048 51 / 44, 1024 154 / 93.
+  if (M < 128) return WIDE_NONE;
+  const long MT = (M + 127) / 128, NT = (N + 191) / 192;
+  const long fills = NT >= WIDE_BY_XCD ? ((NT + 7) / 8 * MT + 63) / 64 : (NT * MT + 511) / 512;
+  const double split = 4 + 1e-6 * N * K + 0.26e-3 * ((M + 31) / 32) * ((N + 31) / 32) * (K / 64);
+  return 6 + fills * (10 + 0.56 * (K / 32)) < split ? WIDE_128 : WIDE_NONE;
 }
 template <int EPI>
 static int pick_wide(int tile, const LmGemm& g, hipStream_t st) {

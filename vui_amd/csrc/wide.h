@@ -136,11 +136,10 @@ struct WideTile {
 // when it has.  Measured (us, K-splitting / large tile): 1024 x 11776 x 2048 147 / 61, 1024 x 2048 x 6144 82 / 39,
 // 1024 x 5120 x 768 26 / 17, 1024 x 768 x 2816 16 / 17, 300 x 768 x 2816 9 / 17.
 enum { WIDE_NONE = -1, WIDE_128 = 0, WIDE_64x128 = 1, WIDE_64 = 2 };
-static inline int wide_pick(int M, int N, int K, double keep, double* us = nullptr) {
+static inline int wide_pick(int M, int N, int K, double keep) {
   static const struct { int bm, bn; double wait, work; } tile[] = {{128, 128, 0.335, 0.144}, {64, 128, 0.21, 0.08}, {64, 64, 0.17, 0.059}};
   int best = WIDE_NONE;
   double cost = keep * 0.38e-3 * ((M + 31) / 32) * ((N + 31) / 32) * (K / 64);
-  if (us) *us = cost;
   if (M < 128) return best;
   for (int i = 0; i < 3; ++i) {
     const long tiles = (long)((M + tile[i].bm - 1) / tile[i].bm) * ((N + tile[i].bn - 1) / tile[i].bn);
