@@ -83,10 +83,10 @@ int32_t vui_codec_block_frames(const vui_codec* c);
  * as many vui_codec_decode_frame calls give (sums in another order), and the same state behind them, so that blocks and
  * single frames may follow each other.  Every weight is read once per block.  The block must fit in front of max_seq:
  * one that does not raises the status flag and its samples are not the frames' own.  scratch: device memory of
- * vui_codec_block_scratch_bytes(cfg) bytes (the block's activations, 257 MB at the reference's dims), 256-byte aligned,
- * used only by this call (it holds nothing between calls; not needed for one frame).  No counterpart in the reference,
- * whose offline forward (qwen_codec.py:1191-1224) takes all frames at once. */
-int64_t vui_codec_block_scratch_bytes(const vui_codec_config* cfg);
+ * vui_codec_block_scratch_bytes(cfg, n_frames) bytes (the block's activations, 8 MB per frame at the reference's dims),
+ * 256-byte aligned, used only by this call (it holds nothing between calls; none is needed for one frame).  No counterpart
+ * in the reference, whose offline forward (qwen_codec.py:1191-1224) takes all frames at once. */
+int64_t vui_codec_block_scratch_bytes(const vui_codec_config* cfg, int32_t n_frames);
 int vui_codec_decode_block(vui_codec* c, const int64_t* codes, int32_t n_frames, int32_t n_q, float* audio_out, void* scratch,
                            int64_t scratch_bytes, vui_stream_t stream);
 

@@ -129,3 +129,20 @@ def test_abi_size_queries():
     h = C.c_void_p()
     assert lib.vui_codec_init(C.byref(c), None, 255, None, 0, None, C.byref(h)) == -22
     assert lib.vui_codec_decode_frame(None, None, 16, None, None) == -22 and "NULL codec" in _lib.last_error()
+
+
+def test_scratch_memory_follows_the_frames_of_a_block():
+    """vui_codec_block_scratch_bytes: none for one frame, in proportion to the frames behind it, and no block length that
+    vui_codec_decode_block refuses."""
+    from vui_amd import _lib
+
+    lib, cc = _lib.load(), K.CodecConfig().to_c()
+    size = [lib.vui_codec_block_scratch_bytes(C.byref(cc), n) for n in range(1, 33)]
+    assert size[0] == 0 and size[31] < 260e6
+    for n in range(2, 33):
+        assert size[n - 1] < (n + 1) * 8.1e6 and size[n - 1] > size[n - 2]
+    for n in (0, -1, 33):
+        assert lib.vui_codec_block_scratch_bytes(C.byref(cc), n) == -22
+    cc.max_seq = 5
+    assert lib.vui_codec_block_scratch_bytes(C.byref(cc), 5) == size[4]
+    assert lib.vui_codec_block_scratch_bytes(C.byref(cc), 6) == -22

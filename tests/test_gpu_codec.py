@@ -277,3 +277,15 @@ def test_blocks_of_wide_pre_transformers(d_model):
         with dec.streaming(1):
             one = torch.cat([dec(codes[:, :, t:t + 1].cuda()).clone() for t in range(T)], dim=-1)
         assert err(got, ora.forward(codes)) < TOL and err(got, one.cpu()) < 2e-5, T
+
+
+def test_memory_of_a_call_follows_its_frames(full):
+    """A call of a few frames allocates scratch memory for those (8 MB each), not for the longest block; a call of one none."""
+    d, sd, dec, fx = full
+    codes = torch.randint(0, d.codebook_size, (1, d.n_codebooks, 3), generator=torch.Generator().manual_seed(8)).cuda()
+    torch.cuda.synchronize()
+    for T, most in ((1, 2 ** 20), (2, 17e6), (3, 26e6)):
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        dec(codes[:, :, :T].contiguous())
+        assert torch.cuda.max_memory_allocated() - before < most

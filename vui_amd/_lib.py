@@ -128,7 +128,7 @@ SIGNATURES = {
     "vui_codec_reset": (_I, [_P, _P]),
     "vui_codec_decode_frame": (_I, [_P, _P, C.c_int32, _P, _P]),
     "vui_codec_block_frames": (C.c_int32, [_P]),
-    "vui_codec_block_scratch_bytes": (_L, [C.POINTER(CodecConfigC)]),
+    "vui_codec_block_scratch_bytes": (_L, [C.POINTER(CodecConfigC), C.c_int32]),
     "vui_codec_decode_block": (_I, [_P, _P, C.c_int32, C.c_int32, _P, _P, _L, _P]),
     "vui_codec_status": (_L, [_P, _P]),
     "vui_codec_persistent": (_I, [_P, _I]),

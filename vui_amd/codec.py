@@ -209,7 +209,7 @@ class QwenCodecDecoder:
         self._streaming = False
         self._frames = 0  # frames since the last reset (of the calls made here)
         self._block = int(lib.vui_codec_block_frames(h))
-        self._block_bytes = int(lib.vui_codec_block_scratch_bytes(C.byref(cc)))
+        self._block_bytes = [0] + [int(lib.vui_codec_block_scratch_bytes(C.byref(cc), n + 1)) for n in range(self._block)]
         self._cap_stream = torch.cuda.Stream(device=self.device)
         self._graphs: dict[int, object] = {}
         self._stream_codes_in = torch.zeros(self.cfg.n_codebooks, dtype=torch.long, device=self.device)
@@ -347,13 +347,15 @@ class QwenCodecDecoder:
         audio = torch.empty(1, 1, T * self.hop, dtype=torch.float32, device=self.device)
         flat = audio.view(-1)
         st = torch.cuda.current_stream().cuda_stream
-        scratch = torch.empty(self._block_bytes if T > 1 else 0, dtype=torch.uint8, device=self.device)
+        scratch = None
         t = 0
         while t < T:  # blocks of frames; single frames past the decoder's window, where only the status flag is left to raise
-            n = min(T - t, self._block)
-            if n > 1 and self._frames + n <= self.cfg.max_seq:
+            n = min(T - t, self._block, self.cfg.max_seq - self._frames)
+            if n > 1:
+                if scratch is None:  # blocks do not grow
+                    scratch = torch.empty(self._block_bytes[n], dtype=torch.uint8, device=self.device)
                 _lib.check(self.lib.vui_codec_decode_block(self.handle, ct[t].data_ptr(), n, n_q, flat[t * self.hop:].data_ptr(),
-                                                           scratch.data_ptr(), self._block_bytes, st),
+                                                           scratch.data_ptr(), scratch.numel(), st),
                            "vui_codec_decode_block")
                 self._frames += n
             else:

@@ -1245,7 +1245,7 @@ __global__ void cv_fill_kernel(float* p, size_t n, float v) {
 }
 // The history columns of every ring into the buffer that stands for it during a block (out = 0), and those behind the
 // block's last frame back into the ring.
-struct CvHist { Ring ring; size_t at; int rs, C; };  // at, rs: the buffer in the scratch memory of the block (floats), its row stride
+struct CvHist { Ring ring; size_t at; int rs, C; };  // of a block length; at, rs: the buffer in the scratch memory of the block (floats), its row stride
 __global__ void cv_history_kernel(const CvHist* h, float* scratch, const int* ctr, int nf, int out) {
   const CvHist r = h[blockIdx.y];
   const int base = ring_base(r.ring, *ctr - (out ? 0 : nf)), at = out ? nf * r.ring.tstep : 0;
@@ -1267,6 +1267,13 @@ struct Step {
   CvDwLn d;
 };
 
+// Where the twins of a block of frames lie in the scratch memory.
+struct CvBlock {
+  std::vector<Ring> twins;
+  std::vector<size_t> at;  // floats from its start
+  size_t floats = 0;
+};
+
 struct vui_codec {
   vui_codec_config cfg;
   int hop;
@@ -1275,10 +1282,8 @@ struct vui_codec {
   float* state0;  // start of the zeroed-on-reset region (rings)
   size_t state_floats;
   // what stands for each ring and buffer while several frames are decoded at once, in the caller's scratch memory
-  std::vector<Ring> twins;
-  std::vector<size_t> twin_at;  // floats from its start
-  int64_t block_bytes = 0;
-  CvHist* hist;                 // device: the rings and their twins
+  std::vector<CvBlock> blocks;  // of n frames at [n]
+  CvHist* hist;                 // device: the rings and their twins, n_hist for every n
   int n_hist = 0;
   int* ctr;  // [0] frames started since reset, [1] error flag
   int* cnt;  // arrival counters of split tiles
@@ -1365,7 +1370,7 @@ struct Arena {
 };
 
 // Frames that one pass takes at most (vui_codec_decode_block).  At 32 the weights pass once per 32 frames (3 us of a
-// frame's 84) and a product's launch costs 0.15 us per frame; the buffers, scratch memory of the caller's, take 0.26 GB.
+// frame's 84) and a product's launch costs 0.15 us per frame; the buffers, scratch memory of the caller's, take 8 MB per frame.
 #define CV_BLOCK 32
 static int block_frames(const vui_codec_config& k) { return k.max_seq < CV_BLOCK ? k.max_seq : CV_BLOCK; }
 
@@ -1374,43 +1379,48 @@ static int block_frames(const vui_codec_config& k) { return k.max_seq < CV_BLOCK
 // lines are never in the caches again when a single frame comes to them: 1 % of the streamed vocoder.
 struct RingMaker {
   Arena& ar;
-  int frames;
-  std::vector<Ring> twins;
-  std::vector<size_t> floats, at;
-  std::vector<int> share;     // twins of one group >= 0 take turns in the same memory
-  std::vector<CvHist> hist;
+  struct Made { Ring ring; int C, T, share; };  // share: twins of one group >= 0 take turns in the same memory
+  std::vector<Made> made;
   Ring make(int C, int pad, int T, bool stream, int group = -1) {
     Ring r;
     r.rs = ipow2(pad + T);
     r.mask = r.rs - 1;
     r.pad = pad;
     r.tstep = stream ? T : 0;
-    r.id = (int)twins.size();
+    r.id = (int)made.size();
     r.p = ar.take((size_t)C * r.rs);
-    Ring t = r;
-    t.rs = (pad + T * frames + 3) & ~3;
-    t.mask = 0x7fffffff;
-    t.tstep = 0;
-    twins.push_back(t);
-    floats.push_back((size_t)C * t.rs + 256);  // a tile reads up to 256 columns behind the last channel's
-    share.push_back(group);
-    if (stream && pad) hist.push_back(CvHist{r, 0, t.rs, C});
+    made.push_back(Made{r, C, T, group});
     return r;
   }
-  size_t place() {  // once every ring is known: the twins' places in the scratch memory, and its floats
-    size_t end = 0;
-    auto take = [&](size_t n) { const size_t o = end; end += (n + 63) & ~(size_t)63; return o; };
-    std::vector<size_t> most;
-    for (size_t i = 0; i < twins.size(); ++i)
-      if (share[i] >= 0) {
-        if ((int)most.size() <= share[i]) most.resize(share[i] + 1, 0);
-        if (floats[i] > most[share[i]]) most[share[i]] = floats[i];
-      }
-    std::vector<size_t> common;
-    for (size_t n : most) common.push_back(take(n));
-    for (size_t i = 0; i < twins.size(); ++i) at.push_back(share[i] >= 0 ? common[share[i]] : take(floats[i]));
-    for (CvHist& h : hist) h.at = at[h.ring.id];
-    return end;
+  static bool keeps(const Made& m) { return m.ring.tstep && m.ring.pad; }
+  int histories() const {
+    int n = 0;
+    for (const Made& m : made) n += keeps(m);
+    return n;
+  }
+  CvBlock block(int frames) const {  // once every ring is known
+    CvBlock b;
+    size_t common[2] = {0, 0};  // floats, then places of the shared groups
+    auto rs = [&](const Made& m) { return (m.ring.pad + m.T * frames + 3) & ~3; };
+    auto need = [&](const Made& m) { return (size_t)m.C * rs(m) + 256; };  // a tile reads up to 256 columns behind the last channel's
+    auto take = [&](size_t n) { const size_t o = b.floats; b.floats += (n + 63) & ~(size_t)63; return o; };
+    for (const Made& m : made)
+      if (m.share >= 0 && need(m) > common[m.share]) common[m.share] = need(m);
+    for (size_t& c : common) c = take(c);
+    for (const Made& m : made) {
+      Ring t = m.ring;
+      t.p = nullptr;
+      t.rs = rs(m);
+      t.mask = 0x7fffffff;
+      t.tstep = 0;
+      b.twins.push_back(t);
+      b.at.push_back(m.share >= 0 ? common[m.share] : take(need(m)));
+    }
+    return b;
+  }
+  void histories(const CvBlock& b, std::vector<CvHist>& out) const {
+    for (const Made& m : made)
+      if (keeps(m)) out.push_back(CvHist{m.ring, b.at[m.ring.id], b.twins[m.ring.id].rs, m.C});
   }
 };
 static Ring no_ring() { Ring r; r.p = nullptr; r.rs = 1; r.mask = 0; r.pad = 0; r.tstep = 0; r.id = -1; return r; }
@@ -1471,7 +1481,7 @@ static CvScratch cv_plan(CvGemm& g) {
 
 // Lays out the workspace and (when tensors != nullptr) packs weights and records the launch plan.
 static int cv_build(vui_codec* cc, const vui_codec_config* c, const void* const* tensors, char* ws, hipStream_t st, int64_t* need,
-                    size_t part_cap, size_t cnt_cap, size_t* part_need, size_t* cnt_need, int64_t* block_need = nullptr) {
+                    size_t part_cap, size_t cnt_cap, size_t* part_need, size_t* cnt_need, int frames = 0, int64_t* block_need = nullptr) {
   Arena ar{ws};
   const bool real = ws != nullptr && tensors != nullptr;
   int ti = 0;
@@ -1516,7 +1526,7 @@ static int cv_build(vui_codec* cc, const vui_codec_config* c, const void* const*
     g.in = in; g.in_mode = IN_PLAIN; g.eps = 1e-6f; g.epi = EPI_NONE;
     g.res = no_ring(); g.out_raw = no_ring(); g.out_act = no_ring(); g.ctr = ctr; g.nf = 1;
     g.part = part; g.cnt = cnt;
-    for (int n = block_frames(*c); n >= 1; --n) {  // the frame's own plan is made last and stays
+    for (int n = real || part_need ? block_frames(*c) : 1; n >= 1; --n) {  // the frame's own plan is made last and stays
       g.T = n * T;
       g.nf = n;
       const CvScratch need = cv_plan(g);
@@ -1542,7 +1552,7 @@ static int cv_build(vui_codec* cc, const vui_codec_config* c, const void* const*
     }
   }
   // ---- state region (zeroed by reset) starts here: all rings ----
-  RingMaker rings{ar, block_frames(*c)};
+  RingMaker rings{ar};
   const size_t state_begin = ar.off;
   Ring pre_in = rings.make(c->vq_dim, 2, 1, true);
   std::vector<Ring> dw_in, tc_in, ru_in;
@@ -1742,9 +1752,9 @@ static int cv_build(vui_codec* cc, const vui_codec_config* c, const void* const*
       cc->fin.in = fin_in; cc->fin.w = fwp; cc->fin.b = fbp; cc->fin.audio = nullptr; cc->fin.C = dim; cc->fin.k = 7; cc->fin.T = hop; cc->fin.ctr = ctr; cc->fin.nf = 1;
     }
   }
-  const size_t twin_floats = rings.place();
-  if (block_need) *block_need = (int64_t)twin_floats * 4;
-  CvHist* hist_dev = (CvHist*)ar.take((sizeof(CvHist) * rings.hist.size() + 3) / 4);
+  if (block_need) *block_need = (int64_t)rings.block(frames).floats * 4;
+  const int n_hist = rings.histories(), n_blocks = block_frames(*c) + 1;
+  CvHist* hist_dev = (CvHist*)ar.take((sizeof(CvHist) * n_hist * n_blocks + 3) / 4);
   if (need) *need = (int64_t)ar.off;
   if (part_need) *part_need = part_floats;
   if (cnt_need) *cnt_need = cnt_ints;
@@ -1760,8 +1770,13 @@ static int cv_build(vui_codec* cc, const vui_codec_config* c, const void* const*
       hipLaunchKernelGGL(cv_fill_kernel, g, dim3(256), 0, st, (float*)ll, ll_words * 2, 0.0f);
       hipLaunchKernelGGL(cv_fill_kernel, dim3(1), dim3(64), 0, st, (float*)tctl, (size_t)16, 0.0f);
     }
-    HIP_TRY(hipMemcpyAsync(hist_dev, rings.hist.data(), sizeof(CvHist) * rings.hist.size(), hipMemcpyHostToDevice, st));
-    HIP_TRY(hipStreamSynchronize(st));  // tl and rings go out of scope
+    std::vector<CvHist> hist;
+    for (int n = 0; n < n_blocks; ++n) {
+      cc->blocks.push_back(rings.block(n));
+      rings.histories(cc->blocks[n], hist);
+    }
+    HIP_TRY(hipMemcpyAsync(hist_dev, hist.data(), sizeof(CvHist) * hist.size(), hipMemcpyHostToDevice, st));
+    HIP_TRY(hipStreamSynchronize(st));  // tl and hist go out of scope
     cc->trunk = tk;
     cc->trunk_steps = trunk_steps;
     if (part_floats > part_cap || cnt_ints > cnt_cap) { vui_set_error("codec: internal scratch sizing"); return VUI_EINVAL; }
@@ -1769,10 +1784,7 @@ static int cv_build(vui_codec* cc, const vui_codec_config* c, const void* const*
     cc->state0 = (float*)(ws + state_begin);
     cc->state_floats = (state_end - state_begin) / 4;
     cc->hist = hist_dev;
-    cc->n_hist = (int)rings.hist.size();
-    cc->twins = rings.twins;
-    cc->twin_at = rings.at;
-    cc->block_bytes = (int64_t)twin_floats * 4;
+    cc->n_hist = n_hist;
     cc->vqx = vqx.id; cc->qkv = qkv.id; cc->att = att.id;
     cc->vq.codes = nullptr; cc->vq.n_q = 0; cc->vq.n_sem = c->n_semantic; cc->vq.CS = CS; cc->vq.cd = cd;
     cc->vq.embed = embed; cc->vq.x = vqx.p; cc->vq.rs = vqx.rs; cc->vq.nf = 1; cc->vq.ctr = ctr; cc->vq.err = ctr + 1; cc->vq.max_seq = c->max_seq;
@@ -1946,10 +1958,16 @@ int32_t vui_codec_block_frames(const vui_codec* c) {
   return block_frames(c->cfg);
 }
 
-int64_t vui_codec_block_scratch_bytes(const vui_codec_config* c) {
-  if (cv_check(c)) return VUI_EINVAL;
+static int block_check(const vui_codec_config& c, int32_t n_frames) {
+  if (n_frames >= 1 && n_frames <= block_frames(c)) return VUI_OK;
+  vui_set_error("codec: %d frames outside [1, %d]", n_frames, block_frames(c));
+  return VUI_EINVAL;
+}
+
+int64_t vui_codec_block_scratch_bytes(const vui_codec_config* c, int32_t n_frames) {
+  if (cv_check(c) || block_check(*c, n_frames)) return VUI_EINVAL;
   int64_t need = 0;
-  if (cv_build(nullptr, c, nullptr, nullptr, nullptr, nullptr, 0, 0, nullptr, nullptr, &need)) return VUI_EINVAL;
+  if (n_frames > 1 && cv_build(nullptr, c, nullptr, nullptr, nullptr, nullptr, 0, 0, nullptr, nullptr, n_frames, &need)) return VUI_EINVAL;
   return need;
 }
 
@@ -1958,17 +1976,20 @@ int vui_codec_decode_block(vui_codec* c, const int64_t* codes, int32_t n_frames,
   if (!c) { vui_set_error("NULL codec"); return VUI_EINVAL; }
   if (!codes || !audio_out) { vui_set_error("NULL argument"); return VUI_EINVAL; }
   if (n_q < 1 || n_q > c->cfg.n_codebooks) { vui_set_error("n_q=%d outside [1,%d]", n_q, c->cfg.n_codebooks); return VUI_EINVAL; }
-  if (n_frames < 1 || n_frames > block_frames(c->cfg)) { vui_set_error("codec: %d frames outside [1, %d]", n_frames, block_frames(c->cfg)); return VUI_EINVAL; }
+  if (block_check(c->cfg, n_frames)) return VUI_EINVAL;
   if (n_frames == 1) return vui_codec_decode_frame(c, codes, n_q, audio_out, stream);
   if (!scratch || ((uintptr_t)scratch) & 255) { vui_set_error("codec: the scratch memory must be given and 256-byte aligned"); return VUI_EINVAL; }
-  if (scratch_bytes < c->block_bytes) { vui_set_error("codec: scratch too small: %lld < %lld", (long long)scratch_bytes, (long long)c->block_bytes); return VUI_ENOMEM; }
+  const CvBlock& block = c->blocks[n_frames];
+  const CvHist* hist = c->hist + (size_t)n_frames * c->n_hist;
+  const int64_t need = (int64_t)block.floats * 4;
+  if (scratch_bytes < need) { vui_set_error("codec: scratch too small: %lld < %lld", (long long)scratch_bytes, (long long)need); return VUI_ENOMEM; }
   hipStream_t st = (hipStream_t)stream;
-  auto buf = [&](int id) { Ring t = c->twins[id]; t.p = (float*)scratch + c->twin_at[id]; return t; };
+  auto buf = [&](int id) { Ring t = block.twins[id]; t.p = (float*)scratch + block.at[id]; return t; };
   auto twin = [&](const Ring& r) { return r.id < 0 ? r : buf(r.id); };
   CvVq vq = c->vq;
   vq.codes = codes; vq.n_q = n_q; vq.nf = n_frames; vq.x = buf(c->vqx).p; vq.rs = buf(c->vqx).rs;
   hipLaunchKernelGGL(cv_vq_kernel, dim3(n_frames), dim3(256), 0, st, vq);
-  hipLaunchKernelGGL(cv_history_kernel, dim3(16, c->n_hist), dim3(256), 0, st, c->hist, (float*)scratch, c->ctr, n_frames, 0);
+  hipLaunchKernelGGL(cv_history_kernel, dim3(16, c->n_hist), dim3(256), 0, st, hist, (float*)scratch, c->ctr, n_frames, 0);
   for (const Step& s0 : c->steps) {
     Step s = s0;
     if (s.kind == 0) {
@@ -1989,7 +2010,7 @@ int vui_codec_decode_block(vui_codec* c, const int64_t* codes, int32_t n_frames,
       hipLaunchKernelGGL(cv_dwln_kernel, dim3(s.g.T * n_frames), dim3(256), 0, st, s.d);
     }
   }
-  hipLaunchKernelGGL(cv_history_kernel, dim3(16, c->n_hist), dim3(256), 0, st, c->hist, (float*)scratch, c->ctr, n_frames, 1);
+  hipLaunchKernelGGL(cv_history_kernel, dim3(16, c->n_hist), dim3(256), 0, st, hist, (float*)scratch, c->ctr, n_frames, 1);
   CvFinal fin = c->fin;
   fin.audio = audio_out; fin.nf = n_frames; fin.T *= n_frames; fin.in = twin(fin.in);
   hipLaunchKernelGGL(cv_final_kernel, dim3((fin.T + FIN_TW - 1) / FIN_TW), dim3(256), (size_t)(fin.C * (FIN_TW + fin.k - 1) + 256 + fin.C * fin.k) * 4, st, fin);
