@@ -344,3 +344,27 @@ def test_a_failed_capture_leaves_the_rows_slots():
     e.decode_step(rows, toks)
     assert e.seen.pop() == full and e.writes == writes + 2
     assert [r._length for r in rows] == [4, 4, 3]
+
+
+def test_less_memory_means_shorter_passes(monkeypatch):
+    """Where the workspace of passes of 2048 positions cannot be had the context takes that of 1024; below that it raises."""
+    from vui_amd.lm import TokenLM
+
+    cfg = U.mixed()
+    model = TokenLM.from_config(cfg, U.weights(cfg, 1), device="cpu", max_seqlen=2304)
+    model.allocate_cache(2)
+    assert model._native.max_rows == 2048
+    zeros, full = torch.zeros, model._native.workspace.numel()
+
+    def short(*a, **kw):
+        if kw.get("dtype") == torch.uint8 and a[0] >= limit:
+            raise torch.OutOfMemoryError("out of memory")
+        return zeros(*a, **kw)
+
+    monkeypatch.setattr(torch, "zeros", short)
+    limit = full
+    model.allocate_cache(2)
+    assert model._native.max_rows == 1024 and model._native.workspace.numel() < full
+    limit = model._native.workspace.numel()
+    with pytest.raises(torch.OutOfMemoryError):
+        model.allocate_cache(2)

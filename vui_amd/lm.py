@@ -94,10 +94,18 @@ class _NativeLM:
                 L.c_cache, L.kr_cache = cache.c[src].data_ptr(), cache.kr[src].data_ptr()
         w = _lib.LmWeightsC()
         w.embed, w.head, w.final_norm = model.embed.data_ptr(), model.head.data_ptr(), model.final_norm.data_ptr()
-        nbytes = lib.vui_lm_workspace_bytes(C.byref(c), layers)
-        if nbytes < 0:
-            raise RuntimeError(f"vui_lm_workspace_bytes: {_lib.last_error()}")
-        self.workspace = torch.zeros(nbytes + 256, dtype=torch.uint8, device=model.device)
+        while True:
+            nbytes = lib.vui_lm_workspace_bytes(C.byref(c), layers)
+            if nbytes < 0:
+                raise RuntimeError(f"vui_lm_workspace_bytes: {_lib.last_error()}")
+            try:
+                self.workspace = torch.zeros(nbytes + 256, dtype=torch.uint8, device=model.device)
+                break
+            except torch.OutOfMemoryError:  # prompts then take more passes
+                if c.max_rows <= model.PREFILL_LEAST:
+                    raise
+                c.max_rows = max(c.max_rows // 2, model.PREFILL_LEAST)
+        self.max_rows = c.max_rows
         base = (self.workspace.data_ptr() + 255) & ~255
         h = C.c_void_p()
         _lib.check(lib.vui_lm_create(C.byref(c), layers, C.byref(w), base, nbytes, C.byref(h)), "vui_lm_create")
@@ -117,7 +125,10 @@ class _NativeLM:
 class TokenLM:
     """Decoder-only token model: weights in the kernels' layout, prefill and decode over a slot cache."""
 
-    PREFILL_CHUNK = 2048  # most positions of one native prefill call
+    # Most positions of one native prefill call.  They size the workspace (width 2048, 8 parallel layers: 246 MB, for 1024
+    # positions 140 MB), so where that cannot be had passes are shorter, down to PREFILL_LEAST.
+    PREFILL_CHUNK = 2048
+    PREFILL_LEAST = 1024
 
     def __init__(self, config: LMConfig, state_dict: "dict[str, Tensor]", device="cuda", dtype=torch.bfloat16,
                  max_seqlen: int = 4096):
@@ -265,7 +276,7 @@ class TokenLM:
             raise ValueError(f"wanted positions outside [0, {T})")
         st = torch.cuda.current_stream().cuda_stream
         out = torch.empty(len(want), self.config.vocab, dtype=torch.float32, device=self.device)
-        step = self._config_c(1).max_rows
+        step = min(nat.max_rows, self._config_c(1).max_rows)
         order = sorted(range(len(want)), key=lambda k: want[k])
         for t0 in range(0, T, step):
             n = min(step, T - t0)
