@@ -547,18 +547,25 @@ def test_lengths_of_several_thousand():
             assert U.err(torch.cat(outs), ref) < 2 * TOL[dt]
 
 
-@pytest.mark.parametrize("T", [129, 255, 640, 1024, 1100])
-def test_large_products_of_a_prompt(T):
-    """As in test_gpu_lm: dense layers, whose projections, activations and outputs fill large tiles, against portions of 100."""
+@pytest.fixture(scope="module")
+def large():
+    """As in test_gpu_lm: dense layers, whose projections, activations and outputs fill large tiles."""
     from vui_amd.synthetic import sandwich_lm_config, token_lm_state_dict
 
     cfg = sandwich_lm_config(1000, 8, 2, 120, 6000, 8, 2, 2, vocab=301)
     for layer in cfg["layers"]:
         layer["mlp"] = {"kind": "dense", "ff": 6000}
-    eng = U.engine(cfg, token_lm_state_dict(cfg, 3, "cuda"), torch.bfloat16, max_seq=1152)
-    toks = torch.tensor(U.tokens(T, 301, T))
+    sd, toks = token_lm_state_dict(cfg, 3, "cpu"), U.tokens(1100, 301, 1100)
+    return U.engine(cfg, sd, torch.bfloat16, max_seq=1152), torch.tensor(toks), O.forward(cfg, sd, toks)
+
+
+@pytest.mark.parametrize("T", [129, 255, 640, 1024, 1100])
+def test_large_products_of_a_prompt(large, T):
+    """Against 64 bits, and against portions of 100 tokens, which take the small tiles and chunks of other lengths: measured
+    per position at most 0.0085 and 0.0044; sixteen features left out move a row by 0.018 to 0.08 in the median."""
+    eng, toks, ref = large
     with eng.new_row() as row:
-        whole = row.extend(toks, range(T)).clone()
+        whole = row.extend(toks[:T], range(T)).clone()
         row.reset()
-        parts = torch.cat([row.extend(toks[i:i + 100], range(len(toks[i:i + 100]))).clone() for i in range(0, T, 100)])
-    assert U.err(whole, parts) < TOL[torch.bfloat16]
+        parts = torch.cat([row.extend(toks[i:min(i + 100, T)], range(min(100, T - i))).clone() for i in range(0, T, 100)])
+    assert U.err(whole, ref[:T]) < 0.015 and U.err(whole, parts) < 0.012
