@@ -205,16 +205,20 @@ def test_prefill_tiles_of_every_size(int8):
 
 @pytest.mark.parametrize("int8", [False, True])
 def test_large_tiles_add_as_the_small_ones_do(int8):
-    """A pass whose products take large tiles against portions that take 32 x 32 tiles: both add the same four parts of K in
-    the same order, and a query's attention does not depend on its portion, so every bit is the same."""
+    """Passes whose products take large tiles (the lengths choose all three for QKV and the pair, two for the others), some
+    ending inside one, against portions of 576 positions, which take 32 x 32 tiles: all add the same four parts of K in the
+    same order, and a query's attention does not depend on its portion, so every bit is the same."""
     d = O.Dims(n_layers=2)
-    m = make_model(d, O.synthetic_state_dict(d, seed=2), BF, int8=int8, max_seqlen=1280)
-    m.decoder.allocate_flash_kv_cache(1, m.device, BF, max_seqlen=1280)
-    x = (torch.randn(1, 1260, d.d_model, generator=torch.Generator().manual_seed(5)) * 0.08).to(BF).cuda()
-    outs = []
-    for portion in (1260, 420):
+    m = make_model(d, O.synthetic_state_dict(d, seed=2), BF, int8=int8, max_seqlen=1792)
+    m.decoder.allocate_flash_kv_cache(1, m.device, BF, max_seqlen=1792)
+    x = (torch.randn(1, 1728, d.d_model, generator=torch.Generator().manual_seed(5)) * 0.08).to(BF).cuda()
+
+    def run(T, portion):
         m.decoder.flash_kv_caches[0].seq_lens.zero_()
-        h = torch.cat([m.decoder.forward_flash(x[:, i:i + portion].contiguous(), None) for i in range(0, 1260, portion)], dim=1)
-        outs.append((h, m.decoder._k[:, 0, :1260].clone(), m.decoder._v[:, 0, :1260].clone()))
-    for a, b in zip(*outs):
-        assert torch.equal(a, b)
+        h = torch.cat([m.decoder.forward_flash(x[:, i:i + portion].contiguous(), None) for i in range(0, T, portion)], dim=1)
+        return h, m.decoder._k[:, 0, :T].clone(), m.decoder._v[:, 0, :T].clone()
+
+    want = run(1728, 576)
+    for T in (397, 700, 1000, 1233, 1600):
+        h, k, v = run(T, T)
+        assert torch.equal(h, want[0][:, :T]) and torch.equal(k, want[1][:, :T]) and torch.equal(v, want[2][:, :T]), T
