@@ -1464,7 +1464,7 @@ static CvScratch cv_plan(CvGemm& g) {
   for (int tt : {2, 4})
     if (T > 8 * tt && tiles(tt) * tt <= tiles(g.tt) * g.tt) g.tt = tt;
   // a tile of 64 columns holds 3 units per wave and round, one of 32 columns 6: the narrower one where that saves the second
-  // round (192 channels x 640 columns: 18.8 / 11.5 us)
+  // round (192 channels x 640 columns: 19.2 / 13.1 us)
   if (g.tt == 4 && U > 24 && U <= 48 && tiles(2) <= 256) g.tt = 2;
   int sp = 1;
   if (U >= 64) {

@@ -6,7 +6,7 @@
 // over the waves of a 32 x 32 or 64 x 64 tile every wave fetches all its operands from L2 (16 flops per byte).  Here the
 // waves share a tile through LDS; S stages of KS x 32 columns each are in flight, written to LDS by the loads themselves (a
 // piece of the layout is 1 KiB in lane order on both sides), and a wave waits only for the oldest.
-// 1024 x 11776 x 2048 without an epilogue: 61 us = 808 TFLOP/s (hipBLASLt reaches 1125 at 8192^3).
+// 1024 x 11776 x 2048 without an epilogue: 63 us = 780 TFLOP/s (62 with one chain of sums; hipBLASLt reaches 1125 at 8192^3).
 #pragma once
 #include "tile.h"
 
@@ -133,8 +133,9 @@ struct WideTile {
 // Which tile takes an M x N x K product, or none (the K-splitting kernels: quicker for the smaller products, at 0.38 us per
 // thousand 32 x 32 tiles and 64 columns, and kept unless `keep` of that is still more).  Estimated microseconds besides the launch and the
 // epilogue (MI355X): a step of 32 columns takes a tile `wait` us when its CU has nothing else to do and `work` us per tile
-// when it has.  Measured (us, K-splitting / large tile): 1024 x 11776 x 2048 147 / 61, 1024 x 2048 x 6144 82 / 39,
-// 1024 x 5120 x 768 26 / 17, 1024 x 768 x 2816 16 / 17, 300 x 768 x 2816 9 / 17.
+// when it has.  Measured (us, K-splitting with its epilogue / quickest large tile without): 1024 x 11776 x 2048 147 / 63,
+// 1024 x 2048 x 6144 82 / 40, 1024 x 5120 x 768 26 / 18, 1024 x 768 x 2816 16 / 14, 300 x 768 x 2816 9 / 14.  The prompt pass of the
+// backbone has estimates of its own.
 enum { WIDE_NONE = -1, WIDE_128 = 0, WIDE_64x128 = 1, WIDE_64 = 2 };
 static inline int wide_pick(int M, int N, int K, double keep) {
   static const struct { int bm, bn; double wait, work; } tile[] = {{128, 128, 0.335, 0.144}, {64, 128, 0.21, 0.08}, {64, 64, 0.17, 0.059}};
