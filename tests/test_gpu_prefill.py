@@ -222,3 +222,40 @@ def test_large_tiles_add_as_the_small_ones_do(int8):
     for T in (397, 700, 1000, 1233, 1600):
         h, k, v = run(T, T)
         assert torch.equal(h, want[0][:, :T]) and torch.equal(k, want[1][:, :T]) and torch.equal(v, want[2][:, :T]), T
+
+
+@pytest.mark.parametrize("heads,kv,window", [(4, 2, 0), (8, 8, 70), (2, 1, 0), (2, 2, 300)])
+def test_short_blocks_behind_a_cache(heads, kv, window):
+    """Short blocks at their edges (one position, tiles of 16 rows, the longest) and the next longer block, behind caches that are
+    empty, end inside a step of 32 keys or inside a workgroup's range of keys, and are long enough for every number of ranges and
+    more; heads of 64, 32 and 128, a window.  The block's outputs and what it appends, against the position-by-position path behind
+    the same cache.  Embeddings start at an odd address."""
+    from tests.util import dims_to_config
+    from vui_amd.model import Vui
+
+    d = O.Dims(d_model=256, n_layers=2, n_heads=heads, n_kv_heads=kv, n_quantizers=4, codebook_size=32, rq_d_model=64, rq_n_layers=1,
+               rq_n_heads=2, vocab_size=50, max_seqlen=1280)
+    cfg = dims_to_config(d, 1280)
+    cfg.model.window_size = window or None
+    m = Vui(cfg, O.synthetic_state_dict(d, **TINY_SD), device="cuda", dtype=BF)
+    m.decoder.allocate_flash_kv_cache(1, m.device, BF)
+    seq = m.decoder.flash_kv_caches[0].seq_lens
+    x = (torch.randn(1, 1200, d.d_model, generator=torch.Generator().manual_seed(8)) * 0.5).to(BF).cuda()
+    m.decoder.forward_flash(x, None)
+    for pos in (0, 3, 126, 129, 257, 640, 1130):
+        for T in (1, 16, 17, 33, 64, 65):
+            block = torch.empty(T * d.d_model + 1, dtype=BF, device="cuda")[1:].view(1, T, d.d_model)
+            block.copy_(x[:, :T])
+            outs = []
+            for minimum in (1, 10 ** 9):
+                seq.fill_(pos)
+                m.decoder.PREFILL_MIN = minimum
+                h = m.decoder.forward_flash(block, None)
+                outs.append((h, m.decoder._k[:, 0, pos:pos + T].clone(), m.decoder._v[:, 0, pos:pos + T].clone()))
+                assert int(seq[0]) == pos + T
+            for a, b in zip(*outs):
+                assert rel_err(a, b) <= BF16_TOL, (pos, T, rel_err(a, b))
+            m.decoder.PREFILL_MIN = 4
+            if pos == 0:  # the cache the other offsets stand on
+                seq.fill_(0)
+                m.decoder.forward_flash(x, None)

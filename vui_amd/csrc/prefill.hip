@@ -3,11 +3,12 @@
 //   Decoder.forward_flash / Engine._prefill_emb with T > 1  (src/vui/model.py:534-549, engine.py:674-694)
 //
 // bf16 activations; the layers' matrices bf16, or int8 with per-row scales (widened in registers inside the GEMMs,
-// the scale on the finished sum).  Per layer: row RMSNorm, QKV GEMM, one kernel that rotates the new keys, appends keys and values to the
-// cache and stages the slot's keys / transposed values in operand layout, causal attention of the new positions
-// against them (the same kernel rotates the queries in place; scores never leave the registers; probabilities
+// the scale on the finished sum).  Per layer: row RMSNorm, QKV GEMM whose epilogue rotates queries and keys, appends keys and
+// values to the cache and leaves both in the attention's operand layout (behind earlier positions a kernel lays out the whole slot
+// instead: the copy of those costs the launch anyway), causal attention of the new positions (scores never leave the registers; probabilities
 // rounded to bf16 before they meet the values), out_proj GEMM with the residual add in its epilogue, row RMSNorm, one GEMM over
-// W1 and W3 with the SwiGLU product in its epilogue, W2 GEMM with residual: eight launches.
+// W1 and W3 with the SwiGLU product in its epilogue, W2 GEMM with residual: seven launches, eight behind earlier positions.
+// A short block (up to PF_SHORT positions) takes five: its GEMMs norm their rows themselves, and attention reads the cache as it is.
 // Every GEMM is C (M x N) = X (M x K) W^T (N x K) on the matrix cores, both operands in the tiled layout below.
 //
 // Rounding points are those of the single-position step (one rounding after each linear, two in
@@ -21,7 +22,7 @@ typedef tl_bf16x8 pf_bf16x8;
 typedef tl_f32x4 pf_floatx4;
 __device__ __forceinline__ pf_bf16x8 pf_frag(const uint4& x) { return Tl<bf16_t>::frag(x); }
 
-enum { PF_BF16 = 0, PF_RESID = 1 };
+enum { PF_BF16 = 0, PF_RESID = 1, PF_QKV = 2 };
 
 // Both operands of the GEMMs are in the tiled layout of tile.h (blocks of 16 rows x 64 columns).  Weights are brought
 // into this form once per context, activations are written in it by their producers.
@@ -35,7 +36,102 @@ struct PfGemm {
   const bf16_t *sc, *sc2;
   void* C;           // output (M x N) bf16: row-major with row stride ldc (PF_RESID: in place on the residual), or tiled
   int M, N, K, ldc;
+  // X is the residual and is normed on its way: sums of squares of every 16 columns (M x K / 16), weights (K)
+  const float* ssq;
+  const bf16_t* nw;
+  float eps;
+  float* ssq_out;    // PF_RESID: the same sums of the new residual, or nullptr
+  // PF_QKV: C receives the rotated queries alone; row m is position pos0 + m of the slot
+  bf16_t *kc, *vc;   // its cache rows
+  bf16_t *kt, *vt;   // operand copies of keys and transposed values (pf_stage_kv_kernel), or nullptr
+  const float* rope;
+  int nq, nkv, hd, rope_dim, pos0, Lpad;
+  // pf_order: tiles of an XCD (the first xcd_more have one more), tiles of one step of the slower index
+  uint32_t xcd_tiles, xcd_more, run, inv_run, inv_hd;
+  int by_rows, n_tiles;
+  int warm, warm_from;  // the last `warm` workgroups only fetch the cached positions warm_from .. pos0 - 1 (see pf_warm)
 };
+
+// i / n for i < 65536 with inv = pf_inv(n): a division by a runtime value costs a workgroup 0.1 us
+static uint32_t pf_inv(uint32_t n) { return n > 1 ? 0xFFFFFFFFu / n + 1u : 0u; }
+__device__ __forceinline__ uint32_t pf_div(uint32_t i, uint32_t inv) { return inv ? __umulhi(i, inv) : i; }
+
+// The attention of a short block is a few workgroups that wait for cached keys and values from memory (2.4 us of its first
+// step, 0.85 where they are in the memory-side cache).  The QKV product before it leaves compute units idle: workgroups of
+// its launch that have no tile read them ahead.
+__device__ __forceinline__ void pf_warm(const PfGemm& p, int part) {
+  const size_t n = (size_t)(p.pos0 - p.warm_from) * p.nkv / 8, at = (size_t)p.warm_from * p.nkv;
+  for (size_t i = (size_t)part * blockDim.x + threadIdx.x; i < n; i += (size_t)p.warm * blockDim.x) {
+    const uint4 k = *reinterpret_cast<const uint4*>(p.kc + at + i * 8), v = *reinterpret_cast<const uint4*>(p.vc + at + i * 8);
+    asm volatile("" ::"v"(k.x), "v"(v.x));
+  }
+}
+
+// Which tile (of MT x NT) a workgroup takes: {row tile, feature tile}.  Workgroups go round the eight XCDs, whose L2s are their
+// own, so each XCD gets a contiguous range of the tiles: of the feature tiles where the weights are more bytes than the rows - it then
+// meets an eighth of the weights and all rows - and of the row tiles otherwise.
+// Whole pass, us, in order of dispatch / so: bf16 300 positions 988 / 916, 576 1246 / 1145, 1733 2155 / 2070; int8 300 833 / 789, 1733
+// 2194 / 1951.  The line lies at twice the rows' bytes, since the rows were written just before (576 positions at equal bytes: 1180).
+__device__ __forceinline__ int2 pf_order(const PfGemm& p) {
+  const uint32_t x = blockIdx.x & 7u;
+  const uint32_t id = x * p.xcd_tiles + min(x, p.xcd_more) + (blockIdx.x >> 3), q = pf_div(id, p.inv_run), r = id - q * p.run;
+  return p.by_rows ? make_int2(q, r) : make_int2(r, q);
+}
+
+// rotation factors of features n .. n + 3 (n % 4 == 0) of a head whose first rope_dim features turn: cos, sin of two pairs
+struct PfRot { float4 a, b; };
+__device__ __forceinline__ PfRot pf_rot(const float* rope, int pos, int rope_dim, int dd) {
+  PfRot r;
+  const float* f = rope + (size_t)pos * rope_dim * 2;
+  r.a = *reinterpret_cast<const float4*>(f + min(dd, rope_dim - 2) * 2);
+  r.b = *reinterpret_cast<const float4*>(f + min(dd + 2, rope_dim - 2) * 2);
+  return r;
+}
+// Where a block of 16 features that begins at n (uniform over the wave) lies: queries, keys or values, its head there, its first
+// dimension in the head (a multiple of 16), and for keys and values its column in a cache row
+struct PfPart { int part, head, dim, col; };
+__device__ __forceinline__ PfPart pf_part(const PfGemm& p, int n) {
+  PfPart r;
+  r.part = n < p.nq ? 0 : (n < p.nq + p.nkv ? 1 : 2);
+  r.col = n - (r.part == 0 ? 0 : (r.part == 1 ? p.nq : p.nq + p.nkv));
+  r.head = pf_div(r.col, p.inv_hd);
+  r.dim = r.col - r.head * p.hd;
+  return r;
+}
+// Epilogue of PF_QKV for features 4 kg .. 4 kg + 3 of such a block, row m: v is rounded, the interleaved pairs of queries and keys are
+// rotated (src/vui/rope.py:16-77), keys and values appended to the cache (src/vui/model.py:234-247), keys laid out for pf_attn_kernel.
+__device__ __forceinline__ void pf_qkv_out(const PfGemm& p, const PfPart& b, int m, int kg, const float* v, const PfRot& rot) {
+  float o[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) o[r] = bf2f(f2bf(v[r]));
+  const int dd = b.dim + 4 * kg, col = b.col + 4 * kg, j = p.pos0 + m;
+  if (b.part < 2) {
+    const float a = rope_mix(o[0], rot.a.x, -o[1], rot.a.y), c = rope_mix(o[1], rot.a.z, o[0], rot.a.w);
+    const float e = rope_mix(o[2], rot.b.x, -o[3], rot.b.y), f = rope_mix(o[3], rot.b.z, o[2], rot.b.w);
+    if (dd < p.rope_dim) { o[0] = a; o[1] = c; }
+    if (dd + 2 < p.rope_dim) { o[2] = e; o[3] = f; }
+  }
+  const uint2 w = make_uint2(f2bf2(o[0], o[1]), f2bf2(o[2], o[3]));
+  if (b.part == 0) {
+    *reinterpret_cast<uint2*>((bf16_t*)p.C + (size_t)m * p.ldc + col) = w;
+  } else if (b.part == 1) {
+    *reinterpret_cast<uint2*>(p.kc + (size_t)j * p.nkv + col) = w;
+    if (p.kt) {
+      const size_t blk = ((size_t)b.head * (p.Lpad >> 4) + (j >> 4)) * (p.hd >> 5) + (dd >> 5);
+      *reinterpret_cast<uint2*>(p.kt + blk * 512 + ((j & 15) + 16 * ((dd & 31) >> 3)) * 8 + (dd & 7)) = w;
+    }
+  } else {
+    *reinterpret_cast<uint2*>(p.vc + (size_t)j * p.nkv + col) = w;
+  }
+}
+// The values of feature l16 of such a block in rows m .. m + 3 (m % 4 == 0), into the transposed layout
+__device__ __forceinline__ void pf_vt_out(const PfGemm& p, const PfPart& b, int m, int l16, const float* v) {
+  const size_t blk0 = ((size_t)b.head * (p.hd >> 4) + (b.dim >> 4)) * (p.Lpad >> 5);
+  auto at = [&](int j) { return p.vt + (blk0 + (j >> 5)) * 512 + (l16 + 16 * ((j & 15) >> 2)) * 8 + 4 * ((j & 31) >> 4) + (j & 3); };
+  const int j = p.pos0 + m;
+  if (!(p.pos0 & 3) && m + 3 < p.M) { *reinterpret_cast<uint2*>(at(j)) = make_uint2(f2bf2(v[0], v[1]), f2bf2(v[2], v[3])); return; }
+  for (int r = 0; r < 4; ++r) if (m + r < p.M) *at(j + r) = f2bf(v[r]);
+}
 
 // row-major (N x K) -> tiled; one 8-element piece per thread
 __global__ __launch_bounds__(256) void pf_tile_kernel(const bf16_t* __restrict__ src, bf16_t* __restrict__ dst, int N, int K) {
@@ -46,6 +142,17 @@ __global__ __launch_bounds__(256) void pf_tile_kernel(const bf16_t* __restrict__
   *reinterpret_cast<uint4*>(dst + pf_toff(n, k, K)) = *reinterpret_cast<const uint4*>(src + (size_t)n * K + k);
 }
 
+// eight residual values of one row -> normed: rnd(rnd(x r) g)
+__device__ __forceinline__ uint4 pf_norm8(const uint4& x, float r, const uint4& g) {
+  uint4 o;
+  uint32_t t;
+  t = f2bf2(bf_lo(x.x) * r, bf_hi(x.x) * r); o.x = f2bf2(bf_lo(t) * bf_lo(g.x), bf_hi(t) * bf_hi(g.x));
+  t = f2bf2(bf_lo(x.y) * r, bf_hi(x.y) * r); o.y = f2bf2(bf_lo(t) * bf_lo(g.y), bf_hi(t) * bf_hi(g.y));
+  t = f2bf2(bf_lo(x.z) * r, bf_hi(x.z) * r); o.z = f2bf2(bf_lo(t) * bf_lo(g.z), bf_hi(t) * bf_hi(g.z));
+  t = f2bf2(bf_lo(x.w) * r, bf_hi(x.w) * r); o.w = f2bf2(bf_lo(t) * bf_lo(g.w), bf_hi(t) * bf_hi(g.w));
+  return o;
+}
+
 // C = X W^T for the projections (K = d_model ... ffn; 64 x 64 tiles would give only 9 x 12 ... 9 x 64
 // workgroups at 576 positions, each a long serial walk over K): a workgroup owns 16 MB rows x 16 NB features and its waves
 // split the K steps between them, so a wave's chain of dependent trips to memory is a fraction as long and more
@@ -53,16 +160,20 @@ __global__ __launch_bounds__(256) void pf_tile_kernel(const bf16_t* __restrict__
 // results do not depend on timing).
 // DUAL: two weight matrices against the same activations, h = rnd(rnd(silu(rnd(a))) * rnd(c)) written once
 // (SwiGLU, src/vui/model.py:282) instead of two products and a pass over both.
-template <int EPI, bool DUAL, bool I8, int WAVES, int MB, int NB>
+// NORM: X is the residual; every wave norms the fragments it multiplies (two roundings, src/vui/model.py:286-297) with the
+// rows' factors from sums of squares that the residual's producer left in pieces of 16 columns.  That costs a launch of a
+// short block 0.5-1.7 us (16 positions: QKV 3.8 -> 5.5, W1 and W3 5.0 -> 5.5) and saves the norm's own of 3.4; repeated for every
+// tile of features it does not pay for longer ones.
+template <int EPI, bool DUAL, bool I8, int WAVES, int MB, int NB, bool NORM>
 __global__ __launch_bounds__(64 * WAVES) void pf_gemm_kernel(const PfGemm p, const void* __restrict__ W2, int c_tiled) {
   constexpr int TILE = MB * NB * 256;  // floats of one partial tile
   constexpr int PW = (DUAL ? 2 : 1) * TILE;
   __shared__ __align__(16) float part[WAVES * PW];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int l16 = lane & 15, kg = lane >> 4;
-  const int MT = (p.M + 16 * MB - 1) / (16 * MB);
-  const int id = blockIdx.x;
-  const int m0 = (id % MT) * 16 * MB, n0 = (id / MT) * 16 * NB;
+  if (EPI == PF_QKV && NORM && (int)blockIdx.x >= p.n_tiles) { pf_warm(p, blockIdx.x - p.n_tiles); return; }
+  const int2 tile = pf_order(p);
+  const int m0 = tile.x * 16 * MB, n0 = tile.y * 16 * NB;
   // A step covers 64 values of k, one block of the tiled operands per 16 rows: the lane's 16-byte piece of half h
   // (k = 64 s + 16 kg + 8 h ...; any assignment of k to lanes is valid as long as both operands share it) is at
   // block + 512 h + 8 lane.
@@ -89,35 +200,66 @@ __global__ __launch_bounds__(64 * WAVES) void pf_gemm_kernel(const PfGemm p, con
   // the residual values this thread will add to (its four outputs, see the epilogue) are requested with the first
   // operands instead of after the last product; clamped to the matrix, unused where the thread has no output
   uint2 old = make_uint2(0, 0);
-  if (EPI == PF_RESID) {
+  PfRot rot = {};
+  {
     const int em = min(m0 + 16 * (wave % MB) + l16, p.M - 1), en = min(n0 + 16 * (wave / MB % NB) + 4 * kg, p.N - 4);
-    old = *reinterpret_cast<const uint2*>((const bf16_t*)p.C + (c_tiled ? pf_toff(em, en, p.N) : (size_t)em * p.ldc + en));
+    if (EPI == PF_RESID) old = *reinterpret_cast<const uint2*>((const bf16_t*)p.C + (c_tiled ? pf_toff(em, en, p.N) : (size_t)em * p.ldc + en));
+    if (EPI == PF_QKV && p.rope_dim >= 2) rot = pf_rot(p.rope, p.pos0 + em, p.rope_dim, pf_part(p, min(n0 + 16 * (wave / MB % NB), p.N - 16)).dim + 4 * kg);
   }
-  for (int s = s0; s < s1; ++s) {
+  uint4 xa[MB][2], wa[NB][2], va[NB][2], g[2];
+  auto load = [&](int s) {
     const int k = s << 10;
-    uint4 xa[MB][2], wa[NB][2], va[NB][2];
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        if (I8 && h) continue;  // both halves of an int8 block are one piece
+        wa[j][h] = *reinterpret_cast<const uint4*>(wr[j] + (size_t)s * WB + 1024 * h);
+        if (DUAL) va[j][h] = *reinterpret_cast<const uint4*>(vr[j] + (size_t)s * WB + 1024 * h);
+      }
 #pragma unroll
       for (int j = 0; j < MB; ++j) xa[j][h] = *reinterpret_cast<const uint4*>(xr[j] + k + 512 * h);
+      if (NORM) g[h] = *reinterpret_cast<const uint4*>(p.nw + 64 * s + 16 * kg + 8 * h);
+    }
+  };
+  float rf[MB];
+  if (NORM) {  // the operands of the first step are on their way meanwhile
+    if (s0 < s1) load(s0);
+    __builtin_amdgcn_sched_barrier(0);
+    float ss[MB] = {};
+    for (int i = kg; i < nsteps; i += 16) {
+      float4 t[MB][4];
+#pragma unroll
+      for (int j = 0; j < MB; ++j)
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          t[j][u] = reinterpret_cast<const float4*>(p.ssq + (size_t)min(m0 + 16 * j + l16, p.M - 1) * (p.K >> 4))[min(i + 4 * u, nsteps - 1)];
+#pragma unroll
+      for (int j = 0; j < MB; ++j)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) ss[j] += i + 4 * u < nsteps ? (t[j][u].x + t[j][u].y) + (t[j][u].z + t[j][u].w) : 0.f;
+    }
+#pragma unroll
+    for (int j = 0; j < MB; ++j) rf[j] = 1.0f / sqrtf(rows_sum(ss[j]) / (float)p.K + p.eps);
+  }
+  for (int s = s0; s < s1; ++s) {
+    if (!NORM || s > s0) load(s);
     if (I8) {
 #pragma unroll
       for (int j = 0; j < NB; ++j) {
-        const uint4 w8 = *reinterpret_cast<const uint4*>(wr[j] + (size_t)s * WB);
+        const uint4 w8 = wa[j][0];
         wa[j][0] = widen8_i8(w8.x, w8.y); wa[j][1] = widen8_i8(w8.z, w8.w);
         if (DUAL) {
-          const uint4 v8 = *reinterpret_cast<const uint4*>(vr[j] + (size_t)s * WB);
+          const uint4 v8 = va[j][0];
           va[j][0] = widen8_i8(v8.x, v8.y); va[j][1] = widen8_i8(v8.z, v8.w);
         }
       }
-    } else {
+    }
+    if (NORM) {
 #pragma unroll
       for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int j = 0; j < NB; ++j) {
-          wa[j][h] = *reinterpret_cast<const uint4*>(wr[j] + (size_t)s * WB + 1024 * h);
-          if (DUAL) va[j][h] = *reinterpret_cast<const uint4*>(vr[j] + (size_t)s * WB + 1024 * h);
-        }
+        for (int j = 0; j < MB; ++j) xa[j][h] = pf_norm8(xa[j][h], rf[j], g[h]);
     }
 #pragma unroll
     for (int h = 0; h < 2; ++h)
@@ -154,10 +296,29 @@ __global__ __launch_bounds__(64 * WAVES) void pf_gemm_kernel(const PfGemm p, con
       if (DUAL) u[r] += part[w * PW + TILE + e];
     }
   }
-  if (m >= p.M || n >= p.N) return;
+  const bool out = m < p.M && n < p.N;  // N is a multiple of 16
+  if (EPI == PF_QKV && p.vt && n0 + 16 * i >= p.nq + p.nkv && n0 + 16 * i < p.N) {
+    // the tile transposed: feature l16 of rows 4 kg .. 4 kg + 3
+    float t[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int e = (wave * 64 + 4 * kg + r + 16 * (l16 >> 2)) * 4 + (l16 & 3);
+      t[r] = part[e];
+#pragma unroll
+      for (int w = 1; w < WAVES; ++w) t[r] += part[w * PW + e];
+      if (I8) t[r] *= bf2f(p.sc[n0 + 16 * i + l16]);
+    }
+    pf_vt_out(p, pf_part(p, n0 + 16 * i), m0 + 16 * j + 4 * kg, l16, t);
+  }
+  if (EPI != PF_RESID && !out) return;
   if (I8) {  // y[n] = scale[n] * sum_k q[n, k] x[k]
-    for (int r = 0; r < 4; ++r)
-      if (n + r < p.N) { v[r] *= bf2f(p.sc[n + r]); if (DUAL) u[r] *= bf2f(p.sc2[n + r]); }
+    const int ns = min(n, p.N - 4);
+    for (int r = 0; r < 4; ++r) { v[r] *= bf2f(p.sc[ns + r]); if (DUAL) u[r] *= bf2f(p.sc2[ns + r]); }
+  }
+  if (EPI == PF_QKV) {
+    const PfPart blk = pf_part(p, n0 + 16 * i);
+    pf_qkv_out(p, blk, m, kg, v, rot);
+    return;
   }
   bf16_t* c = (bf16_t*)p.C + (c_tiled ? pf_toff(m, n, p.N) : (size_t)m * p.ldc + n);  // n % 4 == 0: inside one piece
   if (DUAL) {
@@ -168,15 +329,16 @@ __global__ __launch_bounds__(64 * WAVES) void pf_gemm_kernel(const PfGemm p, con
     }
   }
   if (EPI == PF_RESID) {  // x = rnd(x + rnd(y)), src/vui/model.py:367, 374
-    if (n + 3 < p.N) {
-      v[0] = bf_lo(old.x) + bf2f(f2bf(v[0])); v[1] = bf_hi(old.x) + bf2f(f2bf(v[1]));
-      v[2] = bf_lo(old.y) + bf2f(f2bf(v[2])); v[3] = bf_hi(old.y) + bf2f(f2bf(v[3]));
-    } else {
-      for (int r = 0; r < 4; ++r) if (n + r < p.N) v[r] = bf2f(c[r]) + bf2f(f2bf(v[r]));
-    }
+    v[0] = bf_lo(old.x) + bf2f(f2bf(v[0])); v[1] = bf_hi(old.x) + bf2f(f2bf(v[1]));
+    v[2] = bf_lo(old.y) + bf2f(f2bf(v[2])); v[3] = bf_hi(old.y) + bf2f(f2bf(v[3]));
   }
-  if (n + 3 < p.N) *reinterpret_cast<uint2*>(c) = make_uint2(f2bf2(v[0], v[1]), f2bf2(v[2], v[3]));
-  else for (int r = 0; r < 4; ++r) if (n + r < p.N) c[r] = f2bf(v[r]);
+  const uint2 w = make_uint2(f2bf2(v[0], v[1]), f2bf2(v[2], v[3]));
+  if (out) *reinterpret_cast<uint2*>(c) = w;
+  if (EPI == PF_RESID && p.ssq_out) {  // uniform; a row's sixteen columns are in the four lanes of its column
+    const float a = bf_lo(w.x), b = bf_hi(w.x), e = bf_lo(w.y), f = bf_hi(w.y);
+    const float ss = rows_sum((a * a + b * b) + (e * e + f * f));
+    if (out && kg == 0) p.ssq_out[(size_t)m * (p.N >> 4) + (n >> 4)] = ss;
+  }
 }
 
 // The same product for prompts of a few hundred positions and more: large tiles through LDS (wide.h).  DUAL: a wave's first
@@ -189,8 +351,9 @@ __global__ __launch_bounds__(256, 2) void pf_wide_kernel(const PfGemm p, const v
   __shared__ __align__(16) char lds[Tile::LDS];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int l16 = lane & 15, kg = lane >> 4, wm = wave % WM, wn = wave / WM;
-  const int MBL = (p.M + 15) >> 4, NBL = p.N >> 4, MT = (MBL + MB - 1) / MB;
-  const int mb0 = (int)blockIdx.x % MT * MB, nb0 = (int)blockIdx.x / MT * NB;
+  const int MBL = (p.M + 15) >> 4, NBL = p.N >> 4;
+  const int2 tl = pf_order(p);
+  const int mb0 = tl.x * MB, nb0 = tl.y * NB;
   const size_t xb = (size_t)p.K * 32, wb = (size_t)p.K * (I8 ? 16 : 32);  // bytes of a 16-row block
   Tile tile;
   tile.begin(lds, wave, lane, [&](int i) { return (const char*)p.X + min(mb0 + i, MBL - 1) * xb; },
@@ -220,9 +383,13 @@ __global__ __launch_bounds__(256, 2) void pf_wide_kernel(const PfGemm p, const v
       for (int r = 0; r < 4; ++r) { s1[r] = bf2f(p.sc[n + r]); if (DUAL) s2[r] = bf2f(p.sc2[n + r]); }
     }
     uint2 old[MBW];
+    PfRot rot[MBW] = {};
+    PfPart blk = {};
+    if (EPI == PF_QKV) blk = pf_part(p, nb * 16);
 #pragma unroll
     for (int j = 0; j < MBW; ++j) {
       const int m = min(mw + 16 * j, p.M - 1);
+      if (EPI == PF_QKV && p.rope_dim >= 2 && blk.part < 2) rot[j] = pf_rot(p.rope, p.pos0 + m, p.rope_dim, blk.dim + 4 * kg);
       if (EPI == PF_RESID) old[j] = *reinterpret_cast<const uint2*>((const bf16_t*)p.C + (c_tiled ? pf_toff(m, n, p.N) : (size_t)m * p.ldc + n));
     }
 #pragma unroll
@@ -244,15 +411,32 @@ __global__ __launch_bounds__(256, 2) void pf_wide_kernel(const PfGemm p, const v
         v[0] = bf_lo(old[j].x) + bf2f(f2bf(v[0])); v[1] = bf_hi(old[j].x) + bf2f(f2bf(v[1]));
         v[2] = bf_lo(old[j].y) + bf2f(f2bf(v[2])); v[3] = bf_hi(old[j].y) + bf2f(f2bf(v[3]));
       }
-      if (m < p.M) *reinterpret_cast<uint2*>((bf16_t*)p.C + (c_tiled ? pf_toff(m, n, p.N) : (size_t)m * p.ldc + n)) = make_uint2(f2bf2(v[0], v[1]), f2bf2(v[2], v[3]));
+      if (EPI == PF_QKV) {
+        if (m < p.M) pf_qkv_out(p, blk, m, kg, v, rot[j]);
+        if (blk.part == 2 && p.vt) {  // the block transposed: feature l16 of rows 4 kg .. 4 kg + 3
+          const float* t = reinterpret_cast<const float*>(lds + wave * ROOM * 1024 + (i * MBW + j) * 1024) + (l16 >> 2) * 64 + (l16 & 3);
+          const float sf = I8 ? bf2f(p.sc[nb * 16 + l16]) : 0.f;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[r] = I8 ? t[(4 * kg + r) * 4] * sf : t[(4 * kg + r) * 4];
+          pf_vt_out(p, blk, (mb0 + wm * MBW + j) * 16 + 4 * kg, l16, v);
+        }
+      } else if (m < p.M) *reinterpret_cast<uint2*>((bf16_t*)p.C + (c_tiled ? pf_toff(m, n, p.N) : (size_t)m * p.ldc + n)) = make_uint2(f2bf2(v[0], v[1]), f2bf2(v[2], v[3]));
     }
   }
 }
 
+// the fields of pf_order for tiles of bm x bn; returns their number
+static unsigned pf_set_order(PfGemm& g, int bm, int bn, size_t weight_bytes) {
+  const unsigned MT = (g.M + bm - 1) / bm, NT = (g.N + bn - 1) / bn, n = MT * NT;
+  g.by_rows = weight_bytes < (size_t)g.M * g.K * 4;
+  g.xcd_tiles = n >> 3; g.xcd_more = n & 7; g.run = g.by_rows ? NT : MT; g.inv_run = pf_inv(g.run); g.n_tiles = (int)n;
+  return n;
+}
+
 template <int EPI, bool DUAL, bool I8>
-static int pf_wide(int tile, const PfGemm& g, const void* W2, int c_tiled, hipStream_t st) {
+static int pf_wide(int tile, PfGemm& g, const void* W2, int c_tiled, hipStream_t st) {
   const int bm = tile == WIDE_128 ? 128 : 64, bn = (tile == WIDE_64 ? 64 : 128) / (DUAL ? 2 : 1);
-  const dim3 grid((unsigned)((long)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn)));
+  const dim3 grid(pf_set_order(g, bm, bn, (size_t)g.N * g.K * ((DUAL ? 2 : 1) * (I8 ? 1 : 2))));
   if (tile == WIDE_128) hipLaunchKernelGGL((pf_wide_kernel<EPI, DUAL, I8, 4, 4, 2, 2, I8 ? 3 : 4, I8 ? 2 : 1>), grid, dim3(256), 0, st, g, W2, c_tiled);
   else if (tile == WIDE_64x128) hipLaunchKernelGGL((pf_wide_kernel<EPI, DUAL, I8, 4, 2, 1, 4, I8 ? 4 : 3, 2>), grid, dim3(256), 0, st, g, W2, c_tiled);
   else hipLaunchKernelGGL((pf_wide_kernel<EPI, DUAL, I8, 2, 2, 2, 2, 4, 2>), grid, dim3(256), 0, st, g, W2, c_tiled);
@@ -260,15 +444,17 @@ static int pf_wide(int tile, const PfGemm& g, const void* W2, int c_tiled, hipSt
   return VUI_OK;
 }
 
-// two-rounding RMSNorm of rows (src/vui/model.py:286-297); one wave per row
-__global__ __launch_bounds__(256) void pf_rownorm_kernel(const bf16_t* x, const bf16_t* w, bf16_t* y, int M, int K, float eps, int y_tiled) {
+// two-rounding RMSNorm of rows (src/vui/model.py:286-297); one wave per row.  len != nullptr: the slot's new length goes there
+__global__ __launch_bounds__(256) void pf_rownorm_kernel(const bf16_t* x, const bf16_t* w, bf16_t* y, int M, int K, float eps, int x_tiled,
+                                                         int y_tiled, int32_t* len, int len_to) {
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (len && blockIdx.x == 0 && threadIdx.x == 0) *len = len_to;
   if (row >= M) return;
-  const bf16_t* xr = x + (size_t)row * K;
+  auto xr = [&](int k) { return x + (x_tiled ? pf_toff(row, k, K) : (size_t)row * K + k); };
   float ss = 0.f;
   for (int c = lane; c < K / 8; c += WAVE) {
     float v[8];
-    El<bf16_t>::ld8(xr + c * 8, v);
+    El<bf16_t>::ld8(xr(c * 8), v);
 #pragma unroll
     for (int e = 0; e < 8; ++e) ss = fmaf(v[e], v[e], ss);
   }
@@ -276,7 +462,7 @@ __global__ __launch_bounds__(256) void pf_rownorm_kernel(const bf16_t* x, const 
   const float r = 1.0f / sqrtf(ss / (float)K + eps);
   for (int c = lane; c < K / 8; c += WAVE) {
     float v[8], g[8], o[8];
-    El<bf16_t>::ld8(xr + c * 8, v);
+    El<bf16_t>::ld8(xr(c * 8), v);
     El<bf16_t>::ld8(w + c * 8, g);
 #pragma unroll
     for (int e = 0; e < 8; ++e) o[e] = bf2f(f2bf(v[e] * r)) * g[e];
@@ -284,23 +470,32 @@ __global__ __launch_bounds__(256) void pf_rownorm_kernel(const bf16_t* x, const 
   }
 }
 
-// interleaved rotation (src/vui/rope.py:16-77) of the four pairs of an 8-element piece whose first dim is dd (even)
-// at position pos; pairs at or beyond rope_dim pass through
-__device__ __forceinline__ uint4 pf_rope8(uint4 v, const float* __restrict__ rope, int pos, int rope_dim, int dd) {
-  if (rope_dim < 2) return v;  // uniform
-  uint32_t w[4] = {v.x, v.y, v.z, v.w};
-  // the four factor loads go out together (a pair beyond rope_dim reads the last rotated pair's and ignores it):
-  // behind a branch each, every load would be waited for before the next is issued
-  float4 f[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) f[i] = *reinterpret_cast<const float4*>(rope + ((size_t)pos * rope_dim + min(dd + 2 * i, rope_dim - 2)) * 2);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float a = bf_lo(w[i]), b = bf_hi(w[i]);  // cos, sin of d2 and d2 + 1
-    const uint32_t r = f2bf2(rope_mix(a, f[i].x, -b, f[i].y), rope_mix(b, f[i].z, a, f[i].w));
-    w[i] = (dd + 2 * i < rope_dim) ? r : w[i];
+// The residual of the new positions.  Short block (ssq): tiled, with the sums of squares of every 16 columns of a row, and the
+// attention's arrival counters cleared; otherwise row-major, and the values behind position L in the attention's copy cleared (their weights are zero).  8 columns per thread.
+__global__ __launch_bounds__(256) void pf_begin_kernel(const bf16_t* __restrict__ emb, bf16_t* __restrict__ x, float* __restrict__ ssq,
+                                                       bf16_t* __restrict__ vt, uint32_t* __restrict__ count, int n_count, int T, int d,
+                                                       int nkv, int L, int Lpad) {
+  const int i = blockIdx.x * 256 + threadIdx.x, per_row = d >> 3;
+  if (i < n_count) count[i] = 0;
+  if (i < T * per_row) {  // T d / 8 is a multiple of 8: both lanes of a pair are in
+    const int t = i / per_row, k = (i - t * per_row) * 8;
+    const uint4 v = *reinterpret_cast<const uint4*>(emb + (size_t)i * 8);
+    if (ssq) {
+      float f[8];
+      El<bf16_t>::ld8(reinterpret_cast<const bf16_t*>(&v), f);
+      float ss = ((f[0] * f[0] + f[1] * f[1]) + (f[2] * f[2] + f[3] * f[3])) + ((f[4] * f[4] + f[5] * f[5]) + (f[6] * f[6] + f[7] * f[7]));
+      ss += dpp_f<DPP_QUAD_XOR1>(ss);
+      if (!(k & 8)) ssq[(size_t)t * (d >> 4) + (k >> 4)] = ss;
+      *reinterpret_cast<uint4*>(x + pf_toff(t, k, d)) = v;
+    } else {
+      *reinterpret_cast<uint4*>(x + (size_t)i * 8) = v;
+    }
   }
-  return make_uint4(w[0], w[1], w[2], w[3]);
+  const int n = Lpad - L;
+  if (vt && n > 0 && i < n * nkv) {  // dim by dim of all KV heads
+    const int f = i / n, j = L + i - f * n;
+    vt[((size_t)(f >> 4) * (Lpad >> 5) + (j >> 5)) * 512 + ((f & 15) + 16 * ((j & 15) >> 2)) * 8 + 4 * ((j & 31) >> 4) + (j & 3)] = 0;
+  }
 }
 
 // Attention of the new positions against the row's cache without materialised scores: one workgroup per
@@ -318,9 +513,9 @@ __device__ __forceinline__ uint4 pf_rope8(uint4 v, const float* __restrict__ rop
 // Two tiles of queries per wave or per workgroup, which halves the fetches, measured the same at 1733 and slower below.
 #define PF_ATT_WAVES (HD32 <= 3 ? 8 : 4)  // the partial outputs of the waves must fit 64 KiB of LDS
 template <int HD32>
-__global__ __launch_bounds__(64 * PF_ATT_WAVES, 2) void pf_attn_kernel(const bf16_t* __restrict__ qkv, const bf16_t* __restrict__ kt,
-                                                      const bf16_t* __restrict__ vt, bf16_t* __restrict__ att, int T, int L,
-                                                      int Lpad, int nq, int nkv, int gsz, int pos0, int window, float scale) {
+__global__ __launch_bounds__(64 * PF_ATT_WAVES, 2) void pf_attn_kernel(const bf16_t* __restrict__ qr, const bf16_t* __restrict__ kt,
+                                                      const bf16_t* __restrict__ vt, bf16_t* __restrict__ att, int T, int ldq,
+                                                      int Lpad, int nq, int gsz, int pos0, int window, float scale) {
   constexpr int HD = 32 * HD32, DT = 2 * HD32;
   __shared__ float s_acc[PF_ATT_WAVES][DT * 256];
   __shared__ float s_m[PF_ATT_WAVES][16], s_l[PF_ATT_WAVES][16];
@@ -329,7 +524,6 @@ __global__ __launch_bounds__(64 * PF_ATT_WAVES, 2) void pf_attn_kernel(const bf1
   // neighbouring workgroups take different KV heads (one XCD meets few of them); the tiles with the most keys start first
   const int nkvh = gridDim.x / gsz, kvh = blockIdx.x % nkvh, h = kvh * gsz + blockIdx.x / nkvh;
   const int q0 = (gridDim.y - 1 - blockIdx.y) * 16;
-  const int ldq = nq + 2 * nkv;
   // this lane's query (column of every product below)
   const int tq = min(q0 + l16, T - 1);
   const int qlast = pos0 + tq;                                   // last visible key
@@ -337,7 +531,7 @@ __global__ __launch_bounds__(64 * PF_ATT_WAVES, 2) void pf_attn_kernel(const bf1
   uint4 qf[HD32];
 #pragma unroll
   for (int c = 0; c < HD32; ++c)
-    qf[c] = *reinterpret_cast<const uint4*>(qkv + (size_t)tq * ldq + h * HD + c * 32 + kg * 8);
+    qf[c] = *reinterpret_cast<const uint4*>(qr + (size_t)tq * ldq + h * HD + c * 32 + kg * 8);
   // keys any query of the tile can see
   const int t_hi = min(q0 + 15, T - 1);
   const int kend = pos0 + t_hi + 1;
@@ -438,51 +632,224 @@ __global__ __launch_bounds__(64 * PF_ATT_WAVES, 2) void pf_attn_kernel(const bf1
   }
 }
 
-// Keys and values of one row's cache slab in the operand layouts of pf_attn_kernel, zero beyond position L; the new
-// positions pos0 .. L - 1 are taken from the projection output, the keys rotated (src/vui/model.py:234-247), and
-// appended to the cache on the way.
+// The same attention for short blocks: keys and values come from the cache rows themselves.  A short block is one tile of
+// queries per head or a few, so each cached value is fetched once or twice and a copy in operand layout costs more than it saves
+// (4.8 us of 37 per layer for that launch alone).  A key fragment is 16 bytes of 16 rows (64 contiguous bytes each); values go through
+// a wave's own 32 x HD share of LDS and come back transposed (ds_read_b64_tr_b16: 16 lanes read 4 rows of 16, lane i
+// receives column i).  Bound by what one compute unit can fetch, so the keys of a (head, tile) are dealt to up to PF_SPLITS
+// workgroups of eight waves, a step of 32 keys per wave as far as that reaches; the last one to arrive merges their parts.
+// Whole pass of 16 positions behind 600 / 2000, us: by a staged copy 777 / 964; here with 8 splits of four waves 644 / 704 (with the
+// cache read ahead, see pf_warm, 635 / 695), of eight waves and 256 keys 678 / 712, one workgroup of sixteen waves 830 / 1043.
+#define PF_SPLITS 8
+template <int HD32> struct PfDirect {
+  static constexpr int HD = 32 * HD32, DT = 2 * HD32, WAVES = 4;
+  static constexpr size_t VB = (size_t)WAVES * 32 * HD * 2, ML = (size_t)WAVES * 16 * 4;  // VB = WAVES * DT * 1024: the waves' parts
+  static constexpr size_t LDS = VB + 2 * ML + 16;
+};
+struct PfDirectArgs {
+  const bf16_t *q, *kc, *vc;
+  bf16_t* att;
+  int T, nq, nkv, gsz, pos0, window;
+  float scale;
+  float *part, *ml;  // (head, tile, split): sums (DT x 64 lanes x 4), {max, sum of weights} x 16
+  uint32_t* count;   // arrivals of a (head, tile): a multiple of the splits before the launch
+};
+typedef short pf_s16x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ uint2 pf_read_tr(const char* lds) {
+  return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) pf_s16x4*)lds));
+}
+template <int HD32>
+__global__ __launch_bounds__(64 * PfDirect<HD32>::WAVES) void pf_direct_attn_kernel(const PfDirectArgs a) {
+  typedef PfDirect<HD32> P;
+  constexpr int HD = P::HD, DT = P::DT, WAVES = P::WAVES;
+  extern __shared__ __align__(16) char lds[];
+  float* s_m = (float*)(lds + P::VB);
+  float* s_l = (float*)(lds + P::VB + P::ML);
+  uint32_t* s_last = (uint32_t*)(lds + P::VB + 2 * P::ML);
+  float* s_acc = (float*)lds;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int l16 = lane & 15, kg = lane >> 4;
+  const int h = blockIdx.x, kvh = h / a.gsz, q0 = blockIdx.y * 16, sp = blockIdx.z, nsp = gridDim.z;
+  const int tq = min(q0 + l16, a.T - 1);
+  const int qlast = a.pos0 + tq, qfirst = a.window > 0 ? max(0, qlast - a.window) : 0;  // visible keys of this lane's query
+  const int t_hi = min(q0 + 15, a.T - 1);
+  const int kend = a.pos0 + t_hi + 1, kbeg = (a.window > 0 ? max(0, a.pos0 + q0 - a.window) : 0) & ~31;
+  const int per = ((kend - kbeg + 31) / 32 + nsp - 1) / nsp * 32, lo = kbeg + sp * per, hi = min(lo + per, kend);
+  uint4 qf[HD32];
+#pragma unroll
+  for (int c = 0; c < HD32; ++c) qf[c] = *reinterpret_cast<const uint4*>(a.q + (size_t)tq * a.nq + h * HD + c * 32 + kg * 8);
+  const bf16_t* kb = a.kc + kvh * HD + kg * 8;
+  const bf16_t* vb = a.vc + kvh * HD;
+  char* own = lds + (size_t)wave * 32 * HD * 2;
+  pf_floatx4 acc[DT];
+#pragma unroll
+  for (int d = 0; d < DT; ++d) acc[d] = pf_floatx4{0.f, 0.f, 0.f, 0.f};
+  float m_run = -INFINITY, l_run = 0.f;
+  for (int k0 = lo + 32 * wave; k0 < hi; k0 += 32 * WAVES) {
+    // a key behind the last visible one reads that one again; its weight is zero
+    uint4 kf[2][HD32], vr[DT];
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int c = 0; c < HD32; ++c) kf[kt][c] = *reinterpret_cast<const uint4*>(kb + (size_t)min(k0 + 16 * kt + l16, kend - 1) * a.nkv + c * 32);
+#pragma unroll
+    for (int i = 0; i < DT; ++i) {  // 32 rows of HD values, in the order of LDS
+      const int e = i * 512 + lane * 8, row = e / HD;
+      vr[i] = *reinterpret_cast<const uint4*>(vb + (size_t)min(k0 + row, kend - 1) * a.nkv + (e - row * HD));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    pf_floatx4 sc[2];
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) {
+      sc[kt] = pf_floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int c = 0; c < HD32; ++c) sc[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf_frag(kf[kt][c]), pf_frag(qf[c]), sc[kt], 0, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < DT; ++i) *reinterpret_cast<uint4*>(own + i * 1024 + lane * 16) = vr[i];
+    float mx = -INFINITY;
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int j = k0 + 16 * kt + 4 * kg + r;
+        sc[kt][r] = (j < qfirst || j > qlast) ? -INFINITY : sc[kt][r] * a.scale;
+        mx = fmaxf(mx, sc[kt][r]);
+      }
+    mx = rows_max(mx);
+    const float m_new = fmaxf(m_run, mx);
+    const float m_use = (m_new == -INFINITY) ? 0.f : m_new;  // nothing visible yet: every weight below is zero
+    const float alpha = expf(m_run - m_use);
+    float pv[8], ps = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) { pv[e] = expf(sc[e >> 2][e & 3] - m_use); ps += pv[e]; }
+    l_run = l_run * alpha + ps;
+    m_run = m_new;
+    uint4 pf;
+    pf.x = f2bf2(pv[0], pv[1]); pf.y = f2bf2(pv[2], pv[3]); pf.z = f2bf2(pv[4], pv[5]); pf.w = f2bf2(pv[6], pv[7]);
+#pragma unroll
+    for (int d = 0; d < DT; ++d)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[d][r] *= alpha;
+    // V^T of dims 16 d + l16: keys 4 kg + r and 16 + 4 kg + r, in the order of the lane's scores
+    const char* vrow = own + (4 * kg + (l16 >> 2)) * (HD * 2) + (l16 & 3) * 8;
+#pragma unroll
+    for (int d = 0; d < DT; ++d) {
+      const uint2 x = pf_read_tr(vrow + d * 32), y = pf_read_tr(vrow + 16 * HD * 2 + d * 32);
+      acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf_frag(make_uint4(x.x, x.y, y.x, y.y)), pf_frag(pf), acc[d], 0, 0, 0);
+    }
+  }
+  l_run = rows_sum(l_run);
+  if (kg == 0) { s_m[wave * 16 + l16] = m_run; s_l[wave * 16 + l16] = l_run; }
+  __syncthreads();  // the shares of the values become the waves' parts
+#pragma unroll
+  for (int d = 0; d < DT; ++d) *reinterpret_cast<pf_floatx4*>(&s_acc[((wave * DT + d) * 64 + lane) * 4]) = acc[d];
+  __syncthreads();
+  // blocks d = wave, wave + WAVES, ...: dims 16 d + 4 kg + r of query l16
+  constexpr int ND = (DT + WAVES - 1) / WAVES;
+  float M = -INFINITY, den = 0.f, o[ND][4] = {};
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) M = fmaxf(M, s_m[w * 16 + l16]);
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) {
+    const float m = s_m[w * 16 + l16], f = (m == -INFINITY) ? 0.f : expf(m - M);
+    den = fmaf(f, s_l[w * 16 + l16], den);
+#pragma unroll
+    for (int i = 0; i < ND; ++i) {
+      const pf_floatx4 x = *reinterpret_cast<const pf_floatx4*>(&s_acc[((w * DT + min(wave + i * WAVES, DT - 1)) * 64 + lane) * 4]);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[i][r] = fmaf(f, x[r], o[i][r]);
+    }
+  }
+  if (nsp > 1) {
+    const size_t set = (size_t)h * gridDim.y + blockIdx.y;
+    float* part = a.part + set * nsp * (DT * 256);
+    float* ml = a.ml + set * nsp * 32;
+#pragma unroll
+    for (int i = 0; i < ND; ++i) {
+      const int d = wave + i * WAVES;
+      if (d < DT) {
+        float* mine = part + ((size_t)(sp * DT + d) * 64 + lane) * 4;
+        st_dev(mine, o[i][0], o[i][1]);
+        st_dev(mine + 2, o[i][2], o[i][3]);
+      }
+    }
+    if (tid < 16) st_dev(ml + sp * 32 + tid * 2, M, den);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (tid == 0)
+      *s_last = (__hip_atomic_fetch_add(a.count + set, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1) % nsp == 0;
+    __syncthreads();
+    if (!*s_last) return;
+    uint64_t xm[PF_SPLITS], xo[ND][PF_SPLITS][2];
+#pragma unroll
+    for (int s = 0; s < PF_SPLITS; ++s) {  // a split that is not there reads the last one again and weighs nothing
+      const int t = min(s, nsp - 1);
+      xm[s] = ld_dev(ml + t * 32 + l16 * 2);
+#pragma unroll
+      for (int i = 0; i < ND; ++i) {
+        const float* x = part + ((size_t)(t * DT + min(wave + i * WAVES, DT - 1)) * 64 + lane) * 4;
+        xo[i][s][0] = ld_dev(x); xo[i][s][1] = ld_dev(x + 2);
+      }
+    }
+    M = -INFINITY;
+#pragma unroll
+    for (int s = 0; s < PF_SPLITS; ++s) M = fmaxf(M, lo_f(xm[s]));
+    den = 0.f;
+#pragma unroll
+    for (int i = 0; i < ND; ++i) o[i][0] = o[i][1] = o[i][2] = o[i][3] = 0.f;
+#pragma unroll
+    for (int s = 0; s < PF_SPLITS; ++s) {
+      const float m = lo_f(xm[s]), f = (s >= nsp || m == -INFINITY) ? 0.f : expf(m - M);
+      den = fmaf(f, hi_f(xm[s]), den);
+#pragma unroll
+      for (int i = 0; i < ND; ++i) {
+        o[i][0] = fmaf(f, lo_f(xo[i][s][0]), o[i][0]); o[i][1] = fmaf(f, hi_f(xo[i][s][0]), o[i][1]);
+        o[i][2] = fmaf(f, lo_f(xo[i][s][1]), o[i][2]); o[i][3] = fmaf(f, hi_f(xo[i][s][1]), o[i][3]);
+      }
+    }
+  }
+  const int t = q0 + l16;
+  const float inv = 1.0f / den;
+#pragma unroll
+  for (int i = 0; i < ND; ++i) {
+    const int d = wave + i * WAVES;
+    if (d < DT && t < a.T)
+      *reinterpret_cast<uint2*>(a.att + pf_toff(t, h * HD + 16 * d + 4 * kg, a.nq)) =
+          make_uint2(f2bf2(o[i][0] * inv, o[i][1] * inv), f2bf2(o[i][2] * inv, o[i][3] * inv));
+  }
+}
+template <int HD32> static int pf_direct_attn(const PfDirectArgs& a, int H, hipStream_t st) {
+  constexpr size_t lds = PfDirect<HD32>::LDS;
+  const int L = a.pos0 + a.T, keys = a.window > 0 && a.window + 48 < L ? a.window + 48 : L, n = (keys + 127) / 128;
+  HIP_TRY(hipFuncSetAttribute((const void*)pf_direct_attn_kernel<HD32>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  hipLaunchKernelGGL(pf_direct_attn_kernel<HD32>, dim3(H, (a.T + 15) / 16, n > PF_SPLITS ? PF_SPLITS : n), dim3(64 * PfDirect<HD32>::WAVES), lds, st, a);
+  return VUI_OK;
+}
+
+// The cached keys and values before position L of one slot in the operand layouts of pf_attn_kernel (in a pass that starts an empty
+// slot the QKV product's epilogue writes them).
 // Keys of KV head g: blocks of 16 keys x 32 dims, block ((g * Lpad / 16 + j / 16) * hd / 32 + dim / 32) of 512
 // elements, lane (j % 16) + 16 * ((dim % 32) / 8) holds its 8 dims at 8 * lane.  Values, transposed: blocks of 16
 // dims x 32 keys, block ((g * hd / 16 + dim / 16) * Lpad / 32 + j / 32), lane (dim % 16) + 16 * ((j % 16) / 4)
 // holds keys j % 4 of both halves (j % 32) / 16 of the step at 8 * lane + 4 * half + j % 4 - the order in which a
 // lane of the attention kernel holds the scores of a step.  One workgroup: 32 keys x 32 features.
-__global__ __launch_bounds__(256) void pf_stage_kv_kernel(bf16_t* __restrict__ qkv, bf16_t* __restrict__ kc, bf16_t* __restrict__ vc,
-                                                          bf16_t* __restrict__ kt, bf16_t* __restrict__ vt, const float* __restrict__ rope,
-                                                          int L, int Lpad, int nq, int nkv, int hd, int rope_dim, int pos0) {
+__global__ __launch_bounds__(256) void pf_stage_kv_kernel(const bf16_t* __restrict__ kc, const bf16_t* __restrict__ vc,
+                                                          bf16_t* __restrict__ kt, bf16_t* __restrict__ vt, int L, int Lpad, int nkv, int hd) {
   __shared__ bf16_t tile[32][34];
   const int tid = threadIdx.x;
-  const int ldq = nq + 2 * nkv;
-  if ((int)blockIdx.y >= nkv / 32) {
-    // the other workgroups rotate the queries in place: 32 rows x 32 dims each
-    const int t = blockIdx.x * 32 + (tid >> 2), f = ((int)blockIdx.y - nkv / 32) * 32 + (tid & 3) * 8;
-    if (tid < 128 && t < L - pos0) {
-      uint4* q = reinterpret_cast<uint4*>(qkv + (size_t)t * ldq + f);
-      *q = pf_rope8(*q, rope, pos0 + t, rope_dim, f % hd);
-    }
-    return;
-  }
   const int j0 = blockIdx.x * 32, f0 = blockIdx.y * 32;  // f over nkv (= KV * hd); hd is a multiple of 32
   const int g = f0 / hd, dim0 = f0 % hd;
   if (tid < 128) {  // keys: 32 keys x four 8-dim pieces
     const int key = tid >> 2, pc = tid & 3, j = j0 + key;
-    uint4 v = make_uint4(0, 0, 0, 0);
-    if (j < pos0) v = *reinterpret_cast<const uint4*>(kc + (size_t)j * nkv + f0 + pc * 8);
-    else if (j < L) {
-      v = pf_rope8(*reinterpret_cast<const uint4*>(qkv + (size_t)(j - pos0) * ldq + nq + f0 + pc * 8), rope, j, rope_dim, dim0 + pc * 8);
-      *reinterpret_cast<uint4*>(kc + (size_t)j * nkv + f0 + pc * 8) = v;
+    if (j < L) {
+      const size_t blk = ((size_t)g * (Lpad >> 4) + (j >> 4)) * (hd >> 5) + (dim0 >> 5);
+      *reinterpret_cast<uint4*>(kt + blk * 512 + ((j & 15) + 16 * pc) * 8) = *reinterpret_cast<const uint4*>(kc + (size_t)j * nkv + f0 + pc * 8);
     }
-    const size_t blk = ((size_t)g * (Lpad >> 4) + (j >> 4)) * (hd >> 5) + (dim0 >> 5);
-    *reinterpret_cast<uint4*>(kt + blk * 512 + ((j & 15) + 16 * pc) * 8) = v;
   }
   {
     const int tx = tid & 31, ty = tid >> 5;  // 32 x 8
-    for (int r = ty; r < 32; r += 8) {
-      const int j = j0 + r;
-      bf16_t v = (bf16_t)0;
-      if (j < pos0) v = vc[(size_t)j * nkv + f0 + tx];
-      else if (j < L) { v = qkv[(size_t)(j - pos0) * ldq + nq + nkv + f0 + tx]; vc[(size_t)j * nkv + f0 + tx] = v; }
-      tile[r][tx] = v;
-    }
+    for (int r = ty; r < 32; r += 8) tile[r][tx] = vc[(size_t)min(j0 + r, L - 1) * nkv + f0 + tx];
   }
   __syncthreads();
   {
@@ -490,14 +857,17 @@ __global__ __launch_bounds__(256) void pf_stage_kv_kernel(bf16_t* __restrict__ q
     const int dl = tid >> 3, q = tid & 7, half = q >> 2, kgk = q & 3;
     const int dim = dim0 + dl;
     const int jj = half * 16 + kgk * 4;
-    const uint32_t lo = (uint32_t)tile[jj][dl] | ((uint32_t)tile[jj + 1][dl] << 16);
-    const uint32_t hi = (uint32_t)tile[jj + 2][dl] | ((uint32_t)tile[jj + 3][dl] << 16);
     const size_t blk = ((size_t)g * (hd >> 4) + (dim >> 4)) * (Lpad >> 5) + (j0 >> 5);
-    *reinterpret_cast<uint2*>(vt + blk * 512 + ((dim & 15) + 16 * kgk) * 8 + 4 * half) = make_uint2(lo, hi);
+    bf16_t* dst = vt + blk * 512 + ((dim & 15) + 16 * kgk) * 8 + 4 * half;
+    if (j0 + jj + 3 < L) {
+      const uint32_t lo = (uint32_t)tile[jj][dl] | ((uint32_t)tile[jj + 1][dl] << 16);
+      const uint32_t hi = (uint32_t)tile[jj + 2][dl] | ((uint32_t)tile[jj + 3][dl] << 16);
+      *reinterpret_cast<uint2*>(dst) = make_uint2(lo, hi);
+    } else {
+      for (int r = 0; r < 4; ++r) if (j0 + jj + r < L) dst[r] = tile[jj + r][dl];
+    }
   }
 }
-
-__global__ void pf_set_len_kernel(int32_t* seq_lens, int slot, int v) { seq_lens[slot] = v; }
 
 // The form of a product of M rows (pair: two matrices of N features): estimated microseconds of the large tiles - a launch,
 // and per step of 32 columns `wait` or `work` for each round of 256 tiles - and of the K-splitting form, whose time follows its
@@ -528,55 +898,67 @@ static int pf_pick(int M, int N, int K, bool pair, bool i8) {
   return best;
 }
 
-// bf16 out, K split over the waves of a workgroup; W2 != nullptr: the SwiGLU pair; i8: int8 matrices with g.sc / g.sc2
-static int pf_gemm4(int epi, const PfGemm& g, const void* W2, int c_tiled, bool i8, hipStream_t st) {
-  if (g.K % 64 || g.N % 16 || g.M < 1 || g.N < 1 || (c_tiled && g.N % 64)) { vui_set_error("prefill GEMM: bad shape N=%d K=%d", g.N, g.K); return VUI_EINVAL; }
-  const int tile = pf_pick(g.M, g.N, g.K, W2 != nullptr, i8);
-  if (tile != WIDE_NONE) {
-    if (W2) return i8 ? pf_wide<PF_BF16, true, true>(tile, g, W2, c_tiled, st) : pf_wide<PF_BF16, true, false>(tile, g, W2, c_tiled, st);
-    if (epi == PF_RESID) return i8 ? pf_wide<PF_RESID, false, true>(tile, g, W2, c_tiled, st) : pf_wide<PF_RESID, false, false>(tile, g, W2, c_tiled, st);
-    return i8 ? pf_wide<PF_BF16, false, true>(tile, g, W2, c_tiled, st) : pf_wide<PF_BF16, false, false>(tile, g, W2, c_tiled, st);
-  }
+// bf16 out, K split over the waves of a workgroup; W2 != nullptr: the SwiGLU pair; i8: int8 matrices with g.sc / g.sc2;
+// g.ssq != nullptr: rows are normed on their way (short blocks)
+template <int EPI, bool DUAL, bool I8>
+static int pf_go(PfGemm& g, const void* W2, int c_tiled, hipStream_t st) {
   // Few tiles (short blocks): more waves, so that a wave's chain of dependent trips is one to three steps long, and 16
   // features per workgroup, so that more of the chip pulls weights.  us per launch, 32 x 32 and 4 waves / as chosen here:
   // 16 positions out_proj and W2 8.0 / 4.4, QKV 5.6 / 3.8, W1 and W3 5.9 / 5.0; whole pass of 16 positions 883 / 776
   // (int8 902 / 745), of 230 positions 1069 / 1060 (1013 / 931).
   const long t32 = (long)((g.M + 31) / 32) * ((g.N + 31) / 32);
-  const bool some = t32 <= 256 && g.K >= 512, few = some && t32 <= 128;
+  const bool norm = g.ssq != nullptr, some = t32 <= 256 && g.K >= 512, few = norm || (some && t32 <= 128);
   const int mb = few && g.M <= 16 ? 1 : 2, nb = few ? 1 : 2;
-  const unsigned tiles = (unsigned)(((g.M + 16 * mb - 1) / (16 * mb)) * ((g.N + 16 * nb - 1) / (16 * nb)));
-#define PF_GO(E, D, Q, W, MB, NB) hipLaunchKernelGGL((pf_gemm_kernel<E, D, Q, W, MB, NB>), dim3(tiles), dim3(64 * (W)), 0, st, g, W2, c_tiled)
-#define PF_SIZE(E, D, Q, W) \
-  do { \
-    if (!some) PF_GO(E, D, Q, 4, 2, 2); \
-    else if (!few) PF_GO(E, D, Q, (D ? 8 : 12), 2, 2); \
-    else if (mb == 1) PF_GO(E, D, Q, W, 1, 1); \
-    else PF_GO(E, D, Q, W, 2, 1); \
-  } while (0)
-#define PF_PICK(E, D, W) do { if (i8) PF_SIZE(E, D, true, W); else PF_SIZE(E, D, false, W); } while (0)
-  if (W2) PF_PICK(PF_BF16, true, 12);
-  else if (epi == PF_RESID) PF_PICK(PF_RESID, false, 16);
-  else PF_PICK(PF_BF16, false, 12);
-#undef PF_PICK
-#undef PF_SIZE
+  const unsigned tiles = pf_set_order(g, 16 * mb, 16 * nb, (size_t)g.N * g.K * ((DUAL ? 2 : 1) * (I8 ? 1 : 2))) + g.warm;
+  constexpr int W = EPI == PF_RESID ? 16 : 12;
+#define PF_GO(WV, MB, NB, NORM) hipLaunchKernelGGL((pf_gemm_kernel<EPI, DUAL, I8, WV, MB, NB, NORM>), dim3(tiles), dim3(64 * (WV)), 0, st, g, W2, c_tiled)
+  if constexpr (EPI != PF_RESID) {
+    if (norm) {
+      if (mb == 1) PF_GO(W, 1, 1, true);
+      else PF_GO(W, 2, 1, true);
+      HIP_TRY(hipGetLastError());
+      return VUI_OK;
+    }
+  }
+  if (few && mb == 1) PF_GO(W, 1, 1, false);
+  else if (few) PF_GO(W, 2, 1, false);
+  else if (some) PF_GO((DUAL ? 8 : 12), 2, 2, false);
+  else PF_GO(4, 2, 2, false);
 #undef PF_GO
   HIP_TRY(hipGetLastError());
   return VUI_OK;
 }
+template <int EPI, bool DUAL>
+static int pf_gemm4(PfGemm& g, const void* W2, int c_tiled, bool i8, hipStream_t st) {
+  if (g.K % 64 || g.N % 16 || g.M < 1 || g.N < 1 || (c_tiled && g.N % 64)) { vui_set_error("prefill GEMM: bad shape N=%d K=%d", g.N, g.K); return VUI_EINVAL; }
+  const int tile = g.ssq ? WIDE_NONE : pf_pick(g.M, g.N, g.K, DUAL, i8);
+  if (tile != WIDE_NONE) return i8 ? pf_wide<EPI, DUAL, true>(tile, g, W2, c_tiled, st) : pf_wide<EPI, DUAL, false>(tile, g, W2, c_tiled, st);
+  return i8 ? pf_go<EPI, DUAL, true>(g, W2, c_tiled, st) : pf_go<EPI, DUAL, false>(g, W2, c_tiled, st);
+}
+
+// Blocks of up to this many positions take the five-launch form.
+// Whole pass, us, 65 positions in the long form / in this: bf16 738 / 800, behind 600 912 / 907, behind 2000 1063 / 1071; 100 positions
+// 752 / 905; 64 positions in this form 724, 835, 899 (all by eight launches with a staged copy: 796, 882, 1034).
+#define PF_SHORT 64
+#define PF_WARM 64
 
 static size_t pf_align(size_t b) { return (b + 255) & ~(size_t)255; }
 
-// scratch: residual x, normed xn, qkv, attention output, FFN buffer, staged keys and values
+// (head, tile of queries) pairs of a short block
+static size_t pf_sets(const vui_config& c, int T) { return T <= PF_SHORT ? (size_t)c.n_heads * ((T + 15) / 16) : 0; }
+// scratch: residual x, its sums of squares, normed xn, queries, attention output, FFN buffer, staged keys and values
 size_t prefill_scratch_bytes(const vui_config& c, int T, int L) {
   const size_t d = c.d_model, nq = (size_t)c.n_heads * c.head_dim, nkv = (size_t)c.n_kv_heads * c.head_dim;
   const size_t Lpad = ((size_t)L + 63) & ~(size_t)63;
   const size_t T16 = ((size_t)T + 15) & ~(size_t)15;  // tiled operands come in blocks of 16 rows
   size_t b = 0;
-  b += pf_align((size_t)T * d * 2) + pf_align(T16 * d * 2);
-  b += pf_align((size_t)T * (nq + 2 * nkv) * 2);
+  b += pf_align(T16 * d * 2) * 2 + pf_align(T16 * (d / 16) * 4);
+  b += pf_align((size_t)T * nq * 2);
   b += pf_align(T16 * nq * 2);
   b += pf_align(T16 * c.ffn * 2);
   b += pf_align(nkv * Lpad * 2) * 2;
+  const size_t sets = pf_sets(c, T);
+  b += pf_align(sets * PF_SPLITS * 16 * c.head_dim * 4) + pf_align(sets * PF_SPLITS * 32 * 4) + pf_align(sets * 4);
   return b;
 }
 
@@ -637,62 +1019,91 @@ int launch_prefill(const vui_config& c, const vui_weights& w, const void* tiled_
   const size_t T16 = ((size_t)T + 15) & ~(size_t)15;
   char* sp = (char*)scratch;
   auto take = [&](size_t bytes) { char* r = sp; sp += pf_align(bytes); return r; };
-  bf16_t* x = (bf16_t*)take((size_t)T * d * 2);                 // residual stream, row-major
+  bf16_t* x = (bf16_t*)take(T16 * d * 2);                       // residual stream: row-major, of a short block tiled
+  float* ssq = (float*)take(T16 * (d / 16) * 4);
   bf16_t* xn = (bf16_t*)take(T16 * d * 2);                      // normed rows, tiled (rows past T are never written:
-  bf16_t* qkv = (bf16_t*)take((size_t)T * (nq + 2 * nkv) * 2);  //  what a GEMM reads there only reaches output rows it drops)
+  bf16_t* q = (bf16_t*)take((size_t)T * nq * 2);                //  what a GEMM reads there only reaches output rows it drops)
   bf16_t* att = (bf16_t*)take(T16 * nq * 2);                    // attention output, tiled
   bf16_t* fa = (bf16_t*)take(T16 * F * 2);                      // SwiGLU product, tiled
-  bf16_t* kt = (bf16_t*)take((size_t)nkv * Lpad * 2);                // staged keys and values of the slot
+  bf16_t* kt = (bf16_t*)take((size_t)nkv * Lpad * 2);           // keys and values of the slot in the attention's layout
   bf16_t* vt = (bf16_t*)take((size_t)nkv * Lpad * 2);
-  HIP_TRY(hipMemcpyAsync(x, emb, (size_t)T * d * 2, hipMemcpyDeviceToDevice, st));
-  const size_t slab = (size_t)c.n_slots * S * nkv;
+  const bool tiny = T <= PF_SHORT;
+  const size_t sets = pf_sets(c, T);
+  float* part = (float*)take(sets * PF_SPLITS * 16 * hd * 4);   // parts of a short block's attention
+  float* ml = (float*)take(sets * PF_SPLITS * 32 * 4);
+  uint32_t* count = (uint32_t*)take(sets * 4);
+  const bool i8 = c.int8_backbone != 0;
+  const size_t slab = (size_t)c.n_slots * S * nkv, wsz = i8 ? 1 : 2;
   const float scale = 1.0f / sqrtf((float)hd);
+  if ((uintptr_t)emb & 15) {  // a caller's view may start anywhere
+    HIP_TRY(hipMemcpyAsync(xn, emb, (size_t)T * d * 2, hipMemcpyDeviceToDevice, st));
+    emb = xn;
+  }
+  {
+    size_t n = (size_t)T * (d / 8);
+    const size_t more = tiny ? sets : (size_t)(Lpad - L) * nkv;
+    if (more > n) n = more;
+    hipLaunchKernelGGL(pf_begin_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, (const bf16_t*)emb, x,
+                       tiny ? ssq : nullptr, tiny ? nullptr : vt, count, (int)sets, T, d, nkv, L, Lpad);
+  }
+  auto norm = [&](const void* w, bf16_t* y, int y_tiled, int32_t* len) {
+    hipLaunchKernelGGL(pf_rownorm_kernel, dim3((T + 3) / 4), dim3(256), 0, st, x, (const bf16_t*)w, y, T, d, c.norm_eps, tiny ? 1 : 0, y_tiled, len, L);
+  };
   int rc;
   for (int l = 0; l < c.n_layers; ++l) {
     const vui_layer_weights& lw = w.layers[l];
-    const bool i8 = c.int8_backbone != 0;
-    const size_t wsz = i8 ? 1 : 2;
     const char* t_qkv = (const char*)tiled_w + pf_layer_elems(c) * wsz * l;
     const char* t_o = t_qkv + (size_t)(nq + 2 * nkv) * d * wsz;
     const char* t_1 = t_o + (size_t)d * nq * wsz;
     const char* t_3 = t_1 + (size_t)F * d * wsz;
     const char* t_2 = t_3 + (size_t)F * d * wsz;
-    bf16_t* kc = (bf16_t*)k_cache + slab * l;
-    bf16_t* vc = (bf16_t*)v_cache + slab * l;
-    hipLaunchKernelGGL(pf_rownorm_kernel, dim3((T + 3) / 4), dim3(256), 0, st, x, (const bf16_t*)lw.attn_norm, xn, T, d, c.norm_eps, 1);
     PfGemm g{};
-    g.X = xn; g.W = t_qkv; g.C = qkv; g.M = T; g.N = nq + 2 * nkv; g.K = d; g.ldc = nq + 2 * nkv; g.sc = (const bf16_t*)lw.s_qkv;
-    if ((rc = pf_gemm4(PF_BF16, g, nullptr, 0, i8, st))) return rc;
-    // attention over the L cached positions of this slot
-    bf16_t* krow = kc + (size_t)slot * S * nkv;
-    bf16_t* vrow = vc + (size_t)slot * S * nkv;
-    int rope_dim_l;
-    const float* rope_l = layer_rope(c, w, l, &rope_dim_l);
-    const int window_l = layer_window(c, l);
-    hipLaunchKernelGGL(pf_stage_kv_kernel, dim3(Lpad / 32, (nkv + nq) / 32), dim3(256), 0, st, qkv, krow, vrow, kt, vt, rope_l, L, Lpad, nq, nkv,
-                       hd, rope_dim_l, pos0);
-    {
+    g.X = tiny ? x : xn; g.W = t_qkv; g.C = q; g.M = T; g.N = nq + 2 * nkv; g.K = d; g.ldc = nq; g.sc = (const bf16_t*)lw.s_qkv;
+    if (tiny) { g.ssq = ssq; g.nw = (const bf16_t*)lw.attn_norm; g.eps = c.norm_eps; }
+    else norm(lw.attn_norm, xn, 1, nullptr);
+    g.kc = (bf16_t*)k_cache + slab * l + (size_t)slot * S * nkv;
+    g.vc = (bf16_t*)v_cache + slab * l + (size_t)slot * S * nkv;
+    const int win = layer_window(c, l);
+    if (!tiny && pos0 == 0) { g.kt = kt; g.vt = vt; }
+    if (tiny && pos0 > 0) { g.warm_from = win > 0 && pos0 > win ? pos0 - win : 0; g.warm = PF_WARM; }
+    g.rope = layer_rope(c, w, l, &g.rope_dim);
+    g.nq = nq; g.nkv = nkv; g.hd = hd; g.inv_hd = pf_inv(hd); g.pos0 = pos0; g.Lpad = Lpad;
+    if ((rc = pf_gemm4<PF_QKV, false>(g, nullptr, 0, i8, st))) return rc;
+    if (tiny) {
+      const PfDirectArgs da = {q, g.kc, g.vc, att, T, nq, nkv, H / KV, pos0, win, scale, part, ml, count};
+      switch (hd / 32) {
+        case 1: rc = pf_direct_attn<1>(da, H, st); break;
+        case 2: rc = pf_direct_attn<2>(da, H, st); break;
+        case 3: rc = pf_direct_attn<3>(da, H, st); break;
+        default: rc = pf_direct_attn<4>(da, H, st); break;
+      }
+      if (rc) return rc;
+    } else {
+      if (pos0 > 0)
+        hipLaunchKernelGGL(pf_stage_kv_kernel, dim3((L + 31) / 32, nkv / 32), dim3(256), 0, st, g.kc, g.vc, kt, vt, L, Lpad, nkv, hd);
       const dim3 grid(H, (T + 15) / 16);
       switch (hd / 32) {
-        case 1: hipLaunchKernelGGL(pf_attn_kernel<1>, grid, dim3(512), 0, st, qkv, kt, vt, att, T, L, Lpad, nq, nkv, H / KV, pos0, window_l, scale); break;
-        case 2: hipLaunchKernelGGL(pf_attn_kernel<2>, grid, dim3(512), 0, st, qkv, kt, vt, att, T, L, Lpad, nq, nkv, H / KV, pos0, window_l, scale); break;
-        case 3: hipLaunchKernelGGL(pf_attn_kernel<3>, grid, dim3(512), 0, st, qkv, kt, vt, att, T, L, Lpad, nq, nkv, H / KV, pos0, window_l, scale); break;
-        default: hipLaunchKernelGGL(pf_attn_kernel<4>, grid, dim3(256), 0, st, qkv, kt, vt, att, T, L, Lpad, nq, nkv, H / KV, pos0, window_l, scale); break;
+        case 1: hipLaunchKernelGGL(pf_attn_kernel<1>, grid, dim3(512), 0, st, q, kt, vt, att, T, nq, Lpad, nq, H / KV, pos0, win, scale); break;
+        case 2: hipLaunchKernelGGL(pf_attn_kernel<2>, grid, dim3(512), 0, st, q, kt, vt, att, T, nq, Lpad, nq, H / KV, pos0, win, scale); break;
+        case 3: hipLaunchKernelGGL(pf_attn_kernel<3>, grid, dim3(512), 0, st, q, kt, vt, att, T, nq, Lpad, nq, H / KV, pos0, win, scale); break;
+        default: hipLaunchKernelGGL(pf_attn_kernel<4>, grid, dim3(256), 0, st, q, kt, vt, att, T, nq, Lpad, nq, H / KV, pos0, win, scale); break;
       }
     }
     PfGemm wo{};
     wo.X = att; wo.W = t_o; wo.C = x; wo.ldc = d; wo.M = T; wo.N = d; wo.K = nq; wo.sc = (const bf16_t*)lw.s_o;
-    if ((rc = pf_gemm4(PF_RESID, wo, nullptr, 0, i8, st))) return rc;
-    hipLaunchKernelGGL(pf_rownorm_kernel, dim3((T + 3) / 4), dim3(256), 0, st, x, (const bf16_t*)lw.mlp_norm, xn, T, d, c.norm_eps, 1);
+    if (tiny) wo.ssq_out = ssq;
+    if ((rc = pf_gemm4<PF_RESID, false>(wo, nullptr, tiny ? 1 : 0, i8, st))) return rc;
     PfGemm f1{};
-    f1.X = xn; f1.W = t_1; f1.C = fa; f1.ldc = F; f1.M = T; f1.N = F; f1.K = d; f1.sc = (const bf16_t*)lw.s_1; f1.sc2 = (const bf16_t*)lw.s_3;
-    if ((rc = pf_gemm4(PF_BF16, f1, t_3, 1, i8, st))) return rc;  // written tiled: operand of W2
+    f1.X = tiny ? x : xn; f1.W = t_1; f1.C = fa; f1.ldc = F; f1.M = T; f1.N = F; f1.K = d; f1.sc = (const bf16_t*)lw.s_1; f1.sc2 = (const bf16_t*)lw.s_3;
+    if (tiny) { f1.ssq = ssq; f1.nw = (const bf16_t*)lw.mlp_norm; f1.eps = c.norm_eps; }
+    else norm(lw.mlp_norm, xn, 1, nullptr);
+    if ((rc = pf_gemm4<PF_BF16, true>(f1, t_3, 1, i8, st))) return rc;  // written tiled: operand of W2
     PfGemm f2{};
     f2.X = fa; f2.W = t_2; f2.C = x; f2.ldc = d; f2.M = T; f2.N = d; f2.K = F; f2.sc = (const bf16_t*)lw.s_2;
-    if ((rc = pf_gemm4(PF_RESID, f2, nullptr, 0, i8, st))) return rc;
+    if (tiny) f2.ssq_out = ssq;
+    if ((rc = pf_gemm4<PF_RESID, false>(f2, nullptr, tiny ? 1 : 0, i8, st))) return rc;
   }
-  hipLaunchKernelGGL(pf_rownorm_kernel, dim3((T + 3) / 4), dim3(256), 0, st, x, (const bf16_t*)w.final_norm, (bf16_t*)out, T, d, c.norm_eps, 0);
-  hipLaunchKernelGGL(pf_set_len_kernel, dim3(1), dim3(1), 0, st, seq_lens, slot, L);
+  norm(w.final_norm, (bf16_t*)out, 0, seq_lens + slot);
   HIP_TRY(hipGetLastError());
   return VUI_OK;
 }
