@@ -440,15 +440,14 @@ class Engine(SlotEngine):
         return offset
 
     def _prefill_emb(self, row: Row, emb: Tensor, offset: int | None = None, lane: int = 0) -> Tensor:
-        """offset: the row's current length when the caller keeps count of it (saves reading it back from
-        the device, a synchronisation).  lane: see Decoder._prefill."""
+        """offset: the row's current length when the caller keeps count of it; otherwise it is read back from the device, a
+        synchronisation (the only one: the pass is told the slot and the length, 20-30 us each if it read them again).
+        lane: see Decoder._prefill."""
         T = emb.shape[1]
         off = row.offset if offset is None else offset
         if off + T > self.max_seq:
             raise ValueError(f"prefill of {T} positions at offset {off} exceeds max_seq={self.max_seq}")
-        pos = torch.arange(off, off + T, device=self.device)
-        return self.model.decoder.forward_flash(emb.to(self.dtype), pos, slot_idx=row._slot,
-                                                known=(row.idx, off) if offset is not None else None, lane=lane)
+        return self.model.decoder.forward_flash(emb.to(self.dtype), None, slot_idx=row._slot, known=(row.idx, off), lane=lane)
 
     max_frame_graphs = 32  # captured frame graphs kept (oldest dropped first)
     prefill_lanes = 4  # streams that ingest the blocks of different rows at once (1: one after the other)
