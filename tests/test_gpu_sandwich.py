@@ -429,6 +429,36 @@ def test_all_tokens_to_few_experts(dt):
 
 
 @BOTH
+@pytest.mark.parametrize("experts,top,rows", [(64, 4, 16), (65, 4, 16), (64, 5, 13), (33, 16, 4), (6, 6, 10), (12, 1, 2), (40, 7, 1)])
+def test_routing_of_decode_rows(experts, top, rows, dt):
+    """Rows whose choices their own launch sorts (up to 64 of them) and the next more, both forms of choosing (up to 64 experts, and
+    more), all experts at once, with attention of one piece and of several per row: every row against itself alone, through the
+    prompt pass of its whole sequence where routing takes launches of its own.  Replayed, other rows' steps in between."""
+    cfg = U.sandwich([(U.sig(), U.moe(experts=experts, top=top)), (U.sig(heads=20, kv_heads=1, dim=8, vdim=12), U.dense(40))])
+    sd = U.sandwich_weights(cfg, 51)
+    sd["l0.mlp.router"] = sd["l0.mlp.router"] * 8
+    eng = U.engine(cfg, sd, dt, max_rows=rows, max_seq=500)
+    starts, n = [5 + (k * 137) % 460 for k in range(rows)], 4
+    seqs = [U.tokens(s + n, cfg["vocab"], s) for s in starts]
+    want = []
+    for s, toks in zip(starts, seqs):
+        with eng.new_row() as row:
+            want.append(row.extend(toks, range(s, s + n)).clone())
+    held = [eng.new_row() for _ in seqs]
+    for row, s, toks in zip(held, starts, seqs):
+        row.extend(toks[:s])
+    tol = 2 * TOL[dt]  # two evaluations, each that close to the oracle
+    far = 0
+    for t in range(n):
+        got = eng.decode_step(held, torch.tensor([toks[s + t] for s, toks in zip(starts, seqs)], device="cuda")).clone()
+        for k in range(rows):
+            e = U.err(got[k:k + 1], want[k][t:t + 1])
+            far += not e < tol
+    # in bf16 a close call between two experts may fall either way
+    assert far <= (0 if dt == F32 else 0.1 * n * rows), far
+
+
+@BOTH
 def test_captured_step_replayed(dt):
     """The bucketed graph against the oracle, several replays with other work of the engine in between."""
     cfg = U.sandwich_mixed()

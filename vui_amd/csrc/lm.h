@@ -185,10 +185,15 @@ struct RowArgs {
   const float* router_bias;
   int experts16;
   float* rlog;             // (M, experts16)
-  RouteArgs route;         // of a single row: routed as well
+  RouteArgs route;         // rows are routed as well
+  uint32_t* arrived;       // rows that have made their choices, zero between launches
+  // the first launch of a pass clears the arrival counters (a workspace comes as it is)
+  uint32_t* clear;
+  int n_clear;
 };
 int launch_lm_rows(const RowArgs& a, hipStream_t st);
 bool lm_rows_routes(int M, int experts16);  // it takes the router's product too
+bool lm_rows_sorts(int M, int top);         // ... and the routing
 
 // ---- attention with sigmoid weights (sigattn.hip) ----
 struct SigAttnArgs {
@@ -207,6 +212,7 @@ struct SigAttnArgs {
   void* q;                 // (heads, rows, dim64) tiled
   size_t q_z;
   float* part;             // (rows, heads, n_splits, vdim16)
+  uint32_t* arrived;       // per row and block of heads: pieces that are there, zero between launches
   int n_splits;
   void* act;               // (rows, out_k) tiled
 };
@@ -268,6 +274,8 @@ struct vui_lm_ctx {
   void *xcat, *raw, *ffa, *xg;
   float *y, *bsum, *gupd, *gdec, *rlog, *share;
   int32_t *choice, *ent, *tile_e, *n_tiles;
+  uint32_t* arrived;  // attention pieces of each row's blocks of heads, then rows routed
+  int n_arrived;
   int attn_from, gla_from;
 };
 static inline int lm_pad(int v, int a) { return (v + a - 1) / a * a; }

@@ -7,7 +7,7 @@
 
 __global__ __launch_bounds__(256) void moe_top_kernel(const RouteArgs p) {
   const int m = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (m < p.M) route_row(p, m);
+  if (m < p.M) route_row(p, m, p.logits + (size_t)m * p.ldl);
 }
 
 // One workgroup sorts all entries.  Where an entry lands inside its expert's run has no effect on its numbers.
@@ -17,7 +17,7 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(const RouteArgs p) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = p.M * p.top;
   cnt[tid] = 0;
   if (TOP) {
-    for (int m = wave; m < p.M; m += 16) route_row(p, m);
+    for (int m = wave; m < p.M; m += 16) route_row(p, m, p.logits + (size_t)m * p.ldl);
     __threadfence_block();
   }
   __syncthreads();

@@ -1,9 +1,9 @@
 // Sandwich layers of the token language models: x <- x + norm(mixer(norm(x))), then x <- x + norm(ff(norm(x))).  See
 // include/vui_lm.h and lm.hip, which holds the context and the C ABI.
 //
-// Launches: input projection, mixer (sigmoid attention 2, portions of a prompt 3, blocks of one 2; gated linear
-// attention 1, by chunks 3), output projection, rows, up, down, rows; an expert layer adds 1 for routing (none for one row), with more
-// rows than 16 the router's product, 2 for routing and 1 that puts the rows in order.
+// Launches: input projection, mixer (sigmoid attention 1, portions of a prompt 2, blocks of one 2; gated linear
+// attention 1, by chunks 3), output projection, rows, up, down, rows; an expert layer adds, with more rows than 16, the
+// router's product, 2 for routing and 1 that puts the rows in order.
 // The rows launch (rows.hip) norms and adds what a sublayer produced and norms what the next one reads.
 #include <string.h>
 
@@ -54,7 +54,7 @@ bool sandwich_pointers_ok(const vui_lm_config& c, const vui_lm_layer& L) {
 size_t sandwich_carve(const vui_lm_config* c, const vui_lm_layer* layers, vui_lm_ctx* x, char* base) {
   const size_t e = lm_esz(*c);
   const size_t R = lm_pad(c->max_rows < 16 ? 16 : c->max_rows, 16);
-  size_t q = 0, raw = 0, ac = 0, pt = 0, ff = 0, yr = R, bs = 0, up = 0, de = 0, rl = 0, ch = 0, en = 0, ti = 0, xg = 0;
+  size_t q = 0, raw = 0, ac = 0, pt = 0, ff = 0, yr = R, bs = 0, up = 0, de = 0, rl = 0, ch = 0, en = 0, ti = 0, xg = 0, ar = 0;
   bool loops = false;
   vui_lm_dims d;
   memset(&d, 0, sizeof(d));
@@ -73,6 +73,7 @@ size_t sandwich_carve(const vui_lm_config* c, const vui_lm_layer* layers, vui_lm
       size_t rows = R;  // rows x splits of attention pieces
       for (int M = 1; M <= (int)R && M <= 1024; ++M) mx(rows, (size_t)M * sig_splits(M, L.heads, L.kv_heads));
       mx(pt, rows * H * d.vdim16);
+      mx(ar, R * L.kv_heads * ((H / L.kv_heads + 15) / 16));
     }
     if (L.experts > 0) {
       const size_t n = R * L.top;
@@ -108,6 +109,8 @@ size_t sandwich_carve(const vui_lm_config* c, const vui_lm_layer* layers, vui_lm
   TAKE(ent, int32_t*, en * 4);
   TAKE(tile_e, int32_t*, ti * 4);
   TAKE(n_tiles, int32_t*, 4);
+  TAKE(arrived, uint32_t*, (ar + 1) * 4);
+  if (x) x->n_arrived = (int)ar + 1;
 #undef TAKE
   return off;
 }
@@ -148,7 +151,7 @@ static int mixer(vui_lm_ctx* x, int l, int M, const LmRows& rows, hipStream_t st
     a.scale = L.scale; a.eps = x->c.norm_eps; a.rows = rows; a.d = d; a.raw = x->raw; a.ld = d.in_rows;
     a.q_norm = L.q_norm; a.k_norm = L.k_norm; a.temp_coef = L.temp_coef; a.temp_every = L.temp_every < 1 ? 1 : L.temp_every;
     a.bias = L.dist_bias; a.bias_len = L.bias_len; a.k_cache = L.k_cache; a.v_cache = L.v_cache;
-    a.q = x->qu; a.q_z = (size_t)x->R16 * d.dim64; a.part = x->part; a.act = x->act;
+    a.q = x->qu; a.q_z = (size_t)x->R16 * d.dim64; a.part = x->part; a.arrived = x->arrived; a.act = x->act;
     if (!sig_step_fused(x->c.dtype, rows, d) && (rc = launch_sig_prep(a, st))) return rc;
     if (rows.seq && M >= x->attn_from && x->c.dtype == VUI_DTYPE_BF16 && sig_mfma_ok(d)) {
       rc = launch_sig_prompt(a, st);
@@ -183,7 +186,7 @@ static int feed_forward(vui_lm_ctx* x, int l, int M, const LmRows& rows, hipStre
   }
   if (!lm_rows_routes(M, d.experts16) && (rc = plain(x, d, rows, x->xt, L.w_router, L.router_bias, M, d.experts16, d.w64, x->rlog, st))) return rc;
   const RouteArgs r = routing(x, l, M);
-  if (!lm_rows_routes(M, d.experts16) || M > 1) {
+  if (!lm_rows_routes(M, d.experts16) || !lm_rows_sorts(M, L.top)) {
     if ((rc = launch_moe_route(r, st))) return rc;
   }
   up.ent = x->ent; up.tile_e = x->tile_e; up.n_tiles = x->n_tiles; up.top = L.top; up.wz = (size_t)d.ff16 * d.w64;
@@ -217,7 +220,7 @@ int sandwich_layers(vui_lm_ctx* x, const int64_t* tokens, int M, const LmRows& r
   };
   ahead(0);
   RowArgs emb = r;
-  emb.tokens = tokens;
+  emb.tokens = tokens; emb.clear = x->arrived; emb.n_clear = x->n_arrived;
   int rc = launch_lm_rows(emb, st);
   for (int l = 0; l < n && !rc; ++l) {
     const vui_lm_layer& L = x->layers[l];
@@ -236,7 +239,7 @@ int sandwich_layers(vui_lm_ctx* x, const int64_t* tokens, int M, const LmRows& r
       RowArgs mid = r;
       if (L.experts > 0 && lm_rows_routes(M, d.experts16)) {
         mid.w_router = L.w_router; mid.router_bias = L.router_bias; mid.experts16 = d.experts16; mid.rlog = x->rlog;
-        mid.route = routing(x, l, M);
+        mid.route = routing(x, l, M); mid.arrived = lm_rows_sorts(M, L.top) ? x->arrived + x->n_arrived - 1 : nullptr;
       }
       if ((rc = launch_lm_rows(mid, st))) return rc;
       if ((rc = feed_forward(x, l, M, rows, st))) return rc;

@@ -266,13 +266,51 @@ __global__ __launch_bounds__(256) void sig_piece_mfma_kernel(const SigAttnArgs p
 #pragma unroll
   for (int d = 0; d < VT; ++d) *reinterpret_cast<tl_f32x4*>(&s_acc[wave][(d * 64 + lane) * 4]) = acc[d];
   __syncthreads();
+  const int np = (len + chunk - 1) / chunk;  // pieces that exist
+  auto out = [&](int d, int hh, int k4, const tl_f32x4& o) {
+    const float f = 1.0f / (1.0f + expf(-bf2f(row[sig_cols(p).g + h0 + hh])));
+    const float r[4] = {o[0] * f, o[1] * f, o[2] * f, o[3] * f};
+    Tl<bf16_t>::st4((bf16_t*)p.act + tl_off<bf16_t>(m, (h0 + hh) * p.d.vdim16 + 16 * d + 4 * k4, p.d.out_k), r);
+  };
   for (int sl = tid; sl < nvb * 64; sl += 256) {
     const int d = sl >> 6, hh = sl & 15, k4 = (sl >> 4) & 3;
     if (hh >= nh) continue;
     tl_f32x4 o = *reinterpret_cast<const tl_f32x4*>(&s_acc[0][sl * 4]);
 #pragma unroll
     for (int w = 1; w < 4; ++w) o += *reinterpret_cast<const tl_f32x4*>(&s_acc[w][sl * 4]);
-    *reinterpret_cast<tl_f32x4*>(p.part + (((size_t)m * p.heads + h0 + hh) * p.n_splits + sp) * p.d.vdim16 + 16 * d + 4 * k4) = o;
+    if (np == 1) { out(d, hh, k4, o); continue; }
+    float* dst = p.part + (((size_t)m * p.heads + h0 + hh) * p.n_splits + sp) * p.d.vdim16 + 16 * d + 4 * k4;
+    st_dev(dst, o[0], o[1]);
+    st_dev(dst + 2, o[2], o[3]);
+  }
+  if (np == 1) return;
+  // the last piece of these heads to arrive adds all of them in order (a launch that did it took 4 us, this one takes 1.7 more)
+  __shared__ uint32_t s_last;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (tid == 0) {
+    uint32_t* n = p.arrived + (size_t)m * gridDim.y + blockIdx.y;
+    s_last = __hip_atomic_fetch_add(n, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)np - 1;
+    if (s_last) __hip_atomic_store(n, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  if (!s_last) return;
+  for (int i = tid; i < nvb * 4 * nh; i += 256) {
+    const int hh = i / (nvb * 4), c = i - hh * (nvb * 4);
+    const float* src = p.part + ((size_t)m * p.heads + h0 + hh) * p.n_splits * p.d.vdim16 + 4 * c;
+    tl_f32x4 o = {0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < np; s0 += 8) {
+      uint64_t v[8][2];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const float* q = src + (size_t)min(s0 + u, np - 1) * p.d.vdim16;
+        v[u][0] = ld_dev(q); v[u][1] = ld_dev(q + 2);
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (s0 + u < np) o += tl_f32x4{lo_f(v[u][0]), hi_f(v[u][0]), lo_f(v[u][1]), hi_f(v[u][1])};
+    }
+    out(c >> 2, hh, c & 3, o);
   }
 }
 
@@ -435,11 +473,10 @@ int launch_sig_pieces(const SigAttnArgs& a, hipStream_t st) {
     const size_t lds = (size_t)(a.d.dim64 + a.d.vdim16) * 4;
     if (a.dtype == VUI_DTYPE_F32) hipLaunchKernelGGL(sig_piece_kernel<float>, grid, dim3(256), lds, st, a);
     else hipLaunchKernelGGL(sig_piece_kernel<bf16_t>, grid, dim3(256), lds, st, a);
+    const dim3 merge((a.heads * a.d.vdim16 / 4 + 255) / 256, a.M);
+    if (a.dtype == VUI_DTYPE_F32) hipLaunchKernelGGL(sig_merge_kernel<float>, merge, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL(sig_merge_kernel<bf16_t>, merge, dim3(256), 0, st, a);
   }
-  HIP_TRY(hipGetLastError());
-  const dim3 grid((a.heads * a.d.vdim16 / 4 + 255) / 256, a.M);
-  if (a.dtype == VUI_DTYPE_F32) hipLaunchKernelGGL(sig_merge_kernel<float>, grid, dim3(256), 0, st, a);
-  else hipLaunchKernelGGL(sig_merge_kernel<bf16_t>, grid, dim3(256), 0, st, a);
   HIP_TRY(hipGetLastError());
   return VUI_OK;
 }
