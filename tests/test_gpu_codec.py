@@ -264,6 +264,20 @@ def test_full_dims_blocks_equal_single_frames(full):
         assert err(got, one.cpu()) < 5e-5  # measured 1e-5
 
 
+@pytest.mark.parametrize("power", [-60, -20, 20, 60])
+def test_wide_products_of_any_magnitude(full, power):
+    """Parts of an operand keep its exponent: a layer's weights times a power of two and its scale by the inverse give the same audio,
+    bit by bit, from blocks of frames (power-of-two factors pass through every sum of the three parts)."""
+    d, sd, dec, fx = full
+    other = dict(sd)
+    for i in range(2):
+        for k in ("pwconv2.weight", "pwconv2.bias"):
+            other[f"upsample.{i}.1.{k}"] = sd[f"upsample.{i}.1.{k}"] * 2.0 ** power
+        other[f"upsample.{i}.1.gamma"] = sd[f"upsample.{i}.1.gamma"] * 2.0 ** -power
+    codes = torch.randint(0, d.codebook_size, (1, d.n_codebooks, 35), generator=torch.Generator().manual_seed(9)).cuda()
+    assert torch.equal(native(d, other)(codes), dec(codes))
+
+
 @pytest.mark.parametrize("d_model", [1024, 1312, 2048])
 def test_blocks_of_wide_pre_transformers(d_model):
     """Widths whose normed products take eight waves (25-48 units of 32 channels from 17 frames on, 33-64 below) or split

@@ -21,7 +21,7 @@
 //
 // Several frames at once (vui_codec_decode_block: offline calls, the seeding of a stream): the same steps over
 // frames x columns, on buffers that hold a whole block with the histories in front; wide products run in
-// cv_wide_kernel.  93 frames: 56.6 ms one after the other, 7.9 ms in blocks of 32 (MI355X).
+// cv_wide_kernel.  93 frames: 56.6 ms one after the other, 6.3 ms in blocks of 32 (MI355X).
 #include "common.h"
 #include "internal.h"
 #include "../../include/vui_codec.h"
@@ -329,15 +329,33 @@ __global__ __launch_bounds__(NW * 64, 2) void cv_gemm1_kernel(const CvGemm p) {
 }
 
 // ---- the same product for many columns (several frames at once) ----
-// Bound by the fp32 matrix instructions (157 TFLOP/s): 256 flops per CU and cycle against 8 bytes of operands, so
-// tiles of BM x BN = 128 x 128 (or what divides M) through LDS: a K step is one (tap, 32-channel) unit, fetched into
-// registers while the one before it is multiplied, two LDS buffers, one barrier per step.  v_mfma_f32_32x32x2_f32; the
-// lane halves take k = 8j + s and 8j + 4 + s, so that a lane's weights of four steps are one 16-byte LDS read.
+// On the bf16 matrix instructions, which are 16 times the rate of the fp32 ones (157 TFLOP/s): every fp32 operand is the exact sum of three
+// bf16 numbers (8 bits each, nearest, so that the rest halves once more), and of their nine products the six that
+// reach 2^-24 of the value are summed in fp32, small ones first.  What is left out is 2^-26 of a product; the sums have
+// fewer roundings than with v_mfma_f32_32x32x2_f32 (sixteen products per step instead of two).
+// 32 frames: 7-tap convolutions of 768 / 384 / 192 / 96 channels 86 / 105 / 121 / 91 us -> 55 / 63 / 83 / 62 (1200 TFLOP/s
+// of bf16 products in the first, what hipBLASLt reaches at 8192^3), 1x1 19 / 30 / 32 / 33 -> 16 / 29 / 26 / 29; error of 93
+// frames against 64 bits 4.1e-6 -> 3.9e-6.  An input that is not finite makes its columns NaN.
+// Tiles of BM x BN = 128 x 128 (or what divides M) of four waves through LDS, three planes of each operand: a K step is one (tap,
+// 32-channel) unit, fetched into registers while the one before it is multiplied, split on the way to LDS.  One buffer: two
+// workgroups of a CU overlap better than the steps of one (eight waves with two buffers and one to three units in flight: 75 us of
+// the 384-channel convolution instead of 63).
 // Where the tiles are fewer than the CUs their units are split over workgroups, and cv_finish_kernel adds the parts.
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
+typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 cv_bf16x8;
 
 #define CVW_RUN 4
-#define CVW_AS 36  // floats between weight rows in LDS: 16-byte reads of 8 rows fall on different banks
+// In LDS a row's (or column's) 32 channels of a plane are four pieces of 16 bytes; a piece's place turns with the row, so that 16-byte
+// reads of eight rows fall on different banks.
+__device__ __forceinline__ int cv_at(int row, int piece) { return row * 32 + 8 * (piece ^ (row >> 2 & 3)); }
+
+// two fp32 values -> their three bf16 parts, packed
+__device__ __forceinline__ void cv_split2(float a, float b, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
+  hi = f2bf2(a, b);
+  a -= bf_lo(hi); b -= bf_hi(hi);
+  mid = f2bf2(a, b);
+  lo = f2bf2(a - bf_lo(mid), b - bf_hi(mid));
+}
 
 // bias, activation or residual, and the outputs of one column of eight rows m, m + step, ... (uniform over a wave)
 struct CvBases { int res, raw, act; };
@@ -397,20 +415,28 @@ __device__ __forceinline__ void cv_finish_rows(const CvGemm& p, const CvBases& b
 }
 
 template <int MI, int NI, int WM, int WN>
-__global__ __launch_bounds__(512, MI * WM == 4 ? 4 : 2) void cv_wide_kernel(const CvGemm p) {
-  constexpr int NT = 512, BM = 32 * MI * WM, BN = 32 * NI * WN, BS = BN + 8;  // BS: rows 4 apart start 32 banks apart
-  constexpr int NA = (BM * 8 + NT - 1) / NT, NB = 32 * BN / NT, KR = NT / BN;  // 16-byte / 4-byte loads per thread and step
-  static_assert(WM * WN == 8 && NT % BN == 0, "eight waves, whole rows per pass");
-  constexpr int OPS = 2 * (BM * CVW_AS + 32 * BS);
-  __shared__ __align__(16) float lds[OPS > BM * BS ? OPS : BM * BS];  // the operands, then the sums
-  auto la = [&](int b, int i) -> float& { return lds[b * BM * CVW_AS + i]; };
-  auto lb = [&](int b, int i) -> float& { return lds[2 * BM * CVW_AS + b * 32 * BS + i]; };
+__global__ __launch_bounds__(256, 2) void cv_wide_kernel(const CvGemm p) {
+  constexpr int NT = 256, BM = 32 * MI * WM, BN = 32 * NI * WN, BS = BN + 8;
+  constexpr int NA = (BM * 8 + NT - 1) / NT, NB = 32 * BN / NT;  // 16-byte / 4-byte loads per thread and step
+  static_assert(WM * WN == 4 && NT % BN == 0 && NB % 8 == 0, "four waves, whole columns per thread");
+  constexpr int PL = (BM + BN) * 32;  // bf16 of one plane of both operands
+  constexpr int OPS = 3 * PL * 2;
+  __shared__ __align__(16) char raw[OPS > BM * BS * 4 ? OPS : BM * BS * 4];  // the operands, then the sums
+  float* const lds = reinterpret_cast<float*>(raw);
+  auto la = [&](int plane, int row, int piece) { return reinterpret_cast<bf16_t*>(raw) + plane * PL + cv_at(row, piece); };
+  auto lb = [&](int plane, int col, int piece) { return la(plane, 0, 0) + BM * 32 + cv_at(col, piece); };
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int l32 = lane & 31, h = lane >> 5, wm = wave % WM, wn = wave / WM;
-  const int m0 = blockIdx.x * BM, t0 = blockIdx.y * BN, z = blockIdx.z;
+  // Workgroups go round the eight XCDs, whose L2s are their own: each gets a contiguous range of the tiles, columns slowest, so that
+  // it meets an eighth of the input (or, of few columns, of the weights) instead of all of it.
+  // (384 channels x 5120 columns: 66 -> 63 us, 768 x 1280 54 -> 53.)
+  const int MT = p.M / BM, NTL = (p.T + BN - 1) / BN;
+  const int n8 = MT * NTL * p.splits, x8 = blockIdx.x & 7, at = x8 * (n8 >> 3) + min(x8, n8 & 7) + (int)(blockIdx.x >> 3);
+  const int tz = at / MT, tl = tz / p.splits;
+  const int m0 = (at - tz * MT) * BM, t0 = tl * BN, z = tz - tl * p.splits, cols = NTL * BN;
   const int G = p.Cin >> 5, Uall = p.taps * G;
   const int ub = (int)((int64_t)Uall * z / p.splits), ue = (int)((int64_t)Uall * (z + 1) / p.splits);
-  const int f = *p.ctr - p.nf, ib_ = ring_base(p.in, f);
+  const int f = *p.ctr - p.nf;
 
   // acc: the products of CVW_RUN units; sum: those before.  One chain over all units (168 of them in block 1) would
   // round each step against the full sum: 1.4 times the error against 64 bits of the audio.
@@ -421,54 +447,70 @@ __global__ __launch_bounds__(512, MI * WM == 4 ? 4 : 2) void cv_wide_kernel(cons
 #pragma unroll
     for (int n = 0; n < NI; ++n) acc[i][n] = sum[i][n] = zero;
 
-  const int bc = tid % BN, bk = tid / BN;  // this thread's column and first channel of a step
+  const int bc = tid % BN, bk = tid / BN * NB;  // this thread's column and first channel of a step
   floatx4 ra[NA];  // native vectors: an array of HIP's float4 structs stayed in scratch memory
   float rb[NB];
+  const uint32_t woff = (tid >> 3) * p.Cin + (tid & 7) * 4, xoff = bk * p.in.rs + bc;
   int tap = ub / G, grp = ub - tap * G;
   auto fetch = [&]() {
-    const float* wp = p.W + ((size_t)tap * p.M + m0 + (tid >> 3)) * p.Cin + grp * 32 + (tid & 7) * 4;
+    const float* wp = p.W + ((size_t)tap * p.M + m0) * p.Cin + grp * 32;  // uniform, with offsets of the thread's own
 #pragma unroll
     for (int i = 0; i < NA; ++i)
-      if ((i + 1) * (NT / 8) <= BM || (tid >> 3) + i * (NT / 8) < BM) ra[i] = *reinterpret_cast<const floatx4*>(wp + (size_t)i * (NT / 8) * p.Cin);
-    // columns behind T are whatever the ring holds there: they reach no output
-    const float* xp = ring_ptr(p.in, ib_, grp * 32 + bk, t0 + bc + tap * p.dil);
+      if ((i + 1) * (NT / 8) <= BM || (tid >> 3) + i * (NT / 8) < BM) ra[i] = *reinterpret_cast<const floatx4*>(wp + (size_t)i * (NT / 8) * p.Cin + woff);
+    // a block's buffer has no end to turn at; columns behind T are whatever is there: they reach no output
+    const float* xp = p.in.p + (size_t)grp * 32 * p.in.rs + t0 + tap * p.dil;
 #pragma unroll
-    for (int i = 0; i < NB; ++i) rb[i] = xp[(size_t)i * KR * p.in.rs];
+    for (int i = 0; i < NB; ++i) rb[i] = xp[(size_t)i * p.in.rs + xoff];
     if (++grp == G) { grp = 0; ++tap; }
   };
-  auto stage = [&](int b) {
+  auto stage = [&]() {
 #pragma unroll
     for (int i = 0; i < NA; ++i)
-      if ((i + 1) * (NT / 8) <= BM || (tid >> 3) + i * (NT / 8) < BM)
-        *reinterpret_cast<floatx4*>(&la(b, ((tid >> 3) + (NT / 8) * i) * CVW_AS + (tid & 7) * 4)) = ra[i];
+      if ((i + 1) * (NT / 8) <= BM || (tid >> 3) + i * (NT / 8) < BM) {
+        uint2 q[3];
+        cv_split2(ra[i][0], ra[i][1], q[0].x, q[1].x, q[2].x);
+        cv_split2(ra[i][2], ra[i][3], q[0].y, q[1].y, q[2].y);
 #pragma unroll
-    for (int i = 0; i < NB; ++i) lb(b, (bk + KR * i) * BS + bc) = rb[i];
+        for (int k = 0; k < 3; ++k) *reinterpret_cast<uint2*>(la(k, (tid >> 3) + (NT / 8) * i, (tid & 7) >> 1) + (tid & 1) * 4) = q[k];
+      }
+#pragma unroll
+      for (int i = 0; i < NB; i += 8) {
+        uint4 q[3];
+        cv_split2(rb[i], rb[i + 1], q[0].x, q[1].x, q[2].x);
+        cv_split2(rb[i + 2], rb[i + 3], q[0].y, q[1].y, q[2].y);
+        cv_split2(rb[i + 4], rb[i + 5], q[0].z, q[1].z, q[2].z);
+        cv_split2(rb[i + 6], rb[i + 7], q[0].w, q[1].w, q[2].w);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) *reinterpret_cast<uint4*>(lb(k, bc, (bk + i) >> 3)) = q[k];
+      }
   };
+  auto frag = [](const bf16_t* q) { return __builtin_bit_cast(cv_bf16x8, *reinterpret_cast<const uint4*>(q)); };
   if (ub < ue) {
     fetch();
-    stage(0);
+    stage();
   }
   __syncthreads();
   for (int u = ub; u < ue; ++u) {
-    const int b = (u - ub) & 1;
     if (u + 1 < ue) fetch();
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      floatx4 a[MI];
+    for (int j = 0; j < 2; ++j) {  // 16 channels: a lane holds eight of its row or column
+      cv_bf16x8 a[3][MI], x[3][NI];
 #pragma unroll
-      for (int i = 0; i < MI; ++i)
-        a[i] = *reinterpret_cast<const floatx4*>(&la(b, ((wm * MI + i) * 32 + l32) * CVW_AS + 8 * j + 4 * h));
+      for (int k = 0; k < 3; ++k) {
 #pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        float x[NI];
+        for (int i = 0; i < MI; ++i) a[k][i] = frag(la(k, (wm * MI + i) * 32 + l32, 2 * j + h));
 #pragma unroll
-        for (int n = 0; n < NI; ++n) x[n] = lb(b, (8 * j + 4 * h + s) * BS + (wn * NI + n) * 32 + l32);
-#pragma unroll
-        for (int i = 0; i < MI; ++i) {
-#pragma unroll
-          for (int n = 0; n < NI; ++n) acc[i][n] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][s], x[n], acc[i][n], 0, 0, 0);
-        }
+        for (int n = 0; n < NI; ++n) x[k][n] = frag(lb(k, (wn * NI + n) * 32 + l32, 2 * j + h));
       }
+      // {part of the weight, part of the input}
+      constexpr int PAIR[6][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};
+#pragma unroll
+      for (int c = 0; c < 6; ++c)
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int n = 0; n < NI; ++n)
+            acc[i][n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[PAIR[c][0]][i], x[PAIR[c][1]][n], acc[i][n], 0, 0, 0);
     }
     if ((u - ub) % CVW_RUN == CVW_RUN - 1 || u + 1 == ue) {
 #pragma unroll
@@ -476,19 +518,22 @@ __global__ __launch_bounds__(512, MI * WM == 4 ? 4 : 2) void cv_wide_kernel(cons
 #pragma unroll
         for (int n = 0; n < NI; ++n) { sum[i][n] += acc[i][n]; acc[i][n] = zero; }
     }
-    if (u + 1 < ue) stage(b ^ 1);
     __syncthreads();
+    if (u + 1 < ue) {
+      stage();
+      __syncthreads();
+    }
   }
 
   if (p.splits > 1) {  // cv_finish_kernel adds the parts
-    float* part = p.part + ((size_t)z * p.M + m0) * (gridDim.y * BN) + t0 + wn * NI * 32 + l32;
+    float* part = p.part + ((size_t)z * p.M + m0) * cols + t0 + wn * NI * 32 + l32;
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
       for (int r = 0; r < 16; ++r)
 #pragma unroll
         for (int n = 0; n < NI; ++n)
-          part[(size_t)((wm * MI + i) * 32 + 8 * (r >> 2) + 4 * h + (r & 3)) * (gridDim.y * BN) + n * 32] = sum[i][n][r];
+          part[(size_t)((wm * MI + i) * 32 + 8 * (r >> 2) + 4 * h + (r & 3)) * cols + n * 32] = sum[i][n][r];
     return;
   }
   // The sums go through LDS so that a wave finishes whole rows: what depends on the row is scalar, and 64 columns are
@@ -1429,16 +1474,17 @@ static void grid_for(size_t n, dim3& g) { size_t b = (n + 255) / 256; g = dim3((
 
 // ---- launch shapes ----
 struct CvScratch { size_t part, cnt; };  // floats of partial sums, arrival counters
-// tiles of cv_wide_kernel, and what one unit of a tile costs against 128 x 128 (measured: 2.2 us)
+// tiles of cv_wide_kernel, and what one unit of a tile costs against 128 x 128
 struct WideTile { int bm, bn; float unit; };
-static const WideTile kWide[] = {{128, 128, 1.0f}, {96, 256, 1.5f}, {64, 256, 1.0f}, {128, 64, 0.74f}, {32, 256, 0.74f}};
+#define CVW_PAIR 2.6   // us of a unit of 128 x 128 for two workgroups of a CU, and for one
+#define CVW_ALONE 1.6
+static const WideTile kWide[] = {{128, 128, 1.0f}, {96, 128, 0.79f}, {64, 128, 0.63f}, {128, 64, 0.63f}, {32, 128, 0.55f}};
 
 // Chooses tile width, splits and kernel for g.T columns.
 static CvScratch cv_plan(CvGemm& g) {
   const int U = g.taps * (g.Cin / 32), M = g.M, T = g.T;
   if (g.nf > 1 && T >= CV_WIDE_T && M % 32 == 0 && g.in_mode == IN_PLAIN && g.epi != EPI_SILU_PAIR) {
-    // Tile and splits: the number of rounds over 256 CUs times a workgroup's work in units (about 4 more for what a
-    // tile costs besides its products), and for split tiles the second launch and its traffic.
+    // Tile and splits: what the workgroups of a CU take, in pairs, and for split tiles the second launch and its traffic.
     size_t part = 0;
     double cost = 0;
     for (int i = 0; i < 5; ++i) {
@@ -1446,7 +1492,8 @@ static CvScratch cv_plan(CvGemm& g) {
       if (M % w.bm) continue;
       const int cols = (T + w.bn - 1) / w.bn * w.bn, tiles = (M / w.bm) * (cols / w.bn);
       for (int sp = 1; sp <= 16 && (sp == 1 || U / sp >= 4); ++sp) {
-        const double c = (double)((tiles * sp + 255) / 256) * ((U + sp - 1) / sp + 4) * w.unit + (sp > 1 ? 3 + 9e-7 * sp * M * T : 0);
+        const int wgs = (tiles * sp + 255) / 256;
+        const double c = (wgs / 2 * CVW_PAIR + wgs % 2 * CVW_ALONE) * ((U + sp - 1) / sp) * w.unit + (sp > 1 ? 6 + 1e-6 * sp * M * T : 0);
         if (cost && c >= cost) continue;
         cost = c;
         g.tt = 0; g.wide = i; g.splits = sp;
@@ -1882,15 +1929,16 @@ static int launch_cv_gemm(const CvGemm& g, bool w_nt, hipStream_t st) {
   if (g.M % 16 || g.Cin % 32 || g.T < 1) { vui_set_error("codec gemm: bad shape M=%d Cin=%d T=%d", g.M, g.Cin, g.T); return VUI_EINVAL; }
   if (g.tt == 0) {
     const WideTile& w = kWide[g.wide];
-    const dim3 grid(g.M / w.bm, (g.T + w.bn - 1) / w.bn, g.splits);
-#define CV_WIDE(...) hipLaunchKernelGGL((cv_wide_kernel<__VA_ARGS__>), grid, dim3(512), 0, st, g)
-    if (g.wide == 0) CV_WIDE(2, 1, 2, 4);
-    else if (g.wide == 1) CV_WIDE(3, 1, 1, 8);
-    else if (g.wide == 2) CV_WIDE(2, 1, 1, 8);
-    else if (g.wide == 3) CV_WIDE(1, 1, 4, 2);
-    else CV_WIDE(1, 1, 1, 8);
+    const int tiles = (g.T + w.bn - 1) / w.bn;
+    const dim3 grid(g.M / w.bm * tiles * g.splits);
+#define CV_WIDE(...) hipLaunchKernelGGL((cv_wide_kernel<__VA_ARGS__>), grid, dim3(256), 0, st, g)
+    if (g.wide == 0) CV_WIDE(2, 2, 2, 2);
+    else if (g.wide == 1) CV_WIDE(3, 1, 1, 4);
+    else if (g.wide == 2) CV_WIDE(1, 2, 2, 2);
+    else if (g.wide == 3) CV_WIDE(2, 1, 2, 2);
+    else CV_WIDE(1, 1, 1, 4);
 #undef CV_WIDE
-    if (g.splits > 1) hipLaunchKernelGGL(cv_finish_kernel, dim3((g.T + 63) / 64, g.M / 32), dim3(256), 0, st, g, (int)grid.y * w.bn);
+    if (g.splits > 1) hipLaunchKernelGGL(cv_finish_kernel, dim3((g.T + 63) / 64, g.M / 32), dim3(256), 0, st, g, tiles * w.bn);
     return VUI_OK;
   }
   const dim3 grid(g.M / 16, (g.T + 16 * g.tt - 1) / (16 * g.tt), g.splits);
