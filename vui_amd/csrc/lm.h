@@ -30,8 +30,7 @@ enum {
   LM_IN_GRU_SEQ,    // ... positions of one sequence: update pairs for the scan
   LM_OUT,           // x += W y; operand copy and sums of squares of the new x
   LM_LOGITS,        // fp32 logits of chosen rows
-  LM_EXPAND_K,      // keys of one head per blockIdx.z from cached latents
-  LM_EXPAND_V,      // values, transposed
+  LM_EXPAND,        // keys of one head per blockIdx.z from cached latents, then values, transposed (bf16)
   // sandwich layers (rows arrive normed)
   LM_HEAD,          // LM_LOGITS without a row scale
   LM_PROJ,          // W x + bias in the context's dtype, row-major
@@ -82,9 +81,12 @@ struct LmGemm {
   int32_t* upd_lens;
   const int32_t* upd_inc;
   int upd_rows;
-  // expansion
-  void* kv_out;
-  size_t kv_z;
+  // expansion: keys (N features from W) and values (n_v features from w_v) of every head
+  void *kv_out, *v_out;
+  size_t kv_z, v_z;
+  const void* w_v;
+  size_t wz_v;
+  int n_v, heads;
   // sandwich layers
   void* out;       // (rows, ldo) of the epilogue's type
   int ldo;

@@ -44,8 +44,7 @@ struct LmPre {
   float4 a, b, c;
 };
 
-// One unit of 16 rows x 16 features: a lane holds features n ... n + 3 of row m (LM_EXPAND_V: rows m ... m + 3 of feature
-// n).  mix: the unit is the update gate of a recurrence, xv and gv the candidate and the output gate beside it.
+// One unit of 16 rows x 16 features: a lane holds features n ... n + 3 of row m.  mix: the unit is the update gate of a recurrence, xv and gv the candidate and the output gate beside it.
 template <typename T, int EPI, bool PRE>
 __device__ __forceinline__ void lm_unit(const LmGemm& p, const int m, const int nb, const int n, const int l16, const int kg,
                                         const bool live, const bool mix, float (&v)[4], const float (&xv)[4], const float (&gv)[4],
@@ -156,19 +155,6 @@ __device__ __forceinline__ void lm_unit(const LmGemm& p, const int m, const int 
     Tl<T>::st4((T*)p.act + tl_off<T>(m, n, p.act_k), v);
     return;
   }
-  if (EPI == LM_EXPAND_K) {
-    if (live) Tl<T>::st4((T*)p.kv_out + blockIdx.z * p.kv_z + tl_off<T>(m, n, p.d.dim64), v);
-    return;
-  }
-  if (EPI == LM_EXPAND_V) {
-    // blocks of 16 value dims x 32 keys; a lane of the attention kernel reads the keys 4 kg .. + 3 of both halves
-    if (live) {
-      T* dst = (T*)p.kv_out + blockIdx.z * p.kv_z + ((size_t)nb * (p.d.s64 >> 5) + (m >> 5)) * 512 +
-               (l16 + 16 * ((m & 15) >> 2)) * 8 + 4 * ((m & 31) >> 4);
-      Tl<T>::st4(dst, v);
-    }
-    return;
-  }
 }
 
 template <typename T, int MB, int NB, int WAVES, int EPI>
@@ -176,7 +162,6 @@ __global__ __launch_bounds__(64 * WAVES) void lm_gemm_kernel(const LmGemm p) {
   constexpr bool SCALED = EPI == LM_IN_ATTN || EPI == LM_IN_GRU_STEP || EPI == LM_IN_GRU_SEQ || EPI == LM_LOGITS;
   constexpr bool GRU = EPI == LM_IN_GRU_STEP || EPI == LM_IN_GRU_SEQ;
   constexpr bool LOGITS = EPI == LM_LOGITS || EPI == LM_HEAD, MOE = EPI == LM_MOE_UP || EPI == LM_MOE_DOWN;
-  constexpr bool ROWS_FIRST = EPI == LM_EXPAND_V;  // a lane then holds four consecutive rows of one feature
   constexpr int EP = Tl<T>::EP, P = 16 / EP, TILE = MB * NB * 256;
   __shared__ __align__(16) float part[WAVES * TILE];
   __shared__ float srow[MB * 16];
@@ -209,7 +194,7 @@ __global__ __launch_bounds__(64 * WAVES) void lm_gemm_kernel(const LmGemm p) {
       xr[j] = (const T*)p.X + (size_t)(r >> 4) * nsteps * 1024 + ((r & 15) + 16 * kg) * EP;
     } else {
       // few rows: lanes without a row re-read the last one instead of fetching a block that is mostly padding
-      const int l = MB == 1 && !ROWS_FIRST ? min(l16, p.M - 1 - m0) + 16 * kg : lane;
+      const int l = MB == 1 ? min(l16, p.M - 1 - m0) + 16 * kg : lane;
       xr[j] = (const T*)p.X + (size_t)min((m0 >> 4) + j, MBL - 1) * nsteps * 1024 + l * EP;
     }
   }
@@ -278,7 +263,7 @@ __global__ __launch_bounds__(64 * WAVES) void lm_gemm_kernel(const LmGemm p) {
         for (int i = 0; i < NB; ++i)
 #pragma unroll
           for (int j = 0; j < MB; ++j)
-            acc[i][j] = ROWS_FIRST ? Tl<T>::mma(xa[u][j][h], wa[u][i][h], acc[i][j]) : Tl<T>::mma(wa[u][i][h], xa[u][j][h], acc[i][j]);
+            acc[i][j] = Tl<T>::mma(wa[u][i][h], xa[u][j][h], acc[i][j]);
     }
   }
 #pragma unroll
@@ -301,9 +286,9 @@ __global__ __launch_bounds__(64 * WAVES) void lm_gemm_kernel(const LmGemm p) {
   const int units = mix ? MB : MB * NB;
   for (int u = wave; u < units; u += WAVES) {
     const int j = mix ? u : u % MB, i0 = mix ? 0 : u / MB;
-    const int m = m0 + 16 * j + (ROWS_FIRST ? 4 * kg : l16);
+    const int m = m0 + 16 * j + l16;
     const int nb = nb0 + i0;
-    const int n = nb * 16 + (ROWS_FIRST ? l16 : 4 * kg);
+    const int n = nb * 16 + 4 * kg;
     const bool live = (MOE || m < p.M) && nb < NBL;
     const float sc = SCALED ? srow[16 * j + l16] : 1.f;
     float v[4];
@@ -346,7 +331,9 @@ __global__ __launch_bounds__(256, 2) void lm_wide_kernel(const LmGemm p) {
   __shared__ float srow[MB * 16];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int l16 = lane & 15, kg = lane >> 4, wm = wave % WM, wn = wave / WM;
-  const int MBL = (p.M + 15) >> 4, NBL = p.N >> 4, MT = MOE ? p.max_tiles : (MBL + MB - 1) / MB, NT = (NBL + NB - 1) / NB;
+  const bool val = EPI == LM_EXPAND && (int)blockIdx.z >= p.heads;  // values of a head behind the keys of all
+  const int head = (int)blockIdx.z - (val ? p.heads : 0);
+  const int MBL = (p.M + 15) >> 4, NBL = (val ? p.n_v : p.N) >> 4, MT = MOE ? p.max_tiles : (MBL + MB - 1) / MB, NT = (NBL + NB - 1) / NB;
   int t, nt;
   if (MOE) {
     // Tiles of one expert that share features run on one XCD (workgroup i is on XCD i % 8), which reads those weights from
@@ -364,15 +351,17 @@ __global__ __launch_bounds__(256, 2) void lm_wide_kernel(const LmGemm p) {
     if (nt >= NT) return;
   } else {
     t = (int)blockIdx.x % MT; nt = (int)blockIdx.x / MT;
+    if (EPI == LM_EXPAND && nt >= NT) return;
   }
   const int mb0 = t * MB, nb0 = nt * NB, m0 = mb0 * 16;
   const int Q = p.K / (32 * KS);  // steps
-  const size_t wz = MOE ? (size_t)p.tile_e[t] * p.wz : blockIdx.z * p.wz;
+  const size_t wz = MOE ? (size_t)p.tile_e[t] * p.wz : head * (val ? p.wz_v : p.wz);
+  const char* W = (const char*)(val ? p.w_v : p.W);
 
   Tile tile;
   tile.begin(lds, wave, lane,
              [&](int i) { return (const char*)p.X + (size_t)(MOE ? mb0 + i : min(mb0 + i, MBL - 1)) * Q * (KS * 1024); },
-             [&](int i) { return (const char*)p.W + wz * 2 + (size_t)min(nb0 + i, NBL - 1) * Q * (KS * 1024); });
+             [&](int i) { return W + wz * 2 + (size_t)min(nb0 + i, NBL - 1) * Q * (KS * 1024); });
   tile.prologue(Q);
 
   if (SCALED) {
@@ -434,6 +423,27 @@ __global__ __launch_bounds__(256, 2) void lm_wide_kernel(const LmGemm p) {
         for (int r = 0; r < 4; ++r) o[r] = a[r] * sc;
       };
       const int mw = m0 + wm * MBW * 16 + l16;
+      if (EPI == LM_EXPAND) {
+#pragma unroll
+        for (int j = 0; j < MBW; ++j) {
+          float v[4];
+          if (val) {
+            // Blocks of 16 value dims x 32 keys: a lane of the attention kernel reads the keys 4 kg .. + 3 of both halves.  The
+            // unit is read from LDS the other way round, four rows of a feature.
+            const float* q = reinterpret_cast<const float*>(own - lane * 16 + (i * MBW + j) * 1024) + 4 * (4 * kg + 16 * (l16 >> 2)) + (l16 & 3);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = q[4 * r];
+            const int m = m0 + (wm * MBW + j) * 16 + 4 * kg;
+            if (m < p.M)
+              Tl<bf16_t>::st4((bf16_t*)p.v_out + head * p.v_z + ((size_t)nb * (p.d.s64 >> 5) + (m >> 5)) * 512 +
+                              (l16 + 16 * ((m & 15) >> 2)) * 8 + 4 * ((m & 31) >> 4), v);
+          } else {
+            sums(i, j, v);
+            if (mw + 16 * j < p.M) Tl<bf16_t>::st4((bf16_t*)p.kv_out + head * p.kv_z + tl_off<bf16_t>(mw + 16 * j, n, p.d.dim64), v);
+          }
+        }
+        continue;
+      }
       if ((EPI == LM_IN_ATTN || GRU) && nb >= p.mix_blocks) {  // (gate, up) pairs
         const int f = p.d.ff_off + ((n - p.mix_blocks * 16) >> 1);
 #pragma unroll
@@ -463,9 +473,9 @@ __global__ __launch_bounds__(256, 2) void lm_wide_kernel(const LmGemm p) {
 #define WIDE_BY_XCD 24  // feature tiles from which an XCD's share is taken (with fewer, whole XCDs would have nothing or twice as much to do)
 template <int EPI, int MBW, int NBW, int WM, int WN, int S, int KS>
 static int go_wide(LmGemm g, int nz, hipStream_t st) {
-  const int MT = (g.M + 16 * MBW * WM - 1) / (16 * MBW * WM), NT = (g.N / 16 + NBW * WN - 1) / (NBW * WN);
+  const int MT = (g.M + 16 * MBW * WM - 1) / (16 * MBW * WM), NT = ((EPI == LM_EXPAND && g.n_v > g.N ? g.n_v : g.N) / 16 + NBW * WN - 1) / (NBW * WN);
   const bool moe = EPI == LM_MOE_UP || EPI == LM_MOE_DOWN;
-  g.by_xcd = !moe && NT >= WIDE_BY_XCD;
+  g.by_xcd = !moe && EPI != LM_EXPAND && NT >= WIDE_BY_XCD;
   const int tiles = moe ? g.max_tiles * ((NT + 7) & ~7) : g.by_xcd ? MT * ((NT + 7) & ~7) : MT * NT;
   hipLaunchKernelGGL((lm_wide_kernel<EPI, MBW, NBW, WM, WN, S, KS>), dim3((unsigned)tiles, 1, nz), dim3(256), 0, st, g);
   HIP_TRY(hipGetLastError());
@@ -500,10 +510,11 @@ static int lm_tile(int epi, int M, int N, int K) {
 }
 template <int EPI>
 static int pick_wide(int tile, const LmGemm& g, hipStream_t st) {
+  const int nz = EPI == LM_EXPAND ? 2 * g.heads : 1;
   switch (tile) {
-    case WIDE_128: return go_wide<EPI, 4, 4, 2, 2, 4, 1>(g, 1, st);
-    case WIDE_64x128: return go_wide<EPI, 4, 2, 1, 4, 3, 2>(g, 1, st);
-    default: return go_wide<EPI, 2, 2, 2, 2, 4, 2>(g, 1, st);
+    case WIDE_128: return go_wide<EPI, 4, 4, 2, 2, 4, 1>(g, nz, st);
+    case WIDE_64x128: return go_wide<EPI, 4, 2, 1, 4, 3, 2>(g, nz, st);
+    default: return go_wide<EPI, 2, 2, 2, 2, 4, 2>(g, nz, st);
   }
 }
 
@@ -547,8 +558,6 @@ static int pick(int epi, const LmGemm& g, int nz, hipStream_t st) {
     case LM_ACT: return few ? go<T, 1, 2, 8, LM_ACT>(g, nz, st) : go<T, 2, 2, 4, LM_ACT>(g, nz, st);
     case LM_MOE_UP: return few ? go<T, 1, 2, 8, LM_MOE_UP>(g, nz, st) : go<T, 2, 2, 4, LM_MOE_UP>(g, nz, st);
     case LM_MOE_DOWN: return few ? go<T, 1, 2, 8, LM_MOE_DOWN>(g, nz, st) : go<T, 2, 2, 4, LM_MOE_DOWN>(g, nz, st);
-    case LM_EXPAND_K: return go<T, 2, 2, 4, LM_EXPAND_K>(g, nz, st);
-    case LM_EXPAND_V: return go<T, 2, 2, 4, LM_EXPAND_V>(g, nz, st);
   }
   vui_set_error("lm gemm: unknown epilogue %d", epi);
   return VUI_EINVAL;
@@ -558,6 +567,11 @@ int launch_lm_gemm(int dtype, int epi, const LmGemm& g, int nz, hipStream_t st) 
   if (g.M < 1 || g.N < 16 || (g.N & 15) || g.K < 64 || (g.K & 63) || nz < 1) {
     vui_set_error("lm gemm: bad shape M=%d N=%d K=%d", g.M, g.N, g.K);
     return VUI_EINVAL;
+  }
+  if (epi == LM_EXPAND) {
+    if (dtype != VUI_DTYPE_BF16 || g.heads < 1 || g.n_v < 16 || (g.n_v & 15)) { vui_set_error("lm gemm: bad expansion"); return VUI_EINVAL; }
+    // XXX
+    return pick_wide<LM_EXPAND>(wide_pick(g.M, g.heads * (g.N + g.n_v), g.K, 1e9), g, st);
   }
   const bool gru = epi == LM_IN_GRU_STEP || epi == LM_IN_GRU_SEQ;
   if ((gru && ((g.mix_blocks % 3) || (g.N / 16) % 3)) || (epi == LM_IN_ATTN && (g.mix_blocks % 2))) {
@@ -572,23 +586,33 @@ int launch_lm_gemm(int dtype, int epi, const LmGemm& g, int nz, hipStream_t st) 
 template <typename T>
 __global__ __launch_bounds__(256) void lm_embed_kernel(const int64_t* tokens, const T* table, float* x, T* xt, float* ssq,
                                                        int width, int w64, int np, int vocab) {
-  const int m = blockIdx.x, c = blockIdx.y * 256 + threadIdx.x;
+  const int m = blockIdx.x, c = (blockIdx.y * 256 + threadIdx.x) * 4;  // four columns per lane
   int64_t t = tokens[m];
   t = t < 0 ? 0 : (t >= vocab ? vocab - 1 : t);
-  if (c < np * 16) {  // a multiple of 16: a 16-lane group is whole or absent
-    const float v = c < width ? El<T>::ld(table + (size_t)t * width + c) : 0.f;
-    x[(size_t)m * w64 + c] = v;
-    El<T>::st(xt + tl_off<T>(m, c, w64), v);
-    const float s = group16_sum(v * v);
+  if (c < np * 16) {  // a multiple of 16: four neighbouring lanes are there or absent together
+    const T* row = table + (size_t)t * width;
+    float v[4];
+    if ((width & 3) == 0 && ((uintptr_t)table & (4 * sizeof(T) - 1)) == 0) {  // every row starts on a whole vector
+      if (c < width) Tl<T>::ld4(row + c, v);
+      else v[0] = v[1] = v[2] = v[3] = 0.f;
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = c + r < width ? El<T>::ld(row + c + r) : 0.f;
+    }
+    *reinterpret_cast<float4*>(x + (size_t)m * w64 + c) = make_float4(v[0], v[1], v[2], v[3]);
+    Tl<T>::st4(xt + tl_off<T>(m, c, w64), v);
+    float s = (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
+    s += dpp_f<DPP_QUAD_XOR1>(s);
+    s += dpp_f<DPP_QUAD_XOR2>(s);
     if ((c & 15) == 0) ssq[(size_t)m * np + (c >> 4)] = s;
   }
 }
 int launch_lm_embed(int dtype, const int64_t* tokens, const void* table, float* x, void* xt, float* ssq, int rows, int width,
                     int w64, int np, int vocab, hipStream_t st) {
   if (dtype == VUI_DTYPE_F32)
-    hipLaunchKernelGGL(lm_embed_kernel<float>, dim3(rows, (np + 15) / 16), dim3(256), 0, st, tokens, (const float*)table, x, (float*)xt, ssq, width, w64, np, vocab);
+    hipLaunchKernelGGL(lm_embed_kernel<float>, dim3(rows, (np + 63) / 64), dim3(256), 0, st, tokens, (const float*)table, x, (float*)xt, ssq, width, w64, np, vocab);
   else
-    hipLaunchKernelGGL(lm_embed_kernel<bf16_t>, dim3(rows, (np + 15) / 16), dim3(256), 0, st, tokens, (const bf16_t*)table, x, (bf16_t*)xt, ssq, width, w64, np, vocab);
+    hipLaunchKernelGGL(lm_embed_kernel<bf16_t>, dim3(rows, (np + 63) / 64), dim3(256), 0, st, tokens, (const bf16_t*)table, x, (bf16_t*)xt, ssq, width, w64, np, vocab);
   HIP_TRY(hipGetLastError());
   return VUI_OK;
 }

@@ -27,6 +27,10 @@ template <> struct Tl<bf16_t> {
   static __device__ __forceinline__ void st4(bf16_t* p, const float* v) {
     *reinterpret_cast<uint2*>(p) = make_uint2(f2bf2(v[0], v[1]), f2bf2(v[2], v[3]));
   }
+  static __device__ __forceinline__ void ld4(const bf16_t* p, float* v) {  // 8-byte aligned
+    const uint2 q = *reinterpret_cast<const uint2*>(p);
+    v[0] = bf_lo(q.x); v[1] = bf_hi(q.x); v[2] = bf_lo(q.y); v[3] = bf_hi(q.y);
+  }
   static __device__ __forceinline__ void st2(bf16_t* p, float a, float b) { *reinterpret_cast<uint32_t*>(p) = f2bf2(a, b); }
 };
 template <> struct Tl<float> {
@@ -38,6 +42,10 @@ template <> struct Tl<float> {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.w), __uint_as_float(b.w), acc, 0, 0, 0);
   }
   static __device__ __forceinline__ void st4(float* p, const float* v) { *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]); }
+  static __device__ __forceinline__ void ld4(const float* p, float* v) {
+    const float4 q = *reinterpret_cast<const float4*>(p);
+    v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+  }
   static __device__ __forceinline__ void st2(float* p, float a, float b) { *reinterpret_cast<float2*>(p) = make_float2(a, b); }
 };
 
