@@ -491,6 +491,23 @@ def test_large_products_of_a_prompt(large, T):
     assert U.err(whole, ref[:T]) < 0.012 and U.err(whole, parts) < 0.012
 
 
+@pytest.mark.parametrize("T", [640, 700])
+def test_lone_tiles_of_a_prompt(T):
+    """Products of fewer 64 x 64 tiles than compute units, whose K is split over two halves of waves: an odd number of 64 columns in
+    the output projection (13), 640 rows also in the input projection; embedding rows that start on no whole vector.  Bounds as
+    for the large products above."""
+    from vui_amd.synthetic import token_lm_config, token_lm_state_dict
+
+    cfg = token_lm_config(970, 3, 600, 40, 20, 48, 130, 2, vocab=301)
+    sd, toks = token_lm_state_dict(cfg, 5, "cpu"), torch.tensor(U.tokens(T, 301, T))
+    ref = O.forward(cfg, sd, toks.tolist())
+    with U.engine(cfg, sd, BF16, max_seq=704).new_row() as row:
+        whole = row.extend(toks, range(T)).clone()
+        row.reset()
+        parts = torch.cat([row.extend(toks[i:min(i + 100, T)], range(min(100, T - i))).clone() for i in range(0, T, 100)])
+    assert U.err(whole, ref) < 0.012 and U.err(whole, parts) < 0.012
+
+
 @BOTH
 @pytest.mark.parametrize("T", [5, 150])
 def test_gates_far_below_zero(T, dt):

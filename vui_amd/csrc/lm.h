@@ -97,7 +97,7 @@ struct LmGemm {
   const int32_t *ent, *tile_e, *n_tiles;
   int top, max_tiles, tile_rows;
   int sorted;      // X holds a row per entry instead of a row per position
-  int by_xcd;      // lm_wide_kernel: tiles of one feature range on one XCD
+  int band;        // feature tiles of a band (lm_tile_at)
 };
 int launch_lm_gemm(int dtype, int epi, const LmGemm& g, int nz, hipStream_t st);
 int launch_lm_embed(int dtype, const int64_t* tokens, const void* table, float* x, void* xt, float* ssq, int rows, int width,

@@ -157,6 +157,18 @@ __device__ __forceinline__ void lm_unit(const LmGemm& p, const int m, const int 
   }
 }
 
+// Tile of a workgroup.  Workgroups go round the eight XCDs, whose L2s are their own, so each XCD takes a contiguous range of the tiles, in
+// bands of `band` feature tiles with all row tiles: those that run side by side on an XCD share both operands.  In order of dispatch
+// every XCD met nearly all of both, and that, not the steps of a tile, bound the narrow products (650 x 1024 x 4224 on 176 tiles: 22 us
+// with or without a second half of waves; in bands 19).  Whole prompts, us before / after: sakupel 2048 wide x 200 positions 770 / 650,
+// 650 1186 / 1040, 1500 2025 / 1857; mabidra 1024 wide x 900 1216 / 1142, 2048 wide x 1200 2551 / 2419.
+__device__ __forceinline__ void lm_tile_at(int i, int MT, int NT, int band, int& t, int& nt) {
+  const int n = MT * NT, x = i & 7, at = x * (n >> 3) + min(x, n & 7) + (i >> 3);
+  const int b = at / (band * MT), r = at - b * band * MT, w = min(band, NT - b * band);
+  t = r / w;
+  nt = b * band + r - t * w;
+}
+
 template <typename T, int MB, int NB, int WAVES, int EPI>
 __global__ __launch_bounds__(64 * WAVES) void lm_gemm_kernel(const LmGemm p) {
   constexpr bool SCALED = EPI == LM_IN_ATTN || EPI == LM_IN_GRU_STEP || EPI == LM_IN_GRU_SEQ || EPI == LM_LOGITS;
@@ -169,8 +181,15 @@ __global__ __launch_bounds__(64 * WAVES) void lm_gemm_kernel(const LmGemm p) {
   const int l16 = lane & 15, kg = lane >> 4;
   const int MT = MOE ? p.max_tiles : (p.M + 16 * MB - 1) / (16 * MB);
   // tiles of an expert that share features run on one XCD, whose cache then holds those weights: workgroup i is on XCD i % 8
-  const int slice = MOE ? (int)blockIdx.x >> 3 : (int)blockIdx.x, t = slice % MT;
-  const int m0 = t * 16 * MB, nb0 = (MOE ? (slice / MT) * 8 + ((int)blockIdx.x & 7) : slice / MT) * NB;
+  int t, nt;
+  if (MOE) {
+    t = ((int)blockIdx.x >> 3) % MT; nt = ((int)blockIdx.x >> 3) / MT * 8 + ((int)blockIdx.x & 7);
+  } else if (MB == 1) {  // one tile of rows, mostly
+    t = (int)blockIdx.x % MT; nt = (int)blockIdx.x / MT;
+  } else {
+    lm_tile_at(blockIdx.x, MT, ((p.N >> 4) + NB - 1) / NB, p.band, t, nt);
+  }
+  const int m0 = t * 16 * MB, nb0 = nt * NB;
   size_t wz = blockIdx.z * p.wz;
   if (MOE) {
     if (t >= p.n_tiles[0] || nb0 >= (p.N >> 4)) return;  // uniform
@@ -319,18 +338,19 @@ __global__ __launch_bounds__(64 * WAVES) void lm_gemm_kernel(const LmGemm p) {
 }
 
 // ---- many rows, bf16: large tiles through LDS (wide.h) ----
-// Tiles of one feature range follow each other on one XCD where there are enough of them, whose L2 then holds those weights.
-template <int EPI, int MBW, int NBW, int WM, int WN, int S, int KS>
-__global__ __launch_bounds__(256, 2) void lm_wide_kernel(const LmGemm p) {
+// G = 2: eight waves, each half of them with half of K and stages of its own, for tiles that are alone on their CU: a step of
+// such a tile is a chain of barrier, LDS reads and products, and two chains side by side take little longer than one.
+template <int EPI, int MBW, int NBW, int WM, int WN, int S, int KS, int G>
+__global__ __launch_bounds__(256 * G, 2) void lm_wide_kernel(const LmGemm p) {
   constexpr bool SCALED = EPI == LM_IN_ATTN || EPI == LM_IN_GRU_SEQ;
   constexpr bool GRU = EPI == LM_IN_GRU_SEQ, MOE = EPI == LM_MOE_UP || EPI == LM_MOE_DOWN;
   typedef WideTile<MBW, NBW, WM, WN, S, KS> Tile;
   constexpr int MB = Tile::MB, NB = Tile::NB;
   static_assert(!GRU || NBW % 3 == 0, "a recurrence's blocks come in threes");
-  __shared__ __align__(16) char lds[Tile::LDS];
+  __shared__ __align__(16) char lds[Tile::LDS * G];
   __shared__ float srow[MB * 16];
-  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int l16 = lane & 15, kg = lane >> 4, wm = wave % WM, wn = wave / WM;
+  const int tid = threadIdx.x, wave8 = __builtin_amdgcn_readfirstlane(tid >> 6), half = G == 2 ? wave8 >> 2 : 0, wave = wave8 & 3;
+  const int lane = tid & 63, l16 = lane & 15, kg = lane >> 4, wm = wave % WM, wn = wave / WM;
   const bool val = EPI == LM_EXPAND && (int)blockIdx.z >= p.heads;  // values of a head behind the keys of all
   const int head = (int)blockIdx.z - (val ? p.heads : 0);
   const int MBL = (p.M + 15) >> 4, NBL = (val ? p.n_v : p.N) >> 4, MT = MOE ? p.max_tiles : (MBL + MB - 1) / MB, NT = (NBL + NB - 1) / NB;
@@ -345,64 +365,95 @@ __global__ __launch_bounds__(256, 2) void lm_wide_kernel(const LmGemm p) {
     if (t >= p.n_tiles[0]) return;  // uniform
     nt = (((int)blockIdx.x - p.tile_e[t]) & 7) + 8 * (slice % per);
     if (nt >= NT) return;
-  } else if (p.by_xcd) {  // workgroup i is on XCD i % 8
+  } else if (EPI == LM_EXPAND) {
+    t = (int)blockIdx.x % MT; nt = (int)blockIdx.x / MT;
+    if (nt >= NT) return;
+  } else if (MB == 8 && p.band == 0) {  // every eighth feature tile with all rows
     const int slice = (int)blockIdx.x >> 3;
     t = slice % MT; nt = slice / MT * 8 + ((int)blockIdx.x & 7);
     if (nt >= NT) return;
   } else {
-    t = (int)blockIdx.x % MT; nt = (int)blockIdx.x / MT;
-    if (EPI == LM_EXPAND && nt >= NT) return;
+    lm_tile_at(blockIdx.x, MT, NT, p.band, t, nt);
   }
   const int mb0 = t * MB, nb0 = nt * NB, m0 = mb0 * 16;
   const int Q = p.K / (32 * KS);  // steps
   const size_t wz = MOE ? (size_t)p.tile_e[t] * p.wz : head * (val ? p.wz_v : p.wz);
   const char* W = (const char*)(val ? p.w_v : p.W);
 
+  const int n64 = p.K >> 6, mid = G == 2 ? (n64 >> 1) * 2 / KS : 0, first = half * mid, mine = G == 1 ? Q : half ? Q - mid : mid;
   Tile tile;
-  tile.begin(lds, wave, lane,
-             [&](int i) { return (const char*)p.X + (size_t)(MOE ? mb0 + i : min(mb0 + i, MBL - 1)) * Q * (KS * 1024); },
-             [&](int i) { return W + wz * 2 + (size_t)min(nb0 + i, NBL - 1) * Q * (KS * 1024); });
-  tile.prologue(Q);
+  tile.begin(lds + half * Tile::LDS, wave, lane,
+             [&](int i) { return (const char*)p.X + ((size_t)(MOE ? mb0 + i : min(mb0 + i, MBL - 1)) * Q + first) * (KS * 1024); },
+             [&](int i) { return W + wz * 2 + ((size_t)min(nb0 + i, NBL - 1) * Q + first) * (KS * 1024); });
+  tile.prologue(mine);
 
-  if (SCALED) {
+  if (SCALED && half == 0) {
     // 16 lanes add up one row's sums of squares, in a fixed order, the loads of all the wave's rows side by side (one
     // after the other they took longer than the products: 98 against 61 us at 1024 x 11776 x 2048)
-    constexpr int G = MB;  // rows per 16 lanes: 16 MB rows over 16 groups
+    constexpr int NR = MB;  // rows per 16 lanes: 16 MB rows over 16 groups
     const int grp = wave * 4 + kg;
-    float a[G];
+    float a[NR];
 #pragma unroll
-    for (int i = 0; i < G; ++i) a[i] = 0.f;
+    for (int i = 0; i < NR; ++i) a[i] = 0.f;
     if ((p.np & 3) == 0) {
       for (int c = 4 * l16; c < p.np; c += 64) {
-        float4 v[G];
+        float4 v[NR];
 #pragma unroll
-        for (int i = 0; i < G; ++i) v[i] = *reinterpret_cast<const float4*>(p.ssq + (size_t)min(m0 + grp * G + i, p.M - 1) * p.np + c);
+        for (int i = 0; i < NR; ++i) v[i] = *reinterpret_cast<const float4*>(p.ssq + (size_t)min(m0 + grp * NR + i, p.M - 1) * p.np + c);
 #pragma unroll
-        for (int i = 0; i < G; ++i) a[i] += (v[i].x + v[i].y) + (v[i].z + v[i].w);
+        for (int i = 0; i < NR; ++i) a[i] += (v[i].x + v[i].y) + (v[i].z + v[i].w);
       }
     } else {
       for (int c = l16; c < p.np; c += 16) {
-        float v[G];
+        float v[NR];
 #pragma unroll
-        for (int i = 0; i < G; ++i) v[i] = p.ssq[(size_t)min(m0 + grp * G + i, p.M - 1) * p.np + c];
+        for (int i = 0; i < NR; ++i) v[i] = p.ssq[(size_t)min(m0 + grp * NR + i, p.M - 1) * p.np + c];
 #pragma unroll
-        for (int i = 0; i < G; ++i) a[i] += v[i];
+        for (int i = 0; i < NR; ++i) a[i] += v[i];
       }
     }
 #pragma unroll
-    for (int i = 0; i < G; ++i) {
+    for (int i = 0; i < NR; ++i) {
       const float t = group16_sum(a[i]);
-      if (l16 == 0) srow[grp * G + i] = p.norm[0] / sqrtf(t / (float)p.width + p.eps);
+      if (l16 == 0) srow[grp * NR + i] = p.norm[0] / sqrtf(t / (float)p.width + p.eps);
     }
   }
 
   tl_f32x4 acc[NBW][MBW];
-  tile.run(Q, acc);
+  if constexpr (G == 1) {
+    tile.run(Q, acc);
+  } else {  // the quarters are added in the same order
+    static_assert(8 * NBW * MBW * 1024 <= Tile::LDS, "the other half's sums fit its stages");
+    tl_f32x4 last[NBW][MBW];
+    tile.steps(first, mine, Q - mid, n64, 1 + 2 * half, acc, last);
+    __syncthreads();
+    char* other = lds + Tile::LDS + wave * 2 * NBW * MBW * 1024 + lane * 16;
+#pragma unroll
+    for (int i = 0; i < NBW; ++i)
+#pragma unroll
+      for (int j = 0; j < MBW; ++j) {
+        if (half) {
+          *reinterpret_cast<tl_f32x4*>(other + (i * MBW + j) * 1024) = acc[i][j];
+          *reinterpret_cast<tl_f32x4*>(other + (NBW * MBW + i * MBW + j) * 1024) = last[i][j];
+        } else {
+          acc[i][j] += last[i][j];
+        }
+      }
+    __syncthreads();
+    if (half) return;
+#pragma unroll
+    for (int i = 0; i < NBW; ++i)
+#pragma unroll
+      for (int j = 0; j < MBW; ++j) {
+        acc[i][j] += *reinterpret_cast<const tl_f32x4*>(other + (i * MBW + j) * 1024);
+        acc[i][j] += *reinterpret_cast<const tl_f32x4*>(other + (NBW * MBW + i * MBW + j) * 1024);
+      }
+  }
   // The sums pass through this wave's share of LDS, so that the epilogue is a loop: unrolled over the units it is 100 KB of
   // instructions, and fetching those took longer than the products (98 against 61 us at 1024 x 11776 x 2048).
   constexpr int ROOM = S * Tile::PIECES / 4, CH0 = ROOM / MBW < NBW ? ROOM / MBW : NBW, CH = GRU ? CH0 / 3 * 3 : CH0;  // blocks at a time
   static_assert(CH > 0, "a block of sums fits the wave's share");
-  __syncthreads();
+  if (G == 1) __syncthreads();
   char* own = lds + wave * ROOM * 1024 + lane * 16;
 #pragma unroll
   for (int c = 0; c < NBW; c += CH) {
@@ -470,22 +521,36 @@ __global__ __launch_bounds__(256, 2) void lm_wide_kernel(const LmGemm p) {
   }
 }
 
-#define WIDE_BY_XCD 24  // feature tiles from which an XCD's share is taken (with fewer, whole XCDs would have nothing or twice as much to do)
-template <int EPI, int MBW, int NBW, int WM, int WN, int S, int KS>
+// Feature tiles from which an XCD takes every eighth of them with all rows, if a tile has 128 rows (with fewer, whole XCDs would have
+// nothing or twice as much to do; tiles of 64 rows read their operands twice as often, and there what counts is how little the
+// tiles side by side read together).  us, so / in bands: 1999 x 14400 x 2048 (128 x 192) 155 / 165, 1999 x 7744 x 1024 (128 x 128)
+// 55 / 64; 1500 x 2048 x 6144 (64 x 64) 89 / 76.
+#define WIDE_STRIDED 24
+// Feature tiles of a band: the tiles that an XCD runs side by side (two per CU, or its share) as near to a square of the operands as
+// they come.
+static int lm_band(int MT, int NT, int bm, int bn) {
+  const long side = std::min(64L, ((long)MT * NT + 7) / 8);
+  int w = 1;
+  while (w < NT && (long)w * w * bn < side * bm) ++w;
+  return std::max(w, (int)std::min((long)NT, side / MT));  // few rows: all of them side by side
+}
+template <int EPI, int MBW, int NBW, int WM, int WN, int S, int KS, int G = 1>
 static int go_wide(LmGemm g, int nz, hipStream_t st) {
   const int MT = (g.M + 16 * MBW * WM - 1) / (16 * MBW * WM), NT = ((EPI == LM_EXPAND && g.n_v > g.N ? g.n_v : g.N) / 16 + NBW * WN - 1) / (NBW * WN);
   const bool moe = EPI == LM_MOE_UP || EPI == LM_MOE_DOWN;
-  g.by_xcd = !moe && EPI != LM_EXPAND && NT >= WIDE_BY_XCD;
-  const int tiles = moe ? g.max_tiles * ((NT + 7) & ~7) : g.by_xcd ? MT * ((NT + 7) & ~7) : MT * NT;
-  hipLaunchKernelGGL((lm_wide_kernel<EPI, MBW, NBW, WM, WN, S, KS>), dim3((unsigned)tiles, 1, nz), dim3(256), 0, st, g);
+  const bool strided = MBW * WM == 8 && EPI != LM_EXPAND && NT >= WIDE_STRIDED;
+  g.band = strided ? 0 : lm_band(MT, NT, MBW * WM, NBW * WN);
+  const int tiles = moe ? g.max_tiles * ((NT + 7) & ~7) : MT * (strided ? (NT + 7) & ~7 : NT);
+  hipLaunchKernelGGL((lm_wide_kernel<EPI, MBW, NBW, WM, WN, S, KS, G>), dim3((unsigned)tiles, 1, nz), dim3(256 * G), 0, st, g);
   HIP_TRY(hipGetLastError());
   return VUI_OK;
 }
 
 template <typename T, int MB, int NB, int WAVES, int EPI>
-static int go(const LmGemm& g, int nz, hipStream_t st) {
+static int go(LmGemm g, int nz, hipStream_t st) {
   const bool moe = EPI == LM_MOE_UP || EPI == LM_MOE_DOWN;
   const int nt = (g.N / 16 + NB - 1) / NB;
+  g.band = lm_band((g.M + 16 * MB - 1) / (16 * MB), nt, MB, NB);
   const int tiles = moe ? g.max_tiles * ((nt + 7) & ~7) : (g.M + 16 * MB - 1) / (16 * MB) * nt;
   hipLaunchKernelGGL((lm_gemm_kernel<T, MB, NB, WAVES, EPI>), dim3((unsigned)tiles, 1, nz), dim3(64 * WAVES), 0, st, g);
   HIP_TRY(hipGetLastError());
@@ -497,20 +562,32 @@ static int go(const LmGemm& g, int nz, hipStream_t st) {
 // 1033 / 869 / 865 / 870 and of 1024 x 900 760 / 701 / 691 / 697, x 500 487 / 487 / 497 / 553; experts of 2048 x 300
 // 1463 / 1404 / 1311 / 1320.
 static int lm_tile(int epi, int M, int N, int K) {
-  if (epi != LM_IN_GRU_SEQ) return wide_pick(M, N, K, 1.5);
+  if (epi != LM_IN_GRU_SEQ) {
+    // Tiles that are alone on their CU split K over two halves of waves.  Whole prompts, us, without / with (the same order of tiles):
+    // sakupel 1024 wide x 900 positions 722 / 690, 2048 wide x 333 833 / 805; mabidra 2048 wide x 333 1371 / 1340.
+    const int t = wide_pick(M, N, K, 1.5);
+    const long MT = (M + 63) / 64;
+    if (t == WIDE_64 && K >= 512 && MT * ((N + 63) / 64) <= 256) return WIDE_64_2;
+    if (t == WIDE_64x128 && K >= 512 && MT * ((N + 127) / 128) <= 256) return WIDE_64x128_2;
+    return t;
+  }
   // A minGRU projection takes 128 x 192, whose tiles fill an XCD 64 at a time, or the K-splitting form, which is bound by the
   // weights' way to the chip and by its tiles.  us, K-splitting / large tile (50 products of 130 ... 2048
   // rows, the quicker form is taken in 49): 900 x 6400 x 768 27.6 / 30.0, 1200 32.1 / 31.1, 1600 39.7 / 46.5; 640 x 8704 x 1024 33.1 / 31.9; 300 x 11776 x 1024
   // 33.7 / 31.4, 1200 79 / 64; 130 x 14336 x 2048 51 / 44, 1024 154 / 93.
   if (M < 128) return WIDE_NONE;
   const long MT = (M + 127) / 128, NT = (N + 191) / 192;
-  const long fills = NT >= WIDE_BY_XCD ? ((NT + 7) / 8 * MT + 63) / 64 : (NT * MT + 511) / 512;
+  const long fills = NT >= WIDE_STRIDED ? ((NT + 7) / 8 * MT + 63) / 64 : (NT * MT + 511) / 512;
   const double split = 4 + 1e-6 * N * K + 0.26e-3 * ((M + 31) / 32) * ((N + 31) / 32) * (K / 64);
   return 6 + fills * (10 + 0.56 * (K / 32)) < split ? WIDE_128 : WIDE_NONE;
 }
 template <int EPI>
 static int pick_wide(int tile, const LmGemm& g, hipStream_t st) {
   const int nz = EPI == LM_EXPAND ? 2 * g.heads : 1;
+  if constexpr (EPI != LM_EXPAND) {
+    if (tile == WIDE_64x128_2) return go_wide<EPI, 4, 2, 1, 4, 3, 2, 2>(g, nz, st);
+    if (tile == WIDE_64_2) return go_wide<EPI, 2, 2, 2, 2, 4, 2, 2>(g, nz, st);
+  }
   switch (tile) {
     case WIDE_128: return go_wide<EPI, 4, 4, 2, 2, 4, 1>(g, nz, st);
     case WIDE_64x128: return go_wide<EPI, 4, 2, 1, 4, 3, 2>(g, nz, st);
@@ -571,7 +648,9 @@ int launch_lm_gemm(int dtype, int epi, const LmGemm& g, int nz, hipStream_t st) 
   if (epi == LM_EXPAND) {
     if (dtype != VUI_DTYPE_BF16 || g.heads < 1 || g.n_v < 16 || (g.n_v & 15)) { vui_set_error("lm gemm: bad expansion"); return VUI_EINVAL; }
     // XXX
-    return pick_wide<LM_EXPAND>(wide_pick(g.M, g.heads * (g.N + g.n_v), g.K, 1e9), g, st);
+    // the largest tile that gives every CU two workgroups (16 heads of 128 + 128, rank 512, 1999 positions: 18 us, with 64 x 128 24)
+    auto tiles = [&](int bm, int bn) { return (long)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn + (g.n_v + bn - 1) / bn) * g.heads; };
+    return pick_wide<LM_EXPAND>(g.N > 64 && tiles(128, 128) >= 512 ? WIDE_128 : g.N > 64 && tiles(64, 128) >= 512 ? WIDE_64x128 : WIDE_64, g, st);
   }
   const bool gru = epi == LM_IN_GRU_STEP || epi == LM_IN_GRU_SEQ;
   if ((gru && ((g.mix_blocks % 3) || (g.N / 16) % 3)) || (epi == LM_IN_ATTN && (g.mix_blocks % 2))) {
@@ -585,8 +664,9 @@ int launch_lm_gemm(int dtype, int epi, const LmGemm& g, int nz, hipStream_t st) 
 // ---- embedding rows: residual, operand copy, sums of squares per 16 columns ----
 template <typename T>
 __global__ __launch_bounds__(256) void lm_embed_kernel(const int64_t* tokens, const T* table, float* x, T* xt, float* ssq,
-                                                       int width, int w64, int np, int vocab) {
-  const int m = blockIdx.x, c = (blockIdx.y * 256 + threadIdx.x) * 4;  // four columns per lane
+                                                       int width, int w64, int np, int vocab, int rows) {
+  const int m = blockIdx.x * 16 + (threadIdx.x >> 4), c = blockIdx.y * 64 + (threadIdx.x & 15) * 4;  // a block of the operand's layout
+  if (m >= rows) return;
   int64_t t = tokens[m];
   t = t < 0 ? 0 : (t >= vocab ? vocab - 1 : t);
   if (c < np * 16) {  // a multiple of 16: four neighbouring lanes are there or absent together
@@ -610,9 +690,9 @@ __global__ __launch_bounds__(256) void lm_embed_kernel(const int64_t* tokens, co
 int launch_lm_embed(int dtype, const int64_t* tokens, const void* table, float* x, void* xt, float* ssq, int rows, int width,
                     int w64, int np, int vocab, hipStream_t st) {
   if (dtype == VUI_DTYPE_F32)
-    hipLaunchKernelGGL(lm_embed_kernel<float>, dim3(rows, (np + 63) / 64), dim3(256), 0, st, tokens, (const float*)table, x, (float*)xt, ssq, width, w64, np, vocab);
+    hipLaunchKernelGGL(lm_embed_kernel<float>, dim3((rows + 15) / 16, (np + 3) / 4), dim3(256), 0, st, tokens, (const float*)table, x, (float*)xt, ssq, width, w64, np, vocab, rows);
   else
-    hipLaunchKernelGGL(lm_embed_kernel<bf16_t>, dim3(rows, (np + 63) / 64), dim3(256), 0, st, tokens, (const bf16_t*)table, x, (bf16_t*)xt, ssq, width, w64, np, vocab);
+    hipLaunchKernelGGL(lm_embed_kernel<bf16_t>, dim3((rows + 15) / 16, (np + 3) / 4), dim3(256), 0, st, tokens, (const bf16_t*)table, x, (bf16_t*)xt, ssq, width, w64, np, vocab, rows);
   HIP_TRY(hipGetLastError());
   return VUI_OK;
 }

@@ -71,15 +71,23 @@ struct WideTile {
   // The sums of a quarter of K each (in whole 64 columns) are added in order, as the waves of a K-splitting workgroup leave
   // them, so that a chain of fp32 sums is no longer than there and both forms give the same bits.
   __device__ __forceinline__ void run(int Q, tl_f32x4 (&sum)[NBW][MBW]) {
+    tl_f32x4 acc[NBW][MBW];
+    steps(0, Q, Q, Q * KS / 2, 1, sum, acc);
+#pragma unroll
+    for (int i = 0; i < NBW; ++i)
+#pragma unroll
+      for (int j = 0; j < MBW; ++j) sum[i][j] += acc[i][j];
+  }
+  // Steps first ... first + Q - 1 of K = 64 n64 columns, which begin with quarter `part` - 1: `acc` is left with the sums of the last
+  // quarter, `sum` with those before it.  All waves of the workgroup meet `rounds` >= Q times.
+  __device__ __forceinline__ void steps(int first, int Q, int rounds, int n64, int part, tl_f32x4 (&sum)[NBW][MBW], tl_f32x4 (&acc)[NBW][MBW]) {
     const int wm = wave % WM, wn = wave / WM;
     const tl_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    tl_f32x4 acc[NBW][MBW];
 #pragma unroll
     for (int i = 0; i < NBW; ++i)
 #pragma unroll
       for (int j = 0; j < MBW; ++j) acc[i][j] = sum[i][j] = zero;
-    const int n64 = Q * KS / 2;
-    int slot = 0, part = 1, end = (n64 >> 2) * 2 / KS;  // the first step behind this quarter
+    int slot = 0, end = (n64 * part >> 2) * 2 / KS - first;  // the first step behind this quarter
     for (int q = 0; q < Q; ++q) {
       // the oldest stage has landed once no more than the stages behind it are outstanding, for every wave behind the
       // barrier; the fragments read from the slot that is filled next have arrived as well
@@ -112,7 +120,7 @@ struct WideTile {
         for (int i = 0; i < NBW; ++i)
 #pragma unroll
           for (int j = 0; j < MBW; ++j) { sum[i][j] += acc[i][j]; acc[i][j] = zero; }
-        do end = (n64 * ++part >> 2) * 2 / KS;
+        do end = (n64 * ++part >> 2) * 2 / KS - first;
         while (end == q);
       }
 #pragma unroll
@@ -123,10 +131,7 @@ struct WideTile {
           for (int j = 0; j < MBW; ++j) acc[i][j] = Tl<bf16_t>::mma(wa[k][i], xa[k][j], acc[i][j]);
       slot = slot == S - 1 ? 0 : slot + 1;
     }
-#pragma unroll
-    for (int i = 0; i < NBW; ++i)
-#pragma unroll
-      for (int j = 0; j < MBW; ++j) sum[i][j] += acc[i][j];
+    for (int q = Q; q < rounds; ++q) __builtin_amdgcn_s_barrier();
   }
 };
 
@@ -136,7 +141,7 @@ struct WideTile {
 // when it has.  Measured (us, K-splitting with its epilogue / quickest large tile without): 1024 x 11776 x 2048 147 / 63,
 // 1024 x 2048 x 6144 82 / 40, 1024 x 5120 x 768 26 / 18, 1024 x 768 x 2816 16 / 14, 300 x 768 x 2816 9 / 14.  The prompt pass of the
 // backbone has estimates of its own.
-enum { WIDE_NONE = -1, WIDE_128 = 0, WIDE_64x128 = 1, WIDE_64 = 2 };
+enum { WIDE_NONE = -1, WIDE_128 = 0, WIDE_64x128 = 1, WIDE_64 = 2, WIDE_64x128_2 = 3, WIDE_64_2 = 4 };
 static inline int wide_pick(int M, int N, int K, double keep) {
   static const struct { int bm, bn; double wait, work; } tile[] = {{128, 128, 0.335, 0.144}, {64, 128, 0.21, 0.08}, {64, 64, 0.17, 0.059}};
   int best = WIDE_NONE;
