@@ -21,7 +21,7 @@
 //
 // Several frames at once (vui_codec_decode_block: offline calls, the seeding of a stream): the same steps over
 // frames x columns, on buffers that hold a whole block with the histories in front; wide products run in
-// cv_wide_kernel.  93 frames: 56.6 ms one after the other, 6.3 ms in blocks of 32 (MI355X).
+// cv_wide_kernel.  93 frames: 56.6 ms one after the other, 5.9 ms in blocks of 32 (MI355X).
 #include "common.h"
 #include "internal.h"
 #include "../../include/vui_codec.h"
@@ -201,16 +201,26 @@ __device__ __forceinline__ void cv_gemm_tile(const CvGemm& p, const int m0, cons
   if (p.in_mode == IN_RMS && p.T > 1) {  // a column per frame: 4 threads of every wave share one
     constexpr int SH = 4 * NW;
     __shared__ float sq[TT * 16 * SH];
+    // sixteen loads in flight per column: as a plain loop this was most of the launch (32 frames, 3072 x 512 14.2 -> 9.1 us, 2048 x 512
+    // 13.8 -> 8.4)
+    float ss[TT];
 #pragma unroll
-    for (int tt = 0; tt < TT; ++tt) {
-      const int t = min(t0 + tt * 16 + (tid & 15), p.T - 1);
-      float ss = 0.f;
-      for (int c = tid >> 4; c < Cin; c += SH) {
-        const float v = *ring_ptr(p.in, ib_, c, p.in.pad + t);
-        ss = fmaf(v, v, ss);
-      }
-      sq[(tt * 16 + (tid & 15)) * SH + (tid >> 4)] = ss;
+    for (int tt = 0; tt < TT; ++tt) ss[tt] = 0.f;
+    for (int c0 = tid >> 4; c0 < Cin; c0 += 16 * SH) {
+      float v[TT][16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt)
+          v[tt][i] = *ring_ptr(p.in, ib_, min(c0 + i * SH, Cin - 1), p.in.pad + min(t0 + tt * 16 + (tid & 15), p.T - 1));
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt)
+          if (c0 + i * SH < Cin) ss[tt] = fmaf(v[tt][i], v[tt][i], ss[tt]);
     }
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt) sq[(tt * 16 + (tid & 15)) * SH + (tid >> 4)] = ss[tt];
     __syncthreads();
     if (tid < TT * 64) {
       float ss = 0.f;
@@ -1521,6 +1531,8 @@ static CvScratch cv_plan(CvGemm& g) {
     if (sp > U / 16) sp = U / 16;
     if (sp > 8) sp = 8;
     if (sp < 1) sp = 1;
+  } else if (g.nf > 1 && g.tt > 1 && U >= 32 && tiles(g.tt) <= 100) {
+    sp = 2;  // few tiles of several frames: each streams its rows' weights alone (trunk of 32 frames, 512 x 1024: 11.2 -> 9 us)
   }
   g.splits = sp;
   return CvScratch{(size_t)tiles(g.tt) * sp * g.tt * 256, (size_t)tiles(g.tt)};
