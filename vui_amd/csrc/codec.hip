@@ -1488,6 +1488,7 @@ struct CvScratch { size_t part, cnt; };  // floats of partial sums, arrival coun
 struct WideTile { int bm, bn; float unit; };
 #define CVW_PAIR 2.6   // us of a unit of 128 x 128 for two workgroups of a CU, and for one
 #define CVW_ALONE 1.6
+#define CVW_PARTS (6u << 20)  // floats of the parts of a split product, which the workspace holds
 static const WideTile kWide[] = {{128, 128, 1.0f}, {96, 128, 0.79f}, {64, 128, 0.63f}, {128, 64, 0.63f}, {32, 128, 0.55f}};
 
 // Chooses tile width, splits and kernel for g.T columns.
@@ -1501,7 +1502,7 @@ static CvScratch cv_plan(CvGemm& g) {
       const WideTile& w = kWide[i];
       if (M % w.bm) continue;
       const int cols = (T + w.bn - 1) / w.bn * w.bn, tiles = (M / w.bm) * (cols / w.bn);
-      for (int sp = 1; sp <= 16 && (sp == 1 || U / sp >= 4); ++sp) {
+      for (int sp = 1; sp <= 16 && (sp == 1 || (U / sp >= 4 && (size_t)sp * M * cols <= CVW_PARTS)); ++sp) {
         const int wgs = (tiles * sp + 255) / 256;
         const double c = (wgs / 2 * CVW_PAIR + wgs % 2 * CVW_ALONE) * ((U + sp - 1) / sp) * w.unit + (sp > 1 ? 6 + 1e-6 * sp * M * T : 0);
         if (cost && c >= cost) continue;
