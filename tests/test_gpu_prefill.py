@@ -259,3 +259,44 @@ def test_short_blocks_behind_a_cache(heads, kv, window):
             if pos == 0:  # the cache the other offsets stand on
                 seq.fill_(0)
                 m.decoder.forward_flash(x, None)
+
+
+@pytest.mark.parametrize("window,every", [(128, 3), (300, 2), (300, 4), (40, 2)])
+def test_short_blocks_of_layers_with_and_without_a_window(window, every):
+    """Windowed and global layers in one model, behind caches where the ranges of keys that a layer's attention is dealt in are
+    unequal in number (1 to 3 with the window, 2 to 8 without): outputs and every layer's appended keys and values, each position
+    against the decode step behind the same cache, and the same bits in a second pass.  Two evaluations in bf16 move apart by 0.007
+    of a position's norm per layer where all layers are of one kind (five layers: 0.036); the limit is 2^-6 per layer.  Attention is
+    sharp with these weights (logits of tens), so a range that is left out moves a position by its own size."""
+    from tests.util import dims_to_config
+    from vui_amd.model import Vui
+
+    L = 5
+    d = O.Dims(d_model=256, n_layers=L, n_heads=4, n_kv_heads=2, n_quantizers=4, codebook_size=32, rq_d_model=64, rq_n_layers=1,
+               rq_n_heads=2, vocab_size=50, max_seqlen=1280, window_size=window, global_every=every)
+    m = Vui(dims_to_config(d, 1280), O.synthetic_state_dict(d, **TINY_SD), device="cuda", dtype=BF)
+    dec = m.decoder
+    assert len(set(dec.block_is_global)) == 2
+    dec.allocate_flash_kv_cache(1, m.device, BF)
+    seq = dec.flash_kv_caches[0].seq_lens
+    x = (torch.randn(1, 1200, d.d_model, generator=torch.Generator().manual_seed(9)) * 0.5).to(BF).cuda()
+    dec.forward_flash(x, None)
+
+    def block(pos, T, minimum):
+        seq.fill_(pos)
+        dec.PREFILL_MIN = minimum
+        h = dec.forward_flash(x[:, :T], None)
+        # keys and values (L, T, features), outputs (1, T, features)
+        return [t[:, 0, pos:pos + T].flatten(2).float() for t in (dec._k, dec._v)] + [h.float()]
+
+    for pos in (200, 300, 640, 1130):
+        for T in (4, 16, 33, 64):
+            got, again, want = block(pos, T, 1), block(pos, T, 1), block(pos, T, 10 ** 9)
+            for a, b, c in zip(got, again, want):
+                assert torch.equal(a, b), (pos, T)
+                off = ((a - c).norm(dim=-1) / c.norm(dim=-1)).amax(1)  # the worst position
+                for l, e in enumerate(off.tolist(), 1 if len(off) == L else L):
+                    assert e <= l * 2.0 ** -6, (pos, T, l, e)
+            seq.fill_(pos)
+            dec.PREFILL_MIN = 4
+            dec.forward_flash(x[:, pos:pos + T], None)  # the cache that later positions stand on

@@ -652,7 +652,7 @@ struct PfDirectArgs {
   int T, nq, nkv, gsz, pos0, window;
   float scale;
   float *part, *ml;  // (head, tile, split): sums (DT x 64 lanes x 4), {max, sum of weights} x 16
-  uint32_t* count;   // arrivals of a (head, tile): a multiple of the splits before the launch
+  uint32_t* count;   // arrivals of a (head, tile), zero between launches: layers with a window have fewer splits than those without
 };
 typedef short pf_s16x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ uint2 pf_read_tr(const char* lds) {
@@ -777,8 +777,11 @@ __global__ __launch_bounds__(64 * PfDirect<HD32>::WAVES) void pf_direct_attn_ker
     if (tid < 16) st_dev(ml + sp * 32 + tid * 2, M, den);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (tid == 0)
-      *s_last = (__hip_atomic_fetch_add(a.count + set, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1) % nsp == 0;
+    if (tid == 0) {
+      const bool last = __hip_atomic_fetch_add(a.count + set, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)nsp - 1;
+      if (last) __hip_atomic_store(a.count + set, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      *s_last = last;
+    }
     __syncthreads();
     if (!*s_last) return;
     uint64_t xm[PF_SPLITS], xo[ND][PF_SPLITS][2];
