@@ -264,18 +264,43 @@ def test_full_dims_blocks_equal_single_frames(full):
         assert err(got, one.cpu()) < 5e-5  # measured 1e-5
 
 
-@pytest.mark.parametrize("power", [-60, -20, 20, 60])
-def test_wide_products_of_any_magnitude(full, power):
-    """Parts of an operand keep its exponent: a layer's weights times a power of two and its scale by the inverse give the same audio,
-    bit by bit, from blocks of frames (power-of-two factors pass through every sum of the three parts)."""
-    d, sd, dec, fx = full
+def scaled(sd, power):
+    """The last product of both upsampling blocks' feed-forwards times a power of two, its scale by the inverse."""
     other = dict(sd)
     for i in range(2):
         for k in ("pwconv2.weight", "pwconv2.bias"):
             other[f"upsample.{i}.1.{k}"] = sd[f"upsample.{i}.1.{k}"] * 2.0 ** power
         other[f"upsample.{i}.1.gamma"] = sd[f"upsample.{i}.1.gamma"] * 2.0 ** -power
+    return other
+
+
+@pytest.mark.parametrize("power", [-104, -60, -20, 20, 60, 120])
+def test_wide_products_of_any_magnitude(full, power):
+    """Parts of an operand keep its exponent: scaled weights give the same audio from blocks of frames, bit by bit as long as the least
+    products are above fp32's least normal number (power-of-two factors pass through every sum of the three parts).  Weights of 2^-110
+    keep their three parts; the products' last bits are subnormal (the limit: other orders of the sums differ by 1e-5)."""
+    d, sd, dec, fx = full
     codes = torch.randint(0, d.codebook_size, (1, d.n_codebooks, 35), generator=torch.Generator().manual_seed(9)).cuda()
-    assert torch.equal(native(d, other)(codes), dec(codes))
+    got, want = native(d, scaled(sd, power))(codes), dec(codes)
+    assert err(got, want.cpu()) < 5e-5 if power < -90 else torch.equal(got, want)
+
+
+def test_wide_products_near_the_largest_number(full):
+    """Weights between bf16's largest number and fp32's (1.998 and -1.9999 x 2^127) are finite and count as what they are."""
+    d, sd, dec, fx = full
+    sd = dict(sd)
+    for i in range(2):
+        for k in ("pwconv1.weight", "pwconv1.bias"):  # small hidden values: no product reaches infinity
+            sd[f"upsample.{i}.1.{k}"] = sd[f"upsample.{i}.1.{k}"] * 2.0 ** -6
+        sd[f"upsample.{i}.1.gamma"] = sd[f"upsample.{i}.1.gamma"] * 16  # ... and 2^-127 of it is normal
+        w = sd[f"upsample.{i}.1.pwconv2.weight"].clone()
+        w[::3, ::7], w[1::3, 1::5] = 1.998, -1.9999
+        sd[f"upsample.{i}.1.pwconv2.weight"] = w
+    codes = torch.randint(0, d.codebook_size, (1, d.n_codebooks, 35), generator=torch.Generator().manual_seed(9)).cuda()
+    want, big = native(d, sd)(codes), scaled(sd, 127)
+    assert float(big["upsample.0.1.pwconv2.weight"].abs().max()) > float(torch.finfo(torch.bfloat16).max)
+    got = native(d, big)(codes)
+    assert err(got, want.cpu()) < 5e-5  # measured 1e-5: the parts of the planted weights are others
 
 
 @pytest.mark.parametrize("d_model", [1024, 1312, 2048])

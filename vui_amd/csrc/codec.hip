@@ -339,13 +339,17 @@ __global__ __launch_bounds__(NW * 64, 2) void cv_gemm1_kernel(const CvGemm p) {
 }
 
 // ---- the same product for many columns (several frames at once) ----
-// On the bf16 matrix instructions, which are 16 times the rate of the fp32 ones (157 TFLOP/s): every fp32 operand is the exact sum of three
+// On the bf16 matrix instructions, which are 16 times the rate of the fp32 ones (157 TFLOP/s): every fp32 operand is the sum of three
 // bf16 numbers (8 bits each, nearest, so that the rest halves once more), and of their nine products the six that
-// reach 2^-24 of the value are summed in fp32, small ones first.  What is left out is 2^-26 of a product; the sums have
+// reach 2^-24 of the value are summed in fp32, small ones first (G. Henry, P. T. P. Tang, A. Heinecke, "Leveraging the bfloat16
+// Artificial Intelligence Datatype for Higher-Precision Computations", ARITH 2019).  What is left out is 2^-26 of a product; the sums have
 // fewer roundings than with v_mfma_f32_32x32x2_f32 (sixteen products per step instead of two).
+// The sum is exact for every finite value from 2^-110 up.  Of a smaller one, what lies below bf16's least subnormal, 2^-133, is lost
+// (weights of 2^-118: error of the product 1.4e-5, 2^-122: 2e-4; with fp32 instructions 2e-6).  A value that is not finite makes its
+// columns or rows NaN, an infinite one too.
 // 32 frames: 7-tap convolutions of 768 / 384 / 192 / 96 channels 86 / 105 / 121 / 91 us -> 55 / 63 / 83 / 62 (1200 TFLOP/s
 // of bf16 products in the first, what hipBLASLt reaches at 8192^3), 1x1 19 / 30 / 32 / 33 -> 16 / 29 / 26 / 29; error of 93
-// frames against 64 bits 4.1e-6 -> 3.9e-6.  An input that is not finite makes its columns NaN.
+// frames against 64 bits 4.1e-6 -> 3.9e-6.
 // Tiles of BM x BN = 128 x 128 (or what divides M) of four waves through LDS, three planes of each operand: a K step is one (tap,
 // 32-channel) unit, fetched into registers while the one before it is multiplied, split on the way to LDS.  One buffer: two
 // workgroups of a CU overlap better than the steps of one (eight waves with two buffers and one to three units in flight: 75 us of
@@ -359,9 +363,11 @@ typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 cv_bf16x8;
 // reads of eight rows fall on different banks.
 __device__ __forceinline__ int cv_at(int row, int piece) { return row * 32 + 8 * (piece ^ (row >> 2 & 3)); }
 
-// two fp32 values -> their three bf16 parts, packed
+// two fp32 values -> their three bf16 parts, packed.  The first part of a value above bf16's largest (3.39e38) is that largest: to the
+// nearest it would be infinity, and the column NaN.  That costs 93 frames 0.9 %.
 __device__ __forceinline__ void cv_split2(float a, float b, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
-  hi = f2bf2(a, b);
+  const float top = __uint_as_float(0x7f7f0000u);
+  hi = f2bf2(__builtin_amdgcn_fmed3f(a, -top, top), __builtin_amdgcn_fmed3f(b, -top, top));
   a -= bf_lo(hi); b -= bf_hi(hi);
   mid = f2bf2(a, b);
   lo = f2bf2(a - bf_lo(mid), b - bf_hi(mid));
