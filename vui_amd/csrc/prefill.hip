@@ -43,7 +43,7 @@ struct PfGemm {
   float* ssq_out;    // PF_RESID: the same sums of the new residual, or nullptr
   // PF_QKV: C receives the rotated queries alone; row m is position pos0 + m of the slot
   bf16_t *kc, *vc;   // its cache rows
-  bf16_t *kt, *vt;   // operand copies of keys and transposed values (pf_stage_kv_kernel), or nullptr
+  bf16_t *kt, *vt;   // operand copies of keys and transposed values (pf_stage_kv_kernel); nullptr unless the slot is empty (pos0 == 0)
   const float* rope;
   int nq, nkv, hd, rope_dim, pos0, Lpad;
   // pf_order: tiles of an XCD (the first xcd_more have one more), tiles of one step of the slower index
@@ -117,8 +117,8 @@ __device__ __forceinline__ void pf_qkv_out(const PfGemm& p, const PfPart& b, int
   } else if (b.part == 1) {
     *reinterpret_cast<uint2*>(p.kc + (size_t)j * p.nkv + col) = w;
     if (p.kt) {
-      const size_t blk = ((size_t)b.head * (p.Lpad >> 4) + (j >> 4)) * (p.hd >> 5) + (dd >> 5);
-      *reinterpret_cast<uint2*>(p.kt + blk * 512 + ((j & 15) + 16 * ((dd & 31) >> 3)) * 8 + (dd & 7)) = w;
+      const size_t blk = ((size_t)b.head * (p.Lpad >> 4) + (m >> 4)) * (p.hd >> 5) + (dd >> 5);
+      *reinterpret_cast<uint2*>(p.kt + blk * 512 + ((m & 15) + 16 * ((dd & 31) >> 3)) * 8 + (dd & 7)) = w;
     }
   } else {
     *reinterpret_cast<uint2*>(p.vc + (size_t)j * p.nkv + col) = w;
@@ -127,10 +127,9 @@ __device__ __forceinline__ void pf_qkv_out(const PfGemm& p, const PfPart& b, int
 // The values of feature l16 of such a block in rows m .. m + 3 (m % 4 == 0), into the transposed layout
 __device__ __forceinline__ void pf_vt_out(const PfGemm& p, const PfPart& b, int m, int l16, const float* v) {
   const size_t blk0 = ((size_t)b.head * (p.hd >> 4) + (b.dim >> 4)) * (p.Lpad >> 5);
-  auto at = [&](int j) { return p.vt + (blk0 + (j >> 5)) * 512 + (l16 + 16 * ((j & 15) >> 2)) * 8 + 4 * ((j & 31) >> 4) + (j & 3); };
-  const int j = p.pos0 + m;
-  if (!(p.pos0 & 3) && m + 3 < p.M) { *reinterpret_cast<uint2*>(at(j)) = make_uint2(f2bf2(v[0], v[1]), f2bf2(v[2], v[3])); return; }
-  for (int r = 0; r < 4; ++r) if (m + r < p.M) *at(j + r) = f2bf(v[r]);
+  bf16_t* dst = p.vt + (blk0 + (m >> 5)) * 512 + (l16 + 16 * ((m & 15) >> 2)) * 8 + 4 * ((m & 31) >> 4);
+  if (m + 3 < p.M) { *reinterpret_cast<uint2*>(dst) = make_uint2(f2bf2(v[0], v[1]), f2bf2(v[2], v[3])); return; }
+  for (int r = 0; r < 4; ++r) if (m + r < p.M) dst[r] = f2bf(v[r]);
 }
 
 // row-major (N x K) -> tiled; one 8-element piece per thread
@@ -297,7 +296,7 @@ __global__ __launch_bounds__(64 * WAVES) void pf_gemm_kernel(const PfGemm p, con
     }
   }
   const bool out = m < p.M && n < p.N;  // N is a multiple of 16
-  if (EPI == PF_QKV && p.vt && n0 + 16 * i >= p.nq + p.nkv && n0 + 16 * i < p.N) {
+  if (EPI == PF_QKV && !NORM && p.vt && n0 + 16 * i >= p.nq + p.nkv && n0 + 16 * i < p.N) {
     // the tile transposed: feature l16 of rows 4 kg .. 4 kg + 3
     float t[4];
 #pragma unroll
