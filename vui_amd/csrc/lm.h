@@ -189,7 +189,7 @@ struct RowArgs {
   float* rlog;             // (M, experts16)
   RouteArgs route;         // rows are routed as well
   uint32_t* arrived;       // rows that have made their choices, zero between launches
-  // the first launch of a pass clears the arrival counters (a workspace comes as it is)
+  // the first launch of a pass clears the arrival counters that its rows use (a workspace comes as it is)
   uint32_t* clear;
   int n_clear;
 };
@@ -276,8 +276,8 @@ struct vui_lm_ctx {
   void *xcat, *raw, *ffa, *xg;
   float *y, *bsum, *gupd, *gdec, *rlog, *share;
   int32_t *choice, *ent, *tile_e, *n_tiles;
-  uint32_t* arrived;  // attention pieces of each row's blocks of heads, then rows routed
-  int n_arrived;
+  uint32_t* arrived;  // rows routed, then attention pieces of each row's blocks of heads
+  int arrived_row;    // blocks of heads of a row, at most
   int attn_from, gla_from;
 };
 static inline int lm_pad(int v, int a) { return (v + a - 1) / a * a; }

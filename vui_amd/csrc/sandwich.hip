@@ -73,7 +73,7 @@ size_t sandwich_carve(const vui_lm_config* c, const vui_lm_layer* layers, vui_lm
       size_t rows = R;  // rows x splits of attention pieces
       for (int M = 1; M <= (int)R && M <= 1024; ++M) mx(rows, (size_t)M * sig_splits(M, L.heads, L.kv_heads));
       mx(pt, rows * H * d.vdim16);
-      mx(ar, R * L.kv_heads * ((H / L.kv_heads + 15) / 16));
+      mx(ar, L.kv_heads * ((H / L.kv_heads + 15) / 16));
     }
     if (L.experts > 0) {
       const size_t n = R * L.top;
@@ -109,8 +109,8 @@ size_t sandwich_carve(const vui_lm_config* c, const vui_lm_layer* layers, vui_lm
   TAKE(ent, int32_t*, en * 4);
   TAKE(tile_e, int32_t*, ti * 4);
   TAKE(n_tiles, int32_t*, 4);
-  TAKE(arrived, uint32_t*, (ar + 1) * 4);
-  if (x) x->n_arrived = (int)ar + 1;
+  TAKE(arrived, uint32_t*, (1 + R * ar) * 4);
+  if (x) x->arrived_row = (int)ar;
 #undef TAKE
   return off;
 }
@@ -151,7 +151,7 @@ static int mixer(vui_lm_ctx* x, int l, int M, const LmRows& rows, hipStream_t st
     a.scale = L.scale; a.eps = x->c.norm_eps; a.rows = rows; a.d = d; a.raw = x->raw; a.ld = d.in_rows;
     a.q_norm = L.q_norm; a.k_norm = L.k_norm; a.temp_coef = L.temp_coef; a.temp_every = L.temp_every < 1 ? 1 : L.temp_every;
     a.bias = L.dist_bias; a.bias_len = L.bias_len; a.k_cache = L.k_cache; a.v_cache = L.v_cache;
-    a.q = x->qu; a.q_z = (size_t)x->R16 * d.dim64; a.part = x->part; a.arrived = x->arrived; a.act = x->act;
+    a.q = x->qu; a.q_z = (size_t)x->R16 * d.dim64; a.part = x->part; a.arrived = x->arrived + 1; a.act = x->act;
     if (!sig_step_fused(x->c.dtype, rows, d) && (rc = launch_sig_prep(a, st))) return rc;
     if (rows.seq && M >= x->attn_from && x->c.dtype == VUI_DTYPE_BF16 && sig_mfma_ok(d)) {
       rc = launch_sig_prompt(a, st);
@@ -220,7 +220,7 @@ int sandwich_layers(vui_lm_ctx* x, const int64_t* tokens, int M, const LmRows& r
   };
   ahead(0);
   RowArgs emb = r;
-  emb.tokens = tokens; emb.clear = x->arrived; emb.n_clear = x->n_arrived;
+  emb.tokens = tokens; emb.clear = x->arrived; emb.n_clear = 1 + M * x->arrived_row;
   int rc = launch_lm_rows(emb, st);
   for (int l = 0; l < n && !rc; ++l) {
     const vui_lm_layer& L = x->layers[l];
@@ -239,7 +239,7 @@ int sandwich_layers(vui_lm_ctx* x, const int64_t* tokens, int M, const LmRows& r
       RowArgs mid = r;
       if (L.experts > 0 && lm_rows_routes(M, d.experts16)) {
         mid.w_router = L.w_router; mid.router_bias = L.router_bias; mid.experts16 = d.experts16; mid.rlog = x->rlog;
-        mid.route = routing(x, l, M); mid.arrived = lm_rows_sorts(M, L.top) ? x->arrived + x->n_arrived - 1 : nullptr;
+        mid.route = routing(x, l, M); mid.arrived = lm_rows_sorts(M, L.top) ? x->arrived : nullptr;
       }
       if ((rc = launch_lm_rows(mid, st))) return rc;
       if ((rc = feed_forward(x, l, M, rows, st))) return rc;
