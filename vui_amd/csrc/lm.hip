@@ -1,8 +1,8 @@
 // Token language models: context, step and C ABI.  See include/vui_lm.h.
 //
 // Launches per layer: attention of few rows 5 (input projection; queries into the latent space + append; attention
-// pieces; merge + value expansion; output projection), of a long block 6 (append, two expansions and one attention
-// kernel in the middle); minGRU 2 for one position per slot, 3-4 for a sequence (the scan in the middle).
+// pieces; merge + value expansion; output projection), of a long block 5 (append, expansion and one attention
+// kernel in the middle; 4 on shared latents); minGRU 2 for one position per slot, 3-4 for a sequence (the scan in the middle).
 #include <string.h>
 
 #include <new>

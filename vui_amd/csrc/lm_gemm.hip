@@ -647,7 +647,6 @@ int launch_lm_gemm(int dtype, int epi, const LmGemm& g, int nz, hipStream_t st) 
   }
   if (epi == LM_EXPAND) {
     if (dtype != VUI_DTYPE_BF16 || g.heads < 1 || g.n_v < 16 || (g.n_v & 15)) { vui_set_error("lm gemm: bad expansion"); return VUI_EINVAL; }
-    // XXX
     // the largest tile that gives every CU two workgroups (16 heads of 128 + 128, rank 512, 1999 positions: 18 us, with 64 x 128 24)
     auto tiles = [&](int bm, int bn) { return (long)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn + (g.n_v + bn - 1) / bn) * g.heads; };
     return pick_wide<LM_EXPAND>(g.N > 64 && tiles(128, 128) >= 512 ? WIDE_128 : g.N > 64 && tiles(64, 128) >= 512 ? WIDE_64x128 : WIDE_64, g, st);

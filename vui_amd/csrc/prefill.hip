@@ -636,7 +636,7 @@ __global__ __launch_bounds__(64 * PF_ATT_WAVES, 2) void pf_attn_kernel(const bf1
 // (4.8 us of 37 per layer for that launch alone).  A key fragment is 16 bytes of 16 rows (64 contiguous bytes each); values go through
 // a wave's own 32 x HD share of LDS and come back transposed (ds_read_b64_tr_b16: 16 lanes read 4 rows of 16, lane i
 // receives column i).  Bound by what one compute unit can fetch, so the keys of a (head, tile) are dealt to up to PF_SPLITS
-// workgroups of eight waves, a step of 32 keys per wave as far as that reaches; the last one to arrive merges their parts.
+// workgroups of four waves, 128 keys (a step of 32 per wave) for each as far as that reaches; the last one to arrive merges their parts.
 // Whole pass of 16 positions behind 600 / 2000, us: by a staged copy 777 / 964; here with 8 splits of four waves 644 / 704 (with the
 // cache read ahead, see pf_warm, 635 / 695), of eight waves and 256 keys 678 / 712, one workgroup of sixteen waves 830 / 1043.
 #define PF_SPLITS 8

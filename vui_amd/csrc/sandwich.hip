@@ -1,9 +1,9 @@
 // Sandwich layers of the token language models: x <- x + norm(mixer(norm(x))), then x <- x + norm(ff(norm(x))).  See
 // include/vui_lm.h and lm.hip, which holds the context and the C ABI.
 //
-// Launches: input projection, mixer (sigmoid attention 1, portions of a prompt 2, blocks of one 2; gated linear
-// attention 1, by chunks 3), output projection, rows, up, down, rows; an expert layer adds, with more rows than 16, the
-// router's product, 2 for routing and 1 that puts the rows in order.
+// Launches: input projection, mixer (sigmoid attention 1, portions of a prompt 2, blocks of one 2, without the bf16 matrix cores
+// 3; gated linear attention 1, by chunks 3), output projection, rows, up, down, rows; an expert layer adds, with more rows than
+// 16, the router's product, 2 for routing and 1 that puts the rows in order, with up to 16 rows of more than 64 choices 1 for routing.
 // The rows launch (rows.hip) norms and adds what a sublayer produced and norms what the next one reads.
 #include <string.h>
 
