@@ -21,7 +21,7 @@
 //
 // Several frames at once (vui_codec_decode_block: offline calls, the seeding of a stream): the same steps over
 // frames x columns, on buffers that hold a whole block with the histories in front; wide products run in
-// cv_wide_kernel.  93 frames: 56.6 ms one after the other, 5.9 ms in blocks of 32 (MI355X).
+// cv_wide_kernel.  93 frames: 56.6 ms one after the other, 6.0 ms in blocks of 32 (MI355X).
 #include "common.h"
 #include "internal.h"
 #include "../../include/vui_codec.h"
@@ -348,8 +348,8 @@ __global__ __launch_bounds__(NW * 64, 2) void cv_gemm1_kernel(const CvGemm p) {
 // (weights of 2^-118: error of the product 1.4e-5, 2^-122: 2e-4; with fp32 instructions 2e-6).  A value that is not finite makes its
 // columns or rows NaN, an infinite one too.
 // 32 frames: 7-tap convolutions of 768 / 384 / 192 / 96 channels 86 / 105 / 121 / 91 us -> 55 / 63 / 83 / 62 (1200 TFLOP/s
-// of bf16 products in the first, what hipBLASLt reaches at 8192^3), 1x1 19 / 30 / 32 / 33 -> 16 / 29 / 26 / 29; error of 93
-// frames against 64 bits 4.1e-6 -> 3.9e-6.
+// of bf16 products in the first, what hipBLASLt reaches at 8192^3), 1x1 19 / 30 / 32 / 33 -> 16 / 29 / 26 / 29 (3-4 % more with the clamp
+// of cv_split2); error of 93 frames against 64 bits 4.1e-6 -> 3.9e-6.
 // Tiles of BM x BN = 128 x 128 (or what divides M) of four waves through LDS, three planes of each operand: a K step is one (tap,
 // 32-channel) unit, fetched into registers while the one before it is multiplied, split on the way to LDS.  One buffer: two
 // workgroups of a CU overlap better than the steps of one (eight waves with two buffers and one to three units in flight: 75 us of
@@ -364,7 +364,8 @@ typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 cv_bf16x8;
 __device__ __forceinline__ int cv_at(int row, int piece) { return row * 32 + 8 * (piece ^ (row >> 2 & 3)); }
 
 // two fp32 values -> their three bf16 parts, packed.  The first part of a value above bf16's largest (3.39e38) is that largest: to the
-// nearest it would be infinity, and the column NaN.  That costs 93 frames 0.9 %.
+// nearest it would be infinity, and the column NaN.  Two instructions per pair: the products take 3-4 % more, 93 frames 5960 -> 6050 us.
+// (A tile computed once more with the clamp where a sum is not finite needs 40 registers more: 6070 us.)
 __device__ __forceinline__ void cv_split2(float a, float b, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
   const float top = __uint_as_float(0x7f7f0000u);
   hi = f2bf2(__builtin_amdgcn_fmed3f(a, -top, top), __builtin_amdgcn_fmed3f(b, -top, top));
