@@ -261,8 +261,8 @@ def test_short_blocks_behind_a_cache(heads, kv, window):
                 m.decoder.forward_flash(x, None)
 
 
-@pytest.mark.parametrize("window,every", [(128, 3), (300, 2), (300, 4), (40, 2)])
-def test_short_blocks_of_layers_with_and_without_a_window(window, every):
+@pytest.mark.parametrize("window,every,heads,dim", [(128, 3, 4, 64), (300, 2, 4, 64), (300, 4, 4, 64), (40, 2, 4, 64), (300, 2, 2, 96)])
+def test_short_blocks_of_layers_with_and_without_a_window(window, every, heads, dim):
     """Windowed and global layers in one model, behind caches where the ranges of keys that a layer's attention is dealt in are
     unequal in number (1 to 3 with the window, 2 to 8 without): outputs and every layer's appended keys and values, each position
     against the decode step behind the same cache, and the same bits in a second pass.  Two evaluations in bf16 move apart by 0.007
@@ -272,7 +272,7 @@ def test_short_blocks_of_layers_with_and_without_a_window(window, every):
     from vui_amd.model import Vui
 
     L = 5
-    d = O.Dims(d_model=256, n_layers=L, n_heads=4, n_kv_heads=2, n_quantizers=4, codebook_size=32, rq_d_model=64, rq_n_layers=1,
+    d = O.Dims(d_model=heads * dim, n_layers=L, n_heads=heads, n_kv_heads=heads // 2, n_quantizers=4, codebook_size=32, rq_d_model=64, rq_n_layers=1,
                rq_n_heads=2, vocab_size=50, max_seqlen=1280, window_size=window, global_every=every)
     m = Vui(dims_to_config(d, 1280), O.synthetic_state_dict(d, **TINY_SD), device="cuda", dtype=BF)
     dec = m.decoder
