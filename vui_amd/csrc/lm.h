@@ -97,7 +97,9 @@ struct LmGemm {
   const int32_t *ent, *tile_e, *n_tiles;
   int top, max_tiles, tile_rows;
   int sorted;      // X holds a row per entry instead of a row per position
-  int band;        // feature tiles of a band (lm_tile_at)
+  // lm_tile_at: feature tiles of a band; what divides by a band's tiles, its width and the last one's width
+  int band;
+  uint32_t inv_tiles, inv_band, inv_last;
 };
 int launch_lm_gemm(int dtype, int epi, const LmGemm& g, int nz, hipStream_t st);
 int launch_lm_embed(int dtype, const int64_t* tokens, const void* table, float* x, void* xt, float* ssq, int rows, int width,

@@ -157,16 +157,30 @@ __device__ __forceinline__ void lm_unit(const LmGemm& p, const int m, const int 
   }
 }
 
+// i / n with inv = lm_inv(n); the product is right or one too large
+static uint32_t lm_inv(uint32_t n) { return n > 1 ? 0xFFFFFFFFu / n + 1u : 0u; }
+__device__ __forceinline__ uint32_t lm_div(uint32_t i, uint32_t n, uint32_t inv) {
+  const uint32_t q = inv ? __umulhi(i, inv) : i;
+  return q - (q * n > i ? 1u : 0u);
+}
+
 // Tile of a workgroup.  Workgroups go round the eight XCDs, whose L2s are their own, so each XCD takes a contiguous range of the tiles, in
 // bands of `band` feature tiles with all row tiles: those that run side by side on an XCD share both operands.  In order of dispatch
 // every XCD met nearly all of both, and that, not the steps of a tile, bound the narrow products (650 x 1024 x 4224 on 176 tiles: 22 us
 // with or without a second half of waves; in bands 19).  Whole prompts, us before / after: sakupel 2048 wide x 200 positions 770 / 650,
 // 650 1186 / 1040, 1500 2025 / 1857; mabidra 1024 wide x 900 1216 / 1142, 2048 wide x 1200 2551 / 2419.
-__device__ __forceinline__ void lm_tile_at(int i, int MT, int NT, int band, int& t, int& nt) {
+// The divisions are products with what the host knows: by runtime values they took a launch of few tiles 0.2-0.3 us, and made some
+// short prompts slower than in order of dispatch (768 wide x 64 positions 7.1 -> 6.8 us per launch of 768 features).  Whole prompts:
+// mabidra 768 wide x 150 629 -> 611 us, sakupel 768 x 200 345 -> 339, 2048 wide x 1999 2241 -> 2197.
+__device__ __forceinline__ void lm_tile_at(const LmGemm& p, int i, int MT, int NT, int& t, int& nt) {
   const int n = MT * NT, x = i & 7, at = x * (n >> 3) + min(x, n & 7) + (i >> 3);
-  const int b = at / (band * MT), r = at - b * band * MT, w = min(band, NT - b * band);
-  t = r / w;
-  nt = b * band + r - t * w;
+  const int b = lm_div(at, p.band * MT, p.inv_tiles), r = at - b * p.band * MT, w = min(p.band, NT - b * p.band);
+  t = lm_div(r, w, w == p.band ? p.inv_band : p.inv_last);
+  nt = b * p.band + r - t * w;
+}
+static void lm_set_order(LmGemm& g, int MT, int NT, int band) {
+  g.band = band;
+  g.inv_tiles = lm_inv(band * MT); g.inv_band = lm_inv(band); g.inv_last = lm_inv(NT % band ? NT % band : band);
 }
 
 template <typename T, int MB, int NB, int WAVES, int EPI>
@@ -187,7 +201,7 @@ __global__ __launch_bounds__(64 * WAVES) void lm_gemm_kernel(const LmGemm p) {
   } else if (MB == 1) {  // one tile of rows, mostly
     t = (int)blockIdx.x % MT; nt = (int)blockIdx.x / MT;
   } else {
-    lm_tile_at(blockIdx.x, MT, ((p.N >> 4) + NB - 1) / NB, p.band, t, nt);
+    lm_tile_at(p, blockIdx.x, MT, ((p.N >> 4) + NB - 1) / NB, t, nt);
   }
   const int m0 = t * 16 * MB, nb0 = nt * NB;
   size_t wz = blockIdx.z * p.wz;
@@ -373,7 +387,7 @@ __global__ __launch_bounds__(256 * G, 2) void lm_wide_kernel(const LmGemm p) {
     t = slice % MT; nt = slice / MT * 8 + ((int)blockIdx.x & 7);
     if (nt >= NT) return;
   } else {
-    lm_tile_at(blockIdx.x, MT, NT, p.band, t, nt);
+    lm_tile_at(p, blockIdx.x, MT, NT, t, nt);
   }
   const int mb0 = t * MB, nb0 = nt * NB, m0 = mb0 * 16;
   const int Q = p.K / (32 * KS);  // steps
@@ -539,7 +553,8 @@ static int go_wide(LmGemm g, int nz, hipStream_t st) {
   const int MT = (g.M + 16 * MBW * WM - 1) / (16 * MBW * WM), NT = ((EPI == LM_EXPAND && g.n_v > g.N ? g.n_v : g.N) / 16 + NBW * WN - 1) / (NBW * WN);
   const bool moe = EPI == LM_MOE_UP || EPI == LM_MOE_DOWN;
   const bool strided = MBW * WM == 8 && EPI != LM_EXPAND && NT >= WIDE_STRIDED;
-  g.band = strided ? 0 : lm_band(MT, NT, MBW * WM, NBW * WN);
+  if (strided) g.band = 0;
+  else lm_set_order(g, MT, NT, lm_band(MT, NT, MBW * WM, NBW * WN));
   const int tiles = moe ? g.max_tiles * ((NT + 7) & ~7) : MT * (strided ? (NT + 7) & ~7 : NT);
   hipLaunchKernelGGL((lm_wide_kernel<EPI, MBW, NBW, WM, WN, S, KS, G>), dim3((unsigned)tiles, 1, nz), dim3(256 * G), 0, st, g);
   HIP_TRY(hipGetLastError());
@@ -550,8 +565,9 @@ template <typename T, int MB, int NB, int WAVES, int EPI>
 static int go(LmGemm g, int nz, hipStream_t st) {
   const bool moe = EPI == LM_MOE_UP || EPI == LM_MOE_DOWN;
   const int nt = (g.N / 16 + NB - 1) / NB;
-  g.band = lm_band((g.M + 16 * MB - 1) / (16 * MB), nt, MB, NB);
-  const int tiles = moe ? g.max_tiles * ((nt + 7) & ~7) : (g.M + 16 * MB - 1) / (16 * MB) * nt;
+  const int mt = (g.M + 16 * MB - 1) / (16 * MB);
+  lm_set_order(g, mt, nt, lm_band(mt, nt, MB, NB));
+  const int tiles = moe ? g.max_tiles * ((nt + 7) & ~7) : mt * nt;
   hipLaunchKernelGGL((lm_gemm_kernel<T, MB, NB, WAVES, EPI>), dim3((unsigned)tiles, 1, nz), dim3(64 * WAVES), 0, st, g);
   HIP_TRY(hipGetLastError());
   return VUI_OK;
