@@ -444,12 +444,14 @@ static int pf_wide(int tile, PfGemm& g, const void* W2, int c_tiled, hipStream_t
 }
 
 // two-rounding RMSNorm of rows (src/vui/model.py:286-297); one wave per row.  len != nullptr: the slot's new length goes there
-__global__ __launch_bounds__(256) void pf_rownorm_kernel(const bf16_t* x, const bf16_t* w, bf16_t* y, int M, int K, float eps, int x_tiled,
-                                                         int y_tiled, int32_t* len, int len_to) {
+// (where a row lies is known when compiled: asked for per piece it took a launch 0.3 us, 65 positions behind 600 3.57 -> 3.95)
+template <bool X_TILED>
+__global__ __launch_bounds__(256) void pf_rownorm_kernel(const bf16_t* x, const bf16_t* w, bf16_t* y, int M, int K, float eps, int y_tiled,
+                                                         int32_t* len, int len_to) {
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (len && blockIdx.x == 0 && threadIdx.x == 0) *len = len_to;
   if (row >= M) return;
-  auto xr = [&](int k) { return x + (x_tiled ? pf_toff(row, k, K) : (size_t)row * K + k); };
+  auto xr = [&](int k) { return x + (X_TILED ? pf_toff(row, k, K) : (size_t)row * K + k); };
   float ss = 0.f;
   for (int c = lane; c < K / 8; c += WAVE) {
     float v[8];
@@ -1049,7 +1051,9 @@ int launch_prefill(const vui_config& c, const vui_weights& w, const void* tiled_
                        tiny ? ssq : nullptr, tiny ? nullptr : vt, count, (int)sets, T, d, nkv, L, Lpad);
   }
   auto norm = [&](const void* w, bf16_t* y, int y_tiled, int32_t* len) {
-    hipLaunchKernelGGL(pf_rownorm_kernel, dim3((T + 3) / 4), dim3(256), 0, st, x, (const bf16_t*)w, y, T, d, c.norm_eps, tiny ? 1 : 0, y_tiled, len, L);
+    const dim3 grid((T + 3) / 4);
+    if (tiny) hipLaunchKernelGGL(pf_rownorm_kernel<true>, grid, dim3(256), 0, st, x, (const bf16_t*)w, y, T, d, c.norm_eps, y_tiled, len, L);
+    else hipLaunchKernelGGL(pf_rownorm_kernel<false>, grid, dim3(256), 0, st, x, (const bf16_t*)w, y, T, d, c.norm_eps, y_tiled, len, L);
   };
   int rc;
   for (int l = 0; l < c.n_layers; ++l) {
