@@ -653,7 +653,8 @@ struct PfDirectArgs {
   int T, nq, nkv, gsz, pos0, window;
   float scale;
   float *part, *ml;  // (head, tile, split): sums (DT x 64 lanes x 4), {max, sum of weights} x 16
-  uint32_t* count;   // arrivals of a (head, tile), zero between launches: layers with a window have fewer splits than those without
+  uint32_t* count;   // arrivals of a (head, tile) in the pass; `before`: those of earlier layers (their splits differ: windows)
+  uint32_t before;
 };
 typedef short pf_s16x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ uint2 pf_read_tr(const char* lds) {
@@ -778,11 +779,7 @@ __global__ __launch_bounds__(64 * PfDirect<HD32>::WAVES) void pf_direct_attn_ker
     if (tid < 16) st_dev(ml + sp * 32 + tid * 2, M, den);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (tid == 0) {
-      const bool last = __hip_atomic_fetch_add(a.count + set, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)nsp - 1;
-      if (last) __hip_atomic_store(a.count + set, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      *s_last = last;
-    }
+    if (tid == 0) *s_last = __hip_atomic_fetch_add(a.count + set, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == a.before + nsp - 1;
     __syncthreads();
     if (!*s_last) return;
     uint64_t xm[PF_SPLITS], xo[ND][PF_SPLITS][2];
@@ -823,11 +820,13 @@ __global__ __launch_bounds__(64 * PfDirect<HD32>::WAVES) void pf_direct_attn_ker
           make_uint2(f2bf2(o[i][0] * inv, o[i][1] * inv), f2bf2(o[i][2] * inv, o[i][3] * inv));
   }
 }
-template <int HD32> static int pf_direct_attn(const PfDirectArgs& a, int H, hipStream_t st) {
+template <int HD32> static int pf_direct_attn(PfDirectArgs& a, int H, hipStream_t st) {
   constexpr size_t lds = PfDirect<HD32>::LDS;
   const int L = a.pos0 + a.T, keys = a.window > 0 && a.window + 48 < L ? a.window + 48 : L, n = (keys + 127) / 128;
   HIP_TRY(hipFuncSetAttribute((const void*)pf_direct_attn_kernel<HD32>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  hipLaunchKernelGGL(pf_direct_attn_kernel<HD32>, dim3(H, (a.T + 15) / 16, n > PF_SPLITS ? PF_SPLITS : n), dim3(64 * PfDirect<HD32>::WAVES), lds, st, a);
+  const int splits = n > PF_SPLITS ? PF_SPLITS : n;
+  hipLaunchKernelGGL(pf_direct_attn_kernel<HD32>, dim3(H, (a.T + 15) / 16, splits), dim3(64 * PfDirect<HD32>::WAVES), lds, st, a);
+  if (splits > 1) a.before += splits;
   return VUI_OK;
 }
 
@@ -1055,6 +1054,7 @@ int launch_prefill(const vui_config& c, const vui_weights& w, const void* tiled_
     if (tiny) hipLaunchKernelGGL(pf_rownorm_kernel<true>, grid, dim3(256), 0, st, x, (const bf16_t*)w, y, T, d, c.norm_eps, y_tiled, len, L);
     else hipLaunchKernelGGL(pf_rownorm_kernel<false>, grid, dim3(256), 0, st, x, (const bf16_t*)w, y, T, d, c.norm_eps, y_tiled, len, L);
   };
+  PfDirectArgs da = {q, nullptr, nullptr, att, T, nq, nkv, H / KV, pos0, 0, scale, part, ml, count, 0};
   int rc;
   for (int l = 0; l < c.n_layers; ++l) {
     const vui_layer_weights& lw = w.layers[l];
@@ -1076,7 +1076,7 @@ int launch_prefill(const vui_config& c, const vui_weights& w, const void* tiled_
     g.nq = nq; g.nkv = nkv; g.hd = hd; g.inv_hd = pf_inv(hd); g.pos0 = pos0; g.Lpad = Lpad;
     if ((rc = pf_gemm4<PF_QKV, false>(g, nullptr, 0, i8, st))) return rc;
     if (tiny) {
-      const PfDirectArgs da = {q, g.kc, g.vc, att, T, nq, nkv, H / KV, pos0, win, scale, part, ml, count};
+      da.kc = g.kc; da.vc = g.vc; da.window = win;
       switch (hd / 32) {
         case 1: rc = pf_direct_attn<1>(da, H, st); break;
         case 2: rc = pf_direct_attn<2>(da, H, st); break;
