@@ -170,8 +170,8 @@ __device__ __forceinline__ uint32_t lm_div(uint32_t i, uint32_t n, uint32_t inv)
 // with or without a second half of waves; in bands 19).  Whole prompts, us before / after: sakupel 2048 wide x 200 positions 770 / 650,
 // 650 1186 / 1040, 1500 2025 / 1857; mabidra 1024 wide x 900 1216 / 1142, 2048 wide x 1200 2551 / 2419.
 // The divisions are products with what the host knows: by runtime values they took a launch of few tiles 0.2-0.3 us, and made some
-// short prompts slower than in order of dispatch (768 wide x 64 positions 7.1 -> 6.8 us per launch of 768 features).  Whole prompts:
-// mabidra 768 wide x 150 629 -> 611 us, sakupel 768 x 200 345 -> 339, 2048 wide x 1999 2241 -> 2197.
+// short prompts slower than in order of dispatch (mabidra 768 wide, interleaved, in order / divided / so: 64 positions 544 / 554 / 550 us, 80
+// 557 / 557 / 551, 120 587 / 586 / 579; 768 features of 64 rows 7.1 -> 6.8 us per launch).
 __device__ __forceinline__ void lm_tile_at(const LmGemm& p, int i, int MT, int NT, int& t, int& nt) {
   const int n = MT * NT, x = i & 7, at = x * (n >> 3) + min(x, n & 7) + (i >> 3);
   const int b = lm_div(at, p.band * MT, p.inv_tiles), r = at - b * p.band * MT, w = min(p.band, NT - b * p.band);
