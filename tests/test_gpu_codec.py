@@ -318,6 +318,20 @@ def test_blocks_of_wide_pre_transformers(d_model):
         assert err(got, ora.forward(codes)) < TOL and err(got, one.cpu()) < 2e-5, T
 
 
+@pytest.mark.parametrize("latent, dim, rates", [(96, 1408, (5, 3)), (64, 128, (16, 5)), (1120, 256, (2, 2))])
+def test_tiles_of_few_columns(latent, dim, rates):
+    """Channel groups that do not divide into the workgroups' shares or chunks (44, 22, 11, 35 of 32 channels), tiles of one to
+    four blocks of columns with the last one cut short, single frames and blocks of two and three."""
+    d = dataclasses.replace(small_dims(), latent_dim=latent, decoder_dim=dim, rates=rates)
+    sd = O.synthetic_codec_state_dict(d, seed=6)
+    ora, dec = O.CodecDecoderOracle(d, sd), native(d, sd)
+    codes = torch.randint(0, d.codebook_size, (1, d.n_codebooks, 7), generator=torch.Generator().manual_seed(3))
+    ref = ora.forward(codes)
+    with dec.streaming(1):
+        got = [dec(codes[:, :, t:t + 1].cuda()).clone() for t in range(2)] + [dec(codes[:, :, 2:4].cuda()).clone(), dec(codes[:, :, 4:].cuda()).clone()]
+    assert err(torch.cat(got, dim=-1), ref) < TOL
+
+
 def test_memory_of_a_call_follows_its_frames(full):
     """A call of a few frames allocates scratch memory for those (8 MB each), not for the longest block; a call of one none."""
     d, sd, dec, fx = full

@@ -15,9 +15,9 @@
 // X, X[(tap, ci)][t] = ring[ci][t + tap*dil].  Weights are repacked once to tap-major (taps, M, Cin) so a
 // lane reads 32 contiguous bytes of one output row; a transposed conv with kernel 2*stride is the
 // two-tap conv over (previous column, current column) with M = Cout*stride rows whose results are
-// scattered to column t*stride + r.  A workgroup owns 16 output rows x 16*TT columns; its waves split
-// the (tap, 32-channel) units, multiply on v_mfma_f32_16x16x4_f32 with both operands read straight from
-// global memory / L2 one step ahead, and add their parts through LDS in a fixed order.
+// scattered to column t*stride + r.  A workgroup owns 16 output rows x 16*TT columns; its input columns go through
+// LDS, its waves split the (tap, 32-channel) units, multiply on v_mfma_f32_16x16x4_f32 with the weights read straight from
+// global memory, and add their parts through LDS in a fixed order.
 //
 // Several frames at once (vui_codec_decode_block: offline calls, the seeding of a stream): the same steps over
 // frames x columns, on buffers that hold a whole block with the histories in front; wide products run in
@@ -26,6 +26,7 @@
 #include "internal.h"
 #include "../../include/vui_codec.h"
 
+#include <algorithm>
 #include <math.h>
 #include <new>
 #include <stdio.h>
@@ -71,10 +72,13 @@ struct CvGemm {
   const float* ib;
   const int* ctr;  // frames started; this pass is frames *ctr - nf ... *ctr - 1
   int nf;
-  int splits;      // workgroups that share one tile's (tap, channel) units; > 1: parts meet in `part`
+  int splits;      // workgroups that share one tile's channel groups; > 1: parts meet in `part`
+  int per, chunk;  // cv_cols_kernel: channel groups of a workgroup, and of those at a time
+  int xcols;       // and the input columns of a tile
+  uint32_t inv_xcols, inv_tc;
   float* part;     // (tiles, splits, TT*64*4) partial sums
   int* cnt;        // (tiles) arrival counters, zero between launches
-  int tt;          // 16-column blocks per tile (host side: picks the instantiation); 0: cv_wide_kernel with tile kWide[wide]
+  int tt;          // cv_cols_kernel: 16-column blocks per tile (picks the instantiation); 0: cv_wide_kernel with tile kWide[wide]
   int wide;
 };
 
@@ -94,162 +98,134 @@ template <bool NT> __device__ __forceinline__ float4 cv_ld_w(const float* p) {
   }
 }
 
-// units a wave keeps in registers per round: NU * (8 + 8*TT) VGPRs, twice that when the rounds are
-// double-buffered (DB: for tiles whose waves need several rounds; one wave per SIMD).  Tiles that fit one
-// round use the single-buffered form, which leaves room for two or three waves per SIMD.
-template <int TT, bool DB> struct Nu { static constexpr int N = TT == 1 ? 8 : (TT == 2 ? (DB ? 5 : 6) : 3); };
-
 #define CV_WIDE_T 64  // columns from which cv_wide_kernel takes a product of several frames
 
-// One 16-row x 16*TT-column output tile of NW waves.  `red` is NW * TT * 64 * 4 floats of LDS.
-template <int TT, bool DB, bool NT, int NW>
-__device__ __forceinline__ void cv_gemm_tile(const CvGemm& p, const int m0, const int t0, float* red,
-                                             const int tile, const int part_idx) {
-  constexpr int NU = Nu<TT, DB>::N;
+#define CV_NW 8        // waves of a workgroup of cv_cols_kernel
+#define CV_XROOM 17408 // floats of staged columns, at most: with the waves' parts 80 KiB, so two workgroups fit a CU
+// (tap, 32-channel) units of a wave between two barriers
+template <int TT> struct CvUnits { static constexpr int N = TT <= 2 ? 6 : 4; };
+
+// i / n for i n < 2^32 with inv = cv_inv(n)
+static uint32_t cv_inv(uint32_t n) { return n > 1 ? 0xFFFFFFFFu / n + 1u : 0u; }
+__device__ __forceinline__ uint32_t cv_div(uint32_t i, uint32_t inv) { return inv ? __umulhi(i, inv) : i; }
+
+// One tile of 16 output rows x 16 TT columns.  A workgroup takes `per` of the G = Cin / 32 channel groups with all their taps (splits
+// workgroups share a tile), `chunk` groups at a time: their input columns, taps - 1 dilations of halo among them, are read once,
+// coalesced, and laid into LDS with the channels side by side, from where every tap reads them as whole vectors; the chunk's units are dealt
+// round the waves, whose weights are on their way meanwhile.
+// Bound by its chain of trips: counter, columns, LDS, products, LDS, the parts' meeting.  With the columns read from memory by every tap
+// (eight loads of a float per unit and block of columns, issuing which took 3-4 us) and the outputs four to a lane, us per launch of a
+// single frame / so: 7 taps of 768 channels x 32 columns 16.5 / 11.8, 384 x 160 14.8 / 11.9, 192 x 640 13.0 / 10.7, 96 x 1920 10.7 / 9.2; one tap
+// 9.1 / 6.4, 7.9 / 5.6, 8.3 / 5.9, 7.4 / 5.6; the frame 572 / 482.
+template <int TT, bool NT>
+__global__ __launch_bounds__(64 * CV_NW, 4) void cv_cols_kernel(const CvGemm p) {
+  constexpr int NU = CvUnits<TT>::N, NTH = 64 * CV_NW, RED = CV_NW * TT * 256;
+  extern __shared__ __align__(16) float lds[];
+  float* red = lds;
+  float* xs = lds + RED;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int r16 = lane & 15, g = lane >> 4;
-  const int G = p.Cin >> 5, Uall = p.taps * G;
-  const int M = p.M, Cin = p.Cin;
-  // this workgroup's share of the units, and in it this wave's contiguous run [ub, U): a wave walks along
-  // its 16 weight rows, 128 bytes of each per unit
-  const int per = (Uall + p.splits - 1) / p.splits;
-  const int wb = part_idx * per, we = min(Uall, wb + per);
-  const int per_wave = (we - wb + NW - 1) / NW;
-  const int ub = min(we, wb + wave * per_wave), U = min(we, ub + per_wave);
+  const int m0 = blockIdx.x * 16, t0 = blockIdx.y * (16 * TT), tile = blockIdx.y * gridDim.x + blockIdx.x, part_idx = blockIdx.z;
+  const int M = p.M, Cin = p.Cin, G = Cin >> 5;
+  const int gb = part_idx * p.per, ge = min(G, gb + p.per);
+  const int halo = (p.taps - 1) * p.dil, cols = p.xcols - halo, S = p.chunk * 32 + 4;
 
-  float4 a0[NU][2], a1[DB ? NU : 1][2];
-  float b0[NU][TT][8], b1[DB ? NU : 1][TT][8];
+  // The wave's unit i of a chunk is wave + CV_NW i: group (unit / taps), tap (unit % taps).  The weights do not depend on the frame
+  // counter: those of the first chunk are asked for before the counter is needed.
+  float4 a[NU][2];
+  int off[NU];  // of the unit's first column in LDS
+  const uint32_t w_lane = (uint32_t)(r16 * Cin + g * 8);
+  const int g_step = CV_NW / p.taps, t_step = CV_NW - g_step * p.taps, g_first = wave / p.taps, t_first = wave - g_first * p.taps;
+  auto load_a = [&](int gc, int n) {
+    int gl = g_first, tap = t_first;
+#pragma unroll
+    for (int i = 0; i < NU; ++i) {
+      const bool on = gl < n;  // uniform over the wave
+      off[i] = on ? tap * p.dil * S + gl * 32 : -1;
+      if (on) {
+        const float* wp = p.W + ((size_t)tap * M + m0) * Cin + (gc + gl) * 32;
+        a[i][0] = cv_ld_w<NT>(wp + w_lane);
+        a[i][1] = cv_ld_w<NT>(wp + w_lane + 4);
+      }
+      gl += g_step; tap += t_step;
+      if (tap >= p.taps) { tap -= p.taps; ++gl; }
+    }
+  };
+  const int f = *p.ctr - p.nf;
+  load_a(gb, min(p.chunk, ge - gb));
+  const int ib_ = ring_base(p.in, f);
   floatx4 acc[TT];
 #pragma unroll
   for (int tt = 0; tt < TT; ++tt) acc[tt] = floatx4{0.f, 0.f, 0.f, 0.f};
-
-  // request the operands of units u0, u0 + NW, ... (NU of them); nothing is waited for here.  The weights
-  // do not depend on the frame counter, so the first round asks for them before the counter is needed.
-  auto load_a = [&](int u0, auto& a) {
+  // Every thread finishes NO of the tile's sums: row (tid / 16) % 16, column tid % 16 of block tid / 256 (+ 2).  (Four rows of a column per lane
+  // of the first TT waves was 1 us more per launch: long chains of sines and stores in few waves; the frame 515 / 483.)
+  constexpr int NO = TT == 4 ? 2 : 1;
+  const int em = m0 + ((tid >> 4) & 15), ech = p.tc_stride > 0 ? (int)cv_div(em, p.inv_tc) : em;
+  float e_bias = 0.f, e_sc = 1.f, e_ea = 0.f, e_ib = 0.f, e_res[NO];
+  int ecol[NO];  // of the output, -1: none
+  const float* xrow[TT];  // this lane's columns
 #pragma unroll
-    for (int i = 0; i < NU; ++i) {
-      const int u = u0 + i;
-      const bool on = u < U;
-      const int tap = on ? u / G : 0, grp = on ? u - tap * G : 0;
-      const float* wp = p.W + ((size_t)tap * M + m0 + r16) * Cin + grp * 32 + g * 8;
-      if constexpr (NT) {
-        a[i][0] = on ? cv_ld_w<true>(wp) : make_float4(0.f, 0.f, 0.f, 0.f);
-        a[i][1] = on ? cv_ld_w<true>(wp + 4) : make_float4(0.f, 0.f, 0.f, 0.f);
-      } else {
-        a[i][0] = on ? *reinterpret_cast<const float4*>(wp) : make_float4(0.f, 0.f, 0.f, 0.f);
-        a[i][1] = on ? *reinterpret_cast<const float4*>(wp + 4) : make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int tt = 0; tt < TT; ++tt) xrow[tt] = xs + min(tt * 16 + r16, cols - 1) * S + g * 8;
+  float ss = 0.f;  // IN_RMS: this thread's share of its column's sum of squares
+  constexpr int TPC = NTH / (16 * TT);
+
+  for (int gc = gb; gc < ge; gc += p.chunk) {
+    const int n = min(p.chunk, ge - gc);
+    if (gc > gb) { load_a(gc, n); __syncthreads(); }  // the columns of the chunk before have been read
+    // four channels of a column per thread and round
+    const int total = n * 8 * p.xcols;
+    const float *in0 = p.in.p + (size_t)gc * 32 * p.in.rs, *in1 = in0 + p.in.rs, *in2 = in1 + p.in.rs, *in3 = in2 + p.in.rs;
+    for (int i0 = tid; i0 < total; i0 += 4 * NTH) {
+      float4 v[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int i = min(i0 + k * NTH, total - 1), q = (int)cv_div(i, p.inv_xcols), c = i - q * p.xcols;
+        const uint32_t o = (uint32_t)(4 * q * p.in.rs + ((ib_ + min(t0 + c, p.T - 1 + halo)) & p.in.mask));
+        v[k] = make_float4(in0[o], in1[o], in2[o], in3[o]);
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int i = i0 + k * NTH, q = (int)cv_div(i, p.inv_xcols), c = i - q * p.xcols;
+        if (i < total) *reinterpret_cast<float4*>(xs + c * S + 4 * q) = v[k];
       }
     }
-  };
-  int ib_ = 0;
-  auto load_b = [&](int u0, auto& b) {
+    if (gc == gb) {  // what the epilogue adds is requested now as well
+      const int rb = ring_base(p.res, f);
+      if (p.bias) e_bias = p.bias[ech];
+      if (p.epi == EPI_SCALE_RES) e_sc = p.scale[ech];
+      if (p.out_act.p) { e_ea = p.ea[ech]; e_ib = p.ib[ech]; }
+#pragma unroll
+      for (int k = 0; k < NO; ++k) {
+        const int tt = (tid >> 8) + 2 * k, t = t0 + tt * 16 + (tid & 15);
+        ecol[k] = tt < TT && t < p.T ? (p.tc_stride > 0 ? t * p.tc_stride + em - ech * p.tc_stride : t) : -1;
+        e_res[k] = 0.f;
+        if ((p.epi == EPI_RES || p.epi == EPI_SCALE_RES) && ecol[k] >= 0) e_res[k] = *ring_ptr(p.res, rb, ech, p.res.pad + ecol[k]);
+      }
+    }
+    __syncthreads();
+    if (p.in_mode == IN_RMS) {  // one tap
+      const float* col = xs + min(tid / TPC, cols - 1) * S;
+      for (int q = tid % TPC; q < n * 8; q += TPC) {
+        const float4 v = *reinterpret_cast<const float4*>(col + 4 * q);
+        ss += (v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w);
+      }
+    }
 #pragma unroll
     for (int i = 0; i < NU; ++i) {
-      const int u = u0 + i;
-      const bool on = u < U;
-      const int tap = on ? u / G : 0, grp = on ? u - tap * G : 0;
-      const int ci0 = grp * 32 + g * 8;
+      if (off[i] < 0) break;  // uniform over the wave
+      const float av[8] = {a[i][0].x, a[i][0].y, a[i][0].z, a[i][0].w, a[i][1].x, a[i][1].y, a[i][1].z, a[i][1].w};
+      float bv[TT][8];
 #pragma unroll
       for (int tt = 0; tt < TT; ++tt) {
-        const int t = t0 + tt * 16 + r16;
-        const bool bon = on && t < p.T;
-        const float* xp = ring_ptr(p.in, ib_, bon ? ci0 : 0, bon ? t + tap * p.dil : 0);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) b[i][tt][j] = bon ? xp[(size_t)j * p.in.rs] : 0.f;
+        const float4 lo = *reinterpret_cast<const float4*>(xrow[tt] + off[i]), hi = *reinterpret_cast<const float4*>(xrow[tt] + off[i] + 4);
+        bv[tt][0] = lo.x; bv[tt][1] = lo.y; bv[tt][2] = lo.z; bv[tt][3] = lo.w;
+        bv[tt][4] = hi.x; bv[tt][5] = hi.y; bv[tt][6] = hi.z; bv[tt][7] = hi.w;
       }
-    }
-  };
-  auto load = [&](int u0, auto& a, auto& b) { load_a(u0, a); load_b(u0, b); };
-  auto mma = [&](const auto& a, const auto& b) {
-#pragma unroll
-    for (int i = 0; i < NU; ++i) {
-      const float av[8] = {a[i][0].x, a[i][0].y, a[i][0].z, a[i][0].w, a[i][1].x, a[i][1].y, a[i][1].z, a[i][1].w};
 #pragma unroll
       for (int j = 0; j < 8; ++j)
 #pragma unroll
-        for (int tt = 0; tt < TT; ++tt)
-          acc[tt] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[j], b[i][tt][j], acc[tt], 0, 0, 0);
-    }
-  };
-
-  constexpr int STEP = NU;
-  load_a(ub, a0);
-  const int f = *p.ctr - p.nf;
-  ib_ = ring_base(p.in, f);
-  load_b(ub, b0);
-  // what the epilogue adds is requested now as well
-  const int rb = ring_base(p.res, f), ob = ring_base(p.out_raw, f), ab = ring_base(p.out_act, f);
-  float e_bias[4] = {0.f, 0.f, 0.f, 0.f}, e_res[4] = {0.f, 0.f, 0.f, 0.f}, e_sc[4] = {1.f, 1.f, 1.f, 1.f};
-  float e_ea[4] = {0.f, 0.f, 0.f, 0.f}, e_ib[4] = {0.f, 0.f, 0.f, 0.f};
-  if (tid < TT * 64) {
-    const int t = t0 + (tid >> 6) * 16 + (tid & 15);
-    if (t < p.T) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int m = m0 + 4 * ((tid & 63) >> 4) + r;
-        int ch = m, col = t;
-        if (p.tc_stride > 0) { ch = m / p.tc_stride; col = t * p.tc_stride + m % p.tc_stride; }
-        if (p.bias) e_bias[r] = p.bias[m / p.bias_div];
-        if (p.epi == EPI_RES || p.epi == EPI_SCALE_RES) e_res[r] = *ring_ptr(p.res, rb, ch, p.res.pad + col);
-        if (p.epi == EPI_SCALE_RES) e_sc[r] = p.scale[ch];
-        if (p.out_act.p) { e_ea[r] = p.ea[ch]; e_ib[r] = p.ib[ch]; }
-      }
-    }
-  }
-  // 1/rms of the input column while the first operands are in flight; applied to the sums at the end
-  float rstd = 1.f;
-  if (p.in_mode == IN_RMS && p.T > 1) {  // a column per frame: 4 threads of every wave share one
-    constexpr int SH = 4 * NW;
-    __shared__ float sq[TT * 16 * SH];
-    // sixteen loads in flight per column: as a plain loop this was most of the launch (32 frames, 3072 x 512 14.2 -> 9.1 us, 2048 x 512
-    // 13.8 -> 8.4)
-    float ss[TT];
-#pragma unroll
-    for (int tt = 0; tt < TT; ++tt) ss[tt] = 0.f;
-    for (int c0 = tid >> 4; c0 < Cin; c0 += 16 * SH) {
-      float v[TT][16];
-#pragma unroll
-      for (int i = 0; i < 16; ++i)
-#pragma unroll
-        for (int tt = 0; tt < TT; ++tt)
-          v[tt][i] = *ring_ptr(p.in, ib_, min(c0 + i * SH, Cin - 1), p.in.pad + min(t0 + tt * 16 + (tid & 15), p.T - 1));
-#pragma unroll
-      for (int i = 0; i < 16; ++i)
-#pragma unroll
-        for (int tt = 0; tt < TT; ++tt)
-          if (c0 + i * SH < Cin) ss[tt] = fmaf(v[tt][i], v[tt][i], ss[tt]);
-    }
-#pragma unroll
-    for (int tt = 0; tt < TT; ++tt) sq[(tt * 16 + (tid & 15)) * SH + (tid >> 4)] = ss[tt];
-    __syncthreads();
-    if (tid < TT * 64) {
-      float ss = 0.f;
-#pragma unroll
-      for (int i = 0; i < SH; ++i) ss += sq[((tid >> 6) * 16 + (tid & 15)) * SH + i];
-      rstd = 1.0f / sqrtf(ss / (float)Cin + p.eps);
-    }
-  } else if (p.in_mode == IN_RMS) {
-    float ss = 0.f;
-    for (int c = lane; c < Cin; c += WAVE) {
-      const float v = *ring_ptr(p.in, ib_, c, p.in.pad);
-      ss = fmaf(v, v, ss);
-    }
-    ss = wave_sum(ss);
-    rstd = 1.0f / sqrtf(ss / (float)Cin + p.eps);
-  }
-  if constexpr (DB) {
-    for (int u0 = ub; u0 < U; u0 += 2 * STEP) {
-      if (u0 + STEP < U) load(u0 + STEP, a1, b1);
-      mma(a0, b0);
-      if (u0 + STEP < U) {
-        if (u0 + 2 * STEP < U) load(u0 + 2 * STEP, a0, b0);
-        mma(a1, b1);
-      }
-    }
-  } else {
-    for (int u0 = ub; u0 < U; u0 += STEP) {
-      if (u0 != ub) load(u0, a0, b0);
-      mma(a0, b0);
+        for (int tt = 0; tt < TT; ++tt) acc[tt] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[j], bv[tt][j], acc[tt], 0, 0, 0);
+      if (i & 1) __builtin_amdgcn_sched_barrier(0);  // more units' operands at a time do not fit the registers
     }
   }
 
@@ -258,20 +234,29 @@ __device__ __forceinline__ void cv_gemm_tile(const CvGemm& p, const int m0, cons
   for (int tt = 0; tt < TT; ++tt)
     *reinterpret_cast<float4*>(red + ((size_t)(wave * TT + tt) * 64 + lane) * 4) =
         make_float4(acc[tt][0], acc[tt][1], acc[tt][2], acc[tt][3]);
-  __syncthreads();
-  float v[4] = {0.f, 0.f, 0.f, 0.f};
-  if (tid < TT * 64) {
+  __shared__ float rms[16 * TT];
+  if (p.in_mode == IN_RMS) {  // neighbouring threads share a column
 #pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      const float4 q = *reinterpret_cast<const float4*>(red + ((size_t)w * TT * 64 + tid) * 4);
-      v[0] += q.x; v[1] += q.y; v[2] += q.z; v[3] += q.w;
-    }
+    for (int o = TPC / 2; o >= 1; o >>= 1) ss += __shfl_xor(ss, o);
+    if (tid % TPC == 0) rms[tid / TPC] = 1.0f / sqrtf(ss / (float)Cin + p.eps);
   }
+  __syncthreads();
+  float v[NO];
+#pragma unroll
+  for (int k = 0; k < NO; ++k) {
+    v[k] = 0.f;
+    const float* src = red + (size_t)(min((tid >> 8) + 2 * k, TT - 1) * 64 + ((tid >> 6) & 3) * 16 + (tid & 15)) * 4 + ((tid >> 4) & 3);
+#pragma unroll
+    for (int w = 0; w < CV_NW; ++w) v[k] += src[w * TT * 256];
+  }
+  const bool mine = TT > 1 || tid < 256;
   if (p.splits > 1) {
     // parts of a tile meet in memory; the workgroup that arrives last adds them in part order and finishes
     __shared__ int last;
-    float* mine = p.part + (((size_t)tile * p.splits + part_idx) * TT * 64 + tid) * 4;
-    if (tid < TT * 64) { st_dev(mine, v[0], v[1]); st_dev(mine + 2, v[2], v[3]); }
+    float* part = p.part + (size_t)tile * p.splits * TT * 256 + tid;
+    if (mine)
+#pragma unroll
+      for (int k = 0; k < NO; ++k) __hip_atomic_store(part + part_idx * TT * 256 + 512 * k, v[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the write-through stores have completed
     __syncthreads();
     if (tid == 0) {
@@ -281,61 +266,41 @@ __device__ __forceinline__ void cv_gemm_tile(const CvGemm& p, const int m0, cons
     }
     __syncthreads();
     if (!last) return;
-    if (tid < TT * 64) {
-      uint64_t q[8][2];
+    if (mine) {
+      float q[NO][8];
 #pragma unroll
-      for (int z = 0; z < 8; ++z) {
-        const float* src = p.part + (((size_t)tile * p.splits + z) * TT * 64 + tid) * 4;
-        q[z][0] = z < p.splits ? ld_dev(src) : 0;
-        q[z][1] = z < p.splits ? ld_dev(src + 2) : 0;
-      }
-      v[0] = v[1] = v[2] = v[3] = 0.f;
+      for (int k = 0; k < NO; ++k)
 #pragma unroll
-      for (int z = 0; z < 8; ++z) {
-        v[0] += __uint_as_float((uint32_t)q[z][0]); v[1] += __uint_as_float((uint32_t)(q[z][0] >> 32));
-        v[2] += __uint_as_float((uint32_t)q[z][1]); v[3] += __uint_as_float((uint32_t)(q[z][1] >> 32));
+        for (int z = 0; z < 8; ++z) q[k][z] = z < p.splits ? __hip_atomic_load(part + z * TT * 256 + 512 * k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.f;
+#pragma unroll
+      for (int k = 0; k < NO; ++k) {
+        v[k] = 0.f;
+#pragma unroll
+        for (int z = 0; z < 8; ++z) v[k] += q[k][z];
       }
     }
   }
-  if (tid < TT * 64) {
-    const int tt = tid >> 6, l = tid & 63;
-    const int t = t0 + tt * 16 + (l & 15);
-    if (t >= p.T) return;
+  if (!mine) return;
+  const int ob = ring_base(p.out_raw, f), ab = ring_base(p.out_act, f);
+#pragma unroll
+  for (int k = 0; k < NO; ++k) {
+    if (p.in_mode == IN_RMS) v[k] *= rms[min((tid >> 8) + 2 * k, TT - 1) * 16 + (tid & 15)];
     if (p.epi == EPI_SILU_PAIR) {
-#pragma unroll
-      for (int r = 0; r < 4; r += 2) {
-        const float ga = v[r] * rstd, up = v[r + 1] * rstd;
-        *ring_ptr(p.out_raw, ob, (m0 + 4 * (l >> 4) + r) >> 1, p.out_raw.pad + t) = ga / (1.0f + expf(-ga)) * up;
-      }
-      return;
+      const float up = __shfl_xor(v[k], 16);  // the next row's, for the even ones
+      if (!(tid & 16) && ecol[k] >= 0) *ring_ptr(p.out_raw, ob, em >> 1, p.out_raw.pad + ecol[k]) = v[k] / (1.0f + expf(-v[k])) * up;
+      continue;
     }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int m = m0 + 4 * (l >> 4) + r;
-      float y = v[r] * rstd + e_bias[r];
-      int ch = m, col = t;
-      if (p.tc_stride > 0) { ch = m / p.tc_stride; col = t * p.tc_stride + m % p.tc_stride; }
-      if (p.epi == EPI_GELU) y = 0.5f * y * (1.0f + erff(y * 0.70710678118654752f));
-      else if (p.epi == EPI_RES) y = e_res[r] + y;
-      else if (p.epi == EPI_SCALE_RES) y = e_res[r] + e_sc[r] * y;
-      if (p.out_raw.p) *ring_ptr(p.out_raw, ob, ch, p.out_raw.pad + col) = y;
-      if (p.out_act.p) {
-        const float s = sinf(y * e_ea[r]);
-        *ring_ptr(p.out_act, ab, ch, p.out_act.pad + col) = y + e_ib[r] * s * s;
-      }
+    float y = v[k] + e_bias;
+    if (p.epi == EPI_GELU) y = 0.5f * y * (1.0f + erff(y * 0.70710678118654752f));
+    else if (p.epi == EPI_RES) y = e_res[k] + y;
+    else if (p.epi == EPI_SCALE_RES) y = e_res[k] + e_sc * y;
+    if (ecol[k] < 0) continue;
+    if (p.out_raw.p) *ring_ptr(p.out_raw, ob, ech, p.out_raw.pad + ecol[k]) = y;
+    if (p.out_act.p) {
+      const float sn = sinf(y * e_ea);
+      *ring_ptr(p.out_act, ab, ech, p.out_act.pad + ecol[k]) = y + e_ib * sn * sn;
     }
   }
-}
-
-template <int TT, bool NT>
-__global__ __launch_bounds__(256) void cv_gemm_kernel(const CvGemm p) {
-  __shared__ __align__(16) float red[4 * TT * 64 * 4];
-  cv_gemm_tile<TT, true, NT, 4>(p, blockIdx.x * 16, blockIdx.y * (16 * TT), red, blockIdx.y * gridDim.x + blockIdx.x, blockIdx.z);
-}
-template <int TT, bool NT, int NW>
-__global__ __launch_bounds__(NW * 64, 2) void cv_gemm1_kernel(const CvGemm p) {
-  __shared__ __align__(16) float red[NW * TT * 64 * 4];
-  cv_gemm_tile<TT, false, NT, NW>(p, blockIdx.x * 16, blockIdx.y * (16 * TT), red, blockIdx.y * gridDim.x + blockIdx.x, blockIdx.z);
 }
 
 // ---- the same product for many columns (several frames at once) ----
@@ -1498,10 +1463,27 @@ struct WideTile { int bm, bn; float unit; };
 #define CVW_PARTS (6u << 20)  // floats of the parts of a split product, which the workspace holds
 static const WideTile kWide[] = {{128, 128, 1.0f}, {96, 128, 0.79f}, {64, 128, 0.63f}, {128, 64, 0.63f}, {32, 128, 0.55f}};
 
+static int cv_lds(const CvGemm& g) { return (CV_NW * g.tt * 256 + g.xcols * (g.chunk * 32 + 4)) * 4; }
+// The fields of cv_cols_kernel for a tile shared by up to `splits` workgroups: chunks whose units fit the waves' registers and whose
+// columns fit LDS (one group always does: a tile of 64 columns and its halo of 6 x 9 take 118 x 36 floats).
+static void cv_shape(CvGemm& g, int splits) {
+  const int G = g.Cin / 32, units = (g.tt <= 2 ? CvUnits<2>::N : CvUnits<4>::N) * CV_NW;
+  g.per = (G + splits - 1) / splits;
+  g.splits = (G + g.per - 1) / g.per;
+  g.xcols = (g.T < 16 * g.tt ? g.T : 16 * g.tt) + (g.taps - 1) * g.dil;
+  g.inv_xcols = cv_inv(g.xcols);
+  g.inv_tc = cv_inv(g.tc_stride);
+  const int fit = std::max(1, std::min(units / g.taps, (CV_XROOM / g.xcols - 4) / 32)), rounds = (std::min(g.per, G) + fit - 1) / fit;
+  g.chunk = (g.per + rounds - 1) / rounds;
+}
+
 // Chooses tile width, splits and kernel for g.T columns.
 static CvScratch cv_plan(CvGemm& g) {
   const int U = g.taps * (g.Cin / 32), M = g.M, T = g.T;
-  if (g.nf > 1 && T >= CV_WIDE_T && M % 32 == 0 && g.in_mode == IN_PLAIN && g.epi != EPI_SILU_PAIR) {
+  auto tiles = [&](int tt) { return (M / 16) * ((T + 16 * tt - 1) / (16 * tt)); };
+  // few units and few tiles: a launch of cv_cols_kernel is shorter than the large tiles' two (768 channels x 128 columns, 1x1: 14 / 8 us)
+  const bool few = U <= 32 && tiles(1) <= 512;
+  if (g.nf > 1 && T >= CV_WIDE_T && !few && M % 32 == 0 && g.in_mode == IN_PLAIN && g.epi != EPI_SILU_PAIR) {
     // Tile and splits: what the workgroups of a CU take, in pairs, and for split tiles the second launch and its traffic.
     size_t part = 0;
     double cost = 0;
@@ -1520,30 +1502,16 @@ static CvScratch cv_plan(CvGemm& g) {
     }
     return CvScratch{part, 0};
   }
-  // Tile width: the one that pads the columns least, the wider one on a tie (a wave reuses its weight
-  // registers for every 16-column block).  Then workgroups share a tile's units until about 512 (one
-  // column block: the layer streams weights) or 200 (wider: the layer computes) are in flight, each wave
-  // keeping at least four units.  Measured per layer shape on MI355X.
-  auto tiles = [&](int tt) { return (M / 16) * ((T + 16 * tt - 1) / (16 * tt)); };
-  g.tt = 1;
-  for (int tt : {2, 4})
-    if (T > 8 * tt && tiles(tt) * tt <= tiles(g.tt) * g.tt) g.tt = tt;
-  // a tile of 64 columns holds 3 units per wave and round, one of 32 columns 6: the narrower one where that saves the second
-  // round (192 channels x 640 columns: 19.2 / 13.1 us)
-  if (g.tt == 4 && U > 24 && U <= 48 && tiles(2) <= 256) g.tt = 2;
-  int sp = 1;
-  if (U >= 64) {
-    const int target = g.tt == 1 ? 512 : 200;
-    sp = (2 * target + tiles(g.tt)) / (2 * tiles(g.tt));  // rounded
-    if (g.tt == 1 && sp < (U + 63) / 64) sp = (U + 63) / 64;  // eight waves of one round each
-    if (sp > U / 16) sp = U / 16;
-    if (sp > 8) sp = 8;
-    if (sp < 1) sp = 1;
-  } else if (g.nf > 1 && g.tt > 1 && U >= 32 && tiles(g.tt) <= 100) {
-    sp = 2;  // few tiles of several frames: each streams its rows' weights alone (trunk of 32 frames, 512 x 1024: 11.2 -> 9 us)
-  }
-  g.splits = sp;
-  return CvScratch{(size_t)tiles(g.tt) * sp * g.tt * 256, (size_t)tiles(g.tt)};
+  // The narrowest tiles that are no more than the CUs; products of many units start at 32 columns, where a weight meets two blocks of
+  // columns.  Then workgroups share a tile's channels until the CUs are busy (twice that for one block of columns: the layer
+  // streams weights), each with 32 units or so.
+  const int G = g.Cin / 32, most = g.in_mode == IN_PLAIN ? (U + 16) / 32 : 1;  // a split norm would need the other workgroups' sums
+  g.tt = T > 16 && U > 32 ? 2 : 1;
+  while (g.tt < 4 && T > 16 * g.tt && tiles(g.tt) > 256) g.tt *= 2;
+  const int target = T <= 16 ? 512 : 256;
+  const int sp = std::max(1, std::min(std::min((2 * target + tiles(g.tt)) / (2 * tiles(g.tt)), most), std::min(8, G)));
+  cv_shape(g, sp);
+  return CvScratch{(size_t)tiles(g.tt) * g.splits * g.tt * 256, (size_t)tiles(g.tt)};
 }
 
 // Lays out the workspace and (when tensors != nullptr) packs weights and records the launch plan.
@@ -1602,7 +1570,11 @@ static int cv_build(vui_codec* cc, const vui_codec_config* c, const void* const*
     }
     return g;
   };
-  auto push_gemm = [&](const CvGemm& g) { if (real) { Step s; memset((void*)&s, 0, sizeof(s)); s.kind = 0; s.g = g; cc->steps.push_back(s); } };
+  auto push_gemm = [&](CvGemm& g) {
+    if (!real) return;
+    cv_plan(g);  // with the norm known
+    Step s; memset((void*)&s, 0, sizeof(s)); s.kind = 0; s.g = g; cc->steps.push_back(s);
+  };
 
   const int cd = c->codebook_dim, CS = c->codebook_size, L = c->latent_dim, D = c->d_model, A = c->n_heads * c->head_dim;
   // ---- quantizer: [semantic | acoustic] rows times [W_sem | W_ac] ----
@@ -1906,6 +1878,9 @@ int vui_codec_init(const vui_codec_config* cfg, const void* const* tensors, int3
   }
   if (!rc) rc = vui_codec_reset(c, stream);
   if (rc) { delete c; return rc; }
+  for (const void* k : {(const void*)cv_cols_kernel<1, false>, (const void*)cv_cols_kernel<1, true>, (const void*)cv_cols_kernel<2, false>,
+                        (const void*)cv_cols_kernel<2, true>, (const void*)cv_cols_kernel<4, false>, (const void*)cv_cols_kernel<4, true>})
+    HIP_TRY(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (CV_NW * 4 * 256 + CV_XROOM) * 4));
   // the persistent trunk needs all its workgroups resident at once and the per-wave row counts it was built for
   {
     const vui_codec_config& k = c->cfg;
@@ -1961,22 +1936,12 @@ static int launch_cv_gemm(const CvGemm& g, bool w_nt, hipStream_t st) {
     if (g.splits > 1) hipLaunchKernelGGL(cv_finish_kernel, dim3((g.T + 63) / 64, g.M / 32), dim3(256), 0, st, g, tiles * w.bn);
     return VUI_OK;
   }
-  const dim3 grid(g.M / 16, (g.T + 16 * g.tt - 1) / (16 * g.tt), g.splits);
-  // units a wave of one part works through; one single-buffered round holds 8 / 6 / 3 of them.  Eight waves where four need
-  // more than a round: a second round is a second trip to memory (dilated convs of one frame: 16-18 us with four waves).
-  const int U = g.taps * (g.Cin / 32), part = (U + g.splits - 1) / g.splits, round = g.tt == 1 ? 8 : (g.tt == 2 ? 6 : 3);
-#define CV_TT(TT_)                                                                                                   \
-  do {                                                                                                               \
-    if ((part + 3) / 4 <= round) {                                                                                   \
-      if (w_nt) hipLaunchKernelGGL((cv_gemm1_kernel<TT_, true, 4>), grid, dim3(256), 0, st, g);                      \
-      else hipLaunchKernelGGL((cv_gemm1_kernel<TT_, false, 4>), grid, dim3(256), 0, st, g);                          \
-    } else if ((part + 7) / 8 <= round) {                                                                            \
-      if (w_nt) hipLaunchKernelGGL((cv_gemm1_kernel<TT_, true, 8>), grid, dim3(512), 0, st, g);                      \
-      else hipLaunchKernelGGL((cv_gemm1_kernel<TT_, false, 8>), grid, dim3(512), 0, st, g);                          \
-    } else {                                                                                                         \
-      if (w_nt) hipLaunchKernelGGL((cv_gemm_kernel<TT_, true>), grid, dim3(256), 0, st, g);                          \
-      else hipLaunchKernelGGL((cv_gemm_kernel<TT_, false>), grid, dim3(256), 0, st, g);                              \
-    }                                                                                                                \
+  const dim3 grid(g.M / 16, (g.T + 16 * g.tt - 1) / (16 * g.tt), g.splits), block(64 * CV_NW);
+  const int lds = cv_lds(g);
+#define CV_TT(TT_)                                                                              \
+  do {                                                                                          \
+    if (w_nt) hipLaunchKernelGGL((cv_cols_kernel<TT_, true>), grid, block, lds, st, g);         \
+    else hipLaunchKernelGGL((cv_cols_kernel<TT_, false>), grid, block, lds, st, g);             \
   } while (0)
   if (g.tt == 1) CV_TT(1);
   else if (g.tt == 2) CV_TT(2);
