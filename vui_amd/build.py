@@ -20,6 +20,8 @@ FLAGS = [
     "-O3", "--offload-arch=gfx950", "-fPIC", "-std=c++17", "-Wall", "-Wno-unused-function",
     # packed-fp32 instructions are kept out of every code object of this library
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # the first scalar arguments of a kernel arrive in registers instead of by a trip to memory
+    "-mllvm", "-amdgpu-kernarg-preload-count=14",
 ]
 
 

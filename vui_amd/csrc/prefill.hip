@@ -35,7 +35,8 @@ struct PfGemm {
                      // at 16 * lane) with the per-row scales sc (and sc2 for the second matrix of a SwiGLU pair)
   const bf16_t *sc, *sc2;
   void* C;           // output (M x N) bf16: row-major with row stride ldc (PF_RESID: in place on the residual), or tiled
-  int M, N, K, ldc;
+  int M, N, K, ldc;  // ldc: of PF_QKV
+  int c_tiled;
   // X is the residual and is normed on its way: sums of squares of every 16 columns (M x K / 16), weights (K)
   const float* ssq;
   const bf16_t* nw;
@@ -66,6 +67,15 @@ __device__ __forceinline__ void pf_warm(const PfGemm& p, int part) {
     asm volatile("" ::"v"(k.x), "v"(v.x));
   }
 }
+
+// The first fourteen words of a kernel's scalar arguments are in registers when it starts; a struct behind them is a trip to memory.
+// What the first loads of a product need therefore comes twice, ahead of the struct and in it: 0.2-0.35 us of a launch of 4-6 (16
+// positions, us per launch: QKV 5.4 -> 5.1, W1 and W3 5.6 -> 5.2; whole pass of 576 positions 1160 -> 1121, of 1733 in int8 1976 -> 1952).
+#define PF_HOT const bf16_t *X, const void *W, const void *aux, const bf16_t *nw, int M, uint32_t nk, uint32_t xcd, uint32_t run, uint32_t inv_run
+#define PF_HOT_ARGS(g, aux) g.X, g.W, (const void*)(aux), g.nw, g.M, (uint32_t)(g.N >> 4 | g.K >> 6 << 16) | (uint32_t)g.c_tiled << 31, g.xcd_tiles | g.xcd_more << 28 | (uint32_t)g.by_rows << 31, g.run, g.inv_run
+#define PF_HOT_IN(p)                                                                                                  \
+  p.X = X; p.W = W; p.nw = nw; p.M = M; p.N = (int)(nk & 0xffffu) * 16; p.K = (int)(nk >> 16 & 0x7fffu) * 64; p.c_tiled = (int)(nk >> 31);                  \
+  p.xcd_tiles = xcd & 0xfffffffu; p.xcd_more = xcd >> 28 & 7u; p.by_rows = (int)(xcd >> 31); p.run = run; p.inv_run = inv_run
 
 // Which tile (of MT x NT) a workgroup takes: {row tile, feature tile}.  Workgroups go round the eight XCDs, whose L2s are their
 // own, so each XCD gets a contiguous range of the tiles: of the feature tiles where the weights are more bytes than the rows - it then
@@ -164,7 +174,12 @@ __device__ __forceinline__ uint4 pf_norm8(const uint4& x, float r, const uint4& 
 // short block 0.5-1.7 us (16 positions: QKV 3.8 -> 5.5, W1 and W3 5.0 -> 5.5) and saves the norm's own of 3.4; repeated for every
 // tile of features it does not pay for longer ones.
 template <int EPI, bool DUAL, bool I8, int WAVES, int MB, int NB, bool NORM>
-__global__ __launch_bounds__(64 * WAVES) void pf_gemm_kernel(const PfGemm p, const void* __restrict__ W2, int c_tiled) {
+__global__ __launch_bounds__(64 * WAVES) void pf_gemm_kernel(PF_HOT, const PfGemm p0) {
+  PfGemm p = p0;
+  PF_HOT_IN(p);
+  if (EPI == PF_RESID) p.C = (void*)aux;
+  else if (NORM) p.ssq = (const float*)aux;
+  const char* W2 = (const char*)W + (size_t)p.N * p.K * (I8 ? 1 : 2);  // DUAL: the second matrix lies behind the first
   constexpr int TILE = MB * NB * 256;  // floats of one partial tile
   constexpr int PW = (DUAL ? 2 : 1) * TILE;
   __shared__ __align__(16) float part[WAVES * PW];
@@ -189,22 +204,13 @@ __global__ __launch_bounds__(64 * WAVES) void pf_gemm_kernel(const PfGemm p, con
   for (int j = 0; j < NB; ++j) {
     const size_t wo = (size_t)min((n0 >> 4) + j, NBL - 1) * nsteps * WB + lane * WL;
     wr[j] = (const char*)p.W + wo;
-    vr[j] = DUAL ? (const char*)W2 + wo : (const char*)p.W + wo;
+    vr[j] = (DUAL ? W2 : (const char*)p.W) + wo;
   }
   pf_floatx4 acc[NB][MB], acc2[NB][MB];
 #pragma unroll
   for (int i = 0; i < NB; ++i)
 #pragma unroll
     for (int j = 0; j < MB; ++j) { acc[i][j] = pf_floatx4{0.f, 0.f, 0.f, 0.f}; acc2[i][j] = acc[i][j]; }
-  // the residual values this thread will add to (its four outputs, see the epilogue) are requested with the first
-  // operands instead of after the last product; clamped to the matrix, unused where the thread has no output
-  uint2 old = make_uint2(0, 0);
-  PfRot rot = {};
-  {
-    const int em = min(m0 + 16 * (wave % MB) + l16, p.M - 1), en = min(n0 + 16 * (wave / MB % NB) + 4 * kg, p.N - 4);
-    if (EPI == PF_RESID) old = *reinterpret_cast<const uint2*>((const bf16_t*)p.C + (c_tiled ? pf_toff(em, en, p.N) : (size_t)em * p.ldc + en));
-    if (EPI == PF_QKV && p.rope_dim >= 2) rot = pf_rot(p.rope, p.pos0 + em, p.rope_dim, pf_part(p, min(n0 + 16 * (wave / MB % NB), p.N - 16)).dim + 4 * kg);
-  }
   uint4 xa[MB][2], wa[NB][2], va[NB][2], g[2];
   auto load = [&](int s) {
     const int k = s << 10;
@@ -221,10 +227,19 @@ __global__ __launch_bounds__(64 * WAVES) void pf_gemm_kernel(const PfGemm p, con
       if (NORM) g[h] = *reinterpret_cast<const uint4*>(p.nw + 64 * s + 16 * kg + 8 * h);
     }
   };
+  // The operands of the first step go out before anything else is asked for, then the residual values this thread will add to (its
+  // four outputs, see the epilogue), instead of after the last product; clamped to the matrix, unused where the thread has no output.
+  if (WAVES >= 8 && s0 < s1) load(s0);
+  if (WAVES >= 8) __builtin_amdgcn_sched_barrier(0);
+  uint2 old = make_uint2(0, 0);
+  PfRot rot = {};
+  {
+    const int em = min(m0 + 16 * (wave % MB) + l16, p.M - 1), en = min(n0 + 16 * (wave / MB % NB) + 4 * kg, p.N - 4);
+    if (EPI == PF_RESID) old = *reinterpret_cast<const uint2*>((const bf16_t*)p.C + (p.c_tiled ? pf_toff(em, en, p.N) : (size_t)em * p.N + en));
+    if (EPI == PF_QKV && p.rope_dim >= 2) rot = pf_rot(p.rope, p.pos0 + em, p.rope_dim, pf_part(p, min(n0 + 16 * (wave / MB % NB), p.N - 16)).dim + 4 * kg);
+  }
   float rf[MB];
-  if (NORM) {  // the operands of the first step are on their way meanwhile
-    if (s0 < s1) load(s0);
-    __builtin_amdgcn_sched_barrier(0);
+  if (NORM) {
     float ss[MB] = {};
     for (int i = kg; i < nsteps; i += 16) {
       float4 t[MB][4];
@@ -242,7 +257,7 @@ __global__ __launch_bounds__(64 * WAVES) void pf_gemm_kernel(const PfGemm p, con
     for (int j = 0; j < MB; ++j) rf[j] = 1.0f / sqrtf(rows_sum(ss[j]) / (float)p.K + p.eps);
   }
   for (int s = s0; s < s1; ++s) {
-    if (!NORM || s > s0) load(s);
+    if (WAVES < 8 || s > s0) load(s);
     if (I8) {
 #pragma unroll
       for (int j = 0; j < NB; ++j) {
@@ -319,7 +334,7 @@ __global__ __launch_bounds__(64 * WAVES) void pf_gemm_kernel(const PfGemm p, con
     pf_qkv_out(p, blk, m, kg, v, rot);
     return;
   }
-  bf16_t* c = (bf16_t*)p.C + (c_tiled ? pf_toff(m, n, p.N) : (size_t)m * p.ldc + n);  // n % 4 == 0: inside one piece
+  bf16_t* c = (bf16_t*)p.C + (p.c_tiled ? pf_toff(m, n, p.N) : (size_t)m * p.N + n);  // n % 4 == 0: inside one piece
   if (DUAL) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -344,7 +359,10 @@ __global__ __launch_bounds__(64 * WAVES) void pf_gemm_kernel(const PfGemm p, con
 // NBW / 2 blocks are features of the first matrix, the others the same features of the second.  The sums pass through
 // the wave's share of LDS, so that the epilogue is a loop over blocks.
 template <int EPI, bool DUAL, bool I8, int MBW, int NBW, int WM, int WN, int S, int KS>
-__global__ __launch_bounds__(256, 2) void pf_wide_kernel(const PfGemm p, const void* __restrict__ W2, int c_tiled) {
+__global__ __launch_bounds__(256, 2) void pf_wide_kernel(PF_HOT, const PfGemm p0) {
+  PfGemm p = p0;
+  PF_HOT_IN(p);
+  const char* W2 = (const char*)W + (size_t)p.N * p.K * (I8 ? 1 : 2);
   typedef WideTile<MBW, NBW, WM, WN, S, KS, I8> Tile;
   constexpr int NF = DUAL ? NBW / 2 : NBW, MB = Tile::MB, NB = NF * WN;  // feature blocks of a wave and of the tile
   __shared__ __align__(16) char lds[Tile::LDS];
@@ -358,7 +376,7 @@ __global__ __launch_bounds__(256, 2) void pf_wide_kernel(const PfGemm p, const v
   tile.begin(lds, wave, lane, [&](int i) { return (const char*)p.X + min(mb0 + i, MBL - 1) * xb; },
              [&](int i) {
                const int w = i / NBW, b = i % NBW;  // wave and block of the tile's i-th
-               return (const char*)(DUAL && b >= NF ? W2 : p.W) + min(nb0 + w * NF + b % NF, NBL - 1) * wb;
+               return (DUAL && b >= NF ? W2 : (const char*)p.W) + min(nb0 + w * NF + b % NF, NBL - 1) * wb;
              });
   const int Q = p.K / (32 * KS);
   tile.prologue(Q);
@@ -389,7 +407,7 @@ __global__ __launch_bounds__(256, 2) void pf_wide_kernel(const PfGemm p, const v
     for (int j = 0; j < MBW; ++j) {
       const int m = min(mw + 16 * j, p.M - 1);
       if (EPI == PF_QKV && p.rope_dim >= 2 && blk.part < 2) rot[j] = pf_rot(p.rope, p.pos0 + m, p.rope_dim, blk.dim + 4 * kg);
-      if (EPI == PF_RESID) old[j] = *reinterpret_cast<const uint2*>((const bf16_t*)p.C + (c_tiled ? pf_toff(m, n, p.N) : (size_t)m * p.ldc + n));
+      if (EPI == PF_RESID) old[j] = *reinterpret_cast<const uint2*>((const bf16_t*)p.C + (p.c_tiled ? pf_toff(m, n, p.N) : (size_t)m * p.N + n));
     }
 #pragma unroll
     for (int j = 0; j < MBW; ++j) {
@@ -419,7 +437,7 @@ __global__ __launch_bounds__(256, 2) void pf_wide_kernel(const PfGemm p, const v
           for (int r = 0; r < 4; ++r) v[r] = I8 ? t[(4 * kg + r) * 4] * sf : t[(4 * kg + r) * 4];
           pf_vt_out(p, blk, (mb0 + wm * MBW + j) * 16 + 4 * kg, l16, v);
         }
-      } else if (m < p.M) *reinterpret_cast<uint2*>((bf16_t*)p.C + (c_tiled ? pf_toff(m, n, p.N) : (size_t)m * p.ldc + n)) = make_uint2(f2bf2(v[0], v[1]), f2bf2(v[2], v[3]));
+      } else if (m < p.M) *reinterpret_cast<uint2*>((bf16_t*)p.C + (p.c_tiled ? pf_toff(m, n, p.N) : (size_t)m * p.N + n)) = make_uint2(f2bf2(v[0], v[1]), f2bf2(v[2], v[3]));
     }
   }
 }
@@ -433,12 +451,12 @@ static unsigned pf_set_order(PfGemm& g, int bm, int bn, size_t weight_bytes) {
 }
 
 template <int EPI, bool DUAL, bool I8>
-static int pf_wide(int tile, PfGemm& g, const void* W2, int c_tiled, hipStream_t st) {
+static int pf_wide(int tile, PfGemm& g, hipStream_t st) {
   const int bm = tile == WIDE_128 ? 128 : 64, bn = (tile == WIDE_64 ? 64 : 128) / (DUAL ? 2 : 1);
   const dim3 grid(pf_set_order(g, bm, bn, (size_t)g.N * g.K * ((DUAL ? 2 : 1) * (I8 ? 1 : 2))));
-  if (tile == WIDE_128) hipLaunchKernelGGL((pf_wide_kernel<EPI, DUAL, I8, 4, 4, 2, 2, I8 ? 3 : 4, I8 ? 2 : 1>), grid, dim3(256), 0, st, g, W2, c_tiled);
-  else if (tile == WIDE_64x128) hipLaunchKernelGGL((pf_wide_kernel<EPI, DUAL, I8, 4, 2, 1, 4, I8 ? 4 : 3, 2>), grid, dim3(256), 0, st, g, W2, c_tiled);
-  else hipLaunchKernelGGL((pf_wide_kernel<EPI, DUAL, I8, 2, 2, 2, 2, 4, 2>), grid, dim3(256), 0, st, g, W2, c_tiled);
+  if (tile == WIDE_128) hipLaunchKernelGGL((pf_wide_kernel<EPI, DUAL, I8, 4, 4, 2, 2, I8 ? 3 : 4, I8 ? 2 : 1>), grid, dim3(256), 0, st, PF_HOT_ARGS(g, nullptr), g);
+  else if (tile == WIDE_64x128) hipLaunchKernelGGL((pf_wide_kernel<EPI, DUAL, I8, 4, 2, 1, 4, I8 ? 4 : 3, 2>), grid, dim3(256), 0, st, PF_HOT_ARGS(g, nullptr), g);
+  else hipLaunchKernelGGL((pf_wide_kernel<EPI, DUAL, I8, 2, 2, 2, 2, 4, 2>), grid, dim3(256), 0, st, PF_HOT_ARGS(g, nullptr), g);
   HIP_TRY(hipGetLastError());
   return VUI_OK;
 }
@@ -661,7 +679,10 @@ __device__ __forceinline__ uint2 pf_read_tr(const char* lds) {
   return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) pf_s16x4*)lds));
 }
 template <int HD32>
-__global__ __launch_bounds__(64 * PfDirect<HD32>::WAVES) void pf_direct_attn_kernel(const PfDirectArgs a) {
+__global__ __launch_bounds__(64 * PfDirect<HD32>::WAVES) void pf_direct_attn_kernel(const bf16_t* q, const bf16_t* kc, const bf16_t* vc, int T, int nq,
+                                                                                    int nkv, int gsz, int pos0, int window, const PfDirectArgs a0) {
+  PfDirectArgs a = a0;
+  a.q = q; a.kc = kc; a.vc = vc; a.T = T; a.nq = nq; a.nkv = nkv; a.gsz = gsz; a.pos0 = pos0; a.window = window;  // (see PF_HOT)
   typedef PfDirect<HD32> P;
   constexpr int HD = P::HD, DT = P::DT, WAVES = P::WAVES;
   extern __shared__ __align__(16) char lds[];
@@ -825,7 +846,8 @@ template <int HD32> static int pf_direct_attn(PfDirectArgs& a, int H, hipStream_
   const int L = a.pos0 + a.T, keys = a.window > 0 && a.window + 48 < L ? a.window + 48 : L, n = (keys + 127) / 128;
   HIP_TRY(hipFuncSetAttribute((const void*)pf_direct_attn_kernel<HD32>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   const int splits = n > PF_SPLITS ? PF_SPLITS : n;
-  hipLaunchKernelGGL(pf_direct_attn_kernel<HD32>, dim3(H, (a.T + 15) / 16, splits), dim3(64 * PfDirect<HD32>::WAVES), lds, st, a);
+  hipLaunchKernelGGL(pf_direct_attn_kernel<HD32>, dim3(H, (a.T + 15) / 16, splits), dim3(64 * PfDirect<HD32>::WAVES), lds, st, a.q, a.kc, a.vc, a.T, a.nq,
+                     a.nkv, a.gsz, a.pos0, a.window, a);
   if (splits > 1) a.before += splits;
   return VUI_OK;
 }
@@ -901,10 +923,10 @@ static int pf_pick(int M, int N, int K, bool pair, bool i8) {
   return best;
 }
 
-// bf16 out, K split over the waves of a workgroup; W2 != nullptr: the SwiGLU pair; i8: int8 matrices with g.sc / g.sc2;
+// bf16 out, K split over the waves of a workgroup; DUAL: the SwiGLU pair, its second matrix behind g.W; i8: int8 matrices with g.sc / g.sc2;
 // g.ssq != nullptr: rows are normed on their way (short blocks)
 template <int EPI, bool DUAL, bool I8>
-static int pf_go(PfGemm& g, const void* W2, int c_tiled, hipStream_t st) {
+static int pf_go(PfGemm& g, hipStream_t st) {
   // Few tiles (short blocks): more waves, so that a wave's chain of dependent trips is one to three steps long, and 16
   // features per workgroup, so that more of the chip pulls weights.  us per launch, 32 x 32 and 4 waves / as chosen here:
   // 16 positions out_proj and W2 8.0 / 4.4, QKV 5.6 / 3.8, W1 and W3 5.9 / 5.0; whole pass of 16 positions 883 / 776
@@ -914,7 +936,7 @@ static int pf_go(PfGemm& g, const void* W2, int c_tiled, hipStream_t st) {
   const int mb = few && g.M <= 16 ? 1 : 2, nb = few ? 1 : 2;
   const unsigned tiles = pf_set_order(g, 16 * mb, 16 * nb, (size_t)g.N * g.K * ((DUAL ? 2 : 1) * (I8 ? 1 : 2))) + g.warm;
   constexpr int W = EPI == PF_RESID ? 16 : 12;
-#define PF_GO(WV, MB, NB, NORM) hipLaunchKernelGGL((pf_gemm_kernel<EPI, DUAL, I8, WV, MB, NB, NORM>), dim3(tiles), dim3(64 * (WV)), 0, st, g, W2, c_tiled)
+#define PF_GO(WV, MB, NB, NORM) hipLaunchKernelGGL((pf_gemm_kernel<EPI, DUAL, I8, WV, MB, NB, NORM>), dim3(tiles), dim3(64 * (WV)), 0, st, PF_HOT_ARGS(g, EPI == PF_RESID ? (const void*)g.C : (const void*)g.ssq), g)
   if constexpr (EPI != PF_RESID) {
     if (norm) {
       if (mb == 1) PF_GO(W, 1, 1, true);
@@ -932,11 +954,11 @@ static int pf_go(PfGemm& g, const void* W2, int c_tiled, hipStream_t st) {
   return VUI_OK;
 }
 template <int EPI, bool DUAL>
-static int pf_gemm4(PfGemm& g, const void* W2, int c_tiled, bool i8, hipStream_t st) {
-  if (g.K % 64 || g.N % 16 || g.M < 1 || g.N < 1 || (c_tiled && g.N % 64)) { vui_set_error("prefill GEMM: bad shape N=%d K=%d", g.N, g.K); return VUI_EINVAL; }
+static int pf_gemm4(PfGemm& g, bool i8, hipStream_t st) {
+  if (g.K % 64 || g.N % 16 || g.M < 1 || g.N < 1 || g.N >= 1 << 20 || g.K >= 1 << 21 || (g.c_tiled && g.N % 64)) { vui_set_error("prefill GEMM: bad shape N=%d K=%d", g.N, g.K); return VUI_EINVAL; }
   const int tile = g.ssq ? WIDE_NONE : pf_pick(g.M, g.N, g.K, DUAL, i8);
-  if (tile != WIDE_NONE) return i8 ? pf_wide<EPI, DUAL, true>(tile, g, W2, c_tiled, st) : pf_wide<EPI, DUAL, false>(tile, g, W2, c_tiled, st);
-  return i8 ? pf_go<EPI, DUAL, true>(g, W2, c_tiled, st) : pf_go<EPI, DUAL, false>(g, W2, c_tiled, st);
+  if (tile != WIDE_NONE) return i8 ? pf_wide<EPI, DUAL, true>(tile, g, st) : pf_wide<EPI, DUAL, false>(tile, g, st);
+  return i8 ? pf_go<EPI, DUAL, true>(g, st) : pf_go<EPI, DUAL, false>(g, st);
 }
 
 // Blocks of up to this many positions take the five-launch form.
@@ -1074,7 +1096,7 @@ int launch_prefill(const vui_config& c, const vui_weights& w, const void* tiled_
     if (tiny && pos0 > 0) { g.warm_from = win > 0 && pos0 > win ? pos0 - win : 0; g.warm = PF_WARM; }
     g.rope = layer_rope(c, w, l, &g.rope_dim);
     g.nq = nq; g.nkv = nkv; g.hd = hd; g.inv_hd = pf_inv(hd); g.pos0 = pos0; g.Lpad = Lpad;
-    if ((rc = pf_gemm4<PF_QKV, false>(g, nullptr, 0, i8, st))) return rc;
+    if ((rc = pf_gemm4<PF_QKV, false>(g, i8, st))) return rc;
     if (tiny) {
       da.kc = g.kc; da.vc = g.vc; da.window = win;
       switch (hd / 32) {
@@ -1096,18 +1118,18 @@ int launch_prefill(const vui_config& c, const vui_weights& w, const void* tiled_
       }
     }
     PfGemm wo{};
-    wo.X = att; wo.W = t_o; wo.C = x; wo.ldc = d; wo.M = T; wo.N = d; wo.K = nq; wo.sc = (const bf16_t*)lw.s_o;
+    wo.X = att; wo.W = t_o; wo.C = x; wo.c_tiled = tiny; wo.M = T; wo.N = d; wo.K = nq; wo.sc = (const bf16_t*)lw.s_o;
     if (tiny) wo.ssq_out = ssq;
-    if ((rc = pf_gemm4<PF_RESID, false>(wo, nullptr, tiny ? 1 : 0, i8, st))) return rc;
+    if ((rc = pf_gemm4<PF_RESID, false>(wo, i8, st))) return rc;
     PfGemm f1{};
-    f1.X = tiny ? x : xn; f1.W = t_1; f1.C = fa; f1.ldc = F; f1.M = T; f1.N = F; f1.K = d; f1.sc = (const bf16_t*)lw.s_1; f1.sc2 = (const bf16_t*)lw.s_3;
+    f1.X = tiny ? x : xn; f1.W = t_1; f1.C = fa; f1.c_tiled = 1; f1.M = T; f1.N = F; f1.K = d; f1.sc = (const bf16_t*)lw.s_1; f1.sc2 = (const bf16_t*)lw.s_3;
     if (tiny) { f1.ssq = ssq; f1.nw = (const bf16_t*)lw.mlp_norm; f1.eps = c.norm_eps; }
     else norm(lw.mlp_norm, xn, 1, nullptr);
-    if ((rc = pf_gemm4<PF_BF16, true>(f1, t_3, 1, i8, st))) return rc;  // written tiled: operand of W2
+    if ((rc = pf_gemm4<PF_BF16, true>(f1, i8, st))) return rc;  // written tiled: operand of W2
     PfGemm f2{};
-    f2.X = fa; f2.W = t_2; f2.C = x; f2.ldc = d; f2.M = T; f2.N = d; f2.K = F; f2.sc = (const bf16_t*)lw.s_2;
+    f2.X = fa; f2.W = t_2; f2.C = x; f2.c_tiled = tiny; f2.M = T; f2.N = d; f2.K = F; f2.sc = (const bf16_t*)lw.s_2;
     if (tiny) f2.ssq_out = ssq;
-    if ((rc = pf_gemm4<PF_RESID, false>(f2, nullptr, tiny ? 1 : 0, i8, st))) return rc;
+    if ((rc = pf_gemm4<PF_RESID, false>(f2, i8, st))) return rc;
   }
   norm(w.final_norm, (bf16_t*)out, 0, seq_lens + slot);
   HIP_TRY(hipGetLastError());
