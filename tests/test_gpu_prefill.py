@@ -203,6 +203,23 @@ def test_prefill_tiles_of_every_size(int8):
             assert rel_err(a, b) <= BF16_TOL, (T, rel_err(a, b))
 
 
+@pytest.mark.parametrize("T", [32, 33, 64])
+def test_more_tiles_than_compute_units(T):
+    """Two layers at Vui Nano dims: from 33 positions on a short block's QKV product is 288 tiles and takes eight waves per tile,
+    up to 32 it is 144 of twelve.  Against the position-by-position path, with the tolerance of the test above."""
+    d = O.Dims(n_layers=2)
+    m = make_model(d, O.synthetic_state_dict(d, seed=3), BF, int8=T == 64, max_seqlen=128)
+    m.decoder.allocate_flash_kv_cache(1, m.device, BF, max_seqlen=128)
+    x = (torch.randn(1, T, d.d_model, generator=torch.Generator().manual_seed(6)) * 0.08).to(BF).cuda()
+    outs = []
+    for minimum in (4, 10 ** 9):
+        m.decoder.flash_kv_caches[0].seq_lens.zero_()
+        m.decoder.PREFILL_MIN = minimum
+        outs.append((m.decoder.forward_flash(x, None), m.decoder._k[:, 0, :T].clone(), m.decoder._v[:, 0, :T].clone()))
+    for a, b in zip(*outs):
+        assert rel_err(a, b) <= BF16_TOL, rel_err(a, b)
+
+
 @pytest.mark.parametrize("int8", [False, True])
 def test_large_tiles_add_as_the_small_ones_do(int8):
     """Passes whose products take large tiles (the lengths choose all three for QKV and the pair, two for the others), some
