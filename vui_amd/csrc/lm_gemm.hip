@@ -183,8 +183,23 @@ static void lm_set_order(LmGemm& g, int MT, int NT, int band) {
   g.inv_tiles = lm_inv(band * MT); g.inv_band = lm_inv(band); g.inv_last = lm_inv(NT % band ? NT % band : band);
 }
 
+// The first fourteen words of a kernel's scalar arguments are in registers when it starts, a struct is a trip to memory (0.2-0.35 us of a
+// launch of 4-8): what the first loads need comes twice, ahead of the struct and in it.  aux0, aux1: of experts' products the number of
+// tiles and their experts, otherwise the sums of squares and the norm.  np: of the same, the entries' tiles.
+#define LM_HOT const void *X, const void *W, const void *aux0, const void *aux1, int M, uint32_t nk, uint32_t np_band, uint32_t inv_tiles, uint32_t inv_band, uint32_t inv_last
+#define LM_HOT_ARGS(g, moe)                                                                                                                 \
+  g.X, g.W, (moe) ? (const void*)g.n_tiles : (const void*)g.ssq, (moe) ? (const void*)g.tile_e : (const void*)g.norm, g.M,                   \
+      (uint32_t)(g.N >> 4 | g.K >> 6 << 17), (uint32_t)((moe) ? g.max_tiles : g.np | g.band << 16), g.inv_tiles, g.inv_band, g.inv_last
+#define LM_HOT_IN(p, moe)                                                                                    \
+  p.X = X; p.W = W; p.M = M; p.N = (int)(nk & 0x1ffffu) * 16; p.K = (int)(nk >> 17) * 64;                    \
+  p.inv_tiles = inv_tiles; p.inv_band = inv_band; p.inv_last = inv_last;                                     \
+  if (moe) { p.n_tiles = (const int32_t*)aux0; p.tile_e = (const int32_t*)aux1; p.max_tiles = (int)np_band; } \
+  else { p.ssq = (const float*)aux0; p.norm = (const float*)aux1; p.np = (int)(np_band & 0xffffu); p.band = (int)(np_band >> 16); }
+
 template <typename T, int MB, int NB, int WAVES, int EPI>
-__global__ __launch_bounds__(64 * WAVES) void lm_gemm_kernel(const LmGemm p) {
+__global__ __launch_bounds__(64 * WAVES, sizeof(T) == 2 && MB == 1 && NB < 3 ? 4 : 1) void lm_gemm_kernel(LM_HOT, const LmGemm p0) {
+  LmGemm p = p0;
+  LM_HOT_IN(p, EPI == LM_MOE_UP || EPI == LM_MOE_DOWN);
   constexpr bool SCALED = EPI == LM_IN_ATTN || EPI == LM_IN_GRU_STEP || EPI == LM_IN_GRU_SEQ || EPI == LM_LOGITS;
   constexpr bool GRU = EPI == LM_IN_GRU_STEP || EPI == LM_IN_GRU_SEQ;
   constexpr bool LOGITS = EPI == LM_LOGITS || EPI == LM_HEAD, MOE = EPI == LM_MOE_UP || EPI == LM_MOE_DOWN;
@@ -193,13 +208,13 @@ __global__ __launch_bounds__(64 * WAVES) void lm_gemm_kernel(const LmGemm p) {
   __shared__ float srow[MB * 16];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int l16 = lane & 15, kg = lane >> 4;
-  const int MT = MOE ? p.max_tiles : (p.M + 16 * MB - 1) / (16 * MB);
+  const int MT = MOE ? p.max_tiles : MB == 1 ? 1 : (p.M + 16 * MB - 1) / (16 * MB);  // one block of rows: 16 at most
   // tiles of an expert that share features run on one XCD, whose cache then holds those weights: workgroup i is on XCD i % 8
   int t, nt;
   if (MOE) {
     t = ((int)blockIdx.x >> 3) % MT; nt = ((int)blockIdx.x >> 3) / MT * 8 + ((int)blockIdx.x & 7);
-  } else if (MB == 1) {  // one tile of rows, mostly
-    t = (int)blockIdx.x % MT; nt = (int)blockIdx.x / MT;
+  } else if (MB == 1) {
+    t = 0; nt = (int)blockIdx.x;
   } else {
     lm_tile_at(p, blockIdx.x, MT, ((p.N >> 4) + NB - 1) / NB, t, nt);
   }
@@ -235,7 +250,27 @@ __global__ __launch_bounds__(64 * WAVES) void lm_gemm_kernel(const LmGemm p) {
   for (int i = 0; i < NB; ++i)
     wr[i] = (const T*)p.W + wz + (size_t)min(nb0 + i, NBL - 1) * nsteps * 1024 + lane * EP;
 
-  // What the scale and the epilogue of this wave's first unit will need is requested now, ahead of the operands:
+  // U steps' loads go out together (a step beyond the wave's last re-reads that one and is not multiplied); the first ones now
+  constexpr int U = WAVES >= 8 && sizeof(T) == 2 ? 4 : 1;
+  constexpr bool EARLY = WAVES >= 8 && sizeof(T) == 2;
+  uint4 xa[U][MB][P], wa[U][NB][P];
+  auto load = [&](int s) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const size_t o = (size_t)min(s + u, s1 - 1) * 1024;
+#pragma unroll
+      for (int h = 0; h < P; ++h) {
+#pragma unroll
+        for (int i = 0; i < NB; ++i) wa[u][i][h] = *reinterpret_cast<const uint4*>(wr[i] + o + 64 * EP * h);
+#pragma unroll
+        for (int j = 0; j < MB; ++j) xa[u][j][h] = *reinterpret_cast<const uint4*>(xr[j] + o + 64 * EP * h);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  if (EARLY && s0 < s1) load(s0);
+
+  // What the scale and the epilogue of this wave's first unit will need is requested now as well:
   // fetched where it is used, it would be a chain of dependent loads behind the last product.
   // Scale: TPR neighbouring threads add up one row's sums of squares, in a fixed order.
   constexpr int TPR = WAVES * 64 / (MB * 16) > 64 ? 64 : WAVES * 64 / (MB * 16), NSQ = 4;
@@ -271,22 +306,8 @@ __global__ __launch_bounds__(64 * WAVES) void lm_gemm_kernel(const LmGemm p) {
   for (int i = 0; i < NB; ++i)
 #pragma unroll
     for (int j = 0; j < MB; ++j) acc[i][j] = tl_f32x4{0.f, 0.f, 0.f, 0.f};
-  // U steps' loads go out together (a step beyond the wave's last re-reads that one and is not multiplied)
-  constexpr int U = WAVES >= 8 && sizeof(T) == 2 ? 4 : 1;
   for (int s = s0; s < s1; s += U) {
-    uint4 xa[U][MB][P], wa[U][NB][P];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const size_t o = (size_t)min(s + u, s1 - 1) * 1024;
-#pragma unroll
-      for (int h = 0; h < P; ++h) {
-#pragma unroll
-        for (int i = 0; i < NB; ++i) wa[u][i][h] = *reinterpret_cast<const uint4*>(wr[i] + o + 64 * EP * h);
-#pragma unroll
-        for (int j = 0; j < MB; ++j) xa[u][j][h] = *reinterpret_cast<const uint4*>(xr[j] + o + 64 * EP * h);
-      }
-    }
-    __builtin_amdgcn_sched_barrier(0);
+    if (!EARLY || s > s0) load(s);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if (s + u >= s1) break;  // uniform
@@ -355,7 +376,9 @@ __global__ __launch_bounds__(64 * WAVES) void lm_gemm_kernel(const LmGemm p) {
 // G = 2: eight waves, each half of them with half of K and stages of its own, for tiles that are alone on their CU: a step of
 // such a tile is a chain of barrier, LDS reads and products, and two chains side by side take little longer than one.
 template <int EPI, int MBW, int NBW, int WM, int WN, int S, int KS, int G>
-__global__ __launch_bounds__(256 * G, 2) void lm_wide_kernel(const LmGemm p) {
+__global__ __launch_bounds__(256 * G, 2) void lm_wide_kernel(LM_HOT, const LmGemm p0) {
+  LmGemm p = p0;
+  LM_HOT_IN(p, EPI == LM_MOE_UP || EPI == LM_MOE_DOWN);
   constexpr bool SCALED = EPI == LM_IN_ATTN || EPI == LM_IN_GRU_SEQ;
   constexpr bool GRU = EPI == LM_IN_GRU_SEQ, MOE = EPI == LM_MOE_UP || EPI == LM_MOE_DOWN;
   typedef WideTile<MBW, NBW, WM, WN, S, KS> Tile;
@@ -392,13 +415,13 @@ __global__ __launch_bounds__(256 * G, 2) void lm_wide_kernel(const LmGemm p) {
   const int mb0 = t * MB, nb0 = nt * NB, m0 = mb0 * 16;
   const int Q = p.K / (32 * KS);  // steps
   const size_t wz = MOE ? (size_t)p.tile_e[t] * p.wz : head * (val ? p.wz_v : p.wz);
-  const char* W = (const char*)(val ? p.w_v : p.W);
+  const char* weights = (const char*)(val ? p.w_v : p.W);
 
   const int n64 = p.K >> 6, mid = G == 2 ? (n64 >> 1) * 2 / KS : 0, first = half * mid, mine = G == 1 ? Q : half ? Q - mid : mid;
   Tile tile;
   tile.begin(lds + half * Tile::LDS, wave, lane,
              [&](int i) { return (const char*)p.X + ((size_t)(MOE ? mb0 + i : min(mb0 + i, MBL - 1)) * Q + first) * (KS * 1024); },
-             [&](int i) { return W + wz * 2 + ((size_t)min(nb0 + i, NBL - 1) * Q + first) * (KS * 1024); });
+             [&](int i) { return weights + wz * 2 + ((size_t)min(nb0 + i, NBL - 1) * Q + first) * (KS * 1024); });
   tile.prologue(mine);
 
   if (SCALED && half == 0) {
@@ -556,7 +579,7 @@ static int go_wide(LmGemm g, int nz, hipStream_t st) {
   if (strided) g.band = 0;
   else lm_set_order(g, MT, NT, lm_band(MT, NT, MBW * WM, NBW * WN));
   const int tiles = moe ? g.max_tiles * ((NT + 7) & ~7) : MT * (strided ? (NT + 7) & ~7 : NT);
-  hipLaunchKernelGGL((lm_wide_kernel<EPI, MBW, NBW, WM, WN, S, KS, G>), dim3((unsigned)tiles, 1, nz), dim3(256 * G), 0, st, g);
+  hipLaunchKernelGGL((lm_wide_kernel<EPI, MBW, NBW, WM, WN, S, KS, G>), dim3((unsigned)tiles, 1, nz), dim3(256 * G), 0, st, LM_HOT_ARGS(g, moe), g);
   HIP_TRY(hipGetLastError());
   return VUI_OK;
 }
@@ -568,7 +591,7 @@ static int go(LmGemm g, int nz, hipStream_t st) {
   const int mt = (g.M + 16 * MB - 1) / (16 * MB);
   lm_set_order(g, mt, nt, lm_band(mt, nt, MB, NB));
   const int tiles = moe ? g.max_tiles * ((nt + 7) & ~7) : mt * nt;
-  hipLaunchKernelGGL((lm_gemm_kernel<T, MB, NB, WAVES, EPI>), dim3((unsigned)tiles, 1, nz), dim3(64 * WAVES), 0, st, g);
+  hipLaunchKernelGGL((lm_gemm_kernel<T, MB, NB, WAVES, EPI>), dim3((unsigned)tiles, 1, nz), dim3(64 * WAVES), 0, st, LM_HOT_ARGS(g, moe), g);
   HIP_TRY(hipGetLastError());
   return VUI_OK;
 }
@@ -657,7 +680,7 @@ static int pick(int epi, const LmGemm& g, int nz, hipStream_t st) {
 }
 
 int launch_lm_gemm(int dtype, int epi, const LmGemm& g, int nz, hipStream_t st) {
-  if (g.M < 1 || g.N < 16 || (g.N & 15) || g.K < 64 || (g.K & 63) || nz < 1) {
+  if (g.M < 1 || g.N < 16 || (g.N & 15) || g.K < 64 || (g.K & 63) || nz < 1 || g.N >= 1 << 21 || g.K >= 1 << 21) {
     vui_set_error("lm gemm: bad shape M=%d N=%d K=%d", g.M, g.N, g.K);
     return VUI_EINVAL;
   }
