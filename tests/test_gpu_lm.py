@@ -150,6 +150,23 @@ def test_batch_of_unequal_rows_against_each_alone(dt):
         assert len(got[i]) >= 5 and U.err(torch.stack(got[i]), ref) < U.TOL[dt], i
 
 
+@pytest.mark.parametrize("rows, heads, rank, rot", [(5, 3, 56, 8), (5, 17, 130, 40), (4, 17, 130, 40), (6, 9, 500, 8)])
+def test_pieces_of_two_tiles(rows, heads, rank, rot):
+    """More than four rows take pieces of 64 keys and more, two tiles of 32 side by side: lengths around the borders of tiles and pieces,
+    more heads than one block of sixteen, one and two blocks of rotated dims."""
+    cfg = U.config([U.attn(heads=heads, dim=16, rot_dim=rot, vdim=16, kv_rank=rank)], ff=None)
+    sd = U.weights(cfg, 16)
+    eng = U.engine(cfg, sd, BF16, max_rows=rows, max_seq=2304)
+    lens = [30, 63, 95, 127, 62, 2079][:rows - 1] + [2079]  # 2080 keys over 32 pieces: 65, rounded up to 96 each
+    seqs = [U.tokens(n + 4, cfg["vocab"], 30 + n) for n in lens]
+    held = [eng.new_row() for _ in lens]
+    for row, s, n in zip(held, seqs, lens):
+        row.extend(s[:n], [])
+    got = [eng.decode_step(held, torch.tensor([s[n + t] for s, n in zip(seqs, lens)], device="cuda")).clone() for t in range(4)]
+    for i, (s, n) in enumerate(zip(seqs, lens)):
+        assert U.err(torch.stack([g[i] for g in got]), O.forward(cfg, sd, s)[n:]) < U.TOL[BF16], (i, n)
+
+
 @BOTH
 def test_slots_used_again(dt):
     """A slot that held a long sequence serves short ones; nothing of the old keys, latents or state shows."""

@@ -52,10 +52,11 @@ __global__ __launch_bounds__(GLA_THREADS) void gla_step_kernel(const GlaArgs p) 
   const int c4 = (tid % vq) * 4, r0 = tid / vq;
   const bool work = r0 < per;
   const int m0 = p.rows.seq ? 0 : blockIdx.y, m1 = p.rows.seq ? p.M : m0 + 1;
-  const int slot = lm_slot(p.rows, m0);
+  const int2 at = lm_where(p.rows, m0);
+  const int slot = at.x;
   float* S = p.state + ((size_t)slot * p.heads + h) * D * V;
   for (int m = m0; m < m1; ++m) {
-    const bool fresh = lm_pos(p.rows, m, slot) <= 0;
+    const bool fresh = at.y + m - m0 <= 0;
     tl_f32x4 s[GLA_PRE];  // the first rows are on their way while the decays are computed
 #pragma unroll
     for (int i = 0; i < GLA_PRE; ++i) s[i] = *reinterpret_cast<const tl_f32x4*>(S + (size_t)min(r0 + i * per, D - 1) * V + c4);

@@ -23,7 +23,8 @@ __device__ __forceinline__ void latent_append_row(const LatentArgs& p, int m) {
   }
   ss = wave_sum(ss);
   const float r = 1.0f / sqrtf(ss / (float)p.rank + p.eps);
-  const int slot = lm_slot(p.rows, m), pos = lm_pos(p.rows, m, slot);
+  const int2 at = lm_where(p.rows, m);
+  const int slot = at.x, pos = at.y;
   if (pos < 0 || pos >= p.rows.S) return;
   T* dst = (T*)p.c_cache + (size_t)slot * p.d.s64 * p.d.rank64;
   for (int k = lane * 4; k < p.d.rank16; k += 256) {
@@ -42,7 +43,10 @@ __global__ __launch_bounds__(256) void latent_append_kernel(const LatentArgs p) 
 
 // ---- queries into the latent space: qlat[h] (M x rank) = qu[h] (M x dim) W_uk[h]; a wave owns 16 latent columns ----
 template <typename T>
-__global__ __launch_bounds__(256) void latent_query_kernel(const LatentArgs p) {
+__global__ __launch_bounds__(256) void latent_query_kernel(const void* w_uk_t, const void* qu, const float* craw, size_t qu_z, int heads, int M, int dim64, int rank16,
+                                                           const LatentArgs p0) {
+  LatentArgs p = p0;  // what the first loads need is in registers (see lm_gemm.hip)
+  p.w_uk_t = w_uk_t; p.qu = qu; p.craw = craw; p.qu_z = qu_z; p.heads = heads; p.M = M; p.d.dim64 = dim64; p.d.rank16 = rank16;
   constexpr int EP = Tl<T>::EP, P = 16 / EP;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int h = blockIdx.x, mt = blockIdx.z;
@@ -70,12 +74,13 @@ __global__ __launch_bounds__(256) void latent_query_kernel(const LatentArgs p) {
   const int m = mt * 16 + (lane & 15);
   if (m >= p.M) return;
   const float v[4] = {acc[0], acc[1], acc[2], acc[3]};
-  Tl<T>::st4((T*)p.qlat + h * p.qlat_z + tl_off<T>(m, nb * 16 + 4 * (lane >> 4), p.d.rank64), v);
+  Tl<T>::st4((T*)p.qlat + (size_t)m * p.d.heads16 * p.d.rank64 + tl_off<T>(h, nb * 16 + 4 * (lane >> 4), p.d.rank64), v);
 }
 
 // A row that sees len keys is cut into pieces of this many (whole 32-key tiles), at most ns of them.  With more than
 // four rows a piece has two tiles at least: there are pieces enough, and fewer are merged faster.
-__device__ __forceinline__ int latent_chunk(int len, int ns, int M) { return max(((len + ns - 1) / ns + 31) & ~31, M > 4 ? 64 : 32); }
+__host__ __device__ __forceinline__ int latent_least(int M) { return M > 4 ? 64 : 32; }
+__device__ __forceinline__ int latent_chunk(int len, int ns, int M) { return max(((len + ns - 1) / ns + 31) & ~31, latent_least(M)); }
 // keys [lo, hi) of piece sp
 __device__ __forceinline__ void latent_range(int len, int ns, int M, int sp, int& lo, int& hi) {
   const int chunk = latent_chunk(len, ns, M);
@@ -94,13 +99,13 @@ __global__ __launch_bounds__(256) void latent_attn_kernel(const LatentArgs p) {
   constexpr int EP = Tl<T>::EP;
   const int m = blockIdx.x, h = blockIdx.y, sp = blockIdx.z, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int R = p.d.rank64, RR = p.d.rot32;
-  const int slot = lm_slot(p.rows, m);
-  const int len = min(max(lm_pos(p.rows, m, slot) + 1, 1), p.rows.S);
+  const int2 at = lm_where(p.rows, m);
+  const int slot = at.x, len = min(max(at.y + 1, 1), p.rows.S);
   int lo, hi;
   latent_range(len, p.n_splits, p.M, sp, lo, hi);
   if (lo >= hi) return;  // no such piece: latent_value_kernel does not look for it
   for (int k = tid; k < R + RR; k += 256)
-    lq[k] = k < R ? (k < p.d.rank16 ? El<T>::ld((const T*)p.qlat + h * p.qlat_z + tl_off<T>(m, k, R)) : 0.f)
+    lq[k] = k < R ? (k < p.d.rank16 ? El<T>::ld((const T*)p.qlat + (size_t)m * p.d.heads16 * R + tl_off<T>(h, k, R)) : 0.f)
                   : (k - R < p.d.rot16 ? El<T>::ld((const T*)p.qr + h * p.qr_z + tl_off<T, 32>(m, k - R, RR)) : 0.f);
   const T* cc = (const T*)p.c_cache + (size_t)slot * p.d.s64 * R;
   const T* kc = (const T*)p.kr_cache + (size_t)slot * p.d.s64 * RR;
@@ -157,73 +162,99 @@ __global__ __launch_bounds__(256) void latent_attn_kernel(const LatentArgs p) {
 }
 
 // ---- attention in the latent space on the matrix cores (bf16): one workgroup per (row, 16 heads, split) ----
-// All heads read the same latents, so 32 keys are staged in LDS once and serve 16 heads.  Scores^T (keys x heads) =
-// [c | k_rot] [q_lat | q_rot]^T, the four waves dealing key tile and half of the columns between them; every wave then
+// All heads read the same latents, so 32 KT keys are staged in LDS once and serve 16 heads.  Scores^T (keys x heads) =
+// [c | k_rot] [q_lat | q_rot]^T, the four waves dealing key tiles (and, KT = 1, half of the columns) between them; every wave then
 // has all scores of its lane's head and averages a quarter of the latent columns: out^T (columns x heads) = C^T p^T,
-// the weights as a bf16 pair (value and remainder).  The transposed operand is gathered from LDS element by element.
-// RK = rank64 / 64, RB = rot32 / 32.
-template <int RK, int RB>
-__global__ __launch_bounds__(256) void latent_attn_mfma_kernel(const LatentArgs p) {
+// the weights as a bf16 pair (value and remainder).  The transposed operand comes from LDS by ds_read_b64_tr_b16.
+// RK = rank64 / 64, RB = rot32 / 32.  Pieces of 32 keys (up to four rows) take KT = 1, longer ones two tiles side by side instead of one
+// after the other.  Bound by its chain: length, keys, LDS, scores, LDS, weights, average.  8 heads of rank 512, 16 rows behind up to 1400
+// keys, us per launch: queries of a head each, values element by element, tile by tile 10.9, so 8.8; 16 heads 13.6 / 9.0 (of it two tiles
+// side by side 0.4 us).
+template <int RK, int RB, int KT>
+__global__ __launch_bounds__(256, 2) void latent_attn_mfma_kernel(int2* where, const void* c_cache, const void* kr_cache, const void* qlat, uint32_t m_ns,
+                                                                  int S, int s64, int heads16, const LatentArgs p0) {
+  LatentArgs p = p0;  // what the first loads need is in registers (see lm_gemm.hip)
+  p.rows.where = where; p.c_cache = const_cast<void*>(c_cache); p.kr_cache = const_cast<void*>(kr_cache); p.qlat = const_cast<void*>(qlat);
+  p.M = (int)(m_ns & 0xffffffu); p.n_splits = (int)(m_ns >> 24); p.rows.S = S; p.d.s64 = s64; p.d.heads16 = heads16;
   constexpr int CT = RK * 2048, RT = RB * 1024;  // elements of the staged tiles (32 keys)
-  extern __shared__ __align__(16) bf16_t tile[];  // 2 x (CT + RT)
+  constexpr int NT = 2 * KT, BUFS = KT == 1 ? 2 : 1, BUF = KT * (CT + RT);
+  extern __shared__ __align__(16) bf16_t tile[];  // BUFS x KT x (CT + RT)
   __shared__ __align__(16) float sco[4][64 * 4];
   const int m = blockIdx.x, sp = blockIdx.z, tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l16 = lane & 15, kg = lane >> 4;
-  const int t = wave & 1, half = wave >> 1;
+  const int t = wave % NT, half = wave / NT;  // KT = 2: every wave takes both halves
   const int head = blockIdx.y * 16 + l16, hq = min(head, p.heads - 1);
-  const int slot = lm_slot(p.rows, m);
-  const int len = min(max(lm_pos(p.rows, m, slot) + 1, 1), p.rows.S);
+  const int2 at = lm_where(p.rows, m);
+  const int slot = at.x, len = min(max(at.y + 1, 1), p.rows.S);
   int lo, hi;
   latent_range(len, p.n_splits, p.M, sp, lo, hi);
   const tl_u32x4* cc = reinterpret_cast<const tl_u32x4*>((const bf16_t*)p.c_cache + (size_t)slot * p.d.s64 * (RK * 64));
   const tl_u32x4* kc = reinterpret_cast<const tl_u32x4*>((const bf16_t*)p.kr_cache + (size_t)slot * p.d.s64 * (RB * 32));
   if (lo >= hi) return;  // no such piece
-  // 32 keys are one contiguous run of either cache
-  tl_u32x4 rc[RK], rr;
-#define LAT_FETCH(j)                                                                            \
-  {                                                                                             \
-    const size_t jt = (size_t)((j) >> 5);                                                       \
-    _Pragma("unroll") for (int i = 0; i < RK; ++i) rc[i] = cc[jt * (CT / 8) + tid + 256 * i];   \
-    rr = kc[jt * (RT / 8) + min(tid, RT / 8 - 1)];                                              \
-  }
-#define LAT_STAGE(dst)                                                                          \
-  {                                                                                             \
-    tl_u32x4* sd = reinterpret_cast<tl_u32x4*>(dst);                                                  \
-    _Pragma("unroll") for (int i = 0; i < RK; ++i) sd[tid + 256 * i] = rc[i];                   \
-    if (tid < RT / 8) sd[CT / 8 + tid] = rr;                                                    \
-  }
-  LAT_FETCH(lo);
-  // this wave's columns: piece `half` of every latent block, and a block of the rotated part (one wave pair without, RB = 1)
-  const bool rot = RB == 2 || half == 0;
-  uint4 qf[RK + 1];
+  // 32 keys are one contiguous run of either cache; a tile behind the piece's last re-reads that one, and its keys weigh nothing
+  tl_u32x4 rc[KT][RK], rr[KT];
+  auto fetch = [&](int j) {
+#pragma unroll
+    for (int k = 0; k < KT; ++k) {
+      const size_t jt = (size_t)min((j >> 5) + k, (hi - 1) >> 5);
+#pragma unroll
+      for (int i = 0; i < RK; ++i) rc[k][i] = cc[jt * (CT / 8) + tid + 256 * i];
+      rr[k] = kc[jt * (RT / 8) + min(tid, RT / 8 - 1)];
+    }
+  };
+  auto stage = [&](bf16_t* dst) {
+    tl_u32x4* sd = reinterpret_cast<tl_u32x4*>(dst);
+#pragma unroll
+    for (int k = 0; k < KT; ++k) {
+#pragma unroll
+      for (int i = 0; i < RK; ++i) sd[k * ((CT + RT) / 8) + tid + 256 * i] = rc[k][i];
+      if (tid < RT / 8) sd[k * ((CT + RT) / 8) + CT / 8 + tid] = rr[k];
+    }
+  };
+  fetch(lo);
+  // this wave's columns: of every latent block piece `half` (or both), and a block of the rotated part (KT = 1: of one wave pair
+  // without, RB = 1)
+  const bool rot = KT == 2 || RB == 2 || half == 0;
+  uint4 qf[KT][RK], qr[KT == 2 ? RB : 1];
   const int qrow = ((m & 15) + 16 * kg) * 8;
 #pragma unroll
-  for (int i = 0; i < RK; ++i)
-    qf[i] = *reinterpret_cast<const uint4*>((const bf16_t*)p.qlat + hq * p.qlat_z + ((size_t)(m >> 4) * RK + i) * 1024 + half * 512 + qrow);
-  qf[RK] = *reinterpret_cast<const uint4*>((const bf16_t*)p.qr + hq * p.qr_z + ((size_t)(m >> 4) * RB + (RB == 2 ? half : 0)) * 512 + qrow);
+  for (int k = 0; k < KT; ++k)
+#pragma unroll
+    for (int i = 0; i < RK; ++i)
+      qf[k][i] = *reinterpret_cast<const uint4*>((const bf16_t*)p.qlat + ((size_t)m * (p.d.heads16 >> 4) + blockIdx.y) * RK * 1024 + i * 1024 + (KT == 2 ? k : half) * 512 + lane * 8);
+#pragma unroll
+  for (int k = 0; k < (KT == 2 ? RB : 1); ++k)
+    qr[k] = *reinterpret_cast<const uint4*>((const bf16_t*)p.qr + hq * p.qr_z + ((size_t)(m >> 4) * RB + (KT == 2 ? k : RB == 2 ? half : 0)) * 512 + qrow);
   tl_f32x4 acc[RK];
 #pragma unroll
   for (int i = 0; i < RK; ++i) acc[i] = tl_f32x4{0.f, 0.f, 0.f, 0.f};
   float m_run = -INFINITY, l_run = 0.f;
-  LAT_STAGE(tile);
+  stage(tile);
   __syncthreads();
   int buf = 0;
-  for (int j0 = lo; j0 < hi; j0 += 32) {
-    const bf16_t* cur = tile + buf * (CT + RT);
-    const bool more = j0 + 32 < hi;
-    LAT_FETCH(more ? j0 + 32 : j0);
+  for (int j0 = lo; j0 < hi; j0 += 32 * KT) {
+    const bf16_t* cur = tile + buf * BUF;
+    const bool more = j0 + 32 * KT < hi;
+    if (more) fetch(j0 + 32 * KT);
     tl_f32x4 s = {0.f, 0.f, 0.f, 0.f};
+    const bf16_t* mine = cur + (t >> 1) * (CT + RT);  // tile of 16 keys t
 #pragma unroll
-    for (int i = 0; i < RK; ++i) s = Tl<bf16_t>::mma(*reinterpret_cast<const uint4*>(cur + (t * RK + i) * 1024 + half * 512 + lane * 8), qf[i], s);
+    for (int k = 0; k < KT; ++k)
+#pragma unroll
+      for (int i = 0; i < RK; ++i)
+        s = Tl<bf16_t>::mma(*reinterpret_cast<const uint4*>(mine + ((t & 1) * RK + i) * 1024 + (KT == 2 ? k : half) * 512 + lane * 8), qf[k][i], s);
     if (rot)  // uniform over the wave
-      s = Tl<bf16_t>::mma(*reinterpret_cast<const uint4*>(cur + CT + (t * RB + (RB == 2 ? half : 0)) * 512 + lane * 8), qf[RK], s);
-    *reinterpret_cast<tl_f32x4*>(&sco[half * 2 + t][lane * 4]) = s;
+#pragma unroll
+      for (int k = 0; k < (KT == 2 ? RB : 1); ++k)
+        s = Tl<bf16_t>::mma(*reinterpret_cast<const uint4*>(mine + CT + ((t & 1) * RB + (KT == 2 ? k : RB == 2 ? half : 0)) * 512 + lane * 8), qr[k], s);
+    *reinterpret_cast<tl_f32x4*>(&sco[half * NT + t][lane * 4]) = s;
     __syncthreads();
     // keys j0 + 16 u + 4 kg + r of this lane's head
-    float sv[8], mx = -INFINITY;
+    float sv[4 * NT], mx = -INFINITY;
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const tl_f32x4 a = *reinterpret_cast<const tl_f32x4*>(&sco[u][lane * 4]) + *reinterpret_cast<const tl_f32x4*>(&sco[2 + u][lane * 4]);
+    for (int u = 0; u < NT; ++u) {
+      tl_f32x4 a = *reinterpret_cast<const tl_f32x4*>(&sco[u][lane * 4]);
+      if (KT == 1) a += *reinterpret_cast<const tl_f32x4*>(&sco[(2 + u) & 3][lane * 4]);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const float v = j0 + 16 * u + 4 * kg + r < hi ? a[r] * p.scale : -INFINITY;
@@ -234,33 +265,38 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(const LatentArgs 
     mx = rows_max(mx);
     const float m_new = fmaxf(m_run, mx);  // finite: key j0 is in range
     const float alpha = expf(m_run - m_new);
-    float pv[8], ps = 0.f;
+    float pv[4 * NT], ps = 0.f;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) { pv[e] = expf(sv[e] - m_new); ps += pv[e]; }
+    for (int e = 0; e < 4 * NT; ++e) { pv[e] = expf(sv[e] - m_new); ps += pv[e]; }
     l_run = l_run * alpha + ps;
     m_run = m_new;
-    uint4 hi4, lo4;
-    hi4.x = f2bf2(pv[0], pv[1]); hi4.y = f2bf2(pv[2], pv[3]); hi4.z = f2bf2(pv[4], pv[5]); hi4.w = f2bf2(pv[6], pv[7]);
-    lo4.x = f2bf2(pv[0] - bf_lo(hi4.x), pv[1] - bf_hi(hi4.x)); lo4.y = f2bf2(pv[2] - bf_lo(hi4.y), pv[3] - bf_hi(hi4.y));
-    lo4.z = f2bf2(pv[4] - bf_lo(hi4.z), pv[5] - bf_hi(hi4.z)); lo4.w = f2bf2(pv[6] - bf_lo(hi4.w), pv[7] - bf_hi(hi4.w));
+    uint4 hi4[KT], lo4[KT];
+#pragma unroll
+    for (int k = 0; k < KT; ++k) {
+      const float* w = pv + 8 * k;
+      uint4 &h = hi4[k], &l = lo4[k];
+      h.x = f2bf2(w[0], w[1]); h.y = f2bf2(w[2], w[3]); h.z = f2bf2(w[4], w[5]); h.w = f2bf2(w[6], w[7]);
+      l.x = f2bf2(w[0] - bf_lo(h.x), w[1] - bf_hi(h.x)); l.y = f2bf2(w[2] - bf_lo(h.y), w[3] - bf_hi(h.y));
+      l.z = f2bf2(w[4] - bf_lo(h.z), w[5] - bf_hi(h.z)); l.w = f2bf2(w[6] - bf_lo(h.w), w[7] - bf_hi(h.w));
+    }
+    // 16 columns of block i, column group `wave`: column l16 of keys 4 kg + r and 16 + 4 kg + r; the lane reads four columns of a key
+    const bf16_t* from = cur + (l16 >> 1 & 1) * 512 + (4 * kg + (l16 >> 2) + 16 * wave) * 8 + (l16 & 1) * 4;
 #pragma unroll
     for (int i = 0; i < RK; ++i) {
-      // 16 columns of block i, column group `wave`: column l16, the lane's eight keys
-      const bf16_t* q = cur + i * 1024 + (l16 >> 3) * 512 + (4 * kg + 16 * wave) * 8 + (l16 & 7);
-      uint4 v;
-      v.x = (uint32_t)q[0] | ((uint32_t)q[8] << 16);
-      v.y = (uint32_t)q[16] | ((uint32_t)q[24] << 16);
-      const bf16_t* q1 = q + RK * 1024;
-      v.z = (uint32_t)q1[0] | ((uint32_t)q1[8] << 16);
-      v.w = (uint32_t)q1[16] | ((uint32_t)q1[24] << 16);
 #pragma unroll
       for (int r = 0; r < 4; ++r) acc[i][r] *= alpha;
-      acc[i] = Tl<bf16_t>::mma(v, hi4, acc[i]);
-      acc[i] = Tl<bf16_t>::mma(v, lo4, acc[i]);
+#pragma unroll
+      for (int k = 0; k < KT; ++k) {
+        const uint2 a = tl_read_tr(from + k * (CT + RT) + i * 1024), b = tl_read_tr(from + k * (CT + RT) + (RK + i) * 1024);
+        const uint4 v = make_uint4(a.x, a.y, b.x, b.y);
+        acc[i] = Tl<bf16_t>::mma(v, hi4[k], acc[i]);
+        acc[i] = Tl<bf16_t>::mma(v, lo4[k], acc[i]);
+      }
     }
-    if (more) LAT_STAGE(tile + (buf ^ 1) * (CT + RT));
+    if (BUFS == 1 && more) __syncthreads();
+    if (more) stage(tile + (buf ^ (BUFS - 1)) * BUF);
     __syncthreads();
-    buf ^= 1;
+    buf ^= BUFS - 1;
   }
   l_run = rows_sum(l_run);
   if (head >= p.heads) return;
@@ -273,7 +309,12 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(const LatentArgs 
 
 // ---- merge of the pieces, value expansion through W_uv[h], head gate: up to 16 rows x 128 value dims of one head ----
 template <typename T>
-__global__ __launch_bounds__(512) void latent_value_kernel(const LatentArgs p, int rpw) {
+__global__ __launch_bounds__(512) void latent_value_kernel(int2* where, const void* w_uv, float* part, float* part_ml, int heads, int M, int S, uint32_t ns_rpw,
+                                                           int rank64, int vdim16, const LatentArgs p0) {
+  LatentArgs p = p0;  // what the first loads need is in registers (see lm_gemm.hip)
+  p.rows.where = where; p.w_uv = w_uv; p.part = part; p.part_ml = part_ml; p.heads = heads; p.M = M; p.rows.S = S;
+  p.n_splits = (int)(ns_rpw & 0xffffu); p.d.rank64 = rank64; p.d.vdim16 = vdim16;
+  const int rpw = (int)(ns_rpw >> 16);
   extern __shared__ __align__(16) unsigned char lv_raw[];
   T* xs = (T*)lv_raw;  // 16 x rank64, tiled
   constexpr int EP = Tl<T>::EP, P = 16 / EP, PRE = sizeof(T) == 2 ? 8 : 4;
@@ -281,7 +322,6 @@ __global__ __launch_bounds__(512) void latent_value_kernel(const LatentArgs p, i
   const int h = blockIdx.x, m0 = blockIdx.z * rpw, R = p.d.rank64, ns = p.n_splits, nk = R >> 6;
   const int nb = blockIdx.y * 8 + wave, nvb = p.d.vdim16 >> 4;
   const int nrow = min(rpw, p.M - m0);
-  const float gate = p.gate[(size_t)min(m0 + (lane & 15), p.M - 1) * p.d.heads16 + h];
   // the first weights are requested ahead of the merge
   const T* wv = (const T*)p.w_uv + ((size_t)h * nvb + min(nb, nvb - 1)) * nk * 1024 + lane * EP;
   uint4 wp[PRE][P];
@@ -289,10 +329,10 @@ __global__ __launch_bounds__(512) void latent_value_kernel(const LatentArgs p, i
   for (int k = 0; k < PRE; ++k)
 #pragma unroll
     for (int i = 0; i < P; ++i) wp[k][i] = *reinterpret_cast<const uint4*>(wv + (size_t)min(k, nk - 1) * 1024 + 64 * EP * i);
+  const float gate = p.gate[(size_t)min(m0 + (lane & 15), p.M - 1) * p.d.heads16 + h];
   for (int it = wave; it < nrow * nk; it += 8) {  // a wave merges 64 columns of a row
     const int r = it / nk, k = (it - r * nk) * 64 + lane;
-    const int m = m0 + r, slot = lm_slot(p.rows, m);
-    const int len = min(max(lm_pos(p.rows, m, slot) + 1, 1), p.rows.S);
+    const int m = m0 + r, len = min(max(lm_where(p.rows, m).y + 1, 1), p.rows.S);
     const int chunk = latent_chunk(len, ns, p.M), np = (len + chunk - 1) / chunk;  // pieces that exist
     const size_t piece = ((size_t)m * p.heads + h) * ns;
     const float2 ml = *reinterpret_cast<const float2*>(p.part_ml + 2 * (piece + min(lane, np - 1)));
@@ -473,45 +513,45 @@ int launch_latent_append(const LatentArgs& a, hipStream_t st) {
 
 int launch_latent_query(const LatentArgs& a, hipStream_t st) {
   const dim3 grid(a.heads + (a.own ? 1 : 0), (a.d.rank16 / 16 + 3) / 4, (a.M + 15) / 16);
-  if (a.dtype == VUI_DTYPE_F32) hipLaunchKernelGGL(latent_query_kernel<float>, grid, dim3(256), 0, st, a);
-  else hipLaunchKernelGGL(latent_query_kernel<bf16_t>, grid, dim3(256), 0, st, a);
+  if (a.dtype == VUI_DTYPE_F32) hipLaunchKernelGGL(latent_query_kernel<float>, grid, dim3(256), 0, st, a.w_uk_t, a.qu, a.craw, a.qu_z, a.heads, a.M, a.d.dim64, a.d.rank16, a);
+  else hipLaunchKernelGGL(latent_query_kernel<bf16_t>, grid, dim3(256), 0, st, a.w_uk_t, a.qu, a.craw, a.qu_z, a.heads, a.M, a.d.dim64, a.d.rank16, a);
   HIP_TRY(hipGetLastError());
   return VUI_OK;
 }
 
 bool latent_mfma_ok(const vui_lm_dims& d) { return d.rank64 <= 512 && d.rot32 <= 64; }
 
-template <int RK, int RB>
+template <int RK, int RB, int KT>
 static int lam_go(const LatentArgs& a, hipStream_t st) {
   constexpr int lds = 2 * (RK * 2048 + RB * 1024) * 2;
-  if (lds > 60 * 1024) {
-    static bool set = false;
-    if (!set) {
-      HIP_TRY(hipFuncSetAttribute((const void*)latent_attn_mfma_kernel<RK, RB>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-      set = true;
-    }
-  }
-  hipLaunchKernelGGL((latent_attn_mfma_kernel<RK, RB>), dim3(a.M, (a.heads + 15) / 16, a.n_splits), dim3(256), lds, st, a);
+  if (lds > 60 * 1024)
+    HIP_TRY(hipFuncSetAttribute((const void*)latent_attn_mfma_kernel<RK, RB, KT>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+  hipLaunchKernelGGL((latent_attn_mfma_kernel<RK, RB, KT>), dim3(a.M, (a.heads + 15) / 16, a.n_splits), dim3(256), lds, st, a.rows.where, a.c_cache, a.kr_cache, a.qlat,
+                     (uint32_t)a.M | (uint32_t)a.n_splits << 24, a.rows.S, a.d.s64, a.d.heads16, a);
   HIP_TRY(hipGetLastError());
   return VUI_OK;
 }
-template <int RB>
+template <int RB, int KT>
 static int lam_rank(const LatentArgs& a, hipStream_t st) {
   switch (a.d.rank64 / 64) {
-    case 1: return lam_go<1, RB>(a, st);
-    case 2: return lam_go<2, RB>(a, st);
-    case 3: return lam_go<3, RB>(a, st);
-    case 4: return lam_go<4, RB>(a, st);
-    case 5: return lam_go<5, RB>(a, st);
-    case 6: return lam_go<6, RB>(a, st);
-    case 7: return lam_go<7, RB>(a, st);
-    default: return lam_go<8, RB>(a, st);
+    case 1: return lam_go<1, RB, KT>(a, st);
+    case 2: return lam_go<2, RB, KT>(a, st);
+    case 3: return lam_go<3, RB, KT>(a, st);
+    case 4: return lam_go<4, RB, KT>(a, st);
+    case 5: return lam_go<5, RB, KT>(a, st);
+    case 6: return lam_go<6, RB, KT>(a, st);
+    case 7: return lam_go<7, RB, KT>(a, st);
+    default: return lam_go<8, RB, KT>(a, st);
   }
 }
 
 int launch_latent_attn(const LatentArgs& a, hipStream_t st) {
-  if (a.n_splits < 1 || a.n_splits > 64 || a.d.rank64 > 256 * LAT_ACC) { vui_set_error("latent attention: rank %d, splits %d out of range", a.d.rank64, a.n_splits); return VUI_EINVAL; }
-  if (a.dtype == VUI_DTYPE_BF16 && latent_mfma_ok(a.d)) return a.d.rot32 == 32 ? lam_rank<1>(a, st) : lam_rank<2>(a, st);
+  if (a.n_splits < 1 || a.n_splits > 64 || a.M >= 1 << 24 || a.d.rank64 > 256 * LAT_ACC) { vui_set_error("latent attention: rank %d, splits %d out of range", a.d.rank64, a.n_splits); return VUI_EINVAL; }
+  if (a.dtype == VUI_DTYPE_BF16 && latent_mfma_ok(a.d)) {
+    const bool one = latent_least(a.M) == 32;
+    if (a.d.rot32 == 32) return one ? lam_rank<1, 1>(a, st) : lam_rank<1, 2>(a, st);
+    return one ? lam_rank<2, 1>(a, st) : lam_rank<2, 2>(a, st);
+  }
   const dim3 grid(a.M, a.heads, a.n_splits);
   const size_t lds = (size_t)(a.d.rank64 + a.d.rot32) * 4;
   if (a.dtype == VUI_DTYPE_F32) hipLaunchKernelGGL(latent_attn_kernel<float>, grid, dim3(256), lds, st, a);
@@ -531,8 +571,8 @@ int launch_latent_value(const LatentArgs& a, hipStream_t st) {
     HIP_TRY(hipFuncSetAttribute(f32 ? (const void*)latent_value_kernel<float> : (const void*)latent_value_kernel<bf16_t>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   }
-  if (f32) hipLaunchKernelGGL(latent_value_kernel<float>, grid, dim3(512), lds, st, a, rpw);
-  else hipLaunchKernelGGL(latent_value_kernel<bf16_t>, grid, dim3(512), lds, st, a, rpw);
+  if (f32) hipLaunchKernelGGL(latent_value_kernel<float>, grid, dim3(512), lds, st, a.rows.where, a.w_uv, a.part, a.part_ml, a.heads, a.M, a.rows.S, (uint32_t)a.n_splits | (uint32_t)rpw << 16, a.d.rank64, a.d.vdim16, a);
+  else hipLaunchKernelGGL(latent_value_kernel<bf16_t>, grid, dim3(512), lds, st, a.rows.where, a.w_uv, a.part, a.part_ml, a.heads, a.M, a.rows.S, (uint32_t)a.n_splits | (uint32_t)rpw << 16, a.d.rank64, a.d.vdim16, a);
   HIP_TRY(hipGetLastError());
   return VUI_OK;
 }

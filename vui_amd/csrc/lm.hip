@@ -53,7 +53,7 @@ static size_t lm_carve(const vui_lm_config* c, const vui_lm_layer* layers, vui_l
     mx(ac, R * d.out_k);
     if (L.mixer == VUI_LM_MINGRU) { mx(up, d.gru16); continue; }
     const size_t H = L.heads;
-    mx(qu, H * R * d.dim64); mx(qr, H * R * d.rot32); mx(ql, H * R * d.rank64);
+    mx(qu, H * R * d.dim64); mx(qr, H * R * d.rot32); mx(ql, R * d.heads16 * d.rank64);
     mx(cr, R * d.rank16); mx(ga, R * d.heads16);
     size_t rows = R;  // rows x splits of attention pieces
     for (int M = 1; M <= (int)R && M <= 1024; ++M) mx(rows, (size_t)M * lm_splits(M, L.heads, d.rank64));
@@ -66,6 +66,7 @@ static size_t lm_carve(const vui_lm_config* c, const vui_lm_layer* layers, vui_l
   TAKE(x, float*, R * d.w64 * 4);
   TAKE(xt, void*, R * d.w64 * e);
   TAKE(ssq, float*, R * (d.w16 / 16) * 4);
+  TAKE(where, int2*, VUI_MAX_BATCH * 8);
   TAKE(qu, void*, qu * e);
   TAKE(qr, void*, qr * e);
   TAKE(qlat, void*, ql * e);
@@ -228,7 +229,7 @@ static int lm_attention(vui_lm_ctx* x, int l, int M, const LmRows& rows, LmGemm&
   memset(&a, 0, sizeof(a));
   a.dtype = c.dtype; a.M = M; a.heads = L.heads; a.scale = L.scale; a.rows = rows; a.d = d; a.rank = L.kv_rank;
   a.qu = x->qu; a.qr = x->qr; a.qu_z = g.qu_z; a.qr_z = g.qr_z;
-  a.qlat = x->qlat; a.qlat_z = (size_t)x->R16 * d.rank64;
+  a.qlat = x->qlat;
   a.craw = x->craw; a.latent_norm = L.latent_norm; a.eps = c.norm_eps; a.own = own;
   a.w_uk_t = L.w_uk_t; a.w_uv = L.w_uv; a.c_cache = L.c_cache; a.kr_cache = L.kr_cache;
   a.part = x->part; a.part_ml = x->part_ml; a.gate = x->gate; a.act = x->act;
@@ -268,7 +269,7 @@ static int lm_layers(vui_lm_ctx* x, const int64_t* tokens, int M, const LmRows& 
   const vui_lm_config& c = x->c;
   if (c.norm_groups > 0) return sandwich_layers(x, tokens, M, rows, st);
   const int w64 = x->dims[0].w64, np = x->dims[0].w16 / 16;
-  int rc = launch_lm_embed(c.dtype, tokens, x->w.embed, x->x, x->xt, x->ssq, M, c.width, w64, np, c.vocab, st);
+  int rc = launch_lm_embed(c.dtype, rows, tokens, x->w.embed, x->x, x->xt, x->ssq, M, c.width, w64, np, c.vocab, st);
   if (rc) return rc;
   for (int l = 0; l < c.n_layers; ++l) {
     const vui_lm_layer& L = x->layers[l];
@@ -312,7 +313,7 @@ int vui_lm_decode(vui_lm_ctx* x, const int64_t* tokens, const int32_t* slot_idx,
   hipStream_t st = (hipStream_t)stream;
   LmRows r;
   memset(&r, 0, sizeof(r));
-  r.slot_idx = slot_idx; r.seq_lens = seq_lens; r.S = x->c.max_seqlen; r.n_slots = x->c.n_slots;
+  r.slot_idx = slot_idx; r.seq_lens = seq_lens; r.where = x->where; r.S = x->c.max_seqlen; r.n_slots = x->c.n_slots;
   int rc = lm_layers(x, tokens, B, r, st);
   if (rc) return rc;
   LmGemm g = lm_logits(x, r, B, B, nullptr, logits_out);

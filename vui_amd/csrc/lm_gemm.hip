@@ -94,7 +94,7 @@ __device__ __forceinline__ void lm_unit(const LmGemm& p, const int m, const int 
         Tl<T>::st4((T*)p.qu + h * p.qu_z + tl_off<T>(m, o, p.d.dim64), v);
       } else if (nb < p.b_c) {
         const int dr = p.d.rot16 >> 4, b = nb - p.b_qr, h = b / dr, o = (b - h * dr) * 16 + 4 * kg;
-        const int slot = PRE ? e.slot : lm_slot(p.rows, m), pos = min(max(PRE ? e.pos : lm_pos(p.rows, m, slot), 0), p.rows.S - 1);
+        const int pos = min(max(PRE ? e.pos : lm_where(p.rows, m).y, 0), p.rows.S - 1);
         lm_rotate2(v, p.rope, pos, p.rot_pairs, o >> 1);
         Tl<T>::st4((T*)p.qr + h * p.qr_z + tl_off<T, 32>(m, o, p.d.rot32), v);
       } else if (nb < p.b_kr) {
@@ -102,7 +102,8 @@ __device__ __forceinline__ void lm_unit(const LmGemm& p, const int m, const int 
         *reinterpret_cast<float4*>(p.craw + (size_t)m * p.d.rank16 + o) = make_float4(v[0], v[1], v[2], v[3]);
       } else if (nb < p.b_g) {
         const int o = (nb - p.b_kr) * 16 + 4 * kg;
-        const int slot = PRE ? e.slot : lm_slot(p.rows, m), pos = PRE ? e.pos : lm_pos(p.rows, m, slot);
+        const int2 at = PRE ? make_int2(e.slot, e.pos) : lm_where(p.rows, m);
+        const int slot = at.x, pos = at.y;
         if (pos >= 0 && pos < p.rows.S) {
           lm_rotate2(v, p.rope, pos, p.rot_pairs, o >> 1);
           Tl<T>::st4((T*)p.kr_cache + (size_t)slot * p.d.s64 * p.d.rot32 + tl_off<T, 32>(pos, o, p.d.rot32), v);
@@ -290,8 +291,8 @@ __global__ __launch_bounds__(64 * WAVES, sizeof(T) == 2 && MB == 1 && NB < 3 ? 4
   e.slot = e.pos = 0;
   e.a = e.b = e.c = make_float4(0.f, 0.f, 0.f, 0.f);
   if (PRE && EPI != LM_OUT) {
-    e.slot = lm_slot(p.rows, pm);
-    e.pos = lm_pos(p.rows, pm, e.slot);
+    const int2 at = lm_where(p.rows, pm);
+    e.slot = at.x; e.pos = at.y;
   }
   if (PRE && EPI == LM_OUT) e.a = *reinterpret_cast<const float4*>(p.x + (size_t)pm * p.d.w64 + pb * 16 + 4 * kg);
   if (PRE && EPI == LM_IN_GRU_STEP && nb0 < p.mix_blocks) {
@@ -367,7 +368,7 @@ __global__ __launch_bounds__(64 * WAVES, sizeof(T) == 2 && MB == 1 && NB < 3 ? 4
     if (p.upd_inc) {
       for (int s = tid; s < p.rows.n_slots; s += 64 * WAVES) p.upd_lens[s] += p.upd_inc[s];
     } else {
-      for (int b = tid; b < p.upd_rows; b += 64 * WAVES) atomicAdd(&p.upd_lens[lm_slot(p.rows, b)], 1);
+      for (int b = tid; b < p.upd_rows; b += 64 * WAVES) atomicAdd(&p.upd_lens[lm_where(p.rows, b).x], 1);
     }
   }
 }
@@ -701,10 +702,11 @@ int launch_lm_gemm(int dtype, int epi, const LmGemm& g, int nz, hipStream_t st) 
 
 // ---- embedding rows: residual, operand copy, sums of squares per 16 columns ----
 template <typename T>
-__global__ __launch_bounds__(256) void lm_embed_kernel(const int64_t* tokens, const T* table, float* x, T* xt, float* ssq,
+__global__ __launch_bounds__(256) void lm_embed_kernel(const LmRows where, const int64_t* tokens, const T* table, float* x, T* xt, float* ssq,
                                                        int width, int w64, int np, int vocab, int rows) {
   const int m = blockIdx.x * 16 + (threadIdx.x >> 4), c = blockIdx.y * 64 + (threadIdx.x & 15) * 4;  // a block of the operand's layout
   if (m >= rows) return;
+  if (c == 0) lm_set_where(where, m);
   int64_t t = tokens[m];
   t = t < 0 ? 0 : (t >= vocab ? vocab - 1 : t);
   if (c < np * 16) {  // a multiple of 16: four neighbouring lanes are there or absent together
@@ -725,12 +727,12 @@ __global__ __launch_bounds__(256) void lm_embed_kernel(const int64_t* tokens, co
     if ((c & 15) == 0) ssq[(size_t)m * np + (c >> 4)] = s;
   }
 }
-int launch_lm_embed(int dtype, const int64_t* tokens, const void* table, float* x, void* xt, float* ssq, int rows, int width,
+int launch_lm_embed(int dtype, const LmRows& where, const int64_t* tokens, const void* table, float* x, void* xt, float* ssq, int rows, int width,
                     int w64, int np, int vocab, hipStream_t st) {
   if (dtype == VUI_DTYPE_F32)
-    hipLaunchKernelGGL(lm_embed_kernel<float>, dim3((rows + 15) / 16, (np + 3) / 4), dim3(256), 0, st, tokens, (const float*)table, x, (float*)xt, ssq, width, w64, np, vocab, rows);
+    hipLaunchKernelGGL(lm_embed_kernel<float>, dim3((rows + 15) / 16, (np + 3) / 4), dim3(256), 0, st, where, tokens, (const float*)table, x, (float*)xt, ssq, width, w64, np, vocab, rows);
   else
-    hipLaunchKernelGGL(lm_embed_kernel<bf16_t>, dim3((rows + 15) / 16, (np + 3) / 4), dim3(256), 0, st, tokens, (const bf16_t*)table, x, (bf16_t*)xt, ssq, width, w64, np, vocab, rows);
+    hipLaunchKernelGGL(lm_embed_kernel<bf16_t>, dim3((rows + 15) / 16, (np + 3) / 4), dim3(256), 0, st, where, tokens, (const bf16_t*)table, x, (bf16_t*)xt, ssq, width, w64, np, vocab, rows);
   HIP_TRY(hipGetLastError());
   return VUI_OK;
 }

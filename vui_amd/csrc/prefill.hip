@@ -674,10 +674,6 @@ struct PfDirectArgs {
   uint32_t* count;   // arrivals of a (head, tile) in the pass; `before`: those of earlier layers (their splits differ: windows)
   uint32_t before;
 };
-typedef short pf_s16x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ uint2 pf_read_tr(const char* lds) {
-  return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) pf_s16x4*)lds));
-}
 template <int HD32>
 __global__ __launch_bounds__(64 * PfDirect<HD32>::WAVES) void pf_direct_attn_kernel(const bf16_t* q, const bf16_t* kc, const bf16_t* vc, int T, int nq,
                                                                                     int nkv, int gsz, int pos0, int window, const PfDirectArgs a0) {
@@ -758,7 +754,7 @@ __global__ __launch_bounds__(64 * PfDirect<HD32>::WAVES) void pf_direct_attn_ker
     const char* vrow = own + (4 * kg + (l16 >> 2)) * (HD * 2) + (l16 & 3) * 8;
 #pragma unroll
     for (int d = 0; d < DT; ++d) {
-      const uint2 x = pf_read_tr(vrow + d * 32), y = pf_read_tr(vrow + 16 * HD * 2 + d * 32);
+      const uint2 x = tl_read_tr(vrow + d * 32), y = tl_read_tr(vrow + 16 * HD * 2 + d * 32);
       acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf_frag(make_uint4(x.x, x.y, y.x, y.y)), pf_frag(pf), acc[d], 0, 0, 0);
     }
   }

@@ -148,6 +148,7 @@ __global__ __launch_bounds__(NT) void lm_rows_kernel(const RowArgs p) {
   const int m = blockIdx.x, tid = threadIdx.x, n = p.width / p.groups;
   if (p.clear && m == 0)
     for (int i = tid; i < p.n_clear; i += NT) p.clear[i] = 0;
+  if (p.tokens && tid == 0) lm_set_where(p.rows, m);
   float* xr = p.x + (size_t)m * p.w64;
   const bool add = !p.tokens && !p.step;
   if (p.tokens) {
@@ -250,6 +251,7 @@ __global__ __launch_bounds__(1024) void lm_rows_quad_kernel(const RowArgs p, int
   };
   if (p.clear && m == 0)
     for (int i = tid; i < p.n_clear; i += blockDim.x) p.clear[i] = 0;
+  if (p.tokens && tid == 0) lm_set_where(p.rows, m);
   constexpr bool PRE = ROUTER && sizeof(T) == 2;
   RouterBlock<T> rw[PRE ? RT_PRE : 1];
   float* xr = p.x + (size_t)m * p.w64;

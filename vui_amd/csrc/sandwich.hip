@@ -93,6 +93,7 @@ size_t sandwich_carve(const vui_lm_config* c, const vui_lm_layer* layers, vui_lm
   TAKE(x, float*, R * d.w64 * 4);
   TAKE(xt, void*, R * d.w64 * e);
   TAKE(xcat, void*, loops ? R * 2 * d.w64 * e : 0);
+  TAKE(where, int2*, VUI_MAX_BATCH * 8);
   TAKE(raw, void*, raw * e);
   TAKE(qu, void*, q * e);
   TAKE(part, float*, pt * 4);
@@ -220,7 +221,7 @@ int sandwich_layers(vui_lm_ctx* x, const int64_t* tokens, int M, const LmRows& r
   };
   ahead(0);
   RowArgs emb = r;
-  emb.tokens = tokens; emb.clear = x->arrived; emb.n_clear = 1 + M * x->arrived_row;
+  emb.tokens = tokens; emb.rows = rows; emb.clear = x->arrived; emb.n_clear = 1 + M * x->arrived_row;
   int rc = launch_lm_rows(emb, st);
   for (int l = 0; l < n && !rc; ++l) {
     const vui_lm_layer& L = x->layers[l];

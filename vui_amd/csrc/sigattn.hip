@@ -35,7 +35,8 @@ __global__ __launch_bounds__(256) void sig_prep_kernel(const SigAttnArgs p) {
   const int lane = threadIdx.x & 63, m = blockIdx.y;
   const int u = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const SigCols c = sig_cols(p);
-  const int slot = lm_slot(p.rows, m), pos = lm_pos(p.rows, m, slot);
+  const int2 w_at = lm_where(p.rows, m);
+  const int slot = w_at.x, pos = w_at.y;
   if (u >= p.heads + 2 * p.kv_heads || pos < 0 || pos >= p.rows.S) return;
   const T* row = (const T*)p.raw + (size_t)m * p.ld;
   if (u >= p.heads + p.kv_heads) {
@@ -76,7 +77,8 @@ __global__ __launch_bounds__(256) void sig_piece_kernel(const SigAttnArgs p) {
   __shared__ float sc[SIG_TILE];
   const int m = blockIdx.x, h = blockIdx.y, sp = blockIdx.z, tid = threadIdx.x;
   const int g = h / (p.heads / p.kv_heads), nvb = p.d.vdim16 >> 4, D = p.d.dim64;
-  const int slot = lm_slot(p.rows, m), pos = lm_pos(p.rows, m, slot);
+  const int2 w_at = lm_where(p.rows, m);
+  const int slot = w_at.x, pos = w_at.y;
   const int len = min(max(pos + 1, 1), p.rows.S);
   const int chunk = sig_chunk(len, p.n_splits), lo = min(sp * chunk, len), hi = min(lo + chunk, len);
   if (lo >= hi) return;  // no such piece: the merge does not look for it
@@ -198,7 +200,8 @@ __global__ __launch_bounds__(256) void sig_piece_mfma_kernel(const SigAttnArgs p
   const int m = blockIdx.x, sp = blockIdx.z, per = p.heads / p.kv_heads, nhb = (per + 15) >> 4;
   const int g = (int)blockIdx.y / nhb, h0 = g * per + ((int)blockIdx.y % nhb) * 16, nh = min(16, (g + 1) * per - h0);
   const int head = h0 + min(l16, nh - 1), nvb = p.d.vdim16 >> 4;
-  const int slot = lm_slot(p.rows, m), pos = lm_pos(p.rows, m, slot);
+  const int2 w_at = lm_where(p.rows, m);
+  const int slot = w_at.x, pos = w_at.y;
   const int len = min(max(pos + 1, 1), p.rows.S);
   const int chunk = sig_chunk(len, p.n_splits), lo = min(sp * chunk, len), hi = min(lo + chunk, len);
   if (lo >= hi) return;  // no such piece
@@ -321,7 +324,8 @@ __global__ __launch_bounds__(256) void sig_merge_kernel(const SigAttnArgs p) {
   if (col >= p.heads * p.d.vdim16) return;
   const int h = col / p.d.vdim16, d = col - h * p.d.vdim16;
   const float gate = El<T>::ld((const T*)p.raw + (size_t)m * p.ld + sig_cols(p).g + h);
-  const int slot = lm_slot(p.rows, m), pos = lm_pos(p.rows, m, slot);
+  const int2 w_at = lm_where(p.rows, m);
+  const int pos = w_at.y;
   const int len = min(max(pos + 1, 1), p.rows.S);
   const int chunk = sig_chunk(len, p.n_splits), np = (len + chunk - 1) / chunk;  // pieces that exist
   const float* pc = p.part + ((size_t)m * p.heads + h) * p.n_splits * p.d.vdim16 + d;

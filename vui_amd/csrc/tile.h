@@ -49,6 +49,12 @@ template <> struct Tl<float> {
   static __device__ __forceinline__ void st2(float* p, float a, float b) { *reinterpret_cast<float2*>(p) = make_float2(a, b); }
 };
 
+// Transposed read of 16-bit elements: 16 lanes read eight bytes each, lane 4 r + c columns 4 c ... of row r; lane i receives column i
+typedef short tl_s16x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ uint2 tl_read_tr(const void* lds) {
+  return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) tl_s16x4*)lds));
+}
+
 // element offset of (row r, column k) of a tiled matrix with K columns
 template <typename T, int BK = 64>
 __host__ __device__ __forceinline__ size_t tl_off(int r, int k, int K) {
