@@ -39,10 +39,16 @@ template <> __device__ __forceinline__ void ld4<bf16_t>(const bf16_t* q, float* 
 __device__ __forceinline__ float silu_exact(float v) { return v / (1.0f + expf(-v)); }
 
 // ---- positions one by one; one workgroup per head and slot ----
+// Bound by its chain: place of the row, state, sums, norm.  What the first loads need is in registers (see lm_gemm.hip), and what a position
+// reads of the projection is asked for before the decays, its output gate and norm among it: 4 rows, 16 heads of 128 x 128, 10.8 -> @@ us
+// per launch, 1 row, 8 heads of 96 8.6 -> @@.
 #define GLA_THREADS 512
 #define GLA_PRE 8
 template <typename T>
-__global__ __launch_bounds__(GLA_THREADS) void gla_step_kernel(const GlaArgs p) {
+__global__ __launch_bounds__(GLA_THREADS) void gla_step_kernel(int2* where, const void* raw, float* state, const float* w_a2, int ld, int heads, int dim16,
+                                                               int vdim16, int rank, const GlaArgs p0) {
+  GlaArgs p = p0;
+  p.rows.where = where; p.raw = raw; p.state = state; p.w_a2 = w_a2; p.ld = ld; p.heads = heads; p.d.dim16 = dim16; p.d.vdim16 = vdim16; p.rank = rank;
   extern __shared__ __align__(16) float gl[];  // decay, key, query (dim16 each), value (vdim16), sums (passes, vdim16)
   __shared__ float red[GLA_THREADS / 64];
   const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -61,6 +67,10 @@ __global__ __launch_bounds__(GLA_THREADS) void gla_step_kernel(const GlaArgs p) 
 #pragma unroll
     for (int i = 0; i < GLA_PRE; ++i) s[i] = *reinterpret_cast<const tl_f32x4*>(S + (size_t)min(r0 + i * per, D - 1) * V + c4);
     const T* row = (const T*)p.raw + (size_t)m * p.ld;
+    // of the first GLA_THREADS channels
+    const int dk = min(tid, D - 1), dv = min(tid, V - 1);
+    const float k1 = El<T>::ld(row + c.k + h * D + dk), q1 = El<T>::ld(row + h * D + dk), v1 = El<T>::ld(row + c.v + h * V + dv);
+    const float gate1 = El<T>::ld(row + c.g + h * V + dv), norm1 = p.head_norm[dv];
     for (int d0 = 0; d0 < D; d0 += GLA_THREADS / 4) {  // four lanes share the low-rank sum of a channel
       const int d = min(d0 + (tid >> 2), D - 1);
       const float* w = p.w_a2 + ((size_t)h * D + d) * p.rank;
@@ -72,10 +82,10 @@ __global__ __launch_bounds__(GLA_THREADS) void gla_step_kernel(const GlaArgs p) 
       if ((tid & 3) == 0) la[d] = expf(gla_log_sigmoid(p, z + p.a2_bias[h * D + d]));
     }
     for (int d = tid; d < D; d += GLA_THREADS) {
-      lk[d] = El<T>::ld(row + c.k + h * D + d);
-      lq[d] = El<T>::ld(row + h * D + d) * p.q_scale;
+      lk[d] = d == tid ? k1 : El<T>::ld(row + c.k + h * D + d);
+      lq[d] = (d == tid ? q1 : El<T>::ld(row + h * D + d)) * p.q_scale;
     }
-    for (int d = tid; d < V; d += GLA_THREADS) lv[d] = El<T>::ld(row + c.v + h * V + d);
+    for (int d = tid; d < V; d += GLA_THREADS) lv[d] = d == tid ? v1 : El<T>::ld(row + c.v + h * V + d);
     __syncthreads();
     tl_f32x4 o = {0.f, 0.f, 0.f, 0.f};
     if (work) {
@@ -118,7 +128,8 @@ __global__ __launch_bounds__(GLA_THREADS) void gla_step_kernel(const GlaArgs p) 
     for (int w = 0; w < GLA_THREADS / 64; ++w) t += red[w];
     const float r = 1.0f / sqrtf(t / (float)p.vdim + p.eps);
     for (int d = tid; d < V; d += GLA_THREADS)
-      El<T>::st((T*)p.act + tl_off<T>(m, h * V + d, p.d.out_k), ls[d] * r * p.head_norm[d] * silu_exact(El<T>::ld(row + c.g + h * V + d)));
+      El<T>::st((T*)p.act + tl_off<T>(m, h * V + d, p.d.out_k),
+                ls[d] * r * (d == tid ? norm1 : p.head_norm[d]) * silu_exact(d == tid ? gate1 : El<T>::ld(row + c.g + h * V + d)));
     if (m + 1 < m1) {
       __threadfence_block();
       __syncthreads();
@@ -409,10 +420,10 @@ int launch_gla_step(const GlaArgs& a, hipStream_t st) {
   int rc;
   if (a.dtype == VUI_DTYPE_F32) {
     if ((rc = lds_attr((const void*)gla_step_kernel<float>, lds))) return rc;
-    hipLaunchKernelGGL(gla_step_kernel<float>, grid, dim3(GLA_THREADS), lds, st, a);
+    hipLaunchKernelGGL(gla_step_kernel<float>, grid, dim3(GLA_THREADS), lds, st, a.rows.where, a.raw, a.state, a.w_a2, a.ld, a.heads, a.d.dim16, a.d.vdim16, a.rank, a);
   } else {
     if ((rc = lds_attr((const void*)gla_step_kernel<bf16_t>, lds))) return rc;
-    hipLaunchKernelGGL(gla_step_kernel<bf16_t>, grid, dim3(GLA_THREADS), lds, st, a);
+    hipLaunchKernelGGL(gla_step_kernel<bf16_t>, grid, dim3(GLA_THREADS), lds, st, a.rows.where, a.raw, a.state, a.w_a2, a.ld, a.heads, a.d.dim16, a.d.vdim16, a.rank, a);
   }
   HIP_TRY(hipGetLastError());
   return VUI_OK;

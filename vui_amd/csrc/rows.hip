@@ -230,13 +230,20 @@ __global__ __launch_bounds__(NT) void lm_rows_kernel(const RowArgs p) {
 
 // The same where a wave's lanes hold four columns each of one part (parts of whole quads, no more than 16 waves for all of
 // them): the row stays in registers, and a part of up to 256 columns needs no barrier.
+// What the first loads need is in registers (see lm_gemm.hip): shape is wp, groups << 5, top << 10, whether the launch adds << 31.
 template <typename T, bool ROUTER>
-__global__ __launch_bounds__(1024) void lm_rows_quad_kernel(const RowArgs p, int wp) {
+__global__ __launch_bounds__(1024) void lm_rows_quad_kernel(float* x, const float* y, const float* post_w, const float* next_w, const float* share, int n, int w64,
+                                                            int ldy, uint32_t shape, const RowArgs p0) {
+  RowArgs p = p0;
+  p.x = x; p.y = y; p.post = post_w; p.next = next_w; p.share = share; p.w64 = w64; p.ldy = ldy;
+  p.groups = (int)(shape >> 5 & 31u); p.top = (int)(shape >> 10 & 0xfffffu); p.width = n * p.groups;
+  const int wp = (int)(shape & 31u);
+  const bool add = shape >> 31;
   extern __shared__ __align__(16) float rl[];  // for the router: row (w64), sums
   __shared__ float red[2][16];
-  const int m = blockIdx.x, tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, n = p.width / p.groups;
-  const int g = wave / wp, at = ((wave - g * wp) * 64 + lane) * 4;
-  const bool live = at < n, add = !p.tokens && !p.step;
+  const int m = blockIdx.x, tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int g = wp == 1 ? wave : wp == 2 ? wave >> 1 : wave / wp, at = ((wave - g * wp) * 64 + lane) * 4;
+  const bool live = at < n;
   const int k = g * n + min(at, n - 4);
   auto part_scale = [&](const tl_f32x4& v, int which) {
     float s = live ? (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]) : 0.f;
@@ -249,9 +256,6 @@ __global__ __launch_bounds__(1024) void lm_rows_quad_kernel(const RowArgs p, int
     }
     return 1.0f / sqrtf(s / (float)n + p.eps);
   };
-  if (p.clear && m == 0)
-    for (int i = tid; i < p.n_clear; i += blockDim.x) p.clear[i] = 0;
-  if (p.tokens && tid == 0) lm_set_where(p.rows, m);
   constexpr bool PRE = ROUTER && sizeof(T) == 2;
   RouterBlock<T> rw[PRE ? RT_PRE : 1];
   float* xr = p.x + (size_t)m * p.w64;
@@ -263,6 +267,9 @@ __global__ __launch_bounds__(1024) void lm_rows_quad_kernel(const RowArgs p, int
     old = *reinterpret_cast<const tl_f32x4*>(p.step + k);
   }
   if (p.next) next = *reinterpret_cast<const tl_f32x4*>(p.next + k);
+  if (p.clear && m == 0)
+    for (int i = tid; i < p.n_clear; i += blockDim.x) p.clear[i] = 0;
+  if (p.tokens && tid == 0) lm_set_where(p.rows, m);
   if constexpr (PRE) {
     RouterAt at;
 #pragma unroll
@@ -319,12 +326,17 @@ template <typename T>
 static int quad_go(const RowArgs& a, int wp, hipStream_t st) {
   const int waves = a.groups * wp;
   const size_t lds = a.rlog ? ((size_t)a.w64 + waves * a.experts16) * 4 : 0;
+  const uint32_t shape = (uint32_t)wp | (uint32_t)a.groups << 5 | (uint32_t)a.top << 10 | (!a.tokens && !a.step ? 1u << 31 : 0u);
+  if (a.top < 0 || a.top > 0xfffff) { vui_set_error("lm rows: %d choices", a.top); return VUI_EINVAL; }
+#define QUAD(ROUTER) \
+  hipLaunchKernelGGL((lm_rows_quad_kernel<T, ROUTER>), dim3(a.M), dim3(64 * waves), lds, st, a.x, a.y, a.post, a.next, a.share, a.width / a.groups, a.w64, a.ldy, shape, a)
   if (!a.rlog) {
-    hipLaunchKernelGGL((lm_rows_quad_kernel<T, false>), dim3(a.M), dim3(64 * waves), 0, st, a, wp);
+    QUAD(false);
   } else {
     if (lds > 60 * 1024) HIP_TRY(hipFuncSetAttribute((const void*)lm_rows_quad_kernel<T, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL((lm_rows_quad_kernel<T, true>), dim3(a.M), dim3(64 * waves), lds, st, a, wp);
+    QUAD(true);
   }
+#undef QUAD
   HIP_TRY(hipGetLastError());
   return VUI_OK;
 }

@@ -154,19 +154,31 @@ struct SigTile {
 // sigmoid of a score given t = -log2(e) score
 __device__ __forceinline__ float sig_weight(float t) { return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(t)); }
 
-// a normed row as a lane's part of an operand: columns 64 b + 16 kg .. + 15 in f[2 b], f[2 b + 1]; src: dim16 values
+// a row and its norm's weights as a lane's part of an operand: columns 64 b + 16 kg .. + 15; src: dim16 values
+typedef float sig_f32x4 __attribute__((ext_vector_type(4), aligned(4)));
+template <int DB> struct SigRow { uint4 x[DB][2]; sig_f32x4 w[DB][4]; };
 template <int DB>
-__device__ __forceinline__ void sig_normed(const bf16_t* src, const float* w, int dim16, int dim, float eps, float mul, int kg, uint4* f) {
+__device__ __forceinline__ void sig_row(const bf16_t* src, const float* w, int dim16, int kg, SigRow<DB>& r) {
+#pragma unroll
+  for (int b = 0; b < DB; ++b) {
+    const int col = b * 64 + kg * 16 < dim16 ? b * 64 + kg * 16 : 0;
+    const uint4* q = reinterpret_cast<const uint4*>(src + col);
+    r.x[b][0] = q[0]; r.x[b][1] = q[1];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r.w[b][i] = *reinterpret_cast<const sig_f32x4*>(w + col + 4 * i);
+  }
+}
+// and normed, in f[2 b], f[2 b + 1]
+template <int DB>
+__device__ __forceinline__ void sig_normed(const SigRow<DB>& row, int dim16, int dim, float eps, float mul, int kg, uint4* f) {
   float v[DB][16], ss = 0.f;
 #pragma unroll
   for (int b = 0; b < DB; ++b) {
-    const int col = b * 64 + kg * 16;
-    const bool live = col < dim16;
-    const uint4* q = reinterpret_cast<const uint4*>(src + (live ? col : 0));
-    const uint4 x[2] = {q[0], q[1]};
+    const bool live = b * 64 + kg * 16 < dim16;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const uint32_t u[4] = {x[h].x, x[h].y, x[h].z, x[h].w};
+      const uint4 x = row.x[b][h];
+      const uint32_t u[4] = {x.x, x.y, x.z, x.w};
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         v[b][8 * h + 2 * i] = live ? bf_lo(u[i]) : 0.f;
@@ -179,10 +191,11 @@ __device__ __forceinline__ void sig_normed(const bf16_t* src, const float* w, in
   const float r = mul / sqrtf(rows_sum(ss) / (float)dim + eps);
 #pragma unroll
   for (int b = 0; b < DB; ++b) {
-    const int col = b * 64 + kg * 16;
-    const float* c = w + (col < dim16 ? col : 0);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) v[b][i] *= r * c[i];
+    for (int i = 0; i < 4; ++i) {
+      const sig_f32x4 c = row.w[b][i];
+      v[b][4 * i] *= r * c.x; v[b][4 * i + 1] *= r * c.y; v[b][4 * i + 2] *= r * c.z; v[b][4 * i + 3] *= r * c.w;
+    }
 #pragma unroll
     for (int h = 0; h < 2; ++h)
       f[2 * b + h] = make_uint4(f2bf2(v[b][8 * h], v[b][8 * h + 1]), f2bf2(v[b][8 * h + 2], v[b][8 * h + 3]),
@@ -193,14 +206,37 @@ __device__ __forceinline__ void sig_normed(const bf16_t* src, const float* w, in
 // ---- pieces on the matrix cores (bf16): one workgroup per (row, up to 16 heads of one group, piece) ----
 // STEP (one position per slot): queries are normed here, and the wave that comes to the new position's tile norms its key,
 // puts key and value into its operands and appends them (workgroups of further heads of the group write the same).
+// Bound by its chain: place of the row, keys and values, scores, weights, sums, the pieces' meeting.  What the first loads need is in
+// registers (see lm_gemm.hip); queries, the new key and value and their norms' weights do not depend on the row's place and go out first, the
+// first tile before the query's norm: 4 rows behind 500 positions, 16 heads of 128, 10.5 -> @@ us per launch, 1 row behind 150 8.1 -> @@.
 template <int DB, int VT, bool STEP>
-__global__ __launch_bounds__(256) void sig_piece_mfma_kernel(const SigAttnArgs p) {
+__global__ __launch_bounds__(256) void sig_piece_mfma_kernel(int2* where, const void* raw, const void* k_cache, const void* v_cache, int ld, int s64, int S,
+                                                            uint32_t heads, uint32_t dims, uint32_t splits, const SigAttnArgs p0) {
+  SigAttnArgs p = p0;
+  p.rows.where = where; p.raw = raw; p.k_cache = const_cast<void*>(k_cache); p.v_cache = const_cast<void*>(v_cache);
+  p.ld = ld; p.d.s64 = s64; p.rows.S = S; p.heads = (int)(heads & 0xffffu); p.kv_heads = (int)(heads >> 16);
+  p.d.dim16 = (int)(dims & 0xffffu); p.d.vdim16 = (int)(dims >> 16); p.n_splits = (int)splits;
   __shared__ __align__(16) float s_acc[4][VT * 256];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l16 = lane & 15, kg = lane >> 4;
   const int m = blockIdx.x, sp = blockIdx.z, per = p.heads / p.kv_heads, nhb = (per + 15) >> 4;
   const int g = (int)blockIdx.y / nhb, h0 = g * per + ((int)blockIdx.y % nhb) * 16, nh = min(16, (g + 1) * per - h0);
   const int head = h0 + min(l16, nh - 1), nvb = p.d.vdim16 >> 4;
   const int2 w_at = lm_where(p.rows, m);
+  const bf16_t* row = (const bf16_t*)p.raw + (size_t)m * p.ld;
+  const SigCols cols = sig_cols(p);
+  SigRow<STEP ? DB : 1> q_row, k_row;
+  bf16_t nv[STEP ? VT : 1];
+  uint4 qf[2 * DB];
+  if constexpr (STEP) {
+    sig_row<DB>(row + head * p.d.dim16, p.q_norm, p.d.dim16, kg, q_row);
+    sig_row<DB>(row + cols.k + g * p.d.dim16, p.k_norm, p.d.dim16, kg, k_row);
+#pragma unroll
+    for (int d = 0; d < VT; ++d) nv[d] = row[cols.v + g * p.d.vdim16 + min(d, nvb - 1) * 16 + l16];
+  } else {
+#pragma unroll
+    for (int i = 0; i < 2 * DB; ++i)
+      qf[i] = *reinterpret_cast<const uint4*>((const bf16_t*)p.q + head * p.q_z + ((size_t)(m >> 4) * DB * 2 + i) * 512 + ((m & 15) + 16 * kg) * 8);
+  }
   const int slot = w_at.x, pos = w_at.y;
   const int len = min(max(pos + 1, 1), p.rows.S);
   const int chunk = sig_chunk(len, p.n_splits), lo = min(sp * chunk, len), hi = min(lo + chunk, len);
@@ -208,22 +244,17 @@ __global__ __launch_bounds__(256) void sig_piece_mfma_kernel(const SigAttnArgs p
   const bf16_t* kb = (const bf16_t*)p.k_cache + ((size_t)slot * p.kv_heads + g) * p.d.s64 * (DB * 64) + lane * 8;
   const bf16_t* vb = (const bf16_t*)p.v_cache + ((size_t)slot * p.kv_heads + g) * p.d.s64 * p.d.vdim16 + lane * 8;
   const float* bias = p.bias + (size_t)head * p.bias_len;
-  uint4 qf[2 * DB];
-  const bf16_t* row = (const bf16_t*)p.raw + (size_t)m * p.ld;
-  if (STEP) {
-    sig_normed<DB>(row + head * p.d.dim16, p.q_norm, p.d.dim16, p.dim, p.eps, sig_temp(p, pos), kg, qf);
-  } else {
-#pragma unroll
-    for (int i = 0; i < 2 * DB; ++i)
-      qf[i] = *reinterpret_cast<const uint4*>((const bf16_t*)p.q + head * p.q_z + ((size_t)(m >> 4) * DB * 2 + i) * 512 + ((m & 15) + 16 * kg) * 8);
-  }
   tl_f32x4 acc[VT];
 #pragma unroll
   for (int d = 0; d < VT; ++d) acc[d] = tl_f32x4{0.f, 0.f, 0.f, 0.f};
   const float c = -p.scale * SIG_LOG2E;
-  for (int k0 = lo + 32 * wave; k0 < hi; k0 += 128) {
-    SigTile<DB, VT> t;
-    t.load(kb, vb, k0, nvb);
+  SigTile<DB, VT> t;
+  const int first = lo + 32 * wave;
+  if (first < hi) t.load(kb, vb, first, nvb);
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (STEP) sig_normed<DB>(q_row, p.d.dim16, p.dim, p.eps, sig_temp(p, pos), kg, qf);
+  for (int k0 = first; k0 < hi; k0 += 128) {
+    if (k0 > first) t.load(kb, vb, k0, nvb);
     float b[8], w[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
@@ -231,9 +262,8 @@ __global__ __launch_bounds__(256) void sig_piece_mfma_kernel(const SigAttnArgs p
       b[e] = bias[min(max(len - 1 - j, 0), p.bias_len - 1)];
     }
     if (STEP && pos == len - 1 && (pos >> 5) == (k0 >> 5)) {  // uniform; a position outside the slot is not stored
-      const SigCols cols = sig_cols(p);
       uint4 nk[2 * DB];
-      sig_normed<DB>(row + cols.k + g * p.d.dim16, p.k_norm, p.d.dim16, p.dim, p.eps, 1.f, kg, nk);
+      if constexpr (STEP) sig_normed<DB>(k_row, p.d.dim16, p.dim, p.eps, 1.f, kg, nk);
       const bool mine = l16 == (pos & 15);
       bf16_t* ko = const_cast<bf16_t*>(kb) + (size_t)(pos >> 4) * DB * 1024;
 #pragma unroll
@@ -247,13 +277,13 @@ __global__ __launch_bounds__(256) void sig_piece_mfma_kernel(const SigAttnArgs p
       bf16_t* vo = const_cast<bf16_t*>(vb) + (size_t)(pos >> 5) * nvb * 512 + e;
 #pragma unroll
       for (int d = 0; d < VT; ++d) {
-        const bf16_t nv = row[cols.v + g * p.d.vdim16 + min(d, nvb - 1) * 16 + l16];
-        const uint32_t keep = 0xffffu << (16 - sh), put = (uint32_t)nv << sh;
+        const bf16_t n = nv[STEP ? d : 0];
+        const uint32_t keep = 0xffffu << (16 - sh), put = (uint32_t)n << sh;
         if (vmine && w == 0) t.vf[d].x = (t.vf[d].x & keep) | put;
         if (vmine && w == 1) t.vf[d].y = (t.vf[d].y & keep) | put;
         if (vmine && w == 2) t.vf[d].z = (t.vf[d].z & keep) | put;
         if (vmine && w == 3) t.vf[d].w = (t.vf[d].w & keep) | put;
-        if (vmine && d < nvb) vo[(size_t)d * 512] = nv;
+        if (vmine && d < nvb) vo[(size_t)d * 512] = n;
       }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -271,7 +301,7 @@ __global__ __launch_bounds__(256) void sig_piece_mfma_kernel(const SigAttnArgs p
   __syncthreads();
   const int np = (len + chunk - 1) / chunk;  // pieces that exist
   auto out = [&](int d, int hh, int k4, const tl_f32x4& o) {
-    const float f = 1.0f / (1.0f + expf(-bf2f(row[sig_cols(p).g + h0 + hh])));
+    const float f = 1.0f / (1.0f + expf(-bf2f(row[cols.g + h0 + hh])));
     const float r[4] = {o[0] * f, o[1] * f, o[2] * f, o[3] * f};
     Tl<bf16_t>::st4((bf16_t*)p.act + tl_off<bf16_t>(m, (h0 + hh) * p.d.vdim16 + 16 * d + 4 * k4, p.d.out_k), r);
   };
@@ -441,12 +471,15 @@ int launch_sig_prep(const SigAttnArgs& a, hipStream_t st) {
   return VUI_OK;
 }
 
+#define SIG_HOT_ARGS(a)                                                                                       \
+  a.rows.where, a.raw, a.k_cache, a.v_cache, a.ld, a.d.s64, a.rows.S, (uint32_t)a.heads | (uint32_t)a.kv_heads << 16, \
+      (uint32_t)a.d.dim16 | (uint32_t)a.d.vdim16 << 16, (uint32_t)a.n_splits
 template <int DB, int VT>
 static void piece_go(const SigAttnArgs& a, hipStream_t st) {
   const int per = a.heads / a.kv_heads;
   const dim3 grid(a.M, a.kv_heads * ((per + 15) / 16), a.n_splits);
-  if (a.rows.seq) hipLaunchKernelGGL((sig_piece_mfma_kernel<DB, VT, false>), grid, dim3(256), 0, st, a);
-  else hipLaunchKernelGGL((sig_piece_mfma_kernel<DB, VT, true>), grid, dim3(256), 0, st, a);
+  if (a.rows.seq) hipLaunchKernelGGL((sig_piece_mfma_kernel<DB, VT, false>), grid, dim3(256), 0, st, SIG_HOT_ARGS(a), a);
+  else hipLaunchKernelGGL((sig_piece_mfma_kernel<DB, VT, true>), grid, dim3(256), 0, st, SIG_HOT_ARGS(a), a);
 }
 template <int DB, int VT>
 static void prompt_go(const SigAttnArgs& a, hipStream_t st) {
@@ -469,7 +502,7 @@ static void prompt_go(const SigAttnArgs& a, hipStream_t st) {
   else GO<DB, 16>(a, st);
 
 int launch_sig_pieces(const SigAttnArgs& a, hipStream_t st) {
-  if (a.n_splits < 1 || a.bias_len < 1 || a.heads % a.kv_heads) { vui_set_error("sigmoid attention: bad shape"); return VUI_EINVAL; }
+  if (a.n_splits < 1 || a.bias_len < 1 || a.heads % a.kv_heads || a.heads > 0xffff) { vui_set_error("sigmoid attention: bad shape"); return VUI_EINVAL; }
   if (a.dtype == VUI_DTYPE_BF16 && sig_mfma_ok(a.d)) {
     SIG_DISPATCH(piece_go)
   } else {
