@@ -458,6 +458,24 @@ def test_routing_of_decode_rows(experts, top, rows, dt):
     assert far <= (0 if dt == F32 else 0.1 * n * rows), far
 
 
+@pytest.mark.parametrize("rows", [1, 16])
+def test_an_expert_with_more_entries_than_a_tile(rows):
+    """Logits that are not numbers are never chosen; what is missing is expert 0 with no weight, twice per row here: with 16 rows two
+    tiles of it.  Against the model whose tokens use only the two experts that are left."""
+    cfg = [U.sandwich([(U.sig(), U.moe(experts=6, top=top))]) for top in (4, 2)]
+    sd = [U.sandwich_weights(c, 52) for c in cfg]
+    for s, b in zip(sd, (float("nan"), -1e4)):
+        s["l0.mlp.router.b"] = torch.tensor([b, 0.5, b, 0.0, b, b]).to(torch.bfloat16)
+    outs = []
+    for c, s in zip(cfg, sd):
+        eng = U.engine(c, s, F32, max_rows=rows)
+        held = [eng.new_row() for _ in range(rows)]
+        for k, row in enumerate(held):
+            row.extend(U.tokens(4 + k, c["vocab"], k))
+        outs.append(eng.decode_step(held, torch.arange(rows, device="cuda")).clone())
+    assert U.err(outs[0], outs[1]) < TOL[F32]
+
+
 @BOTH
 def test_captured_step_replayed(dt):
     """The bucketed graph against the oracle, several replays with other work of the engine in between."""

@@ -97,6 +97,7 @@ struct LmGemm {
   float act_pos, act_neg;
   // entries (row top + choice) sorted by expert, every expert's padded with -1 to whole tiles; expert of each tile
   const int32_t *ent, *tile_e, *n_tiles;
+  const int32_t* choice;  // few rows: the experts of the M top entries, from which a product finds its tile's; nullptr: the three above
   int top, max_tiles, tile_rows;
   int sorted;      // X holds a row per entry instead of a row per position
   // lm_tile_at: feature tiles of a band; what divides by a band's tiles, its width and the last one's width
@@ -190,8 +191,7 @@ struct RowArgs {
   const float* router_bias;
   int experts16;
   float* rlog;             // (M, experts16)
-  RouteArgs route;         // rows are routed as well
-  uint32_t* arrived;       // rows that have made their choices, zero between launches
+  RouteArgs route;         // rows are routed as well, or choice nullptr
   LmRows rows;             // of the first launch of a pass (tokens)
   // the first launch of a pass clears the arrival counters that its rows use (a workspace comes as it is)
   uint32_t* clear;
@@ -199,7 +199,7 @@ struct RowArgs {
 };
 int launch_lm_rows(const RowArgs& a, hipStream_t st);
 bool lm_rows_routes(int M, int experts16);  // it takes the router's product too
-bool lm_rows_sorts(int M, int top);         // ... and the routing
+bool lm_entries_in_wave(int M, int top);    // ... and the routing: the products find an expert's entries in `choice`
 
 // ---- attention with sigmoid weights (sigattn.hip) ----
 struct SigAttnArgs {
@@ -281,7 +281,7 @@ struct vui_lm_ctx {
   void *xcat, *raw, *ffa, *xg;
   float *y, *bsum, *gupd, *gdec, *rlog, *share;
   int32_t *choice, *ent, *tile_e, *n_tiles;
-  uint32_t* arrived;  // rows routed, then attention pieces of each row's blocks of heads
+  uint32_t* arrived;  // attention pieces of each row's blocks of heads
   int arrived_row;    // blocks of heads of a row, at most
   int attn_from, gla_from;
 };

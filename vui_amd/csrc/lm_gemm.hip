@@ -139,7 +139,7 @@ __device__ __forceinline__ void lm_unit(const LmGemm& p, const int m, const int 
     return;
   }
   if (EPI == LM_PROJ || EPI == LM_PLAIN || EPI == LM_MOE_DOWN) {
-    const int r = EPI == LM_MOE_DOWN ? p.ent[m] : m;
+    const int r = EPI != LM_MOE_DOWN ? m : p.choice ? e.slot : p.ent[m];
     if (!live || r < 0) return;
     if (EPI != LM_MOE_DOWN && p.bias) {
       const float4 b = *reinterpret_cast<const float4*>(p.bias + n);
@@ -185,16 +185,19 @@ static void lm_set_order(LmGemm& g, int MT, int NT, int band) {
 }
 
 // The first fourteen words of a kernel's scalar arguments are in registers when it starts, a struct is a trip to memory (0.2-0.35 us of a
-// launch of 4-8): what the first loads need comes twice, ahead of the struct and in it.  aux0, aux1: of experts' products the number of
-// tiles and their experts, otherwise the sums of squares and the norm.  np: of the same, the entries' tiles.
+// launch of 4-8): what the first loads need comes twice, ahead of the struct and in it.  aux0, aux1: of experts' products the choices, or
+// the number of tiles and their experts, otherwise the sums of squares and the norm; np_band: of the same the entries' tiles.
 #define LM_HOT const void *X, const void *W, const void *aux0, const void *aux1, int M, uint32_t nk, uint32_t np_band, uint32_t inv_tiles, uint32_t inv_band, uint32_t inv_last
 #define LM_HOT_ARGS(g, moe)                                                                                                                 \
-  g.X, g.W, (moe) ? (const void*)g.n_tiles : (const void*)g.ssq, (moe) ? (const void*)g.tile_e : (const void*)g.norm, g.M,                   \
-      (uint32_t)(g.N >> 4 | g.K >> 6 << 17), (uint32_t)((moe) ? g.max_tiles : g.np | g.band << 16), g.inv_tiles, g.inv_band, g.inv_last
+  g.X, g.W, (moe) ? (const void*)(g.choice ? g.choice : g.n_tiles) : (const void*)g.ssq, (moe) ? (const void*)g.tile_e : (const void*)g.norm, g.M,                   \
+      (uint32_t)(g.N >> 4 | g.K >> 6 << 17), (uint32_t)((moe) ? g.max_tiles : g.np | g.band << 16), (uint32_t)((moe) ? (g.choice ? g.M * g.top : 0) : g.inv_tiles), g.inv_band, g.inv_last
 #define LM_HOT_IN(p, moe)                                                                                    \
   p.X = X; p.W = W; p.M = M; p.N = (int)(nk & 0x1ffffu) * 16; p.K = (int)(nk >> 17) * 64;                    \
   p.inv_tiles = inv_tiles; p.inv_band = inv_band; p.inv_last = inv_last;                                     \
-  if (moe) { p.n_tiles = (const int32_t*)aux0; p.tile_e = (const int32_t*)aux1; p.max_tiles = (int)np_band; } \
+  if (moe) {                                                                                                 \
+    p.choice = inv_tiles ? (const int32_t*)aux0 : nullptr; p.n_tiles = (const int32_t*)aux0; p.tile_e = (const int32_t*)aux1; \
+    p.max_tiles = (int)np_band;                                                                              \
+  }                                                                                                          \
   else { p.ssq = (const float*)aux0; p.norm = (const float*)aux1; p.np = (int)(np_band & 0xffffu); p.band = (int)(np_band >> 16); }
 
 template <typename T, int MB, int NB, int WAVES, int EPI>
@@ -221,7 +224,28 @@ __global__ __launch_bounds__(64 * WAVES, sizeof(T) == 2 && MB == 1 && NB < 3 ? 4
   }
   const int m0 = t * 16 * MB, nb0 = nt * NB;
   size_t wz = blockIdx.z * p.wz;
-  if (MOE) {
+  int entry = -1;  // of the tile's row l16, where the tile is found in the choices
+  if (MOE && MB == 1 && p.choice) {
+    // Experts in the order of their first entry, each with as many tiles of 16 entries as it needs; entries are lanes.
+    if (nb0 >= (p.N >> 4)) return;  // uniform, as what follows
+    const int n = (int)inv_tiles, e = lane < n ? p.choice[lane] : -1;
+    uint64_t left = ~0ull >> (64 - n), mine = 0;
+    int expert = -1, sub = t;  // its tile
+    while (left) {
+      const int c = __builtin_amdgcn_readlane(e, __builtin_ctzll(left));
+      const uint64_t same = __builtin_amdgcn_ballot_w64(e == c);
+      const int tiles = (__popcll(same) + 15) >> 4;
+      if (sub < tiles) { expert = c; mine = same; break; }
+      sub -= tiles;
+      left &= ~same;
+    }
+    if (expert < 0) return;
+    wz = (size_t)expert * p.wz;
+    const int at = __popcll(mine & ((1ull << lane) - 1));
+    const bool in = (mine >> lane & 1) && at >> 4 == sub;
+    const int got = __builtin_amdgcn_ds_permute((in ? at & 15 : 63) * 4, lane + 1);  // lanes 0 ... 15: their entry + 1, or 0
+    entry = __builtin_amdgcn_ds_bpermute(l16 * 4, got) - 1;
+  } else if (MOE) {
     if (t >= p.n_tiles[0] || nb0 >= (p.N >> 4)) return;  // uniform
     wz = (size_t)p.tile_e[t] * p.wz;
   }
@@ -234,7 +258,7 @@ __global__ __launch_bounds__(64 * WAVES, sizeof(T) == 2 && MB == 1 && NB < 3 ? 4
 #pragma unroll
   for (int j = 0; j < MB; ++j) {
     if (EPI == LM_MOE_UP && !p.sorted) {
-      const int e = p.ent[m0 + 16 * j + l16], r = min(max(e, 0) / p.top, p.x_rows - 1);
+      const int e = MB == 1 && p.choice ? entry : p.ent[m0 + 16 * j + l16], r = min(max(e, 0) / p.top, p.x_rows - 1);
       xr[j] = (const T*)p.X + (size_t)(r >> 4) * nsteps * 1024 + ((r & 15) + 16 * kg) * EP;
     } else if (MOE) {
       xr[j] = (const T*)p.X + (size_t)((m0 >> 4) + j) * nsteps * 1024 + lane * EP;
@@ -288,7 +312,7 @@ __global__ __launch_bounds__(64 * WAVES, sizeof(T) == 2 && MB == 1 && NB < 3 ? 4
   constexpr bool PRE = MB == 1 && (EPI == LM_IN_ATTN || EPI == LM_IN_GRU_STEP || EPI == LM_OUT);
   const int pm = min(m0 + l16, p.M - 1), pb = min(nb0 + min(wave, NB - 1), NBL - 1);  // row and block of unit `wave`
   LmPre e;
-  e.slot = e.pos = 0;
+  e.slot = entry; e.pos = 0;
   e.a = e.b = e.c = make_float4(0.f, 0.f, 0.f, 0.f);
   if (PRE && EPI != LM_OUT) {
     const int2 at = lm_where(p.rows, pm);

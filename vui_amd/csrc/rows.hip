@@ -1,9 +1,9 @@
 // Residual rows of sandwich layers: what a sublayer produced is normed and added, and the next sublayer's input is
 // normed, in one pass over the row.  fp32 throughout; a norm divides each of `groups` equal parts of the row by its own
 // root mean square.  One workgroup per row, which stays in registers, or in LDS where its parts do not fit the waves.  For
-// few rows the router of an expert layer reads the normed row here as well, and the rows are routed: each by its workgroup, the
-// last of which sorts their choices (4 rows of 2048, 32 experts: this launch 9.6 -> 11.8 us, that of choosing and sorting 7.1 us less;
-// sorted by every workgroup of the products for itself, those took 2 us more each: their weights wait for it).
+// few rows the router of an expert layer reads the normed row here as well, and every row is routed by its workgroup; which entries an
+// expert has, the products of those few rows find out for themselves (lm_gemm.hip: 4 rows of 2048, 32 experts, this launch with the last
+// row sorting the entries of all 12.0 us, so 8.0; up and down 0.2 us more each).
 #include "common.h"
 #include "lm.h"
 #include "route.h"
@@ -53,32 +53,7 @@ __device__ __forceinline__ void router_load(const RowArgs& p, const RouterAt& at
   for (int h = 0; h < 16 / EP; ++h) r.q[h] = *reinterpret_cast<const uint4*>(w + 64 * EP * h);
 }
 
-// The choices of all rows sorted by expert, every expert's padded to whole tiles.  One wave, an entry per lane.
-__device__ __forceinline__ void route_sort(const RouteArgs& p) {
-  const int lane = threadIdx.x & 63, n = p.M * p.top;
-  const int e = lane < n ? __hip_atomic_load(p.choice + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : -1;
-  uint64_t same = 0;
-  for (int i = 0; i < n; ++i) same |= (uint64_t)(__builtin_amdgcn_readlane(e, i) == e) << i;
-  const uint64_t below = (1ull << lane) - 1;
-  const int count = __popcll(same), at = __popcll(same & below), lead = same ? __builtin_ctzll(same) : 0;
-  const bool leads = lane < n && at == 0;
-  const int tiles = leads ? (count + p.tile_rows - 1) / p.tile_rows : 0;
-  int end = tiles;  // sum up to this lane
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int v = __shfl_up(end, o);
-    if (lane >= o) end += v;
-  }
-  const int first = __shfl(end - tiles, lead);
-  if (lane < n) p.ent[first * p.tile_rows + at] = lane;
-  if (leads) {
-    for (int t = 0; t < tiles; ++t) p.tile_e[first + t] = e;
-    for (int i = count; i < tiles * p.tile_rows; ++i) p.ent[first * p.tile_rows + i] = -1;
-  }
-  if (lane == 63) p.n_tiles[0] = end;
-}
-
-// router logits of the normed row in LDS, its choices, and (the last row) the sorted entries
+// router logits of the normed row in LDS, and its choices
 template <typename T, bool PRE>
 __device__ __forceinline__ void route_logits(const RowArgs& p, const float* v, float* red, int m, const RouterBlock<T> (&pre)[PRE ? RT_PRE : 1]) {
   constexpr int EP = Tl<T>::EP;
@@ -120,25 +95,10 @@ __device__ __forceinline__ void route_logits(const RowArgs& p, const float* v, f
     p.rlog[(size_t)m * p.experts16 + e] = s;
     red[e] = s;  // this column's first sum, read by this thread alone
   }
-  if (!p.arrived) return;
+  if (!p.route.choice) return;
   __syncthreads();
   if (wave) return;
   route_row(p.route, m, red);
-  if (p.M == 1) {  // the tiles of its experts are its choices as they come
-    __threadfence_block();
-    for (int i = lane; i < p.route.top * p.route.tile_rows; i += 64) p.route.ent[i] = i % p.route.tile_rows ? -1 : i / p.route.tile_rows;
-    if (lane < p.route.top) p.route.tile_e[lane] = p.route.choice[lane];
-    if (lane == 0) p.route.n_tiles[0] = p.route.top;
-    return;
-  }
-  // the choices went out by device-scope stores; once they have completed this row is counted
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  uint32_t last = 0;
-  if (lane == 0) {
-    last = __hip_atomic_fetch_add(p.arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)p.M - 1;
-    if (last) __hip_atomic_store(p.arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-  if (__builtin_amdgcn_readfirstlane(last)) route_sort(p.route);
 }
 
 template <typename T, int NT>
@@ -342,7 +302,7 @@ static int quad_go(const RowArgs& a, int wp, hipStream_t st) {
 }
 
 bool lm_rows_routes(int M, int experts16) { return M <= 16 && experts16 <= 128; }
-bool lm_rows_sorts(int M, int top) { return M == 1 || (M <= 16 && M * top <= 64); }  // a lane of one wave per entry
+bool lm_entries_in_wave(int M, int top) { return M <= 16 && M * top <= 64; }  // a lane per entry
 
 template <typename T, int NT>
 static int rows_go(const RowArgs& a, hipStream_t st) {

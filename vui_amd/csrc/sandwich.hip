@@ -110,7 +110,7 @@ size_t sandwich_carve(const vui_lm_config* c, const vui_lm_layer* layers, vui_lm
   TAKE(ent, int32_t*, en * 4);
   TAKE(tile_e, int32_t*, ti * 4);
   TAKE(n_tiles, int32_t*, 4);
-  TAKE(arrived, uint32_t*, (1 + R * ar) * 4);
+  TAKE(arrived, uint32_t*, R * ar * 4);
   if (x) x->arrived_row = (int)ar;
 #undef TAKE
   return off;
@@ -152,7 +152,7 @@ static int mixer(vui_lm_ctx* x, int l, int M, const LmRows& rows, hipStream_t st
     a.scale = L.scale; a.eps = x->c.norm_eps; a.rows = rows; a.d = d; a.raw = x->raw; a.ld = d.in_rows;
     a.q_norm = L.q_norm; a.k_norm = L.k_norm; a.temp_coef = L.temp_coef; a.temp_every = L.temp_every < 1 ? 1 : L.temp_every;
     a.bias = L.dist_bias; a.bias_len = L.bias_len; a.k_cache = L.k_cache; a.v_cache = L.v_cache;
-    a.q = x->qu; a.q_z = (size_t)x->R16 * d.dim64; a.part = x->part; a.arrived = x->arrived + 1; a.act = x->act;
+    a.q = x->qu; a.q_z = (size_t)x->R16 * d.dim64; a.part = x->part; a.arrived = x->arrived; a.act = x->act;
     if (!sig_step_fused(x->c.dtype, rows, d) && (rc = launch_sig_prep(a, st))) return rc;
     if (rows.seq && M >= x->attn_from && x->c.dtype == VUI_DTYPE_BF16 && sig_mfma_ok(d)) {
       rc = launch_sig_prompt(a, st);
@@ -187,9 +187,9 @@ static int feed_forward(vui_lm_ctx* x, int l, int M, const LmRows& rows, hipStre
   }
   if (!lm_rows_routes(M, d.experts16) && (rc = plain(x, d, rows, x->xt, L.w_router, L.router_bias, M, d.experts16, d.w64, x->rlog, st))) return rc;
   const RouteArgs r = routing(x, l, M);
-  if (!lm_rows_routes(M, d.experts16) || !lm_rows_sorts(M, L.top)) {
-    if ((rc = launch_moe_route(r, st))) return rc;
-  }
+  const bool found = lm_rows_routes(M, d.experts16) && lm_entries_in_wave(M, L.top);
+  if (!found && (rc = launch_moe_route(r, st))) return rc;
+  up.choice = found ? x->choice : nullptr;
   up.ent = x->ent; up.tile_e = x->tile_e; up.n_tiles = x->n_tiles; up.top = L.top; up.wz = (size_t)d.ff16 * d.w64;
   up.tile_rows = r.tile_rows;
   up.max_tiles = moe_max_tiles(M * L.top, L.experts, r.tile_rows);
@@ -199,7 +199,7 @@ static int feed_forward(vui_lm_ctx* x, int l, int M, const LmRows& rows, hipStre
   }
   if ((rc = launch_lm_gemm(x->c.dtype, LM_MOE_UP, up, 1, st))) return rc;
   LmGemm down = product(x, d, rows, x->ffa, L.w_down, M, d.out_rows, d.ff64);
-  down.ent = x->ent; down.tile_e = x->tile_e; down.n_tiles = x->n_tiles; down.top = L.top; down.wz = (size_t)d.out_rows * d.ff64;
+  down.ent = x->ent; down.tile_e = x->tile_e; down.n_tiles = x->n_tiles; down.choice = up.choice; down.top = L.top; down.wz = (size_t)d.out_rows * d.ff64;
   down.max_tiles = up.max_tiles; down.tile_rows = r.tile_rows; down.out = x->y; down.ldo = d.out_rows;
   return launch_lm_gemm(x->c.dtype, LM_MOE_DOWN, down, 1, st);
 }
@@ -221,7 +221,7 @@ int sandwich_layers(vui_lm_ctx* x, const int64_t* tokens, int M, const LmRows& r
   };
   ahead(0);
   RowArgs emb = r;
-  emb.tokens = tokens; emb.rows = rows; emb.clear = x->arrived; emb.n_clear = 1 + M * x->arrived_row;
+  emb.tokens = tokens; emb.rows = rows; emb.clear = x->arrived; emb.n_clear = M * x->arrived_row;
   int rc = launch_lm_rows(emb, st);
   for (int l = 0; l < n && !rc; ++l) {
     const vui_lm_layer& L = x->layers[l];
@@ -240,7 +240,7 @@ int sandwich_layers(vui_lm_ctx* x, const int64_t* tokens, int M, const LmRows& r
       RowArgs mid = r;
       if (L.experts > 0 && lm_rows_routes(M, d.experts16)) {
         mid.w_router = L.w_router; mid.router_bias = L.router_bias; mid.experts16 = d.experts16; mid.rlog = x->rlog;
-        mid.route = routing(x, l, M); mid.arrived = lm_rows_sorts(M, L.top) ? x->arrived : nullptr;
+        if (lm_entries_in_wave(M, L.top)) mid.route = routing(x, l, M);
       }
       if ((rc = launch_lm_rows(mid, st))) return rc;
       if ((rc = feed_forward(x, l, M, rows, st))) return rc;

@@ -208,7 +208,7 @@ __device__ __forceinline__ void sig_normed(const SigRow<DB>& row, int dim16, int
 // puts key and value into its operands and appends them (workgroups of further heads of the group write the same).
 // Bound by its chain: place of the row, keys and values, scores, weights, sums, the pieces' meeting.  What the first loads need is in
 // registers (see lm_gemm.hip); queries, the new key and value and their norms' weights do not depend on the row's place and go out first, the
-// first tile before the query's norm: 4 rows behind 500 positions, 16 heads of 128, 10.5 -> @@ us per launch, 1 row behind 150 8.1 -> @@.
+// first tile before the query's norm: 4 rows behind 500 positions, 16 heads of 128, 10.4 -> 8.2 us per launch, 1 row behind 150 8.1 -> 7.4.
 template <int DB, int VT, bool STEP>
 __global__ __launch_bounds__(256) void sig_piece_mfma_kernel(int2* where, const void* raw, const void* k_cache, const void* v_cache, int ld, int s64, int S,
                                                             uint32_t heads, uint32_t dims, uint32_t splits, const SigAttnArgs p0) {
