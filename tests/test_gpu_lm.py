@@ -87,6 +87,22 @@ def test_prompt_against_token_by_token_and_portions(dt):
             assert e < tol, (cuts[:4], e)
 
 
+@pytest.mark.parametrize("want", [[], [39], [0, 1, 2, 39], [39, 0, 17, 17], [5, 4], list(range(40))])
+def test_wanted_positions_in_any_order(want, monkeypatch):
+    """Logits that lie in the result as the passes leave them, and others, in one native call and in several; none at all."""
+    from vui_amd.lm import TokenLM
+
+    cfg = U.mixed()
+    sd, toks = U.weights(cfg, 3), U.tokens(40, cfg["vocab"], 4)
+    ref = O.forward(cfg, sd, toks)
+    for rows in (2048, 16):
+        monkeypatch.setattr(TokenLM, "PREFILL_CHUNK", rows)
+        with U.engine(cfg, sd).new_row() as row:
+            got = row.extend(toks, want)
+            assert got.shape == (len(want), cfg["vocab"])
+            assert not want or U.err(got, ref[want]) < U.TOL[F32]
+
+
 @BOTH
 def test_prompts_longer_than_one_native_call(dt, monkeypatch):
     """Wanted places in any order, in several calls of at most 40 positions, some calls without any."""

@@ -265,6 +265,13 @@ class TokenLM:
         _lib.check(nat.lib.vui_lm_decode(nat.handle, tokens.data_ptr(), _lib.ptr(slot_idx), self.cache.seq_lens.data_ptr(),
                                          _lib.ptr(seq_inc), B, logits_out.data_ptr(), stream), "vui_lm_decode")
 
+    def _index(self, values: "list[int]", dtype) -> Tensor:
+        """A list on the device, by way of pinned memory: a copy from anywhere else waits for all that the stream holds, which made a
+        prompt's call as long as its kernels and its host work together."""
+        if torch.cuda.is_current_stream_capturing():  # a replay would read memory that is long given back
+            raise RuntimeError("a prompt whose logits are wanted cannot be captured")
+        return torch.tensor(values, dtype=dtype, pin_memory=True).to(self.device, non_blocking=True)
+
     def prefill(self, tokens: Tensor, slot: int, pos0: int, want: "list[int]") -> Tensor:
         """tokens (T) int64 on the device, appended to `slot` at pos0 (its length); logits (len(want), vocab) fp32 of
         the positions want (indices into tokens)."""
@@ -281,12 +288,14 @@ class TokenLM:
         for t0 in range(0, T, step):
             n = min(step, T - t0)
             mine = [k for k in order if t0 <= want[k] < t0 + n]
-            idx = torch.tensor([want[k] - t0 for k in mine], dtype=torch.int32, device=self.device)
-            part = torch.empty(len(mine), self.config.vocab, dtype=torch.float32, device=self.device)
+            # neighbouring rows of the result in its order get their logits at once
+            idx = self._index([want[k] - t0 for k in mine], torch.int32) if mine else None
+            whole = bool(mine) and mine == list(range(mine[0], mine[0] + len(mine)))
+            part = out[mine[0]:mine[0] + len(mine)] if whole else torch.empty(len(mine), self.config.vocab, dtype=torch.float32, device=self.device)
             tk = tokens[t0:t0 + n].contiguous()
             _lib.check(nat.lib.vui_lm_prefill(nat.handle, tk.data_ptr(), n, slot, pos0 + t0, self.cache.seq_lens.data_ptr(),
-                                              idx.data_ptr() if mine else None, len(mine), part.data_ptr() if mine else None, st),
+                                              _lib.ptr(idx), len(mine), part.data_ptr() if mine else None, st),
                        "vui_lm_prefill")
-            if mine:
-                out[mine] = part
+            if mine and not whole:
+                out[self._index(mine, torch.long)] = part
         return out
