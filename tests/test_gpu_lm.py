@@ -524,6 +524,19 @@ def test_large_products_of_a_prompt(large, T):
     assert U.err(whole, ref[:T]) < 0.012 and U.err(whole, parts) < 0.012
 
 
+@pytest.mark.parametrize("T", [17, 32, 33, 97, 128, 129, 256])
+def test_small_products_of_a_prompt(large, T):
+    """Products of at most one tile per compute unit, eight waves each: the output projection on tiles of 32 x 16 up to 128 rows and of
+    32 x 32 up to 256, the last row alone in its block or its block full; against 64 bits and against the same tokens in portions
+    of 16, which take another kernel.  Bounds as for the large products above."""
+    eng, toks, ref = large
+    with eng.new_row() as row:
+        whole = row.extend(toks[:T], range(T)).clone()
+        row.reset()
+        parts = torch.cat([row.extend(toks[i:min(i + 16, T)], range(min(16, T - i))).clone() for i in range(0, T, 16)])
+    assert U.err(whole, ref[:T]) < 0.012 and U.err(whole, parts) < 0.012
+
+
 @pytest.mark.parametrize("T", [640, 700])
 def test_lone_tiles_of_a_prompt(T):
     """Products of fewer 64 x 64 tiles than compute units, whose K is split over two halves of waves: an odd number of 64 columns in

@@ -276,8 +276,8 @@ __global__ __launch_bounds__(64 * WAVES, sizeof(T) == 2 && MB == 1 && NB < 3 ? 4
     wr[i] = (const T*)p.W + wz + (size_t)min(nb0 + i, NBL - 1) * nsteps * 1024 + lane * EP;
 
   // U steps' loads go out together (a step beyond the wave's last re-reads that one and is not multiplied); the first ones now
-  constexpr int U = WAVES >= 8 && sizeof(T) == 2 ? 4 : 1;
   constexpr bool EARLY = WAVES >= 8 && sizeof(T) == 2;
+  constexpr int U = !EARLY ? 1 : MB == 1 ? 4 : 2;
   uint4 xa[U][MB][P], wa[U][NB][P];
   auto load = [&](int s) {
 #pragma unroll
@@ -659,6 +659,21 @@ static int pick_wide(int tile, const LmGemm& g, hipStream_t st) {
   }
 }
 
+// More rows, as long as no large tile is quicker.  Few tiles are a wave's chain of trips to memory, not its width: with one tile per CU at
+// most eight waves split K and request two steps at a time, and where half the CUs would have none a tile is 16 features wide.  us per
+// launch, four waves on 32 x 32 / eight / eight on 32 x 16: 50 x 2048 x 6144 18.2 / 15.5 / 12.3, 110 x 1024 x 4096 10.0 / 8.7 / 7.4,
+// 30 x 768 x 2816 7.7 / 6.6 / 5.4; at 224 tiles 7.8 / 6.5 / 7.4 (200 x 1024 x 2048), at 256 11.4 / 9.2 / 10.6 (100 x 2048 x 4096).
+// With more tiles than CUs they are each other's company: 400 x 6400 x 768 (1742 tiles) 16.2 with four waves, 23 with eight.
+template <typename T, int NB, int EPI>
+static int many(const LmGemm& g, int nz, hipStream_t st) {
+  if constexpr (sizeof(T) == 2 && NB == 2) {
+    const long tiles = (long)((g.M + 31) / 32) * ((g.N + 31) / 32) * nz;
+    if (tiles <= 128) return go<T, 2, 1, 8, EPI>(g, nz, st);
+    if (tiles <= 256) return go<T, 2, 2, 8, EPI>(g, nz, st);
+  }
+  return go<T, 2, NB, 4, EPI>(g, nz, st);
+}
+
 // up to 16 rows: one row block, more waves per tile (the weights are streamed once, latency counts)
 template <typename T>
 static int pick(int epi, const LmGemm& g, int nz, hipStream_t st) {
@@ -688,15 +703,15 @@ static int pick(int epi, const LmGemm& g, int nz, hipStream_t st) {
     if (epi == LM_MOE_DOWN) return go<T, 1, 1, 16, LM_MOE_DOWN>(g, nz, st);
   }
   switch (epi) {
-    case LM_IN_ATTN: return few ? go<T, 1, 2, 8, LM_IN_ATTN>(g, nz, st) : go<T, 2, 2, 4, LM_IN_ATTN>(g, nz, st);
+    case LM_IN_ATTN: return few ? go<T, 1, 2, 8, LM_IN_ATTN>(g, nz, st) : many<T, 2, LM_IN_ATTN>(g, nz, st);
     case LM_IN_GRU_STEP: return go<T, 1, 3, 8, LM_IN_GRU_STEP>(g, nz, st);
-    case LM_IN_GRU_SEQ: return few ? go<T, 1, 3, 8, LM_IN_GRU_SEQ>(g, nz, st) : go<T, 2, 3, 4, LM_IN_GRU_SEQ>(g, nz, st);
-    case LM_OUT: return few ? go<T, 1, 1, 16, LM_OUT>(g, nz, st) : go<T, 2, 2, 4, LM_OUT>(g, nz, st);
-    case LM_LOGITS: return few ? go<T, 1, 2, 8, LM_LOGITS>(g, nz, st) : go<T, 2, 2, 4, LM_LOGITS>(g, nz, st);
-    case LM_HEAD: return few ? go<T, 1, 2, 8, LM_HEAD>(g, nz, st) : go<T, 2, 2, 4, LM_HEAD>(g, nz, st);
-    case LM_PROJ: return few ? go<T, 1, 2, 8, LM_PROJ>(g, nz, st) : go<T, 2, 2, 4, LM_PROJ>(g, nz, st);
-    case LM_PLAIN: return few ? go<T, 1, 1, 16, LM_PLAIN>(g, nz, st) : go<T, 2, 2, 4, LM_PLAIN>(g, nz, st);
-    case LM_ACT: return few ? go<T, 1, 2, 8, LM_ACT>(g, nz, st) : go<T, 2, 2, 4, LM_ACT>(g, nz, st);
+    case LM_IN_GRU_SEQ: return few ? go<T, 1, 3, 8, LM_IN_GRU_SEQ>(g, nz, st) : many<T, 3, LM_IN_GRU_SEQ>(g, nz, st);
+    case LM_OUT: return few ? go<T, 1, 1, 16, LM_OUT>(g, nz, st) : many<T, 2, LM_OUT>(g, nz, st);
+    case LM_LOGITS: return few ? go<T, 1, 2, 8, LM_LOGITS>(g, nz, st) : many<T, 2, LM_LOGITS>(g, nz, st);
+    case LM_HEAD: return few ? go<T, 1, 2, 8, LM_HEAD>(g, nz, st) : many<T, 2, LM_HEAD>(g, nz, st);
+    case LM_PROJ: return few ? go<T, 1, 2, 8, LM_PROJ>(g, nz, st) : many<T, 2, LM_PROJ>(g, nz, st);
+    case LM_PLAIN: return few ? go<T, 1, 1, 16, LM_PLAIN>(g, nz, st) : many<T, 2, LM_PLAIN>(g, nz, st);
+    case LM_ACT: return few ? go<T, 1, 2, 8, LM_ACT>(g, nz, st) : many<T, 2, LM_ACT>(g, nz, st);
     case LM_MOE_UP: return few ? go<T, 1, 2, 8, LM_MOE_UP>(g, nz, st) : go<T, 2, 2, 4, LM_MOE_UP>(g, nz, st);
     case LM_MOE_DOWN: return few ? go<T, 1, 2, 8, LM_MOE_DOWN>(g, nz, st) : go<T, 2, 2, 4, LM_MOE_DOWN>(g, nz, st);
   }
