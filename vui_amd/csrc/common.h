@@ -205,5 +205,20 @@ __device__ __forceinline__ void st_dev(float* p, float a, float b) {
 __device__ __forceinline__ uint64_t ld_dev(const float* p) {
   return __hip_atomic_load(reinterpret_cast<const uint64_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+// The same 16 bytes at a time, at byte `at` of a buffer: beyond its size nothing is fetched and zeros come back.
+typedef float dev_f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t dev_u32x4 __attribute__((ext_vector_type(4)));
+#define DEV_SCOPE 16  // sc1
+#define DEV_NOWHERE (1u << 30)  // beyond every buffer
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t dev_buffer(const void* p, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00027000);
+}
+__device__ __forceinline__ void st_dev4(__amdgpu_buffer_rsrc_t b, uint32_t at, const float* v) {
+  const dev_f32x4 x = {v[0], v[1], v[2], v[3]};
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(dev_u32x4, x), b, (int)at, 0, DEV_SCOPE);
+}
+__device__ __forceinline__ dev_f32x4 ld_dev4(__amdgpu_buffer_rsrc_t b, uint32_t at) {
+  return __builtin_bit_cast(dev_f32x4, __builtin_amdgcn_raw_buffer_load_b128(b, (int)at, 0, DEV_SCOPE));
+}
 __device__ __forceinline__ float lo_f(uint64_t v) { return __uint_as_float((uint32_t)v); }
 __device__ __forceinline__ float hi_f(uint64_t v) { return __uint_as_float((uint32_t)(v >> 32)); }

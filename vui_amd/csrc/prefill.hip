@@ -782,33 +782,27 @@ __global__ __launch_bounds__(64 * PfDirect<HD32>::WAVES) void pf_direct_attn_ker
   }
   if (nsp > 1) {
     const size_t set = (size_t)h * gridDim.y + blockIdx.y;
-    float* part = a.part + set * nsp * (DT * 256);
+    const __amdgpu_buffer_rsrc_t part = dev_buffer(a.part + set * nsp * (DT * 256), (uint32_t)(nsp * DT * 1024));
     float* ml = a.ml + set * nsp * 32;
 #pragma unroll
-    for (int i = 0; i < ND; ++i) {
-      const int d = wave + i * WAVES;
-      if (d < DT) {
-        float* mine = part + ((size_t)(sp * DT + d) * 64 + lane) * 4;
-        st_dev(mine, o[i][0], o[i][1]);
-        st_dev(mine + 2, o[i][2], o[i][3]);
-      }
-    }
+    for (int i = 0; i < ND; ++i)
+      if (wave + i * WAVES < DT) st_dev4(part, (uint32_t)(((sp * DT + wave + i * WAVES) * 64 + lane) * 16), o[i]);
     if (tid < 16) st_dev(ml + sp * 32 + tid * 2, M, den);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (tid == 0) *s_last = __hip_atomic_fetch_add(a.count + set, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == a.before + nsp - 1;
     __syncthreads();
     if (!*s_last) return;
-    uint64_t xm[PF_SPLITS], xo[ND][PF_SPLITS][2];
+    // One compute unit takes in all parts, which is what this tail waits for: whole lines, and nothing for splits and blocks that are not
+    // there.  (Eight bytes at a time of eight splits however many there are: 9.1 us per launch of 16 positions behind 700, so 8.4.)
+    uint64_t xm[PF_SPLITS];
+    dev_f32x4 xo[ND][PF_SPLITS];
 #pragma unroll
-    for (int s = 0; s < PF_SPLITS; ++s) {  // a split that is not there reads the last one again and weighs nothing
-      const int t = min(s, nsp - 1);
-      xm[s] = ld_dev(ml + t * 32 + l16 * 2);
+    for (int s = 0; s < PF_SPLITS; ++s) {
+      xm[s] = ld_dev(ml + min(s, nsp - 1) * 32 + l16 * 2);
 #pragma unroll
-      for (int i = 0; i < ND; ++i) {
-        const float* x = part + ((size_t)(t * DT + min(wave + i * WAVES, DT - 1)) * 64 + lane) * 4;
-        xo[i][s][0] = ld_dev(x); xo[i][s][1] = ld_dev(x + 2);
-      }
+      for (int i = 0; i < ND; ++i)
+        xo[i][s] = ld_dev4(part, wave + i * WAVES < DT ? (uint32_t)(((s * DT + wave + i * WAVES) * 64 + lane) * 16) : DEV_NOWHERE);
     }
     M = -INFINITY;
 #pragma unroll
@@ -822,8 +816,8 @@ __global__ __launch_bounds__(64 * PfDirect<HD32>::WAVES) void pf_direct_attn_ker
       den = fmaf(f, hi_f(xm[s]), den);
 #pragma unroll
       for (int i = 0; i < ND; ++i) {
-        o[i][0] = fmaf(f, lo_f(xo[i][s][0]), o[i][0]); o[i][1] = fmaf(f, hi_f(xo[i][s][0]), o[i][1]);
-        o[i][2] = fmaf(f, lo_f(xo[i][s][1]), o[i][2]); o[i][3] = fmaf(f, hi_f(xo[i][s][1]), o[i][3]);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[i][r] = fmaf(f, xo[i][s][r], o[i][r]);
       }
     }
   }
