@@ -90,6 +90,13 @@ int64_t vui_codec_block_scratch_bytes(const vui_codec_config* cfg, int32_t n_fra
 int vui_codec_decode_block(vui_codec* c, const int64_t* codes, int32_t n_frames, int32_t n_q, float* audio_out, void* scratch,
                            int64_t scratch_bytes, vui_stream_t stream);
 
+/* The same for a whole clip, whose products are larger: up to vui_codec_clip_frames(c) frames, which is max_seq or 256 at the
+ * reference's dims, whichever is less (fewer where a buffer of them would exceed 1 GiB, never fewer than a block). */
+int32_t vui_codec_clip_frames(const vui_codec* c);
+int64_t vui_codec_clip_scratch_bytes(const vui_codec_config* cfg, int32_t n_frames);
+int vui_codec_decode_clip(vui_codec* c, const int64_t* codes, int32_t n_frames, int32_t n_q, float* audio_out, void* scratch,
+                          int64_t scratch_bytes, vui_stream_t stream);
+
 /* The one-column steps of a frame (codebook rows ... first upsampling conv) run as one persistent kernel when
  * the device can keep 256 workgroups resident and the dimensions fit, otherwise as separate launches (same
  * sums in another order).  enable = 1/0 switches the persistent form on/off, -1 only queries; returns 1 when

@@ -146,3 +146,18 @@ def test_scratch_memory_follows_the_frames_of_a_block():
     cc.max_seq = 5
     assert lib.vui_codec_block_scratch_bytes(C.byref(cc), 5) == size[4]
     assert lib.vui_codec_block_scratch_bytes(C.byref(cc), 6) == -22
+
+
+def test_scratch_memory_of_a_clip():
+    """vui_codec_clip_scratch_bytes: what a block of as many frames takes, up to max_seq or 256 frames, or as many as
+    a grid's second dimension has tiles for, but never less than a block."""
+    from vui_amd import _lib
+
+    lib, cc = _lib.load(), K.CodecConfig().to_c()
+    size = lambda n: lib.vui_codec_clip_scratch_bytes(C.byref(cc), n)
+    assert [size(n) for n in range(1, 33)] == [lib.vui_codec_block_scratch_bytes(C.byref(cc), n) for n in range(1, 33)]
+    assert size(cc.max_seq) > 0 and size(0) == size(cc.max_seq + 1) == -22
+    cc.max_seq = 4000
+    assert size(256) > size(255) and size(257) == -22
+    cc.rates[3] = 40  # 25600 samples per frame: 20 frames are 2^19
+    assert size(20) > 0 and size(32) > size(31) and size(33) == -22

@@ -188,6 +188,29 @@ def test_full_dims_against_reference_vectors(full):
     assert st.shape[-1] == 4 * 1920
 
 
+@pytest.mark.parametrize("T", [33, 65, 250])
+def test_clips_in_one_pass(full, T, monkeypatch):
+    """A clip of more frames than a block, up to the decoder's window, against the same frames streamed in portions of 32; where
+    its memory cannot be had, in shorter passes.  Each is within 6e-6 to 9e-6 of 64 bits at 93 frames (2 seeds); 5e-5 is three times
+    what two of them can differ by."""
+    d, sd, dec, _ = full
+    codes = torch.randint(0, d.codebook_size, (1, d.n_codebooks, T), generator=torch.Generator().manual_seed(T)).cuda()
+    whole = dec(codes).clone()
+    with dec.streaming(1):
+        parts = torch.cat([dec(codes[:, :, i:i + 32]).clone() for i in range(0, T, 32)], dim=-1)
+    assert float(whole.abs().max()) > 0.05 and err(whole, parts.cpu()) < 5e-5
+    empty, refused = torch.empty, []
+
+    def short(*size, **kw):
+        if kw.get("dtype") == torch.uint8 and size[0] > 260e6:
+            refused.append(size[0])
+            raise torch.OutOfMemoryError("no room")
+        return empty(*size, **kw)
+
+    monkeypatch.setattr(torch, "empty", short)
+    assert err(dec(codes), parts.cpu()) < 5e-5 and refused
+
+
 def _digest(a):
     a = a.detach().cpu().reshape(-1).double()
     return np.array([a.sum().item(), a.abs().sum().item(), *a[:4].tolist(), *a[-4:].tolist()])

@@ -130,6 +130,9 @@ SIGNATURES = {
     "vui_codec_block_frames": (C.c_int32, [_P]),
     "vui_codec_block_scratch_bytes": (_L, [C.POINTER(CodecConfigC), C.c_int32]),
     "vui_codec_decode_block": (_I, [_P, _P, C.c_int32, C.c_int32, _P, _P, _L, _P]),
+    "vui_codec_clip_frames": (C.c_int32, [_P]),
+    "vui_codec_clip_scratch_bytes": (_L, [C.POINTER(CodecConfigC), C.c_int32]),
+    "vui_codec_decode_clip": (_I, [_P, _P, C.c_int32, C.c_int32, _P, _P, _L, _P]),
     "vui_codec_status": (_L, [_P, _P]),
     "vui_codec_persistent": (_I, [_P, _I]),
     "vui_codec_workgroups": (_I, [_P, _I]),

@@ -208,8 +208,8 @@ class QwenCodecDecoder:
         self.hop = self.cfg.hop
         self._streaming = False
         self._frames = 0  # frames since the last reset (of the calls made here)
-        self._block = int(lib.vui_codec_block_frames(h))
-        self._block_bytes = [0] + [int(lib.vui_codec_block_scratch_bytes(C.byref(cc), n + 1)) for n in range(self._block)]
+        self._block, self._clip = int(lib.vui_codec_block_frames(h)), int(lib.vui_codec_clip_frames(h))
+        self._cc, self._pass_bytes = cc, {}  # bytes by frames of a pass
         self._cap_stream = torch.cuda.Stream(device=self.device)
         self._graphs: dict[int, object] = {}
         self._stream_codes_in = torch.zeros(self.cfg.n_codebooks, dtype=torch.long, device=self.device)
@@ -348,15 +348,25 @@ class QwenCodecDecoder:
         flat = audio.view(-1)
         st = torch.cuda.current_stream().cuda_stream
         scratch = None
+        most = self._clip
         t = 0
-        while t < T:  # blocks of frames; single frames past the decoder's window, where only the status flag is left to raise
-            n = min(T - t, self._block, self.cfg.max_seq - self._frames)
+        while t < T:  # passes of equal length; single frames past the decoder's window, where only the status flag is left to raise
+            left = min(T - t, self.cfg.max_seq - self._frames)
+            n = -(-left // -(-left // most)) if left > 0 else 1
             if n > 1:
-                if scratch is None:  # blocks do not grow
-                    scratch = torch.empty(self._block_bytes[n], dtype=torch.uint8, device=self.device)
-                _lib.check(self.lib.vui_codec_decode_block(self.handle, ct[t].data_ptr(), n, n_q, flat[t * self.hop:].data_ptr(),
-                                                           scratch.data_ptr(), scratch.numel(), st),
-                           "vui_codec_decode_block")
+                if scratch is None:  # passes do not grow
+                    if n not in self._pass_bytes:
+                        self._pass_bytes[n] = int(self.lib.vui_codec_clip_scratch_bytes(C.byref(self._cc), n))
+                    try:
+                        scratch = torch.empty(self._pass_bytes[n], dtype=torch.uint8, device=self.device)
+                    except torch.OutOfMemoryError:  # 8 MB per frame: shorter passes need less
+                        if n <= self._block:
+                            raise
+                        most = max(n // 2, self._block)
+                        continue
+                _lib.check(self.lib.vui_codec_decode_clip(self.handle, ct[t].data_ptr(), n, n_q, flat[t * self.hop:].data_ptr(),
+                                                          scratch.data_ptr(), scratch.numel(), st),
+                           "vui_codec_decode_clip")
                 self._frames += n
             else:
                 n = 1

@@ -1396,10 +1396,26 @@ struct Arena {
   }
 };
 
-// Frames that one pass takes at most (vui_codec_decode_block).  At 32 the weights pass once per 32 frames (3 us of a
-// frame's 84) and a product's launch costs 0.15 us per frame; the buffers, scratch memory of the caller's, take 8 MB per frame.
+// Frames that one pass takes at most: CV_BLOCK by vui_codec_decode_block, CV_CLIP by vui_codec_decode_clip, which is as large as
+// products still gain: the weights pass once, the trunk's hundred launches of 5-9 us for a few columns come once, and 32 frames of the
+// last stages are a grid and a half.  us of a clip in passes of 32 / 64 / 96 / 128 / 250 frames: 250 frames 15775 / 13583 / 12500 / 11196 /
+// 10380, 128 7856 / 6804 / 6536 / 5618, 93 5844 / 5329 / 4505.  The buffers, scratch memory of the caller's, take 8 MB per frame.
 #define CV_BLOCK 32
+#define CV_CLIP 256
 static int block_frames(const vui_codec_config& k) { return k.max_seq < CV_BLOCK ? k.max_seq : CV_BLOCK; }
+// A clip's buffers stay under 1 GiB each (offsets are 32 bits) and its tiles of 16 columns within a grid's second dimension.
+static int clip_frames(const vui_codec_config& k) {
+  long wide = std::max({2 * k.codebook_dim, k.vq_dim, k.latent_dim, k.d_model, 3 * k.n_heads * k.head_dim, k.mlp_dim}), T = 1;
+  for (int i = 0; i < k.n_up; ++i) { T *= k.up_ratios[i]; wide = std::max(wide, 4 * T * k.latent_dim); }
+  for (int i = 0, dim = k.decoder_dim; ; ++i, dim /= 2) {
+    wide = std::max(wide, T * dim);
+    if (i == k.n_rates) break;
+    T *= k.rates[i];
+    wide = std::max(wide, T * (dim / 2));
+  }
+  const long n = std::min({(long)CV_CLIP, (long)k.max_seq, (1l << 28) / (wide + 1), (1l << 19) / T});
+  return (int)std::max(n, (long)block_frames(k));
+}
 
 // Rings and buffers of one frame, and of each its twin: a plain buffer of a whole block of frames with the history
 // columns in front.  A ring of 32 frames for both would need no copies of histories (two launches per block), but its
@@ -1478,7 +1494,8 @@ static void cv_shape(CvGemm& g, int splits) {
 }
 
 // Chooses tile width, splits and kernel for g.T columns.
-static CvScratch cv_plan(CvGemm& g) {
+// A clip's products split no further than the scratch memory sized for blocks reaches.
+static CvScratch cv_plan(CvGemm& g, size_t part_cap = CVW_PARTS, size_t cnt_cap = SIZE_MAX) {
   const int U = g.taps * (g.Cin / 32), M = g.M, T = g.T;
   auto tiles = [&](int tt) { return (M / 16) * ((T + 16 * tt - 1) / (16 * tt)); };
   // few units and few tiles: a launch of cv_cols_kernel is shorter than the large tiles' two (768 channels x 128 columns, 1x1: 14 / 8 us)
@@ -1491,7 +1508,7 @@ static CvScratch cv_plan(CvGemm& g) {
       const WideTile& w = kWide[i];
       if (M % w.bm) continue;
       const int cols = (T + w.bn - 1) / w.bn * w.bn, tiles = (M / w.bm) * (cols / w.bn);
-      for (int sp = 1; sp <= 16 && (sp == 1 || (U / sp >= 4 && (size_t)sp * M * cols <= CVW_PARTS)); ++sp) {
+      for (int sp = 1; sp <= 16 && (sp == 1 || (U / sp >= 4 && (size_t)sp * M * cols <= std::min(part_cap, (size_t)CVW_PARTS))); ++sp) {
         const int wgs = (tiles * sp + 255) / 256;
         const double c = (wgs / 2 * CVW_PAIR + wgs % 2 * CVW_ALONE) * ((U + sp - 1) / sp) * w.unit + (sp > 1 ? 6 + 1e-6 * sp * M * T : 0);
         if (cost && c >= cost) continue;
@@ -1511,6 +1528,7 @@ static CvScratch cv_plan(CvGemm& g) {
   const int target = T <= 16 ? 512 : 256;
   const int sp = std::max(1, std::min(std::min((2 * target + tiles(g.tt)) / (2 * tiles(g.tt)), most), std::min(8, G)));
   cv_shape(g, sp);
+  if (g.splits > 1 && ((size_t)tiles(g.tt) * g.splits * g.tt * 256 > part_cap || (size_t)tiles(g.tt) > cnt_cap)) cv_shape(g, 1);
   return CvScratch{(size_t)tiles(g.tt) * g.splits * g.tt * 256, (size_t)tiles(g.tt)};
 }
 
@@ -1792,7 +1810,7 @@ static int cv_build(vui_codec* cc, const vui_codec_config* c, const void* const*
     }
   }
   if (block_need) *block_need = (int64_t)rings.block(frames).floats * 4;
-  const int n_hist = rings.histories(), n_blocks = block_frames(*c) + 1;
+  const int n_hist = rings.histories(), n_blocks = clip_frames(*c) + 1;
   CvHist* hist_dev = (CvHist*)ar.take((sizeof(CvHist) * n_hist * n_blocks + 3) / 4);
   if (need) *need = (int64_t)ar.off;
   if (part_need) *part_need = part_floats;
@@ -1819,7 +1837,7 @@ static int cv_build(vui_codec* cc, const vui_codec_config* c, const void* const*
     cc->trunk = tk;
     cc->trunk_steps = trunk_steps;
     if (part_floats > part_cap || cnt_ints > cnt_cap) { vui_set_error("codec: internal scratch sizing"); return VUI_EINVAL; }
-    cc->ctr = ctr; cc->cnt = cnt; cc->cnt_ints = cnt_cap;
+    cc->ctr = ctr; cc->cnt = cnt; cc->cnt_ints = cnt_cap; cc->part_floats = part_cap;
     cc->state0 = (float*)(ws + state_begin);
     cc->state_floats = (state_end - state_begin) / 4;
     cc->hist = hist_dev;
@@ -1991,25 +2009,38 @@ int32_t vui_codec_block_frames(const vui_codec* c) {
   return block_frames(c->cfg);
 }
 
-static int block_check(const vui_codec_config& c, int32_t n_frames) {
-  if (n_frames >= 1 && n_frames <= block_frames(c)) return VUI_OK;
-  vui_set_error("codec: %d frames outside [1, %d]", n_frames, block_frames(c));
+int32_t vui_codec_clip_frames(const vui_codec* c) {
+  if (!c) { vui_set_error("NULL codec"); return VUI_EINVAL; }
+  return clip_frames(c->cfg);
+}
+
+static int frames_check(int32_t n_frames, int most) {
+  if (n_frames >= 1 && n_frames <= most) return VUI_OK;
+  vui_set_error("codec: %d frames outside [1, %d]", n_frames, most);
   return VUI_EINVAL;
 }
 
-int64_t vui_codec_block_scratch_bytes(const vui_codec_config* c, int32_t n_frames) {
-  if (cv_check(c) || block_check(*c, n_frames)) return VUI_EINVAL;
+static int64_t pass_scratch(const vui_codec_config* c, int32_t n_frames) {
   int64_t need = 0;
   if (n_frames > 1 && cv_build(nullptr, c, nullptr, nullptr, nullptr, nullptr, 0, 0, nullptr, nullptr, n_frames, &need)) return VUI_EINVAL;
   return need;
 }
 
-int vui_codec_decode_block(vui_codec* c, const int64_t* codes, int32_t n_frames, int32_t n_q, float* audio_out, void* scratch,
-                           int64_t scratch_bytes, vui_stream_t stream) {
-  if (!c) { vui_set_error("NULL codec"); return VUI_EINVAL; }
+int64_t vui_codec_block_scratch_bytes(const vui_codec_config* c, int32_t n_frames) {
+  if (cv_check(c) || frames_check(n_frames, block_frames(*c))) return VUI_EINVAL;
+  return pass_scratch(c, n_frames);
+}
+
+int64_t vui_codec_clip_scratch_bytes(const vui_codec_config* c, int32_t n_frames) {
+  if (cv_check(c) || frames_check(n_frames, clip_frames(*c))) return VUI_EINVAL;
+  return pass_scratch(c, n_frames);
+}
+
+static int decode_pass(vui_codec* c, const int64_t* codes, int32_t n_frames, int32_t n_q, float* audio_out, void* scratch, int64_t scratch_bytes,
+                       int most, vui_stream_t stream) {
   if (!codes || !audio_out) { vui_set_error("NULL argument"); return VUI_EINVAL; }
   if (n_q < 1 || n_q > c->cfg.n_codebooks) { vui_set_error("n_q=%d outside [1,%d]", n_q, c->cfg.n_codebooks); return VUI_EINVAL; }
-  if (block_check(c->cfg, n_frames)) return VUI_EINVAL;
+  if (frames_check(n_frames, most)) return VUI_EINVAL;
   if (n_frames == 1) return vui_codec_decode_frame(c, codes, n_q, audio_out, stream);
   if (!scratch || ((uintptr_t)scratch) & 255) { vui_set_error("codec: the scratch memory must be given and 256-byte aligned"); return VUI_EINVAL; }
   const CvBlock& block = c->blocks[n_frames];
@@ -2028,7 +2059,7 @@ int vui_codec_decode_block(vui_codec* c, const int64_t* codes, int32_t n_frames,
     if (s.kind == 0) {
       s.g.T *= n_frames; s.g.nf = n_frames;
       s.g.in = twin(s.g.in); s.g.res = twin(s.g.res); s.g.out_raw = twin(s.g.out_raw); s.g.out_act = twin(s.g.out_act);
-      cv_plan(s.g);
+      cv_plan(s.g, c->part_floats, c->cnt_ints);
       int rc = launch_cv_gemm(s.g, c->w_nt != 0, st);
       if (rc) return rc;
     } else if (s.kind == 1) {
@@ -2049,6 +2080,18 @@ int vui_codec_decode_block(vui_codec* c, const int64_t* codes, int32_t n_frames,
   hipLaunchKernelGGL(cv_final_kernel, dim3((fin.T + FIN_TW - 1) / FIN_TW), dim3(256), (size_t)(fin.C * (FIN_TW + fin.k - 1) + 256 + fin.C * fin.k) * 4, st, fin);
   HIP_TRY(hipGetLastError());
   return VUI_OK;
+}
+
+int vui_codec_decode_block(vui_codec* c, const int64_t* codes, int32_t n_frames, int32_t n_q, float* audio_out, void* scratch,
+                           int64_t scratch_bytes, vui_stream_t stream) {
+  if (!c) { vui_set_error("NULL codec"); return VUI_EINVAL; }
+  return decode_pass(c, codes, n_frames, n_q, audio_out, scratch, scratch_bytes, block_frames(c->cfg), stream);
+}
+
+int vui_codec_decode_clip(vui_codec* c, const int64_t* codes, int32_t n_frames, int32_t n_q, float* audio_out, void* scratch,
+                          int64_t scratch_bytes, vui_stream_t stream) {
+  if (!c) { vui_set_error("NULL codec"); return VUI_EINVAL; }
+  return decode_pass(c, codes, n_frames, n_q, audio_out, scratch, scratch_bytes, clip_frames(c->cfg), stream);
 }
 
 int64_t vui_codec_status(vui_codec* c, vui_stream_t stream) {
