@@ -316,14 +316,18 @@ __global__ __launch_bounds__(64 * CV_NW, 4) void cv_cols_kernel(const CvGemm p) 
 // of bf16 products in the first, what hipBLASLt reaches at 8192^3), 1x1 19 / 30 / 32 / 33 -> 16 / 29 / 26 / 29 (3-4 % more with the clamp
 // of cv_split2); error of 93 frames against 64 bits 4.1e-6 -> 3.9e-6.
 // Tiles of BM x BN = 128 x 128 (or what divides M) of four waves through LDS, three planes of each operand: a K step is one (tap,
-// 32-channel) unit, fetched into registers while the one before it is multiplied, split on the way to LDS.  One buffer: two
-// workgroups of a CU overlap better than the steps of one (eight waves with two buffers and one to three units in flight: 75 us of
-// the 384-channel convolution instead of 63).
+// 32-channel) unit, fetched into registers while the one before it is multiplied, split on the way to LDS.  A group's taps follow each
+// other, so that its columns, with the taps' halo, are fetched, split and stored once for all of them (per tap they were two thirds of
+// the vector instructions and a quarter of what LDS moves, beside matrix instructions that it nearly holds up); where two workgroups of a
+// CU still fit, weights have a second buffer and a unit one barrier.  93 frames, 7-tap convolutions of 768 / 384 / 192 / 96 channels
+// 214 / 247 / 275 / 227 -> 195 / 211 / 240 / 198 us, the clip 4681 -> 4259, 250 frames 10883 -> 9726.  Eight waves with two buffers of both
+// and one to three units in flight: 75 us of the 384-channel convolution of 32 frames when this form took 63.
 // Where the tiles are fewer than the CUs their units are split over workgroups, and cv_finish_kernel adds the parts.
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 cv_bf16x8;
 
 #define CVW_RUN 4
+#define CVW_HALO 56  // columns that the taps reach beyond a tile: 6 x 9
 // In LDS a row's (or column's) 32 channels of a plane are four pieces of 16 bytes; a piece's place turns with the row, so that 16-byte
 // reads of eight rows fall on different banks.
 __device__ __forceinline__ int cv_at(int row, int piece) { return row * 32 + 8 * (piece ^ (row >> 2 & 3)); }
@@ -398,15 +402,16 @@ __device__ __forceinline__ void cv_finish_rows(const CvGemm& p, const CvBases& b
 
 template <int MI, int NI, int WM, int WN>
 __global__ __launch_bounds__(256, 2) void cv_wide_kernel(const CvGemm p) {
-  constexpr int NT = 256, BM = 32 * MI * WM, BN = 32 * NI * WN, BS = BN + 8;
-  constexpr int NA = (BM * 8 + NT - 1) / NT, NB = 32 * BN / NT;  // 16-byte / 4-byte loads per thread and step
-  static_assert(WM * WN == 4 && NT % BN == 0 && NB % 8 == 0, "four waves, whole columns per thread");
-  constexpr int PL = (BM + BN) * 32;  // bf16 of one plane of both operands
-  constexpr int OPS = 3 * PL * 2;
+  constexpr int NT = 256, BM = 32 * MI * WM, BN = 32 * NI * WN, BS = BN + 8, CW = BN + CVW_HALO;
+  constexpr int NA = (BM * 8 + NT - 1) / NT, NB = (CW * 4 + NT - 1) / NT;  // 16-byte loads per thread and unit, pieces of 8 channels and group
+  static_assert(WM * WN == 4 && NT % BN == 0, "four waves, whole columns per thread");
+  constexpr int PA = BM * 64, PB = CW * 64;  // bytes of one plane of the weights, of the columns
+  constexpr bool TWO = 2 * (6 * PA + 3 * PB) <= 160 * 1024;  // a second buffer for weights: two workgroups still share a CU
+  constexpr int OPS = (TWO ? 6 : 3) * PA + 3 * PB;
   __shared__ __align__(16) char raw[OPS > BM * BS * 4 ? OPS : BM * BS * 4];  // the operands, then the sums
   float* const lds = reinterpret_cast<float*>(raw);
-  auto la = [&](int plane, int row, int piece) { return reinterpret_cast<bf16_t*>(raw) + plane * PL + cv_at(row, piece); };
-  auto lb = [&](int plane, int col, int piece) { return la(plane, 0, 0) + BM * 32 + cv_at(col, piece); };
+  auto la = [&](int buf, int plane, int row, int piece) { return reinterpret_cast<bf16_t*>(raw + 3 * PB + (buf * 3 + plane) * PA) + cv_at(row, piece); };
+  auto lb = [&](int plane, int col, int piece) { return reinterpret_cast<bf16_t*>(raw + plane * PB) + cv_at(col, piece); };
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int l32 = lane & 31, h = lane >> 5, wm = wave % WM, wn = wave / WM;
   // Workgroups go round the eight XCDs, whose L2s are their own: each gets a contiguous range of the tiles, columns slowest, so that
@@ -429,23 +434,36 @@ __global__ __launch_bounds__(256, 2) void cv_wide_kernel(const CvGemm p) {
 #pragma unroll
     for (int n = 0; n < NI; ++n) acc[i][n] = sum[i][n] = zero;
 
-  const int bc = tid % BN, bk = tid / BN * NB;  // this thread's column and first channel of a step
   floatx4 ra[NA];  // native vectors: an array of HIP's float4 structs stayed in scratch memory
-  float rb[NB];
-  const uint32_t woff = (tid >> 3) * p.Cin + (tid & 7) * 4, xoff = bk * p.in.rs + bc;
-  int tap = ub / G, grp = ub - tap * G;
-  auto fetch = [&]() {
+  float rb[NB][8];
+  // This thread's pieces of a group's columns, BN and the taps' halo: eight channels of a column each.
+  const int W = BN + (p.taps - 1) * p.dil;
+  int pc[NB];  // column and piece
+  uint32_t xoff[NB];
+#pragma unroll
+  for (int i = 0; i < NB; ++i) {
+    const int q = min(tid + i * NT, 4 * W - 1), k = (q >= W) + (q >= 2 * W) + (q >= 3 * W), c = q - k * W;
+    pc[i] = c * 4 + k;
+    xoff[i] = (uint32_t)(8 * k * p.in.rs + c);
+  }
+  const uint32_t woff = (tid >> 3) * p.Cin + (tid & 7) * 4;
+  auto fetch_w = [&](int tap, int grp) {
     const float* wp = p.W + ((size_t)tap * p.M + m0) * p.Cin + grp * 32;  // uniform, with offsets of the thread's own
 #pragma unroll
     for (int i = 0; i < NA; ++i)
       if ((i + 1) * (NT / 8) <= BM || (tid >> 3) + i * (NT / 8) < BM) ra[i] = *reinterpret_cast<const floatx4*>(wp + (size_t)i * (NT / 8) * p.Cin + woff);
-    // a block's buffer has no end to turn at; columns behind T are whatever is there: they reach no output
-    const float* xp = p.in.p + (size_t)grp * 32 * p.in.rs + t0 + tap * p.dil;
-#pragma unroll
-    for (int i = 0; i < NB; ++i) rb[i] = xp[(size_t)i * p.in.rs + xoff];
-    if (++grp == G) { grp = 0; ++tap; }
   };
-  auto stage = [&]() {
+  auto fetch_x = [&](int grp) {
+    // a block's buffer has no end to turn at; columns behind T are whatever is there: they reach no output
+    const float* xp = p.in.p + (size_t)grp * 32 * p.in.rs + t0;
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+      if ((i + 1) * NT <= 4 * BN || tid + i * NT < 4 * W) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) rb[i][e] = xp[(size_t)e * p.in.rs + xoff[i]];
+      }
+  };
+  auto stage_w = [&](int buf) {
 #pragma unroll
     for (int i = 0; i < NA; ++i)
       if ((i + 1) * (NT / 8) <= BM || (tid >> 3) + i * (NT / 8) < BM) {
@@ -453,36 +471,48 @@ __global__ __launch_bounds__(256, 2) void cv_wide_kernel(const CvGemm p) {
         cv_split2(ra[i][0], ra[i][1], q[0].x, q[1].x, q[2].x);
         cv_split2(ra[i][2], ra[i][3], q[0].y, q[1].y, q[2].y);
 #pragma unroll
-        for (int k = 0; k < 3; ++k) *reinterpret_cast<uint2*>(la(k, (tid >> 3) + (NT / 8) * i, (tid & 7) >> 1) + (tid & 1) * 4) = q[k];
+        for (int k = 0; k < 3; ++k) *reinterpret_cast<uint2*>(la(buf, k, (tid >> 3) + (NT / 8) * i, (tid & 7) >> 1) + (tid & 1) * 4) = q[k];
       }
+  };
+  auto stage_x = [&]() {
 #pragma unroll
-      for (int i = 0; i < NB; i += 8) {
+    for (int i = 0; i < NB; ++i)
+      if ((i + 1) * NT <= 4 * BN || tid + i * NT < 4 * W) {
         uint4 q[3];
-        cv_split2(rb[i], rb[i + 1], q[0].x, q[1].x, q[2].x);
-        cv_split2(rb[i + 2], rb[i + 3], q[0].y, q[1].y, q[2].y);
-        cv_split2(rb[i + 4], rb[i + 5], q[0].z, q[1].z, q[2].z);
-        cv_split2(rb[i + 6], rb[i + 7], q[0].w, q[1].w, q[2].w);
+        cv_split2(rb[i][0], rb[i][1], q[0].x, q[1].x, q[2].x);
+        cv_split2(rb[i][2], rb[i][3], q[0].y, q[1].y, q[2].y);
+        cv_split2(rb[i][4], rb[i][5], q[0].z, q[1].z, q[2].z);
+        cv_split2(rb[i][6], rb[i][7], q[0].w, q[1].w, q[2].w);
 #pragma unroll
-        for (int k = 0; k < 3; ++k) *reinterpret_cast<uint4*>(lb(k, bc, (bk + i) >> 3)) = q[k];
+        for (int k = 0; k < 3; ++k) *reinterpret_cast<uint4*>(lb(k, pc[i] >> 2, pc[i] & 3)) = q[k];
       }
   };
   auto frag = [](const bf16_t* q) { return __builtin_bit_cast(cv_bf16x8, *reinterpret_cast<const uint4*>(q)); };
+  int grp = ub / p.taps, tap = ub - grp * p.taps;  // a group's taps one after the other
   if (ub < ue) {
-    fetch();
-    stage();
+    fetch_w(tap, grp);
+    fetch_x(grp);
+    stage_w(0);
+    stage_x();
   }
   __syncthreads();
   for (int u = ub; u < ue; ++u) {
-    if (u + 1 < ue) fetch();
+    const int col = tap * p.dil, buf = TWO ? (u - ub) & 1 : 0;
+    const bool more = u + 1 < ue, turn = tap + 1 == p.taps;  // uniform; turn: the next unit is another group's
+    if (turn) { tap = 0; ++grp; } else ++tap;
+    if (more) {
+      fetch_w(tap, grp);
+      if (turn) fetch_x(grp);
+    }
 #pragma unroll
     for (int j = 0; j < 2; ++j) {  // 16 channels: a lane holds eight of its row or column
       cv_bf16x8 a[3][MI], x[3][NI];
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
 #pragma unroll
-        for (int i = 0; i < MI; ++i) a[k][i] = frag(la(k, (wm * MI + i) * 32 + l32, 2 * j + h));
+        for (int i = 0; i < MI; ++i) a[k][i] = frag(la(buf, k, (wm * MI + i) * 32 + l32, 2 * j + h));
 #pragma unroll
-        for (int n = 0; n < NI; ++n) x[k][n] = frag(lb(k, (wn * NI + n) * 32 + l32, 2 * j + h));
+        for (int n = 0; n < NI; ++n) x[k][n] = frag(lb(k, (wn * NI + n) * 32 + l32 + col, 2 * j + h));
       }
       // {part of the weight, part of the input}
       constexpr int PAIR[6][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};
@@ -500,9 +530,11 @@ __global__ __launch_bounds__(256, 2) void cv_wide_kernel(const CvGemm p) {
 #pragma unroll
         for (int n = 0; n < NI; ++n) { sum[i][n] += acc[i][n]; acc[i][n] = zero; }
     }
-    __syncthreads();
-    if (u + 1 < ue) {
-      stage();
+    if (TWO && more) stage_w(buf ^ 1);
+    if (!TWO || turn || !more) __syncthreads();
+    if (more) {
+      if (!TWO) stage_w(0);
+      if (turn) stage_x();
       __syncthreads();
     }
   }
@@ -1500,7 +1532,8 @@ static CvScratch cv_plan(CvGemm& g, size_t part_cap = CVW_PARTS, size_t cnt_cap 
   auto tiles = [&](int tt) { return (M / 16) * ((T + 16 * tt - 1) / (16 * tt)); };
   // few units and few tiles: a launch of cv_cols_kernel is shorter than the large tiles' two (768 channels x 128 columns, 1x1: 14 / 8 us)
   const bool few = U <= 32 && tiles(1) <= 512;
-  if (g.nf > 1 && T >= CV_WIDE_T && !few && M % 32 == 0 && g.in_mode == IN_PLAIN && g.epi != EPI_SILU_PAIR) {
+  if (g.nf > 1 && T >= CV_WIDE_T && !few && M % 32 == 0 && g.in_mode == IN_PLAIN && g.epi != EPI_SILU_PAIR &&
+      (g.taps - 1) * g.dil <= CVW_HALO) {
     // Tile and splits: what the workgroups of a CU take, in pairs, and for split tiles the second launch and its traffic.
     size_t part = 0;
     double cost = 0;
