@@ -184,6 +184,24 @@ def test_pieces_of_two_tiles(rows, heads, rank, rot):
 
 
 @BOTH
+@pytest.mark.parametrize("rows, heads, rank, vdim", [(1, 16, 560, 150), (3, 2, 70, 33), (16, 5, 300, 100)])
+def test_shares_of_a_value_expansion(rows, heads, rank, vdim, dt):
+    """Workgroups of two to eight blocks of 16 value features (10, 3, 7 of them) and one to sixteen rows, whose waves share 9, 2 and 5 steps
+    of K; 256 columns of a row at a time (rank 560: the last third is 64), up to 26 pieces."""
+    cfg = U.config([U.attn(heads=heads, dim=16, rot_dim=8, vdim=vdim, kv_rank=rank)], ff=None)
+    sd = U.weights(cfg, 21)
+    eng = U.engine(cfg, sd, dt, max_rows=rows, max_seq=840)
+    lens = [830, 5, 64, 300][:rows] + [7 + 9 * i for i in range(rows - 4)]
+    seqs = [U.tokens(n + 2, cfg["vocab"], 40 + n) for n in lens]
+    held = [eng.new_row() for _ in lens]
+    for row, s, n in zip(held, seqs, lens):
+        row.extend(s[:n], [])
+    got = [eng.decode_step(held, torch.tensor([s[n + t] for s, n in zip(seqs, lens)], device="cuda")).clone() for t in range(2)]
+    for i, (s, n) in enumerate(zip(seqs, lens)):
+        assert U.err(torch.stack([g[i] for g in got]), O.forward(cfg, sd, s)[n:]) < U.TOL[dt], (i, n)
+
+
+@BOTH
 def test_slots_used_again(dt):
     """A slot that held a long sequence serves short ones; nothing of the old keys, latents or state shows."""
     cfg = U.mixed()

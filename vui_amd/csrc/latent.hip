@@ -80,7 +80,7 @@ __global__ __launch_bounds__(256) void latent_query_kernel(const void* w_uk_t, c
 // A row that sees len keys is cut into pieces of this many (whole 32-key tiles), at most ns of them.  With more than
 // four rows a piece has two tiles at least: there are pieces enough, and fewer are merged faster.
 __host__ __device__ __forceinline__ int latent_least(int M) { return M > 4 ? 64 : 32; }
-__device__ __forceinline__ int latent_chunk(int len, int ns, int M) { return max(((len + ns - 1) / ns + 31) & ~31, latent_least(M)); }
+__host__ __device__ __forceinline__ int latent_chunk(int len, int ns, int M) { return max(((len + ns - 1) / ns + 31) & ~31, latent_least(M)); }
 // keys [lo, hi) of piece sp
 __device__ __forceinline__ void latent_range(int len, int ns, int M, int sp, int& lo, int& hi) {
   const int chunk = latent_chunk(len, ns, M);
@@ -309,50 +309,63 @@ __global__ __launch_bounds__(256, 2) void latent_attn_mfma_kernel(int2* where, c
 
 // ---- merge of the pieces, value expansion through W_uv[h], head gate: up to 16 rows x 128 value dims of one head ----
 template <typename T>
-__global__ __launch_bounds__(512) void latent_value_kernel(int2* where, const void* w_uv, float* part, float* part_ml, int heads, int M, int S, uint32_t ns_rpw,
+__global__ __launch_bounds__(512) void latent_value_kernel(int2* where, const void* w_uv, float* part, float* part_ml, int heads, int M, int S, uint32_t split,
                                                            int rank64, int vdim16, const LatentArgs p0) {
   LatentArgs p = p0;  // what the first loads need is in registers (see lm_gemm.hip)
   p.rows.where = where; p.w_uv = w_uv; p.part = part; p.part_ml = part_ml; p.heads = heads; p.M = M; p.rows.S = S;
-  p.n_splits = (int)(ns_rpw & 0xffffu); p.d.rank64 = rank64; p.d.vdim16 = vdim16;
-  const int rpw = (int)(ns_rpw >> 16);
+  p.n_splits = (int)(split & 0xffu); p.d.rank64 = rank64; p.d.vdim16 = vdim16;
+  const int rpw = (int)(split >> 8 & 0xffu), nbw = (int)(split >> 16);  // rows and blocks of 16 features of this workgroup
   extern __shared__ __align__(16) unsigned char lv_raw[];
+  __shared__ __align__(16) float red[8][256];
   T* xs = (T*)lv_raw;  // 16 x rank64, tiled
   constexpr int EP = Tl<T>::EP, P = 16 / EP, PRE = sizeof(T) == 2 ? 8 : 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int h = blockIdx.x, m0 = blockIdx.z * rpw, R = p.d.rank64, ns = p.n_splits, nk = R >> 6;
-  const int nb = blockIdx.y * 8 + wave, nvb = p.d.vdim16 >> 4;
+  const int parts = 8 / nbw, kp = wave / nbw, k0 = nk * kp / parts, k1 = nk * (kp + 1) / parts;  // the waves of a block share its K
+  const int nb = blockIdx.y * nbw + wave % nbw, nvb = p.d.vdim16 >> 4;
   const int nrow = min(rpw, p.M - m0);
   // the first weights are requested ahead of the merge
   const T* wv = (const T*)p.w_uv + ((size_t)h * nvb + min(nb, nvb - 1)) * nk * 1024 + lane * EP;
   uint4 wp[PRE][P];
 #pragma unroll
   for (int k = 0; k < PRE; ++k)
+    if (k0 + k < k1) {  // uniform
 #pragma unroll
-    for (int i = 0; i < P; ++i) wp[k][i] = *reinterpret_cast<const uint4*>(wv + (size_t)min(k, nk - 1) * 1024 + 64 * EP * i);
-  const float gate = p.gate[(size_t)min(m0 + (lane & 15), p.M - 1) * p.d.heads16 + h];
-  for (int it = wave; it < nrow * nk; it += 8) {  // a wave merges 64 columns of a row
-    const int r = it / nk, k = (it - r * nk) * 64 + lane;
-    const int m = m0 + r, len = min(max(lm_where(p.rows, m).y + 1, 1), p.rows.S);
+      for (int i = 0; i < P; ++i) wp[k][i] = *reinterpret_cast<const uint4*>(wv + (size_t)(k0 + k) * 1024 + 64 * EP * i);
+    }
+  const int m16 = min(m0 + (lane & 15), p.M - 1), pos16 = lm_where(p.rows, m16).y;  // of row lane % 16
+  const float gate = p.gate[(size_t)m16 * p.d.heads16 + h];
+  const int nc = (R + 255) >> 8;
+  for (int it = wave; it < nrow * nc; it += 8) {  // a wave merges 256 columns of a row
+    const int r = nc == 1 ? it : it / nc, c = (it - r * nc) * 256 + lane * 4;
+    const int m = m0 + r, len = min(max(__builtin_amdgcn_readlane(pos16, r) + 1, 1), p.rows.S);
     const int chunk = latent_chunk(len, ns, p.M), np = (len + chunk - 1) / chunk;  // pieces that exist
     const size_t piece = ((size_t)m * p.heads + h) * ns;
     const float2 ml = *reinterpret_cast<const float2*>(p.part_ml + 2 * (piece + min(lane, np - 1)));
-    const float* pc = p.part + piece * R + k;
-    float v[16];  // sixteen loads in flight; a piece beyond the last gets weight zero
+    const __amdgpu_buffer_rsrc_t pc = dev_buffer(p.part + piece * R, (uint32_t)(np * R * 4));  // nothing is fetched for pieces beyond the last
+    auto load = [&](int s) {
+      return __builtin_bit_cast(dev_f32x4, __builtin_amdgcn_raw_buffer_load_b128(pc, c < R ? (s * R + c) * 4 : (int)DEV_NOWHERE, 0, 0));
+    };
+    dev_f32x4 v[16];  // in flight together
 #pragma unroll
-    for (int u = 0; u < 16; ++u) v[u] = pc[(size_t)min(u, np - 1) * R];
-    const float M = wave_max(lane < np ? ml.x : -INFINITY);
-    float w = lane < np ? expf(ml.x - M) : 0.f;
+    for (int u = 0; u < 16; ++u) v[u] = load(u);
+    const float mx = wave_max(lane < np ? ml.x : -INFINITY);
+    float w = lane < np ? expf(ml.x - mx) : 0.f;
     w /= wave_sum(w * ml.y);
-    float o = 0.f;
+    float o[4] = {0.f, 0.f, 0.f, 0.f};
     for (int s0 = 0;;) {
 #pragma unroll
-      for (int u = 0; u < 16; ++u) o = fmaf(lane_f(w, min(s0 + u, 63)), s0 + u < np ? v[u] : 0.f, o);
+      for (int u = 0; u < 16; ++u) {
+        const float f = lane_f(w, min(s0 + u, 63));  // zero beyond the last piece
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = fmaf(f, v[u][e], o[e]);
+      }
       s0 += 16;
       if (s0 >= np) break;
 #pragma unroll
-      for (int u = 0; u < 16; ++u) v[u] = pc[(size_t)min(s0 + u, np - 1) * R];
+      for (int u = 0; u < 16; ++u) v[u] = load(s0 + u);
     }
-    El<T>::st(xs + tl_off<T>(r, k, R), o);
+    if (c < R) Tl<T>::st4(xs + tl_off<T>(r, c, R), o);
   }
   // rows without a position: their products are dropped, but must be numbers
   for (int i = threadIdx.x; i < (16 - nrow) * (R / 4); i += 512) {
@@ -360,7 +373,6 @@ __global__ __launch_bounds__(512) void latent_value_kernel(int2* where, const vo
     Tl<T>::st4(xs + tl_off<T>(nrow + i / (R / 4), (i % (R / 4)) * 4, R), z);
   }
   __syncthreads();
-  if (nb >= nvb) return;
   tl_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
   auto step = [&](int k, const uint4* a) {
 #pragma unroll
@@ -369,17 +381,22 @@ __global__ __launch_bounds__(512) void latent_value_kernel(int2* where, const vo
   };
 #pragma unroll
   for (int k = 0; k < PRE; ++k)
-    if (k < nk) step(k, wp[k]);
-  for (int k = PRE; k < nk; ++k) {
+    if (k0 + k < k1) step(k0 + k, wp[k]);
+  for (int k = k0 + PRE; k < k1; ++k) {
     uint4 a[P];
 #pragma unroll
     for (int i = 0; i < P; ++i) a[i] = *reinterpret_cast<const uint4*>(wv + (size_t)k * 1024 + 64 * EP * i);
     step(k, a);
   }
-  const int m = m0 + (lane & 15);
-  if ((lane & 15) >= nrow) return;
+  if (parts > 1) {
+    *reinterpret_cast<tl_f32x4*>(&red[wave][lane * 4]) = acc;
+    __syncthreads();
+    if (kp) return;
+    for (int q = 1; q < parts; ++q) acc += *reinterpret_cast<const tl_f32x4*>(&red[wave + q * nbw][lane * 4]);
+  }
+  if (nb >= nvb || (lane & 15) >= nrow) return;
   const float v[4] = {acc[0] * gate, acc[1] * gate, acc[2] * gate, acc[3] * gate};
-  Tl<T>::st4((T*)p.act + tl_off<T>(m, h * p.d.vdim16 + nb * 16 + 4 * (lane >> 4), p.d.out_k), v);
+  Tl<T>::st4((T*)p.act + tl_off<T>(m0 + (lane & 15), h * p.d.vdim16 + nb * 16 + 4 * (lane >> 4), p.d.out_k), v);
 }
 
 // ---- expanded form for long blocks of one sequence (bf16): one workgroup per 16 queries and head ----
@@ -560,19 +577,39 @@ int launch_latent_attn(const LatentArgs& a, hipStream_t st) {
   return VUI_OK;
 }
 
+// Rows and feature blocks of a workgroup: what a CU takes in (the rows' pieces, which every split of the features reads again, and W_uv,
+// which every split of the rows does) at 60 KB a us, 1.2 us per round of merges, 3 us for the rest, all of it again for every 256
+// workgroups, of which a CU holds one.  us per launch, a row and all 128 features until 192 workgroups / two merges of 64 columns side by side ->
+// so: 16 heads of rank 512, 1 row behind 1200 7.8 -> 6.5 (two blocks), 16 rows behind 300 6.2 -> 5.4 (two rows, four blocks), a prompt of
+// 50 15.3 -> 7.8 (eight rows, four blocks); 8 heads, 16 rows behind 1400 7.0 -> 6.0.
 int launch_latent_value(const LatentArgs& a, hipStream_t st) {
-  // rows per workgroup: all 16 of a tile only when there are enough heads and rows to fill the chip without
-  int rpw = 1;
-  while (rpw < 16 && a.M * a.heads > 192 * rpw) rpw *= 2;
-  const dim3 grid(a.heads, (a.d.vdim16 / 16 + 7) / 8, (a.M + rpw - 1) / rpw);
   const bool f32 = a.dtype == VUI_DTYPE_F32;
+  const int nvb = a.d.vdim16 / 16, R = a.d.rank64;
+  int pieces = (a.n_splits + 1) / 2;  // of a row; known for a prompt
+  if (a.rows.seq) {
+    const int len = std::min(a.rows.pos0 + a.M, a.rows.S), chunk = latent_chunk(len, a.n_splits, a.M);
+    pieces = (len + chunk - 1) / chunk;
+  }
+  int rpw = 1, nbw = 8;
+  float best = 0;
+  const float in_row = pieces * R * 4 / 60e3f, in_block = 16 * R * (f32 ? 4 : 2) / 60e3f;
+  for (int rs = 0; rs <= 4 && (rs == 0 || 1 << (rs - 1) < a.M); ++rs) {
+    const int tiles = (a.M + (1 << rs) - 1) >> rs, r = std::min(1 << rs, a.M);
+    for (int bs = 3; bs >= 1; --bs) {
+      const int n = a.heads * ((nvb + (1 << bs) - 1) >> bs) * tiles;
+      const float c = ((n + 255) >> 8) * (3 + r * in_row + std::min(1 << bs, nvb) * in_block + 1.2f * ((r * ((R + 255) >> 8) + 7) >> 3));
+      if (best == 0 || c < best) { best = c; rpw = 1 << rs; nbw = 1 << bs; }
+    }
+  }
+  const dim3 grid(a.heads, (nvb + nbw - 1) / nbw, (a.M + rpw - 1) / rpw);
+  const uint32_t split = (uint32_t)a.n_splits | (uint32_t)rpw << 8 | (uint32_t)nbw << 16;
   const size_t lds = (size_t)16 * a.d.rank64 * (f32 ? 4 : 2);
   if (lds > 64 * 1024) {
     HIP_TRY(hipFuncSetAttribute(f32 ? (const void*)latent_value_kernel<float> : (const void*)latent_value_kernel<bf16_t>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   }
-  if (f32) hipLaunchKernelGGL(latent_value_kernel<float>, grid, dim3(512), lds, st, a.rows.where, a.w_uv, a.part, a.part_ml, a.heads, a.M, a.rows.S, (uint32_t)a.n_splits | (uint32_t)rpw << 16, a.d.rank64, a.d.vdim16, a);
-  else hipLaunchKernelGGL(latent_value_kernel<bf16_t>, grid, dim3(512), lds, st, a.rows.where, a.w_uv, a.part, a.part_ml, a.heads, a.M, a.rows.S, (uint32_t)a.n_splits | (uint32_t)rpw << 16, a.d.rank64, a.d.vdim16, a);
+  if (f32) hipLaunchKernelGGL(latent_value_kernel<float>, grid, dim3(512), lds, st, a.rows.where, a.w_uv, a.part, a.part_ml, a.heads, a.M, a.rows.S, split, a.d.rank64, a.d.vdim16, a);
+  else hipLaunchKernelGGL(latent_value_kernel<bf16_t>, grid, dim3(512), lds, st, a.rows.where, a.w_uv, a.part, a.part_ml, a.heads, a.M, a.rows.S, split, a.d.rank64, a.d.vdim16, a);
   HIP_TRY(hipGetLastError());
   return VUI_OK;
 }
