@@ -117,8 +117,22 @@ __device__ __forceinline__ uint32_t cv_div(uint32_t i, uint32_t inv) { return in
 // (eight loads of a float per unit and block of columns, issuing which took 3-4 us) and the outputs four to a lane, us per launch of a
 // single frame / so: 7 taps of 768 channels x 32 columns 16.5 / 11.8, 384 x 160 14.8 / 11.9, 192 x 640 13.0 / 10.7, 96 x 1920 10.7 / 9.2; one tap
 // 9.1 / 6.4, 7.9 / 5.6, 8.3 / 5.9, 7.4 / 5.6; the frame 572 / 482.
+// The first fourteen words of scalar arguments are in registers when a kernel starts, a struct is a trip to memory (0.2-0.35 us): what the
+// counter's, the weights' and the columns' addresses need comes twice, ahead of the struct and in it, and the waves' shares of the
+// (group, tap) units as numbers instead of divisions (at most seven taps): 0.5-0.9 us of a
+// launch of 6-12, a streamed frame 481 -> 457 us.
+#define CV_HOT const float *W, const float *in_p, const int *ctr, int M, int Cin, int T, uint32_t taps, int rs, int mask, uint32_t per_chunk, uint32_t inv_xcols
+static uint32_t cv_taps(const CvGemm& g) {
+  const uint32_t taps = g.taps, step = CV_NW / taps;
+  return taps | (uint32_t)g.dil << 8 | step << 16 | (CV_NW - step * taps) << 20 | (256 / taps + 1) << 23;
+}
+#define CV_HOT_ARGS(g) g.W, g.in.p, g.ctr, g.M, g.Cin, g.T, cv_taps(g), g.in.rs, g.in.mask, (uint32_t)g.per | (uint32_t)g.chunk << 16, g.inv_xcols
 template <int TT, bool NT>
-__global__ __launch_bounds__(64 * CV_NW, 4) void cv_cols_kernel(const CvGemm p) {
+__global__ __launch_bounds__(64 * CV_NW, 4) void cv_cols_kernel(CV_HOT, const CvGemm p0) {
+  CvGemm p = p0;
+  p.W = W; p.in.p = const_cast<float*>(in_p); p.ctr = ctr; p.M = M; p.Cin = Cin; p.T = T; p.taps = (int)(taps & 0xffu); p.dil = (int)(taps >> 8 & 0xffu);
+  p.in.rs = rs; p.in.mask = mask; p.per = (int)(per_chunk & 0xffffu); p.chunk = (int)(per_chunk >> 16); p.inv_xcols = inv_xcols;
+  p.xcols = min(T, 16 * TT) + (p.taps - 1) * p.dil;
   constexpr int NU = CvUnits<TT>::N, NTH = 64 * CV_NW, RED = CV_NW * TT * 256;
   extern __shared__ __align__(16) float lds[];
   float* red = lds;
@@ -126,7 +140,7 @@ __global__ __launch_bounds__(64 * CV_NW, 4) void cv_cols_kernel(const CvGemm p) 
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int r16 = lane & 15, g = lane >> 4;
   const int m0 = blockIdx.x * 16, t0 = blockIdx.y * (16 * TT), tile = blockIdx.y * gridDim.x + blockIdx.x, part_idx = blockIdx.z;
-  const int M = p.M, Cin = p.Cin, G = Cin >> 5;
+  const int G = Cin >> 5;
   const int gb = part_idx * p.per, ge = min(G, gb + p.per);
   const int halo = (p.taps - 1) * p.dil, cols = p.xcols - halo, S = p.chunk * 32 + 4;
 
@@ -135,7 +149,7 @@ __global__ __launch_bounds__(64 * CV_NW, 4) void cv_cols_kernel(const CvGemm p) 
   float4 a[NU][2];
   int off[NU];  // of the unit's first column in LDS
   const uint32_t w_lane = (uint32_t)(r16 * Cin + g * 8);
-  const int g_step = CV_NW / p.taps, t_step = CV_NW - g_step * p.taps, g_first = wave / p.taps, t_first = wave - g_first * p.taps;
+  const int g_step = (int)(taps >> 16 & 15u), t_step = (int)(taps >> 20 & 7u), g_first = (int)(wave * (taps >> 23) >> 8), t_first = wave - g_first * p.taps;
   auto load_a = [&](int gc, int n) {
     int gl = g_first, tap = t_first;
 #pragma unroll
@@ -1991,8 +2005,8 @@ static int launch_cv_gemm(const CvGemm& g, bool w_nt, hipStream_t st) {
   const int lds = cv_lds(g);
 #define CV_TT(TT_)                                                                              \
   do {                                                                                          \
-    if (w_nt) hipLaunchKernelGGL((cv_cols_kernel<TT_, true>), grid, block, lds, st, g);         \
-    else hipLaunchKernelGGL((cv_cols_kernel<TT_, false>), grid, block, lds, st, g);             \
+    if (w_nt) hipLaunchKernelGGL((cv_cols_kernel<TT_, true>), grid, block, lds, st, CV_HOT_ARGS(g), g);         \
+    else hipLaunchKernelGGL((cv_cols_kernel<TT_, false>), grid, block, lds, st, CV_HOT_ARGS(g), g);             \
   } while (0)
   if (g.tt == 1) CV_TT(1);
   else if (g.tt == 2) CV_TT(2);
