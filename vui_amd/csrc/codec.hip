@@ -326,8 +326,8 @@ __global__ __launch_bounds__(64 * CV_NW, 4) void cv_cols_kernel(CV_HOT, const Cv
 // The sum is exact for every finite value from 2^-110 up.  Of a smaller one, what lies below bf16's least subnormal, 2^-133, is lost
 // (weights of 2^-118: error of the product 1.4e-5, 2^-122: 2e-4; with fp32 instructions 2e-6).  A value that is not finite makes its
 // columns or rows NaN, an infinite one too.
-// 32 frames: 7-tap convolutions of 768 / 384 / 192 / 96 channels 86 / 105 / 121 / 91 us -> 55 / 63 / 83 / 62 (1200 TFLOP/s
-// of bf16 products in the first, what hipBLASLt reaches at 8192^3), 1x1 19 / 30 / 32 / 33 -> 16 / 29 / 26 / 29 (3-4 % more with the clamp
+// 32 frames: 7-tap convolutions of 768 / 384 / 192 / 96 channels 86 / 105 / 121 / 91 us -> 55 / 63 / 83 / 62 (920 TFLOP/s
+// of bf16 products in the first; hipBLASLt reaches 1125 at 8192^3), 1x1 19 / 30 / 32 / 33 -> 16 / 29 / 26 / 29 (3-4 % more with the clamp
 // of cv_split2); error of 93 frames against 64 bits 4.1e-6 -> 3.9e-6.
 // Tiles of BM x BN = 128 x 128 (or what divides M) of four waves through LDS, three planes of each operand: a K step is one (tap,
 // 32-channel) unit, fetched into registers while the one before it is multiplied, split on the way to LDS.  A group's taps follow each
