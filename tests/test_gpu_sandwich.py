@@ -76,6 +76,21 @@ def test_prompts_of_many_lengths(name, dt):
 
 
 @BOTH
+@pytest.mark.parametrize("width", [2032, 2048, 2064])
+def test_features_by_half_blocks(width, dt):
+    """Products of up to 16 rows and 128 blocks of 16 features (2048) take eight features per workgroup, of 129 blocks whole ones;
+    127 blocks for an odd number of them."""
+    cfg = U.sandwich([(U.sig(heads=2, kv_heads=1, dim=24, vdim=40), U.dense(100))], width=width)
+    sd = U.sandwich_weights(cfg, 13)
+    eng = U.engine(cfg, sd, dt, max_seq=64)
+    for T in (1, 5, 16):
+        toks = U.tokens(T, cfg["vocab"], T)
+        with eng.new_row() as row:
+            e = U.err(run_all(row, toks), oracle(cfg, sd, toks)[0])
+        assert e < TOL[dt], (T, e)
+
+
+@BOTH
 @pytest.mark.parametrize("name", sorted(SINGLE))
 def test_decoding_of_every_mechanism(name, dt):
     """Prompts of unequal lengths, then single tokens of all rows together: over tile, block and chunk borders."""

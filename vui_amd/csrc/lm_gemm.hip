@@ -200,7 +200,8 @@ static void lm_set_order(LmGemm& g, int MT, int NT, int band) {
   }                                                                                                          \
   else { p.ssq = (const float*)aux0; p.norm = (const float*)aux1; p.np = (int)(np_band & 0xffffu); p.band = (int)(np_band >> 16); }
 
-template <typename T, int MB, int NB, int WAVES, int EPI>
+// HALF: a workgroup takes eight of a block's 16 features (few rows and few features, see pick): the matrix instruction sees them twice.
+template <typename T, int MB, int NB, int WAVES, int EPI, bool HALF>
 __global__ __launch_bounds__(64 * WAVES, sizeof(T) == 2 && MB == 1 && NB < 3 ? 4 : 1) void lm_gemm_kernel(LM_HOT, const LmGemm p0) {
   LmGemm p = p0;
   LM_HOT_IN(p, EPI == LM_MOE_UP || EPI == LM_MOE_DOWN);
@@ -218,10 +219,12 @@ __global__ __launch_bounds__(64 * WAVES, sizeof(T) == 2 && MB == 1 && NB < 3 ? 4
   if (MOE) {
     t = ((int)blockIdx.x >> 3) % MT; nt = ((int)blockIdx.x >> 3) / MT * 8 + ((int)blockIdx.x & 7);
   } else if (MB == 1) {
-    t = 0; nt = (int)blockIdx.x;
+    t = 0; nt = HALF ? (int)blockIdx.x >> 1 : (int)blockIdx.x;
   } else {
     lm_tile_at(p, blockIdx.x, MT, ((p.N >> 4) + NB - 1) / NB, t, nt);
   }
+  static_assert(!HALF || (MB == 1 && NB == 1 && EPI == LM_PLAIN), "an epilogue whose features are each by themselves");
+  const int half8 = HALF ? 8 * ((int)blockIdx.x & 1) : 0;
   const int m0 = t * 16 * MB, nb0 = nt * NB;
   size_t wz = blockIdx.z * p.wz;
   int entry = -1;  // of the tile's row l16, where the tile is found in the choices
@@ -273,7 +276,7 @@ __global__ __launch_bounds__(64 * WAVES, sizeof(T) == 2 && MB == 1 && NB < 3 ? 4
   }
 #pragma unroll
   for (int i = 0; i < NB; ++i)
-    wr[i] = (const T*)p.W + wz + (size_t)min(nb0 + i, NBL - 1) * nsteps * 1024 + lane * EP;
+    wr[i] = (const T*)p.W + wz + (size_t)min(nb0 + i, NBL - 1) * nsteps * 1024 + (HALF ? (lane & 0x37) + half8 : lane) * EP;
 
   // U steps' loads go out together (a step beyond the wave's last re-reads that one and is not multiplied); the first ones now
   constexpr bool EARLY = WAVES >= 8 && sizeof(T) == 2;
@@ -367,8 +370,8 @@ __global__ __launch_bounds__(64 * WAVES, sizeof(T) == 2 && MB == 1 && NB < 3 ? 4
     const int j = mix ? u : u % MB, i0 = mix ? 0 : u / MB;
     const int m = m0 + 16 * j + l16;
     const int nb = nb0 + i0;
-    const int n = nb * 16 + 4 * kg;
-    const bool live = (MOE || m < p.M) && nb < NBL;
+    const int n = nb * 16 + (HALF ? half8 + 4 * (kg & 1) : 4 * kg);
+    const bool live = (MOE || m < p.M) && nb < NBL && !(HALF && kg > 1);
     const float sc = SCALED ? srow[16 * j + l16] : 1.f;
     float v[4];
     auto gather = [&](int i, float* o) {
@@ -609,14 +612,14 @@ static int go_wide(LmGemm g, int nz, hipStream_t st) {
   return VUI_OK;
 }
 
-template <typename T, int MB, int NB, int WAVES, int EPI>
+template <typename T, int MB, int NB, int WAVES, int EPI, bool HALF = false>
 static int go(LmGemm g, int nz, hipStream_t st) {
   const bool moe = EPI == LM_MOE_UP || EPI == LM_MOE_DOWN;
   const int nt = (g.N / 16 + NB - 1) / NB;
   const int mt = (g.M + 16 * MB - 1) / (16 * MB);
   lm_set_order(g, mt, nt, lm_band(mt, nt, MB, NB));
-  const int tiles = moe ? g.max_tiles * ((nt + 7) & ~7) : mt * nt;
-  hipLaunchKernelGGL((lm_gemm_kernel<T, MB, NB, WAVES, EPI>), dim3((unsigned)tiles, 1, nz), dim3(64 * WAVES), 0, st, LM_HOT_ARGS(g, moe), g);
+  const int tiles = moe ? g.max_tiles * ((nt + 7) & ~7) : mt * nt * (HALF ? 2 : 1);
+  hipLaunchKernelGGL((lm_gemm_kernel<T, MB, NB, WAVES, EPI, HALF>), dim3((unsigned)tiles, 1, nz), dim3(64 * WAVES), 0, st, LM_HOT_ARGS(g, moe), g);
   HIP_TRY(hipGetLastError());
   return VUI_OK;
 }
@@ -702,6 +705,9 @@ static int pick(int epi, const LmGemm& g, int nz, hipStream_t st) {
     if (epi == LM_MOE_UP) return go<T, 1, 1, 16, LM_MOE_UP>(g, nz, st);
     if (epi == LM_MOE_DOWN) return go<T, 1, 1, 16, LM_MOE_DOWN>(g, nz, st);
   }
+  // few features still: half a block per workgroup where whole ones would leave half the CUs without, and the others take in a block's
+  // weights at 45 KB a us (16 x 2048 x 6144 13.4 -> 11.7 us, the mean of a 2048 wide step's thirteen 7.8 -> 7.0, with 4 rows 6.8 -> 6.5)
+  if (few && epi == LM_PLAIN && (long)g.N / 16 * nz <= 128) return go<T, 1, 1, 16, LM_PLAIN, true>(g, nz, st);
   switch (epi) {
     case LM_IN_ATTN: return few ? go<T, 1, 2, 8, LM_IN_ATTN>(g, nz, st) : many<T, 2, LM_IN_ATTN>(g, nz, st);
     case LM_IN_GRU_STEP: return go<T, 1, 3, 8, LM_IN_GRU_STEP>(g, nz, st);
