@@ -184,10 +184,11 @@ def test_pieces_of_two_tiles(rows, heads, rank, rot):
 
 
 @BOTH
-@pytest.mark.parametrize("rows, heads, rank, vdim", [(1, 16, 560, 150), (3, 2, 70, 33), (16, 5, 300, 100)])
+@pytest.mark.parametrize("rows, heads, rank, vdim", [(1, 16, 560, 150), (3, 2, 70, 33), (16, 5, 300, 100), (2, 2, 970, 33), (2, 2, 1990, 33)])
 def test_shares_of_a_value_expansion(rows, heads, rank, vdim, dt):
     """Workgroups of two to eight blocks of 16 value features (10, 3, 7 of them) and one to sixteen rows, whose waves share 9, 2 and 5 steps
-    of K; 256 columns of a row at a time (rank 560: the last third is 64), up to 26 pieces."""
+    of K; 256 columns of a row at a time (rank 560: the last third is 64), up to 26 pieces.  Ranks of 961-1024 in fp32 and 1985-2048 in
+    bf16: a row's operand is 64 KiB of LDS, the sums of the waves that share K come on top."""
     cfg = U.config([U.attn(heads=heads, dim=16, rot_dim=8, vdim=vdim, kv_rank=rank)], ff=None)
     sd = U.weights(cfg, 21)
     eng = U.engine(cfg, sd, dt, max_rows=rows, max_seq=840)

@@ -604,7 +604,7 @@ int launch_latent_value(const LatentArgs& a, hipStream_t st) {
   const dim3 grid(a.heads, (nvb + nbw - 1) / nbw, (a.M + rpw - 1) / rpw);
   const uint32_t split = (uint32_t)a.n_splits | (uint32_t)rpw << 8 | (uint32_t)nbw << 16;
   const size_t lds = (size_t)16 * a.d.rank64 * (f32 ? 4 : 2);
-  if (lds > 64 * 1024) {
+  if (lds > 56 * 1024) {  // beside it 8 KiB of the waves' sums
     HIP_TRY(hipFuncSetAttribute(f32 ? (const void*)latent_value_kernel<float> : (const void*)latent_value_kernel<bf16_t>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   }
