@@ -326,6 +326,15 @@ class QwenCodecDecoder:
         _lib.check(self.lib.vui_codec_decode_frame(self.handle, codes_q.data_ptr(), n_q, out.data_ptr(),
                                                    torch.cuda.current_stream().cuda_stream), "vui_codec_decode_frame")
 
+    def _scratch_bytes(self, n: int) -> int:
+        """Scratch memory of a pass of n frames: a block's own size, a clip's of 64, 128 or 256 frames.  The allocator keeps what
+        is freed, and a longer clip does not fit in it: with a size for every length, growing clips would leave one buffer each behind."""
+        if n > self._block:
+            n = min(1 << (n - 1).bit_length(), self._clip)
+        if n not in self._pass_bytes:
+            self._pass_bytes[n] = int(self.lib.vui_codec_clip_scratch_bytes(C.byref(self._cc), n))
+        return self._pass_bytes[n]
+
     @torch.inference_mode()
     def forward(self, codes: Tensor) -> Tensor:
         """codes (1, n_q, T) long -> audio (1, 1, T * hop).  Inside `streaming()` the call continues the
@@ -355,10 +364,8 @@ class QwenCodecDecoder:
             n = -(-left // -(-left // most)) if left > 0 else 1
             if n > 1:
                 if scratch is None:  # passes do not grow
-                    if n not in self._pass_bytes:
-                        self._pass_bytes[n] = int(self.lib.vui_codec_clip_scratch_bytes(C.byref(self._cc), n))
                     try:
-                        scratch = torch.empty(self._pass_bytes[n], dtype=torch.uint8, device=self.device)
+                        scratch = torch.empty(self._scratch_bytes(n), dtype=torch.uint8, device=self.device)
                     except torch.OutOfMemoryError:  # 8 MB per frame: shorter passes need less
                         if n <= self._block:
                             raise
