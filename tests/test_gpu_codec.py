@@ -254,8 +254,8 @@ def test_full_dims_codec_ctx_session(full):
 
 @pytest.mark.parametrize("T", [2, 3, 31, 32, 33, 40])
 def test_blocks_of_frames_equal_single_frames(small, T):
-    """Offline calls take up to 32 frames per pass: against the oracle, and against the same frames one at a time (fp32
-    sums in another order through ~60 layers: 2e-5, measured 2e-6), whatever is in the rings from before."""
+    """Offline calls take their frames in one pass here (up to the decoder's window of 40): against the oracle, and against the same
+    frames one at a time (fp32 sums in another order through ~60 layers: 2e-5, measured 2e-6), whatever is in the rings from before."""
     d, ora, dec = small
     codes = torch.randint(0, d.codebook_size, (1, d.n_codebooks, T), generator=torch.Generator().manual_seed(T))
     ref = ora.forward(codes)
@@ -263,6 +263,42 @@ def test_blocks_of_frames_equal_single_frames(small, T):
     with dec.streaming(1):
         one = torch.cat([dec(codes[:, :, t:t + 1].cuda()).clone() for t in range(T)], dim=-1)
     assert err(got, ref) < TOL and err(got, one.cpu()) < 2e-5
+
+
+@pytest.mark.parametrize("T", [33, 40])
+def test_offline_calls_of_several_passes(small, T, monkeypatch):
+    """Calls of more frames than a pass takes: two passes of 17 and 16 or of 20 frames, with the bounds of the test above."""
+    d, ora, dec = small
+    monkeypatch.setattr(dec, "_clip", dec._block)
+    codes = torch.randint(0, d.codebook_size, (1, d.n_codebooks, T), generator=torch.Generator().manual_seed(T))
+    got = dec(codes.cuda())
+    with dec.streaming(1):
+        one = torch.cat([dec(codes[:, :, t:t + 1].cuda()).clone() for t in range(T)], dim=-1)
+    assert err(got, ora.forward(codes)) < TOL and err(got, one.cpu()) < 2e-5
+
+
+def test_block_entry(small):
+    """vui_codec_decode_block, which callers of the C ABI have beside the clip's: as many frames as a block takes are decoded to the
+    same samples, more are refused, and too little scratch memory is."""
+    import ctypes as C
+
+    d, ora, dec = small
+    lib, st = dec.lib, torch.cuda.current_stream().cuda_stream
+    codes = torch.randint(0, d.codebook_size, (1, d.n_codebooks, 33), generator=torch.Generator().manual_seed(12)).cuda()
+    rows = codes[0].t().contiguous()
+    size = [int(lib.vui_codec_block_scratch_bytes(C.byref(dec._cc), n)) for n in (2, 32)]
+    scratch = torch.empty(2 * size[1], dtype=torch.uint8, device="cuda")
+
+    def block(n, room):
+        audio = torch.empty(n * d.hop, device="cuda")
+        dec.reset_streaming()
+        return lib.vui_codec_decode_block(dec.handle, rows.data_ptr(), n, d.n_codebooks, audio.data_ptr(), scratch.data_ptr(), room, st), audio
+
+    for n, room in zip((2, 32), size):
+        rc, audio = block(n, room)
+        assert rc == 0 and torch.equal(audio, dec(codes[:, :, :n].contiguous()).view(-1)), n
+    assert block(33, scratch.numel())[0] == block(0, scratch.numel())[0] == -22 and block(32, size[1] - 1)[0] == -12
+    dec.reset_streaming()
 
 
 def test_blocks_and_single_frames_in_one_stream(small):
