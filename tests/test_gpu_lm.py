@@ -556,6 +556,22 @@ def test_small_products_of_a_prompt(large, T):
     assert U.err(whole, ref[:T]) < 0.012 and U.err(whole, parts) < 0.012
 
 
+@BOTH
+def test_a_vocabulary_of_two_million(dt):
+    """More features than a product takes at once: the head's of few rows, of a decode step (the length moves once) and of more
+    than sixteen rows, the last part with 19 of 32 features."""
+    cfg = U.config([U.attn(heads=2, kv_rank=20)], width=24, vocab=2 ** 21 + 19, ff=7)
+    sd, toks = U.weights(cfg, 8), U.tokens(19, cfg["vocab"], 9)
+    ref = O.forward(cfg, sd, toks, dtype=F32)
+    eng = U.engine(cfg, sd, dt, max_rows=1, max_seq=32)
+    with eng.new_row() as row:
+        assert U.err(row.extend(toks[:17], [3, 16]), ref[[3, 16]]) < U.TOL[dt]
+        for t in (17, 18):
+            assert U.err(eng.decode_step([row], torch.tensor([toks[t]], device="cuda")), ref[t:t + 1]) < U.TOL[dt]
+        row.reset()
+        assert U.err(row.extend(toks, range(19)), ref) < U.TOL[dt]
+
+
 @pytest.mark.parametrize("T", [640, 700])
 def test_lone_tiles_of_a_prompt(T):
     """Products of fewer 64 x 64 tiles than compute units, whose K is split over two halves of waves: an odd number of 64 columns in

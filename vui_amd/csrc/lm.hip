@@ -297,7 +297,7 @@ static LmGemm lm_logits(vui_lm_ctx* x, const LmRows& rows, int M, int x_rows, co
   const vui_lm_dims& d = x->dims[0];
   g.X = x->xt; g.W = x->w.head; g.M = M; g.N = pad(x->c.vocab, 16); g.K = d.w64; g.rowmap = rowmap; g.x_rows = x_rows;
   g.ssq = x->ssq; g.np = d.w16 / 16; g.width = x->c.width; g.eps = x->c.norm_eps; g.norm = x->w.final_norm;
-  g.rows = rows; g.d = d; g.logits = out; g.vocab = x->c.vocab;
+  g.rows = rows; g.d = d; g.logits = out; g.ldo = g.vocab = x->c.vocab;
   return g;
 }
 

@@ -135,7 +135,7 @@ __device__ __forceinline__ void lm_unit(const LmGemm& p, const int m, const int 
   }
   if (LOGITS) {
     if (live)
-      for (int r = 0; r < 4; ++r) if (n + r < p.vocab) p.logits[(size_t)m * p.vocab + n + r] = v[r];
+      for (int r = 0; r < 4; ++r) if (n + r < p.vocab) p.logits[(size_t)m * p.ldo + n + r] = v[r];
     return;
   }
   if (EPI == LM_PROJ || EPI == LM_PLAIN || EPI == LM_MOE_DOWN) {
@@ -186,7 +186,10 @@ static void lm_set_order(LmGemm& g, int MT, int NT, int band) {
 
 // The first fourteen words of a kernel's scalar arguments are in registers when it starts, a struct is a trip to memory (0.2-0.35 us of a
 // launch of 4-8): what the first loads need comes twice, ahead of the struct and in it.  aux0, aux1: of experts' products the choices, or
-// the number of tiles and their experts, otherwise the sums of squares and the norm; np_band: of the same the entries' tiles.
+// the number of tiles and their experts, otherwise the sums of squares and the norm; np_band: of the same the entries' tiles.  The few bits
+// of features and K (below LM_SIZES) keep the arithmetic of addresses short, too: with every size that an int holds 10-25 scalar instructions
+// more, 8 steps of 36 launches 1306 -> 1313 us.
+#define LM_SIZES (1 << 21)
 #define LM_HOT const void *X, const void *W, const void *aux0, const void *aux1, int M, uint32_t nk, uint32_t np_band, uint32_t inv_tiles, uint32_t inv_band, uint32_t inv_last
 #define LM_HOT_ARGS(g, moe)                                                                                                                 \
   g.X, g.W, (moe) ? (const void*)(g.choice ? g.choice : g.n_tiles) : (const void*)g.ssq, (moe) ? (const void*)g.tile_e : (const void*)g.norm, g.M,                   \
@@ -726,7 +729,18 @@ static int pick(int epi, const LmGemm& g, int nz, hipStream_t st) {
 }
 
 int launch_lm_gemm(int dtype, int epi, const LmGemm& g, int nz, hipStream_t st) {
-  if (g.M < 1 || g.N < 16 || (g.N & 15) || g.K < 64 || (g.K & 63) || nz < 1 || g.N >= 1 << 21 || g.K >= 1 << 21) {
+  if ((epi == LM_LOGITS || epi == LM_HEAD) && g.N >= LM_SIZES) {  // a larger vocabulary by parts, the lengths with the last
+    const int part = LM_SIZES / 2;
+    for (int n = 0, rc; n < g.N; n += part) {
+      LmGemm h = g;
+      h.N = std::min(part, g.N - n); h.W = (const char*)g.W + (size_t)n * g.K * (dtype == VUI_DTYPE_F32 ? 4 : 2);
+      h.logits = g.logits + n; h.vocab = g.vocab - n;
+      if (h.N < g.N - n) h.upd_lens = nullptr;
+      if ((rc = launch_lm_gemm(dtype, epi, h, nz, st))) return rc;
+    }
+    return VUI_OK;
+  }
+  if (g.M < 1 || g.N < 16 || (g.N & 15) || g.K < 64 || (g.K & 63) || nz < 1 || g.N >= LM_SIZES || g.K >= LM_SIZES || g.np > 0xffff) {
     vui_set_error("lm gemm: bad shape M=%d N=%d K=%d", g.M, g.N, g.K);
     return VUI_EINVAL;
   }
