@@ -444,10 +444,10 @@ def test_all_tokens_to_few_experts(dt):
 
 
 @BOTH
-@pytest.mark.parametrize("experts,top,rows", [(64, 4, 16), (65, 4, 16), (64, 5, 13), (33, 16, 4), (6, 6, 10), (12, 1, 2), (40, 7, 1)])
+@pytest.mark.parametrize("experts,top,rows", [(64, 4, 16), (65, 4, 16), (64, 5, 13), (33, 16, 4), (6, 6, 10), (12, 1, 2), (40, 7, 1), (30, 6, 4), (30, 5, 5), (128, 4, 16)])
 def test_routing_of_decode_rows(experts, top, rows, dt):
-    """Rows whose choices their own launch sorts (up to 64 of them) and the next more, both forms of choosing (up to 64 experts, and
-    more), all experts at once, with attention of one piece and of several per row: every row against itself alone, through the
+    """Rows whose entries the products find (up to 64 of them, walked to up to 24 tiles, by the bits of the experts' numbers above, 128 of them too) and
+    the next more, both forms of choosing (up to 64 experts, and more), all experts at once, with attention of one piece and of several per row: every row against itself alone, through the
     prompt pass of its whole sequence where routing takes launches of its own.  Replayed, other rows' steps in between."""
     cfg = U.sandwich([(U.sig(), U.moe(experts=experts, top=top)), (U.sig(heads=20, kv_heads=1, dim=8, vdim=12), U.dense(40))])
     sd = U.sandwich_weights(cfg, 51)

@@ -203,14 +203,20 @@ static void lm_set_order(LmGemm& g, int MT, int NT, int band) {
   }                                                                                                          \
   else { p.ssq = (const float*)aux0; p.norm = (const float*)aux1; p.np = (int)(np_band & 0xffffu); p.band = (int)(np_band >> 16); }
 
-// HALF: a workgroup takes eight of a block's 16 features (few rows and few features, see pick): the matrix instruction sees them twice.
-template <typename T, int MB, int NB, int WAVES, int EPI, bool HALF>
+// n and the bits of a mask below this lane
+__device__ __forceinline__ int lane_count(uint32_t lo, uint32_t hi, int n) { return __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, n)); }
+
+// ALT, of LM_PLAIN: HALF, a workgroup takes eight of a block's 16 features (few rows and few features, see pick), which the matrix
+// instruction sees twice; of experts' products: BITS, another way to the tile's entries (see experts).
+template <typename T, int MB, int NB, int WAVES, int EPI, bool ALT>
 __global__ __launch_bounds__(64 * WAVES, sizeof(T) == 2 && MB == 1 && NB < 3 ? 4 : 1) void lm_gemm_kernel(LM_HOT, const LmGemm p0) {
   LmGemm p = p0;
   LM_HOT_IN(p, EPI == LM_MOE_UP || EPI == LM_MOE_DOWN);
   constexpr bool SCALED = EPI == LM_IN_ATTN || EPI == LM_IN_GRU_STEP || EPI == LM_IN_GRU_SEQ || EPI == LM_LOGITS;
   constexpr bool GRU = EPI == LM_IN_GRU_STEP || EPI == LM_IN_GRU_SEQ;
   constexpr bool LOGITS = EPI == LM_LOGITS || EPI == LM_HEAD, MOE = EPI == LM_MOE_UP || EPI == LM_MOE_DOWN;
+  constexpr bool HALF = ALT && EPI == LM_PLAIN, BITS = ALT && MOE;
+  static_assert(ALT == (HALF || BITS) && (!HALF || NB == 1) && (!ALT || MB == 1), "half blocks are for features that are each by themselves");
   constexpr int EP = Tl<T>::EP, P = 16 / EP, TILE = MB * NB * 256;
   __shared__ __align__(16) float part[WAVES * TILE];
   __shared__ float srow[MB * 16];
@@ -226,28 +232,53 @@ __global__ __launch_bounds__(64 * WAVES, sizeof(T) == 2 && MB == 1 && NB < 3 ? 4
   } else {
     lm_tile_at(p, blockIdx.x, MT, ((p.N >> 4) + NB - 1) / NB, t, nt);
   }
-  static_assert(!HALF || (MB == 1 && NB == 1 && EPI == LM_PLAIN), "an epilogue whose features are each by themselves");
   const int half8 = HALF ? 8 * ((int)blockIdx.x & 1) : 0;
   const int m0 = t * 16 * MB, nb0 = nt * NB;
   size_t wz = blockIdx.z * p.wz;
   int entry = -1;  // of the tile's row l16, where the tile is found in the choices
   if (MOE && MB == 1 && p.choice) {
-    // Experts in the order of their first entry, each with as many tiles of 16 entries as it needs; entries are lanes.
+    // Experts in the order of their first entry, each with as many tiles of 16 entries as it needs; entries are lanes
     if (nb0 >= (p.N >> 4)) return;  // uniform, as what follows
     const int n = (int)inv_tiles, e = lane < n ? p.choice[lane] : -1;
-    uint64_t left = ~0ull >> (64 - n), mine = 0;
+    const uint64_t all = ~0ull >> (64 - n);
+    uint64_t mine = 0;
     int expert = -1, sub = t;  // its tile
-    while (left) {
-      const int c = __builtin_amdgcn_readlane(e, __builtin_ctzll(left));
-      const uint64_t same = __builtin_amdgcn_ballot_w64(e == c);
-      const int tiles = (__popcll(same) + 15) >> 4;
-      if (sub < tiles) { expert = c; mine = same; break; }
-      sub -= tiles;
-      left &= ~same;
+    if (!BITS) {  // from expert to expert up to the tile's own
+      uint64_t left = all;
+      while (left) {
+        const int c = __builtin_amdgcn_readlane(e, __builtin_ctzll(left));
+        const uint64_t same = __builtin_amdgcn_ballot_w64(e == c);
+        const int tiles = (__popcll(same) + 15) >> 4;
+        if (sub < tiles) { expert = c; mine = same; break; }
+        sub -= tiles;
+        left &= ~same;
+      }
+    } else {  // every lane finds the entries of its expert by the bits of its number (up to 128 experts, see lm_rows_routes)
+      uint32_t lo = (uint32_t)all, hi = (uint32_t)(all >> 32);
+#pragma unroll
+      for (int b = 0; b < 7; ++b) {
+        const uint64_t set = __builtin_amdgcn_ballot_w64(e >> b & 1);
+        const uint32_t flip = (uint32_t)(e >> b & 1) - 1;
+        lo &= (uint32_t)set ^ flip; hi &= (uint32_t)(set >> 32) ^ flip;
+      }
+      const bool leads = lane < n && lane_count(lo, hi, 0) == 0;
+      const int tiles = leads ? (__popc(lo) + __popc(hi) + 15) >> 4 : 0;
+      int first = 0;  // tiles of the experts before
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const uint64_t more = __builtin_amdgcn_ballot_w64(tiles > k);
+        first = lane_count((uint32_t)more, (uint32_t)(more >> 32), first);
+      }
+      const uint64_t who = __builtin_amdgcn_ballot_w64((uint32_t)(t - first) < (uint32_t)tiles);
+      if (who) {
+        const int lead = __builtin_ctzll(who);
+        expert = __builtin_amdgcn_readlane(e, lead); sub = t - __builtin_amdgcn_readlane(first, lead);
+        mine = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)hi, lead) << 32 | (uint32_t)__builtin_amdgcn_readlane((int)lo, lead);
+      }
     }
     if (expert < 0) return;
     wz = (size_t)expert * p.wz;
-    const int at = __popcll(mine & ((1ull << lane) - 1));
+    const int at = lane_count((uint32_t)mine, (uint32_t)(mine >> 32), 0);
     const bool in = (mine >> lane & 1) && at >> 4 == sub;
     const int got = __builtin_amdgcn_ds_permute((in ? at & 15 : 63) * 4, lane + 1);  // lanes 0 ... 15: their entry + 1, or 0
     entry = __builtin_amdgcn_ds_bpermute(l16 * 4, got) - 1;
@@ -615,14 +646,14 @@ static int go_wide(LmGemm g, int nz, hipStream_t st) {
   return VUI_OK;
 }
 
-template <typename T, int MB, int NB, int WAVES, int EPI, bool HALF = false>
+template <typename T, int MB, int NB, int WAVES, int EPI, bool ALT = false>
 static int go(LmGemm g, int nz, hipStream_t st) {
   const bool moe = EPI == LM_MOE_UP || EPI == LM_MOE_DOWN;
   const int nt = (g.N / 16 + NB - 1) / NB;
   const int mt = (g.M + 16 * MB - 1) / (16 * MB);
   lm_set_order(g, mt, nt, lm_band(mt, nt, MB, NB));
-  const int tiles = moe ? g.max_tiles * ((nt + 7) & ~7) : mt * nt * (HALF ? 2 : 1);
-  hipLaunchKernelGGL((lm_gemm_kernel<T, MB, NB, WAVES, EPI, HALF>), dim3((unsigned)tiles, 1, nz), dim3(64 * WAVES), 0, st, LM_HOT_ARGS(g, moe), g);
+  const int tiles = moe ? g.max_tiles * ((nt + 7) & ~7) : mt * nt * (ALT ? 2 : 1);
+  hipLaunchKernelGGL((lm_gemm_kernel<T, MB, NB, WAVES, EPI, ALT>), dim3((unsigned)tiles, 1, nz), dim3(64 * WAVES), 0, st, LM_HOT_ARGS(g, moe), g);
   HIP_TRY(hipGetLastError());
   return VUI_OK;
 }
@@ -680,6 +711,15 @@ static int many(const LmGemm& g, int nz, hipStream_t st) {
   return go<T, 2, NB, 4, EPI>(g, nz, st);
 }
 
+// Experts' products of few rows, which find their entries themselves.  Up to 24 tiles are walked to from expert to expert; with more, that is a
+// chain of up to 64 steps for the last of them.  Walked / by bits, us: 16 rows of 2048, 32 experts, up 29.3 / 28.2 and down 34.3 / 32.1 per
+// launch; 8 steps with 64 experts 6410 / 6090, 768 wide with 128 4180 / 3995, 7 rows of 1024 (28 tiles) 3280 / 3241, but 4 rows of 768 2420 / 2447
+// and 5 (20 tiles) 2471 / 2494.
+template <typename T, int NB, int WAVES, int EPI>
+static int experts(const LmGemm& g, int nz, hipStream_t st) {
+  return g.choice && g.max_tiles > 24 ? go<T, 1, NB, WAVES, EPI, true>(g, nz, st) : go<T, 1, NB, WAVES, EPI>(g, nz, st);
+}
+
 // up to 16 rows: one row block, more waves per tile (the weights are streamed once, latency counts)
 template <typename T>
 static int pick(int epi, const LmGemm& g, int nz, hipStream_t st) {
@@ -705,8 +745,8 @@ static int pick(int epi, const LmGemm& g, int nz, hipStream_t st) {
   if (few && (long)g.N * (g.max_tiles > 0 ? g.max_tiles : 1) <= 4096) {
     if (epi == LM_PROJ) return go<T, 1, 1, 16, LM_PROJ>(g, nz, st);
     if (epi == LM_ACT) return go<T, 1, 1, 16, LM_ACT>(g, nz, st);
-    if (epi == LM_MOE_UP) return go<T, 1, 1, 16, LM_MOE_UP>(g, nz, st);
-    if (epi == LM_MOE_DOWN) return go<T, 1, 1, 16, LM_MOE_DOWN>(g, nz, st);
+    if (epi == LM_MOE_UP) return experts<T, 1, 16, LM_MOE_UP>(g, nz, st);
+    if (epi == LM_MOE_DOWN) return experts<T, 1, 16, LM_MOE_DOWN>(g, nz, st);
   }
   // few features still: half a block per workgroup where whole ones would leave half the CUs without, and the others take in a block's
   // weights at 45 KB a us (16 x 2048 x 6144 13.4 -> 11.7 us, the mean of a 2048 wide step's thirteen 7.8 -> 7.0, with 4 rows 6.8 -> 6.5)
@@ -721,8 +761,8 @@ static int pick(int epi, const LmGemm& g, int nz, hipStream_t st) {
     case LM_PROJ: return few ? go<T, 1, 2, 8, LM_PROJ>(g, nz, st) : many<T, 2, LM_PROJ>(g, nz, st);
     case LM_PLAIN: return few ? go<T, 1, 1, 16, LM_PLAIN>(g, nz, st) : many<T, 2, LM_PLAIN>(g, nz, st);
     case LM_ACT: return few ? go<T, 1, 2, 8, LM_ACT>(g, nz, st) : many<T, 2, LM_ACT>(g, nz, st);
-    case LM_MOE_UP: return few ? go<T, 1, 2, 8, LM_MOE_UP>(g, nz, st) : go<T, 2, 2, 4, LM_MOE_UP>(g, nz, st);
-    case LM_MOE_DOWN: return few ? go<T, 1, 2, 8, LM_MOE_DOWN>(g, nz, st) : go<T, 2, 2, 4, LM_MOE_DOWN>(g, nz, st);
+    case LM_MOE_UP: return few ? experts<T, 2, 8, LM_MOE_UP>(g, nz, st) : go<T, 2, 2, 4, LM_MOE_UP>(g, nz, st);
+    case LM_MOE_DOWN: return few ? experts<T, 2, 8, LM_MOE_DOWN>(g, nz, st) : go<T, 2, 2, 4, LM_MOE_DOWN>(g, nz, st);
   }
   vui_set_error("lm gemm: unknown epilogue %d", epi);
   return VUI_EINVAL;
