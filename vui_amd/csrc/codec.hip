@@ -19,9 +19,9 @@
 // LDS, its waves split the (tap, 32-channel) units, multiply on v_mfma_f32_16x16x4_f32 with the weights read straight from
 // global memory, and add their parts through LDS in a fixed order.
 //
-// Several frames at once (vui_codec_decode_block: offline calls, the seeding of a stream): the same steps over
-// frames x columns, on buffers that hold a whole block with the histories in front; wide products run in
-// cv_wide_kernel.  93 frames: 56.6 ms one after the other, 6.0 ms in blocks of 32 (MI355X).
+// Several frames at once (vui_codec_decode_clip: offline calls, the seeding of a stream; vui_codec_decode_block up to 32): the same
+// steps over frames x columns, on buffers that hold a whole pass with the histories in front; wide products run in
+// cv_wide_kernel.  93 frames: 42.7 ms one after the other, 5.6 ms in blocks of 32, 4.1 in one pass (MI355X).
 #include "common.h"
 #include "internal.h"
 #include "../../include/vui_codec.h"
@@ -101,7 +101,9 @@ template <bool NT> __device__ __forceinline__ float4 cv_ld_w(const float* p) {
 #define CV_WIDE_T 64  // columns from which cv_wide_kernel takes a product of several frames
 
 #define CV_NW 8        // waves of a workgroup of cv_cols_kernel
-#define CV_XROOM 17408 // floats of staged columns, at most: with the waves' parts 80 KiB, so two workgroups fit a CU
+// Floats of staged columns, at most: 68 KiB, beside them 8 KiB of the waves' parts per block of columns.  Of tiles of one block two workgroups
+// fit a CU whatever they stage, of two and four blocks where they stage less (7 taps 9 apart of 384 channels x 160 columns: 82 KiB, one).
+#define CV_XROOM 17408
 // (tap, 32-channel) units of a wave between two barriers
 template <int TT> struct CvUnits { static constexpr int N = TT <= 2 ? 6 : 4; };
 

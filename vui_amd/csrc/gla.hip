@@ -40,8 +40,9 @@ __device__ __forceinline__ float silu_exact(float v) { return v / (1.0f + expf(-
 
 // ---- positions one by one; one workgroup per head and slot ----
 // Bound by its chain: place of the row, state, sums, norm.  What the first loads need is in registers (see lm_gemm.hip), and what a position
-// reads of the projection is asked for before the decays, its output gate and norm among it.  4 rows, 8 heads of 128 x 128: 11 us, of which
-// the row's place 0.9, requests 1.6, decays 2.2, the state's 64 KiB per workgroup 3.0, sums and norm 1.2; with 1024 threads, and with the
+// reads of the projection is asked for before the decays, its output gate and norm among it.  us per launch without / with those early loads:
+// 1 row of 4 heads of 96 x 192 8.8 / 8.4, 16 rows of 8 heads of 128 x 256 13.3 / 13.0, 4 rows of them 10.9 / 11.0, 16 rows of 4 heads 11.6 / 11.5.  4
+// rows: the row's place 0.9, requests 1.6, decays 2.2, the state's 128 KiB per workgroup 3.0, sums and norm 1.2; with 1024 threads, and with the
 // channels' numbers read side by side, the same.
 #define GLA_THREADS 512
 #define GLA_PRE 8
