@@ -473,14 +473,14 @@ def test_routing_of_decode_rows(experts, top, rows, dt):
     assert far <= (0 if dt == F32 else 0.1 * n * rows), far
 
 
-@pytest.mark.parametrize("rows", [1, 16])
-def test_an_expert_with_more_entries_than_a_tile(rows):
+@pytest.mark.parametrize("rows, experts", [(1, 6), (16, 6), (16, 40)])
+def test_an_expert_with_more_entries_than_a_tile(rows, experts):
     """Logits that are not numbers are never chosen; what is missing is expert 0 with no weight, twice per row here: with 16 rows two
-    tiles of it.  Against the model whose tokens use only the two experts that are left."""
-    cfg = [U.sandwich([(U.sig(), U.moe(experts=6, top=top))]) for top in (4, 2)]
+    tiles of it, walked to and (40 experts) found by the bits of their numbers.  Against the model whose tokens use only the two experts that are left."""
+    cfg = [U.sandwich([(U.sig(), U.moe(experts=experts, top=top))]) for top in (4, 2)]
     sd = [U.sandwich_weights(c, 52) for c in cfg]
     for s, b in zip(sd, (float("nan"), -1e4)):
-        s["l0.mlp.router.b"] = torch.tensor([b, 0.5, b, 0.0, b, b]).to(torch.bfloat16)
+        s["l0.mlp.router.b"] = torch.tensor([b, 0.5, b, 0.0] + [b] * (experts - 4)).to(torch.bfloat16)
     outs = []
     for c, s in zip(cfg, sd):
         eng = U.engine(c, s, F32, max_rows=rows)
