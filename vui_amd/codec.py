@@ -327,8 +327,9 @@ class QwenCodecDecoder:
                                                    torch.cuda.current_stream().cuda_stream), "vui_codec_decode_frame")
 
     def _scratch_bytes(self, n: int) -> int:
-        """Scratch memory of a pass of n frames: a block's own size, a clip's of 64, 128 or 256 frames.  The allocator keeps what
-        is freed, and a longer clip does not fit in it: with a size for every length, growing clips would leave one buffer each behind."""
+        """Scratch memory of a pass of n frames: a block's own, a clip's of 64, 128 or 256 frames or of the longest pass.  The allocator
+        keeps what is freed, and a longer clip does not fit in it: with a size for every length, growing clips would leave one buffer each
+        behind."""
         if n > self._block:
             n = min(1 << (n - 1).bit_length(), self._clip)
         if n not in self._pass_bytes:
