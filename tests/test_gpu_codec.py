@@ -349,8 +349,8 @@ def scaled(sd, power):
 @pytest.mark.parametrize("power", [-104, -60, -20, 20, 60, 120])
 def test_wide_products_of_any_magnitude(full, power):
     """Parts of an operand keep its exponent: scaled weights give the same audio from blocks of frames, bit by bit as long as the least
-    products are above fp32's least normal number (power-of-two factors pass through every sum of the three parts).  Weights of 2^-110
-    keep their three parts; the products' last bits are subnormal (the limit: other orders of the sums differ by 1e-5)."""
+    products are above fp32's least normal number (power-of-two factors pass through every sum of the parts).  Weights of 2^-110
+    keep their parts; the products' last bits are subnormal (the limit: other orders of the sums differ by 1e-5)."""
     d, sd, dec, fx = full
     codes = torch.randint(0, d.codebook_size, (1, d.n_codebooks, 35), generator=torch.Generator().manual_seed(9)).cuda()
     got, want = native(d, scaled(sd, power))(codes), dec(codes)
@@ -373,6 +373,39 @@ def test_wide_products_near_the_largest_number(full):
     assert float(big["upsample.0.1.pwconv2.weight"].abs().max()) > float(torch.finfo(torch.bfloat16).max)
     got = native(d, big)(codes)
     assert err(got, want.cpu()) < 5e-5  # measured 1e-5: the parts of the planted weights are others
+
+
+@pytest.mark.parametrize("powers", [(0, 6, -6, 11, -2), (-12, 2, 3, 0, -1), (9,)])
+def test_wide_products_of_groups_of_different_size(full, powers):
+    """Columns are scaled per group of 32 channels, weights per matrix: the feed-forwards' inputs times a power of two per group and their weights
+    by the inverse give the same audio.  Both keep 22 bits down to 2^-17 of the largest, so the bound is that of other orders of the sums."""
+    d, sd, dec, fx = full
+    sd = dict(sd)
+    for i in range(2):
+        p = f"upsample.{i}.1."
+        n = sd[p + "norm.weight"].shape[0]
+        f = 2.0 ** torch.tensor([powers[c // 32 % len(powers)] for c in range(n)], dtype=torch.float32)
+        for k in ("norm.weight", "norm.bias"):
+            sd[p + k] = sd[p + k] * f
+        sd[p + "pwconv1.weight"] = sd[p + "pwconv1.weight"] / f
+    codes = torch.randint(0, d.codebook_size, (1, d.n_codebooks, 35), generator=torch.Generator().manual_seed(9)).cuda()
+    assert err(native(d, sd)(codes), dec(codes).cpu()) < 5e-5
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_a_frame_that_is_not_finite_leaves_those_before_it(full, bad):
+    """What is not finite does not count in the scale of the columns beside it.  (The last layer's clamp makes a NaN -1.)"""
+    d, sd, dec, fx = full
+    sd = dict(sd)
+    key = "quantizer.semantic.codebooks.0.embed"
+    sd[key] = sd[key].clone()
+    sd[key][5] = bad
+    codes = torch.randint(6, d.codebook_size, (1, d.n_codebooks, 35), generator=torch.Generator().manual_seed(9)).cuda()
+    want = dec(codes)
+    codes[0, 0, 17] = 5
+    got = native(d, sd)(codes)
+    n = 17 * (want.shape[-1] // 35)
+    assert err(got[..., :n], want[..., :n].cpu()) < 5e-5 and bool((got[..., n:] == -1).all())
 
 
 @pytest.mark.parametrize("d_model", [1024, 1312, 2048])
