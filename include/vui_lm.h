@@ -139,6 +139,11 @@ int vui_lm_decode(vui_lm_ctx* ctx, const int64_t* tokens, const int32_t* slot_id
 int vui_lm_prefill(vui_lm_ctx* ctx, const int64_t* tokens, int T, int slot, int pos0, int32_t* seq_lens,
                    const int32_t* want, int n_want, float* logits_out, vui_stream_t stream);
 
+/* What a slot held at an earlier length: n states (sizes[i] fp32 values from from[i] to states[i], device memory that does not overlap)
+ * and seq_lens[slot] = length, in one launch for up to 16 states.  The arrays of pointers and sizes are the host's. */
+int vui_lm_restore(float* const* states, const float* const* from, const int64_t* sizes, int n, int32_t* seq_lens, int slot,
+                   int length, vui_stream_t stream);
+
 /* Test aid: the residual stream behind each layer, for the calls that follow, goes to buf (n_layers, rows of the call,
  * width) fp32; NULL switches it off. */
 int vui_lm_debug_layers(vui_lm_ctx* ctx, float* buf);

@@ -361,6 +361,40 @@ def test_rewind_restores_positions_and_state():
     assert U.err(run_all(row, toks[:9]), O.forward(cfg, sd, toks[:9])) < U.TOL[F32]
 
 
+@pytest.mark.parametrize("sizes, shift", [([], 0), ([1], 0), ([3, 4, 4095], 0), ([4096, 4100, 1 << 20], 0), ([5, 64], 1), ([16] * 17, 0)])
+def test_restore_is_the_copies(sizes, shift):
+    """vui_lm_restore: whole and cut vectors, sources off a 16-byte line, more states than one launch takes; neighbours stay."""
+    import ctypes as C
+
+    from vui_amd import _lib
+
+    lens = torch.zeros(5, dtype=torch.int32, device="cuda")
+    buf = [torch.zeros(n + 8, device="cuda") for n in sizes]
+    src = [torch.randn(n + shift, device="cuda")[shift:] for n in sizes]
+    k = len(sizes)
+    _lib.check(_lib.load().vui_lm_restore((C.c_void_p * k)(*[b.data_ptr() + 16 for b in buf]), (C.c_void_p * k)(*[s.data_ptr() for s in src]),
+                                          (C.c_int64 * k)(*sizes), k, lens.data_ptr(), 3, 77, torch.cuda.current_stream().cuda_stream), "vui_lm_restore")
+    assert lens.tolist() == [0, 0, 0, 77, 0]
+    for b, s in zip(buf, src):
+        assert torch.equal(b[4:-4], s) and not b[:4].any() and not b[-4:].any()
+
+
+def test_restore_takes_what_copies_take():
+    """States that `snapshot` would not leave (on the host, of another type) go through copies as before, a missing one is refused."""
+    eng = U.engine(U.mixed(), U.weights(U.mixed(), 23))
+    cache = eng.model.cache
+    kept = {i: torch.randn_like(s[1]) for i, s in cache.state.items()}
+    for other in (kept, {i: s.cpu() for i, s in kept.items()}, {i: s.double() for i, s in kept.items()}):
+        for s in cache.state.values():
+            s.zero_()
+        cache.restore(1, 7, other)
+        assert int(cache.seq_lens[1]) == 7 and all(torch.equal(cache.state[i][1], s) for i, s in kept.items())
+    with pytest.raises(ValueError):
+        cache.restore(1, 7, None)
+    with pytest.raises(IndexError):
+        cache.restore(99, 7, kept)
+
+
 def margin_ok(cfg, sd, prompt, drawn, dt):
     """Every drawn token is the oracle's choice or within the tolerance of it."""
     L = O.forward(cfg, sd, list(prompt) + drawn)[len(prompt) - 1:-1]

@@ -156,6 +156,7 @@ SIGNATURES = {
     "vui_lm_destroy": (None, [_P]),
     "vui_lm_decode": (_I, [_P, _P, _P, _P, _P, _I, _P, _P]),
     "vui_lm_prefill": (_I, [_P, _P, _I, _I, _I, _P, _P, _I, _P, _P]),
+    "vui_lm_restore": (_I, [_P, _P, _P, _I, _P, _I, _I, _P]),
     "vui_lm_debug_layers": (_I, [_P, _P]),
     "vui_lm_expand_from": (_I, [_P, _I]),
     "vui_lm_block_from": (_I, [_P, _I, _I]),
