@@ -44,11 +44,11 @@ struct LmPre {
   float4 a, b, c;
 };
 
-// One unit of 16 rows x 16 features: a lane holds features n ... n + 3 of row m.  mix: the unit is the update gate of a recurrence, xv and gv the candidate and the output gate beside it.
+// One unit of 16 rows x 16 features: a lane holds features n ... n + 3 of row m.  half: of the block's features, that half alone (LM_OUT).  mix: the unit is the update gate of a recurrence, xv and gv the candidate and the output gate beside it.
 template <typename T, int EPI, bool PRE>
 __device__ __forceinline__ void lm_unit(const LmGemm& p, const int m, const int nb, const int n, const int l16, const int kg,
                                         const bool live, const bool mix, float (&v)[4], const float (&xv)[4], const float (&gv)[4],
-                                        const LmPre& e) {
+                                        const LmPre& e, const int half = -1) {
   constexpr bool GRU = EPI == LM_IN_GRU_STEP || EPI == LM_IN_GRU_SEQ;
   constexpr bool LOGITS = EPI == LM_LOGITS || EPI == LM_HEAD;
   if (GRU && mix) {
@@ -130,7 +130,10 @@ __device__ __forceinline__ void lm_unit(const LmGemm& p, const int m, const int 
         for (int r = 0; r < 4; ++r) if (n + r < p.width) p.layer_out[(size_t)m * p.width + n + r] = v[r];
     }
     sq = rows_sum(sq);  // the 16 columns of this row's block
-    if (live && kg == 0 && nb < p.np) p.ssq_out[(size_t)m * p.np + nb] = sq;
+    if (live && kg == 0 && nb < p.np) {
+      if (half < 0) reinterpret_cast<float2*>(p.ssq_out)[(size_t)m * p.np + nb] = make_float2(sq, 0.f);
+      else p.ssq_out[2 * ((size_t)m * p.np + nb) + half] = sq;
+    }
     return;
   }
   if (LOGITS) {
@@ -203,20 +206,52 @@ static void lm_set_order(LmGemm& g, int MT, int NT, int band) {
   }                                                                                                          \
   else { p.ssq = (const float*)aux0; p.norm = (const float*)aux1; p.np = (int)(np_band & 0xffffu); p.band = (int)(np_band >> 16); }
 
+// sum within aligned groups of N lanes, in every lane, without LDS
+template <int N>
+__device__ __forceinline__ float lanes_sum(float v) {
+  if (N >= 2) v += dpp_f<DPP_QUAD_XOR1>(v);
+  if (N >= 4) v += dpp_f<DPP_QUAD_XOR2>(v);
+  if (N >= 8) v += dpp_f<DPP_ROW_HALF_MIRROR>(v);
+  if (N >= 16) v += dpp_f<DPP_ROW_MIRROR>(v);
+  if (N >= 32) {
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  }
+  if (N >= 64) {
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  }
+  return v;
+}
+
+// a lane of 16 receives what the lane 16 - N above it (around the 16) holds
+template <int N>
+__device__ __forceinline__ uint4 row_ror(const uint4& v) {
+  return make_uint4(dpp_i<0x120 + N>((int)v.x), dpp_i<0x120 + N>((int)v.y), dpp_i<0x120 + N>((int)v.z), dpp_i<0x120 + N>((int)v.w));
+}
+
 // n and the bits of a mask below this lane
 __device__ __forceinline__ int lane_count(uint32_t lo, uint32_t hi, int n) { return __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, n)); }
 
-// ALT, of LM_PLAIN: HALF, a workgroup takes eight of a block's 16 features (few rows and few features, see pick), which the matrix
-// instruction sees twice; of experts' products: BITS, another way to the tile's entries (see experts).
-template <typename T, int MB, int NB, int WAVES, int EPI, bool ALT>
+// ALT, of LM_PLAIN and LM_OUT: HALF, a workgroup takes eight of a block's 16 features (few rows and few features, see pick); of experts'
+// products: BITS, another way to the tile's entries (see experts).
+// A CU's address unit takes a wave's load of 16 bytes per lane in 16 clocks whatever it fetches, and products of few rows wait for that: 176 such loads, 1.3 us,
+// for 16 features of K 2816, half of them for the rows' operands.  So (bf16) half a block's weights fill the lanes of one load per step: lanes 8-15 of a
+// group of 16 hold the second piece of the features of lanes 0-7, the matrix instruction meets them with both pieces of X, and
+// either sum is right for half of its features.  FEW, of up to four rows: one load holds four steps of X, those of the later
+// ones in the lanes of rows that there are not, and a rotation by lanes brings them to their place.  A step of the 768 wide model with one row, us: re-reading
+// a wave's last step where it has no more 152, not so 140, all waves' parts read before the first is added 138, PACK and FEW 134; 16 rows
+// of 1024 wide 225, 214, 212, 207; four rows of 2048 wide with experts 462, 441, 437, 431.
+template <typename T, int MB, int NB, int WAVES, int EPI, bool ALT, bool FEW>
 __global__ __launch_bounds__(64 * WAVES, sizeof(T) == 2 && MB == 1 && NB < 3 ? 4 : 1) void lm_gemm_kernel(LM_HOT, const LmGemm p0) {
   LmGemm p = p0;
   LM_HOT_IN(p, EPI == LM_MOE_UP || EPI == LM_MOE_DOWN);
   constexpr bool SCALED = EPI == LM_IN_ATTN || EPI == LM_IN_GRU_STEP || EPI == LM_IN_GRU_SEQ || EPI == LM_LOGITS;
   constexpr bool GRU = EPI == LM_IN_GRU_STEP || EPI == LM_IN_GRU_SEQ;
   constexpr bool LOGITS = EPI == LM_LOGITS || EPI == LM_HEAD, MOE = EPI == LM_MOE_UP || EPI == LM_MOE_DOWN;
-  constexpr bool HALF = ALT && EPI == LM_PLAIN, BITS = ALT && MOE;
+  constexpr bool HALF = ALT && (EPI == LM_PLAIN || EPI == LM_OUT), BITS = ALT && MOE, PACK = HALF && sizeof(T) == 2;
   static_assert(ALT == (HALF || BITS) && (!HALF || NB == 1) && (!ALT || MB == 1), "half blocks are for features that are each by themselves");
+  static_assert(!FEW || (MB == 1 && WAVES >= 8 && sizeof(T) == 2 && !MOE), "four rows of bf16");
   constexpr int EP = Tl<T>::EP, P = 16 / EP, TILE = MB * NB * 256;
   __shared__ __align__(16) float part[WAVES * TILE];
   __shared__ float srow[MB * 16];
@@ -234,7 +269,7 @@ __global__ __launch_bounds__(64 * WAVES, sizeof(T) == 2 && MB == 1 && NB < 3 ? 4
   }
   const int half8 = HALF ? 8 * ((int)blockIdx.x & 1) : 0;
   const int m0 = t * 16 * MB, nb0 = nt * NB;
-  size_t wz = blockIdx.z * p.wz;
+  size_t wz = 0;
   int entry = -1;  // of the tile's row l16, where the tile is found in the choices
   if (MOE && MB == 1 && p.choice) {
     // Experts in the order of their first entry, each with as many tiles of 16 entries as it needs; entries are lanes
@@ -300,52 +335,64 @@ __global__ __launch_bounds__(64 * WAVES, sizeof(T) == 2 && MB == 1 && NB < 3 ? 4
     } else if (MOE) {
       xr[j] = (const T*)p.X + (size_t)((m0 >> 4) + j) * nsteps * 1024 + lane * EP;
     } else if (LOGITS && p.rowmap) {
-      const int r = min(max(p.rowmap[min(m0 + 16 * j + l16, p.M - 1)], 0), p.x_rows - 1);
+      const int r = min(max(p.rowmap[min(m0 + 16 * j + (FEW ? l16 & 3 : l16), p.M - 1)], 0), p.x_rows - 1);
       xr[j] = (const T*)p.X + (size_t)(r >> 4) * nsteps * 1024 + ((r & 15) + 16 * kg) * EP;
     } else {
       // few rows: lanes without a row re-read the last one instead of fetching a block that is mostly padding
-      const int l = MB == 1 ? min(l16, p.M - 1 - m0) + 16 * kg : lane;
+      const int l = MB == 1 ? min(FEW ? l16 & 3 : l16, p.M - 1 - m0) + 16 * kg : lane;
       xr[j] = (const T*)p.X + (size_t)min((m0 >> 4) + j, MBL - 1) * nsteps * 1024 + l * EP;
     }
   }
 #pragma unroll
   for (int i = 0; i < NB; ++i)
-    wr[i] = (const T*)p.W + wz + (size_t)min(nb0 + i, NBL - 1) * nsteps * 1024 + (HALF ? (lane & 0x37) + half8 : lane) * EP;
+    wr[i] = (const T*)p.W + wz + (size_t)min(nb0 + i, NBL - 1) * nsteps * 1024 + (HALF ? (lane & 0x37) + half8 : lane) * EP + (PACK ? (l16 >> 3) * 512 : 0);
 
-  // U steps' loads go out together (a step beyond the wave's last re-reads that one and is not multiplied); the first ones now
+  // U steps' loads go out together, as far as the wave has steps (re-reading the last one instead was most of what launches of small K waited for);
+  // the first ones now
   constexpr bool EARLY = WAVES >= 8 && sizeof(T) == 2;
   constexpr int U = !EARLY ? 1 : MB == 1 ? 4 : 2;
-  uint4 xa[U][MB][P], wa[U][NB][P];
+  static_assert(!FEW || U == 4, "a row's four steps lie in its lanes' places");
+  constexpr int PW = PACK ? 1 : P, UX = FEW ? 1 : U;
+  uint4 xa[UX][MB][P], wa[U][NB][PW];
   auto load = [&](int s) {
+    if (FEW) {
+      const size_t o = (size_t)min(s + (l16 >> 2), s1 - 1) * 1024;
+#pragma unroll
+      for (int h = 0; h < P; ++h) xa[0][0][h] = *reinterpret_cast<const uint4*>(xr[0] + o + 64 * EP * h);
+    }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const size_t o = (size_t)min(s + u, s1 - 1) * 1024;
+      if (u > 0 && s + u >= s1) break;  // uniform
+      const size_t o = (size_t)(s + u) * 1024;
 #pragma unroll
       for (int h = 0; h < P; ++h) {
 #pragma unroll
-        for (int i = 0; i < NB; ++i) wa[u][i][h] = *reinterpret_cast<const uint4*>(wr[i] + o + 64 * EP * h);
+        for (int i = 0; i < NB; ++i)
+          if (h < PW) wa[u][i][h] = *reinterpret_cast<const uint4*>(wr[i] + o + 64 * EP * h);
+        if (!FEW) {
 #pragma unroll
-        for (int j = 0; j < MB; ++j) xa[u][j][h] = *reinterpret_cast<const uint4*>(xr[j] + o + 64 * EP * h);
+          for (int j = 0; j < MB; ++j) xa[u % UX][j][h] = *reinterpret_cast<const uint4*>(xr[j] + o + 64 * EP * h);
+        }
       }
     }
     __builtin_amdgcn_sched_barrier(0);
   };
-  if (EARLY && s0 < s1) load(s0);
-
   // What the scale and the epilogue of this wave's first unit will need is requested now as well:
   // fetched where it is used, it would be a chain of dependent loads behind the last product.
-  // Scale: TPR neighbouring threads add up one row's sums of squares, in a fixed order.
+  // Scale: TPR neighbouring threads add up one row's sums of squares, in a fixed order, while the operands are on their way.
   constexpr int TPR = WAVES * 64 / (MB * 16) > 64 ? 64 : WAVES * 64 / (MB * 16), NSQ = 4;
   const int sq_r = tid / TPR, sq_q = tid % TPR;
   int sq_m = 0;
-  float sq[NSQ], norm = 0.f;
+  float2 sq[NSQ];  // halves of a block's columns
+  float norm = 0.f;
   if (SCALED) {
     sq_m = min(m0 + min(sq_r, MB * 16 - 1), p.M - 1);
     if (LOGITS && p.rowmap) sq_m = min(max(p.rowmap[sq_m], 0), p.x_rows - 1);
 #pragma unroll
-    for (int i = 0; i < NSQ; ++i) sq[i] = p.ssq[(size_t)sq_m * p.np + min(sq_q + TPR * i, p.np - 1)];
+    for (int i = 0; i < NSQ; ++i) sq[i] = reinterpret_cast<const float2*>(p.ssq)[(size_t)sq_m * p.np + min(sq_q + TPR * i, p.np - 1)];
     norm = p.norm[0];
   }
+  if (EARLY && s0 < s1) load(s0);
   constexpr bool PRE = MB == 1 && (EPI == LM_IN_ATTN || EPI == LM_IN_GRU_STEP || EPI == LM_OUT);
   const int pm = min(m0 + l16, p.M - 1), pb = min(nb0 + min(wave, NB - 1), NBL - 1);  // row and block of unit `wave`
   LmPre e;
@@ -355,7 +402,7 @@ __global__ __launch_bounds__(64 * WAVES, sizeof(T) == 2 && MB == 1 && NB < 3 ? 4
     const int2 at = lm_where(p.rows, pm);
     e.slot = at.x; e.pos = at.y;
   }
-  if (PRE && EPI == LM_OUT) e.a = *reinterpret_cast<const float4*>(p.x + (size_t)pm * p.d.w64 + pb * 16 + 4 * kg);
+  if (PRE && EPI == LM_OUT) e.a = *reinterpret_cast<const float4*>(p.x + (size_t)pm * p.d.w64 + pb * 16 + (HALF ? half8 + 4 * (kg & 1) : 4 * kg));
   if (PRE && EPI == LM_IN_GRU_STEP && nb0 < p.mix_blocks) {
     const int ch = (nb0 / 3) * 16 + 4 * kg;
     e.a = *reinterpret_cast<const float4*>(p.state + (size_t)e.slot * p.d.gru16 + ch);
@@ -363,7 +410,19 @@ __global__ __launch_bounds__(64 * WAVES, sizeof(T) == 2 && MB == 1 && NB < 3 ? 4
     e.c = *reinterpret_cast<const float4*>(p.bx + ch);
   }
 
-  tl_f32x4 acc[NB][MB];
+  if (SCALED) {
+    float t = 0.f;
+#pragma unroll
+    for (int i = 0; i < NSQ; ++i) t += sq_q + TPR * i < p.np ? sq[i].x + sq[i].y : 0.f;
+    for (int i = sq_q + TPR * NSQ; i < p.np; i += TPR) {
+      const float2 v = reinterpret_cast<const float2*>(p.ssq)[(size_t)sq_m * p.np + i];
+      t += v.x + v.y;
+    }
+    t = lanes_sum<TPR>(t);
+    if (sq_r < MB * 16 && sq_q == 0) srow[sq_r] = norm / sqrtf(t / (float)p.width + p.eps);
+  }
+
+  tl_f32x4 acc[NB][MB], odd = {0.f, 0.f, 0.f, 0.f};  // odd: of PACK, the sums with the second pieces of X
 #pragma unroll
   for (int i = 0; i < NB; ++i)
 #pragma unroll
@@ -374,12 +433,28 @@ __global__ __launch_bounds__(64 * WAVES, sizeof(T) == 2 && MB == 1 && NB < 3 ? 4
     for (int u = 0; u < U; ++u) {
       if (s + u >= s1) break;  // uniform
 #pragma unroll
-      for (int h = 0; h < P; ++h)
+      for (int h = 0; h < P; ++h) {
+        uint4 x[MB];
+#pragma unroll
+        for (int j = 0; j < MB; ++j) x[j] = FEW ? (u == 0 ? xa[0][0][h] : u == 1 ? row_ror<12>(xa[0][0][h]) : u == 2 ? row_ror<8>(xa[0][0][h]) : row_ror<4>(xa[0][0][h])) : xa[u % UX][j][h];
+        if (PACK && h == 1) {
+          odd = Tl<T>::mma(wa[u][0][0], x[0], odd);
+          continue;
+        }
 #pragma unroll
         for (int i = 0; i < NB; ++i)
 #pragma unroll
           for (int j = 0; j < MB; ++j)
-            acc[i][j] = Tl<T>::mma(wa[u][i][h], xa[u][j][h], acc[i][j]);
+            acc[i][j] = Tl<T>::mma(wa[u][i][h % PW], x[j], acc[i][j]);
+      }
+    }
+  }
+  if (PACK) {  // features 0-7 with the first pieces (lanes of kg 0, 1) and with the second (kg 2, 3)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const uint32_t v = __float_as_uint(kg < 2 ? acc[0][0][r] : odd[r]);
+      const auto a = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+      acc[0][0][r] = __uint_as_float(a[0]) + __uint_as_float(a[1]);
     }
   }
 #pragma unroll
@@ -387,15 +462,6 @@ __global__ __launch_bounds__(64 * WAVES, sizeof(T) == 2 && MB == 1 && NB < 3 ? 4
 #pragma unroll
     for (int j = 0; j < MB; ++j)
       *reinterpret_cast<tl_f32x4*>(&part[wave * TILE + ((i * MB + j) * 64 + lane) * 4]) = acc[i][j];
-  if (SCALED) {
-    float t = 0.f;
-#pragma unroll
-    for (int i = 0; i < NSQ; ++i) t += sq_q + TPR * i < p.np ? sq[i] : 0.f;
-    for (int i = sq_q + TPR * NSQ; i < p.np; i += TPR) t += p.ssq[(size_t)sq_m * p.np + i];
-#pragma unroll
-    for (int o = TPR / 2; o >= 1; o >>= 1) t += __shfl_xor(t, o);
-    if (sq_r < MB * 16 && sq_q == 0) srow[sq_r] = norm / sqrtf(t / (float)p.width + p.eps);
-  }
   __syncthreads();
 
   const bool mix = GRU && nb0 < p.mix_blocks;  // uniform: a tile is all mixer or all feed-forward (padded that way)
@@ -408,11 +474,19 @@ __global__ __launch_bounds__(64 * WAVES, sizeof(T) == 2 && MB == 1 && NB < 3 ? 4
     const bool live = (MOE || m < p.M) && nb < NBL && !(HALF && kg > 1);
     const float sc = SCALED ? srow[16 * j + l16] : 1.f;
     float v[4];
-    auto gather = [&](int i, float* o) {
+    // all waves' parts are read before the first is added: left to the compiler two reads were in flight at a time, 0.5 us for sixteen parts
+    tl_f32x4 pt[WAVES];
+    auto parts = [&](int i) {
       const float* q = part + ((i * MB + j) * 64 + lane) * 4;
-      tl_f32x4 a = *reinterpret_cast<const tl_f32x4*>(q);
 #pragma unroll
-      for (int w = 1; w < WAVES; ++w) a += *reinterpret_cast<const tl_f32x4*>(q + w * TILE);
+      for (int w = 0; w < WAVES; ++w) pt[w] = *reinterpret_cast<const tl_f32x4*>(q + w * TILE);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto gather = [&](int i, float* o) {
+      parts(i);
+      tl_f32x4 a = pt[0];
+#pragma unroll
+      for (int w = 1; w < WAVES; ++w) a += pt[w];
 #pragma unroll
       for (int r = 0; r < 4; ++r) o[r] = a[r] * sc;
     };
@@ -423,7 +497,7 @@ __global__ __launch_bounds__(64 * WAVES, sizeof(T) == 2 && MB == 1 && NB < 3 ? 4
       gather(NB > 1 ? 1 : 0, xv);
       gather(NB > 2 ? 2 : 0, gv);
     }
-    lm_unit<T, EPI, PRE>(p, m, nb, n, l16, kg, live, mix, v, xv, gv, e);
+    lm_unit<T, EPI, PRE>(p, m, nb, n, l16, kg, live, mix, v, xv, gv, e, HALF ? half8 >> 3 : -1);
   }
   if (LOGITS && p.upd_lens && blockIdx.x == 0) {
     if (p.upd_inc) {
@@ -494,19 +568,20 @@ __global__ __launch_bounds__(256 * G, 2) void lm_wide_kernel(LM_HOT, const LmGem
     float a[NR];
 #pragma unroll
     for (int i = 0; i < NR; ++i) a[i] = 0.f;
-    if ((p.np & 3) == 0) {
-      for (int c = 4 * l16; c < p.np; c += 64) {
+    const int np = 2 * p.np;  // halves of blocks
+    if ((np & 3) == 0) {
+      for (int c = 4 * l16; c < np; c += 64) {
         float4 v[NR];
 #pragma unroll
-        for (int i = 0; i < NR; ++i) v[i] = *reinterpret_cast<const float4*>(p.ssq + (size_t)min(m0 + grp * NR + i, p.M - 1) * p.np + c);
+        for (int i = 0; i < NR; ++i) v[i] = *reinterpret_cast<const float4*>(p.ssq + (size_t)min(m0 + grp * NR + i, p.M - 1) * np + c);
 #pragma unroll
         for (int i = 0; i < NR; ++i) a[i] += (v[i].x + v[i].y) + (v[i].z + v[i].w);
       }
     } else {
-      for (int c = l16; c < p.np; c += 16) {
+      for (int c = l16; c < np; c += 16) {
         float v[NR];
 #pragma unroll
-        for (int i = 0; i < NR; ++i) v[i] = p.ssq[(size_t)min(m0 + grp * NR + i, p.M - 1) * p.np + c];
+        for (int i = 0; i < NR; ++i) v[i] = p.ssq[(size_t)min(m0 + grp * NR + i, p.M - 1) * np + c];
 #pragma unroll
         for (int i = 0; i < NR; ++i) a[i] += v[i];
       }
@@ -646,14 +721,16 @@ static int go_wide(LmGemm g, int nz, hipStream_t st) {
   return VUI_OK;
 }
 
-template <typename T, int MB, int NB, int WAVES, int EPI, bool ALT = false>
+template <typename T, int MB, int NB, int WAVES, int EPI, bool ALT = false, bool FEW = false>
 static int go(LmGemm g, int nz, hipStream_t st) {
+  if constexpr (sizeof(T) == 2 && MB == 1 && !FEW && EPI != LM_MOE_UP && EPI != LM_MOE_DOWN)
+    if (g.M <= 4) return go<T, MB, NB, WAVES, EPI, ALT, true>(g, nz, st);
   const bool moe = EPI == LM_MOE_UP || EPI == LM_MOE_DOWN;
   const int nt = (g.N / 16 + NB - 1) / NB;
   const int mt = (g.M + 16 * MB - 1) / (16 * MB);
   lm_set_order(g, mt, nt, lm_band(mt, nt, MB, NB));
   const int tiles = moe ? g.max_tiles * ((nt + 7) & ~7) : mt * nt * (ALT ? 2 : 1);
-  hipLaunchKernelGGL((lm_gemm_kernel<T, MB, NB, WAVES, EPI, ALT>), dim3((unsigned)tiles, 1, nz), dim3(64 * WAVES), 0, st, LM_HOT_ARGS(g, moe), g);
+  hipLaunchKernelGGL((lm_gemm_kernel<T, MB, NB, WAVES, EPI, ALT, FEW>), dim3((unsigned)tiles, 1, nz), dim3(64 * WAVES), 0, st, LM_HOT_ARGS(g, moe), g);
   HIP_TRY(hipGetLastError());
   return VUI_OK;
 }
@@ -749,8 +826,11 @@ static int pick(int epi, const LmGemm& g, int nz, hipStream_t st) {
     if (epi == LM_MOE_DOWN) return experts<T, 1, 16, LM_MOE_DOWN>(g, nz, st);
   }
   // few features still: half a block per workgroup where whole ones would leave half the CUs without, and the others take in a block's
-  // weights at 45 KB a us (16 x 2048 x 6144 13.4 -> 11.7 us, the mean of a 2048 wide step's thirteen 7.8 -> 7.0, with 4 rows 6.8 -> 6.5)
+  // weights at 45 KB a us (16 x 2048 x 6144 13.4 -> 11.7 us, the mean of a 2048 wide step's thirteen 7.8 -> 7.0, with 4 rows 6.8 -> 6.5; before half a
+  // block's weights were one load per step)
   if (few && epi == LM_PLAIN && (long)g.N / 16 * nz <= 128) return go<T, 1, 1, 16, LM_PLAIN, true>(g, nz, st);
+  if constexpr (sizeof(T) == 2)
+    if (few && epi == LM_OUT && g.N / 16 <= 128) return go<T, 1, 1, 16, LM_OUT, true>(g, nz, st);
   switch (epi) {
     case LM_IN_ATTN: return few ? go<T, 1, 2, 8, LM_IN_ATTN>(g, nz, st) : many<T, 2, LM_IN_ATTN>(g, nz, st);
     case LM_IN_GRU_STEP: return go<T, 1, 3, 8, LM_IN_GRU_STEP>(g, nz, st);
@@ -823,7 +903,7 @@ __global__ __launch_bounds__(256) void lm_embed_kernel(const LmRows where, const
     float s = (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
     s += dpp_f<DPP_QUAD_XOR1>(s);
     s += dpp_f<DPP_QUAD_XOR2>(s);
-    if ((c & 15) == 0) ssq[(size_t)m * np + (c >> 4)] = s;
+    if ((c & 15) == 0) reinterpret_cast<float2*>(ssq)[(size_t)m * np + (c >> 4)] = make_float2(s, 0.f);
   }
 }
 int launch_lm_embed(int dtype, const LmRows& where, const int64_t* tokens, const void* table, float* x, void* xt, float* ssq, int rows, int width,

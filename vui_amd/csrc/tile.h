@@ -59,6 +59,6 @@ __device__ __forceinline__ uint2 tl_read_tr(const void* lds) {
 template <typename T, int BK = 64>
 __host__ __device__ __forceinline__ size_t tl_off(int r, int k, int K) {
   constexpr int EP = 16 / (int)sizeof(T), LC = BK / 4;  // columns per lane
-  const int kb = k % BK, c = kb % LC;
-  return ((size_t)(r >> 4) * (K / BK) + k / BK) * (16 * BK) + (size_t)((c / EP) * (64 * EP) + ((r & 15) + 16 * (kb / LC)) * EP + c % EP);
+  const unsigned ku = (unsigned)k, kb = ku % BK, c = kb % LC;
+  return ((size_t)(r >> 4) * ((unsigned)K / BK) + ku / BK) * (16 * BK) + (size_t)((c / EP) * (64 * EP) + (((unsigned)r & 15) + 16 * (kb / LC)) * EP + c % EP);
 }
