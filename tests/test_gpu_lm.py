@@ -51,6 +51,24 @@ def test_prompts_of_many_lengths(name, dt):
             assert e < U.TOL[dt], (name, T, e)
 
 
+@BOTH
+@pytest.mark.parametrize("width, ff", [(16, 50), (64, 70), (320, 130), (576, 33), (128, 4300), (2112, 90), (2064, 2100)])
+def test_few_rows_at_the_edges_of_steps(width, ff, dt):
+    """Up to four rows share loads of X, up to 16 go by blocks and half blocks of features: K of one step, of fewer steps than waves, of more than a wave's
+    loads hold, features on both sides of 128 blocks; wanted places more than rows."""
+    cfg = U.config([U.attn(), U.gru(50)], width=width, ff=ff)
+    sd = U.weights(cfg, 31)
+    eng = U.engine(cfg, sd, dt, max_seq=32)
+    for T in (1, 2, 3, 4, 5, 16, 17):
+        toks = U.tokens(T, cfg["vocab"], T)
+        ref = O.forward(cfg, sd, toks)
+        with eng.new_row() as row:
+            assert U.err(run_all(row, toks), ref) < U.TOL[dt], T
+        with eng.new_row() as row:
+            want = [i % T for i in range(19)]
+            assert U.err(row.extend(toks, want), ref[want]) < U.TOL[dt], T
+
+
 def test_residual_stream_of_every_layer():
     cfg = U.mixed()
     sd = U.weights(cfg, 12)

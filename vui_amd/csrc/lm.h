@@ -49,7 +49,7 @@ struct LmGemm {
   size_t wz;      // elements between the weights of consecutive blockIdx.z
   const int32_t* rowmap;  // row of X behind output row m, or nullptr
   int x_rows;             // rows of X (bound of rowmap)
-  // row scale norm[0] / sqrt(sum(ssq[m]) / width + eps); ssq: (rows, np) pairs, of eight columns each (or of 16, the other 0)
+  // row scale norm[0] / sqrt(sum(ssq[m]) / width + eps); ssq: (rows, np), pairs with few rows (LM_PAIRS)
   const float* ssq;
   int np, width;
   float eps;

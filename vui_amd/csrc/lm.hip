@@ -65,7 +65,7 @@ static size_t lm_carve(const vui_lm_config* c, const vui_lm_layer* layers, vui_l
 #define TAKE(field, type, bytes) { const size_t o = take(bytes); if (x) x->field = (type)(base + o); }
   TAKE(x, float*, R * d.w64 * 4);
   TAKE(xt, void*, R * d.w64 * e);
-  TAKE(ssq, float*, R * (d.w16 / 16) * 8);
+  TAKE(ssq, float*, (R + 16) * (d.w16 / 16) * 4);  // pairs with up to 16 rows (R is 16 at least)
   TAKE(where, int2*, VUI_MAX_BATCH * 8);
   TAKE(qu, void*, qu * e);
   TAKE(qr, void*, qr * e);

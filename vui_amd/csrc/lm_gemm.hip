@@ -38,6 +38,10 @@ __device__ __forceinline__ float lm_act(float z, int kind, float pos, float neg)
   return (z > 0.f ? pos * z * z : neg * (expm1f(m) - m)) + 0.5f * z;
 }
 
+// Rows of a pass up to which sums of squares come as pairs (rows x np x 2), a half of a block's columns each, or the whole and 0: what half
+// blocks of an output projection can leave.  With more rows there is one per block: two cost a prompt of 1999 positions 1.3 %.
+#define LM_PAIRS 16
+
 // What a unit's epilogue reads besides the sums, requested ahead of the operands (few rows).
 struct LmPre {
   int slot, pos;
@@ -131,8 +135,10 @@ __device__ __forceinline__ void lm_unit(const LmGemm& p, const int m, const int 
     }
     sq = rows_sum(sq);  // the 16 columns of this row's block
     if (live && kg == 0 && nb < p.np) {
-      if (half < 0) reinterpret_cast<float2*>(p.ssq_out)[(size_t)m * p.np + nb] = make_float2(sq, 0.f);
-      else p.ssq_out[2 * ((size_t)m * p.np + nb) + half] = sq;
+      const size_t at = (size_t)m * p.np + nb;
+      if (half >= 0) p.ssq_out[2 * at + half] = sq;
+      else if (p.M <= LM_PAIRS) reinterpret_cast<float2*>(p.ssq_out)[at] = make_float2(sq, 0.f);
+      else p.ssq_out[at] = sq;
     }
     return;
   }
@@ -383,13 +389,18 @@ __global__ __launch_bounds__(64 * WAVES, sizeof(T) == 2 && MB == 1 && NB < 3 ? 4
   constexpr int TPR = WAVES * 64 / (MB * 16) > 64 ? 64 : WAVES * 64 / (MB * 16), NSQ = 4;
   const int sq_r = tid / TPR, sq_q = tid % TPR;
   int sq_m = 0;
-  float2 sq[NSQ];  // halves of a block's columns
+  float2 sq[NSQ];
   float norm = 0.f;
+  const bool pairs = LOGITS ? p.x_rows <= LM_PAIRS : MB == 1;  // of a block's columns there are two sums
+  auto sq_at = [&](int i) {
+    const size_t at = (size_t)sq_m * p.np + i;
+    return pairs ? reinterpret_cast<const float2*>(p.ssq)[at] : make_float2(p.ssq[at], 0.f);
+  };
   if (SCALED) {
     sq_m = min(m0 + min(sq_r, MB * 16 - 1), p.M - 1);
     if (LOGITS && p.rowmap) sq_m = min(max(p.rowmap[sq_m], 0), p.x_rows - 1);
 #pragma unroll
-    for (int i = 0; i < NSQ; ++i) sq[i] = reinterpret_cast<const float2*>(p.ssq)[(size_t)sq_m * p.np + min(sq_q + TPR * i, p.np - 1)];
+    for (int i = 0; i < NSQ; ++i) sq[i] = sq_at(min(sq_q + TPR * i, p.np - 1));
     norm = p.norm[0];
   }
   if (EARLY && s0 < s1) load(s0);
@@ -415,7 +426,7 @@ __global__ __launch_bounds__(64 * WAVES, sizeof(T) == 2 && MB == 1 && NB < 3 ? 4
 #pragma unroll
     for (int i = 0; i < NSQ; ++i) t += sq_q + TPR * i < p.np ? sq[i].x + sq[i].y : 0.f;
     for (int i = sq_q + TPR * NSQ; i < p.np; i += TPR) {
-      const float2 v = reinterpret_cast<const float2*>(p.ssq)[(size_t)sq_m * p.np + i];
+      const float2 v = sq_at(i);
       t += v.x + v.y;
     }
     t = lanes_sum<TPR>(t);
@@ -568,20 +579,19 @@ __global__ __launch_bounds__(256 * G, 2) void lm_wide_kernel(LM_HOT, const LmGem
     float a[NR];
 #pragma unroll
     for (int i = 0; i < NR; ++i) a[i] = 0.f;
-    const int np = 2 * p.np;  // halves of blocks
-    if ((np & 3) == 0) {
-      for (int c = 4 * l16; c < np; c += 64) {
+    if ((p.np & 3) == 0) {
+      for (int c = 4 * l16; c < p.np; c += 64) {
         float4 v[NR];
 #pragma unroll
-        for (int i = 0; i < NR; ++i) v[i] = *reinterpret_cast<const float4*>(p.ssq + (size_t)min(m0 + grp * NR + i, p.M - 1) * np + c);
+        for (int i = 0; i < NR; ++i) v[i] = *reinterpret_cast<const float4*>(p.ssq + (size_t)min(m0 + grp * NR + i, p.M - 1) * p.np + c);
 #pragma unroll
         for (int i = 0; i < NR; ++i) a[i] += (v[i].x + v[i].y) + (v[i].z + v[i].w);
       }
     } else {
-      for (int c = l16; c < np; c += 16) {
+      for (int c = l16; c < p.np; c += 16) {
         float v[NR];
 #pragma unroll
-        for (int i = 0; i < NR; ++i) v[i] = p.ssq[(size_t)min(m0 + grp * NR + i, p.M - 1) * np + c];
+        for (int i = 0; i < NR; ++i) v[i] = p.ssq[(size_t)min(m0 + grp * NR + i, p.M - 1) * p.np + c];
 #pragma unroll
         for (int i = 0; i < NR; ++i) a[i] += v[i];
       }
@@ -903,7 +913,11 @@ __global__ __launch_bounds__(256) void lm_embed_kernel(const LmRows where, const
     float s = (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
     s += dpp_f<DPP_QUAD_XOR1>(s);
     s += dpp_f<DPP_QUAD_XOR2>(s);
-    if ((c & 15) == 0) reinterpret_cast<float2*>(ssq)[(size_t)m * np + (c >> 4)] = make_float2(s, 0.f);
+    if ((c & 15) == 0) {
+      const size_t at = (size_t)m * np + (c >> 4);
+      if (rows <= LM_PAIRS) reinterpret_cast<float2*>(ssq)[at] = make_float2(s, 0.f);
+      else ssq[at] = s;
+    }
   }
 }
 int launch_lm_embed(int dtype, const LmRows& where, const int64_t* tokens, const void* table, float* x, void* xt, float* ssq, int rows, int width,
