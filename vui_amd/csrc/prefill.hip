@@ -211,20 +211,26 @@ __global__ __launch_bounds__(64 * WAVES) void pf_gemm_kernel(PF_HOT, const PfGem
   for (int i = 0; i < NB; ++i)
 #pragma unroll
     for (int j = 0; j < MB; ++j) { acc[i][j] = pf_floatx4{0.f, 0.f, 0.f, 0.f}; acc2[i][j] = acc[i][j]; }
-  uint4 xa[MB][2], wa[NB][2], va[NB][2], g[2];
-  auto load = [&](int s) {
-    const int k = s << 10;
+  // Steps whose loads go out together, as far as the wave has them
+  constexpr int U = WAVES >= 12 && MB * NB <= 2 ? 2 : 1;
+  uint4 xs[U][MB][2], ws[U][NB][2], vs[U][NB][2], gs[U][2];
+  auto load = [&](int s0) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
+    for (int u = 0; u < U; ++u) {
+      const int s = s0 + u, k = s << 10;
+      if (u > 0 && s >= s1) break;  // uniform
 #pragma unroll
-      for (int j = 0; j < NB; ++j) {
-        if (I8 && h) continue;  // both halves of an int8 block are one piece
-        wa[j][h] = *reinterpret_cast<const uint4*>(wr[j] + (size_t)s * WB + 1024 * h);
-        if (DUAL) va[j][h] = *reinterpret_cast<const uint4*>(vr[j] + (size_t)s * WB + 1024 * h);
+      for (int h = 0; h < 2; ++h) {
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+          if (I8 && h) continue;  // both halves of an int8 block are one piece
+          ws[u][j][h] = *reinterpret_cast<const uint4*>(wr[j] + (size_t)s * WB + 1024 * h);
+          if (DUAL) vs[u][j][h] = *reinterpret_cast<const uint4*>(vr[j] + (size_t)s * WB + 1024 * h);
+        }
+#pragma unroll
+        for (int j = 0; j < MB; ++j) xs[u][j][h] = *reinterpret_cast<const uint4*>(xr[j] + k + 512 * h);
+        if (NORM) gs[u][h] = *reinterpret_cast<const uint4*>(p.nw + 64 * s + 16 * kg + 8 * h);
       }
-#pragma unroll
-      for (int j = 0; j < MB; ++j) xa[j][h] = *reinterpret_cast<const uint4*>(xr[j] + k + 512 * h);
-      if (NORM) g[h] = *reinterpret_cast<const uint4*>(p.nw + 64 * s + 16 * kg + 8 * h);
     }
   };
   // The operands of the first step go out before anything else is asked for, then the residual values this thread will add to (its
@@ -256,8 +262,12 @@ __global__ __launch_bounds__(64 * WAVES) void pf_gemm_kernel(PF_HOT, const PfGem
 #pragma unroll
     for (int j = 0; j < MB; ++j) rf[j] = 1.0f / sqrtf(rows_sum(ss[j]) / (float)p.K + p.eps);
   }
-  for (int s = s0; s < s1; ++s) {
+  for (int s = s0; s < s1; s += U) {
     if (WAVES < 8 || s > s0) load(s);
+#pragma unroll
+    for (int q = 0; q < U; ++q) {
+    if (q > 0 && s + q >= s1) break;  // uniform
+    uint4 (&xa)[MB][2] = xs[q], (&wa)[NB][2] = ws[q], (&va)[NB][2] = vs[q], (&g)[2] = gs[q];
     if (I8) {
 #pragma unroll
       for (int j = 0; j < NB; ++j) {
@@ -284,6 +294,7 @@ __global__ __launch_bounds__(64 * WAVES) void pf_gemm_kernel(PF_HOT, const PfGem
           acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf_frag(wa[i][h]), pf_frag(xa[j][h]), acc[i][j], 0, 0, 0);
           if (DUAL) acc2[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf_frag(va[i][h]), pf_frag(xa[j][h]), acc2[i][j], 0, 0, 0);
         }
+    }
   }
   // partial tiles to LDS: [wave][(i, j)][lane] as float4
 #pragma unroll
@@ -299,16 +310,21 @@ __global__ __launch_bounds__(64 * WAVES) void pf_gemm_kernel(PF_HOT, const PfGem
   const int i = wave / MB, j = wave % MB;
   const int m = m0 + 16 * j + l16, n = n0 + 16 * i + 4 * kg;
   float v[4], u[4];
+  {  // all waves' parts are read before the first is added
+    pf_floatx4 a[WAVES], b[DUAL ? WAVES : 1];
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int e = tid * 4 + r;
-    v[r] = part[e];
-    if (DUAL) u[r] = part[TILE + e];
+    for (int w = 0; w < WAVES; ++w) {
+      a[w] = *reinterpret_cast<const pf_floatx4*>(&part[w * PW + tid * 4]);
+      if (DUAL) b[w] = *reinterpret_cast<const pf_floatx4*>(&part[w * PW + TILE + tid * 4]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int w = 1; w < WAVES; ++w) {
-      v[r] += part[w * PW + e];
-      if (DUAL) u[r] += part[w * PW + TILE + e];
+      a[0] += a[w];
+      if (DUAL) b[0] += b[w];
     }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) { v[r] = a[0][r]; if (DUAL) u[r] = b[0][r]; }
   }
   const bool out = m < p.M && n < p.N;  // N is a multiple of 16
   if (EPI == PF_QKV && !NORM && p.vt && n0 + 16 * i >= p.nq + p.nkv && n0 + 16 * i < p.N) {
