@@ -278,6 +278,12 @@ def test_short_blocks_behind_a_cache(heads, kv, window):
                 m.decoder.forward_flash(x, None)
 
 
+@pytest.mark.parametrize("heads,kv,window", [(8, 2, 0), (8, 1, 70), (16, 4, 300)])
+def test_short_blocks_of_a_multiple_of_eight_heads(heads, kv, window):
+    """Cached positions are read ahead by the heads that an XCD attends to, a group's once."""
+    test_short_blocks_behind_a_cache(heads, kv, window)
+
+
 @pytest.mark.parametrize("window,every,heads,dim", [(128, 3, 4, 64), (300, 2, 4, 64), (300, 4, 4, 64), (40, 2, 4, 64), (300, 2, 2, 96)])
 def test_short_blocks_of_layers_with_and_without_a_window(window, every, heads, dim):
     """Windowed and global layers in one model, behind caches where the ranges of keys that a layer's attention is dealt in are

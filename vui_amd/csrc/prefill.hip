@@ -50,6 +50,7 @@ struct PfGemm {
   // pf_order: tiles of an XCD (the first xcd_more have one more), tiles of one step of the slower index
   uint32_t xcd_tiles, xcd_more, run, inv_run, inv_hd;
   int by_rows, n_tiles;
+  int warm_gsz;         // heads per group, or 0 (see pf_warm)
   int warm, warm_from;  // the last `warm` workgroups only fetch the cached positions warm_from .. pos0 - 1 (see pf_warm)
 };
 
@@ -60,7 +61,25 @@ __device__ __forceinline__ uint32_t pf_div(uint32_t i, uint32_t inv) { return in
 // The attention of a short block is a few workgroups that wait for cached keys and values from memory (2.4 us of its first
 // step, 0.85 where they are in the memory-side cache).  The QKV product before it leaves compute units idle: workgroups of
 // its launch that have no tile read them ahead.
+// Where XCD x attends to heads x, x + 8, ... (a number of heads that eight divides), its readers take those heads' columns, so that they lie in
+// its L2 (measured together with pf_ahead below).
 __device__ __forceinline__ void pf_warm(const PfGemm& p, int part) {
+  if (p.warm_gsz > 0) {
+    const int x = (int)blockIdx.x & 7, lead = p.n_tiles + ((x - p.n_tiles) & 7), mine = ((int)blockIdx.x - lead) >> 3, all = ((int)gridDim.x - 1 - lead) / 8 + 1;
+    const int per = p.hd >> 3, rows = (int)blockDim.x / per, row = (int)threadIdx.x / per, col = ((int)threadIdx.x - row * per) * 8;
+    if (row >= rows) return;
+    for (int h = x, last = -1; h * p.hd < p.nq; h += 8) {
+      const int g = h / p.warm_gsz;
+      if (g == last) continue;  // heads of a group share keys
+      last = g;
+      for (int j = p.warm_from + mine * rows + row; j < p.pos0; j += all * rows) {
+        const size_t at = (size_t)j * p.nkv + g * p.hd + col;
+        const uint4 k = *reinterpret_cast<const uint4*>(p.kc + at), v = *reinterpret_cast<const uint4*>(p.vc + at);
+        asm volatile("" ::"v"(k.x), "v"(v.x));
+      }
+    }
+    return;
+  }
   const size_t n = (size_t)(p.pos0 - p.warm_from) * p.nkv / 8, at = (size_t)p.warm_from * p.nkv;
   for (size_t i = (size_t)part * blockDim.x + threadIdx.x; i < n; i += (size_t)p.warm * blockDim.x) {
     const uint4 k = *reinterpret_cast<const uint4*>(p.kc + at + i * 8), v = *reinterpret_cast<const uint4*>(p.vc + at + i * 8);
@@ -689,7 +708,37 @@ struct PfDirectArgs {
   float *part, *ml;  // (head, tile, split): sums (DT x 64 lanes x 4), {max, sum of weights} x 16
   uint32_t* count;   // arrivals of a (head, tile) in the pass; `before`: those of earlier layers (their splits differ: windows)
   uint32_t before;
+  int nsp;           // splits; workgroups of higher blockIdx.z read ahead: `n_ahead` matrices, one behind the other
+  const char* ahead;
+  uint32_t ahead_bytes[5];
+  int n_ahead;
 };
+// A short block's products wait for their weights (1-2 us of launches of 3-5), and its attention leaves most compute units idle: workgroups of its
+// launch read the weights of the products up to the next attention into the L2s that will ask for them.  L2s keep what they hold
+// from launch to launch; pf_order deals an eighth of a matrix's features to an XCD, and workgroup i is on XCD i % 8.  Measured, a whole prompt on
+// the device: 23 positions in bf16 705 -> 635 us, four of 23 2294 -> 2130; 16 of 16 in int8, half the bytes, 8.9 ms both.  No more than PF_AHEAD_BYTES:
+// the L2s of a card hold 32 MB, and what does not stay is read twice.
+#define PF_AHEAD 20  // workgroups per XCD
+#define PF_AHEAD_BYTES (24u << 20)
+__device__ __forceinline__ void pf_ahead(const PfDirectArgs& a) {
+  const uint32_t plane = gridDim.x * gridDim.y, first = plane * a.nsp, i = blockIdx.x + gridDim.x * blockIdx.y + plane * blockIdx.z, x = i & 7u;
+  const uint32_t lead = first + ((x - first) & 7u), mine = (i - lead) >> 3, all = ((plane * gridDim.z - 1 - lead) >> 3) + 1;  // of the XCD's readers
+  const char* base = a.ahead;
+#pragma unroll
+  for (int k = 0; k < 5; ++k) {
+    if (k >= a.n_ahead) break;
+    const uint32_t n = a.ahead_bytes[k] >> 4, lo = (uint32_t)((uint64_t)n * x >> 3), hi = (uint32_t)((uint64_t)n * (x + 1) >> 3);  // in pieces of 16 bytes
+    const uint4* src = reinterpret_cast<const uint4*>(base);
+    for (uint32_t at = lo + mine * 4 * blockDim.x + threadIdx.x; at < hi; at += all * 4 * blockDim.x) {
+      uint4 v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] = src[min(at + u * blockDim.x, hi - 1)];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) asm volatile("" ::"v"(v[u].x));
+    }
+    base += a.ahead_bytes[k];
+  }
+}
 template <int HD32>
 __global__ __launch_bounds__(64 * PfDirect<HD32>::WAVES) void pf_direct_attn_kernel(const bf16_t* q, const bf16_t* kc, const bf16_t* vc, int T, int nq,
                                                                                     int nkv, int gsz, int pos0, int window, const PfDirectArgs a0) {
@@ -698,13 +747,14 @@ __global__ __launch_bounds__(64 * PfDirect<HD32>::WAVES) void pf_direct_attn_ker
   typedef PfDirect<HD32> P;
   constexpr int HD = P::HD, DT = P::DT, WAVES = P::WAVES;
   extern __shared__ __align__(16) char lds[];
+  if ((int)blockIdx.z >= a.nsp) { pf_ahead(a); return; }
   float* s_m = (float*)(lds + P::VB);
   float* s_l = (float*)(lds + P::VB + P::ML);
   uint32_t* s_last = (uint32_t*)(lds + P::VB + 2 * P::ML);
   float* s_acc = (float*)lds;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int l16 = lane & 15, kg = lane >> 4;
-  const int h = blockIdx.x, kvh = h / a.gsz, q0 = blockIdx.y * 16, sp = blockIdx.z, nsp = gridDim.z;
+  const int h = blockIdx.x, kvh = h / a.gsz, q0 = blockIdx.y * 16, sp = blockIdx.z, nsp = a.nsp;
   const int tq = min(q0 + l16, a.T - 1);
   const int qlast = a.pos0 + tq, qfirst = a.window > 0 ? max(0, qlast - a.window) : 0;  // visible keys of this lane's query
   const int t_hi = min(q0 + 15, a.T - 1);
@@ -722,7 +772,8 @@ __global__ __launch_bounds__(64 * PfDirect<HD32>::WAVES) void pf_direct_attn_ker
   float m_run = -INFINITY, l_run = 0.f;
   for (int k0 = lo + 32 * wave; k0 < hi; k0 += 32 * WAVES) {
     // a key behind the last visible one reads that one again; its weight is zero
-    uint4 kf[2][HD32], vr[DT];
+    uint4 kf[2][HD32];
+    tl_u32x4 vr[DT];  // native vectors: an array of HIP's structs stays in scratch memory
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
@@ -730,7 +781,7 @@ __global__ __launch_bounds__(64 * PfDirect<HD32>::WAVES) void pf_direct_attn_ker
 #pragma unroll
     for (int i = 0; i < DT; ++i) {  // 32 rows of HD values, in the order of LDS
       const int e = i * 512 + lane * 8, row = e / HD;
-      vr[i] = *reinterpret_cast<const uint4*>(vb + (size_t)min(k0 + row, kend - 1) * a.nkv + (e - row * HD));
+      vr[i] = *reinterpret_cast<const tl_u32x4*>(vb + (size_t)min(k0 + row, kend - 1) * a.nkv + (e - row * HD));
     }
     __builtin_amdgcn_sched_barrier(0);
     pf_floatx4 sc[2];
@@ -741,7 +792,7 @@ __global__ __launch_bounds__(64 * PfDirect<HD32>::WAVES) void pf_direct_attn_ker
       for (int c = 0; c < HD32; ++c) sc[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf_frag(kf[kt][c]), pf_frag(qf[c]), sc[kt], 0, 0, 0);
     }
 #pragma unroll
-    for (int i = 0; i < DT; ++i) *reinterpret_cast<uint4*>(own + i * 1024 + lane * 16) = vr[i];
+    for (int i = 0; i < DT; ++i) *reinterpret_cast<tl_u32x4*>(own + i * 1024 + lane * 16) = vr[i];
     float mx = -INFINITY;
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt)
@@ -852,7 +903,9 @@ template <int HD32> static int pf_direct_attn(PfDirectArgs& a, int H, hipStream_
   const int L = a.pos0 + a.T, keys = a.window > 0 && a.window + 48 < L ? a.window + 48 : L, n = (keys + 127) / 128;
   HIP_TRY(hipFuncSetAttribute((const void*)pf_direct_attn_kernel<HD32>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   const int splits = n > PF_SPLITS ? PF_SPLITS : n;
-  hipLaunchKernelGGL(pf_direct_attn_kernel<HD32>, dim3(H, (a.T + 15) / 16, splits), dim3(64 * PfDirect<HD32>::WAVES), lds, st, a.q, a.kc, a.vc, a.T, a.nq,
+  a.nsp = splits;
+  const int plane = H * ((a.T + 15) / 16), readers = (8 * PF_AHEAD + plane - 1) / plane;
+  hipLaunchKernelGGL(pf_direct_attn_kernel<HD32>, dim3(H, (a.T + 15) / 16, splits + readers), dim3(64 * PfDirect<HD32>::WAVES), lds, st, a.q, a.kc, a.vc, a.T, a.nq,
                      a.nkv, a.gsz, a.pos0, a.window, a);
   if (splits > 1) a.before += splits;
   return VUI_OK;
@@ -1085,7 +1138,7 @@ int launch_prefill(const vui_config& c, const vui_weights& w, const void* tiled_
     if (tiny) hipLaunchKernelGGL(pf_rownorm_kernel<true>, grid, dim3(256), 0, st, x, (const bf16_t*)w, y, T, d, c.norm_eps, y_tiled, len, L);
     else hipLaunchKernelGGL(pf_rownorm_kernel<false>, grid, dim3(256), 0, st, x, (const bf16_t*)w, y, T, d, c.norm_eps, y_tiled, len, L);
   };
-  PfDirectArgs da = {q, nullptr, nullptr, att, T, nq, nkv, H / KV, pos0, 0, scale, part, ml, count, 0};
+  PfDirectArgs da = {q, nullptr, nullptr, att, T, nq, nkv, H / KV, pos0, 0, scale, part, ml, count};
   int rc;
   for (int l = 0; l < c.n_layers; ++l) {
     const vui_layer_weights& lw = w.layers[l];
@@ -1102,12 +1155,19 @@ int launch_prefill(const vui_config& c, const vui_weights& w, const void* tiled_
     g.vc = (bf16_t*)v_cache + slab * l + (size_t)slot * S * nkv;
     const int win = layer_window(c, l);
     if (!tiny && pos0 == 0) { g.kt = kt; g.vt = vt; }
-    if (tiny && pos0 > 0) { g.warm_from = win > 0 && pos0 > win ? pos0 - win : 0; g.warm = PF_WARM; }
+    if (tiny && pos0 > 0) { g.warm_from = win > 0 && pos0 > win ? pos0 - win : 0; g.warm = PF_WARM; g.warm_gsz = H % 8 == 0 ? H / KV : 0; }
     g.rope = layer_rope(c, w, l, &g.rope_dim);
     g.nq = nq; g.nkv = nkv; g.hd = hd; g.inv_hd = pf_inv(hd); g.pos0 = pos0; g.Lpad = Lpad;
     if ((rc = pf_gemm4<PF_QKV, false>(g, i8, st))) return rc;
     if (tiny) {
       da.kc = g.kc; da.vc = g.vc; da.window = win;
+      da.ahead = t_o;
+      const size_t ff = (size_t)F * d * wsz, sizes[5] = {(size_t)d * nq * wsz, ff, ff, ff, (size_t)(nq + 2 * nkv) * d * wsz};  // the last: the next layer's
+      size_t sum = 0;
+      for (da.n_ahead = 0; da.n_ahead < (l + 1 < c.n_layers ? 5 : 4); ++da.n_ahead) {
+        if ((sum += sizes[da.n_ahead]) > PF_AHEAD_BYTES) break;
+        da.ahead_bytes[da.n_ahead] = (uint32_t)sizes[da.n_ahead];
+      }
       switch (hd / 32) {
         case 1: rc = pf_direct_attn<1>(da, H, st); break;
         case 2: rc = pf_direct_attn<2>(da, H, st); break;
