@@ -498,30 +498,64 @@ static int pf_wide(int tile, PfGemm& g, hipStream_t st) {
 
 // two-rounding RMSNorm of rows (src/vui/model.py:286-297); one wave per row.  len != nullptr: the slot's new length goes there
 // (where a row lies is known when compiled: asked for per piece it took a launch 0.3 us, 65 positions behind 600 3.57 -> 3.95)
-template <bool X_TILED>
+// The row stays in registers, NP pieces of eight columns per lane, and the weights are asked for with it: one trip to memory instead of
+// two, one after the other.  Whole prompts, us: 576 positions 1109 -> 1098, 1733 in int8 1955 -> 1917.  Four and eight rows per wave, which write
+// whole lines of the tiled rows, were slower (576: 1115 and 1170).  NP 0: rows of more than 2048 columns, read twice.
+template <bool X_TILED, int NP>
 __global__ __launch_bounds__(256) void pf_rownorm_kernel(const bf16_t* x, const bf16_t* w, bf16_t* y, int M, int K, float eps, int y_tiled,
                                                          int32_t* len, int len_to) {
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (len && blockIdx.x == 0 && threadIdx.x == 0) *len = len_to;
   if (row >= M) return;
-  auto xr = [&](int k) { return x + (X_TILED ? pf_toff(row, k, K) : (size_t)row * K + k); };
+  const int nc = K >> 3;
+  auto ld = [&](const bf16_t* q) { return *reinterpret_cast<const uint4*>(q); };
+  auto xr = [&](int c) { return ld(x + (X_TILED ? pf_toff(row, c * 8, K) : (size_t)row * K + c * 8)); };
+  uint4 xv[NP > 0 ? NP : 1], wv[NP > 0 ? NP : 1];
+  if constexpr (NP > 0) {
+#pragma unroll
+    for (int i = 0; i < NP; ++i) xv[i] = xr(min(lane + WAVE * i, nc - 1));
+#pragma unroll
+    for (int i = 0; i < NP; ++i) wv[i] = ld(w + min(lane + WAVE * i, nc - 1) * 8);
+    __builtin_amdgcn_sched_barrier(0);
+  }
   float ss = 0.f;
-  for (int c = lane; c < K / 8; c += WAVE) {
+  auto add = [&](const uint4& q) {
     float v[8];
-    El<bf16_t>::ld8(xr(c * 8), v);
+    El<bf16_t>::ld8(reinterpret_cast<const bf16_t*>(&q), v);
 #pragma unroll
     for (int e = 0; e < 8; ++e) ss = fmaf(v[e], v[e], ss);
+  };
+  if constexpr (NP > 0) {
+#pragma unroll
+    for (int i = 0; i < NP; ++i)
+      if (lane + WAVE * i < nc) add(xv[i]);
+  } else {
+    for (int c = lane; c < nc; c += WAVE) add(xr(c));
   }
   ss = wave_sum(ss);
   const float r = 1.0f / sqrtf(ss / (float)K + eps);
-  for (int c = lane; c < K / 8; c += WAVE) {
-    float v[8], g[8], o[8];
-    El<bf16_t>::ld8(xr(c * 8), v);
-    El<bf16_t>::ld8(w + c * 8, g);
+  auto put = [&](int c, const uint4& q, const uint4& g) {
+    *reinterpret_cast<uint4*>(y + (y_tiled ? pf_toff(row, c * 8, K) : (size_t)row * K + c * 8)) = pf_norm8(q, r, g);
+  };
+  if constexpr (NP > 0) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) o[e] = bf2f(f2bf(v[e] * r)) * g[e];
-    El<bf16_t>::st8(y + (y_tiled ? pf_toff(row, c * 8, K) : (size_t)row * K + c * 8), o);
+    for (int i = 0; i < NP; ++i)
+      if (lane + WAVE * i < nc) put(lane + WAVE * i, xv[i], wv[i]);
+  } else {
+    for (int c = lane; c < nc; c += WAVE) put(c, xr(c), ld(w + c * 8));
   }
+}
+template <bool X_TILED>
+static void pf_rownorm(const bf16_t* x, const void* w, bf16_t* y, int M, int K, float eps, int y_tiled, int32_t* len, int len_to, hipStream_t st) {
+#define PF_NORM(NP) hipLaunchKernelGGL((pf_rownorm_kernel<X_TILED, NP>), dim3((M + 3) / 4), dim3(256), 0, st, x, (const bf16_t*)w, y, M, K, eps, y_tiled, len, len_to)
+  switch ((K / 8 + WAVE - 1) / WAVE) {
+    case 1: PF_NORM(1); break;
+    case 2: PF_NORM(2); break;
+    case 3: PF_NORM(3); break;
+    case 4: PF_NORM(4); break;
+    default: PF_NORM(0);
+  }
+#undef PF_NORM
 }
 
 // The residual of the new positions.  Short block (ssq): tiled, with the sums of squares of every 16 columns of a row, and the
@@ -1134,9 +1168,8 @@ int launch_prefill(const vui_config& c, const vui_weights& w, const void* tiled_
                        tiny ? ssq : nullptr, tiny ? nullptr : vt, count, (int)sets, T, d, nkv, L, Lpad);
   }
   auto norm = [&](const void* w, bf16_t* y, int y_tiled, int32_t* len) {
-    const dim3 grid((T + 3) / 4);
-    if (tiny) hipLaunchKernelGGL(pf_rownorm_kernel<true>, grid, dim3(256), 0, st, x, (const bf16_t*)w, y, T, d, c.norm_eps, y_tiled, len, L);
-    else hipLaunchKernelGGL(pf_rownorm_kernel<false>, grid, dim3(256), 0, st, x, (const bf16_t*)w, y, T, d, c.norm_eps, y_tiled, len, L);
+    if (tiny) pf_rownorm<true>(x, w, y, T, d, c.norm_eps, y_tiled, len, L, st);
+    else pf_rownorm<false>(x, w, y, T, d, c.norm_eps, y_tiled, len, L, st);
   };
   PfDirectArgs da = {q, nullptr, nullptr, att, T, nq, nkv, H / KV, pos0, 0, scale, part, ml, count};
   int rc;
