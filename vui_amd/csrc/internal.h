@@ -5,6 +5,28 @@
 
 #include "../../include/vui_amd.h"
 
+// exp(scale (s - m)) for s <= m in eight instructions (expf behind its product and difference takes fifteen): the hardware's power of two at the
+// rounded exponent and a first-order correction by what rounding left out.  NaN stays NaN, anything below 2^-250 is zero.
+// Relative error against 64 bits (root mean square), expf / this / one fma and the power of two alone: heads of 96, s of deviation 4
+// 2.7e-7 / 1.5e-7 / 2.9e-7; of 64, deviation 12 4.5e-7 / 4.5e-7 / 8.5e-7; of 192 8.2e-7 / 4.3e-7 / 8.9e-7.
+struct WeightExp {
+  float hi, lo;  // scale log2 e
+  float floor;   // of s - m
+};
+static inline WeightExp weight_exp(double scale) {
+  const double c = scale * 1.4426950408889634074;
+  WeightExp w;
+  w.hi = (float)c; w.lo = (float)(c - (double)w.hi); w.floor = (float)(-250.0 / c);
+  return w;
+}
+#ifdef __HIPCC__
+__device__ __forceinline__ float weight_of(float s, float m, const WeightExp& w) {
+  const float x = __builtin_elementwise_maximum(s - m, w.floor), p = x * w.hi;
+  const float f = fmaf(x, w.lo, fmaf(x, w.hi, -p)), e = __builtin_amdgcn_exp2f(p);
+  return fmaf(e * 0.69314718f, f, e);
+}
+#endif
+
 // epilogues of the fused GEMV
 enum {
   EPI_STORE = 0,   // y = rnd(acc)

@@ -257,17 +257,17 @@ __global__ __launch_bounds__(256, 2) void latent_attn_mfma_kernel(int2* where, c
       if (KT == 1) a += *reinterpret_cast<const tl_f32x4*>(&sco[(2 + u) & 3][lane * 4]);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const float v = j0 + 16 * u + 4 * kg + r < hi ? a[r] * p.scale : -INFINITY;
+        const float v = j0 + 16 * u + 4 * kg + r < hi ? a[r] : -INFINITY;
         sv[4 * u + r] = v;
         mx = fmaxf(mx, v);
       }
     }
     mx = rows_max(mx);
     const float m_new = fmaxf(m_run, mx);  // finite: key j0 is in range
-    const float alpha = expf(m_run - m_new);
+    const float alpha = weight_of(m_run, m_new, p.we);
     float pv[4 * NT], ps = 0.f;
 #pragma unroll
-    for (int e = 0; e < 4 * NT; ++e) { pv[e] = expf(sv[e] - m_new); ps += pv[e]; }
+    for (int e = 0; e < 4 * NT; ++e) { pv[e] = weight_of(sv[e], m_new, p.we); ps += pv[e]; }
     l_run = l_run * alpha + ps;
     m_run = m_new;
     uint4 hi4[KT], lo4[KT];
@@ -350,7 +350,7 @@ __global__ __launch_bounds__(512) void latent_value_kernel(int2* where, const vo
 #pragma unroll
     for (int u = 0; u < 16; ++u) v[u] = load(u);
     const float mx = wave_max(lane < np ? ml.x : -INFINITY);
-    float w = lane < np ? expf(ml.x - mx) : 0.f;
+    float w = lane < np ? weight_of(ml.x, mx, p.we) : 0.f;
     w /= wave_sum(w * ml.y);
     float o[4] = {0.f, 0.f, 0.f, 0.f};
     for (int s0 = 0;;) {
@@ -405,12 +405,12 @@ __global__ __launch_bounds__(512) void latent_value_kernel(int2* where, const vo
 // average keeps about 16 bits of them.  DB = dim64 / 64, RB = rot32 / 32, VT >= vdim16 / 16.
 // Bound by the keys and values that every tile of queries fetches from L2 (16 heads of 128 + 64 and 128, 1999 positions:
 // 1.7 GB in 60 us).  Neighbouring workgroups take different heads, so that an XCD's L2 holds few of them, masks and the
-// rescaling of the sums only in the steps that need them: 73 -> 60 us there (56 us with weights by v_exp_f32 alone, which are
-// less exact than expf's).  Two tiles of queries per wave were quicker there and slower at 600 positions of eight heads,
+// rescaling of the sums only in the steps that need them: 73 -> 60 us there; weights by weight_of instead of expf 63.7 -> 61.3 (another
+// machine; 56 for 60 by the power of two alone, which is less exact than expf).  Two tiles of queries per wave were quicker there and slower at 600 positions of eight heads,
 // and gave nothing of it in the whole prompt's time.
 #define LPF_WAVES (VT <= 4 ? 8 : 4)
 template <int DB, int RB, int VT>
-__global__ __launch_bounds__(64 * LPF_WAVES, 2) void latent_prefill_kernel(const LatentArgs p) {
+__global__ __launch_bounds__(64 * LPF_WAVES, 2) void latent_prefill_kernel(const LatentArgs p, const WeightExp we) {
   __shared__ __align__(16) float s_acc[LPF_WAVES][VT * 256];
   __shared__ float s_m[LPF_WAVES][16], s_l[LPF_WAVES][16];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -454,8 +454,6 @@ __global__ __launch_bounds__(64 * LPF_WAVES, 2) void latent_prefill_kernel(const
       sc[t] = tl_f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int i = 0; i < 2 * DB + RB; ++i) sc[t] = Tl<bf16_t>::mma(kf[t][i], qf[i], sc[t]);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) sc[t][r] *= p.scale;
     }
     if (k0 + 31 > pos0 + q0) {  // a key that some query of the tile does not see
 #pragma unroll
@@ -470,11 +468,11 @@ __global__ __launch_bounds__(64 * LPF_WAVES, 2) void latent_prefill_kernel(const
     mx = rows_max(mx);
     const float m_new = fmaxf(m_run, mx);
     const float m_use = m_new == -INFINITY ? 0.f : m_new;
-    const float alpha = expf(m_run - m_use);
+    const float alpha = weight_of(m_run, m_use, we);
     float pv[8], lo[8], ps = 0.f;
     uint4 hi4, lo4;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) { pv[e] = expf(sc[e >> 2][e & 3] - m_use); ps += pv[e]; }
+    for (int e = 0; e < 8; ++e) { pv[e] = weight_of(sc[e >> 2][e & 3], m_use, we); ps += pv[e]; }
     l_run = l_run * alpha + ps;
     m_run = m_new;
     hi4.x = f2bf2(pv[0], pv[1]); hi4.y = f2bf2(pv[2], pv[3]); hi4.z = f2bf2(pv[4], pv[5]); hi4.w = f2bf2(pv[6], pv[7]);
@@ -508,7 +506,7 @@ __global__ __launch_bounds__(64 * LPF_WAVES, 2) void latent_prefill_kernel(const
     float den = 0.f, o[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 0; w < LPF_WAVES; ++w) {
-      const float f = s_m[w][q] == -INFINITY ? 0.f : expf(s_m[w][q] - M);
+      const float f = s_m[w][q] == -INFINITY ? 0.f : weight_of(s_m[w][q], M, we);
       den = fmaf(f, s_l[w][q], den);
 #pragma unroll
       for (int r = 0; r < 4; ++r) o[r] = fmaf(f, s_acc[w][sl * 4 + r], o[r]);
@@ -619,9 +617,10 @@ bool latent_expand_ok(const vui_lm_dims& d) { return d.dim64 <= 128 && d.rot32 <
 template <int DB, int RB>
 static void lpf_go(const LatentArgs& a, hipStream_t st) {
   const dim3 grid(a.heads, (a.M + 15) / 16);
-  if (a.d.vdim16 <= 32) hipLaunchKernelGGL((latent_prefill_kernel<DB, RB, 2>), grid, dim3(512), 0, st, a);
-  else if (a.d.vdim16 <= 64) hipLaunchKernelGGL((latent_prefill_kernel<DB, RB, 4>), grid, dim3(512), 0, st, a);
-  else hipLaunchKernelGGL((latent_prefill_kernel<DB, RB, 8>), grid, dim3(256), 0, st, a);
+  const WeightExp we = weight_exp(a.scale);
+  if (a.d.vdim16 <= 32) hipLaunchKernelGGL((latent_prefill_kernel<DB, RB, 2>), grid, dim3(512), 0, st, a, we);
+  else if (a.d.vdim16 <= 64) hipLaunchKernelGGL((latent_prefill_kernel<DB, RB, 4>), grid, dim3(512), 0, st, a, we);
+  else hipLaunchKernelGGL((latent_prefill_kernel<DB, RB, 8>), grid, dim3(256), 0, st, a, we);
 }
 int launch_latent_prefill_attn(const LatentArgs& a, hipStream_t st) {
   if (!latent_expand_ok(a.d) || a.dtype != VUI_DTYPE_BF16 || !a.rows.seq) { vui_set_error("latent prefill: sizes out of range"); return VUI_EINVAL; }

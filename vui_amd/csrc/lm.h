@@ -127,6 +127,7 @@ struct LatentArgs {
   void *c_cache, *kr_cache;
   // pieces (rows, heads, n_splits): unnormalised latent average (rank64), {max, sum}
   float *part, *part_ml;
+  WeightExp we;    // of the maxima in part_ml: scores before their scale from the matrix cores, scaled ones otherwise
   int n_splits;
   const float* gate;
   void* act;

@@ -247,6 +247,7 @@ static int lm_attention(vui_lm_ctx* x, int l, int M, const LmRows& rows, LmGemm&
     return launch_latent_prefill_attn(a, st);
   }
   a.n_splits = lm_splits(M, L.heads, d.rank64);
+  a.we = weight_exp(c.dtype == VUI_DTYPE_BF16 && latent_mfma_ok(d) ? L.scale : 1.0);
   if ((rc = launch_latent_query(a, st))) return rc;
   if ((rc = launch_latent_attn(a, st))) return rc;
   return launch_latent_value(a, st);
