@@ -144,13 +144,27 @@ struct WideTile {
 enum { WIDE_NONE = -1, WIDE_128 = 0, WIDE_64x128 = 1, WIDE_64 = 2, WIDE_64x128_2 = 3, WIDE_64_2 = 4 };
 static inline int wide_pick(int M, int N, int K, double keep) {
   static const struct { int bm, bn; double wait, work; } tile[] = {{128, 128, 0.335, 0.144}, {64, 128, 0.21, 0.08}, {64, 64, 0.17, 0.059}};
-  int best = WIDE_NONE;
   double cost = keep * 0.38e-3 * ((M + 31) / 32) * ((N + 31) / 32) * (K / 64);
-  if (M < 128) return best;
+  if (M < 128) return WIDE_NONE;
+  bool large = false;
   for (int i = 0; i < 3; ++i) {
     const long tiles = (long)((M + tile[i].bm - 1) / tile[i].bm) * ((N + tile[i].bn - 1) / tile[i].bn);
     const double work = (double)((tiles + 255) / 256) * tile[i].work, c = (K / 32) * (work > tile[i].wait ? work : tile[i].wait);
-    if (c < cost) { best = i; cost = c; }
+    if (c < cost) large = true;
+  }
+  if (!large) return WIDE_NONE;
+  // Which one is measured beside each other: a step takes `wait` us alone on a CU and `work` for each of more tiles, of which a last round
+  // that is nearly empty costs little (workgroups start as others end); `base` us of a launch differ by tile.  Fitted to the three tiles
+  // of 107 products (150 ... 1999 rows, the projections of both designs, 768 to 2048 wide): the tile taken is 0.4 us above the quickest on average,
+  // by the estimates above 1.7.  us, by those / so: 1300 x 2048 x 6144 70.5 / 57.2, 500 x 6144 x 2048 35.7 / 28, 1999 x 3136 x 2048
+  // 56 / 48, 650 x 4224 x 1024 19.2 / 17.4.
+  static const struct { double base, wait, work; } each[] = {{0.7, 0.136, 0.145}, {0, 0.12, 0.079}, {-0.35, 0.057, 0.065}};
+  int best = 0;
+  for (int i = 0; i < 3; ++i) {
+    const long tiles = (long)((M + tile[i].bm - 1) / tile[i].bm) * ((N + tile[i].bn - 1) / tile[i].bn);
+    const double rounds = tiles <= 256 ? 0 : 0.9 * (tiles / 256.0) + 0.1 * ((tiles + 255) / 256), work = rounds * each[i].work;
+    const double c = each[i].base + (K / 32) * (work > each[i].wait ? work : each[i].wait);
+    if (i == 0 || c < cost) { best = i; cost = c; }
   }
   return best;
 }
