@@ -993,14 +993,17 @@ __global__ __launch_bounds__(256) void pf_stage_kv_kernel(const bf16_t* __restri
 // its L2.  Up to 256 tiles of 32 x 32 the K-splitting form runs with more waves and is quicker.
 // Fitted to 384 products (130 ... 2048 rows, widths 512, 768, 1024, bf16 and int8, weights of 22 layers in turn): on average 2 %
 // above the best form of each and 6 % below K-splitting alone; 6 products are more than 5 % above that, 19 % at most.
+// The bf16 forms once more, beside each other in whole prompts of 200 ... 2048 positions at widths 512, 768 and 1024: of 204 products the form
+// taken was 0.58 us above the quickest on average and is 0.1 now.  Prompts of width 768 with that and the norms' one trip, us: 1000 1510 -> 1448, 1500 1952 -> 1790, 1733 2049 -> 1918.
 // us, K-splitting / 128 x 128 / 64 x 128 / 64 x 64, bf16 at width 768: W1 and W3 at 577 rows 13.3 / 13.5 / 14.5 / 14.0, at 1000
 // 16.9 / 14.0 / 13.7 / 16.4, at 1733 25.3 / 19.3 / 22.7 / 25.6; W2 at 577 10.6 / 26.2 / 17.3 / 12.0, at 1733 29.4 / 26.3 / 17.6 / 17.8.
 static int pf_pick(int M, int N, int K, bool pair, bool i8) {
   static const struct { int bm, bn; double base[2], wait[2], work[2]; } tile[] = {  // of bf16 and int8 weights
-      {128, 128, {7.0, 7.3}, {0.275, 0.325}, {0.244, 0.274}},
-      {64, 128, {5.1, 5.3}, {0.198, 0.204}, {0.198, 0.181}},
-      {64, 64, {3.9, 4.8}, {0.143, 0.141}, {0.143, 0.112}}};
-  static const struct { double base, k256, tile, over; } split[2] = {{2.8, 0.66, 0.27e-3, 2.6e-6}, {4.3, 0.146, 0.262e-3, 0.44e-6}};
+      {128, 128, {6.37, 7.3}, {0.393, 0.325}, {0.199, 0.274}},
+      {64, 128, {5.63, 5.3}, {0.24, 0.204}, {0.171, 0.181}},
+      {64, 64, {3.25, 4.8}, {0.163, 0.141}, {0.136, 0.112}}};
+  static const double part[2] = {0.6, 0};  // of what a last round's missing tiles would take is saved: the others' workgroups end one by one
+  static const struct { double base, k256, tile, over; } split[2] = {{2.75, 0.635, 0.233e-3, 2.08e-6}, {4.3, 0.146, 0.262e-3, 0.44e-6}};
   const long rows = (M + 31) / 32;
   if (M < 128 || K < 256 || rows * ((N + 31) / 32) <= 256) return WIDE_NONE;
   if (pair) N *= 2;
@@ -1009,8 +1012,8 @@ static int pf_pick(int M, int N, int K, bool pair, bool i8) {
   const double over = 2.0 * M * K - 3e6;
   if ((rows & 1) && over > 0) us += split[i8].over * over;
   for (int i = 0; i < 3; ++i) {
-    const long rounds = ((long)((M + tile[i].bm - 1) / tile[i].bm) * ((N + tile[i].bn - 1) / tile[i].bn) + 255) / 256;
-    const double work = rounds * tile[i].work[i8], c = tile[i].base[i8] + (K / 32) * (work > tile[i].wait[i8] ? work : tile[i].wait[i8]);
+    const long tiles = (long)((M + tile[i].bm - 1) / tile[i].bm) * ((N + tile[i].bn - 1) / tile[i].bn), rounds = (tiles + 255) / 256;
+    const double work = (rounds == 1 ? 1.0 : part[i8] * tiles / 256 + (1 - part[i8]) * rounds) * tile[i].work[i8], c = tile[i].base[i8] + (K / 32) * (work > tile[i].wait[i8] ? work : tile[i].wait[i8]);
     if (c < us) { best = i; us = c; }
   }
   return best;
