@@ -752,7 +752,9 @@ struct PfDirectArgs {
 // from launch to launch; pf_order deals an eighth of a matrix's features to an XCD, and workgroup i is on XCD i % 8.  Measured, a whole prompt on
 // the device: 23 positions in bf16 705 -> 635 us, four of 23 2294 -> 2130; 16 of 16 in int8, half the bytes, 8.9 ms both.  No more than PF_AHEAD_BYTES:
 // the L2s of a card hold 32 MB, and what does not stay is read twice.
-#define PF_AHEAD 20  // workgroups per XCD
+// Workgroups per XCD, 20 / 32 / 48: an empty slot's 9, 23 and 60 positions in bf16 537 / 514 / 520, 604 / 569 / 562, 658 / 612 / 611 us, four turns behind
+// 700 7204 / 7128 / 7129, sixteen in int8 14.95 / 14.96 / 15.09 ms.
+#define PF_AHEAD 32
 #define PF_AHEAD_BYTES (24u << 20)
 __device__ __forceinline__ void pf_ahead(const PfDirectArgs& a) {
   const uint32_t plane = gridDim.x * gridDim.y, first = plane * a.nsp, i = blockIdx.x + gridDim.x * blockIdx.y + plane * blockIdx.z, x = i & 7u;
