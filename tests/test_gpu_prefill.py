@@ -177,6 +177,25 @@ def test_prefill_other_head_dims(heads, kv, rope_dim):
         assert rel_err(mine[:, 0, :pos], theirs[:, 0, :pos]) <= BF16_TOL
 
 
+@pytest.mark.parametrize("width,heads", [(512, 8), (576, 6), (1088, 17), (1600, 25), (2048, 32), (2112, 33)])
+def test_prefill_norms_of_every_width(width, heads):
+    """A norm keeps one to four pieces of eight columns per lane, whole and with lanes that have none, and reads rows of more than
+    2048 columns twice: rows in order (70 positions) and in operand blocks (5)."""
+    d = O.Dims(d_model=width, n_layers=1, n_heads=heads, n_kv_heads=heads, intermediate_size=128, n_quantizers=4, codebook_size=32, rq_d_model=64,
+               rq_n_layers=1, rq_n_heads=2, vocab_size=50, max_seqlen=96)
+    sd = O.synthetic_state_dict(d, **TINY_SD)
+    o = O.OracleModel(d, {k: O.rnd(v, BF) for k, v in sd.items()}, BF, n_slots=1, max_seqlen=96)
+    m = make_model(d, sd, BF, max_seqlen=96)
+    m.decoder.allocate_flash_kv_cache(1, m.device, BF)
+    assert m.decoder._prefill_available()
+    g = torch.Generator().manual_seed(9)
+    for T in (70, 5):
+        emb = O.rnd(torch.randn(T, width, generator=g) * 0.5, BF)
+        ref = o.prefill(emb, slot=0)
+        got = m.decoder.forward_flash(emb[None].to(BF).cuda(), None)[0]
+        assert rel_err(got, ref) <= BF16_TOL, (T, rel_err(got, ref))
+
+
 @pytest.mark.parametrize("int8", [False, True])
 def test_prefill_tiles_of_every_size(int8):
     """Block lengths that choose every form of the products (16- and 32-row tiles of 8 to 16 waves, 32 x 32 tiles, large
