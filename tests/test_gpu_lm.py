@@ -69,6 +69,22 @@ def test_few_rows_at_the_edges_of_steps(width, ff, dt):
             assert U.err(row.extend(toks, want), ref[want]) < U.TOL[dt], T
 
 
+@BOTH
+@pytest.mark.parametrize("scale", [-0.3, 0.0, 1e-32, 1e-3, 2.0])
+def test_latent_attention_of_any_scale(scale, dt):
+    """Maxima are of scores before their scale where that is positive; another sign turns the order round, none makes weights equal.  A
+    prompt's expanded form, the form of few rows, and steps behind both."""
+    cfg = U.config([U.attn(scale=scale), U.attn(scale=scale, heads=5)], width=96, ff=70)
+    sd = U.weights(cfg, 17)
+    eng = U.engine(cfg, sd, dt, max_seq=192)
+    toks = U.tokens(150, cfg["vocab"], 4)
+    ref = O.forward(cfg, sd, toks)
+    for first in (20, 130):
+        with eng.new_row() as row:
+            got = torch.cat([run_all(row, toks[:first]), run_all(row, toks[first:])])
+            assert U.err(got, ref) < U.TOL[dt], (scale, first, U.err(got, ref))
+
+
 def test_residual_stream_of_every_layer():
     cfg = U.mixed()
     sd = U.weights(cfg, 12)

@@ -12,10 +12,13 @@
 struct WeightExp {
   float hi, lo;  // scale log2 e
   float floor;   // of s - m
+  float mul;     // s and m come times this: 1, or a scale that is not positive (or of no ordinary size), which the maximum has to meet
 };
 static inline WeightExp weight_exp(double scale) {
-  const double c = scale * 1.4426950408889634074;
+  const bool plain = scale > 1e-30 && scale < 1e30;
+  const double c = (plain ? scale : 1.0) * 1.4426950408889634074;
   WeightExp w;
+  w.mul = plain ? 1.0f : (float)scale;
   w.hi = (float)c; w.lo = (float)(c - (double)w.hi); w.floor = (float)(-250.0 / c);
   return w;
 }

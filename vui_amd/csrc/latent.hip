@@ -255,6 +255,7 @@ __global__ __launch_bounds__(256, 2) void latent_attn_mfma_kernel(int2* where, c
     for (int u = 0; u < NT; ++u) {
       tl_f32x4 a = *reinterpret_cast<const tl_f32x4*>(&sco[u][lane * 4]);
       if (KT == 1) a += *reinterpret_cast<const tl_f32x4*>(&sco[(2 + u) & 3][lane * 4]);
+      if (p.we.mul != 1.0f) a *= p.we.mul;  // uniform
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const float v = j0 + 16 * u + 4 * kg + r < hi ? a[r] : -INFINITY;
@@ -454,6 +455,7 @@ __global__ __launch_bounds__(64 * LPF_WAVES, 2) void latent_prefill_kernel(const
       sc[t] = tl_f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int i = 0; i < 2 * DB + RB; ++i) sc[t] = Tl<bf16_t>::mma(kf[t][i], qf[i], sc[t]);
+      if (we.mul != 1.0f) sc[t] *= we.mul;  // uniform
     }
     if (k0 + 31 > pos0 + q0) {  // a key that some query of the tile does not see
 #pragma unroll
