@@ -349,8 +349,8 @@ def scaled(sd, power):
 @pytest.mark.parametrize("power", [-104, -60, -20, 20, 60, 120])
 def test_wide_products_of_any_magnitude(full, power):
     """Parts of an operand keep its exponent: scaled weights give the same audio from blocks of frames, bit by bit as long as the least
-    products are above fp32's least normal number (power-of-two factors pass through every sum of the parts).  Weights of 2^-110
-    keep their parts; the products' last bits are subnormal (the limit: other orders of the sums differ by 1e-5)."""
+    products are above fp32's least normal number (power-of-two factors pass through every sum of the three parts).  Weights of 2^-110
+    keep their three parts; the products' last bits are subnormal (the limit: other orders of the sums differ by 1e-5)."""
     d, sd, dec, fx = full
     codes = torch.randint(0, d.codebook_size, (1, d.n_codebooks, 35), generator=torch.Generator().manual_seed(9)).cuda()
     got, want = native(d, scaled(sd, power))(codes), dec(codes)
@@ -377,8 +377,8 @@ def test_wide_products_near_the_largest_number(full):
 
 @pytest.mark.parametrize("powers", [(0, 6, -6, 11, -2), (-12, 2, 3, 0, -1), (9,)])
 def test_wide_products_of_groups_of_different_size(full, powers):
-    """Columns are scaled per group of 32 channels, weights per matrix: the feed-forwards' inputs times a power of two per group and their weights
-    by the inverse give the same audio.  Both keep 22 bits down to 2^-17 of the largest, so the bound is that of other orders of the sums."""
+    """The feed-forwards' inputs times a power of two per group of 32 channels and their weights by the inverse give the same audio (the bound is
+    that of other orders of the sums)."""
     d, sd, dec, fx = full
     sd = dict(sd)
     for i in range(2):
@@ -406,6 +406,90 @@ def test_a_frame_that_is_not_finite_leaves_those_before_it(full, bad):
     got = native(d, sd)(codes)
     n = 17 * (want.shape[-1] // 35)
     assert err(got[..., :n], want[..., :n].cpu()) < 5e-5 and bool((got[..., n:] == -1).all())
+
+
+def by_channel(sd, powers):
+    """The same network with the columns of the wide products' inputs times powers of two, their weights by the inverse: both feed-forwards' inputs, and
+    the second upsampling block's output, which the first 7-tap convolution reads."""
+    sd = dict(sd)
+    n = sd["upsample.0.1.norm.weight"].shape[0]
+    f = 2.0 ** torch.tensor([powers[c % len(powers)] for c in range(n)], dtype=torch.float32)
+    for i in range(2):
+        p = f"upsample.{i}.1."
+        for k in ("norm.weight", "norm.bias"):
+            sd[p + k] = sd[p + k] * f
+        sd[p + "pwconv1.weight"] = sd[p + "pwconv1.weight"] / f
+    sd["upsample.1.0.conv.weight"] = sd["upsample.1.0.conv.weight"] * f[:, None]
+    sd["upsample.1.0.conv.bias"] = sd["upsample.1.0.conv.bias"] * f
+    sd["upsample.1.1.dwconv.conv.weight"] = sd["upsample.1.1.dwconv.conv.weight"] / f[:, None, None]
+    sd["upsample.1.1.gamma"] = sd["upsample.1.1.gamma"] * f
+    sd["decoder.0.conv.weight"] = sd["decoder.0.conv.weight"] / f[:, None]
+    return sd
+
+
+@pytest.mark.parametrize("powers", [(20, -20), (0, 0, 0, 30, 0, 0, -30)])
+def test_wide_products_of_channels_of_different_size(full, powers):
+    """Every operand keeps an exponent of its own: channels of any magnitude beside each other give the same bits."""
+    d, sd, dec, fx = full
+    codes = torch.randint(0, d.codebook_size, (1, d.n_codebooks, 35), generator=torch.Generator().manual_seed(9)).cuda()
+    assert torch.equal(native(d, by_channel(sd, powers))(codes), dec(codes))
+
+
+@pytest.mark.parametrize("power", [20, 30])
+def test_wide_products_of_rows_of_different_size(full, power):
+    """Rows of a matrix times powers of two, the inverse in the scale behind the product: the same bits."""
+    d, sd, dec, fx = full
+    other = dict(sd)
+    for i in range(2):
+        p = f"upsample.{i}.1."
+        f = 2.0 ** torch.tensor([(power, -power, 0, 0, 0)[m % 5] for m in range(sd[p + "gamma"].shape[0])], dtype=torch.float32)
+        other[p + "pwconv2.weight"] = sd[p + "pwconv2.weight"] * f[:, None]
+        other[p + "pwconv2.bias"] = sd[p + "pwconv2.bias"] * f
+        other[p + "gamma"] = sd[p + "gamma"] / f
+    codes = torch.randint(0, d.codebook_size, (1, d.n_codebooks, 35), generator=torch.Generator().manual_seed(9)).cuda()
+    assert torch.equal(native(d, other)(codes), dec(codes))
+
+
+@pytest.mark.parametrize("power, bound", [(30, 5e-5), (48, 5e-5), (62, 1e-2)])
+def test_wide_products_of_two_small_operands(full, power, bound):
+    """Inputs and weights of the second upsampling product times 2^-power each.  At 48 the least of the six products that count, 2^-16 of 2^-96, are
+    normal numbers: the bound is that of other orders of the sums.  At 62 products themselves are below 2^-126, where bits go from the parts' products on
+    (2^-8 of a product and less), while the sums, 2^-122, are normal numbers."""
+    d, sd, dec, fx = full
+    sd = dict(sd)
+    small, least, large = 2.0 ** -power, 2.0 ** (-2 * power), 2.0 ** (2 * power)
+    for k, f in (("upsample.0.0.conv.weight", small), ("upsample.0.0.conv.bias", small), ("upsample.0.1.dwconv.conv.weight", 1 / small),
+                 ("upsample.0.1.gamma", small), ("upsample.1.0.conv.weight", small), ("upsample.1.0.conv.bias", least),
+                 ("upsample.1.1.dwconv.conv.weight", large), ("upsample.1.1.gamma", least), ("decoder.0.conv.weight", large)):
+        sd[k] = sd[k] * f
+    codes = torch.randint(0, d.codebook_size, (1, d.n_codebooks, 35), generator=torch.Generator().manual_seed(9)).cuda()
+    assert err(native(d, sd)(codes), dec(codes).cpu()) < bound
+
+
+@pytest.mark.parametrize("power", [0, 4, 30, 40])
+def test_a_loud_frame_leaves_those_before_it(full, power):
+    """A code that alone reaches one channel of the trunk, which its norm takes times 2^power: not a bit of the frames before it changes."""
+    d, sd, dec, fx = full
+    sd = {k: v.clone() for k, v in sd.items()}
+    for k, v in sd.items():  # feature 0 of the first codebook goes through row 0 of each layer alone
+        if k.startswith("quantizer.") and k.endswith("embed"):
+            v[:, 0] = 0
+        elif k.endswith(("output_proj.weight", "pre_conv.conv.weight", "pre_transformer.input_proj.weight")) and "pre_transformer.output" not in k:
+            v[0], v[:, 0] = 0, 0
+        elif k in ("pre_conv.conv.bias", "pre_transformer.input_proj.bias") or k.endswith(("attn_scale", "mlp_scale")):
+            v[0] = 0
+    sd["quantizer.semantic.codebooks.0.embed"][5, 0] = 100
+    sd["quantizer.semantic.output_proj.weight"][0, 0] = 1
+    sd["pre_conv.conv.weight"][0, 0, -1] = 1
+    sd["pre_transformer.input_proj.weight"][0, 0] = 1
+    sd["pre_transformer.norm.weight"][0] = 2.0 ** power
+    dec = native(d, sd)
+    codes = torch.randint(6, d.codebook_size, (1, d.n_codebooks, 35), generator=torch.Generator().manual_seed(9)).cuda()
+    want = dec(codes)
+    codes[0, 0, 17] = 5
+    got = dec(codes)
+    n = 17 * (want.shape[-1] // 35)
+    assert torch.equal(got[..., :n], want[..., :n]) and not torch.equal(got[..., n:], want[..., n:])
 
 
 @pytest.mark.parametrize("d_model", [1024, 1312, 2048])

@@ -21,7 +21,7 @@
 //
 // Several frames at once (vui_codec_decode_clip: offline calls, the seeding of a stream; vui_codec_decode_block up to 32): the same
 // steps over frames x columns, on buffers that hold a whole pass with the histories in front; wide products run in
-// cv_wide_kernel.  93 frames: 42.7 ms one after the other, 3.3 in one pass (MI355X).
+// cv_wide_kernel.  93 frames: 42.7 ms one after the other, 5.6 ms in blocks of 32, 4.1 in one pass (MI355X).
 #include "common.h"
 #include "internal.h"
 #include "../../include/vui_codec.h"
@@ -56,7 +56,6 @@ enum { EPI_NONE = 0, EPI_GELU = 1, EPI_RES = 2, EPI_SCALE_RES = 3, EPI_SILU_PAIR
 
 struct CvGemm {
   const float* W;     // (taps, M, Cin)
-  const uint32_t* w_mag;  // cv_mag of its largest magnitude
   const float* bias;  // row m uses bias[m / bias_div]; may be null
   int M, Cin, taps, dil, T;
   int bias_div;
@@ -104,8 +103,9 @@ template <bool NT> __device__ __forceinline__ float4 cv_ld_w(const float* p) {
 #define CV_NW 8        // waves of a workgroup of cv_cols_kernel
 // sin(t)^2 for |t| below CV_SIN_FAR: t less a multiple of pi / 2 (in two parts, by fma), then s = r + r^3 P(r^2) on [-pi/4, pi/4], P of degree 2 fitted
 // here to the least relative error (2^-28); s^2, or 1 - s^2 of an odd multiple.  Half of sinf's instructions, root mean square error
-// 0.35 x 2^-24 (a correctly rounded sine, squared: 0.45).  93 frames,
-// with sinf / so: 7-tap convolutions of 96 channels 123 / 118 us, 1x1 76 / 71, of 192 135 / 132 and 63 / 60.
+// 0.35 x 2^-24 (a correctly rounded sine, squared: 0.45).  93 frames, us with sinf / so: 7-tap convolutions of 768 / 384 / 192 / 96 channels
+// 181 / 198 / 220 / 192 and 178 / 196 / 216 / 189, 1x1 59 / 47 / 63 / 74 and 57 / 45 / 58 / 70, the clip 4164 / 4092; six streamed frames 2736 / 2721.
+// Error of the audio against 64 bits 3.24e-6 / 3.23e-6.
 #define CV_SIN_FAR 25000.f
 __device__ __forceinline__ float cv_sin2(float t) {
   const float k = rintf(t * 0.63661975f);
@@ -358,73 +358,46 @@ __global__ __launch_bounds__(64 * CV_NW, 4) void cv_cols_kernel(CV_HOT, const Cv
 }
 
 // ---- the same product for many columns (several frames at once) ----
-// On the fp16 matrix instructions, which are 16 times the rate of the fp32 ones (157 TFLOP/s): every fp32 operand, times a power of two that
-// takes the largest to [2^14, 2^15), is the sum of two fp16 numbers (11 bits each, nearest, so that the rest halves once more: 23 bits), and
-// three of their four products are summed in fp32, small ones first.  The fourth is 2^-24 of a product, as the rounding of an fp32 one.
-// The power of two is one per matrix (cv_mag_kernel, once) and one per 32 channels of a tile's columns, found by the threads that fetch them; it
-// changes only where those are larger, or 2^3 smaller, than the ones before, and the sums with it.  23 bits hold down to 2^-17 of the
-// largest; below, a part's last bits are lost (2^-40 of the largest stay).  Columns that nothing reads (behind the last one) and values that are not
-// finite do not count; the latter make their own columns or rows NaN, infinite ones too.
-// Six products of three bf16 parts (24 bits) / this, us for 93 frames: 7-tap convolutions of 768 / 384 / 192 / 96 channels 195 / 211 / 240 /
-// 198 -> 105 / 114 / 130 / 121 (600-820 TFLOP/s of fp16 products; the products alone, without weights' and columns' way to LDS and
-// without the end of a tile, 82 us of the 114: 1120 TFLOP/s, what hipBLASLt reaches at 8192^3); 1x1 79 / 64 / 47 -> 70 / 59 / 44 (192 channels and less by memory,
-// 270 MB).  The clip 4110-4280 -> 3225-3275; its error against 64 bits, means over two seeds, 3.0-3.6e-6 -> 2.9-3.4e-6.
-// Tiles of BM x BN = 128 x 128 (or what divides M) of four waves through LDS, two planes of each operand, two buffers of both: a K step is one (tap,
-// 32-channel) unit with one barrier.  Fetched into registers are the weights of the next unit, split and stored while this one is
-// multiplied, and the columns of the next channel group: a group's taps follow each other, so that its columns, with the taps' halo, are
-// fetched, split and stored once for all of them.  A unit's operands are read from LDS ahead of its products: left to the compiler they came three at a
-// time into the same registers, each behind a wait (384 channels 118 -> 113 us).
-// Three workgroups per CU (one buffer of columns, 167 registers): 96 channels 117 -> 116, 384 112 -> 130 us.  Sixteen or 24 rows at a time at the end of
-// a tile: the same.
+// On the bf16 matrix instructions, which are 16 times the rate of the fp32 ones (157 TFLOP/s): every fp32 operand is the sum of three
+// bf16 numbers (8 bits each, nearest, so that the rest halves once more), and of their nine products the six that
+// reach 2^-24 of the value are summed in fp32, small ones first (G. Henry, P. T. P. Tang, A. Heinecke, "Leveraging the bfloat16
+// Artificial Intelligence Datatype for Higher-Precision Computations", ARITH 2019).  What is left out is 2^-26 of a product; the sums have
+// fewer roundings than with v_mfma_f32_32x32x2_f32 (sixteen products per step instead of two).
+// The sum is exact for every finite value from 2^-110 up.  Of a smaller one, what lies below bf16's least subnormal, 2^-133, is lost
+// (weights of 2^-118: error of the product 1.4e-5, 2^-122: 2e-4; with fp32 instructions 2e-6).  A value that is not finite makes its
+// columns or rows NaN, an infinite one too.
+// 32 frames: 7-tap convolutions of 768 / 384 / 192 / 96 channels 86 / 105 / 121 / 91 us -> 55 / 63 / 83 / 62 (920 TFLOP/s
+// of bf16 products in the first; hipBLASLt reaches 1125 at 8192^3), 1x1 19 / 30 / 32 / 33 -> 16 / 29 / 26 / 29 (3-4 % more with the clamp
+// of cv_split2); error of 93 frames against 64 bits 4.1e-6 -> 3.9e-6.
+// Tiles of BM x BN = 128 x 128 (or what divides M) of four waves through LDS, three planes of each operand: a K step is one (tap,
+// 32-channel) unit, fetched into registers while the one before it is multiplied, split on the way to LDS.  A group's taps follow each
+// other, so that its columns, with the taps' halo, are fetched, split and stored once for all of them (per tap they were two thirds of
+// the vector instructions and a quarter of what LDS moves, beside matrix instructions that it nearly holds up); where two workgroups of a
+// CU still fit, weights have a second buffer and a unit one barrier.  93 frames, 7-tap convolutions of 768 / 384 / 192 / 96 channels
+// 214 / 247 / 275 / 227 -> 195 / 211 / 240 / 198 us, the clip 4681 -> 4259, 250 frames 10883 -> 9726.  Eight waves with two buffers of both
+// and one to three units in flight: 75 us of the 384-channel convolution of 32 frames when this form took 63.
+// Two fp16 parts of each operand, scaled by a power of two per matrix and per 32 channels of a tile, and three products took the clip 4110 -> 3225 us
+// and the audio was no further off (3.1e-6).  But what is small beside something large in the same block lost its bits: a frame 2^30 larger than those
+// before it put 2e-3 of error into their audio, rows 2^30 apart, or channels 2^40 apart and their weights the inverse, likewise.
 // Where the tiles are fewer than the CUs their units are split over workgroups, and cv_finish_kernel adds the parts.
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
-typedef _Float16 cv_f16x8 __attribute__((ext_vector_type(8)));
+typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 cv_bf16x8;
 
-#define CVW_RUN 4     // units of 32 channels whose products are one chain of sums, at least (whole groups)
-#define CVW_SLACK 3   // columns up to 2^3 times smaller keep the scale of those before
+#define CVW_RUN 4
 #define CVW_HALO 56  // columns that the taps reach beyond a tile: 6 x 9
 // In LDS a row's (or column's) 32 channels of a plane are four pieces of 16 bytes; a piece's place turns with the row, so that 16-byte
 // reads of eight rows fall on different banks.
 __device__ __forceinline__ int cv_at(int row, int piece) { return row * 32 + 8 * (piece ^ (row >> 2 & 3)); }
 
-// two fp32 values -> their two fp16 parts, packed
-__device__ __forceinline__ void cv_split2(float a, float b, uint32_t& hi, uint32_t& lo) {
-  typedef float f2_t __attribute__((ext_vector_type(2)));
-  typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
-  const h2_t h = __builtin_convertvector(f2_t{a, b}, h2_t);
-  const h2_t l = __builtin_convertvector(f2_t{a - (float)h.x, b - (float)h.y}, h2_t);
-  hi = __builtin_bit_cast(uint32_t, h);
-  lo = __builtin_bit_cast(uint32_t, l);
-}
-// Magnitudes as numbers whose maximum is the largest finite one's: what is not finite comes below all that is.  The exponent is 24 bits up, one larger.
-__device__ __forceinline__ uint32_t cv_mag(float v) { return (__float_as_uint(v) << 1) + 0x01000000u; }
-#define CV_NO_MAG 0x01000000u  // of zero
-// The power of two that takes values up to that magnitude to below 2^15 (from 2^-113 up to 2^14 and more), as its exponent
-__device__ __forceinline__ int cv_scale_of(uint32_t mag) { return 141 - max((int)(mag >> 24) - 1, 14); }
-__device__ __forceinline__ float cv_exp2i(int n) { return n < -126 ? (n < -149 ? 0.f : __uint_as_float(1u << (n + 149))) : __uint_as_float((uint32_t)(min(n, 127) + 127) << 23); }
-__device__ __forceinline__ uint32_t cv_wave_max(uint32_t v) {
-  v = max(v, (uint32_t)dpp_i<DPP_QUAD_XOR1>((int)v));
-  v = max(v, (uint32_t)dpp_i<DPP_QUAD_XOR2>((int)v));
-  v = max(v, (uint32_t)dpp_i<DPP_ROW_HALF_MIRROR>((int)v));
-  v = max(v, (uint32_t)dpp_i<DPP_ROW_MIRROR>((int)v));
-  return max(max((uint32_t)__builtin_amdgcn_readlane((int)v, 0), (uint32_t)__builtin_amdgcn_readlane((int)v, 16)),
-             max((uint32_t)__builtin_amdgcn_readlane((int)v, 32), (uint32_t)__builtin_amdgcn_readlane((int)v, 48)));
-}
-// the largest finite magnitude of a matrix (n a multiple of 4), into a word that starts at zero
-__global__ __launch_bounds__(256) void cv_mag_kernel(const float* w, size_t n, uint32_t* out) {
-  __shared__ uint32_t part[4];
-  uint32_t m = 0;
-  for (size_t i = ((size_t)blockIdx.x * 1024 + threadIdx.x) * 4; i < n; i += (size_t)gridDim.x * 4096) {
-    float4 v[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) v[k] = *reinterpret_cast<const float4*>(w + min(i + 1024 * k, n - 4));
-#pragma unroll
-    for (int k = 0; k < 4; ++k) m = max(m, max(max(cv_mag(v[k].x), cv_mag(v[k].y)), max(cv_mag(v[k].z), cv_mag(v[k].w))));
-  }
-  m = cv_wave_max(m);
-  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
-  __syncthreads();
-  if (threadIdx.x == 0) atomicMax(out, max(max(part[0], part[1]), max(part[2], part[3])));
+// two fp32 values -> their three bf16 parts, packed.  The first part of a value above bf16's largest (3.39e38) is that largest: to the
+// nearest it would be infinity, and the column NaN.  Two instructions per pair: the products take 3-4 % more, 93 frames 5960 -> 6050 us.
+// (A tile computed once more with the clamp where a sum is not finite needs 40 registers more: 6070 us.)
+__device__ __forceinline__ void cv_split2(float a, float b, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
+  const float top = __uint_as_float(0x7f7f0000u);
+  hi = f2bf2(__builtin_amdgcn_fmed3f(a, -top, top), __builtin_amdgcn_fmed3f(b, -top, top));
+  a -= bf_lo(hi); b -= bf_hi(hi);
+  mid = f2bf2(a, b);
+  lo = f2bf2(a - bf_lo(mid), b - bf_hi(mid));
 }
 
 // bias, activation or residual, and the outputs of one column of eight rows m, m + step, ... (uniform over a wave)
@@ -489,13 +462,12 @@ __global__ __launch_bounds__(256, 2) void cv_wide_kernel(const CvGemm p) {
   constexpr int NA = (BM * 8 + NT - 1) / NT, NB = (CW * 4 + NT - 1) / NT;  // 16-byte loads per thread and unit, pieces of 8 channels and group
   static_assert(WM * WN == 4 && NT % BN == 0, "four waves, whole columns per thread");
   constexpr int PA = BM * 64, PB = CW * 64;  // bytes of one plane of the weights, of the columns
-  constexpr int OPS = 4 * PA + 4 * PB;
-  static_assert(2 * (OPS + 32) <= 160 * 1024, "two workgroups share a CU");
-  __shared__ __align__(16) char raw[OPS > BM * BS * 4 ? OPS : BM * BS * 4];  // the operands (weights twice), then the sums
-  __shared__ uint32_t mags[2][4];
+  constexpr bool TWO = 2 * (6 * PA + 3 * PB) <= 160 * 1024;  // a second buffer for weights: two workgroups still share a CU
+  constexpr int OPS = (TWO ? 6 : 3) * PA + 3 * PB;
+  __shared__ __align__(16) char raw[OPS > BM * BS * 4 ? OPS : BM * BS * 4];  // the operands, then the sums
   float* const lds = reinterpret_cast<float*>(raw);
-  auto la = [&](int buf, int plane, int row, int piece) { return reinterpret_cast<bf16_t*>(raw + 4 * PB + (buf * 2 + plane) * PA) + cv_at(row, piece); };
-  auto lb = [&](int buf, int plane, int col, int piece) { return reinterpret_cast<bf16_t*>(raw + (buf * 2 + plane) * PB) + cv_at(col, piece); };
+  auto la = [&](int buf, int plane, int row, int piece) { return reinterpret_cast<bf16_t*>(raw + 3 * PB + (buf * 3 + plane) * PA) + cv_at(row, piece); };
+  auto lb = [&](int plane, int col, int piece) { return reinterpret_cast<bf16_t*>(raw + plane * PB) + cv_at(col, piece); };
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int l32 = lane & 31, h = lane >> 5, wm = wave % WM, wn = wave / WM;
   // Workgroups go round the eight XCDs, whose L2s are their own: each gets a contiguous range of the tiles, columns slowest, so that
@@ -509,7 +481,7 @@ __global__ __launch_bounds__(256, 2) void cv_wide_kernel(const CvGemm p) {
   const int ub = (int)((int64_t)Uall * z / p.splits), ue = (int)((int64_t)Uall * (z + 1) / p.splits);
   const int f = *p.ctr - p.nf;
 
-  // acc: the products of the last units, scaled; sum: those before.  One chain over all units (168 of them in block 1) would
+  // acc: the products of CVW_RUN units; sum: those before.  One chain over all units (168 of them in block 1) would
   // round each step against the full sum: 1.4 times the error against 64 bits of the audio.
   floatx16 acc[MI][NI], sum[MI][NI];
   const floatx16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -531,8 +503,6 @@ __global__ __launch_bounds__(256, 2) void cv_wide_kernel(const CvGemm p) {
     xoff[i] = (uint32_t)(8 * k * p.in.rs + c);
   }
   const uint32_t woff = (tid >> 3) * p.Cin + (tid & 7) * 4;
-  const int w_scale = cv_scale_of(*p.w_mag), live = p.T - t0 + W - BN;  // columns from `live` on are nobody's
-  const float w_mul = cv_exp2i(w_scale);
   auto fetch_w = [&](int tap, int grp) {
     const float* wp = p.W + ((size_t)tap * p.M + m0) * p.Cin + grp * 32;  // uniform, with offsets of the thread's own
 #pragma unroll
@@ -553,127 +523,76 @@ __global__ __launch_bounds__(256, 2) void cv_wide_kernel(const CvGemm p) {
 #pragma unroll
     for (int i = 0; i < NA; ++i)
       if ((i + 1) * (NT / 8) <= BM || (tid >> 3) + i * (NT / 8) < BM) {
-        uint2 q[2];
-        cv_split2(ra[i][0] * w_mul, ra[i][1] * w_mul, q[0].x, q[1].x);
-        cv_split2(ra[i][2] * w_mul, ra[i][3] * w_mul, q[0].y, q[1].y);
+        uint2 q[3];
+        cv_split2(ra[i][0], ra[i][1], q[0].x, q[1].x, q[2].x);
+        cv_split2(ra[i][2], ra[i][3], q[0].y, q[1].y, q[2].y);
 #pragma unroll
-        for (int k = 0; k < 2; ++k) *reinterpret_cast<uint2*>(la(buf, k, (tid >> 3) + (NT / 8) * i, (tid & 7) >> 1) + (tid & 1) * 4) = q[k];
+        for (int k = 0; k < 3; ++k) *reinterpret_cast<uint2*>(la(buf, k, (tid >> 3) + (NT / 8) * i, (tid & 7) >> 1) + (tid & 1) * 4) = q[k];
       }
   };
-  auto show_mag = [&](int grp) {  // of the fetched columns, by waves
-    uint32_t m = 0;
-#pragma unroll
-    for (int i = 0; i < NB; ++i)
-      if (((i + 1) * NT <= 4 * BN || tid + i * NT < 4 * W) && pc[i] >> 2 < live) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) m = max(m, cv_mag(rb[i][e]));
-      }
-    m = cv_wave_max(m);
-    if (lane == 0) mags[grp & 1][wave] = m;
-  };
-  auto stage_x = [&](int buf, float mul) {
+  auto stage_x = [&]() {
 #pragma unroll
     for (int i = 0; i < NB; ++i)
       if ((i + 1) * NT <= 4 * BN || tid + i * NT < 4 * W) {
-        uint4 q[2];
-        cv_split2(rb[i][0] * mul, rb[i][1] * mul, q[0].x, q[1].x);
-        cv_split2(rb[i][2] * mul, rb[i][3] * mul, q[0].y, q[1].y);
-        cv_split2(rb[i][4] * mul, rb[i][5] * mul, q[0].z, q[1].z);
-        cv_split2(rb[i][6] * mul, rb[i][7] * mul, q[0].w, q[1].w);
+        uint4 q[3];
+        cv_split2(rb[i][0], rb[i][1], q[0].x, q[1].x, q[2].x);
+        cv_split2(rb[i][2], rb[i][3], q[0].y, q[1].y, q[2].y);
+        cv_split2(rb[i][4], rb[i][5], q[0].z, q[1].z, q[2].z);
+        cv_split2(rb[i][6], rb[i][7], q[0].w, q[1].w, q[2].w);
 #pragma unroll
-        for (int k = 0; k < 2; ++k) *reinterpret_cast<uint4*>(lb(buf, k, pc[i] >> 2, pc[i] & 3)) = q[k];
+        for (int k = 0; k < 3; ++k) *reinterpret_cast<uint4*>(lb(k, pc[i] >> 2, pc[i] & 3)) = q[k];
       }
   };
-  auto frag = [](const bf16_t* q) { return __builtin_bit_cast(cv_f16x8, *reinterpret_cast<const uint4*>(q)); };
-  int x_scale = 127 + CVW_SLACK, run = 0;  // of the columns that are multiplied (whatever comes is less); units in acc
-  auto flush = [&]() {
-    const float mul = cv_exp2i(-x_scale - w_scale);
-#pragma unroll
-    for (int i = 0; i < MI; ++i)
-#pragma unroll
-      for (int n = 0; n < NI; ++n)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) { sum[i][n][r] = fmaf(acc[i][n][r], mul, sum[i][n][r]); acc[i][n][r] = 0.f; }
-    run = 0;
-  };
-  // the scale of the columns shown last, behind a barrier
-  auto next_scale = [&](int grp) {
-    const uint32_t* g = mags[grp & 1];
-    const uint32_t m = __builtin_amdgcn_readfirstlane(max(max(g[0], g[1]), max(g[2], g[3])));
-    const int sc = cv_scale_of(m);
-    return m > CV_NO_MAG && (sc < x_scale || sc > x_scale + CVW_SLACK) ? sc : x_scale;
-  };
-  // A group's taps follow one another.  In flight: the weights of the next unit but one, the columns of the next group but one.
-  int grp = ub / p.taps, tap = ub - grp * p.taps, wt = tap, wg = grp;  // wt, wg: of the weights to fetch next
-  const int groups = ub < ue ? (ue - 1) / p.taps + 1 : grp;  // behind the last
-  int wu = ub;
-  auto next_w = [&]() {
-    fetch_w(wt, wg);
-    if (++wu < ue && ++wt == p.taps) { wt = 0; ++wg; }
-  };
+  auto frag = [](const bf16_t* q) { return __builtin_bit_cast(cv_bf16x8, *reinterpret_cast<const uint4*>(q)); };
+  int grp = ub / p.taps, tap = ub - grp * p.taps;  // a group's taps one after the other
   if (ub < ue) {
-    next_w();
+    fetch_w(tap, grp);
     fetch_x(grp);
-    show_mag(grp);
     stage_w(0);
-    __syncthreads();
-    x_scale = next_scale(grp);
-    stage_x(0, cv_exp2i(x_scale));
-    next_w();
-    if (grp + 1 < groups) {
-      fetch_x(grp + 1);
-      if (tap + 1 == p.taps) show_mag(grp + 1);
-    }
+    stage_x();
   }
   __syncthreads();
-  for (int u = ub, xb = 0; u < ue; ++u) {
-    const int col = tap * p.dil, buf = (u - ub) & 1;
-    const bool turn = tap + 1 == p.taps && grp + 1 < groups;  // uniform; the next unit is another group's
-    int scale = x_scale;
-    // the unit's operands, in the order of their use (one block of registers each: waits are for the first only)
-    cv_f16x8 a[2][2][MI], x[2][2][NI];
+  for (int u = ub; u < ue; ++u) {
+    const int col = tap * p.dil, buf = TWO ? (u - ub) & 1 : 0;
+    const bool more = u + 1 < ue, turn = tap + 1 == p.taps;  // uniform; turn: the next unit is another group's
+    if (turn) { tap = 0; ++grp; } else ++tap;
+    if (more) {
+      fetch_w(tap, grp);
+      if (turn) fetch_x(grp);
+    }
 #pragma unroll
     for (int j = 0; j < 2; ++j) {  // 16 channels: a lane holds eight of its row or column
+      cv_bf16x8 a[3][MI], x[3][NI];
 #pragma unroll
-      for (int k = 0; k < 2; ++k) {
+      for (int k = 0; k < 3; ++k) {
 #pragma unroll
-        for (int n = 0; n < NI; ++n) x[j][k][n] = frag(lb(xb, k, (wn * NI + n) * 32 + l32 + col, 2 * j + h));
+        for (int i = 0; i < MI; ++i) a[k][i] = frag(la(buf, k, (wm * MI + i) * 32 + l32, 2 * j + h));
 #pragma unroll
-        for (int i = 0; i < MI; ++i) a[j][1 - k][i] = frag(la(buf, 1 - k, (wm * MI + i) * 32 + l32, 2 * j + h));
+        for (int n = 0; n < NI; ++n) x[k][n] = frag(lb(k, (wn * NI + n) * 32 + l32 + col, 2 * j + h));
       }
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    // behind the last units the same weights once more
-    stage_w(buf ^ 1);
-    next_w();
-    // {part of the weight, part of the input}
-    constexpr int PAIR[3][2] = {{1, 0}, {0, 1}, {0, 0}};
+      // {part of the weight, part of the input}
+      constexpr int PAIR[6][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int c = 0; c < 3; ++c)
+      for (int c = 0; c < 6; ++c)
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
           for (int n = 0; n < NI; ++n)
-            acc[i][n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[j][PAIR[c][0]][i], x[j][PAIR[c][1]][n], acc[i][n], 0, 0, 0);
+            acc[i][n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[PAIR[c][0]][i], x[PAIR[c][1]][n], acc[i][n], 0, 0, 0);
+    }
+    if ((u - ub) % CVW_RUN == CVW_RUN - 1 || u + 1 == ue) {
 #pragma unroll
-    for (int i = 0; i < 6 * MI * NI; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x2, (NA * 14 + 6 * MI * NI - 1) / (6 * MI * NI), 0);
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int n = 0; n < NI; ++n) { sum[i][n] += acc[i][n]; acc[i][n] = zero; }
     }
-    __builtin_amdgcn_sched_barrier(0);
-    if (turn) {
-      scale = next_scale(grp + 1);
-      stage_x(xb ^ 1, cv_exp2i(scale));
-      if (grp + 2 < groups) fetch_x(grp + 2);
+    if (TWO && more) stage_w(buf ^ 1);
+    if (!TWO || turn || !more) __syncthreads();
+    if (more) {
+      if (!TWO) stage_w(0);
+      if (turn) stage_x();
+      __syncthreads();
     }
-    ++run;
-    if (u + 1 == ue || scale != x_scale || (turn && run >= CVW_RUN)) flush();
-    x_scale = scale;
-    if (turn) { tap = 0; ++grp; xb ^= 1; } else ++tap;
-    if (tap + 1 == p.taps && grp + 1 < groups) show_mag(grp + 1);  // ahead of the group's last unit
-    __syncthreads();
   }
 
   if (p.splits > 1) {  // cv_finish_kernel adds the parts
@@ -1643,10 +1562,10 @@ static void grid_for(size_t n, dim3& g) { size_t b = (n + 255) / 256; g = dim3((
 struct CvScratch { size_t part, cnt; };  // floats of partial sums, arrival counters
 // tiles of cv_wide_kernel, and what one unit of a tile costs against 128 x 128
 struct WideTile { int bm, bn; float unit; };
-#define CVW_PAIR 1.55  // us of a unit of 128 x 128 for two workgroups of a CU, and for one
-#define CVW_ALONE 1.02
+#define CVW_PAIR 2.6   // us of a unit of 128 x 128 for two workgroups of a CU, and for one
+#define CVW_ALONE 1.6
 #define CVW_PARTS (6u << 20)  // floats of the parts of a split product, which the workspace holds
-static const WideTile kWide[] = {{128, 128, 1.0f}, {96, 128, 0.81f}, {64, 128, 0.62f}, {128, 64, 0.7f}, {32, 128, 0.41f}};
+static const WideTile kWide[] = {{128, 128, 1.0f}, {96, 128, 0.79f}, {64, 128, 0.63f}, {128, 64, 0.63f}, {32, 128, 0.55f}};
 
 static int cv_lds(const CvGemm& g) { return (CV_NW * g.tt * 256 + g.xcols * (g.chunk * 32 + 4)) * 4; }
 // The fields of cv_cols_kernel for a tile shared by up to `splits` workgroups: chunks whose units fit the waves' registers and whose
@@ -1742,27 +1661,19 @@ static int cv_build(vui_codec* cc, const vui_codec_config* c, const void* const*
   size_t part_floats = 0, cnt_ints = 0;
   float* part = ar.take(part_cap);
   int* cnt = (int*)ar.take(cnt_cap);
-  const int most_gemms = 8 + 4 * c->n_layers + 3 * c->n_up + 7 * c->n_rates;
-  uint32_t* mags = (uint32_t*)ar.take(most_gemms);  // of the matrices' largest entries
-  int n_mags = 0;
-  if (real) hipLaunchKernelGGL(cv_fill_kernel, dim3(1), dim3(256), 0, st, (float*)mags, (size_t)most_gemms, 0.0f);
   auto gemm = [&](const float* W, const float* bias, int M, int Cin, int taps, int dil, int T, const Ring& in) -> CvGemm {
     CvGemm g;
     memset(&g, 0, sizeof(g));
     g.W = W; g.bias = bias; g.M = M; g.Cin = Cin; g.taps = taps; g.dil = dil; g.T = T; g.bias_div = 1;
     g.in = in; g.in_mode = IN_PLAIN; g.eps = 1e-6f; g.epi = EPI_NONE;
     g.res = no_ring(); g.out_raw = no_ring(); g.out_act = no_ring(); g.ctr = ctr; g.nf = 1;
-    g.part = part; g.cnt = cnt; g.w_mag = mags + n_mags++;
+    g.part = part; g.cnt = cnt;
     for (int n = real || part_need ? block_frames(*c) : 1; n >= 1; --n) {  // the frame's own plan is made last and stays
       g.T = n * T;
       g.nf = n;
       const CvScratch need = cv_plan(g);
       if (need.part > part_floats) part_floats = need.part;
       if (need.cnt > cnt_ints) cnt_ints = need.cnt;
-    }
-    if (real) {
-      const size_t n = (size_t)taps * M * Cin;
-      hipLaunchKernelGGL(cv_mag_kernel, dim3((unsigned)std::min<size_t>((n + 4095) / 4096, 1024)), dim3(256), 0, st, W, n, mags + n_mags - 1);
     }
     return g;
   };
