@@ -492,6 +492,25 @@ def test_a_loud_frame_leaves_those_before_it(full, power):
     assert torch.equal(got[..., :n], want[..., :n]) and not torch.equal(got[..., n:], want[..., n:])
 
 
+def test_snake_activations_of_large_arguments(small):
+    """Arguments on both sides of where the activation's own sine ends, up to where a float has no fraction left: channels that a bias alone makes, each with
+    a scale that shows its sine; a clip and a stream against the oracle."""
+    d, _, _ = small
+    sd = {k: v.clone() for k, v in O.synthetic_codec_state_dict(d, seed=4).items()}
+    t = torch.tensor([24999.0, 24999.998, 25000.0, 25000.002, -24999.5, -25001.5, 3.1e4, -4.7e5, 2.6e7, 5.3e7, -1.0e8, 7.0])
+    n, block = len(t), "decoder.1.block."
+    sd["decoder.0.conv.weight"][:n], sd["decoder.0.conv.bias"][:n] = 0, t
+    sd[block + "0.alpha"][:n], sd[block + "0.beta"][:n] = 0, -t.abs().log()
+    sd[block + "1.conv.weight"][:n] /= t.abs()[:, None, None]
+    ora, dec = O.CodecDecoderOracle(d, sd), native(d, sd)
+    codes = torch.randint(0, d.codebook_size, (1, d.n_codebooks, 33), generator=torch.Generator().manual_seed(3))
+    ref = ora.forward(codes)
+    assert err(dec(codes.cuda()), ref) < TOL
+    with dec.streaming(1):
+        one = torch.cat([dec(codes[:, :, i:i + 1].cuda()).clone() for i in range(33)], dim=-1)
+    assert err(one, ref) < TOL
+
+
 @pytest.mark.parametrize("d_model", [1024, 1312, 2048])
 def test_blocks_of_wide_pre_transformers(d_model):
     """Widths whose normed products take eight waves (25-48 units of 32 channels from 17 frames on, 33-64 below) or split
