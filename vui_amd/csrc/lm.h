@@ -32,7 +32,7 @@ enum {
   LM_IN_GRU_SEQ,    // ... positions of one sequence: update pairs for the scan
   LM_OUT,           // x += W y; operand copy and sums of squares of the new x
   LM_LOGITS,        // fp32 logits of chosen rows
-  LM_EXPAND,        // keys of one head per blockIdx.z from cached latents, then values, transposed (bf16)
+  LM_EXPAND,        // keys of every head from cached latents, then values, transposed (bf16)
   // sandwich layers (rows arrive normed)
   LM_HEAD,          // LM_LOGITS without a row scale
   LM_PROJ,          // W x + bias in the context's dtype, row-major
@@ -46,7 +46,7 @@ struct LmGemm {
   const void* X;  // (M x K) tiled
   const void* W;  // (N x K) tiled
   int M, N, K;    // N a multiple of 16, K of 64
-  size_t wz;      // elements between the weights of consecutive blockIdx.z
+  size_t wz;      // elements between the weights of an expert, of a head (LM_EXPAND), and the next one's
   const int32_t* rowmap;  // row of X behind output row m, or nullptr
   int x_rows;             // rows of X (bound of rowmap)
   // row scale norm[0] / sqrt(sum(ssq[m]) / width + eps); ssq: (rows, np), pairs with few rows (LM_PAIRS)
@@ -104,7 +104,7 @@ struct LmGemm {
   int band;
   uint32_t inv_tiles, inv_band, inv_last;
 };
-int launch_lm_gemm(int dtype, int epi, const LmGemm& g, int nz, hipStream_t st);
+int launch_lm_gemm(int dtype, int epi, const LmGemm& g, hipStream_t st);
 int launch_lm_embed(int dtype, const LmRows& where, const int64_t* tokens, const void* table, float* x, void* xt, float* ssq, int rows, int width,
                     int w64, int np, int vocab, hipStream_t st);
 

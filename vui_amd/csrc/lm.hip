@@ -222,7 +222,7 @@ static int lm_attention(vui_lm_ctx* x, int l, int M, const LmRows& rows, LmGemm&
   g.rot_pairs = L.rot_pairs; g.rope = L.rope;
   g.qu = x->qu; g.qr = x->qr; g.qu_z = (size_t)x->R16 * d.dim64; g.qr_z = (size_t)x->R16 * d.rot32;
   g.craw = x->craw; g.gate = x->gate; g.kr_cache = L.kr_cache;
-  int rc = launch_lm_gemm(c.dtype, LM_IN_ATTN, g, 1, st);
+  int rc = launch_lm_gemm(c.dtype, LM_IN_ATTN, g, st);
   if (rc) return rc;
 
   LatentArgs a;
@@ -242,7 +242,7 @@ static int lm_attention(vui_lm_ctx* x, int l, int M, const LmRows& rows, LmGemm&
     k.heads = L.heads;
     k.W = L.w_uk; k.N = d.dim64; k.wz = (size_t)d.dim64 * d.rank64; k.kv_out = x->kx; k.kv_z = (size_t)d.s64 * d.dim64;
     k.w_v = L.w_uv; k.n_v = d.vdim16; k.wz_v = (size_t)d.vdim16 * d.rank64; k.v_out = x->vx; k.v_z = (size_t)d.s64 * d.vdim16;
-    if ((rc = launch_lm_gemm(c.dtype, LM_EXPAND, k, 1, st))) return rc;
+    if ((rc = launch_lm_gemm(c.dtype, LM_EXPAND, k, st))) return rc;
     a.kx = x->kx; a.vx = x->vx; a.kx_z = (size_t)d.s64 * d.dim64; a.vx_z = (size_t)d.s64 * d.vdim16;
     return launch_latent_prefill_attn(a, st);
   }
@@ -257,7 +257,7 @@ static int lm_recurrence(vui_lm_ctx* x, int l, int M, const LmRows& rows, LmGemm
   const vui_lm_layer& L = x->layers[l];
   const vui_lm_dims& d = x->dims[l];
   g.bz = L.bias_z; g.bx = L.bias_x; g.state = L.state; g.upd = x->upd; g.sg = x->sg;
-  int rc = launch_lm_gemm(x->c.dtype, rows.seq ? LM_IN_GRU_SEQ : LM_IN_GRU_STEP, g, 1, st);
+  int rc = launch_lm_gemm(x->c.dtype, rows.seq ? LM_IN_GRU_SEQ : LM_IN_GRU_STEP, g, st);
   if (rc || !rows.seq) return rc;
   ScanArgs s;
   memset(&s, 0, sizeof(s));
@@ -287,7 +287,7 @@ static int lm_layers(vui_lm_ctx* x, const int64_t* tokens, int M, const LmRows& 
     o.X = x->act; o.W = L.w_out; o.M = M; o.N = d.out_rows; o.K = d.out_k; o.d = d; o.rows = rows;
     o.x = x->x; o.xt = x->xt; o.ssq_out = x->ssq; o.np = np; o.width = c.width;
     o.layer_out = x->layers_out ? x->layers_out + (size_t)l * M * c.width : nullptr;
-    if ((rc = launch_lm_gemm(c.dtype, LM_OUT, o, 1, st))) return rc;
+    if ((rc = launch_lm_gemm(c.dtype, LM_OUT, o, st))) return rc;
   }
   return VUI_OK;
 }
@@ -335,7 +335,7 @@ int vui_lm_decode(vui_lm_ctx* x, const int64_t* tokens, const int32_t* slot_idx,
   if (rc) return rc;
   LmGemm g = lm_logits(x, r, B, B, nullptr, logits_out);
   g.upd_lens = seq_lens; g.upd_inc = seq_inc; g.upd_rows = B;
-  return launch_lm_gemm(x->c.dtype, x->c.norm_groups > 0 ? LM_HEAD : LM_LOGITS, g, 1, st);
+  return launch_lm_gemm(x->c.dtype, x->c.norm_groups > 0 ? LM_HEAD : LM_LOGITS, g, st);
 }
 
 int vui_lm_prefill(vui_lm_ctx* x, const int64_t* tokens, int T, int slot, int pos0, int32_t* seq_lens, const int32_t* want,
@@ -351,7 +351,7 @@ int vui_lm_prefill(vui_lm_ctx* x, const int64_t* tokens, int T, int slot, int po
   r.seq = 1; r.slot = slot; r.pos0 = pos0; r.S = x->c.max_seqlen; r.n_slots = x->c.n_slots;
   int rc = lm_layers(x, tokens, T, r, st);
   if (rc) return rc;
-  if (n_want > 0 && (rc = launch_lm_gemm(x->c.dtype, x->c.norm_groups > 0 ? LM_HEAD : LM_LOGITS, lm_logits(x, r, n_want, T, want, logits_out), 1, st))) return rc;
+  if (n_want > 0 && (rc = launch_lm_gemm(x->c.dtype, x->c.norm_groups > 0 ? LM_HEAD : LM_LOGITS, lm_logits(x, r, n_want, T, want, logits_out), st))) return rc;
   hipLaunchKernelGGL(lm_set_len_kernel, dim3(1), dim3(1), 0, st, seq_lens, slot, pos0 + T);
   HIP_TRY(hipGetLastError());
   return VUI_OK;

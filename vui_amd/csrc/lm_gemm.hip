@@ -719,28 +719,29 @@ static int lm_band(int MT, int NT, int bm, int bn) {
   return std::max(w, (int)std::min((long)NT, side / MT));  // few rows: all of them side by side
 }
 template <int EPI, int MBW, int NBW, int WM, int WN, int S, int KS, int G = 1>
-static int go_wide(LmGemm g, int nz, hipStream_t st) {
+static int go_wide(LmGemm g, hipStream_t st) {
   const int MT = (g.M + 16 * MBW * WM - 1) / (16 * MBW * WM), NT = ((EPI == LM_EXPAND && g.n_v > g.N ? g.n_v : g.N) / 16 + NBW * WN - 1) / (NBW * WN);
   const bool moe = EPI == LM_MOE_UP || EPI == LM_MOE_DOWN;
   const bool strided = MBW * WM == 8 && EPI != LM_EXPAND && NT >= WIDE_STRIDED;
   if (strided) g.band = 0;
   else lm_set_order(g, MT, NT, lm_band(MT, NT, MBW * WM, NBW * WN));
   const int tiles = moe ? g.max_tiles * ((NT + 7) & ~7) : MT * (strided ? (NT + 7) & ~7 : NT);
-  hipLaunchKernelGGL((lm_wide_kernel<EPI, MBW, NBW, WM, WN, S, KS, G>), dim3((unsigned)tiles, 1, nz), dim3(256 * G), 0, st, LM_HOT_ARGS(g, moe), g);
+  const int heads = EPI == LM_EXPAND ? 2 * g.heads : 1;  // keys of every head, values of every head
+  hipLaunchKernelGGL((lm_wide_kernel<EPI, MBW, NBW, WM, WN, S, KS, G>), dim3((unsigned)tiles, 1, heads), dim3(256 * G), 0, st, LM_HOT_ARGS(g, moe), g);
   HIP_TRY(hipGetLastError());
   return VUI_OK;
 }
 
 template <typename T, int MB, int NB, int WAVES, int EPI, bool ALT = false, bool FEW = false>
-static int go(LmGemm g, int nz, hipStream_t st) {
+static int go(LmGemm g, hipStream_t st) {
   if constexpr (sizeof(T) == 2 && MB == 1 && !FEW && EPI != LM_MOE_UP && EPI != LM_MOE_DOWN)
-    if (g.M <= 4) return go<T, MB, NB, WAVES, EPI, ALT, true>(g, nz, st);
+    if (g.M <= 4) return go<T, MB, NB, WAVES, EPI, ALT, true>(g, st);
   const bool moe = EPI == LM_MOE_UP || EPI == LM_MOE_DOWN;
   const int nt = (g.N / 16 + NB - 1) / NB;
   const int mt = (g.M + 16 * MB - 1) / (16 * MB);
   lm_set_order(g, mt, nt, lm_band(mt, nt, MB, NB));
   const int tiles = moe ? g.max_tiles * ((nt + 7) & ~7) : mt * nt * (ALT ? 2 : 1);
-  hipLaunchKernelGGL((lm_gemm_kernel<T, MB, NB, WAVES, EPI, ALT, FEW>), dim3((unsigned)tiles, 1, nz), dim3(64 * WAVES), 0, st, LM_HOT_ARGS(g, moe), g);
+  hipLaunchKernelGGL((lm_gemm_kernel<T, MB, NB, WAVES, EPI, ALT, FEW>), dim3((unsigned)tiles), dim3(64 * WAVES), 0, st, LM_HOT_ARGS(g, moe), g);
   HIP_TRY(hipGetLastError());
   return VUI_OK;
 }
@@ -771,15 +772,14 @@ static int lm_tile(int epi, int M, int N, int K) {
 }
 template <int EPI>
 static int pick_wide(int tile, const LmGemm& g, hipStream_t st) {
-  const int nz = EPI == LM_EXPAND ? 2 * g.heads : 1;
   if constexpr (EPI != LM_EXPAND) {
-    if (tile == WIDE_64x128_2) return go_wide<EPI, 4, 2, 1, 4, 3, 2, 2>(g, nz, st);
-    if (tile == WIDE_64_2) return go_wide<EPI, 2, 2, 2, 2, 4, 2, 2>(g, nz, st);
+    if (tile == WIDE_64x128_2) return go_wide<EPI, 4, 2, 1, 4, 3, 2, 2>(g, st);
+    if (tile == WIDE_64_2) return go_wide<EPI, 2, 2, 2, 2, 4, 2, 2>(g, st);
   }
   switch (tile) {
-    case WIDE_128: return go_wide<EPI, 4, 4, 2, 2, 4, 1>(g, nz, st);
-    case WIDE_64x128: return go_wide<EPI, 4, 2, 1, 4, 3, 2>(g, nz, st);
-    default: return go_wide<EPI, 2, 2, 2, 2, 4, 2>(g, nz, st);
+    case WIDE_128: return go_wide<EPI, 4, 4, 2, 2, 4, 1>(g, st);
+    case WIDE_64x128: return go_wide<EPI, 4, 2, 1, 4, 3, 2>(g, st);
+    default: return go_wide<EPI, 2, 2, 2, 2, 4, 2>(g, st);
   }
 }
 
@@ -789,13 +789,13 @@ static int pick_wide(int tile, const LmGemm& g, hipStream_t st) {
 // 30 x 768 x 2816 7.7 / 6.6 / 5.4; at 224 tiles 7.8 / 6.5 / 7.4 (200 x 1024 x 2048), at 256 11.4 / 9.2 / 10.6 (100 x 2048 x 4096).
 // With more tiles than CUs they are each other's company: 400 x 6400 x 768 (1742 tiles) 16.2 with four waves, 23 with eight.
 template <typename T, int NB, int EPI>
-static int many(const LmGemm& g, int nz, hipStream_t st) {
+static int many(const LmGemm& g, hipStream_t st) {
   if constexpr (sizeof(T) == 2 && NB == 2) {
-    const long tiles = (long)((g.M + 31) / 32) * ((g.N + 31) / 32) * nz;
-    if (tiles <= 128) return go<T, 2, 1, 8, EPI>(g, nz, st);
-    if (tiles <= 256) return go<T, 2, 2, 8, EPI>(g, nz, st);
+    const long tiles = (long)((g.M + 31) / 32) * ((g.N + 31) / 32);
+    if (tiles <= 128) return go<T, 2, 1, 8, EPI>(g, st);
+    if (tiles <= 256) return go<T, 2, 2, 8, EPI>(g, st);
   }
-  return go<T, 2, NB, 4, EPI>(g, nz, st);
+  return go<T, 2, NB, 4, EPI>(g, st);
 }
 
 // Experts' products of few rows, which find their entries themselves.  Up to 24 tiles are walked to from expert to expert; with more, that is a
@@ -803,62 +803,62 @@ static int many(const LmGemm& g, int nz, hipStream_t st) {
 // launch; 8 steps with 64 experts 6410 / 6090, 768 wide with 128 4180 / 3995, 7 rows of 1024 (28 tiles) 3280 / 3241, but 4 rows of 768 2420 / 2447
 // and 5 (20 tiles) 2471 / 2494.
 template <typename T, int NB, int WAVES, int EPI>
-static int experts(const LmGemm& g, int nz, hipStream_t st) {
-  return g.choice && g.max_tiles > 24 ? go<T, 1, NB, WAVES, EPI, true>(g, nz, st) : go<T, 1, NB, WAVES, EPI>(g, nz, st);
+static int experts(const LmGemm& g, hipStream_t st) {
+  return g.choice && g.max_tiles > 24 ? go<T, 1, NB, WAVES, EPI, true>(g, st) : go<T, 1, NB, WAVES, EPI>(g, st);
 }
 
 // up to 16 rows: one row block, more waves per tile (the weights are streamed once, latency counts)
 template <typename T>
-static int pick(int epi, const LmGemm& g, int nz, hipStream_t st) {
+static int pick(int epi, const LmGemm& g, hipStream_t st) {
   const bool few = g.M <= 16;
-  const int tile = sizeof(T) == 2 && nz == 1 ? lm_tile(epi, g.M, g.N, g.K) : WIDE_NONE;
+  const int tile = sizeof(T) == 2 ? lm_tile(epi, g.M, g.N, g.K) : WIDE_NONE;
   if (tile != WIDE_NONE) {
     if (epi == LM_IN_ATTN) return pick_wide<LM_IN_ATTN>(tile, g, st);
-    if (epi == LM_IN_GRU_SEQ) return go_wide<LM_IN_GRU_SEQ, 4, 6, 2, 2, 3, 1>(g, 1, st);
+    if (epi == LM_IN_GRU_SEQ) return go_wide<LM_IN_GRU_SEQ, 4, 6, 2, 2, 3, 1>(g, st);
     if (epi == LM_OUT) return pick_wide<LM_OUT>(tile, g, st);
     if (epi == LM_PROJ) return pick_wide<LM_PROJ>(tile, g, st);
     if (epi == LM_PLAIN) return pick_wide<LM_PLAIN>(tile, g, st);
     if (epi == LM_ACT) return pick_wide<LM_ACT>(tile, g, st);
   }
   if (sizeof(T) == 2 && g.tile_rows == 32) {
-    if (epi == LM_MOE_UP) return go_wide<LM_MOE_UP, 2, 2, 1, 4, 4, 2>(g, nz, st);
-    if (epi == LM_MOE_DOWN) return go_wide<LM_MOE_DOWN, 2, 2, 1, 4, 4, 2>(g, nz, st);
+    if (epi == LM_MOE_UP) return go_wide<LM_MOE_UP, 2, 2, 1, 4, 4, 2>(g, st);
+    if (epi == LM_MOE_DOWN) return go_wide<LM_MOE_DOWN, 2, 2, 1, 4, 4, 2>(g, st);
   }
   if (sizeof(T) == 2 && g.tile_rows == 64) {
-    if (epi == LM_MOE_UP) return go_wide<LM_MOE_UP, 4, 2, 1, 4, 3, 2>(g, nz, st);
-    if (epi == LM_MOE_DOWN) return go_wide<LM_MOE_DOWN, 4, 2, 1, 4, 3, 2>(g, nz, st);
+    if (epi == LM_MOE_UP) return go_wide<LM_MOE_UP, 4, 2, 1, 4, 3, 2>(g, st);
+    if (epi == LM_MOE_DOWN) return go_wide<LM_MOE_DOWN, 4, 2, 1, 4, 3, 2>(g, st);
   }
   // few rows and few features: one block of features per workgroup, so that more of the chip takes part
   if (few && (long)g.N * (g.max_tiles > 0 ? g.max_tiles : 1) <= 4096) {
-    if (epi == LM_PROJ) return go<T, 1, 1, 16, LM_PROJ>(g, nz, st);
-    if (epi == LM_ACT) return go<T, 1, 1, 16, LM_ACT>(g, nz, st);
-    if (epi == LM_MOE_UP) return experts<T, 1, 16, LM_MOE_UP>(g, nz, st);
-    if (epi == LM_MOE_DOWN) return experts<T, 1, 16, LM_MOE_DOWN>(g, nz, st);
+    if (epi == LM_PROJ) return go<T, 1, 1, 16, LM_PROJ>(g, st);
+    if (epi == LM_ACT) return go<T, 1, 1, 16, LM_ACT>(g, st);
+    if (epi == LM_MOE_UP) return experts<T, 1, 16, LM_MOE_UP>(g, st);
+    if (epi == LM_MOE_DOWN) return experts<T, 1, 16, LM_MOE_DOWN>(g, st);
   }
   // few features still: half a block per workgroup where whole ones would leave half the CUs without, and the others take in a block's
   // weights at 45 KB a us (16 x 2048 x 6144 13.4 -> 11.7 us, the mean of a 2048 wide step's thirteen 7.8 -> 7.0, with 4 rows 6.8 -> 6.5; before half a
   // block's weights were one load per step)
-  if (few && epi == LM_PLAIN && (long)g.N / 16 * nz <= 128) return go<T, 1, 1, 16, LM_PLAIN, true>(g, nz, st);
+  if (few && epi == LM_PLAIN && g.N / 16 <= 128) return go<T, 1, 1, 16, LM_PLAIN, true>(g, st);
   if constexpr (sizeof(T) == 2)
-    if (few && epi == LM_OUT && g.N / 16 <= 128) return go<T, 1, 1, 16, LM_OUT, true>(g, nz, st);
+    if (few && epi == LM_OUT && g.N / 16 <= 128) return go<T, 1, 1, 16, LM_OUT, true>(g, st);
   switch (epi) {
-    case LM_IN_ATTN: return few ? go<T, 1, 2, 8, LM_IN_ATTN>(g, nz, st) : many<T, 2, LM_IN_ATTN>(g, nz, st);
-    case LM_IN_GRU_STEP: return go<T, 1, 3, 8, LM_IN_GRU_STEP>(g, nz, st);
-    case LM_IN_GRU_SEQ: return few ? go<T, 1, 3, 8, LM_IN_GRU_SEQ>(g, nz, st) : many<T, 3, LM_IN_GRU_SEQ>(g, nz, st);
-    case LM_OUT: return few ? go<T, 1, 1, 16, LM_OUT>(g, nz, st) : many<T, 2, LM_OUT>(g, nz, st);
-    case LM_LOGITS: return few ? go<T, 1, 2, 8, LM_LOGITS>(g, nz, st) : many<T, 2, LM_LOGITS>(g, nz, st);
-    case LM_HEAD: return few ? go<T, 1, 2, 8, LM_HEAD>(g, nz, st) : many<T, 2, LM_HEAD>(g, nz, st);
-    case LM_PROJ: return few ? go<T, 1, 2, 8, LM_PROJ>(g, nz, st) : many<T, 2, LM_PROJ>(g, nz, st);
-    case LM_PLAIN: return few ? go<T, 1, 1, 16, LM_PLAIN>(g, nz, st) : many<T, 2, LM_PLAIN>(g, nz, st);
-    case LM_ACT: return few ? go<T, 1, 2, 8, LM_ACT>(g, nz, st) : many<T, 2, LM_ACT>(g, nz, st);
-    case LM_MOE_UP: return few ? experts<T, 2, 8, LM_MOE_UP>(g, nz, st) : go<T, 2, 2, 4, LM_MOE_UP>(g, nz, st);
-    case LM_MOE_DOWN: return few ? experts<T, 2, 8, LM_MOE_DOWN>(g, nz, st) : go<T, 2, 2, 4, LM_MOE_DOWN>(g, nz, st);
+    case LM_IN_ATTN: return few ? go<T, 1, 2, 8, LM_IN_ATTN>(g, st) : many<T, 2, LM_IN_ATTN>(g, st);
+    case LM_IN_GRU_STEP: return go<T, 1, 3, 8, LM_IN_GRU_STEP>(g, st);
+    case LM_IN_GRU_SEQ: return few ? go<T, 1, 3, 8, LM_IN_GRU_SEQ>(g, st) : many<T, 3, LM_IN_GRU_SEQ>(g, st);
+    case LM_OUT: return few ? go<T, 1, 1, 16, LM_OUT>(g, st) : many<T, 2, LM_OUT>(g, st);
+    case LM_LOGITS: return few ? go<T, 1, 2, 8, LM_LOGITS>(g, st) : many<T, 2, LM_LOGITS>(g, st);
+    case LM_HEAD: return few ? go<T, 1, 2, 8, LM_HEAD>(g, st) : many<T, 2, LM_HEAD>(g, st);
+    case LM_PROJ: return few ? go<T, 1, 2, 8, LM_PROJ>(g, st) : many<T, 2, LM_PROJ>(g, st);
+    case LM_PLAIN: return few ? go<T, 1, 1, 16, LM_PLAIN>(g, st) : many<T, 2, LM_PLAIN>(g, st);
+    case LM_ACT: return few ? go<T, 1, 2, 8, LM_ACT>(g, st) : many<T, 2, LM_ACT>(g, st);
+    case LM_MOE_UP: return few ? experts<T, 2, 8, LM_MOE_UP>(g, st) : go<T, 2, 2, 4, LM_MOE_UP>(g, st);
+    case LM_MOE_DOWN: return few ? experts<T, 2, 8, LM_MOE_DOWN>(g, st) : go<T, 2, 2, 4, LM_MOE_DOWN>(g, st);
   }
   vui_set_error("lm gemm: unknown epilogue %d", epi);
   return VUI_EINVAL;
 }
 
-int launch_lm_gemm(int dtype, int epi, const LmGemm& g, int nz, hipStream_t st) {
+int launch_lm_gemm(int dtype, int epi, const LmGemm& g, hipStream_t st) {
   if ((epi == LM_LOGITS || epi == LM_HEAD) && g.N >= LM_SIZES) {  // a larger vocabulary by parts, the lengths with the last
     const int part = LM_SIZES / 2;
     for (int n = 0, rc; n < g.N; n += part) {
@@ -866,11 +866,11 @@ int launch_lm_gemm(int dtype, int epi, const LmGemm& g, int nz, hipStream_t st) 
       h.N = std::min(part, g.N - n); h.W = (const char*)g.W + (size_t)n * g.K * (dtype == VUI_DTYPE_F32 ? 4 : 2);
       h.logits = g.logits + n; h.vocab = g.vocab - n;
       if (h.N < g.N - n) h.upd_lens = nullptr;
-      if ((rc = launch_lm_gemm(dtype, epi, h, nz, st))) return rc;
+      if ((rc = launch_lm_gemm(dtype, epi, h, st))) return rc;
     }
     return VUI_OK;
   }
-  if (g.M < 1 || g.N < 16 || (g.N & 15) || g.K < 64 || (g.K & 63) || nz < 1 || g.N >= LM_SIZES || g.K >= LM_SIZES || g.np > 0xffff) {
+  if (g.M < 1 || g.N < 16 || (g.N & 15) || g.K < 64 || (g.K & 63) || g.N >= LM_SIZES || g.K >= LM_SIZES || g.np > 0xffff) {
     vui_set_error("lm gemm: bad shape M=%d N=%d K=%d", g.M, g.N, g.K);
     return VUI_EINVAL;
   }
@@ -886,7 +886,7 @@ int launch_lm_gemm(int dtype, int epi, const LmGemm& g, int nz, hipStream_t st) 
     return VUI_EINVAL;
   }
   if (epi == LM_IN_GRU_STEP && g.M > 16) { vui_set_error("lm gemm: a recurrence step takes at most 16 rows"); return VUI_EINVAL; }
-  return dtype == VUI_DTYPE_F32 ? pick<float>(epi, g, nz, st) : pick<bf16_t>(epi, g, nz, st);
+  return dtype == VUI_DTYPE_F32 ? pick<float>(epi, g, st) : pick<bf16_t>(epi, g, st);
 }
 
 // ---- embedding rows: residual, operand copy, sums of squares per 16 columns ----

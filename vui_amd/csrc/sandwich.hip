@@ -127,7 +127,7 @@ static LmGemm product(const vui_lm_ctx* x, const vui_lm_dims& d, const LmRows& r
 static int plain(const vui_lm_ctx* x, const vui_lm_dims& d, const LmRows& rows, const void* X, const void* W, const float* bias, int M, int N, int K, float* y, hipStream_t st) {
   LmGemm g = product(x, d, rows, X, W, M, N, K);
   g.bias = bias; g.out = y; g.ldo = N;
-  return launch_lm_gemm(x->c.dtype, LM_PLAIN, g, 1, st);
+  return launch_lm_gemm(x->c.dtype, LM_PLAIN, g, st);
 }
 
 static int mixer(vui_lm_ctx* x, int l, int M, const LmRows& rows, hipStream_t st) {
@@ -135,7 +135,7 @@ static int mixer(vui_lm_ctx* x, int l, int M, const LmRows& rows, hipStream_t st
   const vui_lm_dims& d = x->dims[l];
   LmGemm g = product(x, d, rows, x->xt, L.w_in, M, d.in_rows, d.w64);
   g.bias = L.in_bias; g.out = x->raw; g.ldo = d.in_rows;
-  int rc = launch_lm_gemm(x->c.dtype, LM_PROJ, g, 1, st);
+  int rc = launch_lm_gemm(x->c.dtype, LM_PROJ, g, st);
   if (rc) return rc;
   if (L.mixer == VUI_LM_GLA) {
     GlaArgs a;
@@ -182,7 +182,7 @@ static int feed_forward(vui_lm_ctx* x, int l, int M, const LmRows& rows, hipStre
   LmGemm up = product(x, d, rows, x->xt, L.w_up, M, d.ff16, d.w64);
   up.act = x->ffa; up.act_k = d.ff64; up.act_kind = L.act; up.act_pos = L.act_pos; up.act_neg = L.act_neg;
   if (L.experts == 0) {
-    if ((rc = launch_lm_gemm(x->c.dtype, LM_ACT, up, 1, st))) return rc;
+    if ((rc = launch_lm_gemm(x->c.dtype, LM_ACT, up, st))) return rc;
     return plain(x, d, rows, x->ffa, L.w_down, nullptr, M, d.out_rows, d.ff64, x->y, st);
   }
   if (!lm_rows_routes(M, d.experts16) && (rc = plain(x, d, rows, x->xt, L.w_router, L.router_bias, M, d.experts16, d.w64, x->rlog, st))) return rc;
@@ -197,11 +197,11 @@ static int feed_forward(vui_lm_ctx* x, int l, int M, const LmRows& rows, hipStre
     if ((rc = launch_moe_gather(x->c.dtype, r, x->xt, x->xg, d.w64, up.max_tiles, st))) return rc;
     up.X = x->xg; up.sorted = 1;
   }
-  if ((rc = launch_lm_gemm(x->c.dtype, LM_MOE_UP, up, 1, st))) return rc;
+  if ((rc = launch_lm_gemm(x->c.dtype, LM_MOE_UP, up, st))) return rc;
   LmGemm down = product(x, d, rows, x->ffa, L.w_down, M, d.out_rows, d.ff64);
   down.ent = x->ent; down.tile_e = x->tile_e; down.n_tiles = x->n_tiles; down.choice = up.choice; down.top = L.top; down.wz = (size_t)d.out_rows * d.ff64;
   down.max_tiles = up.max_tiles; down.tile_rows = r.tile_rows; down.out = x->y; down.ldo = d.out_rows;
-  return launch_lm_gemm(x->c.dtype, LM_MOE_DOWN, down, 1, st);
+  return launch_lm_gemm(x->c.dtype, LM_MOE_DOWN, down, st);
 }
 
 int sandwich_layers(vui_lm_ctx* x, const int64_t* tokens, int M, const LmRows& rows, hipStream_t st) {
