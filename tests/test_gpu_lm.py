@@ -427,6 +427,10 @@ def test_restore_takes_what_copies_take():
         cache.restore(1, 7, None)
     with pytest.raises(IndexError):
         cache.restore(99, 7, kept)
+    for length in (2 ** 31, 2 ** 32 + 7):  # beyond a slot's 32 bits
+        with pytest.raises(RuntimeError):
+            cache.restore(1, length, kept)
+    assert int(cache.seq_lens[1]) == 7
 
 
 def margin_ok(cfg, sd, prompt, drawn, dt):

@@ -78,7 +78,7 @@ class SlotCache:
         lens = self.seq_lens
         if not lens.is_cuda or lens.device.index != torch.cuda.current_device() or type(slot) is not int or not 0 <= slot < self.n_slots:
             return False
-        if type(length) is not int or (lens.is_inference() and not torch.is_inference_mode_enabled()):
+        if type(length) is not int or length >= 2 ** 31 or (lens.is_inference() and not torch.is_inference_mode_enabled()):
             return False
         to, frm, n = [], [], []
         for i, s in states.items():
