@@ -433,6 +433,20 @@ def test_restore_takes_what_copies_take():
     assert int(cache.seq_lens[1]) == 7
 
 
+def test_restore_of_states_of_the_slot_itself():
+    """Views of the slot's own states, each layer's from the other: one copy after the other, as what is read first counts."""
+    cfg = U.config([U.gru(40), U.attn(), U.gru(40)])
+    cache = U.engine(cfg, U.weights(cfg, 23)).model.cache
+    a, b = cache.state
+    for _ in range(3):
+        kept = {i: torch.randn_like(s[1]) for i, s in cache.state.items()}
+        cache.restore(1, 7, kept)
+        cache.restore(1, 9, {a: cache.state[b][1], b: cache.state[a][1]})
+        assert torch.equal(cache.state[a][1], kept[b]) and torch.equal(cache.state[b][1], kept[b]) and int(cache.seq_lens[1]) == 9
+        cache.restore(1, 8, {a: kept[a], b: kept[a]})  # one source for both
+        assert torch.equal(cache.state[a][1], kept[a]) and torch.equal(cache.state[b][1], kept[a]) and int(cache.seq_lens[1]) == 8
+
+
 def margin_ok(cfg, sd, prompt, drawn, dt):
     """Every drawn token is the oracle's choice or within the tolerance of it."""
     L = O.forward(cfg, sd, list(prompt) + drawn)[len(prompt) - 1:-1]

@@ -15,6 +15,7 @@ from __future__ import annotations
 import ctypes as C
 import json
 import os
+from operator import gt
 
 import torch
 from torch import Tensor
@@ -85,11 +86,11 @@ class SlotCache:
             t = self.state[i]
             if s.dtype != torch.float32 or s.device != t.device or not s.is_contiguous() or not t.is_contiguous() or s.shape != t.shape[1:]:
                 return False
-            at, src, size = t.data_ptr() + slot * t.stride(0) * 4, s.data_ptr(), s.numel()
-            if abs(at - src) < 4 * size:  # a view of the slot itself
-                return False
-            to.append(at), frm.append(src), n.append(size)
+            to.append(t.data_ptr() + slot * t.stride(0) * 4), frm.append(s.data_ptr()), n.append(s.numel())
         k = len(n)
+        begins, ends = sorted(to + frm), sorted([p + 4 * m for p, m in zip(to + frm, n + n)])
+        if any(map(gt, ends, begins[1:])):  # something overlaps: views of the slot's own states, of whatever layer, whose copies are in an order
+            return False
         _lib.check(_lib.load(lm_only=True).vui_lm_restore((C.c_void_p * k)(*to), (C.c_void_p * k)(*frm), (C.c_int64 * k)(*n), k, lens.data_ptr(), slot,
                                                           length, torch.cuda.current_stream().cuda_stream), "vui_lm_restore")
         return True
