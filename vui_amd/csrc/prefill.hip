@@ -750,8 +750,11 @@ struct PfDirectArgs {
 // A short block's products wait for their weights (1-2 us of launches of 3-5), and its attention leaves most compute units idle: workgroups of its
 // launch read the weights of the products up to the next attention into the L2s that will ask for them.  L2s keep what they hold
 // from launch to launch; pf_order deals an eighth of a matrix's features to an XCD, and workgroup i is on XCD i % 8.  Measured, a whole prompt on
-// the device: 23 positions in bf16 705 -> 635 us, four of 23 2294 -> 2130; 16 of 16 in int8, half the bytes, 8.9 ms both.  No more than PF_AHEAD_BYTES:
-// the L2s of a card hold 32 MB, and what does not stay is read twice.
+// the device, us without / with: bf16, an empty slot's 5, 16, 24 and 60 positions 491 / 480, 512 / 484, 591 / 549, 656 / 612, 16 behind 100, 700 and 2000
+// cached ones 528 / 482, 580 / 517, 627 / 576; int8 (half the bytes) 434 / 440, 450 / 455, 533 / 543, 587 / 585, 467 / 465, 517 / 515, 594 / 592, 40 behind 2000
+// 725 / 704, sixteen rows 549 / 549: nothing on average, 2 % lost at most and 3 % gained, so that the type makes no rule.  A vocoder on another stream loses
+// nothing by what its L2s held: 16 behind 700 and six streamed frames beside each other 620 / 561 and 5046 / 4830, in int8 565 / 555 and 4833 / 4810.  No more
+// than PF_AHEAD_BYTES: the L2s of a card hold 32 MB, and what does not stay is read twice.
 // Workgroups per XCD, 20 / 32 / 48: an empty slot's 9, 23 and 60 positions in bf16 537 / 514 / 520, 604 / 569 / 562, 658 / 612 / 611 us, four turns behind
 // 700 7204 / 7128 / 7129, sixteen in int8 14.95 / 14.96 / 15.09 ms.
 #define PF_AHEAD 32
