@@ -999,7 +999,7 @@ __global__ __launch_bounds__(256) void pf_stage_kv_kernel(const bf16_t* __restri
 // Fitted to 384 products (130 ... 2048 rows, widths 512, 768, 1024, bf16 and int8, weights of 22 layers in turn): on average 2 %
 // above the best form of each and 6 % below K-splitting alone; 6 products are more than 5 % above that, 19 % at most.
 // The bf16 forms once more, beside each other in whole prompts of 200 ... 2048 positions at widths 512, 768 and 1024: of 204 products the form
-// taken was 0.58 us above the quickest on average and is 0.1 now.  Prompts of width 768 with that and the norms' one trip, us: 1000 1510 -> 1448, 1500 1952 -> 1790, 1733 2049 -> 1918.
+// taken was 0.58 us above the quickest on average and is 0.1 now.  Prompts of width 768 with that and the norms' one trip, us: 1000 1514 -> 1450, 1500 1970 -> 1810, 1733 2091 -> 1970.
 // us, K-splitting / 128 x 128 / 64 x 128 / 64 x 64, bf16 at width 768: W1 and W3 at 577 rows 13.3 / 13.5 / 14.5 / 14.0, at 1000
 // 16.9 / 14.0 / 13.7 / 16.4, at 1733 25.3 / 19.3 / 22.7 / 25.6; W2 at 577 10.6 / 26.2 / 17.3 / 12.0, at 1733 29.4 / 26.3 / 17.6 / 17.8.
 static int pf_pick(int M, int N, int K, bool pair, bool i8) {
